@@ -93,12 +93,11 @@ const char* lvx_strerror(int code);
  * kv_splits > 1 cuts the shard into that many key ranges computed by separate
  * work-groups and folded before return; it needs a workspace of
  * lvx_fwd_workspace_bytes(shape, row_count, kv_splits) bytes.
- * The bf16 kernel without a dense bias or an interval mask has two forms: a wavefront owns
- * 32 text rows, or 64 rows and its SIMD to itself (half the LDS traffic per MFMA, one
- * work-group per CU).  The second is picked when row_count is a whole number of work-group
- * row blocks and the launch has at least one work-group per CU; the environment variable
- * LVX_FWD_WIDE (0 / 1, read at every call) overrides the choice.
- * Both forms give results within the same tolerance of each other, not the same bits.
+ * (at most 64 of them; lvx_fwd_auto_splits says how many suit a launch).
+ * The kernel has two forms: a wavefront owns 32 text rows of a head (any head_dim, the only one with a
+ * dense bias), or 64 rows and its SIMD to itself (head_dim 128 and 64).  The environment variable
+ * LVX_FWD_WIDE, read at every call, overrides the choice: 0 the first form, 1 the second where it exists.
+ * The forms give results within the same tolerance of each other, not the same bits.
  */
 int lvx_fwd(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tensor* k,
             const lvx_tensor* v, const lvx_tensor* o, float* lse,
@@ -119,6 +118,12 @@ int lvx_fwd_acc(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tens
                 void* workspace, size_t workspace_bytes, void* stream);
 
 size_t lvx_fwd_workspace_bytes(const lvx_attn_shape* shape, int32_t row_count, int32_t kv_splits);
+
+/*
+ * The number of key splits (1 .. 64) with which lvx_fwd is estimated to be fastest for `row_count`
+ * text rows.  Looks at sizes only (and at whether there is a bias); 1 for an invalid shape.
+ */
+int lvx_fwd_auto_splits(const lvx_attn_shape* shape, int32_t row_count);
 
 /*
  * lvx_fwd for callers that cannot allocate device memory (code under HIP graph capture,

@@ -1,51 +1,69 @@
-"""Writes lvx_fwd_loop_wide.inc: the hand-scheduled steady-state loop of the forward kernel whose
-waves own TWO blocks of 32 text rows (lvx_fwd.hip, fwd_kernel_wide).
+"""Writes the key-tile loop of the forward kernel whose waves own TWO blocks of 32 text rows
+(lvx_fwd.hip, fwd_wide_kernel), for one element type and head dimension:
 
-    python gen_fwd_loop_wide.py > lvx_fwd_loop_wide.inc
+    python gen_fwd_loop_wide.py bf16|f16 128|64 > lvx_fwd_loop_wide_<type>_<dim>.inc
 
-Same pipeline as gen_fwd_loop.py - per key tile t the MFMAs of S(t+1) = K(t+1) Q^T and of
-O += V(t)^T P(t) in program order, with the exponentials of tile t, the row maximum of tile t+1,
-the LDS operand reads and the global -> LDS loads between them - but every K or V operand read
-from LDS feeds two MFMAs, one per row block, so a wave reads half as many LDS bytes and a
-work-group requests half as many tile bytes per MFMA.  The wave has the SIMD to itself (512
-registers): the O^T accumulators and Q^T live in accumulation registers, which only MFMAs touch
-(the rare rescale of O goes through a few VGPRs).
+The statement runs ALL key tiles of a work-group, one or more.  Per key tile t it issues in program
+order the MFMAs of S(t+1) = K(t+1) Q^T and of O += V(t)^T P(t), and between any two of them a few
+of the tile's other instructions: the exponentials of tile t, the row maximum of tile t+1, the LDS
+operand reads and the global -> LDS loads of K(t+2) and V(t+1).  Every K or V operand read from LDS
+feeds two MFMAs, one per row block.  The wave has the SIMD to itself (512 registers): the O^T
+accumulators and Q^T live in accumulation registers, which only MFMAs touch (the rare rescale of O
+goes through a few VGPRs).
 
-The statement receives O^T and Q^T in VGPRs, moves them up at entry and back at exit, and uses
-the VGPRs they arrived in for scores, P and operand slots in between.
+What only some tiles need sits behind the loop as out-of-line blocks the stream tests for with a
+scalar compare: the move of a row's reference maximum and the rescale of O, the element mask of a
+tile that some row of the work-group does not see in full, and the clamp of the load addresses to
+the last row of the key range when the next tile to be requested is the last.
 
 Register map (must match the constraints of the asm statement in lvx_fwd.hip), b = row block:
-  at entry / exit: v[64 b : 64 b + 63] O^T of block b, v[128 + 32 b : 159 + 32 b] Q^T of block b
-  inside: a[64 b : 64 b + 63] O^T, a[128 + 32 b : 159 + 32 b] Q^T
-          v[64 b : 64 b + 31] scores set A, v[64 b + 32 : 64 b + 63] scores set B
-          v[128 + 16 b : 143 + 16 b] P^T   v[160:199] ten operand slots
+  at entry: v[128 + 32 b :] Q^T of block b, 4 registers per k-step of 16
+  at exit : v[64 b :] O^T of block b, 16 registers per 32 values of d
+  inside  : a[64 b :] O^T, a[128 + 32 b :] Q^T
+            v[64 b : 64 b + 31] scores set A, v[64 b + 32 : 64 b + 63] scores set B
+            v[128 + 16 b : 143 + 16 b] P^T   v[160:199] ten operand slots
   v[200:207] K read addresses (per k-step)   v[208:215] V read addresses (d tile x half)
-  v[216:219] global offsets of the 4 row groups   v220+b m   v222+b l   v224+b alpha
-  v226+2b -m*c   v230+b .. v236+b scratch
-  s40 c = scale*log2(e)   s41 -inf   s42 8.0   s[44:45] K source of tile t+2   s[46:47] V source of
-  tile t+1   s48 / s49 bytes per K / V tile   s50 LDS address of this wave's part of buffer 0
-  s51 trips left   s[52:53], s[60:61] scratch   s[54:55], s[58:59] rows whose reference moved in the
-  tile before (zero on entry)   s56 scratch
+  v[216:219] / v[220:223] global byte offsets of this wave's pieces of the next K / V tile
+  v224 what of such an offset is not row * stride   v225+b first visible key - 4 * (lane / 32)
+  v227+b visible keys   v229+b m   v231+b l   v233+b alpha   v235+b -m*c   v237+b .. v243+b scratch
+  s40 c = scale*log2(e)   s41 -inf   s42 8.0   s[44:45] next K tile   s[46:47] next V tile
+  s48 / s49 bytes per K / V tile   s50 LDS address of this wave's part of buffer 0
+  s51 tiles after the current one   s57 / s62 tiles after the next K / V tile
+  s64 / s65 byte offset of the last row of the key range in its tile (K / V)
+  s66 first key of the tile whose scores are formed   s67, s68 no row masks anything in the tiles
+  with (s66 - s67) <= s68, unsigned   s[52:53], s[60:61], s[70:71], s56 scratch
+  s[54:55], s[58:59] rows whose reference moved in the tile before
 """
 import os
 import re
+import sys
 
 # experiment switches (comma separated in LVX_GEN_OPTS); none is set in a normal build
 OPTS = dict((o.split("=") + ["1"])[:2] for o in os.environ.get("LVX_GEN_OPTS", "").split(",") if o)
-MFMA = "v_mfma_f32_32x32x16_bf16"
+F16 = len(sys.argv) > 1 and sys.argv[1] == "f16"
+DH = int(sys.argv[2]) if len(sys.argv) > 2 else 128
+MFMA = "v_mfma_f32_32x32x16_f16" if F16 else "v_mfma_f32_32x32x16_bf16"
+CVT = "v_cvt_pk_f16_f32" if F16 else "v_cvt_pk_bf16_f32"
 
+NKK, NDT = DH // 16, DH // 32       # k-steps of S, 32-wide blocks of O^T
+NS, NV = 2 * NKK, 4 * NDT           # operands of the S phase (k-step x key half) and of the V phase
+NLD = DH // 32                      # 1 KiB pieces of a tile per wave
+ROWB = 2 * DH                       # bytes per row of a tile in LDS
+TILE = 64 * ROWB
 NB = 2
 SC = [[0, 32], [64, 96]]            # score sets [block][set]
 PB = [128, 144]
-STG, KA, VA, DO = 160, 200, 208, 216
-MI, LI, AL = [220, 221], [222, 223], [224, 225]
-NMC = [226, 228]
-MX, T0, T1, RS1 = [230, 231], [232, 233], [234, 235], [236, 237]
+STG, KA, VA, DOK, DOV, LDC = 160, 200, 208, 216, 220, 224
+ME, ML = [225, 226], [227, 228]
+MI, LI, AL = [229, 230], [231, 232], [233, 234]
+NMC = [235, 236]
+MX, T0, T1, RS1 = [237, 238], [239, 240], [241, 242], [243, 244]
 AACC, AQ = [0, 64], [128, 160]
 RMASK = ["s[54:55]", "s[58:59]"]
 CMASK = ["s[52:53]", "s[60:61]"]
 NSLOT, AHEAD, WBATCH = 10, int(OPTS.get("ahead", 8)), int(OPTS.get("wbatch", 2))
-TILE = 16384
+# VALU instructions behind an MFMA of the S / V phase: with heads of 64 the same softmax has half as many
+TAKE_S, TAKE_V = (int(OPTS.get("s1", 4)), int(OPTS.get("s2", 5))) if DH == 128 else (int(OPTS.get("s1", 8)), int(OPTS.get("s2", 10)))
 
 
 def vr(base, n=1):
@@ -105,14 +123,45 @@ def exp_group(b, cur, j, nmc, first):
         else:
             pend.append(f"v_add_f32 v{LI[b]}, v{LI[b]}, v{r0}")
             pend.append(f"v_add_f32 v{RS1[b]}, v{RS1[b]}, v{r1}")
-        pend.append(f"v_cvt_pk_bf16_f32 v{PB[b] + 4 * j + e}, v{r0}, v{r1}")
+        pend.append(f"{CVT} v{PB[b] + 4 * j + e}, v{r0}, v{r1}")
     ins.append("s_nop 0")
     ins += pend
     return ins
 
 
-SLOW = []       # out-of-line code: the reference moves of the tiles of the loop
+SLOW = []       # out-of-line code
 N_SLOW = [0]
+
+
+def new_label():
+    N_SLOW[0] += 1
+    return N_SLOW[0]
+
+
+def mask_test(nxt):
+    """Is the next tile one that some row does not see in full?  Then (out of line) its scores at keys a
+    lane's row does not see become -inf, for both row blocks."""
+    n = new_label()
+    out = [f"LVX_FWDW_MASK{n}_%=:", f"v_mov_b32 v{T1[1]}, s41"]
+    pairs = ["s[52:53]", "s[60:61]", "s[70:71]", "vcc"]
+    for b in range(NB):
+        base = T0[b]
+        tmp = [MX[0], MX[1], T1[0], T0[1 - b]]
+        out.append(f"v_sub_u32 v{base}, s66, v{ME[b]}")
+        for q in range(8):                              # scores 4 q .. 4 q + 3
+            regs = [SC[b][nxt] + 4 * q + i for i in range(4)]
+            keys = [32 * (q // 4) + 8 * (q % 4) + i for i in range(4)]
+            for i in range(4):
+                out.append(f"v_add_u32 v{tmp[i]}, {keys[i]}, v{base}")
+            for i in range(4):
+                out.append(f"v_cmp_lt_u32 {pairs[i]}, v{tmp[i]}, v{ML[b]}")
+            out.append("s_nop 1")
+            for i in range(4):
+                out.append(f"v_cndmask_b32 v{regs[i]}, v{T1[1]}, v{regs[i]}, {pairs[i]}")
+    out += ["s_nop 1", f"s_branch LVX_FWDW_MASKED{n}_%="]
+    SLOW.extend(out)
+    return [["s_sub_u32 s56, s66, s67", "s_cmp_gt_u32 s56, s68", f"s_cbranch_scc1 LVX_FWDW_MASK{n}_%=",
+             f"LVX_FWDW_MASKED{n}_%=:"]]
 
 
 def next_max(b, nxt):
@@ -125,8 +174,7 @@ def next_max(b, nxt):
     for v in range(2, 16):
         ins.append(f"v_max3_f32 v{mx}, v{mx}, v{s1 + v - 1}, v{s0 + v}")
     ins.append(f"v_max_f32 v{mx}, v{mx}, v{s1 + 15}")
-    n = N_SLOW[0]
-    N_SLOW[0] += 1
+    n = new_label()
     ins += [
         f"v_mov_b32 v{t0}, v{mx}",
         "s_nop 1",
@@ -167,7 +215,7 @@ def rescale(b, tag, e):
     a time travel through the operand slots, which hold nothing at the top of a tile."""
     e([f"s_cmp_lg_u64 {RMASK[b]}, 0", f"s_cbranch_scc1 LVX_FWDW_RESC{tag}{b}_%=", f"LVX_FWDW_RESCD{tag}{b}_%=:"])
     out = [f"LVX_FWDW_RESC{tag}{b}_%=:", "s_nop 15", "s_nop 3", f"v_mul_f32 v{LI[b]}, v{LI[b]}, v{AL[b]}"]
-    for c in range(4):
+    for c in range(NDT):
         for r in range(16):
             out.append(f"v_accvgpr_read_b32 v{STG + r}, a{AACC[b] + 16 * c + r}")
         for r in range(16):
@@ -178,8 +226,23 @@ def rescale(b, tag, e):
     SLOW.extend(out)
 
 
+def advance(left, lo, hi, stride, offs, limit):
+    """The source of the next K (V) tile moves on unless it stands at the last tile; when it gets there
+    the row part of the offsets is cut to the last row of the key range (out of line)."""
+    n = new_label()
+    SLOW.append(f"LVX_FWDW_LAST{n}_%=:")
+    for j in range(NLD):
+        SLOW.extend([f"v_sub_u32 v{MX[0]}, v{offs + j}, v{LDC}", f"v_min_u32 v{MX[0]}, {limit}, v{MX[0]}",
+                     f"v_add_u32 v{offs + j}, v{MX[0]}, v{LDC}"])
+    SLOW.append(f"s_branch LVX_FWDW_STAY{n}_%=")
+    return [f"s_cmp_eq_u32 {left}, 0", f"s_cbranch_scc1 LVX_FWDW_STAY{n}_%=",
+            f"s_add_u32 {lo}, {lo}, {stride}", f"s_addc_u32 {hi}, {hi}, 0",
+            f"s_sub_u32 {left}, {left}, 1", f"s_cmp_eq_u32 {left}, 0", f"s_cbranch_scc1 LVX_FWDW_LAST{n}_%=",
+            f"LVX_FWDW_STAY{n}_%=:"]
+
+
 def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
-    """One key tile t of the pipelined loop (par = t & 1 relative to the first tile of the run).
+    """One key tile t of the pipelined loop (par = t & 1 relative to the first tile).
     do_cur : P(t) from the current scores, O += V(t)^T P(t)
     do_next: S(t+1) = K(t+1) Q^T into the other score set, its row maximum and reference move
     do_dma : request K(t+2) and V(t+1)"""
@@ -191,22 +254,23 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
         # K(t+1) and V(t) have landed; nobody reads K(t) / V(t-1) any more
         e("s_waitcnt vmcnt(0)")
         e("s_barrier")
+        if do_next:
+            e("s_add_u32 s66, s66, 64")
     if do_cur:
         for b in range(NB):
             rescale(b, tag, e)
 
-    # operand n: 0..15 = K (k-step n/2, key half n%2) from buffer par^1; 16..31 = V (k-step j = (n-16)/4,
-    # d tile (n-16)%4) from buffer par
-    ops = (list(range(16)) if do_next else []) + (list(range(16, 32)) if do_cur else [])
+    # operand n: below NS = K (k-step n/2, key half n%2) from buffer par^1; above = V (k-step j, d tile dt) from buffer par
+    ops = (list(range(NS)) if do_next else []) + (list(range(NS, NS + NV)) if do_cur else [])
 
     def read_op(n):
         slot = STG + 4 * (n % NSLOT)
-        if n < 16:
+        if n < NS:
             kk, half = n // 2, n % 2
-            st.lds_read(f"ds_read_b128 {vr(slot, 4)}, v{KA + kk} offset:{(par ^ 1) * 2 * TILE + half * 8192}", n)
+            st.lds_read(f"ds_read_b128 {vr(slot, 4)}, v{KA + kk} offset:{(par ^ 1) * 2 * TILE + half * 32 * ROWB}", n)
         else:
-            j, dt = (n - 16) // 4, (n - 16) % 4
-            off = par * 2 * TILE + j * 4096
+            j, dt = (n - NS) // NDT, (n - NS) % NDT
+            off = par * 2 * TILE + j * 16 * ROWB
             st.lds_read(f"ds_read_b64_tr_b16 {vr(slot, 2)}, v{VA + 2 * dt} offset:{off}", n)
             st.lds_read(f"ds_read_b64_tr_b16 {vr(slot + 2, 2)}, v{VA + 2 * dt + 1} offset:{off}", n)
 
@@ -230,6 +294,7 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
             valu.append(f"v_add_f32 v{LI[b]}, v{LI[b]}, v{RS1[b]}")
     if do_next:
         first_max = len(valu)
+        valu += mask_test(nxt)
         for b in range(NB):
             valu += next_max(b, nxt)
     for s in valu[:n_pre]:
@@ -238,11 +303,10 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
     # global -> LDS loads: K(t+2) into K buffer par, V(t+1) into V buffer par^1
     dma = []
     if do_dma:
-        for j in range(4):
-            dma.append((f"s_add_i32 m0, s50, {par * 2 * TILE + j * 4096}", f"global_load_lds_dwordx4 v{DO + j}, s[44:45]"))
-        for j in range(4):
-            dma.append((f"s_add_i32 m0, s50, {(par ^ 1) * 2 * TILE + TILE + j * 4096}", f"global_load_lds_dwordx4 v{DO + j}, s[46:47]"))
-    s1, s2 = int(OPTS.get("s1", 4)), int(OPTS.get("s2", 5))
+        for j in range(NLD):
+            dma.append((f"s_add_i32 m0, s50, {par * 2 * TILE + j * 4096}", f"global_load_lds_dwordx4 v{DOK + j}, s[44:45]"))
+        for j in range(NLD):
+            dma.append((f"s_add_i32 m0, s50, {(par ^ 1) * 2 * TILE + TILE + j * 4096}", f"global_load_lds_dwordx4 v{DOV + j}, s[46:47]"))
     n_mfma = 0
     last_s = -100       # index of the last S MFMA
     for i, k in enumerate(ops):
@@ -250,14 +314,14 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
             st.wait_op(ops[min(i + WBATCH - 1, len(ops) - 1)])
         slot = STG + 4 * (k % NSLOT)
         for b in range(NB):
-            if k < 16:
+            if k < NS:
                 kk, half = k // 2, k % 2
                 d = SC[b][nxt] + 16 * half
                 c = "0" if kk == 0 else vr(d, 16)
                 e(f"{MFMA} {vr(d, 16)}, {vr(slot, 4)}, {ar(AQ[b] + 4 * kk, 4)}, {c}")
                 last_s = n_mfma
             else:
-                j, dt = (k - 16) // 4, (k - 16) % 4
+                j, dt = (k - NS) // NDT, (k - NS) % NDT
                 assert pos >= group_end[(b, j)], f"P^T k-step {j} of block {b} is not ready at operand {k}"
                 a = AACC[b] + 16 * dt
                 e(f"{MFMA} {ar(a, 16)}, {vr(slot, 4)}, {vr(PB[b] + 4 * j, 4)}, {ar(a, 16)}")
@@ -265,23 +329,14 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
             if b == NB - 1:
                 if i + AHEAD < len(ops):
                     read_op(ops[i + AHEAD])
-                if dma and k < 16 and k % 2 == 1:
+                if dma and k < NS and k % 2 == 1:
                     x, y = dma[k // 2]
                     e(x)
                     e(y)
-                if do_dma and k == 15:
-                    # the run has 2 * trips + 1 tiles: the last even tile must not move the K source past the
-                    # last tile (the odd tile after it then requests that tile once more, which nobody reads)
-                    if par == 0:
-                        e("s_cmp_lg_u32 s51, 1")
-                        e("s_cselect_b32 s56, s48, 0")
-                        e("s_add_u32 s44, s44, s56")
-                    else:
-                        e("s_add_u32 s44, s44, s48")
-                    e("s_addc_u32 s45, s45, 0")
-                    e("s_add_u32 s46, s46, s49")
-                    e("s_addc_u32 s47, s47, 0")
-            take = (s1 if k < 16 else s2) if do_next else 7
+                if do_dma and k == NS - 1:
+                    e(advance("s57", "s44", "s45", "s48", DOK, "s64"))
+                    e(advance("s62", "s46", "s47", "s49", DOV, "s65"))
+            take = (TAKE_S if k < NS else TAKE_V) if do_next else 7 * 128 // DH
             if i == len(ops) - 1 and b == NB - 1:
                 take = len(valu) - pos
             for _ in range(take):
@@ -289,7 +344,7 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
                     break
                 # the row maximum reads the scores the S MFMAs wrote: not before the last of them has had
                 # its wait states - with the V MFMAs behind it, no earlier than three MFMAs later
-                if pos >= first_max and (n_mfma - 1 < last_s + 4 or k < 16):
+                if pos >= first_max and (n_mfma - 1 < last_s + 4 or k < NS):
                     break
                 e(valu[pos])
                 pos += 1
@@ -361,42 +416,35 @@ def check(ins):
 
 
 def main():
-    # Entry: O^T and Q^T move up into the accumulation registers.
+    # Entry: Q^T moves up into the accumulation registers, O^T starts at 0, no row has a reference.
+    # K and V of the first tile and K of the second have been requested.
     pro = []
     for b in range(NB):
-        for r in range(64):
-            pro.append(f"v_accvgpr_write_b32 a{AACC[b] + r}, v{64 * b + r}")
-        for r in range(32):
+        for r in range(16 * NDT):
+            pro.append(f"v_accvgpr_write_b32 a{AACC[b] + r}, 0")
+        for r in range(4 * NKK):
             pro.append(f"v_accvgpr_write_b32 a{AQ[b] + r}, v{128 + 32 * b + r}")
-    # All loads of the run are the loop's own.  s[44:45] / s[46:47] point at K / V of its first tile.
-    pro += ["s_barrier"]
-    for j in range(4):
-        pro += [f"s_add_i32 m0, s50, {j * 4096}", f"global_load_lds_dwordx4 v{DO + j}, s[44:45]"]
-    for j in range(4):
-        pro += [f"s_add_i32 m0, s50, {TILE + j * 4096}", f"global_load_lds_dwordx4 v{DO + j}, s[46:47]"]
-    pro += ["s_add_u32 s44, s44, s48", "s_addc_u32 s45, s45, 0", "s_add_u32 s46, s46, s49", "s_addc_u32 s47, s47, 0"]
-    for j in range(4):
-        pro += [f"s_add_i32 m0, s50, {2 * TILE + j * 4096}", f"global_load_lds_dwordx4 v{DO + j}, s[44:45]"]
-    pro += ["s_add_u32 s44, s44, s48", "s_addc_u32 s45, s45, 0"]
-    pro += ["s_waitcnt vmcnt(4)", "s_barrier"]
-    for b in range(NB):     # -m*c of the reference the block arrives with (0 without one)
-        pro += [f"v_mul_f32 v{NMC[b]}, v{MI[b]}, -s40", f"v_cmp_neq_f32 vcc, s41, v{MI[b]}", "s_nop 1",
-                f"v_cndmask_b32 v{NMC[b]}, 0, v{NMC[b]}, vcc"]
+        pro += [f"v_mov_b32 v{MI[b]}, s41", f"v_mov_b32 v{LI[b]}, 0", f"v_mov_b32 v{NMC[b]}, 0"]
+    pro += ["s_waitcnt vmcnt(0)", "s_barrier"]
     # scores of the first tile (from K buffer 0 into score set A: the S phase of an odd tile)
     pro += tile(1, do_cur=False, do_next=True, do_dma=False, top=False)
+    # there is nothing to rescale yet
+    pro += ["s_mov_b64 s[54:55], 0", "s_mov_b64 s[58:59], 0"]
     t0, t1 = tile(0), tile(1)
-    fin = tile(0, do_cur=True, do_next=False, do_dma=False)
-    check(pro + t0 + t1 + t0 + t1 + fin)
-    lines = pro + ["LVX_FWDW_LOOP_%=:"] + t0 + t1
-    lines += ["s_sub_i32 s51, s51, 1", "s_cmp_lg_u32 s51, 0", "s_cbranch_scc1 LVX_FWDW_LOOP_%="]
-    lines += fin + ["s_nop 15", "s_nop 3"]
-    lines += ["s_branch LVX_FWDW_END_%="] + SLOW + ["LVX_FWDW_END_%=:"]
-    # Exit: O^T and Q^T come back down.
+    f0, f1 = tile(0, do_next=False, do_dma=False), tile(1, do_next=False, do_dma=False)
+    check(pro + t0 + t1 + t0 + f1)
+    check(pro + t0 + t1 + f0)
+    check(pro + f0)
+    lines = pro + ["LVX_FWDW_LOOP_%=:", "s_cmp_eq_u32 s51, 0", "s_cbranch_scc1 LVX_FWDW_FIN0_%="] + t0
+    lines += ["s_cmp_eq_u32 s51, 1", "s_cbranch_scc1 LVX_FWDW_FIN1_%="] + t1
+    lines += ["s_sub_u32 s51, s51, 2", "s_branch LVX_FWDW_LOOP_%="]
+    lines += SLOW
+    lines += ["LVX_FWDW_FIN1_%=:"] + f1 + ["s_branch LVX_FWDW_END_%="]
+    lines += ["LVX_FWDW_FIN0_%=:"] + f0 + ["LVX_FWDW_END_%=:", "s_nop 15", "s_nop 3"]
+    # Exit: O^T comes down.
     for b in range(NB):
-        for r in range(64):
+        for r in range(16 * NDT):
             lines.append(f"v_accvgpr_read_b32 v{64 * b + r}, a{AACC[b] + r}")
-        for r in range(32):
-            lines.append(f"v_accvgpr_read_b32 v{128 + 32 * b + r}, a{AQ[b] + r}")
     lines += ["s_nop 3"]
     print("// generated by gen_fwd_loop_wide.py - do not edit")
     for l in lines:

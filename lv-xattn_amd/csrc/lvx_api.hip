@@ -51,7 +51,7 @@ inline int gcd(int a, int b) { return b ? gcd(b, a % b) : a; }
 
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr int FWD_BN = 64;
-constexpr int MAX_SPLITS = 16;
+constexpr int MAX_SPLITS = 64;
 
 #define LVX_TRY(expr)            \
     do {                         \
@@ -124,15 +124,49 @@ size_t lvx_fwd_workspace_bytes(const lvx_attn_shape* s, int32_t row_count, int32
 
 static int cu_count();
 
-// Whether the forward runs in its wide form (a wave owns 64 rows and its SIMD; one work-group per
-// CU): bf16, head_dim 128, without a dense bias or an interval mask, whole 64-row blocks, and enough work-groups
-// that every CU has one.
-static bool fwd_wide(const lvx_attn_shape* s, int32_t row_count, int rs, int kv_splits) {
-    if (s->dtype != LVX_BF16 || s->D != 128 || s->bias || s->kv_start) return false;
-    if (const char* e = getenv("LVX_FWD_WIDE")) return atoi(e) != 0;
-    if (row_count % (64 * rs) != 0) return false;
-    const int64_t wgs = (int64_t)s->B * (s->Hq / (4 / rs)) * (row_count / (64 * rs)) * kv_splits;
-    return wgs >= cu_count();
+// Keys per split: whole tiles.
+static int fwd_split_len(const lvx_attn_shape* s, int splits) {
+    return ((s->Lkv + splits - 1) / splits + FWD_BN - 1) / FWD_BN * FWD_BN;
+}
+
+// What a forward launch over `rows` text rows in this form with this many key splits takes, in us; the
+// constants are fits to launches of 1 .. 4096 rows against 600 .. 76848 keys:
+//   wide : 11 us per round of work-groups, and per 64-key tile 1.1 us on an idle chip, 1.5 on a full one
+//          (0.9 and 1.05 with heads of 64).  256 rows x 6404 keys: 138 us whole, 39 in 8 parts
+//   plain: the same with 1.8 us per tile and two work-groups per CU
+// plus, with splits, 4 us for the launch that folds the parts and their bytes at 4 TB/s.
+static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits) {
+    const int hg = gcd(s->Hq / s->Hkv, 4), rs = 4 / hg, n_cu = cu_count();
+    const int64_t split_len = fwd_split_len(s, splits);
+    const int64_t n = (s->Lkv + split_len - 1) / split_len;
+    double t = n > 1 ? 4.0 + (double)n * s->B * s->Hq * rows * (4 * s->D + 8) / 4e6 : 0.0;
+    const int wg_rows = (form == FWD_WIDE ? 64 : 32) * rs;
+    const int64_t wgs = (int64_t)s->B * (s->Hq / hg) * ((rows + wg_rows - 1) / wg_rows) * n;
+    const int64_t slots = form == FWD_WIDE ? n_cu : 2 * n_cu;
+    const double load = std::min(1.0, (double)wgs / slots);
+    const double tile_us = form == FWD_PLAIN ? 0.8 + load : s->D == 128 ? 1.1 + 0.4 * load : 0.9 + 0.15 * load;
+    return t + (double)((wgs + slots - 1) / slots) * (split_len / FWD_BN * tile_us + 11.0);
+}
+
+// The form of the forward kernel.  Head dimensions 128 and 64 without a dense bias take the wide form;
+// the plain one was slower at every size measured (4096 rows x 6404 keys: 429 us against 354; 300 rows
+// x 2 samples: 92 against 88).
+static FwdForm fwd_form(const lvx_attn_shape* s) {
+    if (s->bias || (s->D != 128 && s->D != 64)) return FWD_PLAIN;
+    if (const char* e = getenv("LVX_FWD_WIDE")) return atoi(e) != 0 ? FWD_WIDE : FWD_PLAIN;
+    return FWD_WIDE;
+}
+
+int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
+    if (check_shape(s) != LVX_OK || row_count <= 0) return 1;
+    const FwdForm many = !s->bias && (s->D == 128 || s->D == 64) ? FWD_WIDE : FWD_PLAIN;
+    int best = 1;
+    double best_cost = 0.0;
+    for (int n = 1; n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
+        const double c = fwd_cost(s, row_count, many, n);
+        if (n == 1 || c < best_cost) { best = n; best_cost = c; }
+    }
+    return best;
 }
 
 // lvx_fwd, and lvx_fwd_acc when (o_in, l_in) is given: the result is then merged with that
@@ -165,14 +199,15 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     p.HG = gcd(p.G, 4);
     p.RS = 4 / p.HG;
     p.row_begin = row_begin; p.row_end = row_begin + row_count;
-    p.wide = fwd_wide(s, row_count, p.RS, kv_splits) ? 1 : 0;
-    const int wg_rows = (p.wide ? 64 : 32) * p.RS;
+    const FwdForm form = fwd_form(s);
+    p.form = form;
+    const int wg_rows = (form == FWD_WIDE ? 64 : 32) * p.RS;
     p.n_row_tiles = (row_count + wg_rows - 1) / wg_rows;
     p.n_head_groups = s->Hq / p.HG;
     p.scale = s->scale; p.scale_log2e = s->scale * LOG2E;
 
     int nsplit = kv_splits;
-    int split_len = ((s->Lkv + nsplit - 1) / nsplit + FWD_BN - 1) / FWD_BN * FWD_BN;
+    const int split_len = fwd_split_len(s, nsplit);
     nsplit = (s->Lkv + split_len - 1) / split_len;
     p.nsplit = nsplit;
     p.split_len = split_len;

@@ -6,8 +6,8 @@
 // ONE q head; the 4 waves of a group cover the q heads that share a kv head
 // (G = 4: four heads x 32 rows; G = 1: one head x 128 rows), so the K/V tile
 // staged in LDS is read by the whole GQA group and nothing is expanded in HBM.
-// (The bf16 kernel without a dense bias or an interval mask, fwd_kernel_pipe, also has a wide form in which
-// a wavefront owns 64 rows; see there.)
+// (That is fwd_kernel.  Head dimensions 128 and 64 without a dense bias run fwd_wide_kernel, in which a
+// wavefront owns 64 rows; see there.)
 //
 // Per 64-key tile and wave (all MFMA are v_mfma_f32_32x32x16_bf16):
 //   S^T[key, row]  = K_tile (A, from LDS)  x  Q^T (B, 32 VGPRs held for the whole kernel)
@@ -333,27 +333,37 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
     }
 }
 
-// registers the hand-scheduled loop uses besides its operands (see gen_fwd_loop.py)
-#define LVX_FWD_LOOP_CLOBBERS "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127", "v128", "v129", "v130", "v131", "v132", "v133", "v134", "v135", "v136", "v137", "v138", "v139", "v140", "v141", "v142", "v143", "v144", "v145", "v146", "v147", "v148", "v149", "v150", "v151", "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v160", "v161", "v162", "v163", "v164", "v165", "v166", "v167", "v168", "v169", "v170", "v171", "v172", "v173", "v174", "v175", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", "v187", "v188", "v189", "v190", "v191", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v200", "v201", "v202", "v203", "v204", "v205", "v206", "v207", "v208", "v209", "v210", "v211", "v212", "v213", "v214", "v215", "v246", "v247", "v248", "v249", "v250", "v251", "v252", "v253"
+// registers the wide loop uses besides its operands (see gen_fwd_loop_wide.py), heads of 128 and of 64
+#define LVX_FWD_WIDE_CLOBBERS_128 "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v233", "v234", "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191"
+#define LVX_FWD_WIDE_CLOBBERS_64 "v32", "v33", "v34", "v35", "v36", "v37", "v38", "v39", "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127", "v144", "v145", "v146", "v147", "v148", "v149", "v150", "v151", "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", "v187", "v188", "v189", "v190", "v191", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v204", "v205", "v206", "v207", "v212", "v213", "v214", "v215", "v218", "v219", "v222", "v223", "v233", "v234", "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175"
+#define LVX_FWD_WIDE_CLOBBERS_S "memory", "vcc", "scc", "m0", "s52", "s53", "s54", "s55", "s56", "s58", "s59", "s60", "s61", "s70", "s71"
 
-// the same for the wide loop (gen_fwd_loop_wide.py): its working VGPRs and the accumulation registers
-#define LVX_FWD_WIDE_CLOBBERS "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v224", "v225", "v226", "v227", "v228", "v229", "v230", "v231", "v232", "v233", "v234", "v235", "v236", "v237", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191"
-
-// The bf16 kernel without a dense bias or an interval mask (the one the benchmarks run): fwd_kernel's mapping, LDS
-// layout and tile code, but the run of key tiles that every row of the work-group sees in full
-// goes through a hand-scheduled loop (gen_fwd_loop.py) in which every wave interleaves the
-// MFMAs of a tile with the exponentials of that tile and the scores of the next one.  The
-// tiles before and after that run (the partial last tile, rows past the window) take the plain tile code.
+// The wide form (head dimensions 128 and 64, both element types, any mask but a dense bias): a wave
+// owns two blocks of 32 rows of its head and has its SIMD to itself (one work-group per CU, 512
+// registers per lane), so that every K / V operand read from LDS feeds two MFMAs: half the LDS reads
+// and half the global -> LDS bytes per MFMA of fwd_kernel.  All key tiles of the work-group - whole,
+// partial, masked, one or many - run in one hand-scheduled statement (gen_fwd_loop_wide.py): a tile in
+// compiler-scheduled code costs a wave of 512 registers 4 - 7 us, one in the loop 1.1 - 1.6.
+// Bound by the matrix pipe: 4096 rows x 32 heads x 6404 keys (0.43 TFLOP) takes 354 us, 1215 TFLOP/s,
+// where fwd_kernel takes 429; 2 x 3000 rows with image intervals 332 -> 261; 2 x 1023 rows 202 -> 182;
+// heads of 64, 2048 rows 145 -> 118 (half the MFMAs for the same softmax: bound by the VALU).
+// What a work-group takes besides its tiles is 11 us (one 64-key tile: 12.6): the first loads' latency,
+// the scores of the first tile, which nothing overlaps, and the rows going out.
 //
-// NBLK = 2 is the wide form: a wave owns two blocks of 32 rows of its head (64 rows), has its
-// SIMD to itself (one work-group per CU, 512 registers per lane) and feeds every K / V operand it
-// reads from LDS to two MFMAs, one per block (gen_fwd_loop_wide.py): half the LDS reads and half
-// the global -> LDS bytes per MFMA.
-template <int NBLK>
-__global__ __launch_bounds__(256, 3 - NBLK) void fwd_kernel_pipe(const FwdParams p) {
-    constexpr bool MASKED = false, BIAS = false, F16 = false;
+// LDS tiles: row r of a K or V tile has 2 DH bytes; its 16-byte chunk c sits at position c ^ f(r).
+//   DH = 128: f(r) = ((r & 3) << 2) | ((r >> 2) & 3), as in fwd_kernel
+//   DH = 64 : two rows share the 256 bytes of a pass over the banks, and f(r) = ((r >> 1 & 1) << 2) |
+//             ((r >> 2) & 3): the eight even and the eight odd rows of sixteen consecutive ones land
+//             in eight different positions each, and of the four rows of a transposing read those of
+//             like parity in different 64-byte halves
+template <int DH, bool MASKED, bool F16>
+__global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     using E = Elt<F16>;
-    __shared__ __attribute__((aligned(1024))) char kv_lds[2][2][TILE_BYTES];   // [buffer][K, V]
+    static_assert(DH == 128 || DH == 64, "head dimension");
+    constexpr int NKK = DH / 16, NDT = DH / 32, NLD = DH / 32;
+    constexpr int ROWB = 2 * DH, TB = BN * ROWB, CPR = DH / 8;      // bytes per tile row and tile, chunks per row
+    constexpr int RPL = 64 / CPR;                                   // tile rows one load of a wave fills
+    __shared__ __attribute__((aligned(1024))) char kv_lds[4 * TB];  // [buffer][K, V]
     __shared__ int red[4][4];
 
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
@@ -371,358 +381,222 @@ __global__ __launch_bounds__(256, 3 - NBLK) void fwd_kernel_pipe(const FwdParams
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int h = hg * p.HG + (wave % p.HG);
     const int hk = h / p.G;
-    int row[NBLK];
-    bool row_ok[NBLK];
-#pragma unroll
-    for (int blk = 0; blk < NBLK; ++blk) {
-        row[blk] = p.row_begin + ((tile * p.RS + wave / p.HG) * NBLK + blk) * 32 + l32;
-        row_ok[blk] = row[blk] < p.row_end;
-    }
+    const int row0 = p.row_begin + (tile * p.RS + wave / p.HG) * 64;       // this wave's first row
 
     int kv_len = p.Lkv;
     if (p.kv_len) kv_len = min(p.kv_len[b], p.Lkv);
     const int kv_lo = split * p.split_len;
     const int kv_hi = min(kv_len, kv_lo + p.split_len);
 
-    // this lane's visible key interval, per row block
-    int my_s[NBLK], my_e[NBLK];
-    int lo = BIG, hi = 0, in_lo = 0, in_hi = BIG;
+    // visible key interval of this lane's two rows.  Rows past the window and rows that see nothing
+    // are let see everything - the former are never stored, the latter stored as zeros - so that
+    // they do not make whole tiles take the element mask.
+    int my_s[2] = {kv_lo, kv_lo}, my_e[2] = {kv_hi, kv_hi};
+    bool empty[2] = {kv_hi <= kv_lo, kv_hi <= kv_lo};
+    int lo = kv_lo, hi = kv_hi, in_lo = kv_lo, in_hi = kv_hi;
+    if (MASKED) {
+        lo = BIG; hi = 0; in_lo = 0; in_hi = BIG;
 #pragma unroll
-    for (int blk = 0; blk < NBLK; ++blk) {
-        my_s[blk] = kv_lo;
-        my_e[blk] = kv_hi;
-        if (MASKED) {
-            if (row_ok[blk]) {
-                my_s[blk] = max(kv_lo, p.kv_start[(int64_t)b * p.Lq + row[blk]]);
-                my_e[blk] = min(kv_hi, p.kv_end[(int64_t)b * p.Lq + row[blk]]);
-            } else {
-                my_e[blk] = my_s[blk];
+        for (int blk = 0; blk < 2; ++blk) {
+            const int row = row0 + 32 * blk + l32;
+            if (row < p.row_end) {
+                my_s[blk] = max(kv_lo, p.kv_start[(int64_t)b * p.Lq + row]);
+                my_e[blk] = min(kv_hi, p.kv_end[(int64_t)b * p.Lq + row]);
+                empty[blk] = my_e[blk] <= my_s[blk];
+                if (!empty[blk]) {
+                    lo = min(lo, my_s[blk]);
+                    hi = max(hi, my_e[blk]);
+                    in_lo = max(in_lo, my_s[blk]);
+                    in_hi = min(in_hi, my_e[blk]);
+                }
             }
+            if (row >= p.row_end || empty[blk]) { my_s[blk] = 0; my_e[blk] = BIG; }
         }
-        if (my_e[blk] <= my_s[blk]) { my_s[blk] = BIG; my_e[blk] = 0; }
-        lo = min(lo, my_s[blk]);
-        hi = max(hi, my_e[blk]);
-        in_lo = max(in_lo, my_s[blk]);
-        in_hi = min(in_hi, my_e[blk]);
-    }
-
-    // work-group key range: [lo, hi) covers every non-empty row; tiles inside
-    // [in_lo, in_hi) are visible to every row and need no masking
+        // work-group key range: [lo, hi) covers every row, tiles inside [in_lo, in_hi) are visible to
+        // every row and need no masking
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        lo = min(lo, __shfl_xor(lo, off));
-        hi = max(hi, __shfl_xor(hi, off));
-        in_lo = max(in_lo, __shfl_xor(in_lo, off));
-        in_hi = min(in_hi, __shfl_xor(in_hi, off));
-    }
-    if (lane == 0) { red[wave][0] = lo; red[wave][1] = hi; red[wave][2] = in_lo; red[wave][3] = in_hi; }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        lo = min(lo, red[w][0]);
-        hi = max(hi, red[w][1]);
-        in_lo = max(in_lo, red[w][2]);
-        in_hi = min(in_hi, red[w][3]);
-    }
-    // the same in every lane of the work-group: keep them in scalar registers
-    lo = __builtin_amdgcn_readfirstlane(lo);
-    hi = __builtin_amdgcn_readfirstlane(hi);
-    in_lo = __builtin_amdgcn_readfirstlane(in_lo);
-    in_hi = __builtin_amdgcn_readfirstlane(in_hi);
-
-    // Q^T as B operand, resident for the whole kernel
-    bf16x8 qreg[NBLK][8];
-#pragma unroll
-    for (int blk = 0; blk < NBLK; ++blk) {
-        const uint16_t* qp = p.q + b * p.qs.b + h * p.qs.h + (int64_t)row[blk] * p.qs.s + g * 8;
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) qreg[blk][kk] = as_bf16x8(ldg16(qp + kk * 16, row_ok[blk]));
-    }
-
-    const char* kbase = reinterpret_cast<const char*>(p.k + b * p.ks.b + hk * p.ks.h);
-    const char* vbase = reinterpret_cast<const char*>(p.v + b * p.vs.b + hk * p.vs.h);
-    const uint32_t krow_b = (uint32_t)p.ks.s * 2u, vrow_b = (uint32_t)p.vs.s * 2u;   // bytes per key row
-
-    // global -> LDS: wave w moves the 1 KiB chunks w, w+4, w+8, w+12 (4 rows each)
-    // of the K tile and of the V tile; lane i fills position i & 15 of row i >> 4.
-    const int wave_u = wave;
-    const int ld_r = lane >> 4;
-    const uint32_t ld_c = (uint32_t)((lane & 15) ^ ((ld_r << 2) | wave_u)) * 16u;   // chunk this lane fetches
-    const uint32_t lds0 = (uint32_t)(uintptr_t)&kv_lds[0][0][0];
-    auto issue = [&](int kv0, int buf) {
-        const char* kb = kbase + (int64_t)kv0 * krow_b;
-        const char* vb = vbase + (int64_t)kv0 * vrow_b;
-        const uint32_t slot = lds0 + (uint32_t)buf * (2 * TILE_BYTES) + (uint32_t)wave_u * 1024u;
-        const int last = kv_hi - 1 - kv0;          // rows past `last` repeat it
-        int lr = ld_r + 4 * wave_u;                // (a fresh copy: see the tile loop)
-        asm volatile("" : "+v"(lr));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t r = (uint32_t)min(lr + 16 * j, last);
-            dma16(kb, r * krow_b + ld_c, slot + j * 4096);
-            dma16(vb, r * vrow_b + ld_c, slot + TILE_BYTES + j * 4096);
+        for (int off = 32; off >= 1; off >>= 1) {
+            lo = min(lo, __shfl_xor(lo, off));
+            hi = max(hi, __shfl_xor(hi, off));
+            in_lo = max(in_lo, __shfl_xor(in_lo, off));
+            in_hi = min(in_hi, __shfl_xor(in_hi, off));
         }
-    };
-
-    // LDS -> operands.  K rows (A of S^T): 16 bytes at row * 256 + ((2 kk + g) ^ f(row)) * 16.
-    const int f_row = ((l32 & 3) << 2) | ((l32 >> 2) & 3);
-    const uint32_t k_rd = (uint32_t)(l32 * 256), k_h = (uint32_t)((g ^ f_row) << 4);
-    // V^T (A of O^T += V^T P^T), keys in accumulator order: first half rows 16 j + 4 g + r,
-    // second half 8 rows further down, whose f differs in bit 1.
-    uint32_t v_rd[4][2];
-    {
-        const int r = (lane & 15) >> 2, t = lane & 3, u = (lane >> 4) & 1;
-        const int low = (2 * u + (t >> 1)) ^ g;
+        if (lane == 0) { red[wave][0] = lo; red[wave][1] = hi; red[wave][2] = in_lo; red[wave][3] = in_hi; }
+        __syncthreads();
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-            v_rd[dt][0] = (uint32_t)((4 * g + r) * 256 + (4 * (dt ^ r) + low) * 16 + (t & 1) * 8);
-            v_rd[dt][1] = (uint32_t)((4 * g + r + 8) * 256 + (4 * (dt ^ r) + (low ^ 2)) * 16 + (t & 1) * 8);
+        for (int w = 0; w < 4; ++w) {
+            lo = min(lo, red[w][0]);
+            hi = max(hi, red[w][1]);
+            in_lo = max(in_lo, red[w][2]);
+            in_hi = min(in_hi, red[w][3]);
         }
+        lo = uniform32(lo); hi = uniform32(hi); in_lo = uniform32(in_lo); in_hi = uniform32(in_hi);
     }
 
-    // The same addresses as absolute LDS byte addresses for buffer 0.  The swizzles only touch address
-    // bits that nothing else sets, so the address of k-step kk (K) or d tile dt (V) is the first one
-    // with kk * 32 or dt * 64 XORed in: three registers serve the plain tile code and the
-    // hand-scheduled loop (which wants all sixteen spelled out) alike.
-    const uint32_t kaddr0 = lds0 + k_rd + k_h;
-    const uint32_t vaddr0 = lds0 + TILE_BYTES + v_rd[0][0], vaddr1 = lds0 + TILE_BYTES + v_rd[0][1];
-    const char* const lds_base = &kv_lds[0][0][0] - lds0;     // LDS byte address -> pointer
+    const int tile0 = hi > lo ? lo / BN : 0;
+    const int n = uniform32(hi > lo ? (hi + BN - 1) / BN - tile0 : 0);     // key tiles of the work-group
+    f32x16 acc[2][NDT];
+    float m_i[2] = {-INFINITY, -INFINITY}, l_i[2] = {0.f, 0.f};
+    if (n > 0) {
+        const int kv0 = tile0 * BN;
+        const uint32_t krow_b = (uint32_t)p.ks.s * 2u, vrow_b = (uint32_t)p.vs.s * 2u;   // bytes per key row
+        const char* kp = uniform_ptr(reinterpret_cast<const char*>(p.k + b * p.ks.b + hk * p.ks.h) + (int64_t)kv0 * krow_b);
+        const char* vp = uniform_ptr(reinterpret_cast<const char*>(p.v + b * p.vs.b + hk * p.vs.h) + (int64_t)kv0 * vrow_b);
+        const uint32_t lds0 = (uint32_t)(uintptr_t)&kv_lds[0];
+        const uint32_t lds_w = lds0 + (uint32_t)wave * 1024u;
 
-    f32x16 acc[NBLK][4];
-    float m_i[NBLK], l_i[NBLK];
+        // global -> LDS: wave w fills the 1 KiB pieces w, w + 4, .. of a tile; lane i of a load fills
+        // position i % CPR of row i / CPR of its piece.  Loads past the last key repeat its row
+        // (those keys are masked out of S).
+        const int ld_r = RPL * wave + lane / CPR;
+        const uint32_t ld_c = (uint32_t)((lane % CPR) ^ (DH == 128 ? (((lane >> 4) << 2) | wave)
+                                                                   : ((((lane >> 4) & 1) << 2) | ((2 * wave + (lane >> 5)) & 3)))) * 16u;
+        const int last = hi - 1 - (kv0 + (n - 1) * BN);      // last row of the key range in the last tile
+        auto piece_off = [&](int t, int j, uint32_t rowb) {
+            const int r = ld_r + 4 * RPL * j;
+            return (uint32_t)(t == n - 1 ? min(r, last) : r) * rowb + ld_c;
+        };
+        const int tk1 = min(1, n - 1), tk2 = min(2, n - 1);
 #pragma unroll
-    for (int blk = 0; blk < NBLK; ++blk) {
+        for (int j = 0; j < NLD; ++j) dma16(kp, piece_off(0, j, krow_b), lds_w + j * 4096);
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int j = 0; j < NLD; ++j) dma16(vp, piece_off(0, j, vrow_b), lds_w + TB + j * 4096);
+        kp += (int64_t)tk1 * BN * krow_b;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[blk][dt][v] = 0.f;
-        m_i[blk] = -INFINITY;
-        l_i[blk] = 0.f;
-    }
-    const float c = p.scale_log2e;
-    const float cc = BIAS ? 1.f : c;              // factor from the carried scores to log2 units
-    const float* brow = nullptr;                  // this lane's row of the bias
-    if (BIAS) brow = p.bias + b * p.bias_b + h * p.bias_h + (int64_t)min(row[0], p.row_end - 1) * p.bias_r;
+        for (int j = 0; j < NLD; ++j) dma16(kp, piece_off(tk1, j, krow_b), lds_w + 2 * TB + j * 4096);
+        kp += (int64_t)(tk2 - tk1) * BN * krow_b;
+        vp += (int64_t)tk1 * BN * vrow_b;
+        uint32_t dok[NLD], dov[NLD];
+#pragma unroll
+        for (int j = 0; j < NLD; ++j) { dok[j] = piece_off(tk2, j, krow_b); dov[j] = piece_off(tk1, j, vrow_b); }
 
-    const int t_begin = (hi > lo) ? lo / BN : 0;
-    const int t_end = (hi > lo) ? (hi + BN - 1) / BN : 0;
-
-    // the run [ta, ta + n_fast) of full tiles no row masks: an odd number of at least three
-    int ta = t_begin, n_fast = 0;
-    if (krow_b == vrow_b) {
-        const int fa = max(t_begin, (in_lo + BN - 1) / BN);
-        const int fb = min(t_end, min(in_hi, kv_hi) / BN);
-        if (fb - fa >= 3) { ta = fa; n_fast = (fb - fa - 1) | 1; }
-    }
-
-    for (int phase = 0; phase < 3; ++phase) {
-        if (phase == 1) {
-            if (n_fast == 0) continue;
-            int trips = n_fast >> 1;
-            const char* kp = kbase + (int64_t)(ta * BN) * krow_b;
-            const char* vp = vbase + (int64_t)(ta * BN) * vrow_b;
-            uint32_t doff[4], kaddr[8], vaddr[8];
+        // Q^T as B operand; its loads travel with the first tiles'
+        bf16x8 q[2][NKK];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) doff[j] = (uint32_t)(4 * (wave_u + 4 * j) + ld_r) * krow_b + ld_c;
+        for (int blk = 0; blk < 2; ++blk) {
+            const int row = row0 + 32 * blk + l32;
+            const uint16_t* qp = p.q + b * p.qs.b + h * p.qs.h + (int64_t)row * p.qs.s + g * 8;
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) kaddr[kk] = kaddr0 ^ (uint32_t)(kk * 32);
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
-                vaddr[2 * dt] = vaddr0 ^ (uint32_t)(dt * 64);
-                vaddr[2 * dt + 1] = vaddr1 ^ (uint32_t)(dt * 64);
-            }
-            const uint32_t lds_w = lds0 + (uint32_t)wave_u * 1024u;
-            if constexpr (NBLK == 1) {
-                asm volatile(
-#include "lvx_fwd_loop_bf16.inc"
-                    : "+{v[0:15]}"(acc[0][0]), "+{v[16:31]}"(acc[0][1]), "+{v[32:47]}"(acc[0][2]), "+{v[48:63]}"(acc[0][3]),
-                      "+{v244}"(m_i[0]), "+{v245}"(l_i[0]), "+{s[44:45]}"(kp), "+{s[46:47]}"(vp), "+{s51}"(trips)
-                    : "{v[64:67]}"(qreg[0][0]), "{v[68:71]}"(qreg[0][1]), "{v[72:75]}"(qreg[0][2]), "{v[76:79]}"(qreg[0][3]),
-                      "{v[80:83]}"(qreg[0][4]), "{v[84:87]}"(qreg[0][5]), "{v[88:91]}"(qreg[0][6]), "{v[92:95]}"(qreg[0][7]),
-                      "{v224}"(kaddr[0]), "{v225}"(kaddr[1]), "{v226}"(kaddr[2]), "{v227}"(kaddr[3]),
-                      "{v228}"(kaddr[4]), "{v229}"(kaddr[5]), "{v230}"(kaddr[6]), "{v231}"(kaddr[7]),
-                      "{v232}"(vaddr[0]), "{v233}"(vaddr[1]), "{v234}"(vaddr[2]), "{v235}"(vaddr[3]),
-                      "{v236}"(vaddr[4]), "{v237}"(vaddr[5]), "{v238}"(vaddr[6]), "{v239}"(vaddr[7]),
-                      "{v240}"(doff[0]), "{v241}"(doff[1]), "{v242}"(doff[2]), "{v243}"(doff[3]),
-                      "{s40}"(cc), "{s41}"(-INFINITY), "{s42}"(RESCALE_LOG2), "{s48}"((uint32_t)BN * krow_b),
-                      "{s49}"((uint32_t)BN * vrow_b), "{s50}"(lds_w)
-                    : "memory", "vcc", "scc", "m0", "s52", "s53", "s54", "s55", "s56", LVX_FWD_LOOP_CLOBBERS);
-            } else {
-                // O^T and Q^T travel in VGPRs; the statement parks them in accumulation registers while it
-                // runs and hands them back in the registers they came in
-                asm volatile(
-#include "lvx_fwd_loop_wide.inc"
-                    : "+{v[0:15]}"(acc[0][0]), "+{v[16:31]}"(acc[0][1]), "+{v[32:47]}"(acc[0][2]), "+{v[48:63]}"(acc[0][3]),
-                      "+{v[64:79]}"(acc[NBLK - 1][0]), "+{v[80:95]}"(acc[NBLK - 1][1]), "+{v[96:111]}"(acc[NBLK - 1][2]),
-                      "+{v[112:127]}"(acc[NBLK - 1][3]),
-                      "+{v[128:131]}"(qreg[0][0]), "+{v[132:135]}"(qreg[0][1]), "+{v[136:139]}"(qreg[0][2]), "+{v[140:143]}"(qreg[0][3]),
-                      "+{v[144:147]}"(qreg[0][4]), "+{v[148:151]}"(qreg[0][5]), "+{v[152:155]}"(qreg[0][6]), "+{v[156:159]}"(qreg[0][7]),
-                      "+{v[160:163]}"(qreg[NBLK - 1][0]), "+{v[164:167]}"(qreg[NBLK - 1][1]), "+{v[168:171]}"(qreg[NBLK - 1][2]),
-                      "+{v[172:175]}"(qreg[NBLK - 1][3]), "+{v[176:179]}"(qreg[NBLK - 1][4]), "+{v[180:183]}"(qreg[NBLK - 1][5]),
-                      "+{v[184:187]}"(qreg[NBLK - 1][6]), "+{v[188:191]}"(qreg[NBLK - 1][7]),
-                      "+{v220}"(m_i[0]), "+{v221}"(m_i[NBLK - 1]), "+{v222}"(l_i[0]), "+{v223}"(l_i[NBLK - 1]),
-                      "+{s[44:45]}"(kp), "+{s[46:47]}"(vp), "+{s51}"(trips)
-                    : "{v200}"(kaddr[0]), "{v201}"(kaddr[1]), "{v202}"(kaddr[2]), "{v203}"(kaddr[3]),
-                      "{v204}"(kaddr[4]), "{v205}"(kaddr[5]), "{v206}"(kaddr[6]), "{v207}"(kaddr[7]),
-                      "{v208}"(vaddr[0]), "{v209}"(vaddr[1]), "{v210}"(vaddr[2]), "{v211}"(vaddr[3]),
-                      "{v212}"(vaddr[4]), "{v213}"(vaddr[5]), "{v214}"(vaddr[6]), "{v215}"(vaddr[7]),
-                      "{v216}"(doff[0]), "{v217}"(doff[1]), "{v218}"(doff[2]), "{v219}"(doff[3]),
-                      "{s40}"(cc), "{s41}"(-INFINITY), "{s42}"(RESCALE_LOG2), "{s48}"((uint32_t)BN * krow_b),
-                      "{s49}"((uint32_t)BN * vrow_b), "{s50}"(lds_w)
-                    : "memory", "vcc", "scc", "m0", "s52", "s53", "s54", "s55", "s56", "s58", "s59", "s60", "s61",
-                      LVX_FWD_WIDE_CLOBBERS);
-            }
-            continue;
+            for (int kk = 0; kk < NKK; ++kk) q[blk][kk] = as_bf16x8(ldg16(qp + kk * 16, row < p.row_end));
         }
-        const int t0 = phase == 0 ? t_begin : ta + n_fast;
-        const int t1 = phase == 0 ? ta : t_end;
-        if (t1 <= t0) continue;
-        __syncthreads();     // the tile buffers are free: every wave is done with the previous phase
-        issue(t0 * BN, 0);
-        for (int t = t0; t < t1; ++t) {
-            const int kv0 = t * BN;
-            const int buf = (t - t0) & 1;
-            // fresh copies the compiler cannot hoist: the sixteen derived addresses are then formed
-            // tile by tile (an XOR each) instead of being kept - and spilled - across the whole loop
-            uint32_t ka0 = kaddr0, va0 = vaddr0, va1 = vaddr1;
-            asm volatile("" : "+v"(ka0), "+v"(va0), "+v"(va1));
 
-            // tile t has landed (this wave's part: vmcnt; everyone's: barrier); the
-            // barrier also says every wave is done reading tile t-1, whose buffer
-            // the loads of tile t+1 may now overwrite
-            wait_vmcnt<0>();
-            __syncthreads();
-            if (t + 1 < t1) issue(kv0 + BN, buf ^ 1);
-
-            // S^T = K Q^T : rows = keys (two 32-key sub-tiles), cols = text rows.
-            // All 16 K operands are requested before the first MFMA, so the LDS
-            // latency is paid once per tile and not once per k-step.
-            bf16x8 ka[8][2];
-    #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) {
-                const char* kp = lds_base + (ka0 ^ (uint32_t)(kk * 32)) + buf * (2 * TILE_BYTES);
-                ka[kk][0] = *reinterpret_cast<const bf16x8*>(kp);
-                ka[kk][1] = *reinterpret_cast<const bf16x8*>(kp + 32 * 256);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            f32x16 s0[NBLK], s1[NBLK];
-    #pragma unroll
-            for (int blk = 0; blk < NBLK; ++blk) {
-    #pragma unroll
-                for (int v = 0; v < 16; ++v) { s0[blk][v] = 0.f; s1[blk][v] = 0.f; }
-    #pragma unroll
-                for (int kk = 0; kk < 8; ++kk) {
-                    s0[blk] = E::mfma(ka[kk][0], qreg[blk][kk], s0[blk]);
-                    s1[blk] = E::mfma(ka[kk][1], qreg[blk][kk], s1[blk]);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            // V^T operands of this tile: requested now, they land during the softmax
-            u32x2 va[4][4][2];
-    #pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
-    #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    va[dt][j][0] = lds_read_tr16(reinterpret_cast<const uint16_t*>(lds_base + (va0 ^ (uint32_t)(dt * 64)) + buf * (2 * TILE_BYTES) + j * 4096));
-                    va[dt][j][1] = lds_read_tr16(reinterpret_cast<const uint16_t*>(lds_base + (va1 ^ (uint32_t)(dt * 64)) + buf * (2 * TILE_BYTES) + j * 4096));
-                }
-            __builtin_amdgcn_sched_barrier(0);
-
-    #pragma unroll
-            for (int blk = 0; blk < NBLK; ++blk) {
-                if (kv0 < in_lo || kv0 + BN > in_hi) {
-    #pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int kv = kv0 + acc_row(v, g);
-                        if (kv < my_s[blk] || kv >= my_e[blk]) s0[blk][v] = -INFINITY;
-                        if (kv + 32 < my_s[blk] || kv + 32 >= my_e[blk]) s1[blk][v] = -INFINITY;
-                    }
-                }
-
-                float mx = max3(s0[blk][0], s1[blk][0], s0[blk][1]);
-                mx = max3(mx, s1[blk][1], s0[blk][2]);
-    #pragma unroll
-                for (int v = 3; v < 16; v += 1) mx = max3(mx, s1[blk][v - 1], s0[blk][v]);
-                mx = fmaxf(mx, s1[blk][15]);
-                {   // other half of the wave holds the other 32 keys of the same text row
-                    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-                    mx = max3(__uint_as_float(sw[0]), __uint_as_float(sw[1]), m_i[blk]);
-                }
-                // Lazy rescale: the reference point m_i of a row only moves when the row
-                // maximum has grown by more than 2^RESCALE_LOG2 since it was set, so P may
-                // reach 2^RESCALE_LOG2 instead of 1 (harmless in fp32 / bf16) and the
-                // rescale of O happens a few times per row instead of almost every tile.
-                const float mcand = mx * cc;                      // mx >= m_i
-                const float m_ic = m_i[blk] * cc;
-                const bool move = (mx != -INFINITY) && !(mcand - m_ic <= RESCALE_LOG2);
-                const float alpha = move ? __builtin_amdgcn_exp2f(m_ic - mcand) : 1.f;
-                if (move) m_i[blk] = mx;
-                const float mc = (m_i[blk] == -INFINITY) ? 0.f : m_i[blk] * cc;
-
-                // P^T as B operand: k-step j covers keys 16j..16j+15 of the tile.  The row
-                // sum is taken in fp32 before the rounding to bf16 (summing the rounded
-                // values would put the LSE off by up to a bf16 ulp of the largest term).
-                bf16x8 pb[4];
-                float rs0 = 0.f, rs1 = 0.f;
-    #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    u32x4 u0, u1;
-    #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int v = 8 * j + 2 * e;
-                        const float a0 = __builtin_amdgcn_exp2f(fmaf(s0[blk][v], cc, -mc)), a1 = __builtin_amdgcn_exp2f(fmaf(s0[blk][v + 1], cc, -mc));
-                        const float b0 = __builtin_amdgcn_exp2f(fmaf(s1[blk][v], cc, -mc)), b1 = __builtin_amdgcn_exp2f(fmaf(s1[blk][v + 1], cc, -mc));
-                        rs0 += a0 + a1;
-                        rs1 += b0 + b1;
-                        u0[e] = E::pack(a0, a1);
-                        u1[e] = E::pack(b0, b1);
-                    }
-                    pb[j] = as_bf16x8(u0);
-                    pb[2 + j] = as_bf16x8(u1);
-                }
-                l_i[blk] = l_i[blk] * alpha + (rs0 + rs1);
-
-                if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {   // the running max moved for some row
-    #pragma unroll
-                    for (int dt = 0; dt < 4; ++dt)
-    #pragma unroll
-                        for (int v = 0; v < 16; ++v) acc[blk][dt][v] *= alpha;
-                }
-
-                // O^T += V^T P^T
-                __builtin_amdgcn_sched_barrier(0);
-    #pragma unroll
-                for (int dt = 0; dt < 4; ++dt)
-    #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const u32x4 a = {va[dt][j][0][0], va[dt][j][0][1], va[dt][j][1][0], va[dt][j][1][1]};
-                        acc[blk][dt] = E::mfma(as_bf16x8(a), pb[j], acc[blk][dt]);
-                    }
-            }
+        // LDS -> operands.  K rows (A of S^T): chunk 2 kk + g of row l32 (+ 32).  V^T (A of O^T += V^T P^T),
+        // keys in accumulator order: first half rows 16 j + 4 g + r, second half 8 rows further down.
+        // The swizzle only touches address bits nothing else sets, so k-step kk (d tile dt) is the first
+        // address with kk * 32 (dt * 64) XORed in.
+        const int f_row = DH == 128 ? (((l32 & 3) << 2) | ((l32 >> 2) & 3)) : ((((l32 >> 1) & 1) << 2) | ((l32 >> 2) & 3));
+        const uint32_t kaddr0 = lds0 + (uint32_t)(l32 * ROWB) + (uint32_t)((g ^ f_row) << 4);
+        uint32_t ka[NKK], va[2 * NDT];
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) ka[kk] = kaddr0 ^ (uint32_t)(kk * 32);
+        {
+            const int r = (lane & 15) >> 2, t = lane & 3, u = (lane >> 4) & 1;
+            const int up = DH == 128 ? r : r >> 1;           // the row bits that move a chunk by 64 bytes or more
+            const int low = (2 * u + (t >> 1)) ^ g;
+            const uint32_t v0 = lds0 + TB + (uint32_t)((4 * g + r) * ROWB + ((4 * up) ^ low) * 16 + (t & 1) * 8);
+            const uint32_t v1 = lds0 + TB + (uint32_t)((4 * g + r + 8) * ROWB + ((4 * up) ^ (low ^ 2)) * 16 + (t & 1) * 8);
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) { va[2 * dt] = v0 ^ (uint32_t)(dt * 64); va[2 * dt + 1] = v1 ^ (uint32_t)(dt * 64); }
         }
+        const uint32_t me0 = (uint32_t)(my_s[0] - 4 * g), me1 = (uint32_t)(my_s[1] - 4 * g);
+        const uint32_t ml0 = (uint32_t)(my_e[0] - my_s[0]), ml1 = (uint32_t)(my_e[1] - my_s[1]);
+        // a tile at key kv needs no mask when kv - inner <= inner_n as unsigned numbers
+        const bool inner_any = in_hi - in_lo >= BN;
+        const int inner = inner_any ? in_lo : BIG;
+        const uint32_t inner_n = inner_any ? (uint32_t)(in_hi - BN - in_lo) : 0u;
+        uint32_t left = uniform32((uint32_t)(n - 1)), left_k = uniform32((uint32_t)(n - 1 - tk2));
+        uint32_t left_v = uniform32((uint32_t)(n - 1 - tk1)), kv = uniform32((uint32_t)kv0);
+        kp = uniform_ptr(kp);
+        vp = uniform_ptr(vp);
+#define LVX_FWD_WIDE_SCALARS                                                                                       \
+    "{s40}"(uniform32(p.scale_log2e)), "{s41}"(-INFINITY), "{s42}"(RESCALE_LOG2), "{s48}"(uniform32((uint32_t)BN * krow_b)), \
+        "{s49}"(uniform32((uint32_t)BN * vrow_b)), "{s50}"(uniform32(lds_w)), "{s64}"(uniform32((uint32_t)last * krow_b)),   \
+        "{s65}"(uniform32((uint32_t)last * vrow_b)), "{s67}"(uniform32(inner)), "{s68}"(uniform32(inner_n)),               \
+        "{v224}"(ld_c), "{v225}"(me0), "{v226}"(me1), "{v227}"(ml0), "{v228}"(ml1)
+#define LVX_FWD_WIDE_STATE                                                                                         \
+    "=&{v229}"(m_i[0]), "=&{v230}"(m_i[1]), "=&{v231}"(l_i[0]), "=&{v232}"(l_i[1]), "+{s[44:45]}"(kp), "+{s[46:47]}"(vp), \
+        "+{s51}"(left), "+{s57}"(left_k), "+{s62}"(left_v), "+{s66}"(kv)
+#define LVX_FWD_WIDE_OUT_128                                                                                       \
+          "=&{v[0:15]}"(acc[0][0]), "=&{v[16:31]}"(acc[0][1]), "=&{v[32:47]}"(acc[0][2]), "=&{v[48:63]}"(acc[0][3]),   \
+          "=&{v[64:79]}"(acc[1][0]), "=&{v[80:95]}"(acc[1][1]), "=&{v[96:111]}"(acc[1][2]), "=&{v[112:127]}"(acc[1][3]), \
+          "+{v[128:131]}"(q[0][0]), "+{v[132:135]}"(q[0][1]), "+{v[136:139]}"(q[0][2]), "+{v[140:143]}"(q[0][3]),      \
+          "+{v[144:147]}"(q[0][4]), "+{v[148:151]}"(q[0][5]), "+{v[152:155]}"(q[0][6]), "+{v[156:159]}"(q[0][7]),      \
+          "+{v[160:163]}"(q[1][0]), "+{v[164:167]}"(q[1][1]), "+{v[168:171]}"(q[1][2]), "+{v[172:175]}"(q[1][3]),      \
+          "+{v[176:179]}"(q[1][4]), "+{v[180:183]}"(q[1][5]), "+{v[184:187]}"(q[1][6]), "+{v[188:191]}"(q[1][7]),      \
+          "+{v216}"(dok[0]), "+{v217}"(dok[1]), "+{v218}"(dok[2]), "+{v219}"(dok[3]),                              \
+          "+{v220}"(dov[0]), "+{v221}"(dov[1]), "+{v222}"(dov[2]), "+{v223}"(dov[3]), LVX_FWD_WIDE_STATE
+#define LVX_FWD_WIDE_IN_128                                                                                        \
+          "{v200}"(ka[0]), "{v201}"(ka[1]), "{v202}"(ka[2]), "{v203}"(ka[3]), "{v204}"(ka[4]), "{v205}"(ka[5]),    \
+          "{v206}"(ka[6]), "{v207}"(ka[7]), "{v208}"(va[0]), "{v209}"(va[1]), "{v210}"(va[2]), "{v211}"(va[3]),    \
+          "{v212}"(va[4]), "{v213}"(va[5]), "{v214}"(va[6]), "{v215}"(va[7]), LVX_FWD_WIDE_SCALARS
+#define LVX_FWD_WIDE_OUT_64                                                                                        \
+          "=&{v[0:15]}"(acc[0][0]), "=&{v[16:31]}"(acc[0][1]), "=&{v[64:79]}"(acc[1][0]), "=&{v[80:95]}"(acc[1][1]),   \
+          "+{v[128:131]}"(q[0][0]), "+{v[132:135]}"(q[0][1]), "+{v[136:139]}"(q[0][2]), "+{v[140:143]}"(q[0][3]),      \
+          "+{v[160:163]}"(q[1][0]), "+{v[164:167]}"(q[1][1]), "+{v[168:171]}"(q[1][2]), "+{v[172:175]}"(q[1][3]),      \
+          "+{v216}"(dok[0]), "+{v217}"(dok[1]), "+{v220}"(dov[0]), "+{v221}"(dov[1]), LVX_FWD_WIDE_STATE
+#define LVX_FWD_WIDE_IN_64                                                                                         \
+          "{v200}"(ka[0]), "{v201}"(ka[1]), "{v202}"(ka[2]), "{v203}"(ka[3]),                                      \
+          "{v208}"(va[0]), "{v209}"(va[1]), "{v210}"(va[2]), "{v211}"(va[3]), LVX_FWD_WIDE_SCALARS
+        if constexpr (DH == 128 && !F16) {
+            asm volatile(
+#include "lvx_fwd_loop_wide_bf16_128.inc"
+                : LVX_FWD_WIDE_OUT_128 : LVX_FWD_WIDE_IN_128 : LVX_FWD_WIDE_CLOBBERS_S, LVX_FWD_WIDE_CLOBBERS_128);
+        } else if constexpr (DH == 128) {
+            asm volatile(
+#include "lvx_fwd_loop_wide_f16_128.inc"
+                : LVX_FWD_WIDE_OUT_128 : LVX_FWD_WIDE_IN_128 : LVX_FWD_WIDE_CLOBBERS_S, LVX_FWD_WIDE_CLOBBERS_128);
+        } else if constexpr (!F16) {
+            asm volatile(
+#include "lvx_fwd_loop_wide_bf16_64.inc"
+                : LVX_FWD_WIDE_OUT_64 : LVX_FWD_WIDE_IN_64 : LVX_FWD_WIDE_CLOBBERS_S, LVX_FWD_WIDE_CLOBBERS_64);
+        } else {
+            asm volatile(
+#include "lvx_fwd_loop_wide_f16_64.inc"
+                : LVX_FWD_WIDE_OUT_64 : LVX_FWD_WIDE_IN_64 : LVX_FWD_WIDE_CLOBBERS_S, LVX_FWD_WIDE_CLOBBERS_64);
+        }
+    } else {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[blk][dt][v] = 0.f;
     }
 
-    // epilogue: the two lane halves hold partial row sums of the same row
+    // Epilogue.  A lane holds 4 consecutive values of d of one row per register group; the rows of a
+    // wave go through its quarter of the tile buffers and leave as whole rows, 16 bytes per lane.
+    // Chunk c of row r sits at position c ^ (r mod chunks per row) (DH = 64: c ^ (r / 2 mod 8)), its
+    // 8-byte halves exchanged in rows with bit 4 set: conflict-free both ways.
+    __syncthreads();     // every wave is done with the tiles
+    char* const ep = kv_lds + wave * TB;
 #pragma unroll
-    for (int blk = 0; blk < NBLK; ++blk) {
-        const float l_tot = l_i[blk] + __shfl_xor(l_i[blk], 32);
+    for (int blk = 0; blk < 2; ++blk) {
+        float l_tot = l_i[blk] + __shfl_xor(l_i[blk], 32);     // the two lane halves hold partial sums of the same row
+        if (empty[blk]) l_tot = 0.f;
         const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-        if (row_ok[blk]) {
-            uint16_t* op = p.o + split * p.o_split_stride + b * p.os.b + h * p.os.h + (int64_t)row[blk] * p.os.s;
+        const int r = 32 * blk + l32, pos = DH == 128 ? (r & 15) : ((r >> 1) & 7);
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-                for (int vg = 0; vg < 4; ++vg) {
-                    u32x2 w;
-                    w[0] = E::pack(acc[blk][dt][4 * vg] * inv, acc[blk][dt][4 * vg + 1] * inv);
-                    w[1] = E::pack(acc[blk][dt][4 * vg + 2] * inv, acc[blk][dt][4 * vg + 3] * inv);
-                    *reinterpret_cast<u32x2*>(op + dt * 32 + 8 * vg + 4 * g) = w;
-                }
-            if (g == 0) {
-                const float lse = l_tot > 0.f ? m_i[blk] * (BIAS ? LN2_F : p.scale) + __logf(l_tot) : -INFINITY;
-                p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + h) * p.lse_bh_stride + row[blk]] = lse;
+            for (int vg = 0; vg < 4; ++vg) {
+                u32x2 w;
+                w[0] = E::pack(acc[blk][dt][4 * vg] * inv, acc[blk][dt][4 * vg + 1] * inv);
+                w[1] = E::pack(acc[blk][dt][4 * vg + 2] * inv, acc[blk][dt][4 * vg + 3] * inv);
+                *reinterpret_cast<u32x2*>(ep + r * ROWB + (((4 * dt + vg) ^ pos) << 4) + ((g ^ ((r >> 4) & 1)) << 3)) = w;
             }
+        if (g == 0 && row0 + r < p.row_end) {
+            const float lse = l_tot > 0.f ? m_i[blk] * p.scale + __logf(l_tot) : -INFINITY;
+            p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + h) * p.lse_bh_stride + row0 + r] = lse;
         }
+    }
+    wait_lds();          // this wave's rows are its own
+    uint16_t* const ob = p.o + split * p.o_split_stride + b * p.os.b + h * p.os.h;
+#pragma unroll
+    for (int i = 0; i < CPR; ++i) {
+        const int r = i * RPL + lane / CPR, c = lane % CPR, pos = DH == 128 ? (r & 15) : ((r >> 1) & 7);
+        u32x4 val = *reinterpret_cast<const u32x4*>(ep + r * ROWB + ((c ^ pos) << 4));
+        if ((r >> 4) & 1) val = u32x4{val[2], val[3], val[0], val[1]};
+        if (row0 + r < p.row_end) *reinterpret_cast<u32x4*>(ob + (int64_t)(row0 + r) * p.os.s + c * 8) = val;
     }
 }
 
@@ -732,14 +606,15 @@ namespace {
 template <int DH, bool F16>
 hipError_t launch_fwd_t(const FwdParams& p, bool masked, hipStream_t st) {
     const int grid = ((p.total_wg + 7) / 8) * 8;
+    if constexpr (DH >= 64) {
+        if (p.form == FWD_WIDE) {
+            if (masked) return launch1((fwd_wide_kernel<DH, true, F16>), dim3(grid), dim3(256), st, p);
+            return launch1((fwd_wide_kernel<DH, false, F16>), dim3(grid), dim3(256), st, p);
+        }
+    }
     if (p.bias) {
         if (masked) return launch1((fwd_kernel<DH, true, true, F16>), dim3(grid), dim3(256), st, p);
         else return launch1((fwd_kernel<DH, false, true, F16>), dim3(grid), dim3(256), st, p);
-    } else if (DH == 128 && !F16 && !masked) {
-        // (with an interval mask the plain kernel is the faster one: the edges of the rows' intervals leave
-        // the hand-scheduled loop short runs, and its register needs cost the tile code around it)
-        if (p.wide) return launch1((fwd_kernel_pipe<2>), dim3(grid), dim3(256), st, p);
-        return launch1((fwd_kernel_pipe<1>), dim3(grid), dim3(256), st, p);
     } else {
         if (masked) return launch1((fwd_kernel<DH, true, false, F16>), dim3(grid), dim3(256), st, p);
         else return launch1((fwd_kernel<DH, false, false, F16>), dim3(grid), dim3(256), st, p);

@@ -19,6 +19,10 @@ struct Strides3 {
     int64_t b, h, s;
 };
 
+// Which forward kernel: a wave owns 32 rows of a head (any head dimension, dense bias), 64 rows and its
+// SIMD (head dimensions 128 and 64).
+enum FwdForm { FWD_PLAIN = 0, FWD_WIDE = 1 };
+
 struct FwdParams {
     const uint16_t* q;
     const uint16_t* k;
@@ -39,7 +43,7 @@ struct FwdParams {
     int G;                     // q heads per kv head
     int HG;                    // q heads a work-group covers (one per wave)
     int RS;                    // row sub-tiles a work-group covers per head
-    int wide;                  // 1: a wave owns 64 rows (two blocks of 32) instead of 32; bf16 without bias only
+    int form;                  // FwdForm
     int row_begin, row_end;
     int n_row_tiles, n_head_groups, nsplit, split_len, total_wg;
     float scale, scale_log2e;

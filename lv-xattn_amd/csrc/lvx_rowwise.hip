@@ -8,12 +8,11 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 namespace lvx {
 
 namespace {
-
-constexpr int MAX_PARTS = 16;
 
 // log2 of the 16-byte chunks (lanes) per row
 __device__ __forceinline__ int chunk_shift(int head_dim) {
@@ -29,77 +28,95 @@ __device__ __forceinline__ void unpack8(u32x4 u, float f[8]) {
     }
 }
 
-// (o_acc, l_acc) <- merge(acc?, part_0 .. part_{n-1}) for every (b, h, row).
-template <bool F16>
+// (o_acc, l_acc) <- merge(acc?, part_0 .. part_{n-1}) for every (b, h, row).  PL lanes share the parts
+// of a 16-byte column of a row: with few rows (a token being generated, cut into dozens of key
+// ranges) the launch is as long as a thread's chain of loads, so the parts of a row go side by side
+// and each thread has the loads of four parts in flight, O beside the LSE it will be weighted by.
+template <bool F16, int PL>
 __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     using E = Elt<F16>;
+    constexpr int PSH = PL == 4 ? 2 : PL == 2 ? 1 : 0, BATCH = 4;
     const int nrows = p.row_end - p.row_begin;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int sh = chunk_shift(p.D);
     const int chunk = (int)(idx & ((1 << sh) - 1));
-    const int64_t r = idx >> sh;
-    if (r >= (int64_t)p.B * p.Hq * nrows) return;
+    const int pl = (int)(idx >> sh) & (PL - 1);
+    const int64_t r = idx >> (sh + PSH);
+    if (r >= (int64_t)p.B * p.Hq * nrows) return;      // the lanes of a row leave together
     const int row = p.row_begin + (int)(r % nrows);
     const int bh = (int)(r / nrows);
     const int b = bh / p.Hq, h = bh % p.Hq;
 
-    float la = -INFINITY;
-    if (p.use_acc) la = p.l_in ? p.l_in[(int64_t)bh * p.l_in_bh + row] : p.l_acc[(int64_t)bh * p.l_acc_bh + row];
-    float lp[MAX_PARTS];
-    float m = la;
-#pragma unroll
-    for (int i = 0; i < MAX_PARTS; ++i) {
-        if (i < p.nparts) {
-            lp[i] = p.l_part[i * p.l_part_stride + (int64_t)bh * p.l_part_bh + row];
-            m = fmaxf(m, lp[i]);
-        }
-    }
-    const float ms = (m == -INFINITY) ? 0.f : m;
-    float wa = __expf(la - ms);
-    float den = wa;
-#pragma unroll
-    for (int i = 0; i < MAX_PARTS; ++i) {
-        if (i < p.nparts) {
-            lp[i] = __expf(lp[i] - ms);
-            den += lp[i];
-        }
-    }
-    const float inv = den > 0.f ? 1.f / den : 0.f;
-
-    float out[8];
+    float m = -INFINITY, den = 0.f, out[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) out[j] = 0.f;
-    uint16_t* oa = p.o_acc + b * p.oa.b + h * p.oa.h + (int64_t)row * p.oa.s + chunk * 8;
-    if (p.use_acc) {
-        float f[8];
-        const uint16_t* oin = p.o_in ? p.o_in + b * p.oi.b + h * p.oi.h + (int64_t)row * p.oi.s + chunk * 8 : oa;
-        unpack8<E>(*reinterpret_cast<const u32x4*>(oin), f);
-        const float w = wa * inv;
-        // an accumulator with weight 0 (L = -inf: nothing folded in yet) may hold anything
-        if (w > 0.f) {
+    // folds the parts (l[k], u[k]) in; a part with weight 0 may hold anything (it saw no key, or nothing
+    // had been folded into the accumulator yet)
+    auto fold = [&](const float (&l)[BATCH], const u32x4 (&u)[BATCH]) {
+        float mn = m;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) out[j] = f[j] * w;
+        for (int k = 0; k < BATCH; ++k) mn = fmaxf(mn, l[k]);
+        const float ms = (mn == -INFINITY) ? 0.f : mn;
+        const float keep = __expf(m - ms);
+        den *= keep;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) out[j] *= keep;
+#pragma unroll
+        for (int k = 0; k < BATCH; ++k) {
+            const float w = __expf(l[k] - ms);
+            den += w;
+            float f[8];
+            unpack8<E>(u[k], f);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) out[j] = w > 0.f ? fmaf(f[j], w, out[j]) : out[j];
         }
+        m = mn;
+    };
+    uint16_t* oa = p.o_acc + b * p.oa.b + h * p.oa.h + (int64_t)row * p.oa.s + chunk * 8;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    float la = -INFINITY;
+    u32x4 ua = zero;
+    if (p.use_acc && pl == 0) {
+        la = p.l_in ? p.l_in[(int64_t)bh * p.l_in_bh + row] : p.l_acc[(int64_t)bh * p.l_acc_bh + row];
+        ua = *reinterpret_cast<const u32x4*>(p.o_in ? p.o_in + b * p.oi.b + h * p.oi.h + (int64_t)row * p.oi.s + chunk * 8 : oa);
     }
     const uint16_t* op = p.o_part + b * p.op.b + h * p.op.h + (int64_t)row * p.op.s + chunk * 8;
+    const float* lp = p.l_part + (int64_t)bh * p.l_part_bh + row;
+    for (int i = pl; i < p.nparts; i += PL * BATCH) {
+        float l[BATCH];
+        u32x4 u[BATCH];
 #pragma unroll
-    for (int i = 0; i < MAX_PARTS; ++i) {
-        if (i < p.nparts) {
-            float f[8];
-            unpack8<E>(*reinterpret_cast<const u32x4*>(op + i * p.o_part_stride), f);
-            const float w = lp[i] * inv;
-            // a part with weight 0 may hold anything (it saw no key)
-            if (w > 0.f) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) out[j] = fmaf(f[j], w, out[j]);
-            }
+        for (int k = 0; k < BATCH; ++k) {
+            const int part = i + k * PL;
+            const bool ok = part < p.nparts;
+            l[k] = ok ? lp[part * p.l_part_stride] : -INFINITY;
+            u[k] = ldg16(op + part * p.o_part_stride, ok);
         }
+        fold(l, u);
     }
+    if (p.use_acc) {
+        const float l[BATCH] = {la, -INFINITY, -INFINITY, -INFINITY};
+        const u32x4 u[BATCH] = {ua, zero, zero, zero};
+        fold(l, u);
+    }
+#pragma unroll
+    for (int o = 1; o < PL; o <<= 1) {                  // the lanes that share a row's parts
+        const int d = o << sh;
+        const float m2 = __shfl_xor(m, d), den2 = __shfl_xor(den, d);
+        const float mn = fmaxf(m, m2), ms = (mn == -INFINITY) ? 0.f : mn;
+        const float w1 = __expf(m - ms), w2 = __expf(m2 - ms);
+        den = den * w1 + den2 * w2;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) out[j] = out[j] * w1 + __shfl_xor(out[j], d) * w2;
+        m = mn;
+    }
+    if (pl != 0) return;
+    const float inv = den > 0.f ? 1.f / den : 0.f;
     u32x4 u;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) u[j] = E::pack(out[2 * j], out[2 * j + 1]);
+    for (int j = 0; j < 4; ++j) u[j] = E::pack(out[2 * j] * inv, out[2 * j + 1] * inv);
     *reinterpret_cast<u32x4*>(oa) = u;
-    if (chunk == 0) p.l_acc[(int64_t)bh * p.l_acc_bh + row] = den > 0.f ? ms + __logf(den) : -INFINITY;
+    if (chunk == 0) p.l_acc[(int64_t)bh * p.l_acc_bh + row] = den > 0.f ? m + __logf(den) : -INFINITY;
 }
 
 // The same for one part folded into the accumulator (what lvx_merge does every round), two rows
@@ -472,8 +489,16 @@ hipError_t launch_merge(const MergeParams& p, hipStream_t st) {
         if (p.f16) return launch1(merge_pair_kernel<true>, grid, dim3(256), st, p);
         return launch1(merge_pair_kernel<false>, grid, dim3(256), st, p);
     }
-    if (p.f16) return launch1(merge_kernel<true>, dim3(blocks_for(rows)), dim3(256), st, p);
-    else return launch1(merge_kernel<false>, dim3(blocks_for(rows)), dim3(256), st, p);
+    // as many lanes per row as the parts need (four parts each) and the chip has room for
+    const int pl = p.nparts > 8 && rows < 16384 ? 4 : p.nparts > 4 && rows < 32768 ? 2 : 1;
+    const dim3 grid(blocks_for(rows * pl));
+    auto go = [&](auto f16) {
+        constexpr bool F16 = decltype(f16)::value;
+        if (pl == 4) return launch1(merge_kernel<F16, 4>, grid, dim3(256), st, p);
+        if (pl == 2) return launch1(merge_kernel<F16, 2>, grid, dim3(256), st, p);
+        return launch1(merge_kernel<F16, 1>, grid, dim3(256), st, p);
+    };
+    return p.f16 ? go(std::true_type{}) : go(std::false_type{});
 }
 
 hipError_t launch_preprocess(const PreParams& p, hipStream_t st) {

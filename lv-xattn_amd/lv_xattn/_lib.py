@@ -43,6 +43,7 @@ SYMBOLS = {
     "lvx_version": (C.c_int, []),
     "lvx_strerror": (C.c_char_p, [C.c_int]),
     "lvx_fwd_workspace_bytes": (C.c_size_t, [_SHAPE, C.c_int32, C.c_int32]),
+    "lvx_fwd_auto_splits": (C.c_int, [_SHAPE, C.c_int32]),
     "lvx_fwd": (C.c_int, [_SHAPE, _T, _T, _T, _T, _P, C.c_int32, C.c_int32, C.c_int32, _P, C.c_size_t, _P]),
     "lvx_fwd_acc": (C.c_int, [_SHAPE, _T, _T, _T, _T, _P, _T, _P, C.c_int32, C.c_int32, C.c_int32, _P, C.c_size_t, _P]),
     "lvx_fwd_noalloc": (C.c_int, [_SHAPE, _T, _T, _T, _T, _P, C.c_int32, C.c_int32, C.c_int32, _P]),

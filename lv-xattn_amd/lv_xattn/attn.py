@@ -14,13 +14,15 @@ Everything runs on the current PyTorch stream; nothing here synchronises.
 """
 from __future__ import annotations
 
-import math
+import ctypes as C
+import functools
 from typing import List, Optional, Sequence, Tuple
 
 import torch
 
 from . import ops
 from .async_communication import backward_workspace_cap, get_sequence_parallel_size, workspace
+from ._lib import LVX_BF16, AttnShape, load
 from .ops import Mask
 
 __all__ = ["_attn_forward", "_attn_backward", "q_block_bounds", "Mask"]
@@ -125,18 +127,16 @@ def _bias_and_hull(bias: torch.Tensor, q, k):
     return (None if exact else bias), hull
 
 
-def auto_kv_splits(B: int, Hq: int, Hkv: int, rows: int, Lkv: int, target_wgs: int = 512) -> int:
-    """Key splits for one forward launch over `rows` text rows.  A work-group
-    covers 128 (row, head) pairs of one kv head (4 waves x 32 rows); a one-round
-    launch (256 rows) has 64 of them on a 256-CU GPU, so the key range is cut
-    into up to 8 parts (each at least 512 keys) until there are two work-groups
-    per CU; the parts are folded by the merge kernel."""
-    hg = math.gcd(Hq // Hkv, 4)
-    wgs = B * (Hq // hg) * -(-rows // (32 * (4 // hg)))
-    s = 1
-    while s < 8 and wgs * s < target_wgs and Lkv // (2 * s) >= 512:
-        s *= 2
-    return s
+@functools.lru_cache(maxsize=1024)
+def auto_kv_splits(B: int, Hq: int, Hkv: int, rows: int, Lkv: int, D: int = HEAD_DIM, bias: bool = False) -> int:
+    """Key splits for one forward launch over `rows` text rows of these sizes: as many as give the chip
+    enough work-groups, as few as keep storing and folding the parts cheap.  The library prices
+    the launch (lvx_fwd_auto_splits); its answer depends on the sizes alone and is kept for the last
+    1024 of them (asking costs 5 us of host time, a decoded token's launches take 15 on the GPU)."""
+    s = AttnShape(B, Hq, Hkv, D, rows, Lkv, LVX_BF16, 1.0, None, None, None)
+    if bias:        # only whether there is one matters; any aligned address and strides do
+        s.bias, s.bias_stride_r = 16, (Lkv + 3) // 4 * 4
+    return int(load().lvx_fwd_auto_splits(C.byref(s), rows))
 
 
 def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
@@ -153,8 +153,8 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
     Keyword-only additions: `rounds` (P; default the size set by
     initialize_distributed), `mask`, `acc_in` = (O_in bf16 [B,Hq,Lq,D],
     L_in fp32 [B*Hq,Lq]) for every block, `kv_splits` (key ranges per round
-    computed by separate work-groups; default: enough to give every CU two
-    work-groups, see auto_kv_splits), `batched` (one launch over all P blocks
+    computed by separate work-groups; default: what the library prices lowest, see
+    auto_kv_splits), `batched` (one launch over all P blocks
     instead of one per round), `streams` (the rounds of one call touch disjoint rows, so on one
     GPU they may overlap: round r is queued on stream r % streams, the current stream and
     streams - 1 others of the same priority, joined before the call returns)."""
@@ -179,7 +179,7 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
     windows = [(0, Lq)] if batched else [w for w in q_block_bounds(Lq, P) if w[1] > w[0]]
     max_rows = max(r1 - r0 for r0, r1 in windows)
     if kv_splits is None:
-        kv_splits = auto_kv_splits(B, Hq, k_.shape[1], max_rows, k_.shape[2])
+        kv_splits = auto_kv_splits(B, Hq, k_.shape[1], max_rows, k_.shape[2], D, bias is not None)
     ws = None
     if kv_splits > 1:
         nbytes = ops.fwd_workspace_bytes(q_, k_, max_rows, kv_splits)

@@ -1,0 +1,55 @@
+"""The forward kernel's wide form (head dimensions 128 and 64) at the sizes where its tiles begin and end,
+against the fp32 oracle."""
+import random
+
+import pytest
+import torch
+
+from oracle import lvx_oracle as orc
+from parity import check_lse, check_o
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _check(D, dtype, B, Hq, Hkv, Lq, Lkv, splits, mask_kind, seed):
+    import lv_xattn
+    from lv_xattn import _lib
+    _lib.load()
+    rng = random.Random(seed)
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(dtype) for h, n in ((Hq, Lq), (Hkv, Lkv), (Hkv, Lkv)))
+    mask, allowed = None, None
+    if mask_kind == "kv_len":
+        n = torch.tensor([rng.randint(0, Lkv) for _ in range(B)], dtype=torch.int32)
+        mask = lv_xattn.Mask(n)
+        allowed = (torch.arange(Lkv) < n[:, None])[:, None].expand(B, Lq, Lkv)
+    elif mask_kind != "none":
+        # any two ends (some intervals empty, most tiles cut by some row), or whole images of 100 keys
+        start = torch.randint(0, Lkv, (B, Lq), generator=g, dtype=torch.int32)
+        end = torch.randint(0, Lkv + 1, (B, Lq), generator=g, dtype=torch.int32)
+        if mask_kind == "images":
+            start = start // 100 * 100
+            end = (start + 100).clamp(max=Lkv).int()
+        mask = lv_xattn.Mask(None, start, end)
+        allowed = orc.interval_mask(start.long(), end.long(), Lkv)
+    o_ref, l_ref = orc.attention_dense(q, k, v, D ** -0.5, allowed=allowed)
+    _, _, _, o, lse = lv_xattn._attn_forward(q.to(DEV), k.to(DEV), v.to(DEV), False, D ** -0.5, None, rounds=1,
+                                             batched=True, mask=mask, kv_splits=splits)
+    torch.cuda.synchronize()
+    check_o(o, o_ref)
+    check_lse(lse, l_ref)
+
+
+# key counts around one, two and three tiles of 64; row counts around one and two work-groups (64 rows
+# of four heads, 128 of two, 256 of one)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lkv,splits,mask", [
+    (4, 1, 1, 1, 1, "none"), (4, 1, 64, 64, 1, "none"), (4, 1, 65, 65, 1, "none"), (4, 1, 63, 128, 1, "none"),
+    (8, 2, 128, 129, 1, "kv_len"), (2, 2, 257, 192, 1, "none"), (4, 2, 129, 193, 1, "intervals"),
+    (4, 1, 64, 257, 2, "intervals"), (8, 1, 100, 700, 3, "images"), (3, 1, 70, 640, 1, "images"),
+    (4, 1, 10, 4300, 64, "none")])
+def test_wide_form(D, dtype, Hq, Hkv, Lq, Lkv, splits, mask, monkeypatch):
+    monkeypatch.setenv("LVX_FWD_WIDE", "1")
+    _check(D, dtype, 2, Hq, Hkv, Lq, Lkv, splits, mask, Lq * 1000 + Lkv)
