@@ -94,9 +94,12 @@ const char* lvx_strerror(int code);
  * work-groups and folded before return; it needs a workspace of
  * lvx_fwd_workspace_bytes(shape, row_count, kv_splits) bytes.
  * (at most 64 of them; lvx_fwd_auto_splits says how many suit a launch).
- * The kernel has two forms: a wavefront owns 32 text rows of a head (any head_dim, the only one with a
- * dense bias), or 64 rows and its SIMD to itself (head_dim 128 and 64).  The environment variable
- * LVX_FWD_WIDE, read at every call, overrides the choice: 0 the first form, 1 the second where it exists.
+ * The kernel has three forms, chosen by what the launch is estimated to take in each: a wavefront
+ * owns 32 text rows of a head (any head_dim, the only one with a dense bias); 64 rows and its SIMD
+ * to itself (head_dim 128 and 64); or a share of the keys for up to 32 (row, head) pairs of a kv head at
+ * once (few rows: the launch reads K and V once at the speed of HBM).  The environment variable
+ * LVX_FWD_WIDE, read at every call, overrides the choice: 0 the first form, 1 the second and 2 the third
+ * where they exist.
  * The forms give results within the same tolerance of each other, not the same bits.
  */
 int lvx_fwd(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tensor* k,

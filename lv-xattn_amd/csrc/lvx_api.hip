@@ -124,22 +124,33 @@ size_t lvx_fwd_workspace_bytes(const lvx_attn_shape* s, int32_t row_count, int32
 
 static int cu_count();
 
-// Keys per split: whole tiles.
-static int fwd_split_len(const lvx_attn_shape* s, int splits) {
-    return ((s->Lkv + splits - 1) / splits + FWD_BN - 1) / FWD_BN * FWD_BN;
+// Keys per split: whole tiles (pieces) of the form's kernel.
+static int fwd_split_len(const lvx_attn_shape* s, FwdForm form, int splits) {
+    const int step = form == FWD_FEW ? 32 : FWD_BN;
+    return ((s->Lkv + splits - 1) / splits + step - 1) / step * step;
 }
 
 // What a forward launch over `rows` text rows in this form with this many key splits takes, in us; the
 // constants are fits to launches of 1 .. 4096 rows against 600 .. 76848 keys:
+//   few  : 5 us, and per key of a work-group's range 8 ns (4.2 with heads of 64, 3 below) together with
+//          the time HBM takes for K and V (the root of the sum of squares: the two overlap in part).  One row x 32 heads x 6404 keys: 46 us whole, 12.5 in 16 - 32 parts;
+//          4 rows x 76848 keys in 32 parts: 61 us, 5.2 TB/s
 //   wide : 11 us per round of work-groups, and per 64-key tile 1.1 us on an idle chip, 1.5 on a full one
 //          (0.9 and 1.05 with heads of 64).  256 rows x 6404 keys: 138 us whole, 39 in 8 parts
 //   plain: the same with 1.8 us per tile and two work-groups per CU
 // plus, with splits, 4 us for the launch that folds the parts and their bytes at 4 TB/s.
 static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits) {
-    const int hg = gcd(s->Hq / s->Hkv, 4), rs = 4 / hg, n_cu = cu_count();
-    const int64_t split_len = fwd_split_len(s, splits);
+    const int G = s->Hq / s->Hkv, hg = gcd(G, 4), rs = 4 / hg, n_cu = cu_count();
+    const int64_t split_len = fwd_split_len(s, form, splits);
     const int64_t n = (s->Lkv + split_len - 1) / split_len;
     double t = n > 1 ? 4.0 + (double)n * s->B * s->Hq * rows * (4 * s->D + 8) / 4e6 : 0.0;
+    if (form == FWD_FEW) {
+        const int64_t wgs = (int64_t)s->B * s->Hkv * (((int64_t)rows * G + 31) / 32) * n;
+        const int64_t slots = s->D == 128 ? n_cu : 2 * n_cu;
+        const double key_us = s->D == 128 ? 8e-3 : s->D == 64 ? 4.2e-3 : 3e-3;
+        const double hbm_us = (double)s->B * s->Hkv * s->Lkv * s->D * 4 / 5.2e6;
+        return t + 5.0 + std::hypot((double)((wgs + slots - 1) / slots) * (split_len * key_us + 3.0) - 3.0, hbm_us);
+    }
     const int wg_rows = (form == FWD_WIDE ? 64 : 32) * rs;
     const int64_t wgs = (int64_t)s->B * (s->Hq / hg) * ((rows + wg_rows - 1) / wg_rows) * n;
     const int64_t slots = form == FWD_WIDE ? n_cu : 2 * n_cu;
@@ -148,13 +159,25 @@ static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int spli
     return t + (double)((wgs + slots - 1) / slots) * (split_len / FWD_BN * tile_us + 11.0);
 }
 
-// The form of the forward kernel.  Head dimensions 128 and 64 without a dense bias take the wide form;
-// the plain one was slower at every size measured (4096 rows x 6404 keys: 429 us against 354; 300 rows
-// x 2 samples: 92 against 88).
-static FwdForm fwd_form(const lvx_attn_shape* s) {
-    if (s->bias || (s->D != 128 && s->D != 64)) return FWD_PLAIN;
-    if (const char* e = getenv("LVX_FWD_WIDE")) return atoi(e) != 0 ? FWD_WIDE : FWD_PLAIN;
-    return FWD_WIDE;
+// The form for few rows is for up to 256 (row, head) columns per kv head: it reads K and V from L2 once
+// per 32 of them, and with more the other forms only lose where they are cut into too few splits.
+constexpr int64_t FEW_MAX_COLS = 256;
+static bool fwd_few_ok(const lvx_attn_shape* s, int rows) {
+    return !s->bias && (int64_t)rows * (s->Hq / s->Hkv) <= FEW_MAX_COLS;
+}
+
+// The form of the forward kernel for a window of `rows` rows whose keys are cut into `splits` ranges.
+// Head dimensions 128 and 64 without a dense bias take the wide form or, where reading K and V is the
+// larger part of the work, the form for few rows; the plain one was slower at every size measured
+// (4096 rows x 6404 keys: 429 us against 354; 300 rows x 2 samples: 92 against 88).
+static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits) {
+    if (s->bias) return FWD_PLAIN;
+    const FwdForm many = s->D == 128 || s->D == 64 ? FWD_WIDE : FWD_PLAIN;
+    if (const char* e = getenv("LVX_FWD_WIDE")) {
+        if (atoi(e) == 2 && fwd_few_ok(s, rows)) return FWD_FEW;
+        return atoi(e) != 0 ? many : FWD_PLAIN;
+    }
+    return fwd_few_ok(s, rows) && fwd_cost(s, rows, FWD_FEW, splits) <= fwd_cost(s, rows, many, splits) ? FWD_FEW : many;
 }
 
 int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
@@ -163,7 +186,8 @@ int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
     int best = 1;
     double best_cost = 0.0;
     for (int n = 1; n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
-        const double c = fwd_cost(s, row_count, many, n);
+        double c = fwd_cost(s, row_count, many, n);
+        if (fwd_few_ok(s, row_count)) c = std::min(c, fwd_cost(s, row_count, FWD_FEW, n));
         if (n == 1 || c < best_cost) { best = n; best_cost = c; }
     }
     return best;
@@ -199,15 +223,20 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     p.HG = gcd(p.G, 4);
     p.RS = 4 / p.HG;
     p.row_begin = row_begin; p.row_end = row_begin + row_count;
-    const FwdForm form = fwd_form(s);
+    const FwdForm form = fwd_form(s, row_count, kv_splits);
     p.form = form;
-    const int wg_rows = (form == FWD_WIDE ? 64 : 32) * p.RS;
-    p.n_row_tiles = (row_count + wg_rows - 1) / wg_rows;
-    p.n_head_groups = s->Hq / p.HG;
+    if (form == FWD_FEW) {
+        p.n_row_tiles = (row_count * p.G + 31) / 32;      // tiles of 32 (row, head of the group) columns
+        p.n_head_groups = s->Hkv;
+    } else {
+        const int wg_rows = (form == FWD_WIDE ? 64 : 32) * p.RS;
+        p.n_row_tiles = (row_count + wg_rows - 1) / wg_rows;
+        p.n_head_groups = s->Hq / p.HG;
+    }
     p.scale = s->scale; p.scale_log2e = s->scale * LOG2E;
 
     int nsplit = kv_splits;
-    const int split_len = fwd_split_len(s, nsplit);
+    const int split_len = fwd_split_len(s, form, nsplit);
     nsplit = (s->Lkv + split_len - 1) / split_len;
     p.nsplit = nsplit;
     p.split_len = split_len;

@@ -7,7 +7,7 @@
 // (G = 4: four heads x 32 rows; G = 1: one head x 128 rows), so the K/V tile
 // staged in LDS is read by the whole GQA group and nothing is expanded in HBM.
 // (That is fwd_kernel.  Head dimensions 128 and 64 without a dense bias run fwd_wide_kernel, in which a
-// wavefront owns 64 rows; see there.)
+// wavefront owns 64 rows, and few rows fwd_few_kernel; see there.)
 //
 // Per 64-key tile and wave (all MFMA are v_mfma_f32_32x32x16_bf16):
 //   S^T[key, row]  = K_tile (A, from LDS)  x  Q^T (B, 32 VGPRs held for the whole kernel)
@@ -600,12 +600,274 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     }
 }
 
+// Few rows (text being generated, short questions): the work is reading K and V once, 512 bytes per key
+// and kv head for a handful of multiplications, so the kernel is built around the loads.
+//
+// The rows of ALL q heads of a kv head share one 32-column tile (column = row * G + head of the
+// group), so K and V are read once per 32 of them.  A work-group is 4 waves on one key range; each wave
+// takes every fourth 32-key piece, loads it straight into a ring of two pieces of its own in LDS and
+// works on it alone - no barrier until the four partial results are folded at the end.  Both pieces
+// are requested before anything else happens: 128 KiB in flight per CU, and with ranges of 256 keys
+// or less every byte the work-group will read.  Bound by HBM where there is enough to read: 4 rows x 32
+// heads x 76848 keys (315 MB) take 61 us, 5.2 TB/s, the rate of a large copy, against 75 us in the
+// wide form; one row x 6404 keys (26 MB) 12.4 us with the fold of the parts against 17.4, most of
+// it latency.
+//   S^T[32 keys, 32 cols] = K (A, 16-byte LDS reads) x Q^T (B, registers)
+//   O^T[d, 32 cols]      += V^T (A, transposing LDS reads) x P^T (B, straight from S^T)
+// LDS rows are 2 DH bytes (128 below head dimension 64, the lanes past the head dimension repeat a
+// chunk of the row), chunks permuted as in fwd_wide_kernel.
+template <int DH, bool MASKED, bool F16>
+__global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
+    using E = Elt<F16>;
+    constexpr int LW = DH >= 64 ? DH : 64;                          // elements per LDS row
+    constexpr int NKK = DH / 16, NDT = DH >= 32 ? DH / 32 : 1;
+    constexpr int ROWB = 2 * LW, CPR = LW / 8, RPL = 64 / CPR;      // bytes and chunks per row, rows per load
+    constexpr int PB = 32 * ROWB, NLD = PB / 1024;                  // bytes and loads of a K (or V) piece
+    constexpr int EPS = 32 * NDT + 4;                               // row stride (floats) of the fold tile
+    constexpr int RING = 4 * 2 * 2 * PB, FOLD = 4 * 32 * EPS * 4;
+    __shared__ __attribute__((aligned(1024))) char lds[RING > FOLD ? RING : FOLD];
+    __shared__ float ml[4][2][32];                                  // per wave and column: reference maximum, row sum
+
+    const int wid = xcd_remap(blockIdx.x, p.total_wg);
+    if (wid >= p.total_wg) return;
+    const int ct = wid % p.n_row_tiles;            // column tile
+    const int t1 = wid / p.n_row_tiles;
+    const int split = t1 % p.nsplit;
+    const int t2 = t1 / p.nsplit;
+    const int b = t2 % p.B;
+    const int hk = t2 / p.B;
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int n_cols = p.G * (p.row_end - p.row_begin);
+    const int col = min(ct * 32 + l32, n_cols - 1);                 // columns past the last repeat it and are not stored
+    const int row = p.row_begin + col / p.G, h = hk * p.G + col % p.G;
+
+    u32x4 q[NKK];
+    {
+        const char* qp = reinterpret_cast<const char*>(p.q + b * p.qs.b + h * p.qs.h + (int64_t)row * p.qs.s + g * 8);
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk)
+            asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[kk]) : "v"(qp), "n"(32 * kk));
+    }
+
+    int kv_len = p.Lkv;
+    if (p.kv_len) kv_len = min(p.kv_len[b], p.Lkv);
+    const int kv_lo = split * p.split_len;
+    const int kv_hi = min(kv_len, kv_lo + p.split_len);
+    int my_s = kv_lo, my_e = kv_hi, lo = kv_lo, hi = kv_hi, in_lo = kv_lo, in_hi = kv_hi;
+    bool empty = kv_hi <= kv_lo;
+    if (MASKED) {
+        my_s = max(kv_lo, p.kv_start[(int64_t)b * p.Lq + row]);
+        my_e = min(kv_hi, p.kv_end[(int64_t)b * p.Lq + row]);
+        empty = my_e <= my_s;
+        // a row that sees nothing is let see everything and stored as zeros
+        lo = empty ? BIG : my_s; hi = empty ? 0 : my_e;
+        in_lo = empty ? 0 : my_s; in_hi = empty ? BIG : my_e;
+        if (empty) { my_s = 0; my_e = BIG; }
+#pragma unroll
+        for (int off = 16; off >= 1; off >>= 1) {      // the two halves of a wave hold the same columns
+            lo = min(lo, __shfl_xor(lo, off));
+            hi = max(hi, __shfl_xor(hi, off));
+            in_lo = max(in_lo, __shfl_xor(in_lo, off));
+            in_hi = min(in_hi, __shfl_xor(in_hi, off));
+        }
+        lo = uniform32(lo); hi = uniform32(hi); in_lo = uniform32(in_lo); in_hi = uniform32(in_hi);
+    }
+    const int base = lo / 32 * 32;
+    const int n_piece = hi > lo ? (hi - base + 31) / 32 : 0;
+    const int n = n_piece > wave ? (n_piece - wave + 3) / 4 : 0;    // pieces of this wave
+
+    const char* const kbase = reinterpret_cast<const char*>(p.k + b * p.ks.b + hk * p.ks.h);
+    const char* const vbase = reinterpret_cast<const char*>(p.v + b * p.vs.b + hk * p.vs.h);
+    const uint32_t krow_b = (uint32_t)p.ks.s * 2u, vrow_b = (uint32_t)p.vs.s * 2u;
+    const uint32_t ring = (uint32_t)(uintptr_t)&lds[0] + (uint32_t)wave * (4 * PB);
+    const int ld_r = lane / CPR;
+    auto issue = [&](int i) {       // this wave's piece i into ring slot i & 1; rows past the last key repeat it
+        const int kv0 = base + 32 * (wave + 4 * i);
+        const char* kb = uniform_ptr(kbase + (int64_t)kv0 * krow_b);
+        const char* vb = uniform_ptr(vbase + (int64_t)kv0 * vrow_b);
+        const uint32_t slot = uniform32(ring + (uint32_t)(i & 1) * (2 * PB));
+        const int last = hi - 1 - kv0;
+#pragma unroll
+        for (int j = 0; j < NLD; ++j) {
+            const uint32_t r = (uint32_t)min(RPL * j + ld_r, last);
+            const int f = LW == 128 ? ((lane >> 4) << 2) | (j & 3) : (((lane >> 4) & 1) << 2) | ((2 * j + (lane >> 5)) & 3);
+            const uint32_t c = (uint32_t)(((lane % CPR) ^ f) & (DH / 8 - 1)) * 16u;
+            dma16(kb, r * krow_b + c, slot + j * 1024);
+            dma16(vb, r * vrow_b + c, slot + PB + j * 1024);
+        }
+    };
+    if (n > 0) issue(0);
+    if (n > 1) issue(1);
+
+    // LDS -> operands, as in fwd_wide_kernel
+    const int f_row = LW == 128 ? (((l32 & 3) << 2) | ((l32 >> 2) & 3)) : ((((l32 >> 1) & 1) << 2) | ((l32 >> 2) & 3));
+    const uint32_t k_rd = (uint32_t)(l32 * ROWB) + (uint32_t)((g ^ f_row) << 4);
+    uint32_t v_rd[2];
+    {
+        const int r = (lane & 15) >> 2, t = lane & 3, u = (lane >> 4) & 1;
+        const int up = LW == 128 ? r : r >> 1, low = (2 * u + (t >> 1)) ^ g;
+        v_rd[0] = PB + (uint32_t)((4 * g + r) * ROWB + ((4 * up) ^ low) * 16 + (t & 1) * 8);
+        v_rd[1] = PB + (uint32_t)((4 * g + r + 8) * ROWB + ((4 * up) ^ (low ^ 2)) * 16 + (t & 1) * 8);
+    }
+
+    f32x16 acc[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[dt][v] = 0.f;
+    float m_i = -INFINITY, l_i = 0.f;
+    const float cc = p.scale_log2e;
+
+    // Q was requested first: it is here when at most the pieces' loads are outstanding
+    if (n > 1) wait_vmcnt<4 * NLD>();
+    else if (n == 1) wait_vmcnt<2 * NLD>();
+    else wait_vmcnt<0>();
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) asm volatile("" : "+v"(q[kk]));
+
+    for (int i = 0; i < n; ++i) {
+        const int kv0 = base + 32 * (wave + 4 * i);
+        const char* const pc = lds + wave * (4 * PB) + (i & 1) * (2 * PB);
+        if (i + 1 < n) wait_vmcnt<2 * NLD>();
+        else wait_vmcnt<0>();
+        f32x16 s;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) {
+            const bf16x8 ka = *reinterpret_cast<const bf16x8*>(pc + (k_rd ^ (uint32_t)(kk * 32)));
+            s = E::mfma(ka, as_bf16x8(q[kk]), s);
+        }
+        u32x2 va[NDT][2][2];        // requested now, they land during the softmax
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    va[dt][j][e] = lds_read_tr16(reinterpret_cast<const uint16_t*>(pc + (v_rd[e] ^ (uint32_t)(dt * 64)) + j * 16 * ROWB));
+        if (kv0 < in_lo || kv0 + 32 > in_hi) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int kv = kv0 + acc_row(v, g);
+                if (kv < my_s || kv >= my_e) s[v] = -INFINITY;
+            }
+        }
+        float mx = max3(s[0], s[1], s[2]);
+#pragma unroll
+        for (int v = 3; v < 15; v += 2) mx = max3(mx, s[v], s[v + 1]);
+        mx = fmaxf(mx, s[15]);
+        {
+            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+            mx = max3(__uint_as_float(sw[0]), __uint_as_float(sw[1]), m_i);
+        }
+        // lazy rescale, as in fwd_kernel
+        const float mcand = mx * cc, m_ic = m_i * cc;
+        const bool move = (mx != -INFINITY) && !(mcand - m_ic <= RESCALE_LOG2);
+        const float alpha = move ? __builtin_amdgcn_exp2f(m_ic - mcand) : 1.f;
+        if (move) m_i = mx;
+        const float mc = (m_i == -INFINITY) ? 0.f : m_i * cc;
+        bf16x8 pb[2];
+        float rs = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            u32x4 u;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float a0 = __builtin_amdgcn_exp2f(fmaf(s[8 * j + 2 * e], cc, -mc)), a1 = __builtin_amdgcn_exp2f(fmaf(s[8 * j + 2 * e + 1], cc, -mc));
+                rs += a0 + a1;
+                u[e] = E::pack(a0, a1);
+            }
+            pb[j] = as_bf16x8(u);
+        }
+        l_i = l_i * alpha + rs;
+        if (i > 0 && __builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[dt][v] *= alpha;
+        }
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const u32x4 a = {va[dt][j][0][0], va[dt][j][0][1], va[dt][j][1][0], va[dt][j][1][1]};
+                acc[dt] = E::mfma(as_bf16x8(a), pb[j], acc[dt]);
+            }
+        if (i + 2 < n) {
+            wait_lds();             // this slot has been read
+            issue(i + 2);
+        }
+    }
+
+    // Fold the four waves: every wave leaves its O^T as rows [col][d] in fp32 with its reference and sum;
+    // 8 lanes then share a column.
+    __syncthreads();                // the ring is free
+    float* const ep = reinterpret_cast<float*>(lds) + wave * (32 * EPS);
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int vg = 0; vg < 4; ++vg) {
+            const f32x4 x = {acc[dt][4 * vg], acc[dt][4 * vg + 1], acc[dt][4 * vg + 2], acc[dt][4 * vg + 3]};
+            *reinterpret_cast<f32x4*>(ep + l32 * EPS + dt * 32 + 8 * vg + 4 * g) = x;
+        }
+    const float l_tot = l_i + __shfl_xor(l_i, 32);
+    if (g == 0) {
+        ml[wave][0][l32] = m_i;
+        ml[wave][1][l32] = empty ? 0.f : l_tot;
+    }
+    __syncthreads();
+    constexpr int TPC = 8, DPT = DH / TPC;          // threads per column, values of d per thread
+    const int oc = tid / TPC, part = tid % TPC;
+    if (ct * 32 + oc >= n_cols) return;
+    const int orow = p.row_begin + (ct * 32 + oc) / p.G, oh = hk * p.G + (ct * 32 + oc) % p.G;
+    float M = -INFINITY, w[4], den = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) M = fmaxf(M, ml[k][0][oc]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        w[k] = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((ml[k][0][oc] - M) * cc);
+        den = fmaf(w[k], ml[k][1][oc], den);
+    }
+    const float inv = den > 0.f ? 1.f / den : 0.f;
+    uint16_t* const op = p.o + split * p.o_split_stride + b * p.os.b + oh * p.os.h + (int64_t)orow * p.os.s + part * DPT;
+    const float* const src = reinterpret_cast<const float*>(lds) + oc * EPS + part * DPT;
+    uint32_t out[DPT / 2];
+#pragma unroll
+    for (int d = 0; d < DPT; d += 2) {
+        float x0 = 0.f, x1 = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            x0 = fmaf(w[k], src[k * (32 * EPS) + d], x0);
+            x1 = fmaf(w[k], src[k * (32 * EPS) + d + 1], x1);
+        }
+        out[d / 2] = E::pack(x0 * inv, x1 * inv);
+    }
+    if constexpr (DPT >= 8) {
+#pragma unroll
+        for (int d = 0; d < DPT / 8; ++d)
+            *reinterpret_cast<u32x4*>(op + 8 * d) = u32x4{out[4 * d], out[4 * d + 1], out[4 * d + 2], out[4 * d + 3]};
+    } else {
+#pragma unroll
+        for (int d = 0; d < DPT / 2; ++d) *reinterpret_cast<uint32_t*>(op + 2 * d) = out[d];
+    }
+    if (part == 0)
+        p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + oh) * p.lse_bh_stride + orow] =
+            den > 0.f ? M * p.scale + __logf(den) : -INFINITY;
+}
+
 }  // namespace
 
 namespace {
 template <int DH, bool F16>
 hipError_t launch_fwd_t(const FwdParams& p, bool masked, hipStream_t st) {
     const int grid = ((p.total_wg + 7) / 8) * 8;
+    if (p.form == FWD_FEW) {
+        if (masked) return launch1((fwd_few_kernel<DH, true, F16>), dim3(grid), dim3(256), st, p);
+        return launch1((fwd_few_kernel<DH, false, F16>), dim3(grid), dim3(256), st, p);
+    }
     if constexpr (DH >= 64) {
         if (p.form == FWD_WIDE) {
             if (masked) return launch1((fwd_wide_kernel<DH, true, F16>), dim3(grid), dim3(256), st, p);

@@ -1,5 +1,5 @@
-"""The forward kernel's wide form (head dimensions 128 and 64) at the sizes where its tiles begin and end,
-against the fp32 oracle."""
+"""The forward kernel's wide form (head dimensions 128 and 64) and its form for few rows (all four), at the
+sizes where their tiles begin and end, against the fp32 oracle."""
 import random
 
 import pytest
@@ -53,3 +53,16 @@ def _check(D, dtype, B, Hq, Hkv, Lq, Lkv, splits, mask_kind, seed):
 def test_wide_form(D, dtype, Hq, Hkv, Lq, Lkv, splits, mask, monkeypatch):
     monkeypatch.setenv("LVX_FWD_WIDE", "1")
     _check(D, dtype, 2, Hq, Hkv, Lq, Lkv, splits, mask, Lq * 1000 + Lkv)
+
+
+# key counts around one piece of 32, one round of the four waves (128) and two (256); columns (rows x heads
+# of the group) around one tile of 32
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [128, 64, 32, 16])
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lkv,splits,mask", [
+    (4, 1, 1, 1, 1, "none"), (4, 1, 8, 32, 1, "none"), (4, 1, 9, 33, 1, "none"), (1, 1, 31, 128, 1, "none"),
+    (8, 2, 1, 129, 1, "kv_len"), (3, 1, 11, 257, 1, "none"), (8, 1, 4, 511, 2, "intervals"),
+    (2, 1, 128, 300, 1, "images"), (4, 2, 3, 2500, 64, "none"), (4, 4, 5, 700, 5, "images")])
+def test_few_rows_form(D, dtype, Hq, Hkv, Lq, Lkv, splits, mask, monkeypatch):
+    monkeypatch.setenv("LVX_FWD_WIDE", "2")
+    _check(D, dtype, 2, Hq, Hkv, Lq, Lkv, splits, mask, Lq * 1000 + Lkv + 1)
