@@ -1,4 +1,5 @@
-"""Builds liblvx.so (the gfx950 kernels + C ABI) in-tree with hipcc.
+"""Builds liblvx.so (the gfx950 kernels + C ABI) in-tree with hipcc, and _lvx_host.so (the package's
+per-call host work, against torch's C++ headers) with g++.
 
     python lv-xattn_amd/build.py [--force] [--verbose]
 
@@ -20,6 +21,8 @@ CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "lv_xattn")
 BUILD_DIR = os.path.join(HERE, "build")
 LIB = os.path.join(OUT_DIR, "liblvx.so")
+HOST_SRC = os.path.join(CSRC, "lvx_host.cpp")
+HOST_LIB = os.path.join(OUT_DIR, "_lvx_host.so")
 
 SOURCES = ["lvx_api.hip", "lvx_fwd.hip", "lvx_bwd.hip", "lvx_rowwise.hip", "lvx_gemm.hip"]
 
@@ -73,6 +76,20 @@ def generate() -> None:
                 f.write(r.stdout)
 
 
+def host_command():
+    """g++ command line of the host extension module; it finds liblvx.so beside itself."""
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    inc = [*include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-isystem{i}" for i in inc], HOST_SRC,
+            "-o", HOST_LIB, f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+            f"-L{OUT_DIR}", "-l:liblvx.so", "-Wl,-rpath,$ORIGIN"]
+
+
 def build(force: bool = True, verbose: bool = False, extra_flags=()) -> str:
     os.makedirs(BUILD_DIR, exist_ok=True)
     cc = hipcc()
@@ -92,6 +109,9 @@ def build(force: bool = True, verbose: bool = False, extra_flags=()) -> str:
         list(ex.map(lambda c: _run(c, verbose), jobs))
     if jobs or not os.path.exists(LIB):
         _run([cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", *objs, "-o", LIB], verbose)
+    header = os.path.join(HERE, "..", "include", "lvx.h")
+    if force or not os.path.exists(HOST_LIB) or os.path.getmtime(HOST_LIB) < max(os.path.getmtime(HOST_SRC), os.path.getmtime(header)):
+        _run(host_command(), verbose)
     return LIB
 
 

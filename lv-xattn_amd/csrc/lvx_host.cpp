@@ -1,0 +1,144 @@
+// The per-call host work of the attention operators in native code: what ops.py and attn.py would
+// otherwise do with some forty Python and ctypes operations a call (argument checks, tensor descriptions,
+// the current stream, output and workspace tensors).  A decoded token's two launches take 12 us on the
+// GPU; issuing them through ctypes took 32 us of host time.
+//
+// An operator answers False, and queues nothing, when a call is not one it can pass on as it is (a wrong
+// type, shape or device among the arguments); the caller then goes through its own checks, which word
+// the error.
+#include <torch/csrc/utils/pybind.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+
+#include <optional>
+
+#include "../../include/lvx.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+int dtype_code(const Tensor& t) {
+    return t.scalar_type() == at::kBFloat16 ? LVX_BF16 : t.scalar_type() == at::kHalf ? LVX_F16 : 0;
+}
+
+lvx_tensor t4(const Tensor& t) { return lvx_tensor{t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)}; }
+
+// a 4-d tensor on q's device with unit last stride
+bool plain4(const Tensor& t, const Tensor& q, at::ScalarType type) {
+    return t.dim() == 4 && t.stride(3) == 1 && t.scalar_type() == type && t.device() == q.device();
+}
+
+bool rows_ok(const Tensor& l, const Tensor& q) {        // LSE, delta: contiguous fp32 [B * Hq, Lq]
+    return l.scalar_type() == at::kFloat && l.is_contiguous() && l.numel() == q.size(0) * q.size(1) * q.size(2) && l.device() == q.device();
+}
+
+bool mask_ok(const OptTensor& m, const Tensor& q, bool per_row) {
+    if (!m) return true;
+    return m->scalar_type() == at::kInt && m->device() == q.device() && m->is_contiguous() && m->dim() == (per_row ? 2 : 1) &&
+           m->size(0) == q.size(0) && (!per_row || m->size(1) == q.size(2));
+}
+
+// Fills the shape from tensors of one type and device; false when something does not fit.
+bool fill_shape(lvx_attn_shape& s, const Tensor& q, const Tensor& k, const Tensor& v, double scale, const OptTensor& kv_len,
+                const OptTensor& kv_start, const OptTensor& kv_end) {
+    const int dt = dtype_code(q);
+    if (!q.is_cuda() || !dt || !plain4(q, q, q.scalar_type()) || !plain4(k, q, q.scalar_type()) || !plain4(v, q, q.scalar_type()))
+        return false;
+    if (k.size(0) != q.size(0) || k.size(3) != q.size(3) || v.sizes() != k.sizes()) return false;
+    if (!mask_ok(kv_len, q, false) || !mask_ok(kv_start, q, true) || !mask_ok(kv_end, q, true) || !kv_start != !kv_end) return false;
+    if (c10::hip::current_device() != q.device().index()) return false;       // launches go to the current device
+    s = lvx_attn_shape{};
+    s.B = (int32_t)q.size(0); s.Hq = (int32_t)q.size(1); s.Hkv = (int32_t)k.size(1); s.D = (int32_t)q.size(3);
+    s.Lq = (int32_t)q.size(2); s.Lkv = (int32_t)k.size(2); s.dtype = dt; s.scale = (float)scale;
+    if (kv_len) s.kv_len = kv_len->data_ptr<int32_t>();
+    if (kv_start) { s.kv_start = kv_start->data_ptr<int32_t>(); s.kv_end = kv_end->data_ptr<int32_t>(); }
+    return true;
+}
+
+void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+// A code of the library as the package's own exception.
+void check(int rc, const char* what) {
+    if (rc) py::module_::import("lv_xattn._lib").attr("check")(rc, what);
+}
+
+// Whether the kernels can read every one of these where it lies: unit last stride, the others multiples
+// of 8 elements, 16-byte aligned.
+bool usable(const Tensor& a, const Tensor& b, const Tensor& c) {
+    for (const Tensor* t : {&a, &b, &c})
+        if (t->dim() != 4 || t->stride(3) != 1 || ((t->stride(0) | t->stride(1) | t->stride(2)) & 7) ||
+            (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15))
+            return false;
+    return true;
+}
+
+// (o, lse, workspace or None) of a forward: o like q and contiguous, or the view of [B, Lq, Hq, D] memory with
+// `token_major`; lse fp32 [B * Hq, Lq]; room for the parts of kv_splits key splits over `rows` rows.
+py::tuple forward_buffers(const Tensor& q, int64_t rows, int64_t kv_splits, bool token_major) {
+    const int64_t B = q.size(0), H = q.size(1), L = q.size(2), D = q.size(3);
+    Tensor o = token_major ? at::empty({B, L, H, D}, q.options()).transpose(1, 2) : at::empty({B, H, L, D}, q.options());
+    Tensor lse = at::empty({B * H, L}, q.options().dtype(at::kFloat));
+    if (kv_splits <= 1) return py::make_tuple(std::move(o), std::move(lse), py::none());
+    lvx_attn_shape s{};
+    s.B = (int32_t)B; s.Hq = (int32_t)H; s.D = (int32_t)D;
+    Tensor ws = at::empty({(int64_t)lvx_fwd_workspace_bytes(&s, (int32_t)rows, (int32_t)kv_splits)}, q.options().dtype(at::kByte));
+    return py::make_tuple(std::move(o), std::move(lse), std::move(ws));
+}
+
+bool fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, double scale, int64_t row_begin,
+         int64_t row_count, const OptTensor& kv_len, const OptTensor& kv_start, const OptTensor& kv_end, int64_t kv_splits,
+         const OptTensor& ws, const OptTensor& acc_o, const OptTensor& acc_l) {
+    lvx_attn_shape s;
+    if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end) || !plain4(o, q, q.scalar_type()) || !rows_ok(lse, q)) return false;
+    const lvx_tensor tq = t4(q), tk = t4(k), tv = t4(v), to = t4(o);
+    void* const wp = ws ? ws->data_ptr() : nullptr;
+    const size_t wb = ws ? ws->nbytes() : 0;
+    if (!acc_o) {
+        check(lvx_fwd(&s, &tq, &tk, &tv, &to, lse.data_ptr<float>(), (int32_t)row_begin, (int32_t)row_count, (int32_t)kv_splits, wp, wb,
+                      current_stream()), "lvx_fwd");
+        return true;
+    }
+    if (!plain4(*acc_o, q, q.scalar_type()) || acc_o->sizes() != q.sizes() || !acc_l || !rows_ok(*acc_l, q)) return false;
+    const lvx_tensor ta = t4(*acc_o);
+    check(lvx_fwd_acc(&s, &tq, &tk, &tv, &ta, acc_l->data_ptr<float>(), &to, lse.data_ptr<float>(), (int32_t)row_begin,
+                      (int32_t)row_count, (int32_t)kv_splits, wp, wb, current_stream()), "lvx_fwd_acc");
+    return true;
+}
+
+bool bwd_preprocess(const Tensor& o, const Tensor& dout, const Tensor& delta, int64_t row_begin, int64_t row_count) {
+    lvx_attn_shape s;
+    if (!fill_shape(s, o, dout, dout, 1.0, {}, {}, {}) || o.sizes() != dout.sizes() || !rows_ok(delta, o)) return false;
+    const lvx_tensor to = t4(o), td = t4(dout);
+    check(lvx_bwd_preprocess(&s, &to, &td, delta.data_ptr<float>(), (int32_t)row_begin, (int32_t)row_count, current_stream()),
+          "lvx_bwd_preprocess");
+    return true;
+}
+
+bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
+         const Tensor& dk, const Tensor& dv, double scale, int64_t row_begin, int64_t row_count, const OptTensor& kv_len,
+         const OptTensor& kv_start, const OptTensor& kv_end, bool accumulate_dkv, const Tensor& ws) {
+    lvx_attn_shape s;
+    if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end)) return false;
+    const at::ScalarType kv_type = accumulate_dkv ? at::kFloat : q.scalar_type();
+    if (!plain4(dout, q, q.scalar_type()) || dout.sizes() != q.sizes() || !rows_ok(lse, q) || !rows_ok(delta, q) ||
+        !plain4(dq, q, q.scalar_type()) || dq.sizes() != q.sizes() || !plain4(dk, q, kv_type) || dk.sizes() != k.sizes() ||
+        !plain4(dv, q, kv_type) || dv.sizes() != k.sizes())
+        return false;
+    const lvx_tensor tq = t4(q), tk = t4(k), tv = t4(v), td = t4(dout), tdq = t4(dq), tdk = t4(dk), tdv = t4(dv);
+    check(lvx_bwd(&s, &tq, &tk, &tv, &td, lse.data_ptr<float>(), delta.data_ptr<float>(), &tdq, &tdk, &tdv, accumulate_dkv ? 1 : 0,
+                  (int32_t)row_begin, (int32_t)row_count, ws.data_ptr(), ws.nbytes(), current_stream()), "lvx_bwd");
+    return true;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_lvx_host, m) {
+    m.def("usable", &usable);
+    m.def("forward_buffers", &forward_buffers);
+    m.def("fwd", &fwd);
+    m.def("bwd_preprocess", &bwd_preprocess);
+    m.def("bwd", &bwd);
+}

@@ -89,6 +89,22 @@ def load() -> C.CDLL:
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native side of the operators (_lvx_host.so, built with the library).  Raises if it is absent."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _lvx_host
+        except ImportError as e:
+            raise LvxError("_lvx_host.so is missing or does not load: run `python lv-xattn_amd/build.py`") from e
+        _host = _lvx_host
+    return _host
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load().lvx_strerror(rc).decode()

@@ -22,7 +22,7 @@ import torch
 
 from . import ops
 from .async_communication import backward_workspace_cap, get_sequence_parallel_size, workspace
-from ._lib import LVX_BF16, AttnShape, load
+from ._lib import LVX_BF16, AttnShape, host, load
 from .ops import Mask
 
 __all__ = ["_attn_forward", "_attn_backward", "q_block_bounds", "Mask"]
@@ -143,7 +143,8 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
                   local_bias_args=[], remote_bias_args=[], no_overlap=False, *,
                   rounds: Optional[int] = None, mask: Optional[Mask] = None,
                   acc_in: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
-                  kv_splits: Optional[int] = None, batched: bool = False, streams: int = 1):
+                  kv_splits: Optional[int] = None, batched: bool = False, streams: int = 1,
+                  _token_major: bool = False):
     """Returns (q, k, v, o, L) like the reference (attn.py:435): o [B,Hq,Lq,D]
     bf16, L [B*Hq, Lq] fp32 natural-log LSE of sm_scale * q k^T.
 
@@ -157,10 +158,13 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
     auto_kv_splits), `batched` (one launch over all P blocks
     instead of one per round), `streams` (the rounds of one call touch disjoint rows, so on one
     GPU they may overlap: round r is queued on stream r % streams, the current stream and
-    streams - 1 others of the same priority, joined before the call returns)."""
+    streams - 1 others of the same priority, joined before the call returns).  `_token_major`: o is a view of
+    [B,Lq,Hq,D] memory, the order the layer's output projection reads."""
     _reject_unsupported(causal)
     D_in = q.shape[-1]
-    q_, k_, v_ = (_usable(_pad_head_dim(t)) for t in (q, k, v))
+    q_, k_, v_ = _pad_head_dim(q), _pad_head_dim(k), _pad_head_dim(v)
+    if not host().usable(q_, k_, v_):
+        q_, k_, v_ = _usable(q_), _usable(k_), _usable(v_)
     B, Hq, Lq, D = q_.shape
     P = rounds if rounds is not None else get_sequence_parallel_size()
     dev = q_.device
@@ -169,9 +173,6 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
         mask = mask.to(dev)
     elif bias is not None:
         bias, mask = _bias_and_hull(bias, q_, k_)    # skip what the bias masks out anyway
-
-    o = torch.empty(B, Hq, Lq, D, dtype=q_.dtype, device=dev)
-    L = torch.empty(B * Hq, Lq, dtype=torch.float32, device=dev)
     if acc_in is not None:
         acc_o = _usable(_pad_head_dim(acc_in[0].to(dtype=q_.dtype)))
         acc_l = acc_in[1].to(torch.float32).reshape(B * Hq, Lq).contiguous()
@@ -180,10 +181,8 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
     max_rows = max(r1 - r0 for r0, r1 in windows)
     if kv_splits is None:
         kv_splits = auto_kv_splits(B, Hq, k_.shape[1], max_rows, k_.shape[2], D, bias is not None)
-    ws = None
-    if kv_splits > 1:
-        nbytes = ops.fwd_workspace_bytes(q_, k_, max_rows, kv_splits)
-        ws = workspace("fwd_split", (nbytes,), torch.uint8, dev)
+    # the parts of the key splits live for this call only (from torch's caching allocator, as o and L)
+    o, L, ws = host().forward_buffers(q_, max_rows, kv_splits, _token_major)
 
     # the partial goes straight into (o, L), merged on its way with the incoming accumulator
     # if there is one (with key splits by the launch that folds the splits; neither a copy of
@@ -197,7 +196,7 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
         with _RoundStreams(dev, min(streams, len(windows))) as rs:
             for i, (r0, r1) in enumerate(windows):
                 with rs.stream(i):
-                    ws_i = workspace("fwd_split", (nbytes,), torch.uint8, dev) if kv_splits > 1 else None
+                    ws_i = workspace("fwd_split", (ws.numel(),), torch.uint8, dev) if ws is not None else None
                     one_round(r0, r1, ws_i)
     else:
         for r0, r1 in windows:

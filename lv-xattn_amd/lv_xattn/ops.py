@@ -12,7 +12,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from ._lib import AttnShape, LvxError, check, load, ptr, stream_ptr, t4
+from ._lib import AttnShape, LvxError, check, host, load, ptr, stream_ptr, t4
 
 
 @dataclass
@@ -29,10 +29,16 @@ class Mask:
     kv_end: Optional[torch.Tensor] = None
 
     def to(self, device) -> "Mask":
-        f = lambda t: None if t is None else t.to(device=device, dtype=torch.int32).contiguous()
+        device = torch.device(device)
+
+        def f(t):
+            if t is None or (t.dtype == torch.int32 and t.device == device and t.is_contiguous()):
+                return t
+            return t.to(device=device, dtype=torch.int32).contiguous()
         return Mask(f(self.kv_len), f(self.kv_start), f(self.kv_end))
 
 
+_NO_MASK = Mask()
 _DTYPES = {torch.bfloat16: _lib.LVX_BF16, torch.float16: _lib.LVX_F16}
 
 
@@ -92,6 +98,12 @@ def fwd(q, k, v, o, lse, scale, row_begin=0, row_count=None, mask: Optional[Mask
     `bias`: dense additive fp32 [B|1, Hq|1, Lq, Lkv], added after the scale.
     `acc` = (o_in like o, l_in fp32 [B*Hq, Lq]): an incoming accumulator the result is merged
     with before it is written (lvx_fwd_acc); only read, and not o itself."""
+    if bias is None:
+        m = mask or _NO_MASK
+        a = acc or (None, None)
+        if host().fwd(q, k, v, o, lse, scale, row_begin, q.shape[2] - row_begin if row_count is None else row_count,
+                      m.kv_len, m.kv_start, m.kv_end, kv_splits, workspace, a[0], a[1]):
+            return
     s = _shape(q, k, scale, mask, bias)
     if row_count is None:
         row_count = q.shape[2] - row_begin
@@ -168,6 +180,8 @@ def bias_is_interval(q, k, bias: torch.Tensor, hull: Mask) -> bool:
 
 
 def bwd_preprocess(o, dout, delta, row_begin=0, row_count=None) -> None:
+    if host().bwd_preprocess(o, dout, delta, row_begin, o.shape[2] - row_begin if row_count is None else row_count):
+        return
     B, Hq, Lq, D = o.shape
     s = AttnShape(B, Hq, Hq, D, Lq, 1, dtype_code(o, dout), 1.0, None, None, None)
     if row_count is None:
@@ -192,6 +206,12 @@ def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=Non
     (fp32) dk, dv at Hkv heads.  `workspace`: uint8 tensor of at least
     bwd_workspace_bytes(q, k, row_count, mask) bytes.  `bias` as in fwd (no gradient
     is formed for it)."""
+    if bias is None and workspace is not None:
+        m = mask or _NO_MASK
+        if host().bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin,
+                      q.shape[2] - row_begin if row_count is None else row_count, m.kv_len, m.kv_start, m.kv_end,
+                      accumulate_dkv, workspace):
+            return
     s = _shape(q, k, scale, mask, bias)
     if row_count is None:
         row_count = q.shape[2] - row_begin
