@@ -183,6 +183,19 @@ int lvx_bias_is_interval(const lvx_attn_shape* shape, const int32_t* kv_start, c
                          int32_t* not_interval, void* stream);
 
 /*
+ * kv_start / kv_end [B, Lq] (int32, written): per row of an additive attention mask the interval of keys it
+ * leaves visible, if that is all the mask says of the row: the entries above -30000 are one run of
+ * keys, at least one, and exactly 0.  kv_start = -1 for any other row; if there is none the caller may
+ * run lvx_fwd / lvx_bwd with the intervals in the mask's place.  mask: element (b, row, key) at
+ * mask[b*stride_b + row*stride_r + key], of type `type`: LVX_BF16, LVX_F16, or 0 for fp32, aligned to its
+ * element size.  (The words of 8 bytes that hold the first and the last element of a row are read whole.)
+ * No counterpart in the reference; it is how a mask that transformers has built reaches the kernels
+ * that read none.
+ */
+int lvx_mask_intervals(const void* mask, int32_t type, int64_t stride_b, int64_t stride_r, int32_t B, int32_t Lq,
+                       int32_t Lkv, int32_t* kv_start, int32_t* kv_end, void* stream);
+
+/*
  * delta[b*Hq+h, row] = sum_d O * dO.  Replaces `_bwd_preprocess_do_o_dot`
  * (lv_xattn/flash_attn_kernels.py:287-329, launched at :926-942).
  */

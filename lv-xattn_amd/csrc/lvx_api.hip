@@ -412,6 +412,16 @@ int lvx_bias_is_interval(const lvx_attn_shape* s, const int32_t* kv_start, const
     return static_cast<int>(launch_bias_interval(p, static_cast<hipStream_t>(stream)));
 }
 
+int lvx_mask_intervals(const void* mask, int32_t type, int64_t stride_b, int64_t stride_r, int32_t B, int32_t Lq,
+                       int32_t Lkv, int32_t* kv_start, int32_t* kv_end, void* stream) {
+    if (!mask || !kv_start || !kv_end) return LVX_ERR_NULL;
+    if (type != LVX_BF16 && type != LVX_F16 && type != 0) return LVX_ERR_DTYPE;
+    if (reinterpret_cast<uintptr_t>(mask) & (type ? 1 : 3)) return LVX_ERR_ALIGN;
+    if (B <= 0 || Lq <= 0 || Lkv <= 0 || (int64_t)B * Lq > INT32_MAX || stride_b < 0 || stride_r < 0) return LVX_ERR_SHAPE;
+    const MaskIntervalParams p{mask, stride_b, stride_r, type, kv_start, kv_end, B, Lq, Lkv};
+    return static_cast<int>(launch_mask_intervals(p, static_cast<hipStream_t>(stream)));
+}
+
 int lvx_bwd_preprocess(const lvx_attn_shape* s, const lvx_tensor* o, const lvx_tensor* dout, float* delta,
                        int32_t row_begin, int32_t row_count, void* stream) {
     LVX_TRY(check_shape(s));

@@ -81,6 +81,17 @@ struct BiasHullParams {
     int B, heads, Lq, Lkv;     // heads: 1 (bias broadcast over heads) or Hq
     int32_t* flag;             // interval test only: set to 1 when the bias is not 0 everywhere inside the hull
 };
+// Per text row of an additive mask [B][Lq][Lkv] (type: LVX_BF16, LVX_F16 or 0 for fp32; element strides
+// stride_b, stride_r) the interval of keys it leaves visible, where that is all it says.
+struct MaskIntervalParams {
+    const void* mask;
+    int64_t stride_b, stride_r;
+    int type;
+    int32_t* kv_start;         // [B, Lq]; -1 for a row that is more than an interval
+    int32_t* kv_end;           // [B, Lq]
+    int B, Lq, Lkv;
+};
+hipError_t launch_mask_intervals(const MaskIntervalParams& p, hipStream_t st);
 hipError_t launch_bias_hull(const BiasHullParams& p, hipStream_t st);
 hipError_t launch_bias_interval(const BiasHullParams& p, hipStream_t st);
 

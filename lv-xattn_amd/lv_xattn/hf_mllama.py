@@ -32,7 +32,9 @@ from typing import Optional
 
 import torch
 
+from . import ops
 from ._lib import LvxError
+from .attn import _attn_forward
 from .autograd import create_attention_class, create_attention_class_save_qkv, create_q_projection_class
 
 NAME = "lv_xattn"
@@ -75,9 +77,27 @@ def _mask_bias(mask: torch.Tensor) -> torch.Tensor:
     return bias
 
 
+_interval_cache: list = []  # [key, Mask or None, the mask it was made from] of the last one looked at
+
+
+def _mask_intervals(mask: torch.Tensor):
+    """The interval mask that says all that transformers' additive `mask` says (ops.mask_intervals), or
+    None: the usual case, a row looks at the tiles of the images before it.  Every layer of a model
+    gets the same mask, so the last answer is kept, with the mask, as `_mask_bias` keeps its own."""
+    version = None if mask.is_inference() else mask._version
+    key = (mask.data_ptr(), version, tuple(mask.shape), tuple(mask.stride()), mask.dtype, mask.device)
+    if version is not None and _interval_cache and _interval_cache[0] == key:
+        return _interval_cache[1]
+    intervals = ops.mask_intervals(mask)
+    if version is not None:
+        _interval_cache[:] = [key, intervals, mask]
+    return intervals
+
+
 def clear_mask_cache() -> None:
-    """Drops the converted mask `_mask_bias` keeps (an fp32 tensor of the mask's size)."""
+    """Drops the converted masks `_mask_bias` (an fp32 tensor of the mask's size) and `_mask_intervals` keep."""
     _bias_cache.clear()
+    _interval_cache.clear()
 
 
 def lv_xattn_attention_forward(module, query, key, value, attention_mask: Optional[torch.Tensor],
@@ -94,15 +114,21 @@ def lv_xattn_attention_forward(module, query, key, value, attention_mask: Option
         return sdpa_attention_forward(module, query, key, value, attention_mask, dropout=dropout,
                                       scaling=scaling, **kwargs)
     _require_supported(query, key, dropout)
-    if _attention is None:
-        _attention = create_attention_class_save_qkv("lv_xattn", rounds=1, batched=True).apply
     if scaling is None:
         scaling = query.shape[-1] ** -0.5
-    if attention_mask is None:
-        out = _attention(query, key, value, False, scaling)
+    mask = intervals = None
+    if attention_mask is not None:
+        mask = attention_mask[..., :query.shape[2], :key.shape[2]]
+        intervals = _mask_intervals(mask)
+    if (mask is None or intervals is not None) and not (torch.is_grad_enabled() and (
+            query.requires_grad or key.requires_grad or value.requires_grad)):
+        out = _attn_forward(query, key, value, False, scaling, None, rounds=1, batched=True, mask=intervals, _token_major=True)[3]
+        return out.transpose(1, 2).contiguous(), None
+    if _attention is None:
+        _attention = create_attention_class_save_qkv("lv_xattn", rounds=1, batched=True, token_major=True).apply
+    if mask is None or intervals is not None:
+        out = _attention(query, key, value, False, scaling, None, [], [], intervals)
     else:
-        Lq, Lkv = query.shape[2], key.shape[2]
-        mask = attention_mask[..., :Lq, :Lkv]
         out = _attention(query, key, value, False, scaling, _mask_bias, [mask], [])
     return out.transpose(1, 2).contiguous(), None
 
@@ -146,8 +172,10 @@ def _recompute_forward(self, hidden_states, cross_attention_states=None, past_ke
     mask = kwargs.get("lvx_mask")
     bias = []
     if mask is None and attention_mask is not None:
-        lkv = cross_attention_states.shape[1]
-        bias = [_mask_bias, attention_mask[..., :q_len, :lkv]]
+        dense = attention_mask[..., :q_len, :cross_attention_states.shape[1]]
+        mask = _mask_intervals(dense)
+        if mask is None:
+            bias = [_mask_bias, dense]
     out = _recompute[key](query, cross_attention_states.to(query.dtype), self.k_proj.weight, self.v_proj.weight,
                           self.num_key_value_heads, self.scaling, mask, self.k_norm.weight,
                           self.k_norm.variance_epsilon, *bias)

@@ -179,6 +179,21 @@ def bias_is_interval(q, k, bias: torch.Tensor, hull: Mask) -> bool:
     return int(flag.item()) == 0
 
 
+def mask_intervals(mask: torch.Tensor) -> Optional[Mask]:
+    """The interval mask an additive mask [B, 1, Lq, Lkv] (bf16, fp16 or fp32) amounts to, None when some
+    row of it is more than one run of visible keys (entries of 0; above -30000 counts as visible) or
+    sees none.  Waits for the GPU (the row starts come back)."""
+    B, _, Lq, Lkv = mask.shape
+    code = {torch.bfloat16: _lib.LVX_BF16, torch.float16: _lib.LVX_F16, torch.float32: 0}.get(mask.dtype)
+    if code is None or mask.shape[1] != 1 or mask.stride(3) != 1 or min(mask.stride()) < 0:
+        return None
+    rows = torch.empty(2, B, Lq, dtype=torch.int32, device=mask.device)
+    rc = load().lvx_mask_intervals(mask.data_ptr(), code, mask.stride(0), mask.stride(2), B, Lq, Lkv, rows.data_ptr(),
+                                   rows.data_ptr() + 4 * B * Lq, stream_ptr())
+    check(rc, "lvx_mask_intervals")
+    return Mask(None, rows[0], rows[1]) if int(rows[0].cpu().min()) >= 0 else None
+
+
 def bwd_preprocess(o, dout, delta, row_begin=0, row_count=None) -> None:
     if host().bwd_preprocess(o, dout, delta, row_begin, o.shape[2] - row_begin if row_count is None else row_count):
         return
