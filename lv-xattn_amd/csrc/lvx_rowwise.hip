@@ -478,12 +478,17 @@ __global__ __launch_bounds__(256) void cast_t_kernel(const CastParams p) {
 
 // Backward of y = w * bf16(x * r) over 128-wide rows: with xh = x * r and gg = dy * w,
 //   dx = r * (gg - xh * mean(gg * xh)),   dw += sum over rows of dy * bf16(xh).
-// 16 lanes per row (8 columns each); a thread keeps the dw partial sums of its 8 columns
-// over the rows it visits, the block folds them through LDS and adds them with atomics.
+// 16 lanes per row (8 columns each); a thread keeps the dw partial sums of its 8 columns over the rows
+// it visits, the block folds them through LDS and adds them with 128 atomics.  All blocks add to the
+// same 128 floats, which takes 0.2 ns an addition: with 2048 blocks that was the kernel (57 us on 102464
+// rows, whose 79 MB take 15 us to move), so there is one block of 1024 threads per CU, each thread
+// with the loads of two rows in flight: 19 us.
+constexpr int NORM_THREADS = 1024, NORM_ROWS = NORM_THREADS / 16, NORM_BLOCKS = 256;
+
 template <bool F16>
-__global__ __launch_bounds__(256) void norm_bwd_kernel(const NormBwdParams p) {
+__global__ __launch_bounds__(NORM_THREADS) void norm_bwd_kernel(const NormBwdParams p) {
     using E = Elt<F16>;
-    __shared__ float fold[16][16][8];
+    __shared__ float fold[NORM_ROWS][16][8];
     const int sub = threadIdx.x & 15, grp = threadIdx.x >> 4;
     const int64_t nrows = (int64_t)p.M * p.heads;
     const u32x4 wu = *reinterpret_cast<const u32x4*>(p.w + sub * 8);
@@ -492,34 +497,47 @@ __global__ __launch_bounds__(256) void norm_bwd_kernel(const NormBwdParams p) {
     for (int j = 0; j < 4; ++j) { w[2 * j] = E::lo(wu[j]); w[2 * j + 1] = E::hi(wu[j]); }
 #pragma unroll
     for (int j = 0; j < 8; ++j) dwp[j] = 0.f;
-    for (int64_t row = (int64_t)blockIdx.x * 16 + grp; row < nrows; row += (int64_t)gridDim.x * 16) {
-        const int64_t m = row / p.heads;
-        const int h = (int)(row % p.heads);
-        const u32x4 du = *reinterpret_cast<const u32x4*>(p.dy + m * p.ldy + h * 128 + sub * 8);
-        const u32x4 xu = *reinterpret_cast<const u32x4*>(p.x + m * p.ldx + h * 128 + sub * 8);
-        const float r = p.rstd[row];
-        float gg[8], xh[8], c = 0.f;
+    const int64_t stride = (int64_t)gridDim.x * NORM_ROWS;
+    for (int64_t row0 = (int64_t)blockIdx.x * NORM_ROWS + grp; row0 < nrows; row0 += 2 * stride) {
+        u32x4 du[2], xu[2];
+        float r[2];
+        uint16_t* out[2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float d0 = E::lo(du[j]), d1 = E::hi(du[j]);
-            xh[2 * j] = E::lo(xu[j]) * r;
-            xh[2 * j + 1] = E::hi(xu[j]) * r;
-            gg[2 * j] = d0 * w[2 * j];
-            gg[2 * j + 1] = d1 * w[2 * j + 1];
-            const uint32_t xb = E::pack(xh[2 * j], xh[2 * j + 1]);
-            dwp[2 * j] = fmaf(d0, E::lo(xb), dwp[2 * j]);
-            dwp[2 * j + 1] = fmaf(d1, E::hi(xb), dwp[2 * j + 1]);
+        for (int k = 0; k < 2; ++k) {
+            const bool ok = row0 + k * stride < nrows;          // the lanes of a row agree
+            const int64_t row = ok ? row0 + k * stride : row0;
+            const int64_t m = row / p.heads;
+            const int h = (int)(row % p.heads);
+            du[k] = ldg16(p.dy + m * p.ldy + h * 128 + sub * 8, ok);    // zero: adds nothing to dw
+            xu[k] = ldg16(p.x + m * p.ldx + h * 128 + sub * 8, ok);
+            r[k] = p.rstd[row];
+            out[k] = ok ? p.dx + m * p.lddx + h * 128 + sub * 8 : nullptr;
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) c = fmaf(gg[j], xh[j], c);
+        for (int k = 0; k < 2; ++k) {
+            float gg[8], xh[8], c = 0.f;
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) c += __shfl_xor(c, o);
-        c *= 1.f / 128.f;
-        u32x4 out;
+            for (int j = 0; j < 4; ++j) {
+                const float d0 = E::lo(du[k][j]), d1 = E::hi(du[k][j]);
+                xh[2 * j] = E::lo(xu[k][j]) * r[k];
+                xh[2 * j + 1] = E::hi(xu[k][j]) * r[k];
+                gg[2 * j] = d0 * w[2 * j];
+                gg[2 * j + 1] = d1 * w[2 * j + 1];
+                const uint32_t xb = E::pack(xh[2 * j], xh[2 * j + 1]);
+                dwp[2 * j] = fmaf(d0, E::lo(xb), dwp[2 * j]);
+                dwp[2 * j + 1] = fmaf(d1, E::hi(xb), dwp[2 * j + 1]);
+            }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            out[j] = E::pack(r * (gg[2 * j] - xh[2 * j] * c), r * (gg[2 * j + 1] - xh[2 * j + 1] * c));
-        *reinterpret_cast<u32x4*>(p.dx + m * p.lddx + h * 128 + sub * 8) = out;
+            for (int j = 0; j < 8; ++j) c = fmaf(gg[j], xh[j], c);
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) c += __shfl_xor(c, o);
+            c *= 1.f / 128.f;
+            u32x4 u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                u[j] = E::pack(r[k] * (gg[2 * j] - xh[2 * j] * c), r[k] * (gg[2 * j + 1] - xh[2 * j + 1] * c));
+            if (out[k]) *reinterpret_cast<u32x4*>(out[k]) = u;
+        }
     }
     if (!p.dw) return;
 #pragma unroll
@@ -528,8 +546,8 @@ __global__ __launch_bounds__(256) void norm_bwd_kernel(const NormBwdParams p) {
     if (threadIdx.x < 128) {
         const int s2 = threadIdx.x >> 3, j = threadIdx.x & 7;
         float t = 0.f;
-#pragma unroll
-        for (int gi = 0; gi < 16; ++gi) t += fold[gi][s2][j];
+#pragma unroll 8
+        for (int gi = 0; gi < NORM_ROWS; ++gi) t += fold[gi][s2][j];
         unsafeAtomicAdd(p.dw + threadIdx.x, t);
     }
 }
@@ -605,9 +623,9 @@ hipError_t launch_bias_interval(const BiasHullParams& p, hipStream_t st) {
 hipError_t launch_norm_bwd(const NormBwdParams& p, hipStream_t st) {
     const int64_t rows = (int64_t)p.M * p.heads;
     if (rows == 0) return hipSuccess;
-    const int grid = (int)std::min<int64_t>((rows + 15) / 16, 2048);
-    if (p.f16) return launch1(norm_bwd_kernel<true>, dim3(grid), dim3(256), st, p);
-    else return launch1(norm_bwd_kernel<false>, dim3(grid), dim3(256), st, p);
+    const dim3 grid((unsigned)std::min<int64_t>((rows + NORM_ROWS - 1) / NORM_ROWS, NORM_BLOCKS));
+    if (p.f16) return launch1(norm_bwd_kernel<true>, grid, dim3(NORM_THREADS), st, p);
+    else return launch1(norm_bwd_kernel<false>, grid, dim3(NORM_THREADS), st, p);
 }
 
 hipError_t launch_cast(const CastParams& p, hipStream_t st) {
