@@ -255,7 +255,7 @@ def _cap_windows(windows, nbytes_of_rows, cap):
 def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engine,
                    bias_func=None, local_bias_args=[], remote_bias_args=[], no_overlap=False, *,
                    rounds: Optional[int] = None, mask: Optional[Mask] = None, batched: bool = False,
-                   streams: int = 1):
+                   streams: int = 1, _dq_like_q: bool = False):
     """Returns (dq, dk, dv) like the reference (attn.py:545): dq [B,Hq,Lq,D];
     dk, dv [B,Hkv,Lkv,D]-shaped views of [B,Lkv,Hkv,D] memory, at the Hkv heads
     k and v came in with.  `o` and `L` are the finally merged forward results;
@@ -265,7 +265,8 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
     complete after that round (fp32 sum over all local tokens, rounded once).
     `backward_engine`, `comm_mode`, `no_overlap` are accepted and ignored.  `streams` as in
     `_attn_forward`; every stream sums its rounds' dK, dV in an fp32 accumulator of its own and
-    the accumulators are added before the one rounding."""
+    the accumulators are added before the one rounding.  `_dq_like_q`: dq in q's memory order (a projection's
+    backward then reads it as it lies) instead of contiguous."""
     _reject_unsupported(causal)
     D_in = q.shape[-1]
     q_, k_, v_, o_, do_ = (_usable(_pad_head_dim(t)) for t in (q, k, v, o, do))
@@ -281,7 +282,7 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
     L_ = L.to(torch.float32).reshape(B * Hq, Lq).contiguous()
 
     delta = workspace("bwd_delta", (B * Hq, Lq), torch.float32, dev)
-    dq = torch.empty(B, Hq, Lq, D, dtype=q_.dtype, device=dev)
+    dq = torch.empty_like(q_) if _dq_like_q else torch.empty(B, Hq, Lq, D, dtype=q_.dtype, device=dev)
     dk = torch.empty(B, Lkv, Hkv, D, dtype=q_.dtype, device=dev).transpose(1, 2)
     dv = torch.empty(B, Lkv, Hkv, D, dtype=q_.dtype, device=dev).transpose(1, 2)
 

@@ -13,6 +13,8 @@ that flows into the visual hidden states (dX_vis) and the projection weights.
 """
 from __future__ import annotations
 
+import threading
+from contextlib import contextmanager
 from typing import Callable, Optional
 
 import torch
@@ -21,6 +23,23 @@ from . import ops
 from ._lib import LvxError
 from .attn import Mask, _attn_backward, _attn_forward, _reject_unsupported
 from .async_communication import reset_global_memory_buffer
+
+
+# What the projections below keep from forward to backward.  Nothing but their inputs in general; but a
+# run whose gradient follows at once - the second run of run_function, inside the attention's backward
+# - keeps the raw projection and the norm's r, which backward would otherwise form by running the same
+# GEMM a third time (230 us of a 2700 us step for K and V of 2 x 6404 tokens, 115 us for Q).
+_this_run = threading.local()
+
+
+@contextmanager
+def _gradient_follows():
+    before = getattr(_this_run, "gradient_follows", False)
+    _this_run.gradient_follows = True
+    try:
+        yield
+    finally:
+        _this_run.gradient_follows = before
 
 
 def create_attention_class_save_qkv(attention_mode: str = "lv_xattn", no_overlap: bool = False,
@@ -168,11 +187,12 @@ def create_attention_class(attention_mode: str = "lv_xattn", no_overlap: bool = 
         def backward(ctx, do):
             x, o, L = ctx.saved_tensors
             x_ = x.detach().requires_grad_(x.requires_grad)
-            with torch.enable_grad():
+            with torch.enable_grad(), _gradient_follows():
                 q, k, v = ctx.run_function(x_, get_global_cross_attention_states())
             sm_scale = q.size(-1) ** -0.5
             dq, dk, dv = _attn_backward(do, q.detach(), k.detach(), v.detach(), o, L, ctx.causal, sm_scale, None,
-                                        "flash", None, [], [], no_overlap, rounds=rounds, batched=batched)
+                                        "flash", None, [], [], no_overlap, rounds=rounds, batched=batched,
+                                        _dq_like_q=True)
             outs = [(t, g) for t, g in ((q, dq), (k, dk), (v, dv)) if t.requires_grad]
             if outs:
                 torch.autograd.backward([t for t, _ in outs], [g for _, g in outs])
@@ -217,16 +237,21 @@ def create_kv_projection_class(w_in_major: bool = True, weight_grads: bool = Tru
 
     The visual side of the reference's `project` (test_llama3.py:395-398, 418) as one autograd
     function over the fused GEMMs: K = k_norm(X_vis W_k), V = X_vis W_v.  Nothing but the inputs
-    is kept; backward re-runs the projection for the raw K and its r when there is a norm, goes
-    back through the norm, then dX_vis = dK W_k^T + dV W_v^T and (weight_grads) dW_k, dW_v and
+    is kept (see _gradient_follows); backward re-runs the projection for the raw K and its r when there
+    is a norm, goes back through the norm, then dX_vis = dK W_k^T + dV W_v^T and (weight_grads) dW_k, dW_v and
     the norm weight's gradient."""
 
     class _kv_projection(torch.autograd.Function):
         @staticmethod
         def forward(ctx, x_vis, w_k, w_v, n_kv_heads, k_norm_weight=None, eps=1e-5):
             ctx.has_norm = k_norm_weight is not None
-            ctx.save_for_backward(x_vis, w_k, w_v, *([k_norm_weight] if ctx.has_norm else []))
             ctx.n_kv_heads, ctx.eps = n_kv_heads, eps
+            if ctx.has_norm and getattr(_this_run, "gradient_follows", False):
+                k, v, k_raw, k_rstd = ops.kv_proj(x_vis, w_k, w_v, n_kv_heads, w_in_major, k_norm_weight=k_norm_weight,
+                                                  eps=eps, for_backward=True)
+                ctx.save_for_backward(x_vis, w_k, w_v, k_norm_weight, k_raw, k_rstd)
+                return k, v
+            ctx.save_for_backward(x_vis, w_k, w_v, *([k_norm_weight] if ctx.has_norm else []))
             return ops.kv_proj(x_vis, w_k, w_v, n_kv_heads, w_in_major, k_norm_weight=k_norm_weight, eps=eps)
 
         @staticmethod
@@ -239,8 +264,11 @@ def create_kv_projection_class(w_in_major: bool = True, weight_grads: bool = Tru
 
             dk, dv = token_major(dk), token_major(dv)
             if ctx.has_norm:
-                _, _, k_raw, k_rstd = ops.kv_proj(x_vis, w_k, w_v, ctx.n_kv_heads, w_in_major, k_norm_weight=rest[0],
-                                                  eps=ctx.eps, for_backward=True)
+                if len(rest) == 3:
+                    k_raw, k_rstd = rest[1:]
+                else:
+                    _, _, k_raw, k_rstd = ops.kv_proj(x_vis, w_k, w_v, ctx.n_kv_heads, w_in_major, k_norm_weight=rest[0],
+                                                      eps=ctx.eps, for_backward=True)
                 dk, dwn = ops.k_norm_bwd(dk, k_raw, k_rstd, rest[0], want_dw=weight_grads)
                 if dwn is not None:
                     dwn = dwn.to(rest[0].dtype)
@@ -259,21 +287,25 @@ def create_q_projection_class(w_in_major: bool = True, weight_grads: bool = True
     The text side of the reference's `project` (test_llama3.py:390-393),
     Q = q_norm(X W_q), with the reference's recompute discipline
     (test_llama3.py:184-243: only the layer input is kept): forward saves
-    (x, w_q, norm weight); backward re-runs the fused GEMM to get the raw
+    (x, w_q, norm weight; see _gradient_follows); backward re-runs the fused GEMM to get the raw
     projection and r, goes back through the norm, then dX = dQ_raw W_q^T and
     dW_q = X^T dQ_raw."""
 
     class _q_projection(torch.autograd.Function):
         @staticmethod
         def forward(ctx, x, w_q, n_heads, q_norm_weight, eps=1e-5):
-            ctx.save_for_backward(x, w_q, q_norm_weight)
             ctx.n_heads, ctx.eps = n_heads, eps
+            if getattr(_this_run, "gradient_follows", False):
+                q, q_raw, rstd = ops.q_proj(x, w_q, n_heads, w_in_major, q_norm_weight, eps, for_backward=True)
+                ctx.save_for_backward(x, w_q, q_norm_weight, q_raw, rstd)
+                return q
+            ctx.save_for_backward(x, w_q, q_norm_weight)
             return ops.q_proj(x, w_q, n_heads, w_in_major, q_norm_weight, eps)
 
         @staticmethod
         def backward(ctx, dq):
-            x, w_q, wn = ctx.saved_tensors
-            _, q_raw, rstd = ops.q_proj(x, w_q, ctx.n_heads, w_in_major, wn, ctx.eps, for_backward=True)
+            x, w_q, wn, *kept = ctx.saved_tensors
+            q_raw, rstd = kept if kept else ops.q_proj(x, w_q, ctx.n_heads, w_in_major, wn, ctx.eps, for_backward=True)[1:]
             dq_tm = dq if dq.transpose(1, 2).is_contiguous() else dq.transpose(1, 2).contiguous().transpose(1, 2)
             dq_raw, dwn = ops.k_norm_bwd(dq_tm, q_raw, rstd, wn, want_dw=weight_grads)
             dx, dw = ops.q_proj_bwd(x, dq_raw, w_q, w_in_major, want_dw=weight_grads)
