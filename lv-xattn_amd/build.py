@@ -60,8 +60,7 @@ def _run(cmd, verbose):
 GENERATED = [*[("gen_fwd_loop_wide.py", [t, d], f"lvx_fwd_loop_wide_{t}_{d}.inc") for t in ("bf16", "f16") for d in ("128", "64")],
              ("gen_bwd_loop.py", ["p"], "lvx_bwd_loop_p.inc"),
              ("gen_bwd_loop.py", ["d"], "lvx_bwd_loop_d.inc"),
-             ("gen_gemm_loop.py", ["bp"], "lvx_gemm_loop_bp.inc"),
-             ("gen_gemm_loop.py", ["bt"], "lvx_gemm_loop_bt.inc")]
+             *[("gen_gemm_loop.py", [x, y, n], f"lvx_gemm_loop_{x}{y}_{n}.inc") for x, y in ("pp", "pt", "tt") for n in ("256", "128")]]
 
 
 def generate() -> None:

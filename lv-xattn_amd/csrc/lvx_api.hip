@@ -95,6 +95,20 @@ int scratch_on_current_device(void** out) {
 }
 }  // namespace
 
+namespace lvx {
+int cu_count() {
+    static int cached[MAX_DEVICES];          // 0: not asked yet
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 256;
+    int n = __atomic_load_n(&cached[dev], __ATOMIC_RELAXED);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        __atomic_store_n(&cached[dev], n, __ATOMIC_RELAXED);
+    }
+    return n;
+}
+}  // namespace lvx
+
 extern "C" {
 
 int lvx_version(void) { return LVX_VERSION; }
@@ -121,8 +135,6 @@ size_t lvx_fwd_workspace_bytes(const lvx_attn_shape* s, int32_t row_count, int32
     const size_t rows = (size_t)s->B * s->Hq * row_count;
     return (size_t)kv_splits * rows * (s->D * sizeof(uint16_t) + sizeof(float));
 }
-
-static int cu_count();
 
 // Keys per split: whole tiles (pieces) of the form's kernel.
 static int fwd_split_len(const lvx_attn_shape* s, FwdForm form, int splits) {
@@ -454,19 +466,6 @@ int lvx_bwd_preprocess(const lvx_attn_shape* s, const lvx_tensor* o, const lvx_t
 // visits only the row tiles that see it; half of them is assumed); given at least two per CU the
 // dispatcher fills the tail by itself and rounds(S) is the plain quotient: splitting then
 // rarely pays (cfg4: 0.98 ms with 5 splits, 0.86 ms with none).
-// CUs of the device that is current (the one the caller's stream belongs to), asked for once per device
-static int cu_count() {
-    static int cached[MAX_DEVICES];          // 0: not asked yet
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 256;
-    int n = __atomic_load_n(&cached[dev], __ATOMIC_RELAXED);
-    if (n == 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        __atomic_store_n(&cached[dev], n, __ATOMIC_RELAXED);
-    }
-    return n;
-}
-
 // How the token blocks of a launch are handed to work-groups (see bwd_kernel): per XCD, the first
 // `whole` blocks get one work-group each, the next `mid` blocks `splits` work-groups each and the
 // others `splits2` each.

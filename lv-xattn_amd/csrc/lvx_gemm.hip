@@ -31,9 +31,6 @@ namespace lvx {
 
 namespace {
 
-// registers the hand-scheduled loop uses besides its operands (see gen_gemm_loop.py)
-#define LVX_GEMM_LOOP_CLOBBERS "v128", "v129", "v130", "v131", "v132", "v133", "v134", "v135", "v136", "v137", "v138", "v139", "v140", "v141", "v142", "v143", "v144", "v145", "v146", "v147", "v148", "v149", "v150", "v151", "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v160", "v161", "v162", "v163", "v164", "v165", "v166", "v167", "v168", "v169", "v170", "v171", "v172", "v173", "v174", "v175", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", "v187", "v188", "v189", "v190", "v191", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v200", "v201", "v202", "v203", "v204", "v205", "v206", "v207", "v208", "v209", "v210", "v211", "v212", "v213", "v214", "v215", "v216", "v217", "v218", "v219", "v220", "v221", "v222", "v223"
-
 constexpr int BK = 32;                 // contraction depth of one stage
 __device__ uint32_t zero_chunk[4];     // source of the chunks past the end of a contraction
 
@@ -225,53 +222,6 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
 
-    // The 256 x 256 bf16 tile with A stored [m][k] and whole stages only (the K/V projection and
-    // dX_vis) takes the hand-scheduled loop of gen_gemm_loop.py, one run per contraction segment; every
-    // other case takes the ping-pong loop below.
-    constexpr bool FAST = !F16 && !A_MCONTIG && GM == 2 && GN == 4 && WM == 4 && WN == 2 && NS == 4;
-    if constexpr (FAST) {
-        const int st0 = klen0 / BK, st1 = klen1 / BK;
-        const bool whole = klen0 % BK == 0 && klen1 % BK == 0 && st0 % 4 == 0 && st1 % 4 == 0 && st0 >= 8 &&
-                           (st1 == 0 || st1 >= 8);
-        if (whole) {
-            uint32_t ra[4], rb[4];
-            ra[0] = lds0 + rda[0]; ra[1] = lds0 + rda[1]; ra[2] = ra[0] + 65536u; ra[3] = ra[1] + 65536u;
-            rb[0] = lds0 + rdb[0]; rb[1] = lds0 + rdb[1]; rb[2] = rb[0] + 65536u; rb[3] = rb[1] + 65536u;
-            const uint32_t lds_w = uniform32(lds0 + (uint32_t)wave * 1024u);
-            for (int sg = 0; sg < (st1 ? 2 : 1); ++sg) {
-                const int nst = sg ? st1 : st0;
-                const char* ap = uniform_ptr(abase[sg] + (int64_t)(sg ? 0 : s_lo) * a_kstride);
-                const char* bp = uniform_ptr(bbase[sg] + (int64_t)(sg ? 0 : s_lo) * b_kstride);
-                int trips = uniform32(nst / 4), todo = uniform32(nst);
-                __syncthreads();     // the stage buffers are free
-                if (B_NCONTIG) {
-                    asm volatile(
-#include "lvx_gemm_loop_bt.inc"
-                        : "+{v[0:15]}"(acc[0][0]), "+{v[16:31]}"(acc[0][1]), "+{v[32:47]}"(acc[0][2]), "+{v[48:63]}"(acc[0][3]),
-                          "+{v[64:79]}"(acc[1][0]), "+{v[80:95]}"(acc[1][1]), "+{v[96:111]}"(acc[1][2]), "+{v[112:127]}"(acc[1][3]),
-                          "+{s[44:45]}"(ap), "+{s[46:47]}"(bp), "+{s51}"(trips), "+{s52}"(todo)
-                        : "{v224}"(ra[0]), "{v225}"(ra[1]), "{v226}"(ra[2]), "{v227}"(ra[3]),
-                          "{v228}"(rb[0]), "{v229}"(rb[1]), "{v230}"(rb[2]), "{v231}"(rb[3]),
-                          "{v232}"(voff[0]), "{v233}"(voff[1]), "{v234}"(voff[2]), "{v235}"(voff[3]),
-                          "{s48}"(uniform32((uint32_t)a_kstride)), "{s49}"(uniform32((uint32_t)b_kstride)), "{s50}"(lds_w)
-                        : "memory", "vcc", "scc", "m0", "s53", "s54", "s55", LVX_GEMM_LOOP_CLOBBERS);
-                } else {
-                    asm volatile(
-#include "lvx_gemm_loop_bp.inc"
-                        : "+{v[0:15]}"(acc[0][0]), "+{v[16:31]}"(acc[0][1]), "+{v[32:47]}"(acc[0][2]), "+{v[48:63]}"(acc[0][3]),
-                          "+{v[64:79]}"(acc[1][0]), "+{v[80:95]}"(acc[1][1]), "+{v[96:111]}"(acc[1][2]), "+{v[112:127]}"(acc[1][3]),
-                          "+{s[44:45]}"(ap), "+{s[46:47]}"(bp), "+{s51}"(trips), "+{s52}"(todo)
-                        : "{v224}"(ra[0]), "{v225}"(ra[1]), "{v226}"(ra[2]), "{v227}"(ra[3]),
-                          "{v228}"(rb[0]), "{v229}"(rb[1]), "{v230}"(rb[2]), "{v231}"(rb[3]),
-                          "{v232}"(voff[0]), "{v233}"(voff[1]), "{v234}"(voff[2]), "{v235}"(voff[3]),
-                          "{s48}"(uniform32((uint32_t)a_kstride)), "{s49}"(uniform32((uint32_t)b_kstride)), "{s50}"(lds_w)
-                        : "memory", "vcc", "scc", "m0", "s53", "s54", "s55", LVX_GEMM_LOOP_CLOBBERS);
-                }
-            }
-            goto epilogue;
-        }
-    }
-
     // prologue: stages 0 .. NS-2 in flight, stage 0 landed
 #pragma unroll
     for (int s = 0; s < NS - 1; ++s)
@@ -316,7 +266,6 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     }
     if (set == 0) phase_barrier();
 
-epilogue:
     // C^T tile: accumulator rows = n, cols = m
     if (nks > 1) {   // partial tile of a split contraction: fp32, into this split's slice
         float* const C32 = p.c32 + ksp * p.c32_split + (int64_t)z * p.c32_batch;
@@ -496,6 +445,245 @@ epilogue:
     }
 }
 
+// registers the hand-scheduled tile uses besides its operands (see gen_gemm_loop.py)
+#define LVX_GEMM_TILE_CLOBBERS "memory", "vcc", "scc", "m0", "v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", "v8", "v9", "v10", "v11", "v12", "v13", "v14", "v15", "v16", "v17", "v18", "v19", "v20", "v21", "v22", "v23", "v24", "v25", "v26", "v27", "v28", "v29", "v30", "v31", "v32", "v33", "v34", "v35", "v36", "v37", "v38", "v39", "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "v121", "v122", "v123", "v124", "v125", "v126", "v127", "v128", "v129", "v130", "v131", "v132", "v133", "v134", "v135", "v136", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191", "a192", "a193", "a194", "a195", "a196", "a197", "a198", "a199", "a200", "a201", "a202", "a203", "a204", "a205", "a206", "a207", "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", "a222", "a223", "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
+
+// One operand's part of a stage of gemm_tile_kernel: ROWS rows x 64 k in pieces of 1 KiB (what one load of a
+// wave fills).
+//   !TRANS (memory [row][k]): LDS row r at r * 128 B; its 16-byte chunk c (k = 8c .. 8c+7) sits at position
+//       c ^ ((r >> 1) & 7): of 16 consecutive rows the eight even and the eight odd ones, which share
+//       the 256 bytes of a pass over the banks pairwise, each land in eight different positions
+//    TRANS (memory [k][row]): LDS k-row at k * ROWS * 2 B; its chunk q (rows 8q .. 8q+7) at q ^ ((k & 3) << 2)
+constexpr int TK = 64;                 // contraction depth of one stage
+template <bool TRANS, int ROWS>
+struct TileOperand {
+    static constexpr int BYTES = ROWS * TK * 2, PIECES = BYTES / 1024, LPR = ROWS / 8;
+    // what lane `lane` fetches of piece `ch`: byte offset from row r0 (column r0) of the operand, clamped to
+    // its last row, and the k position inside the stage
+    __device__ __forceinline__ static uint32_t src(int ch, int lane, int r0, int R, int64_t ld, int& kpos) {
+        if (!TRANS) {
+            const int row = 8 * ch + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+            kpos = c * 8;
+            return (uint32_t)(min(r0 + row, R - 1) - r0) * (uint32_t)ld * 2u + (uint32_t)c * 16u;
+        }
+        const int k = ch * (64 / LPR) + lane / LPR, q = (lane % LPR) ^ ((k & 3) << 2);
+        kpos = k;
+        return (uint32_t)k * (uint32_t)ld * 2u + (uint32_t)(min(r0 + q * 8, R - 8) - r0) * 2u;
+    }
+    // LDS byte offsets of a wave's operand reads, first 32-row tile j0: !TRANS per k-step (add tile * 4096),
+    // TRANS per tile (add k-step * 32 * ROWS)
+    __device__ __forceinline__ static void read_offsets(uint32_t (&rd)[4], int j0, int lane) {
+        const int l32 = lane & 31, g = lane >> 5, r = (lane & 15) >> 2, t = lane & 3, u = (lane >> 4) & 1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            rd[i] = TRANS ? (uint32_t)((8 * g + r) * ROWS * 2 + 64 * ((j0 + i) ^ r) + (2 * u + (t >> 1)) * 16 + (t & 1) * 8)
+                          : (uint32_t)(j0 * 4096 + l32 * 128 + (((2 * i + g) ^ ((l32 >> 1) & 7)) << 4));
+    }
+};
+
+// The 256 x TN tile of the projections and their gradients: four waves of 128 x TN / 2 in one generated
+// statement (gen_gemm_loop.py), then the C tile, 16-bit in LDS by then, leaves as whole row segments -
+// through the RMS norm where problem 0 has one (16 lanes hold a head's 128 columns of a row).
+// Bound by the matrix pipe and the power it may draw: MFMAs alone on N(0, 1) data sustain 1800 TFLOP/s on the
+// chip, this kernel 1341 (65536 x 4096 x 1024 twice, W [N][K]; 1215 with eight waves of 128 x 64 and stages
+// of 32).  us before and after: that 905 -> 820; 12808 rows 183 -> 176; 2046 x 4096 x 4096 77 -> 60; the
+// weight gradients, until then compiler-scheduled, 12808 rows 258 -> 168 and 6404 rows 134 -> 88.
+template <bool A_T, bool B_T, int TN, bool F16>
+__global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
+    using E = Elt<F16>;
+    constexpr int TM = 256, WM = 4, WN = TN / 64;
+    using RA = TileOperand<A_T, TM>;
+    using RB = TileOperand<B_T, TN>;
+    constexpr int NSA = 3, NSB = TN == 256 ? 2 : 3, NLA = RA::PIECES / 4, NLB = RB::PIECES / 4, NL = NLA + NLB;
+    __shared__ __attribute__((aligned(1024))) char lds[NSA * RA::BYTES + NSB * RB::BYTES];
+    static_assert(sizeof(lds) >= TM * TN * 2, "the C tile takes the stages' place");
+
+    const int wid = xcd_remap(blockIdx.x, p.total_wg);
+    if (wid >= p.total_wg) return;
+    const int tn = wid % p.tiles_n, t1 = wid / p.tiles_n;
+    // the problems of an M tile side by side: they share an operand (K and V the visual states), which then
+    // is read from HBM once
+    const int prob = t1 % p.nprob, tm = t1 / p.nprob;
+    const GemmProblem& pr = p.prob[prob];
+    const int m0 = tm * TM, n0 = tn * TN;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wm = wave & 1, wn = wave >> 1;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+    const int64_t lda = pr.lda[0], ldb = pr.ldb[0];
+    const int st0 = (pr.K[0] + TK - 1) / TK, nst = st0 + (pr.nseg > 1 ? st0 : 0);      // both segments have one length
+    const int tail = pr.K[0] % TK;
+
+    // This wave's pieces of a stage: offsets from the tile's first row (column) of the operand.  In the last
+    // stage, 16-byte pieces past the end of a contraction that is contiguous in memory are sent out of
+    // the descriptor's range; where it is not contiguous the range itself ends with it.
+    uint32_t voff[16], vtail[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        if (j >= NL) { voff[j] = vtail[j] = 0; continue; }
+        int kpos;
+        const int ch = wave + 4 * (j < NLA ? j : j - NLA);
+        voff[j] = j < NLA ? RA::src(ch, lane, m0, p.M_ld, lda, kpos) : RB::src(ch, lane, n0, p.N, ldb, kpos);
+        vtail[j] = tail && kpos >= tail && !(j < NLA ? A_T : B_T) ? 0x80000000u : voff[j];
+        if (nst == 1) voff[j] = vtail[j];
+    }
+    typedef __attribute__((ext_vector_type(4))) uint32_t srd_t;
+    auto descriptor = [&](const uint16_t* base, int64_t ld, bool trans) {
+        const uint64_t addr = (uint64_t)(uintptr_t)base;
+        srd_t d;
+        d[0] = uniform32((uint32_t)addr);
+        d[1] = uniform32((uint32_t)(addr >> 32) & 0xffffu);
+        d[2] = uniform32(trans ? (uint32_t)((uint64_t)pr.K[0] * (uint64_t)ld * 2u) : 0x7fffffffu);
+        d[3] = 0x00020000u;
+        return d;
+    };
+    auto a_base = [&](int i) { return pr.A[i] + (A_T ? (int64_t)m0 : (int64_t)m0 * lda); };
+    auto b_base = [&](int i) { return pr.Bm[i] + (B_T ? (int64_t)n0 : (int64_t)n0 * ldb); };
+    srd_t sa = descriptor(a_base(0), lda, A_T), sb = descriptor(b_base(0), ldb, B_T);
+    const int second = pr.nseg > 1 ? 1 : 0;
+    const uint64_t a1 = (uint64_t)uniform64((int64_t)(uintptr_t)a_base(second) & 0xffffffffffffll);
+    const uint64_t b1 = (uint64_t)uniform64((int64_t)(uintptr_t)b_base(second) & 0xffffffffffffll);
+    const uint32_t a_step = (uint32_t)(A_T ? lda * TK * 2 : TK * 2), b_step = (uint32_t)(B_T ? ldb * TK * 2 : TK * 2);
+
+    uint32_t rda[4], rdb[4], ra[12], rb[12];
+    RA::read_offsets(rda, WM * wm, lane);
+    RB::read_offsets(rdb, WN * wn, lane);
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+        ra[i] = lds0 + rda[i & 3] + (i >> 2) * RA::BYTES;
+        rb[i] = lds0 + NSA * RA::BYTES + rdb[i & 3] + min(i >> 2, NSB - 1) * RB::BYTES;
+    }
+    // The C tile in LDS: 16-byte chunk c of row r at position c ^ (r mod chunks per row), its two 8-byte halves
+    // exchanged in rows where bits 3 and 4 differ: the 8-byte writes of 32 rows and the 16-byte reads of
+    // whole rows are both conflict-free.
+    constexpr int CPR = TN / 8;
+    const uint32_t ep = lds0 + (uint32_t)((128 * wm + l32) * (TN * 2) + (((4 * WN * wn) ^ (l32 & (CPR - 1))) << 4) +
+                                          ((g ^ ((l32 >> 3) & 1) ^ (l32 >> 4)) << 3));
+    uint32_t left = uniform32((uint32_t)nst), ahead = uniform32((uint32_t)(nst - 1)), soa = 0, sob = 0;
+    uint32_t to_second = uniform32((uint32_t)(pr.nseg > 1 ? st0 : 0)), ahead_b = ahead, to_second_b = to_second;
+#define LVX_GEMM_TILE_OPERANDS \
+    : "+{v64}"(voff[0]), "+{v65}"(voff[1]), "+{v66}"(voff[2]), "+{v67}"(voff[3]), "+{v68}"(voff[4]), "+{v69}"(voff[5]), \
+      "+{v70}"(voff[6]), "+{v71}"(voff[7]), "+{v72}"(voff[8]), "+{v73}"(voff[9]), "+{v74}"(voff[10]), "+{v75}"(voff[11]), \
+      "+{v76}"(voff[12]), "+{v77}"(voff[13]), "+{v78}"(voff[14]), "+{v79}"(voff[15]), "+{s[40:43]}"(sa), "+{s[44:47]}"(sb), \
+      "+{s51}"(left), "+{s52}"(ahead), "+{s53}"(soa), "+{s54}"(sob), "+{s55}"(to_second), "+{s60}"(ahead_b), "+{s61}"(to_second_b) \
+    : "{v80}"(vtail[0]), "{v81}"(vtail[1]), "{v82}"(vtail[2]), "{v83}"(vtail[3]), "{v84}"(vtail[4]), "{v85}"(vtail[5]), \
+      "{v86}"(vtail[6]), "{v87}"(vtail[7]), "{v88}"(vtail[8]), "{v89}"(vtail[9]), "{v90}"(vtail[10]), "{v91}"(vtail[11]), \
+      "{v92}"(vtail[12]), "{v93}"(vtail[13]), "{v94}"(vtail[14]), "{v95}"(vtail[15]), "{v96}"(ra[0]), "{v97}"(ra[1]), \
+      "{v98}"(ra[2]), "{v99}"(ra[3]), "{v100}"(ra[4]), "{v101}"(ra[5]), "{v102}"(ra[6]), "{v103}"(ra[7]), \
+      "{v104}"(ra[8]), "{v105}"(ra[9]), "{v106}"(ra[10]), "{v107}"(ra[11]), "{v108}"(rb[0]), "{v109}"(rb[1]), \
+      "{v110}"(rb[2]), "{v111}"(rb[3]), "{v112}"(rb[4]), "{v113}"(rb[5]), "{v114}"(rb[6]), "{v115}"(rb[7]), \
+      "{v116}"(rb[8]), "{v117}"(rb[9]), "{v118}"(rb[10]), "{v119}"(rb[11]), "{v120}"(ep), \
+      "{s48}"(uniform32(a_step)), "{s49}"(uniform32(b_step)), "{s50}"(uniform32(lds0 + (uint32_t)wave * 1024u)),  \
+      "{s[56:57]}"(a1), "{s[58:59]}"(b1)                                                                         \
+    : LVX_GEMM_TILE_CLOBBERS
+    // one statement per layout, width and type; the text takes the instruction names from these macros
+    if constexpr (!F16) {
+#define LVX_GEMM_MFMA "v_mfma_f32_32x32x16_bf16"
+#define LVX_GEMM_CVT "v_cvt_pk_bf16_f32"
+        if constexpr (!A_T && !B_T && TN == 256) {
+            asm volatile(
+#include "lvx_gemm_loop_pp_256.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && !B_T && TN == 128) {
+            asm volatile(
+#include "lvx_gemm_loop_pp_128.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && B_T && TN == 256) {
+            asm volatile(
+#include "lvx_gemm_loop_pt_256.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && B_T && TN == 128) {
+            asm volatile(
+#include "lvx_gemm_loop_pt_128.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (A_T && B_T && TN == 256) {
+            asm volatile(
+#include "lvx_gemm_loop_tt_256.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (A_T && B_T && TN == 128) {
+            asm volatile(
+#include "lvx_gemm_loop_tt_128.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+#undef LVX_GEMM_MFMA
+#undef LVX_GEMM_CVT
+    } else {
+#define LVX_GEMM_MFMA "v_mfma_f32_32x32x16_f16"
+#define LVX_GEMM_CVT "v_cvt_pk_f16_f32"
+        if constexpr (!A_T && !B_T && TN == 256) {
+            asm volatile(
+#include "lvx_gemm_loop_pp_256.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && !B_T && TN == 128) {
+            asm volatile(
+#include "lvx_gemm_loop_pp_128.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && B_T && TN == 256) {
+            asm volatile(
+#include "lvx_gemm_loop_pt_256.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && B_T && TN == 128) {
+            asm volatile(
+#include "lvx_gemm_loop_pt_128.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (A_T && B_T && TN == 256) {
+            asm volatile(
+#include "lvx_gemm_loop_tt_256.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (A_T && B_T && TN == 128) {
+            asm volatile(
+#include "lvx_gemm_loop_tt_128.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+#undef LVX_GEMM_MFMA
+#undef LVX_GEMM_CVT
+    }
+    __syncthreads();
+
+    uint16_t* const C = pr.C;
+    const bool norm = p.norm_w && prob == 0;
+    const int cc = tid % CPR, n = n0 + cc * 8;
+    const u32x4 wt = norm && n < p.N ? *reinterpret_cast<const u32x4*>(p.norm_w + (n & 127)) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll 4
+    for (int i = 0; i < TM * CPR / 256; ++i) {
+        const int row = i * (256 / CPR) + tid / CPR, m = m0 + row;
+        u32x4 val = *reinterpret_cast<const u32x4*>(lds + row * (TN * 2) + ((cc ^ (row & (CPR - 1))) << 4));
+        if (((row >> 3) ^ (row >> 4)) & 1) val = u32x4{val[2], val[3], val[0], val[1]};
+        const bool ok = m < p.M && n < p.N;
+        if (norm) {
+            // RMS norm over the head's 128 columns, 16 lanes: y = rn(w * rn(x * r)), x the product as 16 bits
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                ss = fmaf(E::lo(val[j]), E::lo(val[j]), ss);
+                ss = fmaf(E::hi(val[j]), E::hi(val[j]), ss);
+            }
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o);
+            const float r = rsqrtf(ss * (1.f / 128.f) + p.norm_eps);
+            if (ok && p.rstd && (cc & 15) == 0) p.rstd[(int64_t)m * (p.N >> 7) + (n >> 7)] = r;
+            if (ok && p.c_raw) __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(p.c_raw + (int64_t)m * pr.ldc + n));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t h = E::pack(E::lo(val[j]) * r, E::hi(val[j]) * r);
+                val[j] = E::pack(E::lo(wt[j]) * E::lo(h), E::hi(wt[j]) * E::hi(h));
+            }
+        }
+        // (a streaming store: nobody on this CU reads the tile again)
+        if (ok) __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(C + (int64_t)m * pr.ldc + n));
+    }
+}
+
 template <int GM, int GN, int WM, int WN, int NS, bool F16>
 hipError_t launch_cfg_t(const GemmParams& p, int grid, bool a_mcontig, bool b_ncontig, hipStream_t st) {
     if (!a_mcontig && !b_ncontig)
@@ -519,10 +707,38 @@ hipError_t launch_cfg(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t 
     return launch_cfg_t<GM, GN, WM, WN, NS, false>(p, grid, a_mcontig, b_ncontig, st);
 }
 
+
+template <int TN, bool F16>
+hipError_t launch_tile(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t st) {
+    p.tiles_m = (p.M + 255) / 256;
+    p.tiles_n = (p.N + TN - 1) / TN;
+    p.total_wg = p.nprob * p.tiles_m * p.tiles_n;
+    const dim3 grid((p.total_wg + 7) / 8 * 8);
+    if (!a_mcontig && !b_ncontig) return launch1((gemm_tile_kernel<false, false, TN, F16>), grid, dim3(256), st, p);
+    if (!a_mcontig) return launch1((gemm_tile_kernel<false, true, TN, F16>), grid, dim3(256), st, p);
+    return launch1((gemm_tile_kernel<true, true, TN, F16>), grid, dim3(256), st, p);
+}
+
+// What gemm_tile_kernel takes: no batch, one contraction length for both segments (whole stages of it where
+// there are two), offsets inside an operand below 2^32, and not the layout nothing uses.
+bool gemm_tile_ok(const GemmParams& p, bool a_mcontig, bool b_ncontig) {
+    const GemmProblem& pr = p.prob[0];
+    if (p.nbatch != 1 || p.k_len || p.k_range || p.k_splits > 1 || p.a_tiled_m || (a_mcontig && !b_ncontig)) return false;
+    if (pr.nseg > 1 && (pr.K[1] != pr.K[0] || pr.K[0] % TK)) return false;
+    // (the descriptor of a row-major operand covers 2 GiB, the other kind ends with the contraction)
+    const int64_t limit = (int64_t)1 << 32;
+    const int64_t a_end = (a_mcontig ? (pr.K[0] + 2 * TK) * pr.lda[0] : 256 * pr.lda[0] + pr.K[0]) * 2;
+    const int64_t b_end = (b_ncontig ? (pr.K[0] + 2 * TK) * pr.ldb[0] : 256 * pr.ldb[0] + pr.K[0]) * 2;
+    return a_end < (a_mcontig ? limit : limit / 2) && b_end < (b_ncontig ? limit : limit / 2);
+}
+
 }  // namespace
 
-// Work-group tile by shape: 256 x 256 in general; for a narrow C (N <= 128, the
-// dQ GEMM) 512 x 128, or 256 x 128 when there are not 512 rows or when M tiles have
+// Work-group tile by shape.  C wider than 128 columns (projections, their gradients): the hand-scheduled tile
+// of 256 x 256, or 256 x 128 where that fills the chip's rounds better: a 128-wide tile takes about 0.6 of
+// the time of a 256-wide one (2046 x 4096 x 4096: 128 tiles of 256 on 256 CUs 81 us, 256 of 128 60; 12808 x 4096 x
+// 1024 twice: 2 rounds 176 us, 4 rounds 208).
+// A narrow C (the dQ GEMM): 512 x 128, or 256 x 128 when there are not 512 rows or when M tiles have
 // their own contraction ranges (k_range is kept per 256 rows: finer ranges skip more).
 hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipStream_t st) {
     for (int i = 0; i < p.nprob; ++i) {
@@ -530,6 +746,14 @@ hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipS
         // all problems and both contraction segments share the per-thread load offsets
         if (pr.lda[0] != p.prob[0].lda[0] || pr.ldb[0] != p.prob[0].ldb[0]) return hipErrorInvalidValue;
         if (pr.nseg > 1 && (pr.lda[1] != pr.lda[0] || pr.ldb[1] != pr.ldb[0])) return hipErrorInvalidValue;
+    }
+    if (p.N > 128 && gemm_tile_ok(p, a_mcontig, b_ncontig)) {
+        const int n_cu = cu_count();
+        const int64_t rows = (p.M + 255) / 256 * (int64_t)p.nprob;
+        const int64_t wide = (rows * ((p.N + 255) / 256) + n_cu - 1) / n_cu, narrow = (rows * ((p.N + 127) / 128) + n_cu - 1) / n_cu;
+        const bool use_narrow = 10 * wide > 6 * narrow;
+        if (use_narrow) return p.f16 ? launch_tile<128, true>(p, a_mcontig, b_ncontig, st) : launch_tile<128, false>(p, a_mcontig, b_ncontig, st);
+        return p.f16 ? launch_tile<256, true>(p, a_mcontig, b_ncontig, st) : launch_tile<256, false>(p, a_mcontig, b_ncontig, st);
     }
     if (p.N > 128) return launch_cfg<2, 4, 4, 2, 4>(p, a_mcontig, b_ncontig, st);
     if (p.m_order && (!p.k_range || p.nprob != 1 || p.k_splits > 1 || p.N > 128)) return hipErrorInvalidValue;

@@ -15,6 +15,9 @@ inline hipError_t launch1(void (*kernel)(P), dim3 grid, dim3 block, hipStream_t 
     return hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, args, 0, st);
 }
 
+// CUs of the device that is current (the one the caller's stream belongs to), asked for once per device.
+int cu_count();
+
 struct Strides3 {
     int64_t b, h, s;
 };
