@@ -1,17 +1,25 @@
 """Writes the hand-scheduled steady-state loops of the gfx950 backward kernel (lvx_bwd.hip):
 
-    python gen_bwd_loop.py p > lvx_bwd_loop_p.inc      (P-waves: S, P = exp2(..), dV^T)
-    python gen_bwd_loop.py d > lvx_bwd_loop_d.inc      (D-waves: dP, dS, dK^T)
+    python gen_bwd_loop.py p bf16 128 plain > lvx_bwd_loop_p_bf16_128_plain.inc   (P-waves: S, P = exp2(..), dV^T)
+    python gen_bwd_loop.py d bf16 128 > lvx_bwd_loop_d_bf16_128.inc               (D-waves: dP, dS, dK^T)
 
-Each is one inline-asm statement with every register named here.  One trip does six steps (the
+for bf16 and f16, head dimensions 128 and 64, and P-waves without ("plain") and with ("masked") key
+intervals per row.  Each is one inline-asm statement with every register named here.  One trip does six steps (the
 six tile buffers of each ring and the two-deep P / dS^T buffers then sit at immediate offsets);
-the first step of a trip is a step i with i % 6 == 3.  Inside a step the 16 MFMAs of a wave are
+the first step of a trip is a step i with i % 6 == 3.  Inside a step the 16 MFMAs of a wave (8 with heads of 64) are
 spread over its other instructions (LDS operand reads eight operands ahead, the exponentials or
 the dS arithmetic of an earlier tile, the global -> LDS loads and the dS^T copy-out), so that a
 wave keeps the matrix pipe fed by itself.
 
 LDS map in bytes (lvx_bwd.hip): Q ring 6 x 8192 at 0, dO ring at 49152, dS^T tiles 2 x 10240 at
-98304, P hand-over 2 x 8192 at 118784; the metadata records 6 x 512 bytes are a separate array.
+98304, P hand-over 2 x 8192 at 118784; the metadata of a tile, 6 x 768 bytes, is a separate array: 256 bytes
+of LSE and delta, with intervals per row 256 each of starts and ends (32 rows, twice).
+
+The last tile of a head may have fewer than 32 rows: when the walk comes to it, the lanes' load offsets are
+replaced by ones whose rows are clamped to the window's last (RAGGED, out of line), and restored with the
+next head.  Masked: a step asks with one compare per lane whether any
+row of the tile cuts the wave's 32 tokens and only then goes through the out-of-line block that zeroes
+the hidden elements of P.
 
 Registers, both roles: v[0:63] resident accumulators (dV^T / dK^T)   v[64:95] resident B operands
 (K rows / V rows)   v[96:111], v[112:127] the two score sets (raw S / dP), swapping every step
@@ -20,13 +28,19 @@ v[208:215] transposing-read addresses into the other ring.   s40 scale*log2(e) (
 P-waves: v[168:175] P packed   v[176:191] LSE*log2(e) of 16 rows   v[192:199] dS^T copy-out data
   v216 P hand-over write address   v217 metadata read address   v218 dS^T copy-out read address
   v219, v220 copy-out global offsets   v221..v224 global offsets of the four tile loads   v225 of
-  the metadata load
+  the metadata load   v226, v227 rows by which the lane's two rows of a head's last tile are past the window
+  v229 scratch   masked: v228 read address of the interval of row lane % 32   v229, v230 that interval
+  v231 the lane's token, out of every interval if it is past the sample   v232 bytes by which the lane's row of
+  a head's last tile is past the window, in the waves that fetch intervals
   s41 / s42 bytes per Q / dO tile   s[44:45] Q, s[46:47] dO, s[48:49] metadata, s[50:51] dS^T
   workspace address of the next tile to request   s52 tiles left in its head   s53 tiles per head
   s[54:55] / s[56:57] / s[60:61] what a head change adds to the Q / dO / workspace address
   s62 LDS address of this wave's part of Q buffer 0   s63 of the metadata records   s64 trips
-  s65 1 in wave 0 (it requests the metadata)   s[66:77] workspace addresses of the tiles in flight
-  s[78:79] scratch
+  s65 1 in the waves that request metadata: wave 0 LSE and delta, wave 1 interval starts, wave 2 ends
+  s[66:77] workspace addresses of the tiles in flight   s[78:79], s[88:89] scratch
+  s[80:81] what a head change adds to the metadata address   s82 1 if the last tile of a head has clamped
+  rows, else -1   s83 / s84 bytes per Q / dO row   masked: s85 bytes of metadata per tile   s86 first token of the wave, s87 one
+  past its last   s[90:91] all ones if not all of them exist
 D-waves: v[168:175] P handed over   v[176:183] dS packed   v[184:199] delta*scale of 16 rows
   v216 P hand-over read address   v217 metadata read address   v218 dS^T staging write address
 """
@@ -40,15 +54,22 @@ ROLE = sys.argv[1] if len(sys.argv) > 1 else "p"
 for _o in list(OPTS):      # a switch for one role only: p_novalu, d_nolds, ...
     if _o.startswith(ROLE + "_"):
         OPTS[_o[2:]] = OPTS[_o]
-F16 = False
-MFMA = "v_mfma_f32_32x32x16_bf16"
+F16 = len(sys.argv) > 2 and sys.argv[2] == "f16"
+DH = int(sys.argv[3]) if len(sys.argv) > 3 else 128
+MASKED = len(sys.argv) > 4 and sys.argv[4] == "masked"
+MFMA = "v_mfma_f32_32x32x16_f16" if F16 else "v_mfma_f32_32x32x16_bf16"
+CVT = "v_cvt_pk_f16_f32" if F16 else "v_cvt_pk_bf16_f32"
+NKK, NDT = DH // 16, DH // 32           # k-steps of S / dP, 32-wide blocks of dV^T / dK^T
+NOP = NKK + 2 * NDT                     # MFMAs of a step, one LDS operand each
 
 ACC, BREG, SET, STG, RA, TA = 0, 64, (96, 112), 128, 200, 208
 NSLOT, AHEAD = 8, 7
-TILE_B, DO_RING, DST_B, DST_SZ, PB_SZ, META_SZ = 8192, 49152, 98304, 10240, 8192, 512
+TILE_B, DO_RING, DST_B, DST_SZ, PB_SZ, META_SZ = 8192, 49152, 98304, 10240, 8192, 768
 # P role
 PU, LSE, CPD = 168, 176, 192
 A_PB, A_META, A_CP, G_CP0, G_CP1, G_DMA, G_META = 216, 217, 218, 219, 220, 221, 225
+EXCESS, A_IV, IV, TOKEN = 226, 228, 229, 231
+IV_EXCESS = 232
 # D role
 DSU, DELTA, TMP = 176, 184, 219
 
@@ -140,13 +161,13 @@ def spread(st, mfmas, side, shares):
 
 
 def p_read_op(st, u, n):
-    """LDS read of operand n of P-wave step u: 0..7 Q rows of tile i (k-step n), 8..15 dO^T of tile i-1."""
+    """LDS read of operand n of P-wave step u: Q rows of tile i (k-step n), then dO^T of tile i-1."""
     sl_i, sl_p = (u + 3) % 6, (u + 2) % 6
     slot = STG + 4 * (n % NSLOT)
-    if n < 8:
+    if n < NKK:
         st.lds(f"ds_read_b128 {vr(slot, 4)}, v{RA + n} offset:{sl_i * TILE_B}", ("op", u, n))
     else:
-        j, dt = (n - 8) // 4, (n - 8) % 4
+        j, dt = (n - NKK) // NDT, (n - NKK) % NDT
         off = sl_p * TILE_B + j * 4096
         st.lds(f"ds_read_b64_tr_b16 {vr(slot, 2)}, v{TA + 2 * dt} offset:{off}")
         st.lds(f"ds_read_b64_tr_b16 {vr(slot + 2, 2)}, v{TA + 2 * dt + 1} offset:{off}", ("op", u, n))
@@ -163,11 +184,41 @@ def p_fetch(u, ahead):
         f.append(f"global_load_lds_dwordx4 v{G_DMA + n}, {src}")
     f.append(f"s_mov_b64 {sr(ws_new, 2)}, s[50:51]")
     f += ["s_add_u32 s44, s44, s41", "s_addc_u32 s45, s45, 0", "s_add_u32 s46, s46, s42", "s_addc_u32 s47, s47, 0",
-          "s_add_u32 s48, s48, 256", "s_addc_u32 s49, s49, 0", "s_add_u32 s50, s50, 8192", "s_addc_u32 s51, s51, 0",
+          "s_add_u32 s48, s48, s85", "s_addc_u32 s49, s49, 0", "s_add_u32 s50, s50, 8192", "s_addc_u32 s51, s51, 0",
           ["s_sub_i32 s52, s52, 1", "s_cmp_lg_u32 s52, 0", f"s_cbranch_scc1 LVX_BWD_SAMEHEAD{u}{ahead}_%=",
            "s_add_u32 s44, s44, s54", "s_addc_u32 s45, s45, s55", "s_add_u32 s46, s46, s56", "s_addc_u32 s47, s47, s57",
-           "s_add_u32 s50, s50, s60", "s_addc_u32 s51, s51, s61", "s_mov_b32 s52, s53", f"LVX_BWD_SAMEHEAD{u}{ahead}_%=:"]]
+           "s_add_u32 s48, s48, s80", "s_addc_u32 s49, s49, s81",
+           "s_add_u32 s50, s50, s60", "s_addc_u32 s51, s51, s61", "s_mov_b32 s52, s53",
+           "s_cmp_eq_u32 s82, 1", f"s_cbranch_scc1 LVX_BWD_WHOLE{u}{ahead}_%=", f"LVX_BWD_SAMEHEAD{u}{ahead}_%=:",
+           "s_cmp_eq_u32 s52, s82", f"s_cbranch_scc1 LVX_BWD_RAGGED{u}{ahead}_%=", f"LVX_BWD_WALKED{u}{ahead}_%=:"]]
     return f
+
+
+def p_ragged(u, ahead):
+    """Out of line: the tile the walk has come to is a head's last and has clamped rows, so that the lanes'
+    load offsets go back by the rows they are too far; or a head with such a tile begins, and they return."""
+    def move(op):
+        return [x for n in range(4) for x in (f"v_mul_lo_u32 v{IV}, v{EXCESS + n % 2}, s{83 + n // 2}",
+                                              f"{op} v{G_DMA + n}, v{G_DMA + n}, v{IV}")] \
+            + ([f"{op} v{G_META}, v{G_META}, v{IV_EXCESS}"] if MASKED else [])
+    return [f"LVX_BWD_WHOLE{u}{ahead}_%=:", *move("v_add_u32"), f"s_branch LVX_BWD_SAMEHEAD{u}{ahead}_%=",
+            f"LVX_BWD_RAGGED{u}{ahead}_%=:", *move("v_sub_u32"), f"s_branch LVX_BWD_WALKED{u}{ahead}_%="]
+
+
+def p_mask(u):
+    """Out of line: some row of tile i-1 cuts this wave's tokens.  P's elements outside their row's interval
+    become 0; the intervals of the lane's 16 rows are read 8 rows at a time into the registers the LSE had."""
+    carry, rec = SET[u & 1], (u + 2) % 6 * META_SZ
+    out = [f"LVX_BWD_MASK{u}_%=:"]
+    for half in range(2):
+        for n in range(4):      # two groups of four interval starts, then their ends
+            vg = 2 * half + n % 2
+            out.append(f"ds_read_b128 {vr(LSE + 4 * n, 4)}, v{A_META} offset:{rec + 256 + 256 * (n // 2) + 32 * vg}")
+        out.append("s_waitcnt lgkmcnt(0)")
+        for v in range(8):
+            out += [f"v_cmp_ge_i32 s[88:89], v{TOKEN}, v{LSE + v}", f"v_cmp_lt_i32 vcc, v{TOKEN}, v{LSE + 8 + v}",
+                    "s_and_b64 vcc, vcc, s[88:89]", f"v_cndmask_b32 v{carry + 8 * half + v}, 0, v{carry + 8 * half + v}, vcc"]
+    return out + [f"s_branch LVX_BWD_SEEN{u}_%="]
 
 
 def flat(items):
@@ -190,6 +241,9 @@ def p_step(u, seed):
     e("s_barrier")
     for vg in range(4):
         st.lds(f"ds_read_b128 {vr(LSE + 4 * vg, 4)}, v{A_META} offset:{sl_p * META_SZ + vg * 32}", ("lse", vg))
+    if MASKED:
+        st.lds(f"ds_read_b32 v{IV}, v{A_IV} offset:{sl_p * META_SZ}")
+        st.lds(f"ds_read_b32 v{IV + 1}, v{A_IV} offset:{sl_p * META_SZ + 256}", "iv")
 
     # P(i-1) = exp2(S(i-1) * c - LSE), packed
     valu = []
@@ -200,14 +254,18 @@ def p_step(u, seed):
             valu.append(f"v_fma_f32 v{carry + v}, v{carry + v}, s40, -v{LSE + v}")
         for r in range(4):
             valu.append(f"v_exp_f32 v{carry + 4 * vg + r}, v{carry + 4 * vg + r}")
-        if vg >= 1:
+        if vg >= 1 and not MASKED:
             for e2 in range(2):
                 v = 4 * (vg - 1) + 2 * e2
-                valu.append(f"v_cvt_pk_bf16_f32 v{PU + v // 2}, v{carry + v}, v{carry + v + 1}")
-    valu.append("s_nop 0")
-    for e2 in range(2):
-        v = 12 + 2 * e2
-        valu.append(f"v_cvt_pk_bf16_f32 v{PU + v // 2}, v{carry + v}, v{carry + v + 1}")
+                valu.append(f"{CVT} v{PU + v // 2}, v{carry + v}, v{carry + v + 1}")
+    if MASKED:
+        valu.append(lambda: st.wait("iv"))
+        valu.append([f"v_cmp_lt_i32 vcc, s86, v{IV}", f"v_cmp_gt_i32 s[88:89], s87, v{IV + 1}", "s_or_b64 vcc, vcc, s[88:89]",
+                     "s_or_b64 vcc, vcc, s[90:91]", f"s_cbranch_vccnz LVX_BWD_MASK{u}_%=", f"LVX_BWD_SEEN{u}_%=:"])
+    else:
+        valu.append("s_nop 0")
+    for v in range(0 if MASKED else 12, 16, 2):
+        valu.append(f"{CVT} v{PU + v // 2}, v{carry + v}, v{carry + v + 1}")
     # hand P over to the D-wave
     valu.append(lambda: st.lds(f"ds_write_b128 v{A_PB}, {vr(PU, 4)} offset:{par * PB_SZ}"))
     valu.append(lambda: st.lds(f"ds_write_b128 v{A_PB}, {vr(PU + 4, 4)} offset:{par * PB_SZ + 1024}"))
@@ -233,25 +291,25 @@ def p_step(u, seed):
         tail += store
 
     mf = []
-    for k in range(16):
+    for k in range(NOP):
         def m(k=k):
             st.wait(("op", u, k))
             slot = STG + 4 * (k % NSLOT)
-            if k < 8:
+            if k < NKK:
                 c = "0" if k == 0 else vr(new, 16)
                 e(f"{MFMA} {vr(new, 16)}, {vr(slot, 4)}, {vr(BREG + 4 * k, 4)}, {c}")
             else:
-                j, dt = (k - 8) // 4, (k - 8) % 4
+                j, dt = (k - NKK) // NDT, (k - NKK) % NDT
                 e(f"{MFMA} {vr(ACC + 16 * dt, 16)}, {vr(slot, 4)}, {vr(PU + 4 * j, 4)}, {vr(ACC + 16 * dt, 16)}")
-            if k + AHEAD < 16:
+            if k + AHEAD < NOP:
                 p_read_op(st, u, k + AHEAD)
             else:
-                p_read_op(st, (u + 1) % 6, k + AHEAD - 16)
+                p_read_op(st, (u + 1) % 6, k + AHEAD - NOP)
         mf.append(m)
     side = valu + tail
-    nv = len(valu)
+    nv = sum(len(x) if isinstance(x, list) else 1 for x in valu)
     nt = sum(len(x) if isinstance(x, list) else 1 for x in tail)
-    shares = [(nv + 7) // 8] * 8 + [(nt + 6) // 7] * 8
+    shares = [-(-nv // NKK)] * NKK + [-(-nt // (2 * NDT - 1))] * (2 * NDT)
     spread(st, mf, side, shares)
     return st.out, st.carry_over((u + 1) % 6)
 
@@ -271,13 +329,13 @@ def p_prologue():
 
 
 def d_read_op(st, u, n):
-    """LDS read of operand n of D-wave step u: 0..7 dO rows of tile i-1, 8..15 Q^T of tile i-2."""
+    """LDS read of operand n of D-wave step u: dO rows of tile i-1, then Q^T of tile i-2."""
     sl_p, sl_pp = (u + 2) % 6, (u + 1) % 6
     slot = STG + 4 * (n % NSLOT)
-    if n < 8:
+    if n < NKK:
         st.lds(f"ds_read_b128 {vr(slot, 4)}, v{RA + n} offset:{sl_p * TILE_B}", ("op", u, n))
     else:
-        j, dt = (n - 8) // 4, (n - 8) % 4
+        j, dt = (n - NKK) // NDT, (n - NKK) % NDT
         off = sl_pp * TILE_B + j * 4096
         st.lds(f"ds_read_b64_tr_b16 {vr(slot, 2)}, v{TA + 2 * dt} offset:{off}")
         st.lds(f"ds_read_b64_tr_b16 {vr(slot + 2, 2)}, v{TA + 2 * dt + 1} offset:{off}", ("op", u, n))
@@ -305,35 +363,40 @@ def d_step(u, seed):
         for r in range(4):
             v = 4 * q + r
             valu.append(f"v_fma_f32 v{carry + v}, v{carry + v}, s40, -v{DELTA + v}")
-        valu.append(f"v_lshlrev_b32 v{t[0]}, 16, v{PU + 2 * q}")
-        valu.append(f"v_and_b32 v{t[1]}, 0xffff0000, v{PU + 2 * q}")
-        valu.append(f"v_lshlrev_b32 v{t[2]}, 16, v{PU + 2 * q + 1}")
-        valu.append(f"v_and_b32 v{t[3]}, 0xffff0000, v{PU + 2 * q + 1}")
-        for r in range(4):
-            v = 4 * q + r
-            valu.append(f"v_mul_f32 v{carry + v}, v{t[r]}, v{carry + v}")
-        valu.append(f"v_cvt_pk_bf16_f32 v{DSU + 2 * q}, v{carry + 4 * q}, v{carry + 4 * q + 1}")
-        valu.append(f"v_cvt_pk_bf16_f32 v{DSU + 2 * q + 1}, v{carry + 4 * q + 2}, v{carry + 4 * q + 3}")
+        if F16:     # a half of the packed P times the fp32 value, in one instruction
+            for r in range(4):
+                v = 4 * q + r
+                valu.append(f"v_fma_mix_f32 v{carry + v}, v{PU + 2 * q + r // 2}, v{carry + v}, 0 op_sel:[{r % 2},0,0] op_sel_hi:[1,0,0]")
+        else:
+            valu.append(f"v_lshlrev_b32 v{t[0]}, 16, v{PU + 2 * q}")
+            valu.append(f"v_and_b32 v{t[1]}, 0xffff0000, v{PU + 2 * q}")
+            valu.append(f"v_lshlrev_b32 v{t[2]}, 16, v{PU + 2 * q + 1}")
+            valu.append(f"v_and_b32 v{t[3]}, 0xffff0000, v{PU + 2 * q + 1}")
+            for r in range(4):
+                v = 4 * q + r
+                valu.append(f"v_mul_f32 v{carry + v}, v{t[r]}, v{carry + v}")
+        valu.append(f"{CVT} v{DSU + 2 * q}, v{carry + 4 * q}, v{carry + 4 * q + 1}")
+        valu.append(f"{CVT} v{DSU + 2 * q + 1}, v{carry + 4 * q + 2}, v{carry + 4 * q + 3}")
     for vg in range(4):
         valu.append(lambda vg=vg: st.lds(f"ds_write_b64 v{218}, {vr(DSU + 2 * vg, 2)} offset:{par * DST_SZ + 16 * vg}"))
 
     mf = []
-    for k in range(16):
+    for k in range(NOP):
         def m(k=k):
             st.wait(("op", u, k))
             slot = STG + 4 * (k % NSLOT)
-            if k < 8:
+            if k < NKK:
                 c = "0" if k == 0 else vr(new, 16)
                 e(f"{MFMA} {vr(new, 16)}, {vr(slot, 4)}, {vr(BREG + 4 * k, 4)}, {c}")
             else:
-                j, dt = (k - 8) // 4, (k - 8) % 4
+                j, dt = (k - NKK) // NDT, (k - NKK) % NDT
                 e(f"{MFMA} {vr(ACC + 16 * dt, 16)}, {vr(slot, 4)}, {vr(DSU + 4 * j, 4)}, {vr(ACC + 16 * dt, 16)}")
-            if k + AHEAD < 16:
+            if k + AHEAD < NOP:
                 d_read_op(st, u, k + AHEAD)
             else:
-                d_read_op(st, (u + 1) % 6, k + AHEAD - 16)
+                d_read_op(st, (u + 1) % 6, k + AHEAD - NOP)
         mf.append(m)
-    shares = [6] * 8 + [4, 4, 4, 2, 2, 2, 0, 0]
+    shares = [6] * 8 + [4, 4, 4, 2, 2, 2, 0, 0] if DH == 128 else [12] * 4 + [8, 8, 0, 0]
     spread(st, mf, valu, shares)
     return st.out, st.carry_over((u + 1) % 6)
 
@@ -409,6 +472,11 @@ def main():
     cnt = "s64"
     lines = (p_prologue() if ROLE == "p" else d_prologue()) + ["LVX_BWD_LOOP_%=:"] + body + [f"s_sub_i32 {cnt}, {cnt}, 1", f"s_cmp_lg_u32 {cnt}, 0", "s_cbranch_scc1 LVX_BWD_LOOP_%=",
                                            "s_waitcnt lgkmcnt(0)", "s_nop 15", "s_nop 3"]
+    if ROLE == "p":
+        lines += ["s_branch LVX_BWD_END_%="] + p_ragged(0, 2)
+        for u in range(6):
+            lines += p_ragged(u, 3) + (p_mask(u) if MASKED else [])
+        lines.append("LVX_BWD_END_%=:")
     print("// generated by gen_bwd_loop.py - do not edit")
     for l in lines:
         print(f'"{l}\\n"')

@@ -67,10 +67,37 @@ constexpr int EPS = D + 1;                          // row stride (floats) of th
 constexpr int EPI_ELEMS = 8 * 32 * EPS * 2;         // 8 waves x [32 tokens][128 + 1] floats, in uint16 units
 constexpr int SMEM_ELEMS = LOOP_ELEMS > EPI_ELEMS ? LOOP_ELEMS : EPI_ELEMS;
 
+constexpr uint32_t META_B = 768;   // bytes of a tile's metadata
 constexpr float LOG2E = 1.4426950408889634f;
 
 // registers the hand-scheduled loops use besides their operands (see gen_bwd_loop.py)
 #define LVX_BWD_LOOP_CLOBBERS "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127", "v128", "v129", "v130", "v131", "v132", "v133", "v134", "v135", "v136", "v137", "v138", "v139", "v140", "v141", "v142", "v143", "v144", "v145", "v146", "v147", "v148", "v149", "v150", "v151", "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v160", "v161", "v162", "v163", "v164", "v165", "v166", "v167", "v168", "v169", "v170", "v171", "v172", "v173", "v174", "v175", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", "v187", "v188", "v189", "v190", "v191", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199"
+
+// operands of the hand-scheduled loops, one list per role for all element types, head dimensions and masks
+#define LVX_BWD_COMMON_OUT "+{v[0:15]}"(acc[0]), "+{v[16:31]}"(acc[1]), "+{v[32:47]}"(acc[2]), "+{v[48:63]}"(acc[3]), \
+    "+{v[96:111]}"(carry), "+{s64}"(trips)
+#define LVX_BWD_COMMON_IN "{v[64:67]}"(breg[0]), "{v[68:71]}"(breg[1]), "{v[72:75]}"(breg[2]), "{v[76:79]}"(breg[3]), \
+    "{v[80:83]}"(breg[4]), "{v[84:87]}"(breg[5]), "{v[88:91]}"(breg[6]), "{v[92:95]}"(breg[7]),                      \
+    "{v200}"(ra[0]), "{v201}"(ra[1]), "{v202}"(ra[2]), "{v203}"(ra[3]),                                              \
+    "{v204}"(ra[4]), "{v205}"(ra[5]), "{v206}"(ra[6]), "{v207}"(ra[7]),                                              \
+    "{v208}"(ta[0]), "{v209}"(ta[1]), "{v210}"(ta[2]), "{v211}"(ta[3]),                                              \
+    "{v212}"(ta[4]), "{v213}"(ta[5]), "{v214}"(ta[6]), "{v215}"(ta[7]), "{v216}"(a_pb), "{v217}"(a_meta)
+#define LVX_BWD_P_OPERANDS                                                                                           \
+    : LVX_BWD_COMMON_OUT, "+{s[44:45]}"(qp), "+{s[46:47]}"(dop), "+{s[48:49]}"(mp), "+{s[50:51]}"(wn), "+{s52}"(left), \
+      "+{s[66:67]}"(w0), "+{s[68:69]}"(w1), "+{s[70:71]}"(w2), "+{s[72:73]}"(w3), "+{s[74:75]}"(w4), "+{s[76:77]}"(w5), \
+      "+{v221}"(g_t[0]), "+{v222}"(g_t[1]), "+{v223}"(g_t[2]), "+{v224}"(g_t[3]), "+{v225}"(g_meta)                   \
+    : LVX_BWD_COMMON_IN, "{v218}"(a_cp), "{v219}"(g_cp0), "{v220}"(g_cp1), "{v232}"(past_iv),                        \
+      "{v226}"(past0), "{v227}"(past1), "{v228}"(a_iv), "{v231}"(token), "{s83}"(uniform32(qrow_b)), "{s84}"(uniform32(dorow_b)), \
+      "{s40}"(uniform32(c)), "{s41}"(uniform32((uint32_t)BM * qrow_b)), "{s42}"(uniform32((uint32_t)BM * dorow_b)),  \
+      "{s53}"(uniform32(n_live)), "{s[54:55]}"(hdq), "{s[56:57]}"(hddo), "{s[60:61]}"(hdws), "{s[80:81]}"(hdm),      \
+      "{s62}"(uniform32(lds0 + (uint32_t)slice * 2048u)), "{s63}"(uniform32(meta0 + meta_w)),                        \
+      "{s65}"(uniform32(wave < META_WAVES ? 1 : 0)), "{s82}"(uniform32(ragged ? 1 : -1)),                            \
+      "{s85}"(uniform32(meta_w ? BM * 4 : 256)), "{s86}"(uniform32(slice_lo)), "{s87}"(uniform32(slice_lo + 32)),     \
+      "{s[90:91]}"(uniform64(slice_valid ? (int64_t)0 : (int64_t)-1))                                                \
+    : "memory", "vcc", "scc", "m0", "s78", "s79", "s88", "s89", "v229", "v230", LVX_BWD_LOOP_CLOBBERS
+#define LVX_BWD_D_OPERANDS                                                                                           \
+    : LVX_BWD_COMMON_OUT : LVX_BWD_COMMON_IN, "{v218}"(a_ds), "{s40}"(uniform32(p.scale))                            \
+    : "memory", "vcc", "scc", LVX_BWD_LOOP_CLOBBERS, "v219", "v220", "v221", "v222"
 
 // BIAS: a dense fp32 bias joins the exponent, P = exp2(S*c + bias*log2e - LSE*log2e).
 // DH: head dimension, 16, 32, 64 or 128.  The LDS tiles keep their 256-byte rows and chunk
@@ -83,10 +110,11 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     using E = Elt<F16>;
     static_assert(DH == 16 || DH == 32 || DH == 64 || DH == 128, "head dimension");
     constexpr int NKK = DH / 16, NDT = DH >= 32 ? DH / 32 : 1;
+    constexpr int META_WAVES = MASKED ? 3 : 1;      // waves that fetch a part of a tile's metadata
     __shared__ __attribute__((aligned(1024))) uint16_t smem[SMEM_ELEMS];
-    // per-row metadata of a staged tile, one per tile buffer: 8 x 16 bytes each of
-    // LSE*log2e, delta*scale, kv_start, kv_end
-    __shared__ __attribute__((aligned(256))) u32x4 meta_s4[NQD][BM];
+    // per-row metadata of a staged tile, one per tile buffer: 8 x 16 bytes each of LSE*log2e and
+    // delta*scale; with an interval mask kv_start and kv_end follow, each twice (a load moves 64 lanes)
+    __shared__ __attribute__((aligned(256))) u32x4 meta_s4[NQD][META_B / 16];
 
     // Work-group ids are dealt to the 8 XCDs round-robin.  XCD x takes the token blocks
     // [x * blocks_per_xcd, (x + 1) * blocks_per_xcd) of the list (b, kv head, block), so that the
@@ -234,17 +262,18 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     // Every load is unconditional and goes straight to LDS: rows past the window are
     // clamped to its last row (their LSE record is +inf, so P = 0 and nothing they
     // carry reaches a result).  Wave 0 also fetches the tile's metadata record
-    // (32 x LSE*log2e, 32 x delta*scale; 256 bytes) and, with a mask, the rows'
-    // key intervals, ahead of its tile loads so that "tile landed" implies both.
+    // (32 x LSE*log2e, 32 x delta*scale; 256 bytes) and, with an interval mask, waves
+    // 1 and 2 the rows' first and last keys, ahead of their tile loads so that "tile landed" implies both.
     auto prefetch = [&](int buf) {
         const int r0 = p.row_begin + cur_qt * BM;
-        if (wave == 0) {
-            const uint32_t mslot = meta0 + (uint32_t)buf * (BM * 16);
-            dma4(reinterpret_cast<const char*>(meta_head + cur_qt * 64), (uint32_t)lane * 4u, mslot);
-            if (MASKED) {
-                const int32_t* iv = (lane < 32 ? p.kv_start : p.kv_end) + (int64_t)b * p.Lq + min(r0 + l32, p.row_end - 1);
-                dma4_addr(reinterpret_cast<const char*>(iv), mslot + 256);
+        if (wave < META_WAVES) {
+            const char* src = reinterpret_cast<const char*>(meta_head + cur_qt * 64);
+            uint32_t off = (uint32_t)lane * 4u;
+            if (MASKED && wave > 0) {
+                src = reinterpret_cast<const char*>((wave == 1 ? p.kv_start : p.kv_end) + (int64_t)b * p.Lq + r0);
+                off = (uint32_t)min(l32, p.row_end - 1 - r0) * 4u;
             }
+            dma4(src, off, meta0 + (uint32_t)buf * META_B + (uint32_t)wave * 256u);
         }
         const uint32_t row0 = (uint32_t)min(r0 + ld_r, p.row_end - 1);
         const uint32_t row1 = (uint32_t)min(r0 + ld_r + 4, p.row_end - 1);
@@ -305,7 +334,7 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         if (MASKED && pv_live) {
             const int32_t* iv = reinterpret_cast<const int32_t*>(meta + 16);
             iv_s = iv[l32];
-            iv_e = iv[32 + l32];
+            iv_e = iv[64 + l32];
         }
         if (s_live) {
 #pragma unroll
@@ -348,7 +377,7 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
 #pragma unroll
                     for (int vg = 0; vg < 4; ++vg) {
                         const u32x4 sp = meta[16 + 2 * vg + g];
-                        const u32x4 ep = meta[24 + 2 * vg + g];
+                        const u32x4 ep = meta[32 + 2 * vg + g];
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
                             const bool vis = kv_valid && my_kv >= (int)sp[r] && my_kv < (int)ep[r];
@@ -513,14 +542,19 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         const int last = n_iter + 1;
         int i = 0;
         for (; i < 3 && i <= last; ++i) step(i, i < n_iter, i >= 1 && i <= n_iter, i >= 2, false);
-        // Steady state of the plain bf16 kernel: steps 3 .. 3 + 6 trips - 1 (every one of them with all
-        // its parts alive and a tile to request) run in the hand-scheduled loops of gen_bwd_loop.py,
-        // six steps a trip; the steps after them continue below as if they had run here.
-        if constexpr (DH == 128 && !MASKED && !BIAS && !F16 && !decltype(tail_c)::value) {
+        // Steady state: steps 3 .. 3 + 6 trips - 1 (every one of them with all its parts alive and a tile to
+        // request) run in the hand-scheduled loops of gen_bwd_loop.py, six steps a trip; the steps after
+        // them continue below as if they had run here.  Left to the code above: heads of 32 and 16, a dense
+        // bias, the last token block where there is no mask, and token blocks whose live tiles are not one run.
+        // The code above leaves the matrix pipe to the compiler's order and, masked, keeps its walk in spilled
+        // scalar registers.  Forward and backward of an attention, us, that code against the loops: 2 x 3000 rows,
+        // images of 3202 tokens 1423 -> 1199; 2 x 1023 rows x 6404 tokens 2039 -> 1999 (whole layer);
+        // heads of 64, 2048 x 6404 708 -> 697.
+        if constexpr ((DH == 128 || DH == 64) && !BIAS && !decltype(tail_c)::value) {
             int trips = uniform32((n_iter - 5) / 6);
-            if (i == 3 && trips >= 1 && (p.row_end - p.row_begin) % BM == 0) {
+            if (i == 3 && trips >= 1 && run_n[1] == 0) {
                 const int steps = 6 * trips;
-                uint32_t ra[8], ta[8];
+                uint32_t ra[8], ta[8];      // with heads of 64 half of each stays unused
 #pragma unroll
                 for (int kk = 0; kk < 8; ++kk)
                     ra[kk] = lds0 + (DROLE ? OFF_DO : OFF_Q) * 2 + row_rd + ((uint32_t)(kk * 32) ^ row_h);
@@ -532,10 +566,14 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                 const uint32_t a_pb = lds0 + OFF_PB * 2 + (uint32_t)pb_off * 2;
                 const uint32_t a_meta = meta0 + (uint32_t)g * 16u;
                 if constexpr (!DROLE) {
+                    const uint32_t meta_w = wave < META_WAVES ? (uint32_t)wave * 256u : 0u;
                     uint16_t* ws_k = p.ds_ws + (int64_t)kblk * p.ws_ld;
                     const char* qp = uniform_ptr(q_head + (int64_t)(p.row_begin + cur_qt * BM) * qrow_b);
                     const char* dop = uniform_ptr(do_head + (int64_t)(p.row_begin + cur_qt * BM) * dorow_b);
-                    const char* mp = uniform_ptr(reinterpret_cast<const char*>(meta_head + cur_qt * 64));
+                    const char* m_src = reinterpret_cast<const char*>(meta_head + cur_qt * 64);
+                    if (meta_w) m_src = reinterpret_cast<const char*>((wave == 1 ? p.kv_start : p.kv_end) + (int64_t)b * p.Lq +
+                                                                      p.row_begin + cur_qt * BM);
+                    const char* mp = uniform_ptr(m_src);
                     const char* wn = uniform_ptr(reinterpret_cast<const char*>(ws_k + ws_head + (int64_t)cur_qt * (BN * BM)));
                     const char* w0 = uniform_ptr(reinterpret_cast<const char*>(ws_k + w_q[0]));
                     const char* w1 = uniform_ptr(reinterpret_cast<const char*>(ws_k + w_q[1]));
@@ -544,33 +582,58 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                     const char* w4 = uniform_ptr(reinterpret_cast<const char*>(ws_k + w_q[4]));
                     const char* w5 = w4;
                     int left = uniform32(cur_left);
-                    const int64_t hdq = uniform64((int64_t)p.qs.h * 2 - (int64_t)n_qtiles * BM * qrow_b);
-                    const int64_t hddo = uniform64((int64_t)p.dos.h * 2 - (int64_t)n_qtiles * BM * dorow_b);
-                    const int64_t hdws = uniform64((int64_t)p.ws_bh * 2 - (int64_t)n_qtiles * (BN * BM * 2));
+                    const int64_t hdq = uniform64((int64_t)p.qs.h * 2 - (int64_t)n_live * BM * qrow_b);
+                    const int64_t hddo = uniform64((int64_t)p.dos.h * 2 - (int64_t)n_live * BM * dorow_b);
+                    const int64_t hdws = uniform64((int64_t)p.ws_bh * 2 - (int64_t)n_live * (BN * BM * 2));
+                    const int64_t hdm = uniform64(meta_w ? -(int64_t)n_live * (BM * 4) : (int64_t)(n_qtiles - n_live) * 256);
                     const uint32_t a_cp = lds0 + OFF_DST * 2 + (uint32_t)(cp_token * DSS + cp_part * 8) * 2;
                     const uint32_t g_cp0 = (uint32_t)(cp_token * BM + cp_part * 8) * 2, g_cp1 = g_cp0 + 64 * BM * 2;
-                    const uint32_t lr = (uint32_t)(lane >> 4) + 8u * slice;
-                    const uint32_t g_q0 = lr * qrow_b + ld_c0, g_q1 = (lr + 4) * qrow_b + ld_c1;
-                    const uint32_t g_d0 = lr * dorow_b + ld_c0, g_d1 = (lr + 4) * dorow_b + ld_c1;
+                    // the four loads of a tile; in a window's last one the rows end at `last`
+                    const int last = (p.row_end - p.row_begin - 1) % BM;
+                    const bool ragged = last != BM - 1 && run_s[0] + n_live == n_qtiles;
+                    const int lr = (lane >> 4) + 8 * slice;
+                    const uint32_t past0 = (uint32_t)max(lr - last, 0), past1 = (uint32_t)max(lr + 4 - last, 0);
+                    const bool now = ragged && left == 1;       // the first tile to request is such a tile
+                    const uint32_t rl0 = (uint32_t)lr - (now ? past0 : 0u), rl1 = (uint32_t)(lr + 4) - (now ? past1 : 0u);
+                    uint32_t g_t[4] = {rl0 * qrow_b + ld_c0, rl1 * qrow_b + ld_c1, rl0 * dorow_b + ld_c0, rl1 * dorow_b + ld_c1};
+                    const uint32_t past_iv = meta_w ? (uint32_t)max(l32 - last, 0) * 4u : 0u;
+                    uint32_t g_meta = (meta_w ? (uint32_t)l32 : (uint32_t)lane) * 4u - (now ? past_iv : 0u);
+                    const uint32_t a_iv = meta0 + 256u + (uint32_t)l32 * 4u;
+                    const int token = kv_valid ? my_kv : 0x7fffffff;
                     wait_vmcnt<4>();    // tile 3 (the loads of tile 4 may be in flight); the loop counts from there
-                    asm volatile(
-#include "lvx_bwd_loop_p.inc"
-                        : "+{v[0:15]}"(acc[0]), "+{v[16:31]}"(acc[1]), "+{v[32:47]}"(acc[2]), "+{v[48:63]}"(acc[3]),
-                          "+{v[96:111]}"(carry), "+{s[44:45]}"(qp), "+{s[46:47]}"(dop), "+{s[48:49]}"(mp), "+{s[50:51]}"(wn),
-                          "+{s52}"(left), "+{s64}"(trips), "+{s[66:67]}"(w0), "+{s[68:69]}"(w1), "+{s[70:71]}"(w2),
-                          "+{s[72:73]}"(w3), "+{s[74:75]}"(w4), "+{s[76:77]}"(w5)
-                        : "{v[64:67]}"(breg[0]), "{v[68:71]}"(breg[1]), "{v[72:75]}"(breg[2]), "{v[76:79]}"(breg[3]),
-                          "{v[80:83]}"(breg[4]), "{v[84:87]}"(breg[5]), "{v[88:91]}"(breg[6]), "{v[92:95]}"(breg[7]),
-                          "{v200}"(ra[0]), "{v201}"(ra[1]), "{v202}"(ra[2]), "{v203}"(ra[3]),
-                          "{v204}"(ra[4]), "{v205}"(ra[5]), "{v206}"(ra[6]), "{v207}"(ra[7]),
-                          "{v208}"(ta[0]), "{v209}"(ta[1]), "{v210}"(ta[2]), "{v211}"(ta[3]),
-                          "{v212}"(ta[4]), "{v213}"(ta[5]), "{v214}"(ta[6]), "{v215}"(ta[7]),
-                          "{v216}"(a_pb), "{v217}"(a_meta), "{v218}"(a_cp), "{v219}"(g_cp0), "{v220}"(g_cp1),
-                          "{v221}"(g_q0), "{v222}"(g_q1), "{v223}"(g_d0), "{v224}"(g_d1), "{v225}"((uint32_t)lane * 4u),
-                          "{s40}"(uniform32(c)), "{s41}"(uniform32((uint32_t)BM * qrow_b)), "{s42}"(uniform32((uint32_t)BM * dorow_b)), "{s53}"(uniform32(n_qtiles)),
-                          "{s[54:55]}"(hdq), "{s[56:57]}"(hddo), "{s[60:61]}"(hdws),
-                          "{s62}"(uniform32(lds0 + (uint32_t)slice * 2048u)), "{s63}"(uniform32(meta0)), "{s65}"(uniform32(wave == 0 ? 1 : 0))
-                        : "memory", "vcc", "scc", "m0", "s78", "s79", LVX_BWD_LOOP_CLOBBERS);
+                    if constexpr (!F16 && DH == 128 && !MASKED) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_bf16_128_plain.inc"
+                            LVX_BWD_P_OPERANDS);
+                    } else if constexpr (!F16 && DH == 128) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_bf16_128_masked.inc"
+                            LVX_BWD_P_OPERANDS);
+                    } else if constexpr (!F16 && !MASKED) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_bf16_64_plain.inc"
+                            LVX_BWD_P_OPERANDS);
+                    } else if constexpr (!F16) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_bf16_64_masked.inc"
+                            LVX_BWD_P_OPERANDS);
+                    } else if constexpr (DH == 128 && !MASKED) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_f16_128_plain.inc"
+                            LVX_BWD_P_OPERANDS);
+                    } else if constexpr (DH == 128) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_f16_128_masked.inc"
+                            LVX_BWD_P_OPERANDS);
+                    } else if constexpr (!MASKED) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_f16_64_plain.inc"
+                            LVX_BWD_P_OPERANDS);
+                    } else {
+                        asm volatile(
+#include "lvx_bwd_loop_p_f16_64_masked.inc"
+                            LVX_BWD_P_OPERANDS);
+                    }
                     wait_vmcnt<0>();    // the steps below count the operations in flight from scratch
                     w_q[0] = reinterpret_cast<const uint16_t*>(w0) - ws_k;
                     w_q[1] = reinterpret_cast<const uint16_t*>(w1) - ws_k;
@@ -579,25 +642,31 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                     w_q[4] = reinterpret_cast<const uint16_t*>(w4) - ws_k;
                 } else {
                     const uint32_t a_ds = lds0 + OFF_DST * 2 + (uint32_t)((32 * slice + l32) * DSS + 4 * g) * 2;
-                    asm volatile(
-#include "lvx_bwd_loop_d.inc"
-                        : "+{v[0:15]}"(acc[0]), "+{v[16:31]}"(acc[1]), "+{v[32:47]}"(acc[2]), "+{v[48:63]}"(acc[3]),
-                          "+{v[96:111]}"(carry), "+{s64}"(trips)
-                        : "{v[64:67]}"(breg[0]), "{v[68:71]}"(breg[1]), "{v[72:75]}"(breg[2]), "{v[76:79]}"(breg[3]),
-                          "{v[80:83]}"(breg[4]), "{v[84:87]}"(breg[5]), "{v[88:91]}"(breg[6]), "{v[92:95]}"(breg[7]),
-                          "{v200}"(ra[0]), "{v201}"(ra[1]), "{v202}"(ra[2]), "{v203}"(ra[3]),
-                          "{v204}"(ra[4]), "{v205}"(ra[5]), "{v206}"(ra[6]), "{v207}"(ra[7]),
-                          "{v208}"(ta[0]), "{v209}"(ta[1]), "{v210}"(ta[2]), "{v211}"(ta[3]),
-                          "{v212}"(ta[4]), "{v213}"(ta[5]), "{v214}"(ta[6]), "{v215}"(ta[7]),
-                          "{v216}"(a_pb), "{v217}"(a_meta), "{v218}"(a_ds), "{s40}"(uniform32(p.scale))
-                        : "memory", "vcc", "scc", LVX_BWD_LOOP_CLOBBERS, "v219", "v220", "v221", "v222");
+                    if constexpr (!F16 && DH == 128) {
+                        asm volatile(
+#include "lvx_bwd_loop_d_bf16_128.inc"
+                            LVX_BWD_D_OPERANDS);
+                    } else if constexpr (!F16) {
+                        asm volatile(
+#include "lvx_bwd_loop_d_bf16_64.inc"
+                            LVX_BWD_D_OPERANDS);
+                    } else if constexpr (DH == 128) {
+                        asm volatile(
+#include "lvx_bwd_loop_d_f16_128.inc"
+                            LVX_BWD_D_OPERANDS);
+                    } else {
+                        asm volatile(
+#include "lvx_bwd_loop_d_f16_64.inc"
+                            LVX_BWD_D_OPERANDS);
+                    }
                 }
                 i += steps;
                 // the walk stands at the tile after the last one requested
                 const int pos = it_lo + i + 2;
                 cur_gi = pos / n_live;
-                cur_qt = pos % n_live;
-                cur_left = n_live - cur_qt;
+                cur_run = 0;
+                cur_qt = run_s[0] + pos % n_live;
+                cur_left = n_live - pos % n_live;
                 if (cur_gi >= p.G) cur_gi = 0;
                 enter_head();
             }
@@ -608,10 +677,10 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         if (!DROLE) copy_out(dst((n_iter - 1) & 1), w_q[0]);
     };
     if (d_role) {
-        if (tail_block) run(std::true_type{}, std::true_type{});
+        if (!MASKED && tail_block) run(std::true_type{}, std::true_type{});
         else run(std::false_type{}, std::true_type{});
     } else {
-        if (tail_block) run(std::true_type{}, std::false_type{});
+        if (!MASKED && tail_block) run(std::true_type{}, std::false_type{});
         else run(std::false_type{}, std::false_type{});
     }
 
