@@ -40,7 +40,7 @@ P-waves: v[168:175] P packed   v[176:191] LSE*log2(e) of 16 rows   v[192:199] dS
   s[66:77] workspace addresses of the tiles in flight   s[78:79], s[88:89] scratch
   s[80:81] what a head change adds to the metadata address   s82 1 if the last tile of a head has clamped
   rows, else -1   s83 / s84 bytes per Q / dO row   masked: s85 bytes of metadata per tile   s86 first token of the wave, s87 one
-  past its last   s[90:91] all ones if not all of them exist
+  past its last   s[90:91] all ones if not all of them exist   s92 1 if dS^T leaves as streaming stores
 D-waves: v[168:175] P handed over   v[176:183] dS packed   v[184:199] delta*scale of 16 rows
   v216 P hand-over read address   v217 metadata read address   v218 dS^T staging write address
 """
@@ -205,6 +205,15 @@ def p_ragged(u, ahead):
             f"LVX_BWD_RAGGED{u}{ahead}_%=:", *move("v_sub_u32"), f"s_branch LVX_BWD_WALKED{u}{ahead}_%="]
 
 
+def p_store(hint):
+    return [f"global_store_dwordx4 v{G_CP0}, {vr(CPD, 4)}, s[78:79]{hint}", f"global_store_dwordx4 v{G_CP1}, {vr(CPD + 4, 4)}, s[78:79]{hint}"]
+
+
+def p_keep(u):
+    """Out of line: the launch's dS^T fits the memory-side cache and is stored without the streaming hint."""
+    return [f"LVX_BWD_KEEP{u}_%=:", *p_store(""), f"s_branch LVX_BWD_STORED{u}_%="]
+
+
 def p_mask(u):
     """Out of line: some row of tile i-1 cuts this wave's tokens.  P's elements outside their row's interval
     become 0; the intervals of the lane's 16 rows are read 8 rows at a time into the registers the LSE had."""
@@ -236,7 +245,7 @@ def p_step(u, seed):
     par = u & 1                                                  # (i + 1) & 1: P(i-1) hand-over, dS^T(i-3)
     carry, new = SET[u & 1], SET[(u + 1) & 1]
     # tile i+1 has landed: after its loads this wave issued 2 stores, 4 (wave 0: 5) loads and 2 stores
-    e("s_waitcnt vmcnt(6)" if "storefirst" in OPTS else "s_waitcnt vmcnt(8)")
+    e("s_waitcnt vmcnt(8)")
     e(f"s_waitcnt lgkmcnt({st.n_lds})")
     e("s_barrier")
     for vg in range(4):
@@ -279,16 +288,9 @@ def p_step(u, seed):
     fetch = p_fetch(u, 3)
     if u == 5:      # the last step of the last trip requests nothing: the steps after the loop do
         fetch = [["s_cmp_eq_u32 s64, 1", "s_cbranch_scc1 LVX_BWD_NOFETCH_%="] + flat(fetch) + ["LVX_BWD_NOFETCH_%=:"]]
-    store = [lambda: st.wait("cp0"), f"global_store_dwordx4 v{G_CP0}, {vr(CPD, 4)}, {sr(ws_old, 2)}",
-             lambda: st.wait("cp1"), f"global_store_dwordx4 v{G_CP1}, {vr(CPD + 4, 4)}, {sr(ws_old, 2)}"]
-    if "storefirst" in OPTS:
-        tail += store + fetch
-    else:
-        # the stores read the workspace address of tile i-3 before the walk overwrites it: keep a copy
-        tail += [f"s_mov_b64 s[78:79], {sr(ws_old, 2)}"] + fetch
-        store[1] = f"global_store_dwordx4 v{G_CP0}, {vr(CPD, 4)}, s[78:79]"
-        store[3] = f"global_store_dwordx4 v{G_CP1}, {vr(CPD + 4, 4)}, s[78:79]"
-        tail += store
+    # the stores read the workspace address of tile i-3 before the walk overwrites it: keep a copy
+    tail += [f"s_mov_b64 s[78:79], {sr(ws_old, 2)}"] + fetch + [lambda: st.wait("cp1")]
+    tail.append(["s_cmp_eq_u32 s92, 0", f"s_cbranch_scc1 LVX_BWD_KEEP{u}_%=", *p_store(" nt"), f"LVX_BWD_STORED{u}_%=:"])
 
     mf = []
     for k in range(NOP):
@@ -475,7 +477,7 @@ def main():
     if ROLE == "p":
         lines += ["s_branch LVX_BWD_END_%="] + p_ragged(0, 2)
         for u in range(6):
-            lines += p_ragged(u, 3) + (p_mask(u) if MASKED else [])
+            lines += p_ragged(u, 3) + p_keep(u) + (p_mask(u) if MASKED else [])
         lines.append("LVX_BWD_END_%=:")
     print("// generated by gen_bwd_loop.py - do not edit")
     for l in lines:

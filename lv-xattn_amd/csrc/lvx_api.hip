@@ -539,8 +539,7 @@ static size_t dkv_scratch_bytes(const lvx_attn_shape* s) {
 // rounded to bf16 afterwards (fp32 atomics into one slice were measured slower).  Returns
 // the number of splits (1: none) and the tokens per split.
 static int dq_k_splits(const lvx_attn_shape* s, int32_t row_count, int* split_len) {
-    const int tile_rows = s->kv_start ? 256 : 512;      // as launch_gemm picks them
-    const int tiles = row_count > 256 ? (row_count + tile_rows - 1) / tile_rows : 1;
+    const int tiles = (row_count + 255) / 256;          // of launch_gemm's 256-row tile
     const int wgs = s->B * s->Hq * tiles;
     const int blocks = (s->Lkv + 127) / 128;
     int ks = 1;
@@ -634,6 +633,13 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     p.ds_ws = static_cast<uint16_t*>(workspace);
     p.ws_ld = rows * 128;          // one token block: (rows / 32) tiles of 128 x 32
     p.ws_bh = tokens * rows;
+    // dS^T is written once and read once.  Where it does not fit the memory-side cache (256 MB) it should not
+    // push out of the caches what is read again (Q and dO tiles by the token blocks of a head, K by the dQ
+    // GEMM): streaming stores, streaming loads.  us, forward + backward, without and with: 6404 tokens x 4096 rows x
+    // 32 heads (1.7 GB) 1879 -> 1821, x 1024 rows (0.4 GB) 794 -> 774, heads of 64 x 2048 rows (0.8 GB) 676 ->
+    // 595, 2 x 3000 rows with image intervals 1205 -> 1152.  Where it fits, the hint costs a little: x 512 rows of
+    // heads of 64 (0.2 GB) 208 -> 213, rounds of 256 rows (0.1 GB) 2940 -> 2966 for sixteen.
+    p.ds_stream = (int64_t)s->B * s->Hq * p.ws_bh * 2 > ((int64_t)240 << 20);
 
     const BwdWorkspace wsl = bwd_workspace(s, row_count);
     char* const wsb = static_cast<char*>(workspace);
@@ -729,6 +735,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     g.c_outer = dq->stride_b; g.c_inner = dq->stride_h;
     g.k_len = s->kv_len;
     g.a_tiled_m = (int)(rows / 32);
+    g.a_stream = p.ds_stream;
     g.k_range = hull;            // [B][M tiles][2]: the group hulls are per M tile of this GEMM
     g.m_order = order;
     fill_grid(g, row_count, s->D, 1, s->B * s->Hq);

@@ -22,8 +22,9 @@
 // so dQ is not formed here: the D-waves gather scale*dS (bf16) in LDS and the
 // group streams it to a workspace in HBM, one contiguous 8 KB tile
 // [128 tokens][32 rows] per step, indexed [b, h, token block, row tile]; a
-// batched GEMM (launched by the caller right after) contracts it with K.  The workspace costs 2 bytes per (row, token, head),
-// written once and read once.
+// batched GEMM (launched by the caller right after) contracts it with K.  The workspace costs 2 bytes per
+// (row, token, head), written once and read once; the caller says when it is large enough for
+// streaming stores (ds_stream).
 //
 // All MFMA are 32x32x16 bf16.  A operands come from LDS.  The Q and dO tiles
 // ([32 rows][128] bf16, 8 KiB each) go from global memory straight into LDS
@@ -93,6 +94,7 @@ constexpr float LOG2E = 1.4426950408889634f;
       "{s62}"(uniform32(lds0 + (uint32_t)slice * 2048u)), "{s63}"(uniform32(meta0 + meta_w)),                        \
       "{s65}"(uniform32(wave < META_WAVES ? 1 : 0)), "{s82}"(uniform32(ragged ? 1 : -1)),                            \
       "{s85}"(uniform32(meta_w ? BM * 4 : 256)), "{s86}"(uniform32(slice_lo)), "{s87}"(uniform32(slice_lo + 32)),     \
+      "{s92}"(uniform32(p.ds_stream)),                                                                               \
       "{s[90:91]}"(uniform64(slice_valid ? (int64_t)0 : (int64_t)-1))                                                \
     : "memory", "vcc", "scc", "m0", "s78", "s79", "s88", "s89", "v229", "v230", LVX_BWD_LOOP_CLOBBERS
 #define LVX_BWD_D_OPERANDS                                                                                           \
@@ -299,8 +301,14 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     auto copy_out = [&](const uint16_t* dst, int64_t ws_off) {
         const u32x4 a = *reinterpret_cast<const u32x4*>(dst + cp_token * DSS + cp_part * 8);
         const u32x4 c2 = *reinterpret_cast<const u32x4*>(dst + (cp_token + 64) * DSS + cp_part * 8);
-        *reinterpret_cast<u32x4*>(ws_lane + ws_off) = a;
-        *reinterpret_cast<u32x4*>(ws_lane + ws_off + 64 * BM) = c2;
+        u32x4* const o = reinterpret_cast<u32x4*>(ws_lane + ws_off);
+        if (p.ds_stream) {
+            __builtin_nontemporal_store(a, o);
+            __builtin_nontemporal_store(c2, o + 64 * BM / 8);
+        } else {
+            o[0] = a;
+            o[64 * BM / 8] = c2;
+        }
     };
 
     // The work on a tile is spread over three steps so that, inside every wave, the

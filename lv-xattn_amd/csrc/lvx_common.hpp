@@ -135,6 +135,11 @@ __device__ __forceinline__ void dma16(const char* sbase, uint32_t voff, uint32_t
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte), "v"(voff), "s"(sbase)
                  : "memory", "m0");
 }
+// the same, not kept in the caches: for what nobody reads again
+__device__ __forceinline__ void dma16_stream(const char* sbase, uint32_t voff, uint32_t lds_byte) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_byte), "v"(voff), "s"(sbase)
+                 : "memory", "m0");
+}
 __device__ __forceinline__ void dma16_addr(const char* addr, uint32_t lds_byte) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_byte), "v"(addr) : "memory", "m0");
 }

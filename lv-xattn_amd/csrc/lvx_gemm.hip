@@ -98,7 +98,8 @@ struct Region {
 };
 
 // GM x GN waves, each WM x WN MFMA tiles: work-group tile (32 WM GM) x (32 WN GN).
-template <bool A_MCONTIG, bool B_NCONTIG, int GM, int GN, int WM, int WN, int NS, bool F16>
+// STREAM_A: A is loaded with the streaming hint (as a test at run time it costs a one-round dQ launch 10 %).
+template <bool A_MCONTIG, bool B_NCONTIG, int GM, int GN, int WM, int WN, int NS, bool F16, bool STREAM_A = false>
 __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     using E = Elt<F16>;
     static_assert(GM * GN == 8, "8 waves");
@@ -198,7 +199,8 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
         if (krem >= BK) {
 #pragma unroll
             for (int j = 0; j < LPG; ++j)
-                dma16(j < LPG_A ? ab : bb, voff[j], slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
+                if (STREAM_A && j < LPG_A) dma16_stream(ab, voff[j], slot + j * 8192);
+                else dma16(j < LPG_A ? ab : bb, voff[j], slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
         } else {
             const char* zc = reinterpret_cast<const char*>(zero_chunk);
 #pragma unroll
@@ -692,8 +694,10 @@ hipError_t launch_cfg_t(const GemmParams& p, int grid, bool a_mcontig, bool b_nc
         return launch1((gemm_kernel<false, true, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
     else if (a_mcontig && !b_ncontig)
         return launch1((gemm_kernel<true, false, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
-    else
+    else if (!p.a_stream)
         return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
+    else
+        return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16, true>), dim3(grid), dim3(512), st, p);
 }
 
 template <int GM, int GN, int WM, int WN, int NS>
@@ -738,8 +742,10 @@ bool gemm_tile_ok(const GemmParams& p, bool a_mcontig, bool b_ncontig) {
 // of 256 x 256, or 256 x 128 where that fills the chip's rounds better: a 128-wide tile takes about 0.6 of
 // the time of a 256-wide one (2046 x 4096 x 4096: 128 tiles of 256 on 256 CUs 81 us, 256 of 128 60; 12808 x 4096 x
 // 1024 twice: 2 rounds 176 us, 4 rounds 208).
-// A narrow C (the dQ GEMM): 512 x 128, or 256 x 128 when there are not 512 rows or when M tiles have
-// their own contraction ranges (k_range is kept per 256 rows: finer ranges skip more).
+// A narrow C (the dQ GEMM): 256 x 128, four stages, at which one load of a wave covers whole cache lines of
+// dS^T's 64-byte rows (two tokens x 256 rows; of a 512-row tile it takes one token, half of each line, and the
+// streaming hint then costs a second fetch: 6404 tokens x 4096 rows x 32 heads 1868 us a step against 1821),
+// and the M tiles of a masked launch have finer contraction ranges.
 hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipStream_t st) {
     for (int i = 0; i < p.nprob; ++i) {
         const GemmProblem& pr = p.prob[i];
@@ -757,7 +763,6 @@ hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipS
     }
     if (p.N > 128) return launch_cfg<2, 4, 4, 2, 4>(p, a_mcontig, b_ncontig, st);
     if (p.m_order && (!p.k_range || p.nprob != 1 || p.k_splits > 1 || p.N > 128)) return hipErrorInvalidValue;
-    if (p.M > 256 && !p.k_range) return launch_cfg<8, 1, 2, 4, 3>(p, a_mcontig, b_ncontig, st);
     return launch_cfg<4, 2, 2, 2, 4>(p, a_mcontig, b_ncontig, st);
 }
 

@@ -117,6 +117,7 @@ struct BwdParams {
     uint16_t* ds_ws;           // dS^T workspace [B*Hq][token blocks][row tiles][128 tokens][32 rows]
     int64_t ws_ld;             // elements per token block (row tiles * 4096)
     int64_t ws_bh;             // elements per (b, h) slab
+    int ds_stream;             // 1: dS^T is stored with streaming stores (see lvx_bwd)
     void* dk;
     void* dv;
     Strides3 qs, ks, vs, dos, dks, dvs;
@@ -257,6 +258,7 @@ struct GemmParams {
     // a_tiled_m > 0: A (stored [K][M]) is cut into contiguous [128 k][32 m] tiles,
     // a_tiled_m of them per block of 128 k; lda is ignored
     int a_tiled_m;
+    int a_stream;              // 1: A is loaded with the streaming hint (A and B stored [K][..] only)
 };
 
 hipError_t launch_fwd(const FwdParams& p, bool masked, hipStream_t st);   // p.bias selects the bias variant
