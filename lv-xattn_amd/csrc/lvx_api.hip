@@ -659,11 +659,13 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     int split_len = 0;
     const int ks = dq_k_splits(s, row_count, &split_len);
     float* const dq32 = ks > 1 ? reinterpret_cast<float*>(wsb + wsl.dq32) : nullptr;
+    // the token blocks several work-groups share, and the fp32 scratch of the call that sums them
+    SharedBlocks sb{s->B, s->Hkv, s->Lkv, s->D, p.n_kv_blocks, p.n_blocks, p.blocks_per_xcd, p.whole_blocks};
     {
         float* meta = reinterpret_cast<float*>(wsb + wsl.meta);
         MetaParams mp{lse, delta, meta, s->B, s->Hq, s->Lq, row_begin, row_begin + row_count, (int)(rows / 32), s->scale};
-        mp.zero_dst[0] = reinterpret_cast<uint32_t*>(scratch);
-        mp.zero_n16[0] = scratch ? (int64_t)(dkv_scratch_bytes(s) / 16) : 0;
+        mp.scratch = scratch;
+        mp.sb = sb;
         hipError_t em = launch_bwd_meta(mp, st);
         if (em != hipSuccess) return static_cast<int>(em);
         p.meta = meta;
@@ -699,22 +701,8 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     hipError_t e = launch_bwd(p, s->kv_start != nullptr, st);
     if (e != hipSuccess) return static_cast<int>(e);
     if (scratch) {
-        // scratch memory order is [B, Lkv, Hkv, D]: cast with (H, L) = (Lkv, Hkv); dK and dV in one launch
-        CastParams cp{};
-        cp.f16 = p.f16;
-        cp.D = s->D;
-        cp.src = scratch;
-        cp.dst = static_cast<uint16_t*>(dk->ptr);
-        cp.ds = Strides3{dk->stride_b, dk->stride_s, dk->stride_h};
-        cp.src2 = scratch + dkv_elems;
-        cp.dst2 = static_cast<uint16_t*>(dv->ptr);
-        cp.ds2 = Strides3{dv->stride_b, dv->stride_s, dv->stride_h};
-        cp.B = s->B; cp.H = s->Lkv; cp.L = s->Hkv;
-        if (p.whole_blocks > 0) {
-            cp.skip_bpx = p.blocks_per_xcd; cp.skip_whole = p.whole_blocks;
-            cp.skip_nkvb = p.n_kv_blocks; cp.skip_nblocks = p.n_blocks;
-        }
-        e = launch_cast(cp, st);
+        CastSharedParams cp{sb, scratch, static_cast<uint16_t*>(dk->ptr), static_cast<uint16_t*>(dv->ptr), st3(dk), st3(dv), p.f16};
+        e = launch_cast_shared(cp, st);
         if (e != hipSuccess) return static_cast<int>(e);
     }
 

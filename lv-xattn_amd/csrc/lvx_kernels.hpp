@@ -166,6 +166,13 @@ struct LiveParams {
 };
 hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st);
 
+// The token blocks of a backward launch that several work-groups share, hence whose dK / dV are summed in the
+// fp32 scratch [2][B, Lkv, Hkv, D].  They are listed (b, kv head, block) with the block fastest, the
+// sample next; XCD x takes blocks_per_xcd of them and shares all but its first `whole`.
+struct SharedBlocks {
+    int B, Hkv, Lkv, D, n_kv_blocks, n_blocks, blocks_per_xcd, whole;
+};
+
 // Row metadata of the backward in the form its kernel consumes, one 256-byte
 // record per (b, h, 32-row tile of the window).
 struct MetaParams {
@@ -174,26 +181,25 @@ struct MetaParams {
     float* out;
     int B, Hq, Lq, row_begin, row_end, n_tiles;
     float scale;
-    // up to two regions the same launch zero-fills (the fp32 scratches the call accumulates
-    // into); dst 16-byte aligned, n16 = number of 16-byte chunks, 0: none
-    uint32_t* zero_dst[2];
-    int64_t zero_n16[2];
+    float* scratch;            // null, or the fp32 dK / dV scratch whose shared token blocks the same launch zeroes
+    SharedBlocks sb;
     int meta_blocks;           // filled by the launcher: blocks [0, meta_blocks) write records
 };
 
+// The shared token blocks of the scratch, rounded into dK and dV.
+struct CastSharedParams {
+    SharedBlocks sb;
+    const float* scratch;
+    uint16_t* dk;
+    uint16_t* dv;
+    Strides3 dks, dvs;
+    int f16;
+};
 
 struct CastParams {
     const float* src;
     uint16_t* dst;
     Strides3 ds;
-    // a second tensor of the same sizes, cast by the same launch (null: none)
-    const float* src2;
-    uint16_t* dst2;
-    Strides3 ds2;
-    // the fp32 dK / dV scratch of the backward, (H, L) = (tokens, kv heads): rows of token blocks that
-    // the kernel wrote directly (the first skip_whole of every skip_bpx blocks of the list (b, kv
-    // head, block), skip_nkvb blocks per (b, kv head), skip_nblocks in all) are left alone.  skip_bpx 0: none.
-    int skip_bpx, skip_whole, skip_nkvb, skip_nblocks;
     int B, H, L;
     int transposed;   // 0: src is [B*H][L][D]; 1: src is [B*H][D][L]
     int nsum;         // transposed only: the result is the sum of nsum such sources (0 or 1: one),
@@ -266,6 +272,7 @@ hipError_t launch_merge(const MergeParams& p, hipStream_t st);
 hipError_t launch_preprocess(const PreParams& p, hipStream_t st);
 hipError_t launch_bwd(const BwdParams& p, bool masked, hipStream_t st);
 hipError_t launch_cast(const CastParams& p, hipStream_t st);
+hipError_t launch_cast_shared(const CastSharedParams& p, hipStream_t st);
 hipError_t launch_bwd_meta(const MetaParams& p, hipStream_t st);
 
 // Backward of the 128-wide RMS norm: rows of dy, x [M][heads][128] (row strides ldy, ldx), r [M][heads].
