@@ -92,7 +92,8 @@ bool fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, con
          int64_t row_count, const OptTensor& kv_len, const OptTensor& kv_start, const OptTensor& kv_end, int64_t kv_splits,
          const OptTensor& ws, const OptTensor& acc_o, const OptTensor& acc_l) {
     lvx_attn_shape s;
-    if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end) || !plain4(o, q, q.scalar_type()) || !rows_ok(lse, q)) return false;
+    if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end) || !plain4(o, q, q.scalar_type()) || o.sizes() != q.sizes() || !rows_ok(lse, q))
+        return false;
     const lvx_tensor tq = t4(q), tk = t4(k), tv = t4(v), to = t4(o);
     void* const wp = ws ? ws->data_ptr() : nullptr;
     const size_t wb = ws ? ws->nbytes() : 0;

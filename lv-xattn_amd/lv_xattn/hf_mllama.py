@@ -77,27 +77,37 @@ def _mask_bias(mask: torch.Tensor) -> torch.Tensor:
     return bias
 
 
-_interval_cache: list = []  # [key, Mask or None, the mask it was made from] of the last one looked at
+_interval_cache: tuple = ()     # (key, Mask or None, the mask it was made from) of the last one looked at
 
 
-def _mask_intervals(mask: torch.Tensor):
+def _mask_intervals(mask: torch.Tensor, query: torch.Tensor, lkv: int):
     """The interval mask that says all that transformers' additive `mask` says (ops.mask_intervals), or
     None: the usual case, a row looks at the tiles of the images before it.  Every layer of a model
-    gets the same mask, so the last answer is kept, with the mask, as `_mask_bias` keeps its own."""
+    gets the same mask, so the last answer is kept, with the mask, as `_mask_bias` keeps its own, for
+    calls on the stream it was made on.  A mask of another form or place than the query's rows and keys, and
+    one first seen while a graph is captured (the answer has to come back to the host), are `_mask_bias`'s."""
+    global _interval_cache
+    if tuple(mask.shape) != (query.shape[0], 1, query.shape[2], lkv) or mask.device != query.device:
+        return None
     version = None if mask.is_inference() else mask._version
-    key = (mask.data_ptr(), version, tuple(mask.shape), tuple(mask.stride()), mask.dtype, mask.device)
-    if version is not None and _interval_cache and _interval_cache[0] == key:
-        return _interval_cache[1]
+    key = (mask.data_ptr(), version, tuple(mask.shape), tuple(mask.stride()), mask.dtype, mask.device,
+           torch.cuda.current_stream(mask.device).cuda_stream)
+    kept = _interval_cache          # read once: another thread may put its own in place
+    if version is not None and kept and kept[0] == key:
+        return kept[1]
+    if torch.cuda.is_current_stream_capturing():
+        return None
     intervals = ops.mask_intervals(mask)
     if version is not None:
-        _interval_cache[:] = [key, intervals, mask]
+        _interval_cache = (key, intervals, mask)
     return intervals
 
 
 def clear_mask_cache() -> None:
     """Drops the converted masks `_mask_bias` (an fp32 tensor of the mask's size) and `_mask_intervals` keep."""
+    global _interval_cache
     _bias_cache.clear()
-    _interval_cache.clear()
+    _interval_cache = ()
 
 
 def lv_xattn_attention_forward(module, query, key, value, attention_mask: Optional[torch.Tensor],
@@ -119,7 +129,7 @@ def lv_xattn_attention_forward(module, query, key, value, attention_mask: Option
     mask = intervals = None
     if attention_mask is not None:
         mask = attention_mask[..., :query.shape[2], :key.shape[2]]
-        intervals = _mask_intervals(mask)
+        intervals = _mask_intervals(mask, query, key.shape[2])
     if (mask is None or intervals is not None) and not (torch.is_grad_enabled() and (
             query.requires_grad or key.requires_grad or value.requires_grad)):
         out = _attn_forward(query, key, value, False, scaling, None, rounds=1, batched=True, mask=intervals, _token_major=True)[3]
@@ -173,7 +183,7 @@ def _recompute_forward(self, hidden_states, cross_attention_states=None, past_ke
     bias = []
     if mask is None and attention_mask is not None:
         dense = attention_mask[..., :q_len, :cross_attention_states.shape[1]]
-        mask = _mask_intervals(dense)
+        mask = _mask_intervals(dense, query, cross_attention_states.shape[1])
         if mask is None:
             bias = [_mask_bias, dense]
     out = _recompute[key](query, cross_attention_states.to(query.dtype), self.k_proj.weight, self.v_proj.weight,

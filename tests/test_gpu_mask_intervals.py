@@ -35,3 +35,48 @@ def test_mask_intervals(dtype, B, Lq, Lkv, offset):
         gap = torch.zeros_like(mask)
         gap[0, 0, 0, Lkv // 2] = float("-inf")
         assert ops.mask_intervals(gap) is None
+
+
+class _Layer(torch.nn.Module):
+    k_norm = None
+    is_causal = False
+
+
+def _attend(q, k, v, mask):
+    from lv_xattn import hf_mllama
+    hf_mllama.clear_mask_cache()
+    return hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)[0]
+
+
+def test_masks_of_another_form_take_the_general_path():
+    """A mask shared by the batch and one in host memory give what the mask written out on the GPU gives;
+    one with fewer keys than there are is refused as it is without intervals."""
+    torch.manual_seed(0)
+    q, k, v = (torch.randn(2, h, n, 64, device=DEV, dtype=torch.bfloat16) for h, n in ((8, 5), (2, 333), (2, 333)))
+    mask = torch.zeros(1, 1, 5, 333, device=DEV, dtype=torch.bfloat16)
+    mask[..., 100:] = torch.finfo(torch.bfloat16).min
+    want = _attend(q, k, v, mask.expand(2, 1, 5, 333).contiguous())
+    for other in (mask, mask.cpu()):
+        torch.testing.assert_close(_attend(q, k, v, other), want, rtol=2.0 ** -7, atol=2.0 ** -7)
+    with pytest.raises(ValueError):
+        _attend(q, k, v, mask.expand(2, 1, 5, 333)[..., :200].contiguous())
+
+
+def test_a_mask_first_seen_under_capture():
+    """In inference mode a mask has no version by which an answer could be kept: a captured call takes the path
+    that asks nothing of the host, and every replay reads the mask as it is then."""
+    torch.manual_seed(1)
+    with torch.inference_mode():
+        q, k, v = (torch.randn(1, h, n, 64, device=DEV, dtype=torch.bfloat16) for h, n in ((8, 5), (2, 333), (2, 333)))
+        mask = torch.zeros(1, 1, 5, 333, device=DEV, dtype=torch.bfloat16)
+        _attend(q, k, v, mask)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = _attend(q, k, v, mask)
+        for visible in (333, 100, 7):
+            mask.zero_()
+            mask[..., visible:] = torch.finfo(torch.bfloat16).min
+            graph.replay()
+            torch.cuda.synchronize()
+            torch.testing.assert_close(out, _attend(q, k, v, mask), rtol=2.0 ** -7, atol=2.0 ** -7)
