@@ -222,6 +222,7 @@ int lvx_bwd(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tensor* 
             const lvx_tensor* dq, const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate,
             int32_t row_begin, int32_t row_count, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Never less for more rows: a workspace of the longest window of a call serves all its windows. */
 size_t lvx_bwd_workspace_bytes(const lvx_attn_shape* shape, int32_t row_count);
 
 /*

@@ -550,6 +550,21 @@ static int dq_k_splits(const lvx_attn_shape* s, int32_t row_count, int* split_le
     return (blocks + per - 1) / per;
 }
 
+// Bytes of the split contraction's partial tiles that a window of up to row_count rows can need.  Fewer rows may
+// need more: a window of another 256 rows has half the splits (32 heads x 6404 tokens: 8 splits of
+// 256 rows 33.6 MB, 4 of 257 18.9 MB), and a call sizes its workspace for the longest of its windows.
+static size_t dq_partial_bytes(const lvx_attn_shape* s, int32_t row_count) {
+    size_t most = 0;
+    for (int32_t r = 0; r < row_count;) {
+        r = row_count - r > 256 ? r + 256 : row_count;
+        int split_len;
+        const int ks = dq_k_splits(s, r, &split_len);
+        if (ks <= 1) break;             // nor do longer windows split
+        most = std::max(most, (size_t)ks * s->B * s->Hq * (((size_t)r + 31) / 32 * 32) * s->D * sizeof(float));
+    }
+    return most;
+}
+
 // Regions of the backward workspace, in order: dS^T tiles; fp32 dK/dV scratch (split-steps mode
 // with bf16 outputs); row metadata records (2 floats per row and head); fp32 dQ partial tiles,
 // one slice per split (split dQ contraction only); with an interval mask the live-tile tables (group hulls, runs
@@ -571,10 +586,7 @@ static BwdWorkspace bwd_workspace(const lvx_attn_shape* s, int32_t row_count) {
     w.ds = off; off += (size_t)s->B * s->Hq * tokens * rows * sizeof(uint16_t);
     w.dkv = off; off += dkv_scratch_bytes(s);
     w.meta = off; off += (size_t)s->B * s->Hq * rows * 2 * sizeof(float);
-    int sl;
-    w.dq32 = off;
-    const int ks = dq_k_splits(s, row_count, &sl);
-    if (ks > 1) off += (size_t)ks * s->B * s->Hq * rows * s->D * sizeof(float);
+    w.dq32 = off; off += dq_partial_bytes(s, row_count);
     if (s->kv_start) {
         const size_t nkb = tokens / 128;
         w.hull = off; off += up16((size_t)s->B * w.n_groups * 2 * sizeof(int32_t));
