@@ -31,6 +31,7 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
+from torch.autograd.forward_ad import unpack_dual
 
 from . import ops
 from ._lib import LvxError
@@ -130,8 +131,10 @@ def lv_xattn_attention_forward(module, query, key, value, attention_mask: Option
     if attention_mask is not None:
         mask = attention_mask[..., :query.shape[2], :key.shape[2]]
         intervals = _mask_intervals(mask, query, key.shape[2])
-    if (mask is None or intervals is not None) and not (torch.is_grad_enabled() and (
-            query.requires_grad or key.requires_grad or value.requires_grad)):
+    # the autograd function is only passed by where it has nothing to do: no gradient is recorded, and no input
+    # carries a forward-mode tangent, which it refuses (it has no jvp) and the kernels would silently drop
+    if (mask is None or intervals is not None) and not any(
+            (torch.is_grad_enabled() and t.requires_grad) or unpack_dual(t).tangent is not None for t in (query, key, value)):
         out = _attn_forward(query, key, value, False, scaling, None, rounds=1, batched=True, mask=intervals, _token_major=True)[3]
         return out.transpose(1, 2).contiguous(), None
     if _attention is None:
