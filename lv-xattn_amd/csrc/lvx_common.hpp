@@ -171,8 +171,14 @@ __device__ __forceinline__ int64_t uniform64(int64_t x) {
 template <typename T>
 __device__ __forceinline__ const T* uniform_ptr(const T* x) { return reinterpret_cast<const T*>(uniform64((int64_t)(uintptr_t)x)); }
 
+// The wait states between an MFMA and the inline assembly that reads its result next: the compiler sees neither
+// that the assembly is a VALU instruction nor that 12 of them have to pass (a 32x32x16 MFMA has 8
+// passes), and leaves as few as none.
+__device__ __forceinline__ void mfma_settle(f32x16& a) { asm volatile("s_nop 11" : "+v"(a)); }
+__device__ __forceinline__ void mfma_settle(f32x16& a, f32x16& b) { asm volatile("s_nop 11" : "+v"(a), "+v"(b)); }
+
 // max of three (one instruction; fmaxf chains cost an extra canonicalising
-// v_max per MFMA result)
+// v_max per MFMA result).  MFMA results go through mfma_settle first.
 __device__ __forceinline__ float max3(float a, float b, float c) {
     float r;
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));

@@ -250,6 +250,7 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
             }
         }
 
+        mfma_settle(s0, s1);
         float mx = max3(s0[0], s1[0], s0[1]);
         mx = max3(mx, s1[1], s0[2]);
 #pragma unroll
@@ -755,6 +756,7 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
                 if (kv < my_s || kv >= my_e) s[v] = -INFINITY;
             }
         }
+        mfma_settle(s);
         float mx = max3(s[0], s[1], s[2]);
 #pragma unroll
         for (int v = 3; v < 15; v += 2) mx = max3(mx, s[v], s[v + 1]);

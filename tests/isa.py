@@ -1,0 +1,111 @@
+"""The gfx950 code of the built library, read for what the compiler cannot check: inline assembly is opaque
+to its hazard recognizer and to its bookkeeping of loads in flight, so these look at every path of the
+finished machine code instead."""
+import os
+import re
+import shutil
+import subprocess
+
+OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
+
+# Wait states between a 32x32x16 MFMA (8 passes) and whatever else touches its result: passes + 4 on gfx950
+MFMA_WAIT = 12
+
+
+class Ins:
+    __slots__ = ("addr", "op", "args", "target")
+
+    def __init__(self, addr, op, args, target=None):
+        self.addr, self.op, self.args, self.target = addr, op, args, target
+
+    def __repr__(self):
+        return f"{self.addr:x}: {self.op} {', '.join(self.args)}"
+
+
+def functions(lib, tmp):
+    """{name: [Ins]} of every kernel in the library's code objects (extracted into the folder `tmp`)."""
+    shutil.copy(lib, os.path.join(tmp, "lib.so"))
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=tmp, check=True, capture_output=True)
+    out = {}
+    for f in sorted(os.listdir(tmp)):
+        if "gfx950" in f:
+            text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", f], cwd=tmp, check=True, capture_output=True, text=True).stdout
+            out.update(parse(text))
+    return out
+
+
+def parse(text):
+    out, body = {}, None
+    for line in text.splitlines():
+        m = re.match(r"[0-9a-f]+ <(\S+)>:$", line)
+        if m:
+            if not m.group(1).startswith("LVX_"):       # a label of a generated loop
+                body = out[m.group(1)] = []
+            continue
+        m = re.match(r"\s+(\S+)\s*(.*?)\s*// ([0-9A-F]+): ([0-9A-F]+)", line)
+        if m is None or body is None:
+            continue
+        op, args, addr, word = m.groups()
+        addr, target = int(addr, 16), None
+        if op.startswith(("s_branch", "s_cbranch")):    # a signed distance in words from the next instruction
+            target = addr + 4 + 4 * ((int(word, 16) & 0xffff ^ 0x8000) - 0x8000)
+        body.append(Ins(addr, re.sub(r"_e(32|64)$", "", op), [a.strip() for a in args.split(",")], target))
+    return {n: b for n, b in out.items() if b}
+
+
+def regs(arg):
+    """{(file, number)} of the vector registers an operand names."""
+    arg = arg.split(" ")[0].strip("-|")
+    m = re.match(r"([va])\[(\d+):(\d+)\]$", arg)
+    if m:
+        return {(m.group(1), r) for r in range(int(m.group(2)), int(m.group(3)) + 1)}
+    m = re.match(r"([va])(\d+)$", arg)
+    return {(m.group(1), int(m.group(2)))} if m else set()
+
+
+def touched(ins):
+    return set().union(*(regs(a) for a in ins.args)) if ins.args else set()
+
+
+def after(body, index):
+    """Index of an instruction by address, and the successors of instruction i."""
+    def successors(i):
+        ins = body[i]
+        if ins.op == "s_endpgm":
+            return []
+        nxt = [] if ins.op == "s_branch" else [i + 1]
+        if ins.target is not None and ins.target in index:
+            nxt.append(index[ins.target])
+        return [n for n in nxt if n < len(body)]
+    return successors
+
+
+def mfma_results_touched_early(body):
+    """[(mfma, instruction, wait states)]: instructions that read or write an MFMA's result - another MFMA that
+    adds to it aside - fewer than MFMA_WAIT wait states behind it on some path."""
+    index = {ins.addr: i for i, ins in enumerate(body)}
+    successors = after(body, index)
+    found = []
+    for i, ins in enumerate(body):
+        if not ins.op.startswith("v_mfma"):
+            continue
+        result = regs(ins.args[0])
+        best = {}
+        todo = [(n, 0) for n in successors(i)]
+        while todo:
+            j, waited = todo.pop()
+            if waited >= MFMA_WAIT or best.get(j, MFMA_WAIT) <= waited:
+                continue
+            best[j] = waited
+            x = body[j]
+            if x.op.startswith("v_mfma"):
+                if (regs(x.args[1]) | regs(x.args[2])) & result:
+                    found.append((ins, x, waited))
+                if regs(x.args[0]) == result:       # its own wait is counted from there
+                    continue
+            elif touched(x) & result:
+                found.append((ins, x, waited))
+                continue
+            step = int(x.args[0], 0) + 1 if x.op == "s_nop" else 1
+            todo += [(n, waited + step) for n in successors(j)]
+    return found

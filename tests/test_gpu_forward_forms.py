@@ -66,3 +66,18 @@ def test_wide_form(D, dtype, Hq, Hkv, Lq, Lkv, splits, mask, monkeypatch):
 def test_few_rows_form(D, dtype, Hq, Hkv, Lq, Lkv, splits, mask, monkeypatch):
     monkeypatch.setenv("LVX_FWD_WIDE", "2")
     _check(D, dtype, 2, Hq, Hkv, Lq, Lkv, splits, mask, Lq * 1000 + Lkv + 1)
+
+
+# nothing in a forward depends on the order in which anything arrives
+@pytest.mark.parametrize("form", ["0", "1", "2"])
+@pytest.mark.parametrize("D", [128, 64, 32])
+def test_every_form_repeats_itself(D, form, monkeypatch):
+    import lv_xattn
+    monkeypatch.setenv("LVX_FWD_WIDE", form)
+    g = torch.Generator(device=DEV).manual_seed(D)
+    q, k, v = (torch.empty(2, h, n, D, device=DEV, dtype=torch.bfloat16).normal_(generator=g) for h, n in ((32, 7), (8, 3000), (8, 3000)))
+    first = None
+    for _ in range(20):
+        _, _, _, o, lse = lv_xattn._attn_forward(q, k, v, False, D ** -0.5, None, rounds=1, batched=True)
+        first = first or (o, lse)
+        assert torch.equal(o, first[0]) and torch.equal(lse, first[1])

@@ -1,0 +1,41 @@
+"""What inline assembly leaves to the kernels' author, checked on the built library's machine code (see isa.py)."""
+import os
+
+import pytest
+
+import isa
+
+needs_objdump = pytest.mark.skipif(not os.path.exists(isa.OBJDUMP), reason="no llvm-objdump")
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    from lv_xattn import _lib
+    _lib.load()
+    return isa.functions(_lib.LIB_PATH, str(tmp_path_factory.mktemp("code")))
+
+
+@needs_objdump
+def test_mfma_results_have_their_wait_states(kernels):
+    assert sum(any(i.op.startswith("v_mfma") for i in body) for body in kernels.values()) > 50
+    early = {name: found for name, found in ((n, isa.mfma_results_touched_early(b)) for n, b in kernels.items()) if found}
+    assert not early, {name: found[:2] for name, found in early.items()}
+
+
+PLANTED = """
+0000000000001000 <kernel>:
+\tv_mfma_f32_32x32x16_bf16 v[4:19], v[20:23], v[82:85], 0    // 000000001000: D3B58004 02
+\ts_cbranch_vccnz 2                                         // 000000001008: BF870002 <kernel+0x14>
+\ts_nop 11                                                  // 00000000100C: BF80000B
+\tv_mov_b32_e32 v4, 0                                       // 000000001010: 7E080280
+\tv_max3_f32 v2, v30, v5, v6                                // 000000001014: D1D30002
+\ts_endpgm                                                  // 00000000101C: BF810000
+"""
+
+
+def test_the_check_takes_every_path():
+    (body,) = isa.parse(PLANTED).values()
+    (found,) = isa.mfma_results_touched_early(body)
+    assert found[1].op == "v_max3_f32" and found[2] == 1
+    (body,) = isa.parse(PLANTED.replace("BF870002", "BF87FFFD")).values()      # the branch goes back instead
+    assert [x[1].op for x in isa.mfma_results_touched_early(body)] == []
