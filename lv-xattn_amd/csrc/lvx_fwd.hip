@@ -721,10 +721,12 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     float m_i = -INFINITY, l_i = 0.f;
     const float cc = p.scale_log2e;
 
-    // Q was requested first: it is here when at most the pieces' loads are outstanding
-    if (n > 1) wait_vmcnt<4 * NLD>();
-    else if (n == 1) wait_vmcnt<2 * NLD>();
-    else wait_vmcnt<0>();
+    // Q was requested first: it is here when at most two pieces' loads are outstanding (with fewer of them, when
+    // nothing is).  The compiler takes q for loaded from its request on, so nothing must make it touch those
+    // registers before this wait, which is one statement that every path comes by; the tests follow
+    // the paths of the built code from the request to here.
+    asm volatile("s_cmp_gt_i32 %0, 1\n\ts_cbranch_scc1 LVX_FEW_TWO_%=\n\ts_waitcnt vmcnt(0)\nLVX_FEW_TWO_%=:\n\ts_waitcnt vmcnt(%1)"
+                 ::"s"(uniform32(n)), "n"(4 * NLD) : "memory", "scc");
 #pragma unroll
     for (int kk = 0; kk < NKK; ++kk) asm volatile("" : "+v"(q[kk]));
 

@@ -109,3 +109,32 @@ def mfma_results_touched_early(body):
             step = int(x.args[0], 0) + 1 if x.op == "s_nop" else 1
             todo += [(n, waited + step) for n in successors(j)]
     return found
+
+
+def loads_touched_early(body):
+    """[(load, instruction)]: instructions that touch the destination of a load to registers on a path that has
+    not come by any wait for loads yet: what a compiler would do with registers that inline assembly
+    requested, if it copied or spilled them."""
+    index = {ins.addr: i for i, ins in enumerate(body)}
+    successors = after(body, index)
+    found = []
+    for i, ins in enumerate(body):
+        to_lds = "_lds_" in ins.op or ins.args[-1].split(" ")[-1] == "lds"
+        if not ins.op.startswith(("global_load", "buffer_load", "scratch_load", "flat_load")) or to_lds:
+            continue
+        result = regs(ins.args[0])
+        seen = set()
+        todo = list(successors(i))
+        while todo:
+            j = todo.pop()
+            if j in seen:
+                continue
+            seen.add(j)
+            x = body[j]
+            if x.op == "s_waitcnt" and "vmcnt" in " ".join(x.args):
+                continue
+            if touched(x) & result:
+                found.append((ins, x))
+                continue
+            todo += successors(j)
+    return found

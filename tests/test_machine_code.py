@@ -22,6 +22,17 @@ def test_mfma_results_have_their_wait_states(kernels):
     assert not early, {name: found[:2] for name, found in early.items()}
 
 
+@needs_objdump
+def test_registers_that_assembly_loads_are_left_alone_until_the_wait(kernels):
+    """fwd_few_kernel requests Q by inline assembly long before it waits for it: no path of the built code may copy,
+    spill or use those registers in between."""
+    few = {n: b for n, b in kernels.items() if "fwd_few_kernel" in n}
+    assert len(few) == 16
+    for name, body in few.items():
+        assert sum(i.op == "global_load_dwordx4" for i in body) >= 1
+        assert not isa.loads_touched_early(body), name
+
+
 PLANTED = """
 0000000000001000 <kernel>:
 \tv_mfma_f32_32x32x16_bf16 v[4:19], v[20:23], v[82:85], 0    // 000000001000: D3B58004 02
@@ -39,3 +50,11 @@ def test_the_check_takes_every_path():
     assert found[1].op == "v_max3_f32" and found[2] == 1
     (body,) = isa.parse(PLANTED.replace("BF870002", "BF87FFFD")).values()      # the branch goes back instead
     assert [x[1].op for x in isa.mfma_results_touched_early(body)] == []
+
+
+def test_a_copy_of_a_register_in_flight_is_found():
+    text = PLANTED.replace("v_mfma_f32_32x32x16_bf16 v[4:19], v[20:23], v[82:85], 0    ", "global_load_dwordx4 v[4:7], v[20:21], off    ")
+    (body,) = isa.parse(text).values()
+    assert sorted(x[1].op for x in isa.loads_touched_early(body)) == ["v_max3_f32", "v_mov_b32"]
+    (body,) = isa.parse(text.replace("s_nop 11 ", "s_waitcnt vmcnt(0) ").replace("v5, v6", "v8, v9")).values()
+    assert not isa.loads_touched_early(body)
