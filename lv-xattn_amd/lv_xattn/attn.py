@@ -98,11 +98,17 @@ def _dense_bias(bias_func, local_bias_args, remote_bias_args, B, Hq, Lq, Lkv, de
         padded = torch.zeros(*bias.shape[:3], Lkv + pad, dtype=torch.float32, device=dev)
         padded[..., :Lkv] = bias
         view = padded[..., :Lkv]
-        if getattr(bias, "lvx_reused", False):      # see _bias_and_hull: the copy is kept with it
+        if getattr(bias, "lvx_reused", False) and not _capturing():      # see _bias_and_hull: the copy is kept with it
             view.lvx_reused = True
             bias.lvx_padded = view
         bias = view
     return bias
+
+
+def _capturing() -> bool:
+    """Whether the current stream's work is being recorded into a graph: nothing may come back to the host then,
+    and what is recorded has not been computed when the call returns."""
+    return torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()
 
 
 def _bias_and_hull(bias: torch.Tensor, q, k):
@@ -112,15 +118,15 @@ def _bias_and_hull(bias: torch.Tensor, q, k):
     the mask it converts once per model call) is also tested once for being nothing but that
     interval mask - 0 wherever it is not -inf - and is then dropped: the interval-mask kernels give
     the same result without reading it.  The test waits for the GPU, which is why it is only made
-    for a bias that comes back; hull and verdict stay with the tensor (and so does the padded copy
-    _dense_bias may have to make of it), so a tensor marked `lvx_reused` must not be written to
-    afterwards."""
+    for a bias that comes back, and never under graph capture; hull and verdict stay with the tensor (and so
+    does the padded copy _dense_bias may have to make of it), so a tensor marked `lvx_reused` must not
+    be written to afterwards."""
     key = (tuple(q.shape[:3]), k.shape[2])
     kept = getattr(bias, "lvx_hull", None)
     if kept is not None and kept[0] == key:
         return (None if kept[2] else bias), kept[1]
     hull = ops.bias_hull(q, k, bias)
-    if not getattr(bias, "lvx_reused", False):
+    if not getattr(bias, "lvx_reused", False) or _capturing():
         return bias, hull
     exact = ops.bias_is_interval(q, k, bias, hull)
     bias.lvx_hull = (key, hull, exact)

@@ -35,12 +35,22 @@ from torch.autograd.forward_ad import unpack_dual
 
 from . import ops
 from ._lib import LvxError
-from .attn import _attn_forward
+from .attn import _attn_forward, _capturing
 from .autograd import create_attention_class, create_attention_class_save_qkv, create_q_projection_class
 
 NAME = "lv_xattn"
 _attention = None
 _bias_cache: list = []      # [key, fp32 bias, the mask it was made from] of the last conversion
+
+
+def _sees_a_key(visible: torch.Tensor) -> torch.Tensor:
+    """visible.any(-1, keepdim=True), 1024 keys at a time: for a long row torch shares a reduction among blocks and
+    clears their counters with a memset, which gives wrong results when a captured graph is replayed."""
+    n = visible.shape[-1] // 1024
+    if n <= 1:
+        return visible.any(-1, keepdim=True)
+    whole = visible[..., :n * 1024].unflatten(-1, (n, 1024)).any(-1).any(-1, keepdim=True)
+    return whole | visible[..., n * 1024:].any(-1, keepdim=True)
 
 
 def _mask_bias(mask: torch.Tensor) -> torch.Tensor:
@@ -68,11 +78,11 @@ def _mask_bias(mask: torch.Tensor) -> torch.Tensor:
         return _bias_cache[1]
     m = mask.float()
     masked = m <= -30000.0
-    sees_a_key = (~masked).any(-1, keepdim=True)
-    bias = torch.where(masked & sees_a_key, float("-inf"), m.clamp_min(-30000.0))
+    bias = torch.where(masked & _sees_a_key(~masked), float("-inf"), m.clamp_min(-30000.0))
     # every cross-attention layer of a model gets the same mask, in forward and again in backward:
-    # the last conversion is kept (with the mask itself, so that its address cannot be reused)
-    if version is not None:
+    # the last conversion is kept (with the mask itself, so that its address cannot be reused).  Not one
+    # that a graph capture records: its values do not exist until the graph is replayed
+    if version is not None and not _capturing():
         bias.lvx_reused = True      # attn._bias_and_hull: worth testing once whether it is an interval mask
         _bias_cache[:] = [key, bias, mask]
     return bias

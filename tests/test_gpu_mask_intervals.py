@@ -80,3 +80,39 @@ def test_a_mask_first_seen_under_capture():
             graph.replay()
             torch.cuda.synchronize()
             torch.testing.assert_close(out, _attend(q, k, v, mask), rtol=2.0 ** -7, atol=2.0 ** -7)
+
+
+def _capture(stream, q, k, v, mask):
+    from lv_xattn import hf_mllama
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)[0]
+    return graph, out
+
+
+def _replays_read_the_mask(graph, out, q, k, v, mask):
+    """Every replay sees the mask as it is then, with eager work, other masks and synchronizations in between."""
+    for visible in (mask.shape[-1], 100, 7, mask.shape[-1] - 1):
+        new = torch.zeros_like(mask)
+        new[..., visible:] = torch.finfo(mask.dtype).min
+        want = _attend(q, k, v, new)
+        mask.copy_(new)
+        graph.replay()
+        torch.cuda.synchronize()
+        torch.testing.assert_close(out, want, rtol=2.0 ** -7, atol=2.0 ** -7)
+
+
+# 20000 keys: long enough for torch to share a reduction over a row among several blocks
+@pytest.mark.parametrize("keys", [333, 20000])
+def test_an_ordinary_mask_under_capture_after_an_eager_warm_up(keys):
+    """As generation with a static mask buffer has it: eager calls on the default stream, then a capture on
+    torch.cuda.graph's own, nothing cleared in between."""
+    torch.manual_seed(2)
+    with torch.no_grad():
+        q, k, v = (torch.randn(1, h, n, 64, device=DEV, dtype=torch.bfloat16) for h, n in ((8, 1), (2, keys), (2, keys)))
+        mask = torch.zeros(1, 1, 1, keys, device=DEV, dtype=torch.bfloat16)
+        mask[..., keys // 2:] = torch.finfo(torch.bfloat16).min
+        _attend(q, k, v, mask)
+        torch.cuda.synchronize()
+        graph, out = _capture(None, q, k, v, mask)
+        _replays_read_the_mask(graph, out, q, k, v, mask)

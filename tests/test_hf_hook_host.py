@@ -4,7 +4,7 @@ import pytest
 import torch
 from torch.autograd import forward_ad
 
-from lv_xattn import autograd, hf_mllama
+from lv_xattn import attn, autograd, hf_mllama, ops
 
 
 class _Layer(torch.nn.Module):
@@ -43,3 +43,88 @@ def test_a_forward_mode_tangent_is_refused(no_kernels, which, grad):
         qkv[which] = forward_ad.make_dual(qkv[which], torch.ones_like(qkv[which]))
         with pytest.raises(NotImplementedError, match="jvp"):
             hf_mllama.lv_xattn_attention_forward(_Layer(), *qkv, None)
+
+
+class _Gpu:
+    """Stands in for the current stream: its number, and whether it is capturing."""
+
+    def __init__(self, monkeypatch):
+        self.stream, self.capturing, self.waits = 1, False, []
+        monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: self.capturing)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: self)
+
+        def intervals(mask):
+            assert not self.capturing, "a host read under capture"
+            self.waits.append("mask_intervals")
+            visible = mask[:, 0] > -30000
+            first = visible.int().argmax(-1)
+            return ops.Mask(None, first.int(), (first + visible.sum(-1)).int())
+
+        def is_interval(*a):
+            assert not self.capturing, "a host read under capture"
+            self.waits.append("bias_is_interval")
+            return True
+
+        monkeypatch.setattr(ops, "mask_intervals", intervals)
+        monkeypatch.setattr(ops, "bias_is_interval", is_interval)
+        monkeypatch.setattr(ops, "bias_hull", lambda *a: ops.Mask())
+
+    @property
+    def cuda_stream(self):
+        return self.stream
+
+
+@pytest.fixture
+def gpu(monkeypatch):
+    hf_mllama.clear_mask_cache()
+    yield _Gpu(monkeypatch)
+    hf_mllama.clear_mask_cache()
+
+
+@pytest.fixture
+def seen(monkeypatch):
+    """What the kernels are given of a call's mask: the intervals, or the dense bias."""
+    calls = []
+
+    def forward(q, k, v, causal, scale, mode, bias_func=None, local=(), remote=(), *args, mask=None, **kw):
+        bias = attn._dense_bias(bias_func, local, remote, q.shape[0], q.shape[1], q.shape[2], k.shape[2], q.device)
+        if mask is None and bias is not None:
+            bias, mask = attn._bias_and_hull(bias, q, k)
+        calls.append((mask, bias))
+        return q, k, v, torch.zeros_like(q), torch.zeros(q.shape[0] * q.shape[1], q.shape[2])
+
+    for module in (hf_mllama, autograd):
+        monkeypatch.setattr(module, "_attn_forward", forward)
+    monkeypatch.setattr(hf_mllama, "_require_supported", lambda *a: None)
+    return calls
+
+
+def _mask(visible):
+    mask = torch.zeros(1, 1, 5, 33, dtype=torch.bfloat16)
+    mask[..., visible:] = torch.finfo(torch.bfloat16).min
+    return mask
+
+
+def test_a_captured_call_reads_nothing_back(gpu, seen):
+    """A warm-up on one stream and a capture on another, as torch.cuda.graph has it: the captured calls ask
+    nothing of the host, and nothing a capture recorded (but did not compute) is kept for a later call."""
+    q, k, v = _qkv()
+    mask = _mask(20)
+    with torch.no_grad():
+        hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)
+        gpu.stream, gpu.capturing = 2, True
+        for _ in range(2):
+            hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)
+        gpu.capturing = False
+        recorded = [bias for _, bias in seen[1:]]
+        assert all(b is not None for b in recorded)
+        assert all(b is not hf_mllama._mask_bias(mask) and not hasattr(b, "lvx_hull") for b in recorded)
+
+
+@pytest.mark.parametrize("keys", [1, 1023, 1024, 2047, 2048, 2049, 5000])
+def test_a_row_that_sees_one_key_anywhere(keys):
+    visible = torch.zeros(3, 1, keys, keys, dtype=torch.bool) if keys < 10 else torch.zeros(1, 1, 4, keys, dtype=torch.bool)
+    for row, key in enumerate((0, keys // 2, keys - 1)[:visible.shape[2]]):
+        visible[0, 0, row, key] = True
+    assert torch.equal(hf_mllama._sees_a_key(visible), visible.any(-1, keepdim=True))
