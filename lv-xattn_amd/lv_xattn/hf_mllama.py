@@ -74,7 +74,8 @@ def _mask_bias(mask: torch.Tensor) -> torch.Tensor:
     # apart from an edited copy at the same address, so it is converted every time and not kept
     version = None if mask.is_inference() else mask._version
     key = (mask.data_ptr(), version, tuple(mask.shape), tuple(mask.stride()), mask.dtype, mask.device)
-    if version is not None and _bias_cache and _bias_cache[0] == key:
+    keep = version is not None and not _capturing()     # a capture records the conversion, and reads nothing that is kept
+    if keep and _bias_cache and _bias_cache[0] == key:
         return _bias_cache[1]
     m = mask.float()
     masked = m <= -30000.0
@@ -82,7 +83,7 @@ def _mask_bias(mask: torch.Tensor) -> torch.Tensor:
     # every cross-attention layer of a model gets the same mask, in forward and again in backward:
     # the last conversion is kept (with the mask itself, so that its address cannot be reused).  Not one
     # that a graph capture records: its values do not exist until the graph is replayed
-    if version is not None and not _capturing():
+    if keep:
         bias.lvx_reused = True      # attn._bias_and_hull: worth testing once whether it is an interval mask
         _bias_cache[:] = [key, bias, mask]
     return bias
@@ -95,10 +96,11 @@ def _mask_intervals(mask: torch.Tensor, query: torch.Tensor, lkv: int):
     """The interval mask that says all that transformers' additive `mask` says (ops.mask_intervals), or
     None: the usual case, a row looks at the tiles of the images before it.  Every layer of a model
     gets the same mask, so the last answer is kept, with the mask, as `_mask_bias` keeps its own, for
-    calls on the stream it was made on.  A mask of another form or place than the query's rows and keys, and
-    one first seen while a graph is captured (the answer has to come back to the host), are `_mask_bias`'s."""
+    calls on the stream it was made on.  A mask of another form or place than the query's rows and keys is
+    `_mask_bias`'s, and so is any mask while a graph is captured: a replay has to read the mask as it is
+    then, not as it was when the answer was kept, and the graph does not own what is kept here."""
     global _interval_cache
-    if tuple(mask.shape) != (query.shape[0], 1, query.shape[2], lkv) or mask.device != query.device:
+    if tuple(mask.shape) != (query.shape[0], 1, query.shape[2], lkv) or mask.device != query.device or _capturing():
         return None
     version = None if mask.is_inference() else mask._version
     key = (mask.data_ptr(), version, tuple(mask.shape), tuple(mask.stride()), mask.dtype, mask.device,
@@ -106,8 +108,6 @@ def _mask_intervals(mask: torch.Tensor, query: torch.Tensor, lkv: int):
     kept = _interval_cache          # read once: another thread may put its own in place
     if version is not None and kept and kept[0] == key:
         return kept[1]
-    if torch.cuda.is_current_stream_capturing():
-        return None
     intervals = ops.mask_intervals(mask)
     if version is not None:
         _interval_cache = (key, intervals, mask)

@@ -116,3 +116,23 @@ def test_an_ordinary_mask_under_capture_after_an_eager_warm_up(keys):
         torch.cuda.synchronize()
         graph, out = _capture(None, q, k, v, mask)
         _replays_read_the_mask(graph, out, q, k, v, mask)
+
+
+@pytest.mark.parametrize("plain", [True, False])
+def test_a_capture_on_the_stream_of_the_warm_up(plain):
+    """What the warm-up kept for this very stream - the intervals, or the converted mask of one that is more than
+    intervals - is not what a replay may use once the mask was written to."""
+    torch.manual_seed(3)
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        q, k, v = (torch.randn(1, h, n, 64, device=DEV, dtype=torch.bfloat16) for h, n in ((8, 3), (2, 400), (2, 400)))
+        mask = torch.zeros(1, 1, 3, 400, device=DEV, dtype=torch.bfloat16)
+        mask[..., 50:] = torch.finfo(torch.bfloat16).min
+        if not plain:
+            mask[..., 10] = -1.0
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            _attend(q, k, v, mask)
+        torch.cuda.synchronize()
+        graph, out = _capture(side, q, k, v, mask)
+        _replays_read_the_mask(graph, out, q, k, v, mask)

@@ -128,3 +128,17 @@ def test_a_row_that_sees_one_key_anywhere(keys):
     for row, key in enumerate((0, keys // 2, keys - 1)[:visible.shape[2]]):
         visible[0, 0, row, key] = True
     assert torch.equal(hf_mllama._sees_a_key(visible), visible.any(-1, keepdim=True))
+
+
+def test_a_capture_uses_no_answer_that_was_kept(gpu, seen):
+    """On the very stream of the warm-up: the captured calls convert the mask in the graph, whether the intervals or
+    the converted mask had been kept, so that a replay reads the mask as it is then."""
+    q, k, v = _qkv()
+    with torch.no_grad():
+        for mask in (_mask(20), _mask(20).masked_fill(torch.arange(33) == 3, -1.0)):     # an interval mask, and another
+            hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)
+            kept = hf_mllama._mask_bias(mask)
+            gpu.capturing = True
+            hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)
+            gpu.capturing = False
+            assert seen[-1][1] is not None and seen[-1][1] is not kept
