@@ -77,7 +77,7 @@ def generate() -> None:
 
 
 def host_command():
-    """g++ command line of the host extension module; it finds liblvx.so beside itself."""
+    """g++ command line of the host extension module (the library's functions reach it by address)."""
     import sysconfig
     import torch
     from torch.utils.cpp_extension import include_paths
@@ -86,8 +86,7 @@ def host_command():
     inc = [*include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
     return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-isystem{i}" for i in inc], HOST_SRC,
-            "-o", HOST_LIB, f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
-            f"-L{OUT_DIR}", "-l:liblvx.so", "-Wl,-rpath,$ORIGIN"]
+            "-o", HOST_LIB, f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
 
 
 def build(force: bool = True, verbose: bool = False, extra_flags=()) -> str:

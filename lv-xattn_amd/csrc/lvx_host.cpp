@@ -3,6 +3,9 @@
 // the current stream, output and workspace tensors).  A decoded token's two launches take 12 us on the
 // GPU; issuing them through ctypes took 32 us of host time.
 //
+// The library's functions are those of the liblvx.so that the package has loaded, handed over by address
+// (bind): this module is linked to none.
+//
 // An operator answers False, and queues nothing, when a call is not one it can pass on as it is (a wrong
 // type, shape or device among the arguments); the caller then goes through its own checks, which word
 // the error.
@@ -11,7 +14,9 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
+#include <map>
 #include <optional>
+#include <string>
 
 #include "../../include/lvx.h"
 
@@ -19,6 +24,23 @@ namespace {
 
 using at::Tensor;
 using OptTensor = std::optional<Tensor>;
+
+struct Library {
+    decltype(&lvx_fwd_workspace_bytes) fwd_workspace_bytes;
+    decltype(&lvx_fwd) fwd;
+    decltype(&lvx_fwd_acc) fwd_acc;
+    decltype(&lvx_bwd_preprocess) bwd_preprocess;
+    decltype(&lvx_bwd) bwd;
+} lib;
+
+void bind(const std::map<std::string, uintptr_t>& addresses) {
+    auto set = [&](auto& f, const char* name) { f = reinterpret_cast<std::remove_reference_t<decltype(f)>>(addresses.at(name)); };
+    set(lib.fwd_workspace_bytes, "lvx_fwd_workspace_bytes");
+    set(lib.fwd, "lvx_fwd");
+    set(lib.fwd_acc, "lvx_fwd_acc");
+    set(lib.bwd_preprocess, "lvx_bwd_preprocess");
+    set(lib.bwd, "lvx_bwd");
+}
 
 int dtype_code(const Tensor& t) {
     return t.scalar_type() == at::kBFloat16 ? LVX_BF16 : t.scalar_type() == at::kHalf ? LVX_F16 : 0;
@@ -84,7 +106,7 @@ py::tuple forward_buffers(const Tensor& q, int64_t rows, int64_t kv_splits, bool
     if (kv_splits <= 1) return py::make_tuple(std::move(o), std::move(lse), py::none());
     lvx_attn_shape s{};
     s.B = (int32_t)B; s.Hq = (int32_t)H; s.D = (int32_t)D;
-    Tensor ws = at::empty({(int64_t)lvx_fwd_workspace_bytes(&s, (int32_t)rows, (int32_t)kv_splits)}, q.options().dtype(at::kByte));
+    Tensor ws = at::empty({(int64_t)lib.fwd_workspace_bytes(&s, (int32_t)rows, (int32_t)kv_splits)}, q.options().dtype(at::kByte));
     return py::make_tuple(std::move(o), std::move(lse), std::move(ws));
 }
 
@@ -98,13 +120,13 @@ bool fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, con
     void* const wp = ws ? ws->data_ptr() : nullptr;
     const size_t wb = ws ? ws->nbytes() : 0;
     if (!acc_o) {
-        check(lvx_fwd(&s, &tq, &tk, &tv, &to, lse.data_ptr<float>(), (int32_t)row_begin, (int32_t)row_count, (int32_t)kv_splits, wp, wb,
+        check(lib.fwd(&s, &tq, &tk, &tv, &to, lse.data_ptr<float>(), (int32_t)row_begin, (int32_t)row_count, (int32_t)kv_splits, wp, wb,
                       current_stream()), "lvx_fwd");
         return true;
     }
     if (!plain4(*acc_o, q, q.scalar_type()) || acc_o->sizes() != q.sizes() || !acc_l || !rows_ok(*acc_l, q)) return false;
     const lvx_tensor ta = t4(*acc_o);
-    check(lvx_fwd_acc(&s, &tq, &tk, &tv, &ta, acc_l->data_ptr<float>(), &to, lse.data_ptr<float>(), (int32_t)row_begin,
+    check(lib.fwd_acc(&s, &tq, &tk, &tv, &ta, acc_l->data_ptr<float>(), &to, lse.data_ptr<float>(), (int32_t)row_begin,
                       (int32_t)row_count, (int32_t)kv_splits, wp, wb, current_stream()), "lvx_fwd_acc");
     return true;
 }
@@ -113,7 +135,7 @@ bool bwd_preprocess(const Tensor& o, const Tensor& dout, const Tensor& delta, in
     lvx_attn_shape s;
     if (!fill_shape(s, o, dout, dout, 1.0, {}, {}, {}) || o.sizes() != dout.sizes() || !rows_ok(delta, o)) return false;
     const lvx_tensor to = t4(o), td = t4(dout);
-    check(lvx_bwd_preprocess(&s, &to, &td, delta.data_ptr<float>(), (int32_t)row_begin, (int32_t)row_count, current_stream()),
+    check(lib.bwd_preprocess(&s, &to, &td, delta.data_ptr<float>(), (int32_t)row_begin, (int32_t)row_count, current_stream()),
           "lvx_bwd_preprocess");
     return true;
 }
@@ -129,7 +151,7 @@ bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, 
         !plain4(dv, q, kv_type) || dv.sizes() != k.sizes())
         return false;
     const lvx_tensor tq = t4(q), tk = t4(k), tv = t4(v), td = t4(dout), tdq = t4(dq), tdk = t4(dk), tdv = t4(dv);
-    check(lvx_bwd(&s, &tq, &tk, &tv, &td, lse.data_ptr<float>(), delta.data_ptr<float>(), &tdq, &tdk, &tdv, accumulate_dkv ? 1 : 0,
+    check(lib.bwd(&s, &tq, &tk, &tv, &td, lse.data_ptr<float>(), delta.data_ptr<float>(), &tdq, &tdk, &tdv, accumulate_dkv ? 1 : 0,
                   (int32_t)row_begin, (int32_t)row_count, ws.data_ptr(), ws.nbytes(), current_stream()), "lvx_bwd");
     return true;
 }
@@ -137,6 +159,7 @@ bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, 
 }  // namespace
 
 PYBIND11_MODULE(_lvx_host, m) {
+    m.def("bind", &bind);
     m.def("usable", &usable);
     m.def("forward_buffers", &forward_buffers);
     m.def("fwd", &fwd);

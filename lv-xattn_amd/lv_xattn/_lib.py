@@ -90,19 +90,21 @@ def load() -> C.CDLL:
     return lib
 
 
-_host = None
+_host = _host_lib = None       # the module, and the library whose functions it calls
 
 
 def host():
-    """The native side of the operators (_lvx_host.so, built with the library).  Raises if it is absent."""
-    global _host
-    if _host is None:
-        load()
+    """The native side of the operators (_lvx_host.so, built with the library), calling the functions of the
+    library that load() gives.  Raises if it is absent."""
+    global _host, _host_lib
+    lib = _lib or load()
+    if _host_lib is not lib:
         try:
             from . import _lvx_host
         except ImportError as e:
             raise LvxError("_lvx_host.so is missing or does not load: run `python lv-xattn_amd/build.py`") from e
-        _host = _lvx_host
+        _lvx_host.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SYMBOLS})
+        _host, _host_lib = _lvx_host, lib
     return _host
 
 
