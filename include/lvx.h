@@ -35,7 +35,8 @@
 extern "C" {
 #endif
 
-#define LVX_VERSION 103
+/* 104: lvx_fwd_auto_splits, lvx_mask_intervals, up to 64 kv_splits (were 16) */
+#define LVX_VERSION 104
 
 #define LVX_OK 0
 #define LVX_ERR_NULL (-1)        /* a required pointer is NULL */

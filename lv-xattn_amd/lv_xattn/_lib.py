@@ -14,6 +14,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("LVX_LIB") or os.path.join(_HERE, "liblvx.so")
 
+VERSION = 104           # of the library (include/lvx.h) this package is written against
 LVX_BF16 = 1
 LVX_F16 = 2
 
@@ -73,7 +74,7 @@ _lib: Optional[C.CDLL] = None
 
 
 def load() -> C.CDLL:
-    """dlopen liblvx.so and type every entry point.  Raises if it is absent."""
+    """dlopen liblvx.so and type every entry point.  Raises if it is absent or of another version."""
     global _lib
     if _lib is not None:
         return _lib
@@ -82,6 +83,8 @@ def load() -> C.CDLL:
             f"{LIB_PATH} is missing: the HIP kernels are not built. "
             "Run `python lv-xattn_amd/build.py` (needs hipcc); there is no CPU fallback.")
     lib = C.CDLL(LIB_PATH)
+    if lib.lvx_version() != VERSION:
+        raise LvxError(f"{LIB_PATH} is version {lib.lvx_version()} of the library, this package needs {VERSION}")
     for name, (res, args) in SYMBOLS.items():
         fn = getattr(lib, name)          # AttributeError if the symbol is not exported
         fn.restype = res

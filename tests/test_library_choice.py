@@ -1,8 +1,11 @@
 """LVX_LIB names the library every operator runs, the native ones included."""
 import os
+import re
 import shutil
 import subprocess
 import sys
+
+import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -26,3 +29,19 @@ def test_one_library_is_mapped_and_it_is_the_named_one(tmp_path):
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
     assert r.stdout.strip().splitlines()[-1] == str([named])
+
+
+def test_a_library_of_another_version_is_refused(monkeypatch, tmp_path):
+    """An older build lacks functions this package calls; its version says so."""
+    from lv_xattn import _lib
+    header = open(os.path.join(ROOT, "include", "lvx.h")).read()
+    assert _lib.VERSION == int(re.search(r"^#define\s+LVX_VERSION\s+(\d+)", header, re.M).group(1))
+    gcc = shutil.which("gcc")
+    if gcc is None:
+        pytest.skip("no gcc")
+    (tmp_path / "old.c").write_text("int lvx_version(void) { return 103; }")
+    subprocess.run([gcc, "-shared", "-fPIC", "-o", str(tmp_path / "old.so"), str(tmp_path / "old.c")], check=True)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "old.so"))
+    with pytest.raises(_lib.LvxError, match="version 103"):
+        _lib.load()
