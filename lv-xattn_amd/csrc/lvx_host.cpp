@@ -82,8 +82,15 @@ bool fill_shape(lvx_attn_shape& s, const Tensor& q, const Tensor& k, const Tenso
 
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
-// A code of the library as the package's own exception.
-void check(int rc, const char* what) {
+// Calls the library without the interpreter's lock - a launch may block on a full queue, and other Python threads go
+// on meanwhile, as they do through ctypes - and gives its code as the package's own exception.
+template <typename F>
+void call(const char* what, F f) {
+    int rc;
+    {
+        py::gil_scoped_release unlocked;
+        rc = f();
+    }
     if (rc) py::module_::import("lv_xattn._lib").attr("check")(rc, what);
 }
 
@@ -119,15 +126,20 @@ bool fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, con
     const lvx_tensor tq = t4(q), tk = t4(k), tv = t4(v), to = t4(o);
     void* const wp = ws ? ws->data_ptr() : nullptr;
     const size_t wb = ws ? ws->nbytes() : 0;
+    float* const lp = lse.data_ptr<float>();
+    void* const st = current_stream();
     if (!acc_o) {
-        check(lib.fwd(&s, &tq, &tk, &tv, &to, lse.data_ptr<float>(), (int32_t)row_begin, (int32_t)row_count, (int32_t)kv_splits, wp, wb,
-                      current_stream()), "lvx_fwd");
+        call("lvx_fwd", [&] {
+            return lib.fwd(&s, &tq, &tk, &tv, &to, lp, (int32_t)row_begin, (int32_t)row_count, (int32_t)kv_splits, wp, wb, st);
+        });
         return true;
     }
     if (!plain4(*acc_o, q, q.scalar_type()) || acc_o->sizes() != q.sizes() || !acc_l || !rows_ok(*acc_l, q)) return false;
     const lvx_tensor ta = t4(*acc_o);
-    check(lib.fwd_acc(&s, &tq, &tk, &tv, &ta, acc_l->data_ptr<float>(), &to, lse.data_ptr<float>(), (int32_t)row_begin,
-                      (int32_t)row_count, (int32_t)kv_splits, wp, wb, current_stream()), "lvx_fwd_acc");
+    const float* const la = acc_l->data_ptr<float>();
+    call("lvx_fwd_acc", [&] {
+        return lib.fwd_acc(&s, &tq, &tk, &tv, &ta, la, &to, lp, (int32_t)row_begin, (int32_t)row_count, (int32_t)kv_splits, wp, wb, st);
+    });
     return true;
 }
 
@@ -135,8 +147,9 @@ bool bwd_preprocess(const Tensor& o, const Tensor& dout, const Tensor& delta, in
     lvx_attn_shape s;
     if (!fill_shape(s, o, dout, dout, 1.0, {}, {}, {}) || o.sizes() != dout.sizes() || !rows_ok(delta, o)) return false;
     const lvx_tensor to = t4(o), td = t4(dout);
-    check(lib.bwd_preprocess(&s, &to, &td, delta.data_ptr<float>(), (int32_t)row_begin, (int32_t)row_count, current_stream()),
-          "lvx_bwd_preprocess");
+    float* const dp = delta.data_ptr<float>();
+    void* const st = current_stream();
+    call("lvx_bwd_preprocess", [&] { return lib.bwd_preprocess(&s, &to, &td, dp, (int32_t)row_begin, (int32_t)row_count, st); });
     return true;
 }
 
@@ -151,8 +164,13 @@ bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, 
         !plain4(dv, q, kv_type) || dv.sizes() != k.sizes())
         return false;
     const lvx_tensor tq = t4(q), tk = t4(k), tv = t4(v), td = t4(dout), tdq = t4(dq), tdk = t4(dk), tdv = t4(dv);
-    check(lib.bwd(&s, &tq, &tk, &tv, &td, lse.data_ptr<float>(), delta.data_ptr<float>(), &tdq, &tdk, &tdv, accumulate_dkv ? 1 : 0,
-                  (int32_t)row_begin, (int32_t)row_count, ws.data_ptr(), ws.nbytes(), current_stream()), "lvx_bwd");
+    const float *const lp = lse.data_ptr<float>(), *const dp = delta.data_ptr<float>();
+    void *const wp = ws.data_ptr(), *const st = current_stream();
+    const size_t wb = ws.nbytes();
+    call("lvx_bwd", [&] {
+        return lib.bwd(&s, &tq, &tk, &tv, &td, lp, dp, &tdq, &tdk, &tdv, accumulate_dkv ? 1 : 0, (int32_t)row_begin, (int32_t)row_count,
+                       wp, wb, st);
+    });
     return true;
 }
 
