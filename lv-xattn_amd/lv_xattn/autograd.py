@@ -43,9 +43,9 @@ def _gradient_follows():
 
 
 def create_attention_class_save_qkv(attention_mode: str = "lv_xattn", no_overlap: bool = False,
-                                    rounds: Optional[int] = None, batched: bool = False, token_major: bool = False):
+                                    rounds: Optional[int] = None, batched: bool = False):
     """apply(q, k, v, causal, sm_scale, bias_func=None, local_bias_args=[],
-    remote_bias_args=[], mask=None) -> o [B, Hq, Lq, D], a view of [B, Lq, Hq, D] memory with `token_major`"""
+    remote_bias_args=[], mask=None) -> o"""
     if attention_mode != "lv_xattn":
         raise ValueError("only attention_mode='lv_xattn' exists on this path")
 
@@ -55,7 +55,7 @@ def create_attention_class_save_qkv(attention_mode: str = "lv_xattn", no_overlap
                     remote_bias_args=[], mask=None):
             q, k, v, o, L = _attn_forward(q, k, v, causal, sm_scale, None, bias_func, local_bias_args,
                                           remote_bias_args, no_overlap, rounds=rounds, mask=mask,
-                                          batched=batched, _token_major=token_major)
+                                          batched=batched)
             # like the reference (test_llama3.py:144-149): the bias arguments are kept and the
             # bias is rebuilt in backward
             ctx.save_for_backward(q, k, v, o, L, *local_bias_args, *remote_bias_args)

@@ -148,12 +148,12 @@ def lv_xattn_attention_forward(module, query, key, value, attention_mask: Option
         out = _attn_forward(query, key, value, False, scaling, None, rounds=1, batched=True, mask=intervals, _token_major=True)[3]
         return out.transpose(1, 2).contiguous(), None
     if _attention is None:
-        _attention = create_attention_class_save_qkv("lv_xattn", rounds=1, batched=True, token_major=True).apply
+        _attention = create_attention_class_save_qkv("lv_xattn", rounds=1, batched=True).apply
     if mask is None or intervals is not None:
         out = _attention(query, key, value, False, scaling, None, [], [], intervals)
     else:
         out = _attention(query, key, value, False, scaling, _mask_bias, [mask], [])
-    return out.transpose(1, 2).contiguous(), None
+    return out.transpose(1, 2).contiguous(), None       # a copy: backward keeps `out`, the caller may write to its result
 
 
 def _require_supported(query, key, dropout):

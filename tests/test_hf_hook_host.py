@@ -142,3 +142,14 @@ def test_a_capture_uses_no_answer_that_was_kept(gpu, seen):
             hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)
             gpu.capturing = False
             assert seen[-1][1] is not None and seen[-1][1] is not kept
+
+
+def test_the_result_of_a_recorded_call_may_be_written_to(no_kernels):
+    """A caller may scale or mask the attention's output in place before it is projected: what backward needs is
+    not that memory."""
+    q, k, v = (t.requires_grad_() for t in _qkv())
+    out = hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, None)[0]
+    assert out.is_contiguous() and out.shape == (1, 5, 8, 64)
+    out.mul_(0.5)
+    out.float().sum().backward()
+    assert all(t.grad is not None for t in (q, k, v))
