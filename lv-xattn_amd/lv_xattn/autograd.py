@@ -295,7 +295,7 @@ def create_q_projection_class(w_in_major: bool = True, weight_grads: bool = True
         @staticmethod
         def forward(ctx, x, w_q, n_heads, q_norm_weight, eps=1e-5):
             ctx.n_heads, ctx.eps = n_heads, eps
-            if getattr(_this_run, "gradient_follows", False):
+            if q_norm_weight is not None and getattr(_this_run, "gradient_follows", False):
                 q, q_raw, rstd = ops.q_proj(x, w_q, n_heads, w_in_major, q_norm_weight, eps, for_backward=True)
                 ctx.save_for_backward(x, w_q, q_norm_weight, q_raw, rstd)
                 return q

@@ -153,3 +153,29 @@ def test_the_result_of_a_recorded_call_may_be_written_to(no_kernels):
     out.mul_(0.5)
     out.float().sum().backward()
     assert all(t.grad is not None for t in (q, k, v))
+
+
+def test_a_projection_without_a_norm_inside_run_function(monkeypatch):
+    """run_function may project a part that needs no gradient - here q, from frozen weights on detached states -
+    without a norm, in both of its runs."""
+    calls = []
+
+    def q_proj(x, w, heads, w_in_major=True, norm=None, eps=1e-5, for_backward=False):
+        assert norm is not None or not for_backward        # ops.q_proj refuses that
+        calls.append(for_backward)
+        q = (x @ w).view(x.shape[0], x.shape[1], heads, -1).transpose(1, 2)
+        return (q, q, torch.ones(1)) if for_backward else q
+
+    monkeypatch.setattr(ops, "q_proj", q_proj)
+    monkeypatch.setattr(autograd, "_attn_forward", lambda q, k, v, *a, **kw: (q, k, v, torch.zeros_like(q), torch.zeros(8, 5)))
+    monkeypatch.setattr(autograd, "_attn_backward", lambda do, q, k, v, *a, **kw: (torch.ones_like(q), torch.ones_like(k), torch.ones_like(v)))
+    project_q = autograd.create_q_projection_class().apply
+    w_q, w_kv = torch.randn(16, 8 * 4), torch.randn(16, 8 * 4, requires_grad=True)
+
+    def run_function(x, states):
+        k = (x @ w_kv).view(1, 5, 8, 4).transpose(1, 2)
+        return project_q(x.detach(), w_q, 8, None, 1e-5), k, k
+
+    x = torch.randn(1, 5, 16, requires_grad=True)
+    autograd.create_attention_class("lv_xattn").apply(x, run_function, False).sum().backward()
+    assert x.grad is not None and w_kv.grad is not None and calls == [False, False]
