@@ -35,7 +35,7 @@
 extern "C" {
 #endif
 
-/* 104: lvx_fwd_auto_splits, lvx_mask_intervals, up to 64 kv_splits (were 16) */
+/* 104: lvx_fwd_auto_splits, lvx_mask_intervals, up to 64 kv_splits (were 16), LVX_SPLITS_FP32 */
 #define LVX_VERSION 104
 
 #define LVX_OK 0
@@ -94,7 +94,9 @@ const char* lvx_strerror(int code);
  * kv_splits > 1 cuts the shard into that many key ranges computed by separate
  * work-groups and folded before return; it needs a workspace of
  * lvx_fwd_workspace_bytes(shape, row_count, kv_splits) bytes.
- * (at most 64 of them; lvx_fwd_auto_splits says how many suit a launch).
+ * (at most 64 of them; lvx_fwd_auto_splits says how many suit a launch).  The O of a range waits for the
+ * fold in 16 bits, a rounding that a launch of one range does not have (its error against exact arithmetic
+ * grows by about a fifth), or with kv_splits = n | LVX_SPLITS_FP32 in fp32, in twice the workspace.
  * The kernel has three forms, chosen by what the launch is estimated to take in each: a wavefront
  * owns 32 text rows of a head (any head_dim, the only one with a dense bias); 64 rows and its SIMD
  * to itself (head_dim 128 and 64); or a share of the keys for up to 32 (row, head) pairs of a kv head at
@@ -121,11 +123,14 @@ int lvx_fwd_acc(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tens
                 int32_t row_begin, int32_t row_count, int32_t kv_splits,
                 void* workspace, size_t workspace_bytes, void* stream);
 
+#define LVX_SPLITS_FP32 256
 size_t lvx_fwd_workspace_bytes(const lvx_attn_shape* shape, int32_t row_count, int32_t kv_splits);
 
 /*
  * The number of key splits (1 .. 64) with which lvx_fwd is estimated to be fastest for `row_count`
- * text rows.  Looks at sizes only (and at whether there is a bias); 1 for an invalid shape.
+ * text rows, as lvx_fwd takes it: with LVX_SPLITS_FP32 unless that costs speed in a launch that needs the
+ * splits to fill the chip.  Looks at sizes only (and at whether there is a bias); 1 for an
+ * invalid shape.
  */
 int lvx_fwd_auto_splits(const lvx_attn_shape* shape, int32_t row_count);
 

@@ -131,9 +131,11 @@ const char* lvx_strerror(int code) {
 }
 
 size_t lvx_fwd_workspace_bytes(const lvx_attn_shape* s, int32_t row_count, int32_t kv_splits) {
+    const bool f32 = kv_splits > 0 && (kv_splits & LVX_SPLITS_FP32);
+    if (f32) kv_splits &= ~LVX_SPLITS_FP32;
     if (!s || kv_splits <= 1 || row_count <= 0) return 0;
     const size_t rows = (size_t)s->B * s->Hq * row_count;
-    return (size_t)kv_splits * rows * (s->D * sizeof(uint16_t) + sizeof(float));
+    return (size_t)kv_splits * rows * (s->D * (f32 ? sizeof(float) : sizeof(uint16_t)) + sizeof(float));
 }
 
 // Keys per split: whole tiles (pieces) of the form's kernel.
@@ -150,12 +152,13 @@ static int fwd_split_len(const lvx_attn_shape* s, FwdForm form, int splits) {
 //   wide : 11 us per round of work-groups, and per 64-key tile 1.1 us on an idle chip, 1.5 on a full one
 //          (0.9 and 1.05 with heads of 64).  256 rows x 6404 keys: 138 us whole, 39 in 8 parts
 //   plain: the same with 1.8 us per tile and two work-groups per CU
-// plus, with splits, 4 us for the launch that folds the parts and their bytes at 4 TB/s.
-static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits) {
+// plus, with splits, 4 us for the launch that folds the parts and their bytes at 4 TB/s, what fp32 adds to them at 9.
+static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32) {
     const int G = s->Hq / s->Hkv, hg = gcd(G, 4), rs = 4 / hg, n_cu = cu_count();
     const int64_t split_len = fwd_split_len(s, form, splits);
     const int64_t n = (s->Lkv + split_len - 1) / split_len;
-    double t = n > 1 ? 4.0 + (double)n * s->B * s->Hq * rows * (4 * s->D + 8) / 4e6 : 0.0;
+    const double fold_us = (4 * s->D + 8) / 4e6 + (parts_f32 ? 4 * s->D / 9e6 : 0.0);       // per row, head and part
+    double t = n > 1 ? 4.0 + (double)n * s->B * s->Hq * rows * fold_us : 0.0;
     if (form == FWD_FEW) {
         const int64_t wgs = (int64_t)s->B * s->Hkv * (((int64_t)rows * G + 31) / 32) * n;
         const int64_t slots = s->D == 128 ? n_cu : 2 * n_cu;
@@ -182,14 +185,29 @@ static bool fwd_few_ok(const lvx_attn_shape* s, int rows) {
 // Head dimensions 128 and 64 without a dense bias take the wide form or, where reading K and V is the
 // larger part of the work, the form for few rows; the plain one was slower at every size measured
 // (4096 rows x 6404 keys: 429 us against 354; 300 rows x 2 samples: 92 against 88).
-static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits) {
+static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits, bool parts_f32) {
     if (s->bias) return FWD_PLAIN;
     const FwdForm many = s->D == 128 || s->D == 64 ? FWD_WIDE : FWD_PLAIN;
     if (const char* e = getenv("LVX_FWD_WIDE")) {
         if (atoi(e) == 2 && fwd_few_ok(s, rows)) return FWD_FEW;
         return atoi(e) != 0 ? many : FWD_PLAIN;
     }
-    return fwd_few_ok(s, rows) && fwd_cost(s, rows, FWD_FEW, splits) <= fwd_cost(s, rows, many, splits) ? FWD_FEW : many;
+    return fwd_few_ok(s, rows) && fwd_cost(s, rows, FWD_FEW, splits, parts_f32) <= fwd_cost(s, rows, many, splits, parts_f32) ? FWD_FEW : many;
+}
+
+// Whether the parts of a launch whose splits are chosen here wait for the fold in fp32.  In 16 bits they are a
+// rounding that a launch of one range does not have: relative error against 64 bits 2.83e-3 instead of 2.32e-3
+// (bf16, N(0, 1) inputs), whatever the number of parts.  The form for few rows has too little O for fp32 to show
+// (one row x 6404 keys 10.2 us in 16 bits, 10.3 in fp32).  In the others fp32 costs 2 - 7 % of the launch, and cutting
+// either is what fills the chip - fewer than two work-groups of 32-row waves per CU, ranges of 512 keys and
+// more: 256 rows x 6404 keys 137 us whole, 37.4 in 8 parts, 40.1 with those in fp32 - where they stay in 16
+// bits, or it only evens out the last round of work-groups (2100 rows x 6404 keys 310 us whole, 263 in 2 parts, 270
+// with those in fp32) or cuts a short range shorter: there the result keeps the precision of the whole launch.
+static bool fwd_parts_f32(const lvx_attn_shape* s, int rows, FwdForm form) {
+    if (form == FWD_FEW) return true;
+    const int hg = gcd(s->Hq / s->Hkv, 4), wg_rows = 32 * (4 / hg);
+    const int64_t wgs = (int64_t)s->B * (s->Hq / hg) * (((int64_t)rows + wg_rows - 1) / wg_rows);
+    return wgs >= 2 * cu_count() || s->Lkv < 1024;
 }
 
 int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
@@ -197,10 +215,13 @@ int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
     const FwdForm many = !s->bias && (s->D == 128 || s->D == 64) ? FWD_WIDE : FWD_PLAIN;
     int best = 1;
     double best_cost = 0.0;
-    for (int n = 1; n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
-        double c = fwd_cost(s, row_count, many, n);
-        if (fwd_few_ok(s, row_count)) c = std::min(c, fwd_cost(s, row_count, FWD_FEW, n));
-        if (n == 1 || c < best_cost) { best = n; best_cost = c; }
+    for (const FwdForm form : {many, FWD_FEW}) {
+        if (form == FWD_FEW && !fwd_few_ok(s, row_count)) continue;
+        const bool f32 = fwd_parts_f32(s, row_count, form);
+        for (int n = 1; n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
+            const double c = fwd_cost(s, row_count, form, n, f32);
+            if (best_cost == 0.0 || c < best_cost) { best = n > 1 && f32 ? n | LVX_SPLITS_FP32 : n; best_cost = c; }
+        }
     }
     return best;
 }
@@ -217,6 +238,8 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     LVX_TRY(check_tensor(o));
     if (!lse) return LVX_ERR_NULL;
     LVX_TRY(check_rows(s, row_begin, row_count));
+    const int f32 = kv_splits > 0 ? kv_splits & LVX_SPLITS_FP32 : 0;
+    kv_splits -= f32;
     if (kv_splits < 1 || kv_splits > MAX_SPLITS) return LVX_ERR_SHAPE;
     if (row_count == 0) return LVX_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -235,7 +258,7 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     p.HG = gcd(p.G, 4);
     p.RS = 4 / p.HG;
     p.row_begin = row_begin; p.row_end = row_begin + row_count;
-    const FwdForm form = fwd_form(s, row_count, kv_splits);
+    const FwdForm form = fwd_form(s, row_count, kv_splits, f32 != 0);
     p.form = form;
     if (form == FWD_FEW) {
         p.n_row_tiles = (row_count * p.G + 31) / 32;      // tiles of 32 (row, head of the group) columns
@@ -282,14 +305,16 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     }
 
     // key splits: partials [split][B*Hq][row_count][D] + LSE [split][B*Hq][row_count]
-    const size_t need = lvx_fwd_workspace_bytes(s, row_count, nsplit);
+    const size_t need = lvx_fwd_workspace_bytes(s, row_count, nsplit | f32);
     if (!workspace || workspace_bytes < need) return LVX_ERR_WORKSPACE;
     if (!aligned16(workspace)) return LVX_ERR_ALIGN;
     const int64_t rows = (int64_t)s->B * s->Hq * row_count;
     uint16_t* o_ws = static_cast<uint16_t*>(workspace);
-    float* l_ws = reinterpret_cast<float*>(o_ws + (int64_t)nsplit * rows * s->D);
+    const int words = f32 ? 2 : 1;       // of 16 bits per element of a part
+    float* l_ws = reinterpret_cast<float*>(o_ws + (int64_t)nsplit * rows * s->D * words);
     // the kernel indexes partials by absolute row: bias the bases by -row_begin
-    p.o = o_ws - (int64_t)row_begin * s->D;
+    p.o = o_ws - (int64_t)row_begin * s->D * words;
+    p.o_f32 = f32 != 0;
     p.os = Strides3{(int64_t)s->Hq * row_count * s->D, (int64_t)row_count * s->D, s->D};
     p.o_split_stride = rows * s->D;
     p.lse = l_ws - row_begin;
@@ -312,6 +337,7 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     m.l_acc_bh = s->Lq;
     m.l_part_bh = row_count;
     m.nparts = nsplit;
+    m.part_f32 = p.o_f32;
     m.use_acc = 0;
     if (o_in) {      // the partials and the incoming accumulator in one launch
         m.use_acc = 1;
@@ -369,7 +395,7 @@ int lvx_fwd_noalloc(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
                     void* stream) {
     // argument errors first, as lvx_fwd reports them
     LVX_TRY(check_shape(s));
-    if (kv_splits < 1 || kv_splits > MAX_SPLITS) return LVX_ERR_SHAPE;
+    if (kv_splits < 1 || (kv_splits & ~LVX_SPLITS_FP32) < 1 || (kv_splits & ~LVX_SPLITS_FP32) > MAX_SPLITS) return LVX_ERR_SHAPE;
     if (row_count > 0 && lvx_fwd_workspace_bytes(s, row_count, kv_splits) > NOALLOC_SCRATCH_BYTES)
         return LVX_ERR_WORKSPACE;     // the partials of this call do not fit the library's own array
     void* ws = nullptr;

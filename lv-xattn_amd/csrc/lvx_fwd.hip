@@ -316,12 +316,18 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
     const float l_tot = l_i + __shfl_xor(l_i, 32);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if (row_ok) {
-        uint16_t* op = p.o + split * p.o_split_stride + b * p.os.b + h * p.os.h + (int64_t)row * p.os.s;
+        const int64_t at = split * p.o_split_stride + b * p.os.b + h * p.os.h + (int64_t)row * p.os.s;
+        uint16_t* op = p.o + at;
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
             for (int vg = 0; vg < 4; ++vg) {
                 if (dt * 32 + 8 * vg + 4 * g >= DH) continue;      // only with DH = 16
+                if (p.o_f32) {
+                    const f32x4 x = {acc[dt][4 * vg] * inv, acc[dt][4 * vg + 1] * inv, acc[dt][4 * vg + 2] * inv, acc[dt][4 * vg + 3] * inv};
+                    *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.o) + at + dt * 32 + 8 * vg + 4 * g) = x;
+                    continue;
+                }
                 u32x2 w;
                 w[0] = E::pack(acc[dt][4 * vg] * inv, acc[dt][4 * vg + 1] * inv);
                 w[1] = E::pack(acc[dt][4 * vg + 2] * inv, acc[dt][4 * vg + 3] * inv);
@@ -568,30 +574,52 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     // wave go through its quarter of the tile buffers and leave as whole rows, 16 bytes per lane.
     // Chunk c of row r sits at position c ^ (r mod chunks per row) (DH = 64: c ^ (r / 2 mod 8)), its
     // 8-byte halves exchanged in rows with bit 4 set: conflict-free both ways.
+    // Parts in fp32 go one block of 32 rows at a time, chunk c of row r at position c ^ (r mod chunks per row).
     __syncthreads();     // every wave is done with the tiles
     char* const ep = kv_lds + wave * TB;
+    const int64_t o_head = split * p.o_split_stride + b * p.os.b + h * p.os.h;
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
         float l_tot = l_i[blk] + __shfl_xor(l_i[blk], 32);     // the two lane halves hold partial sums of the same row
         if (empty[blk]) l_tot = 0.f;
         const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
         const int r = 32 * blk + l32, pos = DH == 128 ? (r & 15) : ((r >> 1) & 7);
+        if (p.o_f32) {
+            constexpr int CPF = DH / 4;                          // chunks of a row of floats
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
+            for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-            for (int vg = 0; vg < 4; ++vg) {
-                u32x2 w;
-                w[0] = E::pack(acc[blk][dt][4 * vg] * inv, acc[blk][dt][4 * vg + 1] * inv);
-                w[1] = E::pack(acc[blk][dt][4 * vg + 2] * inv, acc[blk][dt][4 * vg + 3] * inv);
-                *reinterpret_cast<u32x2*>(ep + r * ROWB + (((4 * dt + vg) ^ pos) << 4) + ((g ^ ((r >> 4) & 1)) << 3)) = w;
+                for (int vg = 0; vg < 4; ++vg) {
+                    const f32x4 x = {acc[blk][dt][4 * vg] * inv, acc[blk][dt][4 * vg + 1] * inv, acc[blk][dt][4 * vg + 2] * inv, acc[blk][dt][4 * vg + 3] * inv};
+                    *reinterpret_cast<f32x4*>(ep + l32 * (4 * DH) + (((8 * dt + 2 * vg + g) ^ (l32 & (CPF - 1))) << 4)) = x;
+                }
+            wait_lds();
+#pragma unroll
+            for (int i = 0; i < CPF / 2; ++i) {
+                const int rf = i * (64 / CPF) + lane / CPF, c = lane % CPF, row = row0 + 32 * blk + rf;
+                const f32x4 x = *reinterpret_cast<const f32x4*>(ep + rf * (4 * DH) + ((c ^ (rf & (CPF - 1))) << 4));
+                if (row < p.row_end) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.o) + o_head + (int64_t)row * p.os.s + c * 4) = x;
             }
+            wait_lds();          // read before the next block takes its place
+        } else {
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int vg = 0; vg < 4; ++vg) {
+                    u32x2 w;
+                    w[0] = E::pack(acc[blk][dt][4 * vg] * inv, acc[blk][dt][4 * vg + 1] * inv);
+                    w[1] = E::pack(acc[blk][dt][4 * vg + 2] * inv, acc[blk][dt][4 * vg + 3] * inv);
+                    *reinterpret_cast<u32x2*>(ep + r * ROWB + (((4 * dt + vg) ^ pos) << 4) + ((g ^ ((r >> 4) & 1)) << 3)) = w;
+                }
+        }
         if (g == 0 && row0 + r < p.row_end) {
             const float lse = l_tot > 0.f ? m_i[blk] * p.scale + __logf(l_tot) : -INFINITY;
             p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + h) * p.lse_bh_stride + row0 + r] = lse;
         }
     }
+    if (p.o_f32) return;
     wait_lds();          // this wave's rows are its own
-    uint16_t* const ob = p.o + split * p.o_split_stride + b * p.os.b + h * p.os.h;
+    uint16_t* const ob = p.o + o_head;
 #pragma unroll
     for (int i = 0; i < CPR; ++i) {
         const int r = i * RPL + lane / CPR, c = lane % CPR, pos = DH == 128 ? (r & 15) : ((r >> 1) & 7);
@@ -836,9 +864,12 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
         den = fmaf(w[k], ml[k][1][oc], den);
     }
     const float inv = den > 0.f ? 1.f / den : 0.f;
-    uint16_t* const op = p.o + split * p.o_split_stride + b * p.os.b + oh * p.os.h + (int64_t)orow * p.os.s + part * DPT;
+    const int64_t at = split * p.o_split_stride + b * p.os.b + oh * p.os.h + (int64_t)orow * p.os.s + part * DPT;
+    uint16_t* const op = p.o + at;
+    float* const op32 = reinterpret_cast<float*>(p.o) + at;
     const float* const src = reinterpret_cast<const float*>(lds) + oc * EPS + part * DPT;
     uint32_t out[DPT / 2];
+    float out32[DPT];
 #pragma unroll
     for (int d = 0; d < DPT; d += 2) {
         float x0 = 0.f, x1 = 0.f;
@@ -847,9 +878,14 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
             x0 = fmaf(w[k], src[k * (32 * EPS) + d], x0);
             x1 = fmaf(w[k], src[k * (32 * EPS) + d + 1], x1);
         }
-        out[d / 2] = E::pack(x0 * inv, x1 * inv);
+        out32[d] = x0 * inv;
+        out32[d + 1] = x1 * inv;
+        out[d / 2] = E::pack(out32[d], out32[d + 1]);
     }
-    if constexpr (DPT >= 8) {
+    if (p.o_f32) {
+#pragma unroll
+        for (int d = 0; d < DPT; d += 2) *reinterpret_cast<float2*>(op32 + d) = float2{out32[d], out32[d + 1]};
+    } else if constexpr (DPT >= 8) {
 #pragma unroll
         for (int d = 0; d < DPT / 8; ++d)
             *reinterpret_cast<u32x4*>(op + 8 * d) = u32x4{out[4 * d], out[4 * d + 1], out[4 * d + 2], out[4 * d + 3]};

@@ -30,7 +30,7 @@ struct FwdParams {
     const uint16_t* q;
     const uint16_t* k;
     const uint16_t* v;
-    uint16_t* o;
+    uint16_t* o;               // float* with o_f32
     float* lse;
     Strides3 qs, ks, vs, os;
     int64_t o_split_stride;    // elements between the partial O of two key splits
@@ -51,12 +51,13 @@ struct FwdParams {
     int n_row_tiles, n_head_groups, nsplit, split_len, total_wg;
     float scale, scale_log2e;
     int f16;                   // element type of q, k, v, o: 0 bf16, 1 fp16
+    int o_f32;                 // 1: o (the parts of a launch with key splits) is fp32
 };
 
 struct MergeParams {
     uint16_t* o_acc;
     float* l_acc;
-    const uint16_t* o_part;
+    const uint16_t* o_part;    // const float* with part_f32
     const float* l_part;
     Strides3 oa, op;
     int64_t o_part_stride;     // elements between consecutive partials
@@ -73,6 +74,7 @@ struct MergeParams {
     int B, Hq, Lq, row_begin, row_end;
     int f16;
     int D;                     // head dimension: 16, 32, 64 or 128 (0 reads as 128)
+    int part_f32;              // 1: the parts are fp32 (not for one part folded into an accumulator)
 };
 
 // Per text row the hull of the keys a dense bias leaves visible (entries other than -inf).

@@ -31,8 +31,9 @@ __device__ __forceinline__ void unpack8(u32x4 u, float f[8]) {
 // (o_acc, l_acc) <- merge(acc?, part_0 .. part_{n-1}) for every (b, h, row).  PL lanes share the parts
 // of a 16-byte column of a row: with few rows (a token being generated, cut into dozens of key
 // ranges) the launch is as long as a thread's chain of loads, so the parts of a row go side by side
-// and each thread has the loads of four parts in flight, O beside the LSE it will be weighted by.
-template <bool F16, int PL>
+// and each thread has the loads of four parts in flight, O beside the LSE it will be weighted by.  PART32: the
+// parts are fp32.
+template <bool F16, int PL, bool PART32>
 __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     using E = Elt<F16>;
     constexpr int PSH = PL == 4 ? 2 : PL == 2 ? 1 : 0, BATCH = 4;
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     for (int j = 0; j < 8; ++j) out[j] = 0.f;
     // folds the parts (l[k], u[k]) in; a part with weight 0 may hold anything (it saw no key, or nothing
     // had been folded into the accumulator yet)
-    auto fold = [&](const float (&l)[BATCH], const u32x4 (&u)[BATCH]) {
+    auto fold = [&](const float (&l)[BATCH], auto&& part) {
         float mn = m;
 #pragma unroll
         for (int k = 0; k < BATCH; ++k) mn = fmaxf(mn, l[k]);
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
             const float w = __expf(l[k] - ms);
             den += w;
             float f[8];
-            unpack8<E>(u[k], f);
+            part(k, f);
 #pragma unroll
             for (int j = 0; j < 8; ++j) out[j] = w > 0.f ? fmaf(f[j], w, out[j]) : out[j];
         }
@@ -80,24 +81,37 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
         la = p.l_in ? p.l_in[(int64_t)bh * p.l_in_bh + row] : p.l_acc[(int64_t)bh * p.l_acc_bh + row];
         ua = *reinterpret_cast<const u32x4*>(p.o_in ? p.o_in + b * p.oi.b + h * p.oi.h + (int64_t)row * p.oi.s + chunk * 8 : oa);
     }
-    const uint16_t* op = p.o_part + b * p.op.b + h * p.op.h + (int64_t)row * p.op.s + chunk * 8;
+    const int64_t at = b * p.op.b + h * p.op.h + (int64_t)row * p.op.s + chunk * 8;
+    const uint16_t* op = p.o_part + at;
+    const float* op32 = reinterpret_cast<const float*>(p.o_part) + at;
     const float* lp = p.l_part + (int64_t)bh * p.l_part_bh + row;
     for (int i = pl; i < p.nparts; i += PL * BATCH) {
         float l[BATCH];
-        u32x4 u[BATCH];
+        u32x4 u[BATCH], u2[PART32 ? BATCH : 1];
 #pragma unroll
         for (int k = 0; k < BATCH; ++k) {
             const int part = i + k * PL;
             const bool ok = part < p.nparts;
             l[k] = ok ? lp[part * p.l_part_stride] : -INFINITY;
-            u[k] = ldg16(op + part * p.o_part_stride, ok);
+            if constexpr (PART32) {
+                u[k] = ldg16(op32 + part * p.o_part_stride, ok);
+                u2[k] = ldg16(op32 + part * p.o_part_stride + 4, ok);
+            } else {
+                u[k] = ldg16(op + part * p.o_part_stride, ok);
+            }
         }
-        fold(l, u);
+        fold(l, [&](int k, float (&f)[8]) {
+            if constexpr (PART32) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) { f[j] = __uint_as_float(u[k][j]); f[4 + j] = __uint_as_float(u2[k][j]); }
+            } else {
+                unpack8<E>(u[k], f);
+            }
+        });
     }
     if (p.use_acc) {
         const float l[BATCH] = {la, -INFINITY, -INFINITY, -INFINITY};
-        const u32x4 u[BATCH] = {ua, zero, zero, zero};
-        fold(l, u);
+        fold(l, [&](int k, float (&f)[8]) { unpack8<E>(k ? zero : ua, f); });
     }
 #pragma unroll
     for (int o = 1; o < PL; o <<= 1) {                  // the lanes that share a row's parts
@@ -601,13 +615,15 @@ hipError_t launch_merge(const MergeParams& p, hipStream_t st) {
     // as many lanes per row as the parts need (four parts each) and the chip has room for
     const int pl = p.nparts > 8 && rows < 16384 ? 4 : p.nparts > 4 && rows < 32768 ? 2 : 1;
     const dim3 grid(blocks_for(rows * pl));
-    auto go = [&](auto f16) {
+    auto go = [&](auto f16, auto part32) {
         constexpr bool F16 = decltype(f16)::value;
-        if (pl == 4) return launch1(merge_kernel<F16, 4>, grid, dim3(256), st, p);
-        if (pl == 2) return launch1(merge_kernel<F16, 2>, grid, dim3(256), st, p);
-        return launch1(merge_kernel<F16, 1>, grid, dim3(256), st, p);
+        constexpr bool PART32 = decltype(part32)::value;
+        if (pl == 4) return launch1(merge_kernel<F16, 4, PART32>, grid, dim3(256), st, p);
+        if (pl == 2) return launch1(merge_kernel<F16, 2, PART32>, grid, dim3(256), st, p);
+        return launch1(merge_kernel<F16, 1, PART32>, grid, dim3(256), st, p);
     };
-    return p.f16 ? go(std::true_type{}) : go(std::false_type{});
+    if (p.part_f32) return p.f16 ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
+    return p.f16 ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
 }
 
 hipError_t launch_preprocess(const PreParams& p, hipStream_t st) {

@@ -81,3 +81,39 @@ def test_every_form_repeats_itself(D, form, monkeypatch):
         _, _, _, o, lse = lv_xattn._attn_forward(q, k, v, False, D ** -0.5, None, rounds=1, batched=True)
         first = first or (o, lse)
         assert torch.equal(o, first[0]) and torch.equal(lse, first[1])
+
+
+# the parts of key splits in fp32 (LVX_SPLITS_FP32), at the edges of every form's tiles
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [128, 64, 32, 16])
+@pytest.mark.parametrize("form", ["0", "1", "2"])
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lkv,splits,mask", [
+    (4, 1, 1, 65, 2, "none"), (4, 1, 63, 129, 3, "intervals"), (8, 2, 33, 300, 5, "kv_len"), (2, 2, 65, 700, 9, "images"),
+    (4, 2, 3, 2500, 64, "none")])
+def test_parts_in_fp32(D, dtype, form, Hq, Hkv, Lq, Lkv, splits, mask, monkeypatch):
+    monkeypatch.setenv("LVX_FWD_WIDE", form)
+    _check(D, dtype, 2, Hq, Hkv, Lq, Lkv, splits | 256, mask, Lq * 1000 + Lkv + 2)
+
+
+# few rows, a short range, and 528 work-groups of 32-row waves (a last round that the splits even out).  A part in
+# 16 bits would add a rounding of the size of the result's own, sqrt(2) in quadrature less what P's rounding
+# adds to both: 1.2 measured; 1.05 leaves room for the sample (at least 25600 elements, 1 % of a norm).
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Lq,Lkv", [(25, 929), (256, 929), (2100, 6404)])
+def test_splits_chosen_by_the_library_keep_the_precision_of_a_whole_launch(Lq, Lkv, dtype):
+    import lv_xattn
+    from lv_xattn.attn import auto_kv_splits
+    B, Hq, Hkv, D = 1, 32, 8, 128
+    assert auto_kv_splits(B, Hq, Hkv, Lq, Lkv) & 255 > 1
+    g = torch.Generator(device=DEV).manual_seed(Lq)
+    q, k, v = (torch.empty(B, h, n, D, device=DEV, dtype=dtype).normal_(generator=g) for h, n in ((Hq, Lq), (Hkv, Lkv), (Hkv, Lkv)))
+    error = []
+    for splits in (None, 1):
+        o = lv_xattn._attn_forward(q, k, v, False, D ** -0.5, None, rounds=1, batched=True, kv_splits=splits)[3]
+        diff = ref = 0.0
+        for h in range(0, Hq, 4):
+            exact = torch.softmax(q[0, h].double() @ k[0, h // 4].double().T.contiguous() * D ** -0.5, -1) @ v[0, h // 4].double()
+            diff += (o[0, h].double() - exact).square().sum().item()
+            ref += exact.square().sum().item()
+        error.append((diff / ref) ** 0.5)
+    assert error[0] < 1.05 * error[1], error
