@@ -98,19 +98,19 @@ def _mask_intervals(mask: torch.Tensor, query: torch.Tensor, lkv: int):
     gets the same mask, so the last answer is kept, with the mask, as `_mask_bias` keeps its own, for
     calls on the stream it was made on.  A mask of another form or place than the query's rows and keys is
     `_mask_bias`'s, and so is any mask while a graph is captured: a replay has to read the mask as it is
-    then, not as it was when the answer was kept, and the graph does not own what is kept here."""
+    then, not as it was when the answer was kept, and the graph does not own what is kept here.  An inference
+    tensor (torch.inference_mode) has no version counter, so that no answer for it can be kept: asking would make
+    every layer wait for the GPU, and it is `_mask_bias`'s as well, whose path asks nothing back."""
     global _interval_cache
-    if tuple(mask.shape) != (query.shape[0], 1, query.shape[2], lkv) or mask.device != query.device or _capturing():
+    if tuple(mask.shape) != (query.shape[0], 1, query.shape[2], lkv) or mask.device != query.device or _capturing() or mask.is_inference():
         return None
-    version = None if mask.is_inference() else mask._version
-    key = (mask.data_ptr(), version, tuple(mask.shape), tuple(mask.stride()), mask.dtype, mask.device,
+    key = (mask.data_ptr(), mask._version, tuple(mask.shape), tuple(mask.stride()), mask.dtype, mask.device,
            torch.cuda.current_stream(mask.device).cuda_stream)
     kept = _interval_cache          # read once: another thread may put its own in place
-    if version is not None and kept and kept[0] == key:
+    if kept and kept[0] == key:
         return kept[1]
     intervals = ops.mask_intervals(mask)
-    if version is not None:
-        _interval_cache = (key, intervals, mask)
+    _interval_cache = (key, intervals, mask)
     return intervals
 
 

@@ -144,6 +144,23 @@ def test_a_capture_uses_no_answer_that_was_kept(gpu, seen):
             assert seen[-1][1] is not None and seen[-1][1] is not kept
 
 
+def test_layers_in_inference_mode_wait_for_nothing(gpu, seen):
+    """A mask without a version counter: nothing can be kept for it, so nothing that has to come back to the host is
+    asked in any of the layers; with a version, the first layer asks and the others find the answer."""
+    with torch.inference_mode():
+        q, k, v = _qkv()
+        mask = _mask(20)
+        for _ in range(4):
+            hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)
+    assert gpu.waits == [] and all(bias is not None for _, bias in seen)
+    with torch.no_grad():
+        q, k, v = _qkv()
+        mask = _mask(20)
+        for _ in range(4):
+            hf_mllama.lv_xattn_attention_forward(_Layer(), q, k, v, mask)
+    assert gpu.waits == ["mask_intervals"]
+
+
 def test_the_result_of_a_recorded_call_may_be_written_to(no_kernels):
     """A caller may scale or mask the attention's output in place before it is projected: what backward needs is
     not that memory."""
