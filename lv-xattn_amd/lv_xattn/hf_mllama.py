@@ -100,9 +100,12 @@ def _mask_intervals(mask: torch.Tensor, query: torch.Tensor, lkv: int):
     `_mask_bias`'s, and so is any mask while a graph is captured: a replay has to read the mask as it is
     then, not as it was when the answer was kept, and the graph does not own what is kept here.  An inference
     tensor (torch.inference_mode) has no version counter, so that no answer for it can be kept: asking would make
-    every layer wait for the GPU, and it is `_mask_bias`'s as well, whose path asks nothing back."""
+    every layer wait for the GPU, and it is `_mask_bias`'s as well, whose path asks nothing back.  So is a mask under
+    torch.jit.trace, which would record the answer for the mask of the trace as a constant."""
     global _interval_cache
-    if tuple(mask.shape) != (query.shape[0], 1, query.shape[2], lkv) or mask.device != query.device or _capturing() or mask.is_inference():
+    if tuple(mask.shape) != (query.shape[0], 1, query.shape[2], lkv) or mask.device != query.device:
+        return None
+    if _capturing() or mask.is_inference() or torch.jit.is_tracing():
         return None
     key = (mask.data_ptr(), mask._version, tuple(mask.shape), tuple(mask.stride()), mask.dtype, mask.device,
            torch.cuda.current_stream(mask.device).cuda_stream)
@@ -142,8 +145,9 @@ def lv_xattn_attention_forward(module, query, key, value, attention_mask: Option
         mask = attention_mask[..., :query.shape[2], :key.shape[2]]
         intervals = _mask_intervals(mask, query, key.shape[2])
     # the autograd function is only passed by where it has nothing to do: no gradient is recorded, and no input
-    # carries a forward-mode tangent, which it refuses (it has no jvp) and the kernels would silently drop
-    if (mask is None or intervals is not None) and not any(
+    # carries a forward-mode tangent, which it refuses (it has no jvp) and the kernels would silently drop, and no
+    # torch.jit.trace is on, which records the function as one step but nothing of the kernels' work by itself
+    if (mask is None or intervals is not None) and not torch.jit.is_tracing() and not any(
             (torch.is_grad_enabled() and t.requires_grad) or unpack_dual(t).tangent is not None for t in (query, key, value)):
         out = _attn_forward(query, key, value, False, scaling, None, rounds=1, batched=True, mask=intervals, _token_major=True)[3]
         return out.transpose(1, 2).contiguous(), None

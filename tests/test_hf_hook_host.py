@@ -45,6 +45,38 @@ def test_a_forward_mode_tangent_is_refused(no_kernels, which, grad):
             hf_mllama.lv_xattn_attention_forward(_Layer(), *qkv, None)
 
 
+class _Net(_Layer):
+    def forward(self, q, k, v, mask=None):
+        return hf_mllama.lv_xattn_attention_forward(self, q, k, v, mask)[0]
+
+
+@pytest.mark.filterwarnings("ignore")       # the tracer's, about the stand-in
+def test_a_traced_call_computes(monkeypatch):
+    """torch.jit.trace without gradients: what it records runs the kernels on the inputs of each later call.  The
+    kernels write where the tracer does not look, so a trace without the autograd function would return memory that
+    nothing has written.  A mask, which the function takes in a list, is refused by the tracer, where the intervals
+    of the mask it saw would be a constant to it."""
+    def forward(q, k, v, causal, scale, mode, bias_func=None, local=(), *args, mask=None, _token_major=False, **kw):
+        assert mask is None
+        bias_func is None or bias_func(*local)
+        o = torch.empty(q.shape)
+        o.detach().numpy()[...] = 5 * q.detach().numpy()
+        return q, k, v, o, torch.zeros(q.shape[0] * q.shape[1], q.shape[2])
+
+    for module in (hf_mllama, autograd):
+        monkeypatch.setattr(module, "_attn_forward", forward)
+    monkeypatch.setattr(hf_mllama, "_require_supported", lambda *a: None)
+    monkeypatch.setattr(ops, "mask_intervals", lambda mask: ops.Mask())
+    hf_mllama.clear_mask_cache()
+    with torch.no_grad():
+        traced = torch.jit.trace(_Net(), tuple(t.float() for t in _qkv()), check_trace=False)
+        q, k, v = (t.float() for t in _qkv())
+        assert torch.equal(traced(q, k, v), 5 * q.transpose(1, 2))
+        with pytest.raises(RuntimeError):
+            torch.jit.trace(_Net(), (q, k, v, _mask(20)), check_trace=False)
+    hf_mllama.clear_mask_cache()
+
+
 class _Gpu:
     """Stands in for the current stream: its number, and whether it is capturing."""
 
