@@ -396,8 +396,9 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     const int kv_hi = min(kv_len, kv_lo + p.split_len);
 
     // visible key interval of this lane's two rows.  Rows past the window and rows that see nothing
-    // are let see everything - the former are never stored, the latter stored as zeros - so that
-    // they do not make whole tiles take the element mask.
+    // are let see everything, with a Q of zeros - the former are never stored, the latter stored as zeros, which
+    // 0 times what a Q of infinities or NaN gives would not be - so that they do not make whole tiles take the
+    // element mask.
     int my_s[2] = {kv_lo, kv_lo}, my_e[2] = {kv_hi, kv_hi};
     bool empty[2] = {kv_hi <= kv_lo, kv_hi <= kv_lo};
     int lo = kv_lo, hi = kv_hi, in_lo = kv_lo, in_hi = kv_hi;
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
             const int row = row0 + 32 * blk + l32;
             const uint16_t* qp = p.q + b * p.qs.b + h * p.qs.h + (int64_t)row * p.qs.s + g * 8;
 #pragma unroll
-            for (int kk = 0; kk < NKK; ++kk) q[blk][kk] = as_bf16x8(ldg16(qp + kk * 16, row < p.row_end));
+            for (int kk = 0; kk < NKK; ++kk) q[blk][kk] = as_bf16x8(ldg16(qp + kk * 16, row < p.row_end && !empty[blk]));
         }
 
         // LDS -> operands.  K rows (A of S^T): chunk 2 kk + g of row l32 (+ 32).  V^T (A of O^T += V^T P^T),
@@ -690,7 +691,7 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
         my_s = max(kv_lo, p.kv_start[(int64_t)b * p.Lq + row]);
         my_e = min(kv_hi, p.kv_end[(int64_t)b * p.Lq + row]);
         empty = my_e <= my_s;
-        // a row that sees nothing is let see everything and stored as zeros
+        // a row that sees nothing is let see everything, with a Q of zeros, and stored as zeros (see fwd_wide_kernel)
         lo = empty ? BIG : my_s; hi = empty ? 0 : my_e;
         in_lo = empty ? 0 : my_s; in_hi = empty ? BIG : my_e;
         if (empty) { my_s = 0; my_e = BIG; }
@@ -756,7 +757,10 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     asm volatile("s_cmp_gt_i32 %0, 1\n\ts_cbranch_scc1 LVX_FEW_TWO_%=\n\ts_waitcnt vmcnt(0)\nLVX_FEW_TWO_%=:\n\ts_waitcnt vmcnt(%1)"
                  ::"s"(uniform32(n)), "n"(4 * NLD) : "memory", "scc");
 #pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) asm volatile("" : "+v"(q[kk]));
+    for (int kk = 0; kk < NKK; ++kk) {
+        asm volatile("" : "+v"(q[kk]));
+        if (MASKED && empty) q[kk] = u32x4{0u, 0u, 0u, 0u};
+    }
 
     for (int i = 0; i < n; ++i) {
         const int kv0 = base + 32 * (wave + 4 * i);

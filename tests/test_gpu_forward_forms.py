@@ -117,3 +117,28 @@ def test_splits_chosen_by_the_library_keep_the_precision_of_a_whole_launch(Lq, L
             ref += exact.square().sum().item()
         error.append((diff / ref) ** 0.5)
     assert error[0] < 1.05 * error[1], error
+
+
+# Rows with an empty interval (padding, whose q may hold anything) among rows that see keys: zeros and -inf, exactly
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form,D", [("0", 128), ("0", 64), ("1", 128), ("1", 64), ("2", 128), ("2", 64), ("2", 32), ("2", 16)])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("junk", [float("nan"), float("inf")])
+def test_a_row_that_sees_nothing_is_zero_whatever_its_q(form, D, dtype, splits, junk, monkeypatch):
+    import lv_xattn
+    monkeypatch.setenv("LVX_FWD_WIDE", form)
+    B, Hq, Hkv, Lq, Lkv = 2, 4, 2, 40, 300
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(dtype) for h, n in ((Hq, Lq), (Hkv, Lkv), (Hkv, Lkv)))
+    start = torch.randint(0, Lkv - 1, (B, Lq), generator=g, dtype=torch.int32)
+    end = torch.randint(1, Lkv + 1, (B, Lq), generator=g, dtype=torch.int32)
+    end = torch.maximum(end, start + 1)
+    dead = torch.arange(Lq)[None] % 3 == torch.tensor([[0], [1]])
+    end[dead] = start[dead] - torch.arange(Lq).expand(B, Lq)[dead].int() % 2        # [s, s) and [s, s - 1)
+    o_ref, l_ref = orc.attention_dense(q, k, v, D ** -0.5, allowed=orc.interval_mask(start.long(), end.long(), Lkv))
+    q.transpose(1, 2)[dead] = junk
+    _, _, _, o, lse = lv_xattn._attn_forward(q.to(DEV), k.to(DEV), v.to(DEV), False, D ** -0.5, None, rounds=1, batched=True,
+                                             mask=lv_xattn.Mask(None, start, end), kv_splits=splits)
+    check_o(o, o_ref)
+    check_lse(lse, l_ref)
+    assert not o.cpu().transpose(1, 2)[dead].any()
