@@ -486,8 +486,11 @@ int lvx_bwd_preprocess(const lvx_attn_shape* s, const lvx_tensor* o, const lvx_t
 // and rounded after) evens that out.  S minimises
 //     rounds(S) * (steps / S + WG_COST) + (S > 1 ? SPLIT_COST : 0)        [in steps]
 // with ranges of at least 32 steps; WG_COST is what a work-group spends outside its
-// steps (operand load, ring fill, epilogue: about 8 us = 6 steps), SPLIT_COST the zero-fill, the
-// two casts and the slower atomic epilogue (about 70 us).  rounds(S) = ceil(blocks * S / CUs)
+// steps (operand load, ring fill, epilogue: about 8 us = 6 steps), SPLIT_COST what sharing blocks
+// adds to the launch.  55 steps, about 70 us, were measured where every block is shared and the
+// whole scratch zeroed and rounded; only the shared blocks are by now, and nothing is in a call that
+// accumulates, so for a few shared blocks it is an upper bound, which errs on the side of not
+// cutting.  rounds(S) = ceil(blocks * S / CUs)
 // for equal work-groups.  With an interval mask they differ in length (a token block
 // visits only the row tiles that see it; half of them is assumed); given at least two per CU the
 // dispatcher fills the tail by itself and rounds(S) is the plain quotient: splitting then
