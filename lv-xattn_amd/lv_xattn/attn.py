@@ -188,8 +188,10 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
     max_rows = max(r1 - r0 for r0, r1 in windows)
     if kv_splits is None:
         kv_splits = auto_kv_splits(B, Hq, k_.shape[1], max_rows, k_.shape[2], D, bias is not None)
-    # the parts of the key splits live for this call only (from torch's caching allocator, as o and L)
-    o, L, ws = host().forward_buffers(q_, max_rows, kv_splits, _token_major)
+    # the parts of the key splits live for this call only (from torch's caching allocator, as o and L); rounds
+    # on several streams have a buffer per stream
+    overlap = streams > 1 and len(windows) > 1
+    o, L, ws = host().forward_buffers(q_, max_rows, 1 if overlap else kv_splits, _token_major)
 
     # the partial goes straight into (o, L), merged on its way with the incoming accumulator
     # if there is one (with key splits by the launch that folds the splits; neither a copy of
@@ -199,11 +201,12 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
     def one_round(r0, r1, ws):
         ops.fwd(q_, k_, v_, o, L, sm_scale, r0, r1 - r0, mask, kv_splits, ws, bias, acc=acc)
 
-    if streams > 1 and len(windows) > 1:
+    if overlap:
+        nbytes = ops.fwd_workspace_bytes(q_, k_, max_rows, kv_splits) if kv_splits > 1 else 0
         with _RoundStreams(dev, min(streams, len(windows))) as rs:
             for i, (r0, r1) in enumerate(windows):
                 with rs.stream(i):
-                    ws_i = workspace("fwd_split", (ws.numel(),), torch.uint8, dev) if ws is not None else None
+                    ws_i = workspace("fwd_split", (nbytes,), torch.uint8, dev) if nbytes else None
                     one_round(r0, r1, ws_i)
     else:
         for r0, r1 in windows:
