@@ -289,17 +289,16 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
         return;
     }
     // A lane holds 4 consecutive columns of one C row, so storing from the registers writes 8
-    // bytes per lane into 32 different rows per instruction.  Where 256 rows of the tile fit the
-    // stage buffers (free by now) they go through LDS instead, 256 rows at a time, and leave as
-    // whole row segments (TN * 2 bytes), 16 bytes per lane.  16-byte chunk c of row r sits at
-    // position c ^ (r mod chunks per row), with its two 8-byte halves exchanged in rows where
-    // bits 3 and 4 differ: the 32 rows a half-wave's 8-byte writes touch then land in different
+    // bytes per lane into 32 different rows per instruction.  The rows go through the stage buffers
+    // (free by now) instead, 256 at a time, and leave as whole row segments (TN * 2 bytes; N is a
+    // multiple of 8), 16 bytes per lane.  16-byte chunk c of row r sits at position
+    // c ^ (r mod chunks per row), with its two 8-byte halves exchanged in rows where bits 3 and 4 differ: the 32 rows a half-wave's 8-byte writes touch then land in different
     // chunks or, where they share a chunk position or banks (positions 8 or 16 apart), in
     // different halves; a read instruction takes whole rows.  Both are conflict-free.
     // `pair(mt, nt, vg)`: the 4 values of accumulator tile (nt, mt), register group vg, as two
     // packed words.
     constexpr int CPR = TN / 8;                 // 16-byte chunks per row
-    constexpr bool VIA_LDS = (TN == 256 || TN == 128) && TM % 256 == 0 && 256 * TN * 2 <= NS * STAGE;
+    static_assert((TN == 256 || TN == 128) && TM % 256 == 0 && 256 * TN * 2 <= NS * STAGE, "256 rows of the tile fit the stages");
     auto store_via_lds = [&](auto pair, uint16_t* dst) __attribute__((always_inline)) {
 #pragma unroll
         for (int pass = 0; pass < TM / 256; ++pass) {
@@ -359,92 +358,41 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
             for (int mt = 0; mt < WM; ++mt) rs[mt] += red[(pw * WM + mt) * 32 + l32];
         }
         const int groups = p.N >> 7;
-        if (VIA_LDS) {       // (N is a multiple of 128 here)
-            float rr[WM];
-#pragma unroll
-            for (int mt = 0; mt < WM; ++mt) {
-                const int m = m0 + 32 * (WM * wm + mt) + l32;
-                rr[mt] = rsqrtf(rs[mt] * (1.f / 128.f) + p.norm_eps);
-                const int ncol = n0 + 32 * WN * wn;
-                if (m < p.M && p.rstd && g == 0 && (wn & (HW - 1)) == 0 && ncol < p.N) p.rstd[(int64_t)m * groups + (ncol >> 7)] = rr[mt];
-            }
-            if (p.c_raw)
-                store_via_lds([&](int mt, int nt, int vg) {
-                    u32x2 w;
-                    w[0] = E::pack(acc[nt][mt][4 * vg], acc[nt][mt][4 * vg + 1]);
-                    w[1] = E::pack(acc[nt][mt][4 * vg + 2], acc[nt][mt][4 * vg + 3]);
-                    return w;
-                }, p.c_raw + (Cz - pr.C));
-            store_via_lds([&](int mt, int nt, int vg) {
-                const int n = 32 * (WN * wn + nt) + 8 * vg + 4 * g;       // n0 is a multiple of 128
-                const u32x2 wt = *reinterpret_cast<const u32x2*>(p.norm_w + (n & 127));
-                const float r = rr[mt];
-                const u32x2 h = {E::pack(acc[nt][mt][4 * vg] * r, acc[nt][mt][4 * vg + 1] * r),
-                                 E::pack(acc[nt][mt][4 * vg + 2] * r, acc[nt][mt][4 * vg + 3] * r)};
-                u32x2 y;
-                y[0] = E::pack(E::lo(wt[0]) * E::lo(h[0]), E::hi(wt[0]) * E::hi(h[0]));
-                y[1] = E::pack(E::lo(wt[1]) * E::lo(h[1]), E::hi(wt[1]) * E::hi(h[1]));
-                return y;
-            }, Cz);
-            return;
-        }
+        // (N is a multiple of 128 here)
+        float rr[WM];
 #pragma unroll
         for (int mt = 0; mt < WM; ++mt) {
             const int m = m0 + 32 * (WM * wm + mt) + l32;
-            if (m >= p.M) continue;
-            const float r = rsqrtf(rs[mt] * (1.f / 128.f) + p.norm_eps);
+            rr[mt] = rsqrtf(rs[mt] * (1.f / 128.f) + p.norm_eps);
             const int ncol = n0 + 32 * WN * wn;
-            if (p.rstd && g == 0 && (wn & (HW - 1)) == 0 && ncol < p.N) p.rstd[(int64_t)m * groups + (ncol >> 7)] = r;
-#pragma unroll
-            for (int nt = 0; nt < WN; ++nt)
-#pragma unroll
-                for (int vg = 0; vg < 4; ++vg) {
-                    const int n = n0 + 32 * (WN * wn + nt) + 8 * vg + 4 * g;
-                    if (n < p.N) {
-                        const float a[4] = {acc[nt][mt][4 * vg], acc[nt][mt][4 * vg + 1], acc[nt][mt][4 * vg + 2], acc[nt][mt][4 * vg + 3]};
-                        if (p.c_raw) {
-                            u32x2 w;
-                            w[0] = E::pack(a[0], a[1]);
-                            w[1] = E::pack(a[2], a[3]);
-                            *reinterpret_cast<u32x2*>(p.c_raw + (Cz - pr.C) + (int64_t)m * pr.ldc + n) = w;
-                        }
-                        const u32x2 wt = *reinterpret_cast<const u32x2*>(p.norm_w + (n & 127));
-                        const u32x2 h = {E::pack(a[0] * r, a[1] * r), E::pack(a[2] * r, a[3] * r)};
-                        u32x2 y;
-                        y[0] = E::pack(E::lo(wt[0]) * E::lo(h[0]), E::hi(wt[0]) * E::hi(h[0]));
-                        y[1] = E::pack(E::lo(wt[1]) * E::lo(h[1]), E::hi(wt[1]) * E::hi(h[1]));
-                        *reinterpret_cast<u32x2*>(Cz + (int64_t)m * pr.ldc + n) = y;
-                    }
-                }
+            if (m < p.M && p.rstd && g == 0 && (wn & (HW - 1)) == 0 && ncol < p.N) p.rstd[(int64_t)m * groups + (ncol >> 7)] = rr[mt];
         }
-        return;
-    }
-    if (VIA_LDS && (p.N & 7) == 0) {
+        if (p.c_raw)
+            store_via_lds([&](int mt, int nt, int vg) {
+                u32x2 w;
+                w[0] = E::pack(acc[nt][mt][4 * vg], acc[nt][mt][4 * vg + 1]);
+                w[1] = E::pack(acc[nt][mt][4 * vg + 2], acc[nt][mt][4 * vg + 3]);
+                return w;
+            }, p.c_raw + (Cz - pr.C));
         store_via_lds([&](int mt, int nt, int vg) {
-            u32x2 w;
-            w[0] = E::pack(acc[nt][mt][4 * vg], acc[nt][mt][4 * vg + 1]);
-            w[1] = E::pack(acc[nt][mt][4 * vg + 2], acc[nt][mt][4 * vg + 3]);
-            return w;
+            const int n = 32 * (WN * wn + nt) + 8 * vg + 4 * g;       // n0 is a multiple of 128
+            const u32x2 wt = *reinterpret_cast<const u32x2*>(p.norm_w + (n & 127));
+            const float r = rr[mt];
+            const u32x2 h = {E::pack(acc[nt][mt][4 * vg] * r, acc[nt][mt][4 * vg + 1] * r),
+                             E::pack(acc[nt][mt][4 * vg + 2] * r, acc[nt][mt][4 * vg + 3] * r)};
+            u32x2 y;
+            y[0] = E::pack(E::lo(wt[0]) * E::lo(h[0]), E::hi(wt[0]) * E::hi(h[0]));
+            y[1] = E::pack(E::lo(wt[1]) * E::lo(h[1]), E::hi(wt[1]) * E::hi(h[1]));
+            return y;
         }, Cz);
         return;
     }
-#pragma unroll
-    for (int mt = 0; mt < WM; ++mt) {
-        const int m = m0 + 32 * (WM * wm + mt) + l32;
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int nt = 0; nt < WN; ++nt)
-#pragma unroll
-            for (int vg = 0; vg < 4; ++vg) {
-                const int n = n0 + 32 * (WN * wn + nt) + 8 * vg + 4 * g;
-                if (n < p.N) {
-                    u32x2 w;
-                    w[0] = E::pack(acc[nt][mt][4 * vg], acc[nt][mt][4 * vg + 1]);
-                    w[1] = E::pack(acc[nt][mt][4 * vg + 2], acc[nt][mt][4 * vg + 3]);
-                    *reinterpret_cast<u32x2*>(Cz + (int64_t)m * pr.ldc + n) = w;
-                }
-            }
-    }
+    store_via_lds([&](int mt, int nt, int vg) {
+        u32x2 w;
+        w[0] = E::pack(acc[nt][mt][4 * vg], acc[nt][mt][4 * vg + 1]);
+        w[1] = E::pack(acc[nt][mt][4 * vg + 2], acc[nt][mt][4 * vg + 3]);
+        return w;
+    }, Cz);
 }
 
 // registers the hand-scheduled tile uses besides its operands (see gen_gemm_loop.py)
@@ -747,6 +695,7 @@ bool gemm_tile_ok(const GemmParams& p, bool a_mcontig, bool b_ncontig) {
 // streaming hint then costs a second fetch: 6404 tokens x 4096 rows x 32 heads 1868 us a step against 1821),
 // and the M tiles of a masked launch have finer contraction ranges.
 hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipStream_t st) {
+    if (p.N % 8) return hipErrorInvalidValue;
     for (int i = 0; i < p.nprob; ++i) {
         const GemmProblem& pr = p.prob[i];
         // all problems and both contraction segments share the per-thread load offsets
