@@ -97,12 +97,12 @@ const char* lvx_strerror(int code);
  * (at most 64 of them; lvx_fwd_auto_splits says how many suit a launch).  The O of a range waits for the
  * fold in 16 bits, a rounding that a launch of one range does not have (its error against exact arithmetic
  * grows by about a fifth), or with kv_splits = n | LVX_SPLITS_FP32 in fp32, in twice the workspace.
- * The kernel has three forms, chosen by what the launch is estimated to take in each: a wavefront
- * owns 32 text rows of a head (any head_dim, the only one with a dense bias); 64 rows and its SIMD
- * to itself (head_dim 128 and 64); or a share of the keys for up to 32 (row, head) pairs of a kv head at
- * once (few rows: the launch reads K and V once at the speed of HBM).  The environment variable
- * LVX_FWD_WIDE, read at every call, overrides the choice: 0 the first form, 1 the second and 2 the third
- * where they exist.
+ * The kernel has three forms: a wavefront owns 32 text rows of a head (with a dense bias, and at head_dim
+ * 16 and 32); 64 rows and its SIMD to itself (head_dim 128 and 64 without a bias); or, where that is
+ * estimated to take less, a share of the keys for up to 32 (row, head) pairs of a kv head at once (few rows
+ * without a bias, any head_dim: the launch reads K and V once at the speed of HBM).  The environment
+ * variable LVX_FWD_WIDE, read at every call, overrides that last choice: 2 the third form where it can run,
+ * any other value (0 and 1 alike) never.
  * The forms give results within the same tolerance of each other, not the same bits.
  */
 int lvx_fwd(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tensor* k,

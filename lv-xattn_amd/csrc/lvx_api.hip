@@ -184,13 +184,12 @@ static bool fwd_few_ok(const lvx_attn_shape* s, int rows) {
 // The form of the forward kernel for a window of `rows` rows whose keys are cut into `splits` ranges.
 // Head dimensions 128 and 64 without a dense bias take the wide form or, where reading K and V is the
 // larger part of the work, the form for few rows; the plain one was slower at every size measured
-// (4096 rows x 6404 keys: 429 us against 354; 300 rows x 2 samples: 92 against 88).
+// (4096 rows x 6404 keys: 429 us against 354; 300 rows x 2 samples: 92 against 88) and is not built for them.
 static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits, bool parts_f32) {
     if (s->bias) return FWD_PLAIN;
     const FwdForm many = s->D == 128 || s->D == 64 ? FWD_WIDE : FWD_PLAIN;
     if (const char* e = getenv("LVX_FWD_WIDE")) {
-        if (atoi(e) == 2 && fwd_few_ok(s, rows)) return FWD_FEW;
-        return atoi(e) != 0 ? many : FWD_PLAIN;
+        return atoi(e) == 2 && fwd_few_ok(s, rows) ? FWD_FEW : many;
     }
     return fwd_few_ok(s, rows) && fwd_cost(s, rows, FWD_FEW, splits, parts_f32) <= fwd_cost(s, rows, many, splits, parts_f32) ? FWD_FEW : many;
 }

@@ -917,14 +917,17 @@ hipError_t launch_fwd_t(const FwdParams& p, bool masked, hipStream_t st) {
             if (masked) return launch1((fwd_wide_kernel<DH, true, F16>), dim3(grid), dim3(256), st, p);
             return launch1((fwd_wide_kernel<DH, false, F16>), dim3(grid), dim3(256), st, p);
         }
+        if (!p.bias) return hipErrorInvalidValue;      // fwd_form never asks for it
     }
     if (p.bias) {
         if (masked) return launch1((fwd_kernel<DH, true, true, F16>), dim3(grid), dim3(256), st, p);
-        else return launch1((fwd_kernel<DH, false, true, F16>), dim3(grid), dim3(256), st, p);
-    } else {
-        if (masked) return launch1((fwd_kernel<DH, true, false, F16>), dim3(grid), dim3(256), st, p);
-        else return launch1((fwd_kernel<DH, false, false, F16>), dim3(grid), dim3(256), st, p);
+        return launch1((fwd_kernel<DH, false, true, F16>), dim3(grid), dim3(256), st, p);
     }
+    if constexpr (DH < 64) {
+        if (masked) return launch1((fwd_kernel<DH, true, false, F16>), dim3(grid), dim3(256), st, p);
+        return launch1((fwd_kernel<DH, false, false, F16>), dim3(grid), dim3(256), st, p);
+    }
+    return hipErrorInvalidValue;
 }
 }  // namespace
 

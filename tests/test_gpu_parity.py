@@ -267,11 +267,10 @@ def test_preprocess_delta(lvx):
 # ------------------------------------------------------------------ forward
 @pytest.fixture(params=["auto", "wide"])
 def form(request, monkeypatch):
-    """The bf16 forward kernel for launches without interval mask or bias has two forms: a wave owns 32
-    rows, or 64 rows and its SIMD (picked when every CU gets a work-group).  'wide' forces the second
-    on these small shapes - also with ragged row counts, ragged key lengths, key splits and incoming
-    accumulators - through the environment variable the library reads at every call (masked launches
-    take the plain kernel either way)."""
+    """'wide' keeps the form for few rows out of these small launches, through the environment variable the
+    library reads at every call: those without a bias then run the form in which a wave owns 64 rows and its
+    SIMD (32 at head_dim 16 and 32), also with ragged row counts, ragged key lengths, key splits and
+    incoming accumulators."""
     if request.param == "wide":
         monkeypatch.setenv("LVX_FWD_WIDE", "1")
     return request.param
