@@ -28,7 +28,9 @@ from .async_communication import reset_global_memory_buffer
 # What the projections below keep from forward to backward.  Nothing but their inputs in general; but a
 # run whose gradient follows at once - the second run of run_function, inside the attention's backward
 # - keeps the raw projection and the norm's r, which backward would otherwise form by running the same
-# GEMM a third time (230 us of a 2700 us step for K and V of 2 x 6404 tokens, 115 us for Q).
+# GEMM a third time (230 us of a 2700 us step for K and V of 2 x 6404 tokens, 115 us for Q).  They are kept beside
+# the saved tensors (ctx.kept), whose number must not depend on this: torch.utils.checkpoint inside run_function
+# compares it with that of a recomputation, which it makes later, in a run of its own.
 _this_run = threading.local()
 
 
@@ -246,12 +248,12 @@ def create_kv_projection_class(w_in_major: bool = True, weight_grads: bool = Tru
         def forward(ctx, x_vis, w_k, w_v, n_kv_heads, k_norm_weight=None, eps=1e-5):
             ctx.has_norm = k_norm_weight is not None
             ctx.n_kv_heads, ctx.eps = n_kv_heads, eps
-            if ctx.has_norm and getattr(_this_run, "gradient_follows", False):
-                k, v, k_raw, k_rstd = ops.kv_proj(x_vis, w_k, w_v, n_kv_heads, w_in_major, k_norm_weight=k_norm_weight,
-                                                  eps=eps, for_backward=True)
-                ctx.save_for_backward(x_vis, w_k, w_v, k_norm_weight, k_raw, k_rstd)
-                return k, v
             ctx.save_for_backward(x_vis, w_k, w_v, *([k_norm_weight] if ctx.has_norm else []))
+            ctx.kept = None
+            if ctx.has_norm and getattr(_this_run, "gradient_follows", False):
+                k, v, *ctx.kept = ops.kv_proj(x_vis, w_k, w_v, n_kv_heads, w_in_major, k_norm_weight=k_norm_weight,
+                                              eps=eps, for_backward=True)
+                return k, v
             return ops.kv_proj(x_vis, w_k, w_v, n_kv_heads, w_in_major, k_norm_weight=k_norm_weight, eps=eps)
 
         @staticmethod
@@ -264,11 +266,9 @@ def create_kv_projection_class(w_in_major: bool = True, weight_grads: bool = Tru
 
             dk, dv = token_major(dk), token_major(dv)
             if ctx.has_norm:
-                if len(rest) == 3:
-                    k_raw, k_rstd = rest[1:]
-                else:
-                    _, _, k_raw, k_rstd = ops.kv_proj(x_vis, w_k, w_v, ctx.n_kv_heads, w_in_major, k_norm_weight=rest[0],
-                                                      eps=ctx.eps, for_backward=True)
+                kept, ctx.kept = ctx.kept, None
+                k_raw, k_rstd = kept or ops.kv_proj(x_vis, w_k, w_v, ctx.n_kv_heads, w_in_major, k_norm_weight=rest[0],
+                                                    eps=ctx.eps, for_backward=True)[2:]
                 dk, dwn = ops.k_norm_bwd(dk, k_raw, k_rstd, rest[0], want_dw=weight_grads)
                 if dwn is not None:
                     dwn = dwn.to(rest[0].dtype)
@@ -295,17 +295,18 @@ def create_q_projection_class(w_in_major: bool = True, weight_grads: bool = True
         @staticmethod
         def forward(ctx, x, w_q, n_heads, q_norm_weight, eps=1e-5):
             ctx.n_heads, ctx.eps = n_heads, eps
-            if q_norm_weight is not None and getattr(_this_run, "gradient_follows", False):
-                q, q_raw, rstd = ops.q_proj(x, w_q, n_heads, w_in_major, q_norm_weight, eps, for_backward=True)
-                ctx.save_for_backward(x, w_q, q_norm_weight, q_raw, rstd)
-                return q
             ctx.save_for_backward(x, w_q, q_norm_weight)
+            ctx.kept = None
+            if q_norm_weight is not None and getattr(_this_run, "gradient_follows", False):
+                q, *ctx.kept = ops.q_proj(x, w_q, n_heads, w_in_major, q_norm_weight, eps, for_backward=True)
+                return q
             return ops.q_proj(x, w_q, n_heads, w_in_major, q_norm_weight, eps)
 
         @staticmethod
         def backward(ctx, dq):
-            x, w_q, wn, *kept = ctx.saved_tensors
-            q_raw, rstd = kept if kept else ops.q_proj(x, w_q, ctx.n_heads, w_in_major, wn, ctx.eps, for_backward=True)[1:]
+            x, w_q, wn = ctx.saved_tensors
+            kept, ctx.kept = ctx.kept, None
+            q_raw, rstd = kept or ops.q_proj(x, w_q, ctx.n_heads, w_in_major, wn, ctx.eps, for_backward=True)[1:]
             dq_tm = dq if dq.transpose(1, 2).is_contiguous() else dq.transpose(1, 2).contiguous().transpose(1, 2)
             dq_raw, dwn = ops.k_norm_bwd(dq_tm, q_raw, rstd, wn, want_dw=weight_grads)
             dx, dw = ops.q_proj_bwd(x, dq_raw, w_q, w_in_major, want_dw=weight_grads)

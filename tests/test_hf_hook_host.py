@@ -228,3 +228,40 @@ def test_a_projection_without_a_norm_inside_run_function(monkeypatch):
     x = torch.randn(1, 5, 16, requires_grad=True)
     autograd.create_attention_class("lv_xattn").apply(x, run_function, False).sum().backward()
     assert x.grad is not None and w_kv.grad is not None and calls == [False, False]
+
+
+def test_a_checkpointed_projection_inside_run_function(monkeypatch):
+    """A projection that run_function puts under torch.utils.checkpoint saves as many tensors in the attention's
+    backward, where its gradient follows, as in the recomputation that checkpoint makes of it later: checkpoint
+    refuses anything else."""
+    from torch.utils.checkpoint import checkpoint
+    raw = []
+
+    def q_proj(x, w, heads, w_in_major=True, norm=None, eps=1e-5, for_backward=False):
+        q = (x @ w).view(x.shape[0], x.shape[1], heads, -1).transpose(1, 2)
+        raw.append(for_backward)
+        return (q, q.clone(), torch.ones(1)) if for_backward else q
+
+    def kv_proj(x, w_k, w_v, heads, w_in_major=True, k_norm_weight=None, eps=1e-5, for_backward=False):
+        k, v = (q_proj(x, w, heads) for w in (w_k, w_v))
+        return (k, v, k.clone(), torch.ones(1)) if for_backward else (k, v)
+
+    monkeypatch.setattr(ops, "q_proj", q_proj)
+    monkeypatch.setattr(ops, "kv_proj", kv_proj)
+    monkeypatch.setattr(ops, "k_norm_bwd", lambda d, raw, r, w, want_dw: (d, torch.ones_like(w)))
+    monkeypatch.setattr(ops, "q_proj_bwd", lambda x, d, w, *a, **kw: (torch.ones_like(x), torch.ones_like(w)))
+    monkeypatch.setattr(ops, "dx_vis", lambda dk, dv, w_k, *a: torch.ones(1, 5, 16))
+    monkeypatch.setattr(ops, "dw_kv", lambda x, dk, dv, *a: (torch.ones(16, 32), torch.ones(16, 32)))
+    monkeypatch.setattr(autograd, "_attn_forward", lambda q, k, v, *a, **kw: (q, k, v, torch.zeros_like(q), torch.zeros(8, 5)))
+    monkeypatch.setattr(autograd, "_attn_backward", lambda do, q, k, v, *a, **kw: (torch.ones_like(q), torch.ones_like(k), torch.ones_like(v)))
+    project_q, project_kv = autograd.create_q_projection_class().apply, autograd.create_kv_projection_class().apply
+    w_q, w_k, w_v = (torch.randn(16, 8 * 4, requires_grad=True) for _ in range(3))
+    norm = torch.ones(4, requires_grad=True)
+
+    def run_function(x, states):
+        q = checkpoint(project_q, x, w_q, 8, norm, 1e-5, use_reentrant=False)
+        return q, *checkpoint(project_kv, x, w_k, w_v, 8, norm, 1e-5, use_reentrant=False)
+
+    x = torch.randn(1, 5, 16, requires_grad=True)
+    autograd.create_attention_class("lv_xattn").apply(x, run_function, False).sum().backward()
+    assert all(t.grad is not None for t in (x, w_q, w_k, w_v, norm)) and True in raw
