@@ -93,8 +93,8 @@ const char* lvx_strerror(int code);
  * expansion (:271-277, :392-393), which happens in-kernel here.
  * kv_splits > 1 cuts the shard into that many key ranges computed by separate
  * work-groups and folded before return; it needs a workspace of
- * lvx_fwd_workspace_bytes(shape, row_count, kv_splits) bytes.
- * (at most 64 of them; lvx_fwd_auto_splits says how many suit a launch).  The O of a range waits for the
+ * lvx_fwd_workspace_bytes(shape, row_count, kv_splits) bytes
+ * (at most 64 ranges; lvx_fwd_auto_splits says how many suit a launch).  The O of a range waits for the
  * fold in 16 bits, a rounding that a launch of one range does not have (its error against exact arithmetic
  * grows by about a fifth), or with kv_splits = n | LVX_SPLITS_FP32 in fp32, in twice the workspace.
  * The kernel has three forms: a wavefront owns 32 text rows of a head (with a dense bias, and at head_dim

@@ -44,6 +44,11 @@ constexpr int BIG = 0x3fffffff;
 constexpr float RESCALE_LOG2 = 8.f;
 constexpr float LOG2E_F = 1.4426950408889634f, LN2_F = 0.6931471805599453f;
 
+// LSE of a row whose sum of exponentials is not positive: -inf where it saw no key (0).  A NaN among its scores makes the
+// sum NaN; a part of a launch with key splits then says NaN, so that the fold does not take it for a part that saw
+// nothing and give the result without it.
+__device__ __forceinline__ float no_lse(const FwdParams& p, float sum) { return (p.nsplit > 1 ? sum : 0.f) - INFINITY; }
+
 // BIAS: a dense fp32 bias is added to scale * S before the softmax; the scores are
 // then carried in log2 units (S*c + bias*log2e) instead of raw.
 // DH: head dimension, 16, 32, 64 or 128.  The LDS tiles keep their 256-byte rows and chunk
@@ -334,7 +339,7 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
                 *reinterpret_cast<u32x2*>(op + dt * 32 + 8 * vg + 4 * g) = w;
             }
         if (g == 0) {
-            const float lse = l_tot > 0.f ? m_i * (BIAS ? LN2_F : p.scale) + __logf(l_tot) : -INFINITY;
+            const float lse = l_tot > 0.f ? m_i * (BIAS ? LN2_F : p.scale) + __logf(l_tot) : no_lse(p, l_tot);
             p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + h) * p.lse_bh_stride + row] = lse;
         }
     }
@@ -614,7 +619,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
                 }
         }
         if (g == 0 && row0 + r < p.row_end) {
-            const float lse = l_tot > 0.f ? m_i[blk] * p.scale + __logf(l_tot) : -INFINITY;
+            const float lse = l_tot > 0.f ? m_i[blk] * p.scale + __logf(l_tot) : no_lse(p, l_tot);
             p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + h) * p.lse_bh_stride + row0 + r] = lse;
         }
     }
@@ -899,7 +904,7 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     }
     if (part == 0)
         p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + oh) * p.lse_bh_stride + orow] =
-            den > 0.f ? M * p.scale + __logf(den) : -INFINITY;
+            den > 0.f ? M * p.scale + __logf(den) : no_lse(p, den);
 }
 
 }  // namespace

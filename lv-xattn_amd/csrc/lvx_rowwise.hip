@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) out[j] = 0.f;
     // folds the parts (l[k], u[k]) in; a part with weight 0 may hold anything (it saw no key, or nothing
-    // had been folded into the accumulator yet)
+    // had been folded into the accumulator yet), one with weight NaN makes the row NaN
     auto fold = [&](const float (&l)[BATCH], auto&& part) {
         float mn = m;
 #pragma unroll
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
             float f[8];
             part(k, f);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) out[j] = w > 0.f ? fmaf(f[j], w, out[j]) : out[j];
+            for (int j = 0; j < 8; ++j) out[j] = w != 0.f ? fmaf(f[j], w, out[j]) : out[j];
         }
         m = mn;
     };

@@ -146,3 +146,34 @@ def test_a_row_that_sees_nothing_is_zero_whatever_its_q(form, D, dtype, splits, 
     check_o(o, o_ref)
     check_lse(lse, l_ref)
     assert not o.cpu().transpose(1, 2)[dead].any()
+
+
+# A NaN among a row's scores gives a row of NaN, whether its keys are cut into ranges (with the range that holds it
+# in any place) or not; the other rows, and the heads it is not in, stay as they are.
+@pytest.mark.parametrize("form,D,kind", [("1", 128, "none"), ("1", 64, "images"), ("1", 32, "none"), ("1", 128, "bias"),
+                                         ("2", 128, "none"), ("2", 64, "images"), ("2", 16, "none")])
+@pytest.mark.parametrize("splits", [1, 3, 3 | 256, 12, 12 | 256])
+@pytest.mark.parametrize("key", [0, 130, 699])
+def test_a_nan_is_not_lost_between_key_splits(form, D, kind, splits, key, monkeypatch):
+    import lv_xattn
+    monkeypatch.setenv("LVX_FWD_WIDE", form)
+    B, Hq, Hkv, Lq, Lkv = 1, 4, 2, 40, 700
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).bfloat16() for h, n in ((Hq, Lq), (Hkv, Lkv), (Hkv, Lkv)))
+    start, end = torch.zeros(B, Lq, dtype=torch.int32), torch.full((B, Lq), Lkv, dtype=torch.int32)
+    if kind == "images":
+        start[0] = torch.arange(Lq) % 7 * 100
+        end = start + 100
+    bias = torch.randn(B, 1, Lq, Lkv, generator=g)
+    mask = lv_xattn.Mask(None, start, end) if kind == "images" else None
+    bias_args = dict(bias_func=lambda b: b, local_bias_args=[bias.to(DEV)]) if kind == "bias" else {}
+    o_ref, l_ref = orc.attention_dense(q, k, v, D ** -0.5, bias=bias if kind == "bias" else None,
+                                       allowed=orc.interval_mask(start.long(), end.long(), Lkv))
+    k[0, 1, key] = q[0, 0, 7] = float("nan")
+    nan = torch.zeros(B, Hq, Lq, dtype=torch.bool)
+    nan[0, 2:] = (start[0] <= key) & (key < end[0])
+    nan[0, 0, 7] = True
+    o = lv_xattn._attn_forward(q.to(DEV), k.to(DEV), v.to(DEV), False, D ** -0.5, None, rounds=1, batched=True, mask=mask,
+                               kv_splits=splits, **bias_args)[3].cpu()
+    assert torch.equal(o.isnan().all(-1), nan) and torch.equal(o.isnan().any(-1), nan)
+    check_o(o[~nan], o_ref[~nan])
