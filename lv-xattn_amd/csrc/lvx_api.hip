@@ -196,8 +196,9 @@ static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits, bool part
 
 // Whether the parts of a launch whose splits are chosen here wait for the fold in fp32.  In 16 bits they are a
 // rounding that a launch of one range does not have: relative error against 64 bits 2.83e-3 instead of 2.32e-3
-// (bf16, N(0, 1) inputs), whatever the number of parts.  The form for few rows has too little O for fp32 to show
-// (one row x 6404 keys 10.2 us in 16 bits, 10.3 in fp32).  In the others fp32 costs 2 - 7 % of the launch, and cutting
+// (bf16, N(0, 1) inputs), whatever the number of parts.  The form for few rows has little O: fp32 does not show in
+// a decoded token (one row x 6404 keys 10.2 us in 16 bits, 10.3 in fp32) and costs 4 % at 145 (row, head) columns per
+// kv head (four rounds of 145 rows, 3 x 8 heads of 32, 8149 keys: 74.9 us, 77.9).  In the others fp32 costs 2 - 7 % of the launch, and cutting
 // either is what fills the chip - fewer than two work-groups of 32-row waves per CU, ranges of 512 keys and
 // more: 256 rows x 6404 keys 137 us whole, 37.4 in 8 parts, 40.1 with those in fp32 - where they stay in 16
 // bits, or it only evens out the last round of work-groups (2100 rows x 6404 keys 310 us whole, 263 in 2 parts, 270
