@@ -17,13 +17,13 @@ tile that some row of the work-group does not see in full, and the clamp of the 
 the last row of the key range when the next tile to be requested is the last.
 
 Register map (must match the constraints of the asm statement in lvx_fwd.hip), b = row block:
-  at entry: v[128 + 32 b :] Q^T of block b, 4 registers per k-step of 16
+  at entry: v[128 + 2 b : 129 + 2 b] this lane's address in the Q row of block b
   at exit : v[64 b :] O^T of block b, 16 registers per 32 values of d
   inside  : a[64 b :] O^T, a[128 + 32 b :] Q^T
             v[64 b : 64 b + 31] scores set A, v[64 b + 32 : 64 b + 63] scores set B
             v[128 + 16 b : 143 + 16 b] P^T   v[160:199] ten operand slots
   v[200:207] K read addresses (per k-step)   v[208:215] V read addresses (d tile x half)
-  v[216:219] / v[220:223] global byte offsets of this wave's pieces of the next K / V tile
+  v[216:219] / v[220:223] global byte offsets of this wave's pieces of the next K / V tile (at entry: the first)
   v224 what of such an offset is not row * stride   v225+b first visible key - 4 * (lane / 32)
   v227+b visible keys   v229+b m   v231+b l   v233+b alpha   v235+b -m*c   v237+b .. v243+b scratch
   s40 c = scale*log2(e)   s41 -inf   s42 8.0   s[44:45] next K tile   s[46:47] next V tile
@@ -241,6 +241,14 @@ def advance(left, lo, hi, stride, offs, limit):
             f"LVX_FWDW_STAY{n}_%=:"]
 
 
+def request(offs, base, lds):
+    """This wave's pieces of a tile, into the buffer at byte `lds` of the tile buffers."""
+    out = []
+    for j in range(NLD):
+        out += [f"s_add_i32 m0, s50, {lds + j * 4096}", f"global_load_lds_dwordx4 v{offs + j}, {base}"]
+    return out
+
+
 def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
     """One key tile t of the pipelined loop (par = t & 1 relative to the first tile).
     do_cur : P(t) from the current scores, O += V(t)^T P(t)
@@ -416,16 +424,19 @@ def check(ins):
 
 
 def main():
-    # Entry: Q^T moves up into the accumulation registers, O^T starts at 0, no row has a reference.
-    # K and V of the first tile and K of the second have been requested.
-    pro = []
+    # Entry.  What the first scores need is requested first, K(0) and Q^T - Q^T straight into the accumulation
+    # registers it lives in - then V(0) and K(1), which the wait leaves in flight.  O^T starts at 0 meanwhile.
+    pro = request(DOK, "s[44:45]", 0) + advance("s57", "s44", "s45", "s48", DOK, "s64")
+    for b in range(NB):
+        for kk in range(NKK):
+            pro.append(f"global_load_dwordx4 {ar(AQ[b] + 4 * kk, 4)}, {vr(128 + 2 * b, 2)}, off offset:{32 * kk}")
+    pro += request(DOV, "s[46:47]", TILE) + advance("s62", "s46", "s47", "s49", DOV, "s65")
+    pro += request(DOK, "s[44:45]", 2 * TILE) + advance("s57", "s44", "s45", "s48", DOK, "s64")
     for b in range(NB):
         for r in range(16 * NDT):
             pro.append(f"v_accvgpr_write_b32 a{AACC[b] + r}, 0")
-        for r in range(4 * NKK):
-            pro.append(f"v_accvgpr_write_b32 a{AQ[b] + r}, v{128 + 32 * b + r}")
         pro += [f"v_mov_b32 v{MI[b]}, s41", f"v_mov_b32 v{LI[b]}, 0", f"v_mov_b32 v{NMC[b]}, 0"]
-    pro += ["s_waitcnt vmcnt(0)", "s_barrier"]
+    pro += [f"s_waitcnt vmcnt({2 * NLD})", "s_barrier"]
     # scores of the first tile (from K buffer 0 into score set A: the S phase of an odd tile)
     pro += tile(1, do_cur=False, do_next=True, do_dma=False, top=False)
     # there is nothing to rescale yet

@@ -185,6 +185,24 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
     return r;
 }
 
+// Brings every 64-byte line of the kernel's arguments (BYTES of them, at most 512) into the scalar cache with one wait.  The
+// compiler loads an argument where it is needed, and a kernel that comes by five lines one after the other stands
+// still five times for the way to memory, 0.3 us each, before its first load of data leaves.
+template <int BYTES>
+__device__ __forceinline__ void fetch_kernargs() {
+    static_assert(BYTES <= 512, "eight lines");
+    constexpr int LAST = (BYTES - 4) & ~3;
+    constexpr auto at = [](int line) { return line * 64 < LAST ? line * 64 : LAST; };
+    uint32_t r0, r1, r2, r3, r4, r5, r6, r7;
+    asm volatile("s_load_dword %0, %8, %9\n\ts_load_dword %1, %8, %10\n\ts_load_dword %2, %8, %11\n\ts_load_dword %3, %8, %12\n\t"
+                 "s_load_dword %4, %8, %13\n\ts_load_dword %5, %8, %14\n\ts_load_dword %6, %8, %15\n\ts_load_dword %7, %8, %16\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&s"(r0), "=&s"(r1), "=&s"(r2), "=&s"(r3), "=&s"(r4), "=&s"(r5), "=&s"(r6), "=&s"(r7)
+                 : "s"(__builtin_amdgcn_kernarg_segment_ptr()), "n"(at(0)), "n"(at(1)), "n"(at(2)), "n"(at(3)), "n"(at(4)),
+                   "n"(at(5)), "n"(at(6)), "n"(at(7)));
+    __builtin_amdgcn_sched_barrier(0);      // no argument is asked for before
+}
+
 // Work-groups are dealt to the 8 XCDs of an MI355X round-robin by linear id.  Remap so that
 // each XCD receives one contiguous range of the work list: neighbours in the
 // list (which share K/V or Q tiles) then share that XCD's L2.  A placement hint only: every id

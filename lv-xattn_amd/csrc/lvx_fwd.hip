@@ -49,6 +49,9 @@ constexpr float LOG2E_F = 1.4426950408889634f, LN2_F = 0.6931471805599453f;
 // nothing and give the result without it.
 __device__ __forceinline__ float no_lse(const FwdParams& p, float sum) { return (p.nsplit > 1 ? sum : 0.f) - INFINITY; }
 
+// What a row that sees nothing has for Q (see fwd_wide_kernel).
+__device__ const uint16_t zero_row[D] __attribute__((aligned(16))) = {};
+
 // BIAS: a dense fp32 bias is added to scale * S before the softmax; the scores are
 // then carried in log2 units (S*c + bias*log2e) instead of raw.
 // DH: head dimension, 16, 32, 64 or 128.  The LDS tiles keep their 256-byte rows and chunk
@@ -346,8 +349,8 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
 }
 
 // registers the wide loop uses besides its operands (see gen_fwd_loop_wide.py), heads of 128 and of 64
-#define LVX_FWD_WIDE_CLOBBERS_128 "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v233", "v234", "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191"
-#define LVX_FWD_WIDE_CLOBBERS_64 "v32", "v33", "v34", "v35", "v36", "v37", "v38", "v39", "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127", "v144", "v145", "v146", "v147", "v148", "v149", "v150", "v151", "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", "v187", "v188", "v189", "v190", "v191", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v204", "v205", "v206", "v207", "v212", "v213", "v214", "v215", "v218", "v219", "v222", "v223", "v233", "v234", "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175"
+#define LVX_FWD_WIDE_CLOBBERS_128 "v132", "v133", "v134", "v135", "v136", "v137", "v138", "v139", "v140", "v141", "v142", "v143", "v144", "v145", "v146", "v147", "v148", "v149", "v150", "v151", "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v160", "v161", "v162", "v163", "v164", "v165", "v166", "v167", "v168", "v169", "v170", "v171", "v172", "v173", "v174", "v175", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", "v187", "v188", "v189", "v190", "v191", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v233", "v234", "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191"
+#define LVX_FWD_WIDE_CLOBBERS_64 "v32", "v33", "v34", "v35", "v36", "v37", "v38", "v39", "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127", "v132", "v133", "v134", "v135", "v136", "v137", "v138", "v139", "v140", "v141", "v142", "v143", "v144", "v145", "v146", "v147", "v148", "v149", "v150", "v151", "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v160", "v161", "v162", "v163", "v164", "v165", "v166", "v167", "v168", "v169", "v170", "v171", "v172", "v173", "v174", "v175", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", "v187", "v188", "v189", "v190", "v191", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v204", "v205", "v206", "v207", "v212", "v213", "v214", "v215", "v218", "v219", "v222", "v223", "v233", "v234", "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175"
 #define LVX_FWD_WIDE_CLOBBERS_S "memory", "vcc", "scc", "m0", "s52", "s53", "s54", "s55", "s56", "s58", "s59", "s60", "s61", "s70", "s71"
 
 // The wide form (head dimensions 128 and 64, both element types, any mask but a dense bias): a wave
@@ -359,8 +362,11 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
 // Bound by the matrix pipe: 4096 rows x 32 heads x 6404 keys (0.43 TFLOP) takes 354 us, 1215 TFLOP/s,
 // where fwd_kernel takes 429; 2 x 3000 rows with image intervals 332 -> 261; 2 x 1023 rows 202 -> 182;
 // heads of 64, 2048 rows 145 -> 118 (half the MFMAs for the same softmax: bound by the VALU).
-// What a work-group takes besides its tiles is 11 us (one 64-key tile: 12.6): the first loads' latency,
-// the scores of the first tile, which nothing overlaps, and the rows going out.
+// What a work-group takes besides its tiles, which is all that launches of few tiles have to save: the first scores are
+// formed 3.3 us after its first instruction (4.9 when the arguments came line by line, the numbers of the work-group
+// from four integer divisions, and all loads behind 28 address computations with Q^T going through VGPRs), and 2.1 us
+// pass behind the last tile.  One tile: 6.9 us from the first instruction to the last (8.7); sixteen launches of 256 rows
+// x 6404 keys with their folds 661 -> 611, 2 x 300 rows eight times 574 -> 556.
 //
 // LDS tiles: row r of a K or V tile has 2 DH bytes; its 16-byte chunk c sits at position c ^ f(r).
 //   DH = 128: f(r) = ((r & 3) << 2) | ((r >> 2) & 3), as in fwd_kernel
@@ -375,25 +381,26 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     constexpr int NKK = DH / 16, NDT = DH / 32, NLD = DH / 32;
     constexpr int ROWB = 2 * DH, TB = BN * ROWB, CPR = DH / 8;      // bytes per tile row and tile, chunks per row
     constexpr int RPL = 64 / CPR;                                   // tile rows one load of a wave fills
-    __shared__ __attribute__((aligned(1024))) char kv_lds[4 * TB];  // [buffer][K, V]
+    constexpr int EP16 = ROWB + 16, EP32 = 4 * DH + 16;             // row strides of the tile that O leaves through
+    constexpr int EPB = 64 * EP16;                                  // its bytes per wave (32 rows of floats fit too)
+    static_assert(32 * EP32 <= EPB);
+    __shared__ __attribute__((aligned(1024))) char kv_lds[4 * EPB]; // 4 TB: [buffer][K, V]; then O
     __shared__ int red[4][4];
 
+    fetch_kernargs<sizeof(FwdParams)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
     if (wid >= p.total_wg) return;
-    const int tile = wid % p.n_row_tiles;
-    const int t1 = wid / p.n_row_tiles;
-    const int split = t1 % p.nsplit;
-    const int t2 = t1 / p.nsplit;
+    uint32_t tile, split, b;
+    const uint32_t t1 = p.by_row_tiles.split(wid, tile), t2 = p.by_splits.split(t1, split);
     // samples vary faster than head groups: every XCD (a contiguous range of ids) then gets
     // work-groups of all samples, and ragged samples do not leave some XCDs idle early
-    const int b = t2 % p.B;
-    const int hg = t2 / p.B;
+    const uint32_t hg = p.by_B.split(t2, b);
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
-    const int h = hg * p.HG + (wave % p.HG);
-    const int hk = h / p.G;
-    const int row0 = p.row_begin + (tile * p.RS + wave / p.HG) * 64;       // this wave's first row
+    const int h = hg * p.HG + (wave & (p.HG - 1));       // HG is 1, 2 or 4, and RS = 4 / HG
+    const int hk = p.by_head_groups.quotient(hg);
+    const int row0 = p.row_begin + (tile * p.RS + (wave >> (p.HG >> 1))) * 64;      // this wave's first row
 
     int kv_len = p.Lkv;
     if (p.kv_len) kv_len = min(p.kv_len[b], p.Lkv);
@@ -465,32 +472,21 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
         const uint32_t ld_c = (uint32_t)((lane % CPR) ^ (DH == 128 ? (((lane >> 4) << 2) | wave)
                                                                    : ((((lane >> 4) & 1) << 2) | ((2 * wave + (lane >> 5)) & 3)))) * 16u;
         const int last = hi - 1 - (kv0 + (n - 1) * BN);      // last row of the key range in the last tile
-        auto piece_off = [&](int t, int j, uint32_t rowb) {
+        auto piece_off = [&](int j, uint32_t rowb) {         // in the first tile, which may be the last
             const int r = ld_r + 4 * RPL * j;
-            return (uint32_t)(t == n - 1 ? min(r, last) : r) * rowb + ld_c;
+            return (uint32_t)(n == 1 ? min(r, last) : r) * rowb + ld_c;
         };
-        const int tk1 = min(1, n - 1), tk2 = min(2, n - 1);
-#pragma unroll
-        for (int j = 0; j < NLD; ++j) dma16(kp, piece_off(0, j, krow_b), lds_w + j * 4096);
-#pragma unroll
-        for (int j = 0; j < NLD; ++j) dma16(vp, piece_off(0, j, vrow_b), lds_w + TB + j * 4096);
-        kp += (int64_t)tk1 * BN * krow_b;
-#pragma unroll
-        for (int j = 0; j < NLD; ++j) dma16(kp, piece_off(tk1, j, krow_b), lds_w + 2 * TB + j * 4096);
-        kp += (int64_t)(tk2 - tk1) * BN * krow_b;
-        vp += (int64_t)tk1 * BN * vrow_b;
         uint32_t dok[NLD], dov[NLD];
 #pragma unroll
-        for (int j = 0; j < NLD; ++j) { dok[j] = piece_off(tk2, j, krow_b); dov[j] = piece_off(tk1, j, vrow_b); }
+        for (int j = 0; j < NLD; ++j) { dok[j] = piece_off(j, krow_b); dov[j] = piece_off(j, vrow_b); }
 
-        // Q^T as B operand; its loads travel with the first tiles'
-        bf16x8 q[2][NKK];
+        // Q^T as B operand: this lane's 16 bytes of each k-step, of its row in either block
+        const char* qa[2];
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
-            const int row = row0 + 32 * blk + l32;
-            const uint16_t* qp = p.q + b * p.qs.b + h * p.qs.h + (int64_t)row * p.qs.s + g * 8;
-#pragma unroll
-            for (int kk = 0; kk < NKK; ++kk) q[blk][kk] = as_bf16x8(ldg16(qp + kk * 16, row < p.row_end && !empty[blk]));
+            const int row = min(row0 + 32 * blk + l32, p.row_end - 1);      // rows past the window repeat the last
+            qa[blk] = reinterpret_cast<const char*>(p.q + b * p.qs.b + h * p.qs.h + (int64_t)row * p.qs.s + g * 8);
+            if (MASKED && empty[blk]) qa[blk] = reinterpret_cast<const char*>(zero_row + g * 8);
         }
 
         // LDS -> operands.  K rows (A of S^T): chunk 2 kk + g of row l32 (+ 32).  V^T (A of O^T += V^T P^T),
@@ -517,10 +513,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
         const bool inner_any = in_hi - in_lo >= BN;
         const int inner = inner_any ? in_lo : BIG;
         const uint32_t inner_n = inner_any ? (uint32_t)(in_hi - BN - in_lo) : 0u;
-        uint32_t left = uniform32((uint32_t)(n - 1)), left_k = uniform32((uint32_t)(n - 1 - tk2));
-        uint32_t left_v = uniform32((uint32_t)(n - 1 - tk1)), kv = uniform32((uint32_t)kv0);
-        kp = uniform_ptr(kp);
-        vp = uniform_ptr(vp);
+        uint32_t left = uniform32((uint32_t)(n - 1)), left_k = left, left_v = left, kv = uniform32((uint32_t)kv0);
 #define LVX_FWD_WIDE_SCALARS                                                                                       \
     "{s40}"(uniform32(p.scale_log2e)), "{s41}"(-INFINITY), "{s42}"(RESCALE_LOG2), "{s48}"(uniform32((uint32_t)BN * krow_b)), \
         "{s49}"(uniform32((uint32_t)BN * vrow_b)), "{s50}"(uniform32(lds_w)), "{s64}"(uniform32((uint32_t)last * krow_b)),   \
@@ -532,11 +525,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
 #define LVX_FWD_WIDE_OUT_128                                                                                       \
           "=&{v[0:15]}"(acc[0][0]), "=&{v[16:31]}"(acc[0][1]), "=&{v[32:47]}"(acc[0][2]), "=&{v[48:63]}"(acc[0][3]),   \
           "=&{v[64:79]}"(acc[1][0]), "=&{v[80:95]}"(acc[1][1]), "=&{v[96:111]}"(acc[1][2]), "=&{v[112:127]}"(acc[1][3]), \
-          "+{v[128:131]}"(q[0][0]), "+{v[132:135]}"(q[0][1]), "+{v[136:139]}"(q[0][2]), "+{v[140:143]}"(q[0][3]),      \
-          "+{v[144:147]}"(q[0][4]), "+{v[148:151]}"(q[0][5]), "+{v[152:155]}"(q[0][6]), "+{v[156:159]}"(q[0][7]),      \
-          "+{v[160:163]}"(q[1][0]), "+{v[164:167]}"(q[1][1]), "+{v[168:171]}"(q[1][2]), "+{v[172:175]}"(q[1][3]),      \
-          "+{v[176:179]}"(q[1][4]), "+{v[180:183]}"(q[1][5]), "+{v[184:187]}"(q[1][6]), "+{v[188:191]}"(q[1][7]),      \
-          "+{v216}"(dok[0]), "+{v217}"(dok[1]), "+{v218}"(dok[2]), "+{v219}"(dok[3]),                              \
+          "+{v[128:129]}"(qa[0]), "+{v[130:131]}"(qa[1]), "+{v216}"(dok[0]), "+{v217}"(dok[1]), "+{v218}"(dok[2]), "+{v219}"(dok[3]),                              \
           "+{v220}"(dov[0]), "+{v221}"(dov[1]), "+{v222}"(dov[2]), "+{v223}"(dov[3]), LVX_FWD_WIDE_STATE
 #define LVX_FWD_WIDE_IN_128                                                                                        \
           "{v200}"(ka[0]), "{v201}"(ka[1]), "{v202}"(ka[2]), "{v203}"(ka[3]), "{v204}"(ka[4]), "{v205}"(ka[5]),    \
@@ -544,9 +533,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
           "{v212}"(va[4]), "{v213}"(va[5]), "{v214}"(va[6]), "{v215}"(va[7]), LVX_FWD_WIDE_SCALARS
 #define LVX_FWD_WIDE_OUT_64                                                                                        \
           "=&{v[0:15]}"(acc[0][0]), "=&{v[16:31]}"(acc[0][1]), "=&{v[64:79]}"(acc[1][0]), "=&{v[80:95]}"(acc[1][1]),   \
-          "+{v[128:131]}"(q[0][0]), "+{v[132:135]}"(q[0][1]), "+{v[136:139]}"(q[0][2]), "+{v[140:143]}"(q[0][3]),      \
-          "+{v[160:163]}"(q[1][0]), "+{v[164:167]}"(q[1][1]), "+{v[168:171]}"(q[1][2]), "+{v[172:175]}"(q[1][3]),      \
-          "+{v216}"(dok[0]), "+{v217}"(dok[1]), "+{v220}"(dov[0]), "+{v221}"(dov[1]), LVX_FWD_WIDE_STATE
+          "+{v[128:129]}"(qa[0]), "+{v[130:131]}"(qa[1]), "+{v216}"(dok[0]), "+{v217}"(dok[1]), "+{v220}"(dov[0]), "+{v221}"(dov[1]), LVX_FWD_WIDE_STATE
 #define LVX_FWD_WIDE_IN_64                                                                                         \
           "{v200}"(ka[0]), "{v201}"(ka[1]), "{v202}"(ka[2]), "{v203}"(ka[3]),                                      \
           "{v208}"(va[0]), "{v209}"(va[1]), "{v210}"(va[2]), "{v211}"(va[3]), LVX_FWD_WIDE_SCALARS
@@ -576,62 +563,90 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
                 for (int v = 0; v < 16; ++v) acc[blk][dt][v] = 0.f;
     }
 
-    // Epilogue.  A lane holds 4 consecutive values of d of one row per register group; the rows of a
-    // wave go through its quarter of the tile buffers and leave as whole rows, 16 bytes per lane.
-    // Chunk c of row r sits at position c ^ (r mod chunks per row) (DH = 64: c ^ (r / 2 mod 8)), its
-    // 8-byte halves exchanged in rows with bit 4 set: conflict-free both ways.
-    // Parts in fp32 go one block of 32 rows at a time, chunk c of row r at position c ^ (r mod chunks per row).
+    // Epilogue.  A lane holds 4 consecutive values of d of one row per register group; the rows of a wave go through
+    // its quarter of the tile buffers and leave as whole rows, 16 bytes per lane.  Rows are 16 bytes longer there
+    // than their values, which spreads sixteen of them over the banks and leaves every address a constant away from one
+    // register; of rows 16 apart one has the 8-byte halves of its chunks exchanged.  All reads are
+    // issued before the first store.  From the last tile to the end 2.1 us; 3.0 with the chunks permuted by XOR, read one by
+    // one and stored behind a 64-bit product per row.
+    // Parts in fp32 go one block of 32 rows at a time.
     __syncthreads();     // every wave is done with the tiles
-    char* const ep = kv_lds + wave * TB;
-    const int64_t o_head = split * p.o_split_stride + b * p.os.b + h * p.os.h;
+    char* const ep = kv_lds + wave * EPB;
+    const int64_t o_head = split * p.o_split_stride + b * p.os.b + h * p.os.h + row0 * p.os.s;
+    const int rows = p.row_end - row0;                           // of this wave, where fewer than 64
+    float l_tot[2], inv[2];
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
-        float l_tot = l_i[blk] + __shfl_xor(l_i[blk], 32);     // the two lane halves hold partial sums of the same row
-        if (empty[blk]) l_tot = 0.f;
-        const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-        const int r = 32 * blk + l32, pos = DH == 128 ? (r & 15) : ((r >> 1) & 7);
-        if (p.o_f32) {
-            constexpr int CPF = DH / 4;                          // chunks of a row of floats
+        l_tot[blk] = l_i[blk] + __shfl_xor(l_i[blk], 32);       // the two lane halves hold partial sums of the same row
+        if (empty[blk]) l_tot[blk] = 0.f;
+        inv[blk] = l_tot[blk] > 0.f ? 1.f / l_tot[blk] : 0.f;
+    }
+    if (p.o_f32) {
+        constexpr int CPF = DH / 4, RPS = 64 / CPF;              // chunks of a row of floats, rows per store
+        float* const ob = reinterpret_cast<float*>(p.o) + o_head;
+        const uint32_t oo = (uint32_t)(lane / CPF) * (uint32_t)p.os.s + (uint32_t)(lane % CPF) * 4u;
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
                 for (int vg = 0; vg < 4; ++vg) {
-                    const f32x4 x = {acc[blk][dt][4 * vg] * inv, acc[blk][dt][4 * vg + 1] * inv, acc[blk][dt][4 * vg + 2] * inv, acc[blk][dt][4 * vg + 3] * inv};
-                    *reinterpret_cast<f32x4*>(ep + l32 * (4 * DH) + (((8 * dt + 2 * vg + g) ^ (l32 & (CPF - 1))) << 4)) = x;
+                    const f32x4 x = {acc[blk][dt][4 * vg] * inv[blk], acc[blk][dt][4 * vg + 1] * inv[blk],
+                                     acc[blk][dt][4 * vg + 2] * inv[blk], acc[blk][dt][4 * vg + 3] * inv[blk]};
+                    *reinterpret_cast<f32x4*>(ep + l32 * EP32 + g * 16 + (8 * dt + 2 * vg) * 16) = x;
                 }
             wait_lds();
+            f32x4 x[32 / RPS];
 #pragma unroll
-            for (int i = 0; i < CPF / 2; ++i) {
-                const int rf = i * (64 / CPF) + lane / CPF, c = lane % CPF, row = row0 + 32 * blk + rf;
-                const f32x4 x = *reinterpret_cast<const f32x4*>(ep + rf * (4 * DH) + ((c ^ (rf & (CPF - 1))) << 4));
-                if (row < p.row_end) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.o) + o_head + (int64_t)row * p.os.s + c * 4) = x;
-            }
+            for (int i = 0; i < 32 / RPS; ++i)
+                x[i] = *reinterpret_cast<const f32x4*>(ep + (lane / CPF) * EP32 + (lane % CPF) * 16 + i * (RPS * EP32));
+            auto store = [&](bool all) {
+#pragma unroll
+                for (int i = 0; i < 32 / RPS; ++i) {
+                    const int r = 32 * blk + i * RPS;
+                    if (all || r + lane / CPF < rows) *reinterpret_cast<f32x4*>(ob + r * p.os.s + oo) = x[i];
+                }
+            };
+            if (rows >= 64) store(true);
+            else store(false);
             wait_lds();          // read before the next block takes its place
-        } else {
+        }
+    } else {
+        char* const wr = ep + l32 * EP16 + ((g ^ (l32 >> 4)) << 3);
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
                 for (int vg = 0; vg < 4; ++vg) {
-                    u32x2 w;
-                    w[0] = E::pack(acc[blk][dt][4 * vg] * inv, acc[blk][dt][4 * vg + 1] * inv);
-                    w[1] = E::pack(acc[blk][dt][4 * vg + 2] * inv, acc[blk][dt][4 * vg + 3] * inv);
-                    *reinterpret_cast<u32x2*>(ep + r * ROWB + (((4 * dt + vg) ^ pos) << 4) + ((g ^ ((r >> 4) & 1)) << 3)) = w;
+                    u32x2 u;
+                    u[0] = E::pack(acc[blk][dt][4 * vg] * inv[blk], acc[blk][dt][4 * vg + 1] * inv[blk]);
+                    u[1] = E::pack(acc[blk][dt][4 * vg + 2] * inv[blk], acc[blk][dt][4 * vg + 3] * inv[blk]);
+                    *reinterpret_cast<u32x2*>(wr + blk * (32 * EP16) + (4 * dt + vg) * 16) = u;
                 }
-        }
-        if (g == 0 && row0 + r < p.row_end) {
-            const float lse = l_tot > 0.f ? m_i[blk] * p.scale + __logf(l_tot) : no_lse(p, l_tot);
+        wait_lds();          // this wave's rows are its own
+        u32x4 x[CPR];
+#pragma unroll
+        for (int i = 0; i < CPR; ++i) x[i] = *reinterpret_cast<const u32x4*>(ep + (lane / CPR) * EP16 + (lane % CPR) * 16 + i * (RPL * EP16));
+        uint16_t* const ob = p.o + o_head;
+        const uint32_t oo = (uint32_t)(lane / CPR) * (uint32_t)p.os.s + (uint32_t)(lane % CPR) * 8u;
+        auto store = [&](bool all) {
+#pragma unroll
+            for (int i = 0; i < CPR; ++i) {
+                const u32x4 y = (i * RPL >> 4) & 1 ? u32x4{x[i][2], x[i][3], x[i][0], x[i][1]} : x[i];
+                if (all || i * RPL + lane / CPR < rows) *reinterpret_cast<u32x4*>(ob + i * RPL * p.os.s + oo) = y;
+            }
+        };
+        if (rows >= 64) store(true);
+        else store(false);
+    }
+#pragma unroll
+    for (int blk = 0; blk < 2; ++blk) {
+        const int r = 32 * blk + l32;
+        if (g == 0 && r < rows) {
+            const float lse = l_tot[blk] > 0.f ? m_i[blk] * p.scale + __logf(l_tot[blk]) : no_lse(p, l_tot[blk]);
             p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + h) * p.lse_bh_stride + row0 + r] = lse;
         }
-    }
-    if (p.o_f32) return;
-    wait_lds();          // this wave's rows are its own
-    uint16_t* const ob = p.o + o_head;
-#pragma unroll
-    for (int i = 0; i < CPR; ++i) {
-        const int r = i * RPL + lane / CPR, c = lane % CPR, pos = DH == 128 ? (r & 15) : ((r >> 1) & 7);
-        u32x4 val = *reinterpret_cast<const u32x4*>(ep + r * ROWB + ((c ^ pos) << 4));
-        if ((r >> 4) & 1) val = u32x4{val[2], val[3], val[0], val[1]};
-        if (row0 + r < p.row_end) *reinterpret_cast<u32x4*>(ob + (int64_t)(row0 + r) * p.os.s + c * 8) = val;
     }
 }
 
@@ -936,7 +951,13 @@ hipError_t launch_fwd_t(const FwdParams& p, bool masked, hipStream_t st) {
 }
 }  // namespace
 
-hipError_t launch_fwd(const FwdParams& p, bool masked, hipStream_t st) {
+hipError_t launch_fwd(const FwdParams& params, bool masked, hipStream_t st) {
+    FwdParams p = params;
+    p.by_row_tiles = divisor(p.n_row_tiles);
+    p.by_splits = divisor(p.nsplit);
+    p.by_B = divisor(p.B);
+    p.by_G = divisor(p.G);
+    p.by_head_groups = divisor(p.G / p.HG);
     switch (p.D) {
         case 16: return p.f16 ? launch_fwd_t<16, true>(p, masked, st) : launch_fwd_t<16, false>(p, masked, st);
         case 32: return p.f16 ? launch_fwd_t<32, true>(p, masked, st) : launch_fwd_t<32, false>(p, masked, st);

@@ -26,6 +26,20 @@ struct Strides3 {
 // SIMD (head dimensions 128 and 64), or a share of the keys for up to 32 (row, head) pairs at once.
 enum FwdForm { FWD_PLAIN = 0, FWD_WIDE = 1, FWD_FEW = 2 };
 
+// Division of work-group numbers by something the host knows: a product and a correction instead of the forty
+// instructions of an integer division.  floor((2^32 - 1) / d) times x / 2^32 is x / d or one less.
+struct Divisor {
+    uint32_t d, m;
+    __host__ __device__ uint32_t split(uint32_t x, uint32_t& rest) const {
+        uint32_t q = (uint32_t)((uint64_t)x * m >> 32);
+        rest = x - q * d;
+        if (rest >= d) { ++q; rest -= d; }
+        return q;
+    }
+    __host__ __device__ uint32_t quotient(uint32_t x) const { uint32_t rest; return split(x, rest); }
+};
+inline Divisor divisor(int d) { return Divisor{(uint32_t)d, 0xffffffffu / (uint32_t)d}; }
+
 struct FwdParams {
     const uint16_t* q;
     const uint16_t* k;
@@ -52,6 +66,8 @@ struct FwdParams {
     float scale, scale_log2e;
     int f16;                   // element type of q, k, v, o: 0 bf16, 1 fp16
     int o_f32;                 // 1: o (the parts of a launch with key splits) is fp32
+    // filled in by launch_fwd: divisors by n_row_tiles, nsplit, B, G and G / HG
+    Divisor by_row_tiles, by_splits, by_B, by_G, by_head_groups;
 };
 
 struct MergeParams {
