@@ -660,8 +660,8 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
 // are requested before anything else happens: 128 KiB in flight per CU, and with ranges of 256 keys
 // or less every byte the work-group will read.  Bound by HBM where there is enough to read: 4 rows x 32
 // heads x 76848 keys (315 MB) take 61 us, 5.2 TB/s, the rate of a large copy, against 75 us in the
-// wide form; one row x 6404 keys (26 MB) 12.4 us with the fold of the parts against 17.4, most of
-// it latency.
+// wide form; one row x 6404 keys (26 MB) 12.0 us with the fold of the parts against 17.4, most of
+// it latency (the kernel alone 6.1 us; 6.7 with the arguments fetched line by line and integer divisions for where it is).
 //   S^T[32 keys, 32 cols] = K (A, 16-byte LDS reads) x Q^T (B, registers)
 //   O^T[d, 32 cols]      += V^T (A, transposing LDS reads) x P^T (B, straight from S^T)
 // LDS rows are 2 DH bytes (128 below head dimension 64, the lanes past the head dimension repeat a
@@ -678,20 +678,18 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[RING > FOLD ? RING : FOLD];
     __shared__ float ml[4][2][32];                                  // per wave and column: reference maximum, row sum
 
+    fetch_kernargs<sizeof(FwdParams)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
     if (wid >= p.total_wg) return;
-    const int ct = wid % p.n_row_tiles;            // column tile
-    const int t1 = wid / p.n_row_tiles;
-    const int split = t1 % p.nsplit;
-    const int t2 = t1 / p.nsplit;
-    const int b = t2 % p.B;
-    const int hk = t2 / p.B;
+    uint32_t ct, split, b;                         // column tile, key range, sample
+    const uint32_t t1 = p.by_row_tiles.split(wid, ct), t2 = p.by_splits.split(t1, split), hk = p.by_B.split(t2, b);
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int n_cols = p.G * (p.row_end - p.row_begin);
-    const int col = min(ct * 32 + l32, n_cols - 1);                 // columns past the last repeat it and are not stored
-    const int row = p.row_begin + col / p.G, h = hk * p.G + col % p.G;
+    const int col = min((int)ct * 32 + l32, n_cols - 1);            // columns past the last repeat it and are not stored
+    uint32_t head;
+    const int row = p.row_begin + p.by_G.split(col, head), h = hk * p.G + head;
 
     u32x4 q[NKK];
     {
@@ -877,8 +875,8 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     __syncthreads();
     constexpr int TPC = 8, DPT = DH / TPC;          // threads per column, values of d per thread
     const int oc = tid / TPC, part = tid % TPC;
-    if (ct * 32 + oc >= n_cols) return;
-    const int orow = p.row_begin + (ct * 32 + oc) / p.G, oh = hk * p.G + (ct * 32 + oc) % p.G;
+    if ((int)ct * 32 + oc >= n_cols) return;
+    const int orow = p.row_begin + p.by_G.split(ct * 32 + oc, head), oh = hk * p.G + head;
     float M = -INFINITY, w[4], den = 0.f;
 #pragma unroll
     for (int k = 0; k < 4; ++k) M = fmaxf(M, ml[k][0][oc]);

@@ -91,6 +91,7 @@ struct MergeParams {
     int f16;
     int D;                     // head dimension: 16, 32, 64 or 128 (0 reads as 128)
     int part_f32;              // 1: the parts are fp32 (not for one part folded into an accumulator)
+    Divisor by_rows, by_Hq;    // filled in by launch_merge: rows of the window, q heads
 };
 
 // Per text row the hull of the keys a dense bias leaves visible (entries other than -inf).
@@ -100,6 +101,7 @@ struct BiasHullParams {
     int32_t* kv_start;         // [B, Lq]: written by the hull kernel, read by the interval test
     int32_t* kv_end;           // [B, Lq]
     int B, heads, Lq, Lkv;     // heads: 1 (bias broadcast over heads) or Hq
+    Divisor by_Lq;             // filled in by the launchers
     int32_t* flag;             // interval test only: set to 1 when the bias is not 0 everywhere inside the hull
 };
 // Per text row of an additive mask [B][Lq][Lkv] (type: LVX_BF16, LVX_F16 or 0 for fp32; element strides
@@ -111,6 +113,7 @@ struct MaskIntervalParams {
     int32_t* kv_start;         // [B, Lq]; -1 for a row that is more than an interval
     int32_t* kv_end;           // [B, Lq]
     int B, Lq, Lkv;
+    Divisor by_Lq;             // filled in by launch_mask_intervals
 };
 hipError_t launch_mask_intervals(const MaskIntervalParams& p, hipStream_t st);
 hipError_t launch_bias_hull(const BiasHullParams& p, hipStream_t st);
@@ -124,6 +127,7 @@ struct PreParams {
     int B, Hq, Lq, row_begin, row_end;
     int f16;
     int D;                     // head dimension: 16, 32, 64 or 128 (0 reads as 128)
+    Divisor by_rows, by_Hq;    // filled in by launch_preprocess
 };
 
 struct BwdParams {
@@ -202,6 +206,7 @@ struct MetaParams {
     float* scratch;            // null, or the fp32 dK / dV scratch whose shared token blocks the same launch zeroes
     SharedBlocks sb;
     int meta_blocks;           // filled by the launcher: blocks [0, meta_blocks) write records
+    Divisor by_rows;           // and the divisor by the rows of the window's whole tiles
 };
 
 // The shared token blocks of the scratch, rounded into dK and dV.
@@ -224,6 +229,7 @@ struct CastParams {
     int64_t sum_stride;   // sum_stride floats apart
     int f16;          // destination type: 0 bf16, 1 fp16
     int D;            // head dimension: 16, 32, 64 or 128 (0 reads as 128)
+    Divisor by_L, by_H;    // filled in by launch_cast
 };
 
 // One GEMM problem C[M,N] = sum over segments A_s[M,K_s] * B_s[K_s,N].

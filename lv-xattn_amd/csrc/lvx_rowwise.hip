@@ -19,6 +19,19 @@ __device__ __forceinline__ int chunk_shift(int head_dim) {
     return head_dim == 64 ? 3 : head_dim == 32 ? 2 : head_dim == 16 ? 1 : 4;
 }
 
+// Where the r-th of the rows of all (b, h) is.  Rows are counted in 32 bits: 2^32 of them, 32 bytes each at the least, are
+// not in the card's memory twice.
+struct RowOf {
+    int row, bh, b, h;
+    __device__ __forceinline__ RowOf(uint32_t r, const Divisor& by_rows, const Divisor& by_H) {
+        uint32_t x, y;
+        bh = (int)by_rows.split(r, x);
+        b = (int)by_H.split((uint32_t)bh, y);
+        row = (int)x;
+        h = (int)y;
+    }
+};
+
 template <class E>
 __device__ __forceinline__ void unpack8(u32x4 u, float f[8]) {
 #pragma unroll
@@ -37,6 +50,7 @@ template <bool F16, int PL, bool PART32>
 __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     using E = Elt<F16>;
     constexpr int PSH = PL == 4 ? 2 : PL == 2 ? 1 : 0, BATCH = 4;
+    fetch_kernargs<sizeof(MergeParams)>();
     const int nrows = p.row_end - p.row_begin;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int sh = chunk_shift(p.D);
@@ -44,9 +58,8 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     const int pl = (int)(idx >> sh) & (PL - 1);
     const int64_t r = idx >> (sh + PSH);
     if (r >= (int64_t)p.B * p.Hq * nrows) return;      // the lanes of a row leave together
-    const int row = p.row_begin + (int)(r % nrows);
-    const int bh = (int)(r / nrows);
-    const int b = bh / p.Hq, h = bh % p.Hq;
+    const RowOf at_row((uint32_t)r, p.by_rows, p.by_Hq);
+    const int row = p.row_begin + at_row.row, bh = at_row.bh, b = at_row.b, h = at_row.h;
 
     float m = -INFINITY, den = 0.f, out[8];
 #pragma unroll
@@ -139,6 +152,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
 template <bool F16>
 __global__ __launch_bounds__(256) void merge_pair_kernel(const MergeParams p) {
     using E = Elt<F16>;
+    fetch_kernargs<sizeof(MergeParams)>();
     const int nrows = p.row_end - p.row_begin;
     const int64_t total = (int64_t)p.B * p.Hq * nrows;
     const int64_t half = (total + 1) / 2;
@@ -157,9 +171,8 @@ __global__ __launch_bounds__(256) void merge_pair_kernel(const MergeParams p) {
     u32x4 ua[2], ub[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        const int row = p.row_begin + (int)(rr[k] % nrows);
-        const int bh = (int)(rr[k] / nrows);
-        const int b = bh / p.Hq, h = bh % p.Hq;
+        const RowOf at_row((uint32_t)rr[k], p.by_rows, p.by_Hq);
+        const int row = p.row_begin + at_row.row, bh = at_row.bh, b = at_row.b, h = at_row.h;
         oa[k] = p.o_acc + b * p.oa.b + h * p.oa.h + (int64_t)row * p.oa.s + chunk * 8;
         op[k] = p.o_part + b * p.op.b + h * p.op.h + (int64_t)row * p.op.s + chunk * 8;
         la_p[k] = p.l_acc + (int64_t)bh * p.l_acc_bh + row;
@@ -198,6 +211,7 @@ __global__ __launch_bounds__(256) void merge_pair_kernel(const MergeParams p) {
 template <bool F16>
 __global__ __launch_bounds__(256) void preprocess_kernel(const PreParams p) {
     using E = Elt<F16>;
+    fetch_kernargs<sizeof(PreParams)>();
     const int nrows = p.row_end - p.row_begin;
     const int64_t total = (int64_t)p.B * p.Hq * nrows;
     const int64_t half = (total + 1) / 2;
@@ -212,9 +226,8 @@ __global__ __launch_bounds__(256) void preprocess_kernel(const PreParams p) {
     float* out[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        const int row = p.row_begin + (int)(rr[k] % nrows);
-        const int bh = (int)(rr[k] / nrows);
-        const int b = bh / p.Hq, h = bh % p.Hq;
+        const RowOf at_row((uint32_t)rr[k], p.by_rows, p.by_Hq);
+        const int row = p.row_begin + at_row.row, bh = at_row.bh, b = at_row.b, h = at_row.h;
         const bool ok = k ? ok1 : ok0;
         uo[k] = ldg16(p.o + b * p.os.b + h * p.os.h + (int64_t)row * p.os.s + chunk * 8, ok);
         ud[k] = ldg16(p.dout + b * p.ds.b + h * p.ds.h + (int64_t)row * p.ds.s + chunk * 8, ok);
@@ -251,6 +264,7 @@ __device__ __forceinline__ int shared_block(const SharedBlocks& s, int i) {
 // window (so that P = exp2(x - inf) = 0 there), and delta * scale (0 past the
 // window), grouped per 32-row tile so that one 256-byte load fetches a tile's lot.
 __global__ __launch_bounds__(256) void bwd_meta_kernel(const MetaParams p) {
+    fetch_kernargs<sizeof(MetaParams)>();
     // the other blocks of the launch zero the scratches (stores rather than hipMemsetAsync, so
     // that callers may capture the stream)
     if ((int)blockIdx.x >= p.meta_blocks) {
@@ -272,8 +286,8 @@ __global__ __launch_bounds__(256) void bwd_meta_kernel(const MetaParams p) {
     const int rows_pad = p.n_tiles * 32;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (int64_t)p.B * p.Hq * rows_pad) return;
-    const int r = (int)(idx % rows_pad);
-    const int64_t bh = idx / rows_pad;
+    uint32_t r;
+    const int64_t bh = p.by_rows.split((uint32_t)idx, r);
     const int row = p.row_begin + r;
     const bool ok = row < p.row_end;
     const float l = ok ? p.lse[bh * p.Lq + row] : -INFINITY;
@@ -283,31 +297,50 @@ __global__ __launch_bounds__(256) void bwd_meta_kernel(const MetaParams p) {
     o[32] = d * p.scale;
 }
 
-// One wave per (b, text row): first and one-past-last key whose bias is not -inf, over all heads
-// the bias distinguishes.  An empty row gets (0, 0).
-__global__ __launch_bounds__(256) void bias_hull_kernel(const BiasHullParams p) {
-    const int64_t rw = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (rw >= (int64_t)p.B * p.Lq) return;
-    const int b = (int)(rw / p.Lq), row = (int)(rw % p.Lq);
-    int lo = INT_MAX, hi = 0;
-    for (int h = 0; h < p.heads; ++h) {
-        const float* br = p.bias + b * p.bias_b + h * p.bias_h + (int64_t)row * p.bias_r;
-        for (int k0 = 4 * lane; k0 < p.Lkv; k0 += 256) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(br + k0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (k0 + j < p.Lkv && !(v[j] == -INFINITY)) { lo = min(lo, k0 + j); hi = max(hi, k0 + j + 1); }
-        }
-    }
+// First and one-past-last key of a set that the threads of a work-group of 256 have each seen a part of.
+__device__ __forceinline__ void block_hull(int& lo, int& hi) {
+    __shared__ int red[4][2];
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         lo = min(lo, __shfl_xor(lo, o));
         hi = max(hi, __shfl_xor(hi, o));
     }
-    if (lane == 0) {
-        p.kv_start[rw] = hi > 0 ? lo : 0;
-        p.kv_end[rw] = hi;
+    if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6][0] = lo; red[threadIdx.x >> 6][1] = hi; }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 4; ++w) { lo = min(lo, red[w][0]); hi = max(hi, red[w][1]); }
+}
+
+// One work-group per (b, text row): first and one-past-last key whose bias is not -inf, over all heads the bias
+// distinguishes.  An empty row gets (0, 0).  Bound by reading the bias once: four loads of 16 bytes per thread in flight
+// (1024 rows x 4096 keys, 16.8 MB: 5.0 us; one wave per row, a load at a time, 8.7).
+__global__ __launch_bounds__(256) void bias_hull_kernel(const BiasHullParams p) {
+    fetch_kernargs<sizeof(BiasHullParams)>();
+    for (uint32_t rw = blockIdx.x; rw < (uint32_t)(p.B * p.Lq); rw += gridDim.x) {
+        uint32_t row;
+        const uint32_t b = p.by_Lq.split(rw, row);
+        int lo = INT_MAX, hi = 0;
+        for (int h = 0; h < p.heads; ++h) {
+            const float* br = p.bias + b * p.bias_b + h * p.bias_h + (int64_t)row * p.bias_r;
+            for (int k0 = 4 * (int)threadIdx.x; k0 < p.Lkv; k0 += 4 * 1024) {
+                f32x4 v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const f32x4*>(br + min(k0 + i * 1024, (p.Lkv - 1) & ~3));
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int key = k0 + i * 1024 + j;
+                        if (key < p.Lkv && !(v[i][j] == -INFINITY)) { lo = min(lo, key); hi = max(hi, key + 1); }
+                    }
+            }
+        }
+        block_hull(lo, hi);
+        if (threadIdx.x == 0) {
+            p.kv_start[rw] = hi > 0 ? lo : 0;
+            p.kv_end[rw] = hi;
+        }
+        __syncthreads();        // the work-group's numbers have been read
     }
 }
 
@@ -336,19 +369,29 @@ __global__ __launch_bounds__(256) void bias_interval_kernel(const BiasHullParams
 // masked (an entry above -30000), and whether the row is that interval and nothing else - every
 // entry inside it exactly 0, at least one.  Reads the mask once, 2 bytes per (row, key), where turning
 // it into an fp32 bias and looking for the hull of that took ten launches and 16 bytes (2 x 300 rows x
-// 6404 keys: 75 us, this: 6).  Rows start on any element, so an 8-byte load may begin before the row or end
+// 6404 keys: 75 us, this: 8; 4 x 1 rows 5.4, 7.0 with one 8-byte word of a thread in flight instead of four).  Rows start on any element, so an 8-byte load may begin before the row or end
 // behind it; it stays inside the 8-byte word that holds an element of the row.
 template <typename T>
 __global__ __launch_bounds__(256) void mask_interval_kernel(const MaskIntervalParams p) {
     constexpr int EPW = 8 / sizeof(T);                  // elements per 8-byte word
     __shared__ int red[4][4];
-    const int b = blockIdx.x / p.Lq, row = blockIdx.x % p.Lq;
+    fetch_kernargs<sizeof(MaskIntervalParams)>();
+    uint32_t row;
+    const uint32_t b = p.by_Lq.split(blockIdx.x, row);
     const T* r = static_cast<const T*>(p.mask) + b * p.stride_b + (int64_t)row * p.stride_r;
     const int skew = (int)((reinterpret_cast<uintptr_t>(r) & 7) / sizeof(T));       // elements of the first word before the row
     const uint2* words = reinterpret_cast<const uint2*>(r - skew);
     int lo = INT_MAX, hi = 0, n = 0, other = 0;
-    for (int w = threadIdx.x; w * EPW < p.Lkv + skew; w += 256) {
-        const uint2 u = words[w];
+    const int n_words = (p.Lkv + skew + EPW - 1) / EPW;
+    constexpr int BATCH = 4;                            // words of a thread in flight
+    for (int w0 = threadIdx.x; w0 < n_words; w0 += BATCH * 256) {
+      uint2 us[BATCH];
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) us[i] = words[min(w0 + i * 256, n_words - 1)];
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) {
+        const int w = w0 + i * 256;
+        const uint2 u = us[i];
 #pragma unroll
         for (int e = 0; e < EPW; ++e) {
             const int key = w * EPW + e - skew;
@@ -366,6 +409,7 @@ __global__ __launch_bounds__(256) void mask_interval_kernel(const MaskIntervalPa
                 other |= !(x == 0.f);
             }
         }
+      }
     }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -453,15 +497,15 @@ __global__ __launch_bounds__(64) void bwd_live_kernel(const LiveParams p) {
 template <bool F16>
 __global__ __launch_bounds__(256) void cast_kernel(const CastParams p) {
     using E = Elt<F16>;
+    fetch_kernargs<sizeof(CastParams)>();
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int sh = chunk_shift(p.D);
     const int Dh = 8 << sh;
     const int chunk = (int)(idx & ((1 << sh) - 1));
     const int64_t r = idx >> sh;
     if (r >= (int64_t)p.B * p.H * p.L) return;
-    const int row = (int)(r % p.L);
-    const int bh = (int)(r / p.L);
-    const int b = bh / p.H, h = bh % p.H;
+    const RowOf at_row((uint32_t)r, p.by_L, p.by_H);
+    const int row = at_row.row, b = at_row.b, h = at_row.h;
     const f32x4* s = reinterpret_cast<const f32x4*>(p.src + r * Dh + chunk * 8);
     const f32x4 a = s[0], c = s[1];
     u32x4 u;
@@ -501,14 +545,15 @@ __global__ __launch_bounds__(256) void cast_shared_kernel(const CastSharedParams
 template <bool F16>
 __global__ __launch_bounds__(256) void cast_t_kernel(const CastParams p) {
     using E = Elt<F16>;
+    fetch_kernargs<sizeof(CastParams)>();
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int sh = chunk_shift(p.D);
     const int Dh = 8 << sh;
     if (idx >= ((int64_t)p.B * p.H * p.L << sh)) return;
-    const int row = (int)(idx % p.L);
-    const int chunk = (int)((idx / p.L) & ((1 << sh) - 1));
-    const int bh = (int)(idx / ((int64_t)p.L << sh));
-    const int b = bh / p.H, h = bh % p.H;
+    uint32_t row, h;       // launch_cast checks that a thread's number fits 32 bits
+    const uint32_t col = p.by_L.split((uint32_t)idx, row);      // a chunk of a (b, h)
+    const int chunk = (int)(col & ((1u << sh) - 1)), bh = (int)(col >> sh);
+    const int b = (int)p.by_H.split((uint32_t)bh, h);
     const float* s = p.src + ((int64_t)bh * Dh + chunk * 8) * p.L + row;
     float a[8];
 #pragma unroll
@@ -604,9 +649,12 @@ inline int blocks_for(int64_t rows) { return (int)((rows * 16 + 255) / 256); }
 
 }  // namespace
 
-hipError_t launch_merge(const MergeParams& p, hipStream_t st) {
+hipError_t launch_merge(const MergeParams& params, hipStream_t st) {
+    MergeParams p = params;
     const int64_t rows = (int64_t)p.B * p.Hq * (p.row_end - p.row_begin);
     if (rows == 0) return hipSuccess;
+    p.by_rows = divisor(p.row_end - p.row_begin);
+    p.by_Hq = divisor(p.Hq);
     if (p.nparts == 1 && p.use_acc && !p.o_in) {
         const dim3 grid(blocks_for((rows + 1) / 2));
         if (p.f16) return launch1(merge_pair_kernel<true>, grid, dim3(256), st, p);
@@ -626,9 +674,12 @@ hipError_t launch_merge(const MergeParams& p, hipStream_t st) {
     return p.f16 ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
 }
 
-hipError_t launch_preprocess(const PreParams& p, hipStream_t st) {
+hipError_t launch_preprocess(const PreParams& params, hipStream_t st) {
+    PreParams p = params;
     const int64_t rows = (int64_t)p.B * p.Hq * (p.row_end - p.row_begin);
     if (rows == 0) return hipSuccess;
+    p.by_rows = divisor(p.row_end - p.row_begin);
+    p.by_Hq = divisor(p.Hq);
     if (p.f16) return launch1(preprocess_kernel<true>, dim3(blocks_for((rows + 1) / 2)), dim3(256), st, p);
     else return launch1(preprocess_kernel<false>, dim3(blocks_for((rows + 1) / 2)), dim3(256), st, p);
 }
@@ -639,6 +690,7 @@ hipError_t launch_bwd_meta(const MetaParams& p0, hipStream_t st) {
     const int zero_blocks = p.scratch ? 8 * (p.sb.blocks_per_xcd - p.sb.whole) * SHARE_PARTS : 0;
     if (n == 0 && zero_blocks == 0) return hipSuccess;
     p.meta_blocks = (int)((n + 255) / 256);
+    p.by_rows = divisor(std::max(1, p.n_tiles * 32));
     return launch1(bwd_meta_kernel, dim3((unsigned)(p.meta_blocks + zero_blocks)), dim3(256), st, p);
 }
 
@@ -650,13 +702,17 @@ hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st) {
     return launch1(bwd_live_kernel, dim3((p.n_kv_blocks + 63) / 64 + rank_blocks, p.B), dim3(64), st, p);
 }
 
-hipError_t launch_bias_hull(const BiasHullParams& p, hipStream_t st) {
+hipError_t launch_bias_hull(const BiasHullParams& params, hipStream_t st) {
+    BiasHullParams p = params;
     const int64_t rows = (int64_t)p.B * p.Lq;
     if (rows == 0) return hipSuccess;
-    return launch1(bias_hull_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), st, p);
+    p.by_Lq = divisor(p.Lq);
+    return launch1(bias_hull_kernel, dim3((unsigned)std::min<int64_t>(rows, 1 << 20)), dim3(256), st, p);
 }
 
-hipError_t launch_mask_intervals(const MaskIntervalParams& p, hipStream_t st) {
+hipError_t launch_mask_intervals(const MaskIntervalParams& params, hipStream_t st) {
+    MaskIntervalParams p = params;
+    p.by_Lq = divisor(p.Lq);
     const dim3 grid((unsigned)((int64_t)p.B * p.Lq));
     if (p.type == 1) return launch1(mask_interval_kernel<uint16_t>, grid, dim3(256), st, p);
     if (p.type == 2) return launch1(mask_interval_kernel<_Float16>, grid, dim3(256), st, p);
@@ -684,9 +740,13 @@ hipError_t launch_cast_shared(const CastSharedParams& p, hipStream_t st) {
     return launch1(cast_shared_kernel<false>, grid, dim3(256), st, p);
 }
 
-hipError_t launch_cast(const CastParams& p, hipStream_t st) {
+hipError_t launch_cast(const CastParams& params, hipStream_t st) {
+    CastParams p = params;
     const int64_t rows = (int64_t)p.B * p.H * p.L;
     if (rows == 0) return hipSuccess;
+    if (p.transposed && rows * 16 > UINT32_MAX) return hipErrorInvalidValue;    // 256 rows of dQ at most per CU
+    p.by_L = divisor(p.L);
+    p.by_H = divisor(p.H);
     const dim3 grid(blocks_for(rows));
     if (p.transposed) {
         if (p.f16) return launch1(cast_t_kernel<true>, grid, dim3(256), st, p);
