@@ -64,8 +64,7 @@ constexpr int OFF_DO = OFF_Q + NQD * TILE_ELEMS; // x NQD
 constexpr int OFF_DST = OFF_DO + NQD * TILE_ELEMS; // x2
 constexpr int OFF_PB = OFF_DST + 2 * DST_ELEMS;  // x2
 constexpr int LOOP_ELEMS = OFF_PB + 2 * PB_ELEMS;
-constexpr int EPS = D + 1;                          // row stride (floats) of the epilogue's transposed tile
-constexpr int EPI_ELEMS = 8 * 32 * EPS * 2;         // 8 waves x [32 tokens][128 + 1] floats, in uint16 units
+constexpr int EPI_ELEMS = 8 * 32 * (D + 4) * 2;     // 8 waves x [32 tokens][128 + 4] floats of the epilogue, in uint16 units
 constexpr int SMEM_ELEMS = LOOP_ELEMS > EPI_ELEMS ? LOOP_ELEMS : EPI_ELEMS;
 
 constexpr uint32_t META_B = 768;   // bytes of a tile's metadata
@@ -124,30 +123,26 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     // each, then `mid_blocks` with q_splits work-groups each, then the others with q_splits2
     // each - the longer work-groups first.  (A placement hint only: every (block, range) is
     // produced exactly once whatever the hardware does with the ids.)
+    fetch_kernargs<sizeof(BwdParams)>();
     const int xcd = blockIdx.x % 8, local = blockIdx.x / 8;
     const int blk0 = xcd * p.blocks_per_xcd;
     const int nblk = min(p.blocks_per_xcd, p.n_blocks - blk0);
     const int whole = max(0, min(p.whole_blocks, nblk));
     const int mid = max(0, min(p.mid_blocks, nblk - whole));
-    int blk, sp = 0, S = 1;
+    int blk, S = 1;
+    uint32_t sp = 0, kblk, b;
     if (local < whole) {
         blk = blk0 + local;
     } else if (local < whole + mid * p.q_splits) {
-        const int l2 = local - whole;
         S = p.q_splits;
-        sp = l2 % S;
-        blk = blk0 + whole + l2 / S;
+        blk = blk0 + whole + p.by_splits.split(local - whole, sp);
     } else {
-        const int l3 = local - whole - mid * p.q_splits;
         S = p.q_splits2;
-        sp = l3 % S;
-        blk = blk0 + whole + mid + l3 / S;
+        blk = blk0 + whole + mid + p.by_splits2.split(local - whole - mid * p.q_splits, sp);
         if (blk >= blk0 + nblk) return;
     }
-    const int kblk = blk % p.n_kv_blocks;
-    const int bh = blk / p.n_kv_blocks;
-    const int b = bh % p.B;            // samples interleaved: ragged samples then share the tail of the launch
-    const int hk = bh / p.B;
+    const uint32_t bh = p.by_kv_blocks.split(blk, kblk);
+    const uint32_t hk = p.by_B.split(bh, b);        // samples interleaved: ragged samples then share the tail of the launch
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -179,7 +174,7 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         }
         n_live = run_n[0] + run_n[1] + run_n[2] + run_n[3];
     }
-    const int split_steps = (p.G * n_live + S - 1) / S;
+    const int split_steps = S == 1 ? p.G * n_live : (p.G * n_live + S - 1) / S;
     auto sel4 = [](int r, const int (&a)[4]) { return r == 0 ? a[0] : r == 1 ? a[1] : r == 2 ? a[2] : a[3]; };
     const int it_lo = sp * split_steps;
     const int n_iter = (kvb < kv_len) ? max(0, min(split_steps, p.G * n_live - it_lo)) : 0;
@@ -242,8 +237,11 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     // re-derived only when the head changes, everything else advances by constants.
     int cur_gi = 0, cur_run = 0, cur_qt = 0, cur_left = 1;    // cur_left: tiles left in the run, this one included
     if (n_iter > 0) {
-        cur_gi = it_lo / n_live;
-        int idx = it_lo % n_live;
+        int idx = 0;
+        if (it_lo > 0) {
+            cur_gi = it_lo / n_live;
+            idx = it_lo % n_live;
+        }
         while (idx >= sel4(cur_run, run_n)) { idx -= sel4(cur_run, run_n); ++cur_run; }
         cur_qt = sel4(cur_run, run_s) + idx;
         cur_left = sel4(cur_run, run_n) - idx;
@@ -692,60 +690,78 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         else run(std::false_type{}, std::false_type{});
     }
 
-    // ---- epilogue: rows of acc = head-dim, cols = this wave's tokens; P-waves hold dV^T, D-waves dK^T
-    if (dkv_mode == 2) {
-        // Several work-groups (ranges of steps) share this token block: add with
-        // atomics.  The accumulator has tokens along the lanes; it is turned
-        // through LDS so that each atomic instruction covers 64 consecutive
-        // floats (two full lines) of one token row.
-        __syncthreads();   // the staging buffers are free now
-        if (n_iter > 0) {
-            float* ep = reinterpret_cast<float*>(smem) + wave * (32 * EPS);
+    // ---- epilogue: rows of acc = head-dim, cols = this wave's tokens; P-waves hold dV^T, D-waves dK^T.
+    // A lane holds 4 consecutive values of d of one token per register group.  The accumulator is turned through LDS, in
+    // the type it leaves in, so that the lanes of an instruction cover whole token rows; rows are 16 bytes longer there
+    // than their values, as in the forward.  Stored from the registers, 16 or 32 bytes of 32 rows at a time, adding to an
+    // fp32 accumulator took 9.5 us at the end of a work-group of 32 steps (46 us in all) and 16-bit rows 3 - 5; so 7.5 -
+    // all CUs at once then move 67 MB, 9 TB/s; lines brought into the L2 ahead of it cost the steps what they save
+    // here - and 1.2 - 1.7.
+    __syncthreads();   // the staging buffers are free now
+    constexpr int EP32 = 4 * DH + 16, EP16 = 2 * DH + 16;
+    static_assert(8 * 32 * EP32 <= SMEM_ELEMS * 2);
+    char* const ep = reinterpret_cast<char*>(smem) + wave * (32 * EP32);
+    const int n_tok = p.Lkv - slice_lo;                 // of this wave's 32 tokens those that exist, where fewer
+    if (n_tok <= 0) return;
+    const Strides3 os = alone ? (d_role ? p.dks_whole : p.dvs_whole) : (d_role ? p.dks : p.dvs);
+    void* const optr = alone ? (d_role ? p.dk_whole : p.dv_whole) : (d_role ? p.dk : p.dv);
+    const int64_t o_at = b * os.b + hk * os.h + (int64_t)slice_lo * os.s;
+    auto turn_f32 = [&]() {
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
+        for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) ep[l32 * EPS + dt * 32 + acc_row(v, g)] = acc[dt][v];
-            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wave's LDS writes have landed
-            const Strides3 os = d_role ? p.dks : p.dvs;
-            float* obase = reinterpret_cast<float*>(d_role ? p.dk : p.dv) + b * os.b + hk * os.h;
-            for (int t = 0; t < 32; ++t) {
-                const int token = kvb + 32 * slice + t;
-                if (token >= p.Lkv) break;
-                float* op = obase + (int64_t)token * os.s;
-                if (DH >= 64 || lane < DH) unsafeAtomicAdd(op + lane, ep[t * EPS + lane]);
-                if (DH == 128) unsafeAtomicAdd(op + 64 + lane, ep[t * EPS + 64 + lane]);
+            for (int vg = 0; vg < 4; ++vg) {
+                if (dt * 32 + 8 * vg >= DH) continue;   // only with DH = 16
+                const f32x4 x = {acc[dt][4 * vg], acc[dt][4 * vg + 1], acc[dt][4 * vg + 2], acc[dt][4 * vg + 3]};
+                *reinterpret_cast<f32x4*>(ep + l32 * EP32 + g * 16 + (8 * dt + 2 * vg) * 16) = x;
             }
+        wait_lds();     // this wave's rows are its own
+    };
+    if (dkv_mode == 2) {
+        // Several work-groups (ranges of steps) share this token block: atomic adds, 64 consecutive floats
+        // (two full lines) of one token row each
+        if (n_iter == 0) return;
+        turn_f32();
+        float* const op = reinterpret_cast<float*>(optr) + o_at + lane;
+        const float* const src = reinterpret_cast<const float*>(ep) + lane;
+        for (int t = 0; t < min(n_tok, 32); ++t) {
+            if (DH >= 64 || lane < DH) unsafeAtomicAdd(op + t * os.s, src[t * (EP32 / 4)]);
+            if (DH == 128) unsafeAtomicAdd(op + t * os.s + 64, src[t * (EP32 / 4) + 64]);
         }
-    } else if (my_kv < p.Lkv) {
-        const Strides3 os = alone ? (d_role ? p.dks_whole : p.dvs_whole) : (d_role ? p.dks : p.dvs);
-        void* optr = alone ? (d_role ? p.dk_whole : p.dv_whole) : (d_role ? p.dk : p.dv);
-        const int64_t off = b * os.b + hk * os.h + (int64_t)my_kv * os.s;
-        if (dkv_mode == 1) {
-            float* op = reinterpret_cast<float*>(optr) + off;
+    } else if (dkv_mode == 1) {
+        constexpr int CPF = DH / 4, RPS = 64 / CPF;     // chunks of a row of floats, rows per instruction
+        float* const op = reinterpret_cast<float*>(optr) + o_at + (lane % CPF) * 4;
+        f32x4 old[32 / RPS];                            // on their way while the accumulator is turned
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
+        for (int i = 0; i < 32 / RPS; ++i) old[i] = *reinterpret_cast<const f32x4*>(op + min(i * RPS + lane / CPF, n_tok - 1) * os.s);
+        turn_f32();
 #pragma unroll
-                for (int vg = 0; vg < 4; ++vg) {
-                    const int d = dt * 32 + 8 * vg + 4 * g;
-                    if (d >= DH) continue;      // only with DH = 16
-                    f32x4 a = *reinterpret_cast<f32x4*>(op + d);
+        for (int i = 0; i < 32 / RPS; ++i) {
+            const int t = i * RPS + lane / CPF;
+            const f32x4 x = *reinterpret_cast<const f32x4*>(ep + (lane / CPF) * EP32 + (lane % CPF) * 16 + i * (RPS * EP32));
+            if (t < n_tok) *reinterpret_cast<f32x4*>(op + t * os.s) = old[i] + x;
+        }
+    } else {
+        constexpr int CPR = DH / 8, RPS = 64 / CPR;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) a[r] += acc[dt][4 * vg + r];
-                    *reinterpret_cast<f32x4*>(op + d) = a;
-                }
-        } else {
-            uint16_t* op = reinterpret_cast<uint16_t*>(optr) + off;
+        for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
+            for (int vg = 0; vg < 4; ++vg) {
+                if (dt * 32 + 8 * vg >= DH) continue;   // only with DH = 16
+                u32x2 a;
+                a[0] = E::pack(acc[dt][4 * vg], acc[dt][4 * vg + 1]);
+                a[1] = E::pack(acc[dt][4 * vg + 2], acc[dt][4 * vg + 3]);
+                // of rows 16 apart one has the halves of its chunks exchanged: conflict-free
+                *reinterpret_cast<u32x2*>(ep + l32 * EP16 + ((g ^ (l32 >> 4)) << 3) + (4 * dt + vg) * 16) = a;
+            }
+        wait_lds();
+        uint16_t* const op = reinterpret_cast<uint16_t*>(optr) + o_at + (lane % CPR) * 8;
 #pragma unroll
-                for (int vg = 0; vg < 4; ++vg) {
-                    const int d = dt * 32 + 8 * vg + 4 * g;
-                    if (d >= DH) continue;      // only with DH = 16
-                    u32x2 a;
-                    a[0] = E::pack(acc[dt][4 * vg], acc[dt][4 * vg + 1]);
-                    a[1] = E::pack(acc[dt][4 * vg + 2], acc[dt][4 * vg + 3]);
-                    *reinterpret_cast<u32x2*>(op + d) = a;
-                }
+        for (int i = 0; i < 32 / RPS; ++i) {
+            const int t = i * RPS + lane / CPR;
+            const u32x4 x = *reinterpret_cast<const u32x4*>(ep + (lane / CPR) * EP16 + (lane % CPR) * 16 + i * (RPS * EP16));
+            const u32x4 y = (t >> 4) & 1 ? u32x4{x[2], x[3], x[0], x[1]} : x;
+            if (t < n_tok) *reinterpret_cast<u32x4*>(op + t * os.s) = y;
         }
     }
 }
@@ -767,7 +783,12 @@ hipError_t launch_bwd_t(const BwdParams& p, bool masked, hipStream_t st) {
 }
 }  // namespace
 
-hipError_t launch_bwd(const BwdParams& p, bool masked, hipStream_t st) {
+hipError_t launch_bwd(const BwdParams& params, bool masked, hipStream_t st) {
+    BwdParams p = params;
+    p.by_splits = divisor(p.q_splits);
+    p.by_splits2 = divisor(p.q_splits2);
+    p.by_kv_blocks = divisor(p.n_kv_blocks);
+    p.by_B = divisor(p.B);
     switch (p.D) {
         case 16: return p.f16 ? launch_bwd_t<16, true>(p, masked, st) : launch_bwd_t<16, false>(p, masked, st);
         case 32: return p.f16 ? launch_bwd_t<32, true>(p, masked, st) : launch_bwd_t<32, false>(p, masked, st);

@@ -169,6 +169,7 @@ struct BwdParams {
     // + 2 i + {0, 1}] = first tile and number of tiles of run i (0 tiles: unused).  Null: every tile.
     const int32_t* live_runs;
     int f16;                   // element type of q, k, v, dout, the dS^T workspace and (mode 0) dk, dv
+    Divisor by_splits, by_splits2, by_kv_blocks, by_B;     // filled in by launch_bwd
 };
 
 // Which (token block, 32-row tile) pairs an interval mask leaves alive, at the granularity the
