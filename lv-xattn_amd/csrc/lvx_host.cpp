@@ -31,6 +31,8 @@ struct Library {
     decltype(&lvx_fwd_acc) fwd_acc;
     decltype(&lvx_bwd_preprocess) bwd_preprocess;
     decltype(&lvx_bwd) bwd;
+    decltype(&lvx_bwd_workspace_bytes) bwd_workspace_bytes;
+    decltype(&lvx_bias_hull) bias_hull;
 } lib;
 
 void bind(const std::map<std::string, uintptr_t>& addresses) {
@@ -40,6 +42,8 @@ void bind(const std::map<std::string, uintptr_t>& addresses) {
     set(lib.fwd_acc, "lvx_fwd_acc");
     set(lib.bwd_preprocess, "lvx_bwd_preprocess");
     set(lib.bwd, "lvx_bwd");
+    set(lib.bwd_workspace_bytes, "lvx_bwd_workspace_bytes");
+    set(lib.bias_hull, "lvx_bias_hull");
 }
 
 int dtype_code(const Tensor& t) {
@@ -78,6 +82,23 @@ bool fill_shape(lvx_attn_shape& s, const Tensor& q, const Tensor& k, const Tenso
     if (kv_len) s.kv_len = kv_len->data_ptr<int32_t>();
     if (kv_start) { s.kv_start = kv_start->data_ptr<int32_t>(); s.kv_end = kv_end->data_ptr<int32_t>(); }
     return true;
+}
+
+// The dense bias of a call, fp32 [B|1, Hq|1, Lq, Lkv]; false when the library would refuse it.  A dimension of extent
+// 1 is never stepped over: the library is told the stride its own checks accept, whatever the tensor says.
+bool fill_bias(lvx_attn_shape& s, const OptTensor& bias, const Tensor& q) {
+    if (!bias) return true;
+    const Tensor& t = *bias;
+    if (!plain4(t, q, at::kFloat) || (t.size(0) != 1 && t.size(0) != s.B) || (t.size(1) != 1 && t.size(1) != s.Hq) || t.size(2) != s.Lq ||
+        t.size(3) != s.Lkv)
+        return false;
+    const int64_t row = ((int64_t)s.Lkv + 3) / 4 * 4;
+    s.bias = t.data_ptr<float>();
+    s.bias_stride_b = t.size(0) > 1 ? t.stride(0) : 0;
+    s.bias_stride_h = t.size(1) > 1 ? t.stride(1) : 0;
+    s.bias_stride_r = s.Lq > 1 ? t.stride(2) : row;
+    return s.bias_stride_r >= row && !((s.bias_stride_b | s.bias_stride_h | s.bias_stride_r) & 3) &&
+           !(reinterpret_cast<uintptr_t>(s.bias) & 15);
 }
 
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
@@ -119,9 +140,9 @@ py::tuple forward_buffers(const Tensor& q, int64_t rows, int64_t kv_splits, bool
 
 bool fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, double scale, int64_t row_begin,
          int64_t row_count, const OptTensor& kv_len, const OptTensor& kv_start, const OptTensor& kv_end, int64_t kv_splits,
-         const OptTensor& ws, const OptTensor& acc_o, const OptTensor& acc_l) {
+         const OptTensor& ws, const OptTensor& acc_o, const OptTensor& acc_l, const OptTensor& bias) {
     lvx_attn_shape s;
-    if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end) || !plain4(o, q, q.scalar_type()) || o.sizes() != q.sizes() || !rows_ok(lse, q))
+    if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end) || !fill_bias(s, bias, q) || !plain4(o, q, q.scalar_type()) || o.sizes() != q.sizes() || !rows_ok(lse, q))
         return false;
     const lvx_tensor tq = t4(q), tk = t4(k), tv = t4(v), to = t4(o);
     void* const wp = ws ? ws->data_ptr() : nullptr;
@@ -155,9 +176,9 @@ bool bwd_preprocess(const Tensor& o, const Tensor& dout, const Tensor& delta, in
 
 bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
          const Tensor& dk, const Tensor& dv, double scale, int64_t row_begin, int64_t row_count, const OptTensor& kv_len,
-         const OptTensor& kv_start, const OptTensor& kv_end, bool accumulate_dkv, const Tensor& ws) {
+         const OptTensor& kv_start, const OptTensor& kv_end, bool accumulate_dkv, const Tensor& ws, const OptTensor& bias) {
     lvx_attn_shape s;
-    if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end)) return false;
+    if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end) || !fill_bias(s, bias, q)) return false;
     const at::ScalarType kv_type = accumulate_dkv ? at::kFloat : q.scalar_type();
     if (!plain4(dout, q, q.scalar_type()) || dout.sizes() != q.sizes() || !rows_ok(lse, q) || !rows_ok(delta, q) ||
         !plain4(dq, q, q.scalar_type()) || dq.sizes() != q.sizes() || !plain4(dk, q, kv_type) || dk.sizes() != k.sizes() ||
@@ -174,6 +195,38 @@ bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, 
     return true;
 }
 
+// (kv_start, kv_end) of the hull of what a bias leaves visible, int32 [B, Lq] each, or None.
+py::object bias_hull(const Tensor& q, const Tensor& k, const Tensor& bias) {
+    lvx_attn_shape s;
+    if (!fill_shape(s, q, k, k, 1.0, {}, {}, {}) || !fill_bias(s, bias, q)) return py::none();
+    Tensor start = at::empty({s.B, s.Lq}, q.options().dtype(at::kInt)), end = at::empty({s.B, s.Lq}, q.options().dtype(at::kInt));
+    int32_t *const sp = start.data_ptr<int32_t>(), *const ep = end.data_ptr<int32_t>();
+    void* const st = current_stream();
+    call("lvx_bias_hull", [&] { return lib.bias_hull(&s, sp, ep, st); });
+    return py::make_tuple(std::move(start), std::move(end));
+}
+
+// Bytes of the backward's workspace for a window of `rows` rows, or -1.
+int64_t bwd_workspace_bytes(const Tensor& q, const Tensor& k, int64_t rows, const OptTensor& kv_len, const OptTensor& kv_start,
+                            const OptTensor& kv_end) {
+    lvx_attn_shape s;
+    if (!fill_shape(s, q, k, k, 1.0, kv_len, kv_start, kv_end)) return -1;
+    return (int64_t)lib.bwd_workspace_bytes(&s, (int32_t)rows);
+}
+
+// (dq, dk, dv) of a backward: dq contiguous, or in q's memory order with `like_q`; dk and dv views of
+// [B, Lkv, Hkv, D] memory.
+py::tuple backward_outputs(const Tensor& q, const Tensor& k, bool like_q) {
+    Tensor dq = like_q ? at::empty_like(q) : at::empty(q.sizes(), q.options());
+    const auto kv = [&] { return at::empty({k.size(0), k.size(2), k.size(1), k.size(3)}, q.options()).transpose(1, 2); };
+    Tensor dk = kv(), dv = kv();
+    return py::make_tuple(std::move(dq), std::move(dk), std::move(dv));
+}
+
+uintptr_t stream_of(int64_t device) {
+    return reinterpret_cast<uintptr_t>(c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream());
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_lvx_host, m) {
@@ -183,4 +236,8 @@ PYBIND11_MODULE(_lvx_host, m) {
     m.def("fwd", &fwd);
     m.def("bwd_preprocess", &bwd_preprocess);
     m.def("bwd", &bwd);
+    m.def("bwd_workspace_bytes", &bwd_workspace_bytes);
+    m.def("bias_hull", &bias_hull);
+    m.def("backward_outputs", &backward_outputs);
+    m.def("stream_of", &stream_of);
 }

@@ -118,7 +118,7 @@ def check(rc: int, what: str) -> None:
 
 
 def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return host().stream_of(-1)         # of the current device
 
 
 def t4(t: torch.Tensor) -> Tensor4:

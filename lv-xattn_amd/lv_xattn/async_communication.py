@@ -14,6 +14,8 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
+from ._lib import host
+
 _ROUNDS = 1
 _INITIALISED = False
 _WORKSPACES: Dict[Tuple, torch.Tensor] = {}
@@ -102,12 +104,12 @@ def workspace(tag: str, shape, dtype, device) -> torch.Tensor:
     dev = torch.device(device)
     if dev.type == "cuda" and dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
-    stream = torch.cuda.current_stream(dev).cuda_stream if dev.type == "cuda" else 0
+    stream = host().stream_of(dev.index) if dev.type == "cuda" else 0
     key = (tag, str(dev), stream)
     numel = 1
     for n in shape:
         numel *= int(n)
-    nbytes = numel * torch.empty((), dtype=dtype).element_size()
+    nbytes = numel * dtype.itemsize
     buf = _WORKSPACES.get(key)
     if buf is None or buf.numel() < nbytes:
         _WORKSPACES.pop(key, None)

@@ -279,7 +279,9 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
     backward then reads it as it lies) instead of contiguous."""
     _reject_unsupported(causal)
     D_in = q.shape[-1]
-    q_, k_, v_, o_, do_ = (_usable(_pad_head_dim(t)) for t in (q, k, v, o, do))
+    q_, k_, v_, o_, do_ = (_pad_head_dim(t) for t in (q, k, v, o, do))
+    if not (host().usable(q_, k_, v_) and host().usable(o_, do_, do_)):
+        q_, k_, v_, o_, do_ = (_usable(t) for t in (q_, k_, v_, o_, do_))
     B, Hq, Lq, D = q_.shape
     Hkv, Lkv = k_.shape[1], k_.shape[2]
     P = rounds if rounds is not None else get_sequence_parallel_size()
@@ -292,9 +294,7 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
     L_ = L.to(torch.float32).reshape(B * Hq, Lq).contiguous()
 
     delta = workspace("bwd_delta", (B * Hq, Lq), torch.float32, dev)
-    dq = torch.empty_like(q_) if _dq_like_q else torch.empty(B, Hq, Lq, D, dtype=q_.dtype, device=dev)
-    dk = torch.empty(B, Lkv, Hkv, D, dtype=q_.dtype, device=dev).transpose(1, 2)
-    dv = torch.empty(B, Lkv, Hkv, D, dtype=q_.dtype, device=dev).transpose(1, 2)
+    dq, dk, dv = host().backward_outputs(q_, k_, _dq_like_q)
 
     windows = [(0, Lq)] if batched else [w for w in q_block_bounds(Lq, P) if w[1] > w[0]]
     windows = _cap_windows(windows, lambda rows: ops.bwd_workspace_bytes(q_, k_, rows, mask), backward_workspace_cap())

@@ -98,12 +98,11 @@ def fwd(q, k, v, o, lse, scale, row_begin=0, row_count=None, mask: Optional[Mask
     `bias`: dense additive fp32 [B|1, Hq|1, Lq, Lkv], added after the scale.
     `acc` = (o_in like o, l_in fp32 [B*Hq, Lq]): an incoming accumulator the result is merged
     with before it is written (lvx_fwd_acc); only read, and not o itself."""
-    if bias is None:
-        m = mask or _NO_MASK
-        a = acc or (None, None)
-        if host().fwd(q, k, v, o, lse, scale, row_begin, q.shape[2] - row_begin if row_count is None else row_count,
-                      m.kv_len, m.kv_start, m.kv_end, kv_splits, workspace, a[0], a[1]):
-            return
+    m = mask or _NO_MASK
+    a = acc or (None, None)
+    if host().fwd(q, k, v, o, lse, scale, row_begin, q.shape[2] - row_begin if row_count is None else row_count,
+                  m.kv_len, m.kv_start, m.kv_end, kv_splits, workspace, a[0], a[1], bias):
+        return
     s = _shape(q, k, scale, mask, bias)
     if row_count is None:
         row_count = q.shape[2] - row_begin
@@ -158,6 +157,9 @@ def bias_hull(q, k, bias: torch.Tensor) -> Mask:
     """The interval mask a dense bias implies: per text row the hull of its entries other
     than -inf.  Given to fwd / bwd together with the bias it lets them skip what the bias
     masks anyway."""
+    rows = host().bias_hull(q, k, bias)
+    if rows is not None:
+        return Mask(None, *rows)
     s = _shape(q, k, 1.0, None, bias)
     B, Lq = q.shape[0], q.shape[2]
     start = torch.empty(B, Lq, dtype=torch.int32, device=q.device)
@@ -210,6 +212,10 @@ def bwd_preprocess(o, dout, delta, row_begin=0, row_count=None) -> None:
 def bwd_workspace_bytes(q, k, row_count: int, mask: Optional[Mask] = None) -> int:
     """Bytes lvx_bwd needs for `row_count` rows; pass the mask the call will use
     (an interval mask adds its live-tile tables)."""
+    m = mask or _NO_MASK
+    n = host().bwd_workspace_bytes(q, k, row_count, m.kv_len, m.kv_start, m.kv_end)
+    if n >= 0:
+        return n
     s = _shape(q, k, 1.0, mask)
     return int(load().lvx_bwd_workspace_bytes(C.byref(s), row_count))
 
@@ -221,11 +227,11 @@ def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=Non
     (fp32) dk, dv at Hkv heads.  `workspace`: uint8 tensor of at least
     bwd_workspace_bytes(q, k, row_count, mask) bytes.  `bias` as in fwd (no gradient
     is formed for it)."""
-    if bias is None and workspace is not None:
+    if workspace is not None:
         m = mask or _NO_MASK
         if host().bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin,
                       q.shape[2] - row_begin if row_count is None else row_count, m.kv_len, m.kv_start, m.kv_end,
-                      accumulate_dkv, workspace):
+                      accumulate_dkv, workspace, bias):
             return
     s = _shape(q, k, scale, mask, bias)
     if row_count is None:
