@@ -67,22 +67,23 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
     __shared__ __attribute__((aligned(1024))) char kv_lds[2][2][TILE_BYTES];   // [buffer][K, V]
     __shared__ int red[4][4];
 
+    fetch_kernargs<sizeof(FwdParams)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
     if (wid >= p.total_wg) return;
-    const int tile = wid % p.n_row_tiles;
-    const int t1 = wid / p.n_row_tiles;
-    const int split = t1 % p.nsplit;
-    const int t2 = t1 / p.nsplit;
+    uint32_t tile, split, b;
+    const uint32_t t1 = p.by_row_tiles.split(wid, tile), t2 = p.by_splits.split(t1, split);
     // samples vary faster than head groups: every XCD (a contiguous range of ids) then gets
     // work-groups of all samples, and ragged samples do not leave some XCDs idle early
-    const int b = t2 % p.B;
-    const int hg = t2 / p.B;
+    const uint32_t hg = p.by_B.split(t2, b);
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
-    const int h = hg * p.HG + (wave % p.HG);
-    const int hk = h / p.G;
-    const int row = p.row_begin + (tile * p.RS + wave / p.HG) * 32 + l32;
+    // HG is 1, 2 or 4: the wave's head of the group and its row sub-tile
+    const int wave_head = wave & (p.HG - 1), wave_rows = wave >> (p.HG >> 1);
+    const int h = hg * p.HG + wave_head;
+    uint32_t of_group;
+    const int hk = p.by_G.split(h, of_group);
+    const int row = p.row_begin + (tile * p.RS + wave_rows) * 32 + l32;
     const bool row_ok = row < p.row_end;
 
     int kv_len = p.Lkv;
@@ -184,10 +185,33 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
     const float cc = BIAS ? 1.f : c;              // factor from the carried scores to log2 units
     const float* brow = nullptr;                  // this lane's row of the bias
     if (BIAS) brow = p.bias + b * p.bias_b + h * p.bias_h + (int64_t)min(row, p.row_end - 1) * p.bias_r;
+    // The bias of a tile: register group vg of lane-half g holds keys kv0 + 8 vg + 4 g + 0..3, the second four 32 keys
+    // further; groups past the end re-read the last one (those keys are masked).  A tile's values are requested
+    // during the tile before, between the loads of its own K and V and those of the next.  (Requested where they are
+    // used, behind the loads of the next tile, they were waited for together with those: 1024 rows x 16 heads x 4096
+    // keys forward and backward 268 us, so 255.)  The request is assembly,
+    // so the compiler does not know of the wait: nothing may touch the registers before it.
+    u32x4 bq[8];
+    const int last_k = (p.Lkv - 1) & ~3;
+    auto request_bias = [&](int kv0) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float* at = brow + min(kv0 + 8 * (i & 3) + 4 * g + 32 * (i >> 2), last_k);
+            asm volatile("global_load_dwordx4 %0, %1, off" : "+v"(bq[i]) : "v"(at) : "memory");
+            __builtin_amdgcn_sched_barrier(0);      // one address at a time
+        }
+    };
 
     const int t_begin = (hi > lo) ? lo / BN : 0;
     const int t_end = (hi > lo) ? (hi + BN - 1) / BN : 0;
-    if (t_end > t_begin) issue(t_begin * BN, 0);
+    if (t_end > t_begin) {
+        issue(t_begin * BN, 0);
+        if (BIAS) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) bq[i] = u32x4{0u, 0u, 0u, 0u};
+            request_bias(t_begin * BN);
+        }
+    }
 
     for (int t = t_begin; t < t_end; ++t) {
         const int kv0 = t * BN;
@@ -198,8 +222,9 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
         // tile t has landed (this wave's part: vmcnt; everyone's: barrier); the
         // barrier also says every wave is done reading tile t-1, whose buffer
         // the loads of tile t+1 may now overwrite
-        wait_vmcnt<0>();
-        __syncthreads();
+        if (BIAS) wait_vmcnt<8>();          // the tile's bias, requested after it, may be on its way
+        else wait_vmcnt<0>();
+        lds_barrier();
         if (t + 1 < t_end) issue(kv0 + BN, buf ^ 1);
 
         // S^T = K Q^T : rows = keys (two 32-key sub-tiles), cols = text rows.
@@ -222,6 +247,20 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
             s1 = E::mfma(ka[kk][1], qreg[kk], s1);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if (BIAS) {
+            if (t + 1 < t_end) wait_vmcnt<8>();         // all but the loads of the next tile
+            else wait_vmcnt<0>();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(bq[i]));
+#pragma unroll
+            for (int vg = 0; vg < 4; ++vg)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    s0[4 * vg + r] = fmaf(s0[4 * vg + r], c, __uint_as_float(bq[vg][r]) * LOG2E_F);
+                    s1[4 * vg + r] = fmaf(s1[4 * vg + r], c, __uint_as_float(bq[4 + vg][r]) * LOG2E_F);
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
         // V^T operands of this tile: requested now, they land during the softmax
         u32x2 va[NDT][4][2];
 #pragma unroll
@@ -232,22 +271,6 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
                 va[dt][j][1] = lds_read_tr16(reinterpret_cast<const uint16_t*>(Vs + v_rd[dt][1] + j * 4096));
             }
         __builtin_amdgcn_sched_barrier(0);
-
-        if (BIAS) {
-            // register group vg of lane-half g holds keys kv0 + 8 vg + 4 g + 0..3 (+32 for s1);
-            // groups past the end re-read the last one (those keys are masked below)
-#pragma unroll
-            for (int vg = 0; vg < 4; ++vg) {
-                const int k0 = kv0 + 8 * vg + 4 * g;
-                const f32x4 ba = *reinterpret_cast<const f32x4*>(brow + min(k0, (p.Lkv - 1) & ~3));
-                const f32x4 bb = *reinterpret_cast<const f32x4*>(brow + min(k0 + 32, (p.Lkv - 1) & ~3));
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    s0[4 * vg + r] = fmaf(s0[4 * vg + r], c, ba[r] * LOG2E_F);
-                    s1[4 * vg + r] = fmaf(s1[4 * vg + r], c, bb[r] * LOG2E_F);
-                }
-            }
-        }
 
         if (kv0 < in_lo || kv0 + BN > in_hi) {
 #pragma unroll
@@ -317,9 +340,16 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
             for (int j = 0; j < 4; ++j) {
                 const u32x4 a = {va[dt][j][0][0], va[dt][j][0][1], va[dt][j][1][0], va[dt][j][1][1]};
                 acc[dt] = E::mfma(as_bf16x8(a), pb[j], acc[dt]);
+                // registers that the first half of V^T has left take the next tile's bias
+                if (BIAS && dt == (NDT - 1) / 2 && j == 3) request_bias(min(kv0 + BN, last_k));
             }
     }
 
+    if (BIAS && t_end > t_begin) {      // the last request has to land before its registers serve anything else
+        wait_vmcnt<0>();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) asm volatile("" ::"v"(bq[i]));
+    }
     // epilogue: the two lane halves hold partial row sums of the same row
     const float l_tot = l_i + __shfl_xor(l_i, 32);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;

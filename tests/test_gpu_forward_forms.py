@@ -72,6 +72,16 @@ def test_few_rows_form(D, dtype, Hq, Hkv, Lq, Lkv, splits, mask, monkeypatch):
     _check(D, dtype, 2, Hq, Hkv, Lq, Lkv, splits, mask, Lq * 1000 + Lkv + 1)
 
 
+# with a dense bias, whose values are requested a tile ahead: one tile and less, two, the last of them partial, key
+# ranges that begin inside the bias, every grouping of heads and rows into a work-group
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [128, 64, 32, 16])
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lkv,splits", [
+    (1, 1, 1, 1, 1), (4, 1, 33, 63, 1), (4, 4, 129, 64, 1), (2, 1, 65, 65, 1), (4, 2, 31, 130, 2), (3, 1, 40, 257, 1), (8, 1, 32, 1000, 5)])
+def test_form_with_a_bias(D, dtype, Hq, Hkv, Lq, Lkv, splits):
+    _check(D, dtype, 2, Hq, Hkv, Lq, Lkv, splits, "bias", Lq * 1000 + Lkv + 2)
+
+
 # nothing in a forward depends on the order in which anything arrives
 @pytest.mark.parametrize("form", ["1", "2"])
 @pytest.mark.parametrize("D", [128, 64, 32])

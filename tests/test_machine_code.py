@@ -1,5 +1,6 @@
 """What inline assembly leaves to the kernels' author, checked on the built library's machine code (see isa.py)."""
 import os
+import re
 
 import pytest
 
@@ -30,6 +31,15 @@ def test_registers_that_assembly_loads_are_left_alone_until_the_wait(kernels):
     assert len(few) == 16
     for name, body in few.items():
         assert sum(i.op == "global_load_dwordx4" for i in body) >= 1
+        assert not isa.loads_touched_early(body), name
+
+
+@needs_objdump
+def test_a_bias_on_its_way_is_left_alone_until_the_wait(kernels):
+    """The forward with a dense bias requests it by inline assembly a tile ahead: the same."""
+    biased = {n: b for n, b in kernels.items() if re.search(r"fwd_kernelILi\d+ELb[01]ELb1E", n)}
+    assert len(biased) == 16
+    for name, body in biased.items():
         assert not isa.loads_touched_early(body), name
 
 
