@@ -1,11 +1,12 @@
 """Writes the hand-scheduled body of the 256-row GEMM tiles (lvx_gemm.hip, gemm_tile_kernel):
 
-    python gen_gemm_loop.py p|t p|t 256|128 > lvx_gemm_loop_<A><B>_<TN>.inc
+    python gen_gemm_loop.py p|t p|t 256|128 256|224 > lvx_gemm_loop_<A><B>_<TN>_<TM>.inc
 
 p: the operand is stored [row][k], read with 16-byte LDS reads; t: stored [k][row], read with transposing
 LDS reads.  The tile is 256 x TN, four waves (2 x 2) of 128 x TN / 2, each with its SIMD to itself: the
 accumulators (16 registers per 32 x 32) live in accumulation registers, and a wave's operands serve
-twice the MFMAs per LDS byte that eight waves' would.
+twice the MFMAs per LDS byte that eight waves' would.  A tile of 224 rows x 256 has its waves side by side, 224 x 64
+each (seven blocks of rows do not halve): nine operands for 14 MFMAs where the others have eight for 16.
 
 One statement runs all stages (64 values of k each) of a tile, one or more, and leaves the C tile in LDS as
 16-bit values.  A stage is 64 deep because a piece of an operand stored [row][k] is then 128 bytes of
@@ -26,7 +27,7 @@ Registers (must match the asm statement in lvx_gemm.hip):
   v[0:63] two operand sets   v[64:79] byte offsets of this wave's pieces (A, then B)   v[80:95] the same for
   the last stage   v[96:107] A read addresses, four per slot   v[108:119] the same for B
   v120 address of this lane's first piece of the C tile   v[121:136] those of its pieces
-  a[16 (WM nt + mt) :] accumulators
+  a[16 (WM nt + mt) :] accumulators   224 rows: v[122:129] the operands that do not fit v[0:63]
   s[40:43], s[44:47] descriptors of A, B   s48, s49 bytes per stage   s50 LDS address of this wave's part of slot
   0   s51 stages left to run   s52, s60 stages of A, B to request after the next   s53, s54 offset of the next
   stage in A, B   s55, s61 stages to request before the second pair of operands (0: none)   s[56:57],
@@ -38,12 +39,13 @@ import sys
 
 # experiment switches (comma separated in LVX_GEMM_OPTS); none is set in a normal build
 OPTS = set(o for o in os.environ.get("LVX_GEMM_OPTS", "").split(",") if o)
-AT, BT, TN = sys.argv[1] == "t", sys.argv[2] == "t", int(sys.argv[3])
-WM, WN = 4, TN // 64
+AT, BT, TN, TM = sys.argv[1] == "t", sys.argv[2] == "t", int(sys.argv[3]), int(sys.argv[4])
+assert TM == 256 or (TM == 224 and TN == 256 and not AT)
+WM, WN = (4, TN // 64) if TM == 256 else (7, 2)
 NSA, NSB = 3, 2 if TN == 256 else 3
 UNROLL = 6 if NSB == 2 else 3
-A_BYTES, B_BYTES = 256 * 128, TN * 128
-NLA, NLB = 8, TN // 32              # 1 KiB pieces per wave and stage
+A_BYTES, B_BYTES = TM * 128, TN * 128
+NLA, NLB = TM // 32, TN // 32              # 1 KiB pieces per wave and stage
 NL = NLA + NLB
 OPER, VOFF, VTAIL, RA, RB, EP, EPA = 0, 64, 80, 96, 108, 120, 121
 MFMA, CVT = '" LVX_GEMM_MFMA "', '" LVX_GEMM_CVT "'
@@ -62,6 +64,8 @@ def am(s, mt):
 
 
 def bn(s, nt):
+    if TM == 224:
+        return OPER + 32 * s + 28 if nt == 0 else 122 + 4 * s
     return OPER + 32 * s + 16 + 4 * nt
 
 
@@ -79,7 +83,7 @@ def reads(u, kk, s):
         out += one(BT, RB + 4 * (u % NSB), bn(s, nt), nt, TN)
         if nt == 0:
             for mt in range(WM):
-                out += one(AT, RA + 4 * (u % NSA), am(s, mt), mt, 256)
+                out += one(AT, RA + 4 * (u % NSA), am(s, mt), mt, TM)
     return out
 
 
@@ -164,15 +168,19 @@ def main():
     for c in range(4 * WN):
         lines.append(f"v_xor_b32 v{EPA + c}, {c * 16}, v{EP}")
     group = 0
-    for nt in range(WN):
-        for vg in range(4):
-            for mt in range(WM):
-                t = 4 * (group % 16)
-                group += 1
-                a = 16 * (WM * nt + mt) + 4 * vg
-                lines += [f"v_accvgpr_read_b32 v{t + i}, a{a + i}" for i in range(4)]
-                lines += [f"{CVT} v{t}, v{t}, v{t + 1}", f"{CVT} v{t + 1}, v{t + 2}, v{t + 3}",
-                          f"ds_write_b64 v{EPA + 4 * nt + vg}, {vr(t, 2)} offset:{mt * 32 * TN * 2}"]
+    in_reach = 65536 // (32 * TN * 2)       # blocks of rows an instruction's offset reaches
+    for m0 in range(0, WM, in_reach):
+        for nt in range(WN):
+            for vg in range(4):
+                if m0:
+                    lines.append(f"v_add_u32 v{EPA + 4 * nt + vg}, 0x10000, v{EPA + 4 * nt + vg}")
+                for mt in range(m0, min(WM, m0 + in_reach)):
+                    t = 4 * (group % 16)
+                    group += 1
+                    a = 16 * (WM * nt + mt) + 4 * vg
+                    lines += [f"v_accvgpr_read_b32 v{t + i}, a{a + i}" for i in range(4)]
+                    lines += [f"{CVT} v{t}, v{t}, v{t + 1}", f"{CVT} v{t + 1}, v{t + 2}, v{t + 3}",
+                              f"ds_write_b64 v{EPA + 4 * nt + vg}, {vr(t, 2)} offset:{(mt - m0) * 32 * TN * 2}"]
     lines += ["s_waitcnt lgkmcnt(0)"]
     if "nodma" in OPTS:
         lines = [l for l in lines if not l.startswith("buffer_load") and not l.startswith("s_add_i32 m0")]

@@ -22,6 +22,8 @@
 //    is kept as it lies, [k][rows], and read with the transposing LDS read.
 //  * The MFMA computes C^T (A operand = rows of the B tile), so a lane ends up
 //    with 4 consecutive columns of one C row and stores 8 bytes.
+#include <algorithm>
+#include <cstdint>
 #include <type_traits>
 
 #include "lvx_common.hpp"
@@ -431,17 +433,18 @@ struct TileOperand {
     }
 };
 
-// The 256 x TN tile of the projections and their gradients: four waves of 128 x TN / 2 in one generated
-// statement (gen_gemm_loop.py), then the C tile, 16-bit in LDS by then, leaves as whole row segments -
+// The TM x TN tile of the projections and their gradients: four waves of 128 x TN / 2 (TM = 224: 224 x 64) in one
+// generated statement (gen_gemm_loop.py), then the C tile, 16-bit in LDS by then, leaves as whole row segments -
 // through the RMS norm where problem 0 has one (16 lanes hold a head's 128 columns of a row).
 // Bound by the matrix pipe and the power it may draw: MFMAs alone on N(0, 1) data sustain 1800 TFLOP/s on the
 // chip, this kernel 1341 (65536 x 4096 x 1024 twice, W [N][K]; 1215 with eight waves of 128 x 64 and stages
 // of 32).  us before and after: that 905 -> 820; 12808 rows 183 -> 176; 2046 x 4096 x 4096 77 -> 60; the
 // weight gradients, until then compiler-scheduled, 12808 rows 258 -> 168 and 6404 rows 134 -> 88.
-template <bool A_T, bool B_T, int TN, bool F16>
+template <bool A_T, bool B_T, int TN, bool F16, int TM>
 __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
     using E = Elt<F16>;
-    constexpr int TM = 256, WM = 4, WN = TN / 64;
+    static_assert(TM == 256 || (TM == 224 && TN == 256 && !A_T), "the tiles that are generated");
+    constexpr int WM = TM == 256 ? 4 : 7, WN = TM == 256 ? TN / 64 : 2;
     using RA = TileOperand<A_T, TM>;
     using RB = TileOperand<B_T, TN>;
     constexpr int NSA = 3, NSB = TN == 256 ? 2 : 3, NLA = RA::PIECES / 4, NLB = RB::PIECES / 4, NL = NLA + NLB;
@@ -458,7 +461,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
     const int m0 = tm * TM, n0 = tn * TN;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
-    const int wm = wave & 1, wn = wave >> 1;
+    const int wm = TM == 256 ? wave & 1 : 0, wn = TM == 256 ? wave >> 1 : wave;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
     const int64_t lda = pr.lda[0], ldb = pr.ldb[0];
     const int st0 = (pr.K[0] + TK - 1) / TK, nst = st0 + (pr.nseg > 1 ? st0 : 0);      // both segments have one length
@@ -530,34 +533,44 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
     if constexpr (!F16) {
 #define LVX_GEMM_MFMA "v_mfma_f32_32x32x16_bf16"
 #define LVX_GEMM_CVT "v_cvt_pk_bf16_f32"
-        if constexpr (!A_T && !B_T && TN == 256) {
+        if constexpr (!A_T && !B_T && TN == 256 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_pp_256.inc"
+#include "lvx_gemm_loop_pp_256_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (!A_T && !B_T && TN == 128) {
+        else if constexpr (!A_T && !B_T && TN == 128 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_pp_128.inc"
+#include "lvx_gemm_loop_pp_128_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (!A_T && B_T && TN == 256) {
+        else if constexpr (!A_T && B_T && TN == 256 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_pt_256.inc"
+#include "lvx_gemm_loop_pt_256_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (!A_T && B_T && TN == 128) {
+        else if constexpr (!A_T && B_T && TN == 128 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_pt_128.inc"
+#include "lvx_gemm_loop_pt_128_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (A_T && B_T && TN == 256) {
+        else if constexpr (A_T && B_T && TN == 256 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_tt_256.inc"
+#include "lvx_gemm_loop_tt_256_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (A_T && B_T && TN == 128) {
+        else if constexpr (A_T && B_T && TN == 128 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_tt_128.inc"
+#include "lvx_gemm_loop_tt_128_256.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && B_T && TM == 224) {
+            asm volatile(
+#include "lvx_gemm_loop_pt_256_224.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && !B_T && TM == 224) {
+            asm volatile(
+#include "lvx_gemm_loop_pp_256_224.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
 #undef LVX_GEMM_MFMA
@@ -565,34 +578,44 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
     } else {
 #define LVX_GEMM_MFMA "v_mfma_f32_32x32x16_f16"
 #define LVX_GEMM_CVT "v_cvt_pk_f16_f32"
-        if constexpr (!A_T && !B_T && TN == 256) {
+        if constexpr (!A_T && !B_T && TN == 256 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_pp_256.inc"
+#include "lvx_gemm_loop_pp_256_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (!A_T && !B_T && TN == 128) {
+        else if constexpr (!A_T && !B_T && TN == 128 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_pp_128.inc"
+#include "lvx_gemm_loop_pp_128_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (!A_T && B_T && TN == 256) {
+        else if constexpr (!A_T && B_T && TN == 256 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_pt_256.inc"
+#include "lvx_gemm_loop_pt_256_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (!A_T && B_T && TN == 128) {
+        else if constexpr (!A_T && B_T && TN == 128 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_pt_128.inc"
+#include "lvx_gemm_loop_pt_128_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (A_T && B_T && TN == 256) {
+        else if constexpr (A_T && B_T && TN == 256 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_tt_256.inc"
+#include "lvx_gemm_loop_tt_256_256.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
-        else if constexpr (A_T && B_T && TN == 128) {
+        else if constexpr (A_T && B_T && TN == 128 && TM == 256) {
             asm volatile(
-#include "lvx_gemm_loop_tt_128.inc"
+#include "lvx_gemm_loop_tt_128_256.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && B_T && TM == 224) {
+            asm volatile(
+#include "lvx_gemm_loop_pt_256_224.inc"
+                LVX_GEMM_TILE_OPERANDS);
+        }
+        else if constexpr (!A_T && !B_T && TM == 224) {
+            asm volatile(
+#include "lvx_gemm_loop_pp_256_224.inc"
                 LVX_GEMM_TILE_OPERANDS);
         }
 #undef LVX_GEMM_MFMA
@@ -660,15 +683,16 @@ hipError_t launch_cfg(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t 
 }
 
 
-template <int TN, bool F16>
+template <int TN, bool F16, int TM = 256>
 hipError_t launch_tile(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t st) {
-    p.tiles_m = (p.M + 255) / 256;
+    p.tiles_m = (p.M + TM - 1) / TM;
     p.tiles_n = (p.N + TN - 1) / TN;
     p.total_wg = p.nprob * p.tiles_m * p.tiles_n;
     const dim3 grid((p.total_wg + 7) / 8 * 8);
-    if (!a_mcontig && !b_ncontig) return launch1((gemm_tile_kernel<false, false, TN, F16>), grid, dim3(256), st, p);
-    if (!a_mcontig) return launch1((gemm_tile_kernel<false, true, TN, F16>), grid, dim3(256), st, p);
-    return launch1((gemm_tile_kernel<true, true, TN, F16>), grid, dim3(256), st, p);
+    if (!a_mcontig && !b_ncontig) return launch1((gemm_tile_kernel<false, false, TN, F16, TM>), grid, dim3(256), st, p);
+    if (!a_mcontig) return launch1((gemm_tile_kernel<false, true, TN, F16, TM>), grid, dim3(256), st, p);
+    if constexpr (TM == 256) return launch1((gemm_tile_kernel<true, true, TN, F16, TM>), grid, dim3(256), st, p);
+    return hipErrorInvalidValue;
 }
 
 // What gemm_tile_kernel takes: no batch, one contraction length for both segments (whole stages of it where
@@ -687,9 +711,12 @@ bool gemm_tile_ok(const GemmParams& p, bool a_mcontig, bool b_ncontig) {
 }  // namespace
 
 // Work-group tile by shape.  C wider than 128 columns (projections, their gradients): the hand-scheduled tile
-// of 256 x 256, or 256 x 128 where that fills the chip's rounds better: a 128-wide tile takes about 0.6 of
+// of 256 x 256, or 256 x 128 or 224 x 256 where that fills the chip's rounds better: a 128-wide tile takes about 0.6 of
 // the time of a 256-wide one (2046 x 4096 x 4096: 128 tiles of 256 on 256 CUs 81 us, 256 of 128 60; 12808 x 4096 x
-// 1024 twice: 2 rounds 176 us, 4 rounds 208).
+// 1024 twice: 2 rounds 176 us, 4 rounds 208), one of 224 rows about 0.9 (an eighth less work, a quarter more LDS reads per
+// MFMA, and more CUs at work under the same power: 6404 x 4096 x 1024 twice 208 tiles 97 us, 232 lower ones 90; dX
+// 6404 x 4096 of 2 x 1024 416 tiles 108, 464 lower 100; a layer's K and V, 12808 x 4096 x 1024 twice with the norm, 408 tiles
+// 234, 464 lower 224).
 // A narrow C (the dQ GEMM): 256 x 128, four stages, at which one load of a wave covers whole cache lines of
 // dS^T's 64-byte rows (two tokens x 256 rows; of a 512-row tile it takes one token, half of each line, and the
 // streaming hint then costs a second fetch: 6404 tokens x 4096 rows x 32 heads 1868 us a step against 1821),
@@ -704,10 +731,11 @@ hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipS
     }
     if (p.N > 128 && gemm_tile_ok(p, a_mcontig, b_ncontig)) {
         const int n_cu = cu_count();
-        const int64_t rows = (p.M + 255) / 256 * (int64_t)p.nprob;
-        const int64_t wide = (rows * ((p.N + 255) / 256) + n_cu - 1) / n_cu, narrow = (rows * ((p.N + 127) / 128) + n_cu - 1) / n_cu;
-        const bool use_narrow = 10 * wide > 6 * narrow;
-        if (use_narrow) return p.f16 ? launch_tile<128, true>(p, a_mcontig, b_ncontig, st) : launch_tile<128, false>(p, a_mcontig, b_ncontig, st);
+        auto rounds = [&](int tm, int tn) { return ((p.M + tm - 1) / tm * (int64_t)p.nprob * ((p.N + tn - 1) / tn) + n_cu - 1) / n_cu; };
+        const int64_t wide = 10 * rounds(256, 256), narrow = 6 * rounds(256, 128), lower = a_mcontig ? INT64_MAX : 9 * rounds(224, 256);
+        if (lower < std::min(wide, narrow))
+            return p.f16 ? launch_tile<256, true, 224>(p, a_mcontig, b_ncontig, st) : launch_tile<256, false, 224>(p, a_mcontig, b_ncontig, st);
+        if (narrow < wide) return p.f16 ? launch_tile<128, true>(p, a_mcontig, b_ncontig, st) : launch_tile<128, false>(p, a_mcontig, b_ncontig, st);
         return p.f16 ? launch_tile<256, true>(p, a_mcontig, b_ncontig, st) : launch_tile<256, false>(p, a_mcontig, b_ncontig, st);
     }
     if (p.N > 128) return launch_cfg<2, 4, 4, 2, 4>(p, a_mcontig, b_ncontig, st);

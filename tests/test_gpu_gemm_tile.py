@@ -1,5 +1,5 @@
 """The hand-scheduled GEMM tile behind the projections and their gradients, against float64: contractions that end
-inside a 64-deep stage (and inside its first), rows and columns around one tile, both widths of the
+inside a 64-deep stage (and inside its first), rows and columns around one tile, all three sizes of the
 tile, both weight layouts and element types, with and without the norm."""
 import pytest
 import torch
@@ -8,13 +8,14 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# (rows, model width, heads, head_dim); the widths of C (heads x head_dim, or the model width for dX) above
-# 2048 with 2300 rows make the 256-wide tile the choice, the others the 128-wide one
+# (rows, model width, heads, head_dim).  On 256 CUs the tile is 224 x 256 for K and V of 6404 and 12700 rows and dX of
+# 2300 rows x 4104, 256 x 256 for K and V of 8190 rows and dX of 4090 x 4096, and 256 x 128 for the others
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("w_in_major", [True, False])
 @pytest.mark.parametrize("M,Dm,H,D", [(1, 136, 2, 128), (33, 64, 9, 32), (100, 1000, 3, 128), (255, 32, 2, 128),
                                       (257, 512, 4, 128), (300, 264, 10, 16), (1601, 72, 4, 128), (2300, 136, 32, 128),
-                                      (2300, 4104, 2, 128)])
+                                      (2300, 4104, 2, 128), (6404, 72, 8, 128), (12700, 32, 8, 128),
+                                      (8190, 136, 8, 128), (4090, 4096, 1, 128)])
 def test_projection_and_gradients(dtype, w_in_major, M, Dm, H, D):
     from lv_xattn import ops
     g = torch.Generator(device=DEV).manual_seed(M * 7 + Dm)
