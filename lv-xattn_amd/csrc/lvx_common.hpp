@@ -185,6 +185,21 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
     return r;
 }
 
+// Sum over aligned groups of 16 lanes, in every one of them: neighbours, pairs, quads and halves across (the mirrored
+// lanes of a group whose quads are uniform are the ones 4 and 8 away).  Four VALU instructions, where a shuffle is a
+// trip through LDS.
+template <int CTRL>
+__device__ __forceinline__ float lanes_moved(float x) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float sum16(float x) {
+    x += lanes_moved<0xb1>(x);      // quad_perm [1, 0, 3, 2]
+    x += lanes_moved<0x4e>(x);      // quad_perm [2, 3, 0, 1]
+    x += lanes_moved<0x141>(x);     // row_half_mirror
+    x += lanes_moved<0x140>(x);     // row_mirror
+    return x;
+}
+
 // Brings every 64-byte line of the kernel's arguments (BYTES of them, at most 512) into the scalar cache with one wait.  The
 // compiler loads an argument where it is needed, and a kernel that comes by five lines one after the other stands
 // still five times for the way to memory, 0.3 us each, before its first load of data leaves.

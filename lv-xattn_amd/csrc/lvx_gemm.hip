@@ -115,35 +115,29 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     constexpr int NRA = RA::NRD(WM), NRB = RB::NRD(WN);
     __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE];
 
+    fetch_kernargs<sizeof(GemmParams)>();
     const int wid0 = p.m_order ? (int)blockIdx.x : xcd_remap(blockIdx.x, p.total_wg);
     if (wid0 >= p.total_wg) return;
     const int nks = p.k_splits > 1 ? p.k_splits : 1;
-    const int ksp = wid0 % nks;
-    const int wid = wid0 / nks;
-    const int tn = wid % p.tiles_n;
-    const int t1 = wid / p.tiles_n;
-    int tm, z, t2 = 0;
+    uint32_t ksp, tn, tm, zo, zi, prob = 0;
+    const uint32_t t1 = p.by_tiles_n.split(p.by_splits.split(wid0, ksp), tn);
     if (p.m_order) {
         // M tiles with their own contraction ranges, ranked by length: the ids walk the ranking
         // (the inner batch index fastest), so the hardware's in-order hand-out of work-groups
         // starts the longest first, on every XCD alike
-        const int item = p.m_order[t1 / p.batch_inner];
-        tm = item % p.tiles_m;
-        z = (item / p.tiles_m) * p.batch_inner + t1 % p.batch_inner;
+        zo = p.by_tiles_m.split((uint32_t)p.m_order[p.by_inner.split(t1, zi)], tm);
     } else {
-        tm = t1 % p.tiles_m;
-        t2 = t1 / p.tiles_m;
         // the outer batch index (the sample, where there is one) varies fastest over the ids, so that
         // every XCD's contiguous id range holds work of all samples (ragged ones differ in length)
-        const int zr = t2 % p.nbatch;
-        const int n_outer = p.nbatch / p.batch_inner;
-        z = (zr % n_outer) * p.batch_inner + zr / n_outer;
+        uint32_t zr;
+        prob = p.by_nbatch.split(p.by_tiles_m.split(t1, tm), zr);
+        zi = p.by_outer.split(zr, zo);
     }
-    const GemmProblem& pr = p.prob[t2 / p.nbatch];
+    const GemmProblem& pr = p.prob[prob];
+    const int z = zo * p.batch_inner + zi;
     const int m0 = tm * TM, n0 = tn * TN;
-    const int zo = z / p.batch_inner, zi = z % p.batch_inner;
     const int64_t a_off = (int64_t)z * p.a_batch;
-    const int64_t b_off = zo * p.b_outer + (zi / p.b_group) * p.b_inner;
+    const int64_t b_off = zo * p.b_outer + p.by_group.quotient(zi) * p.b_inner;
     uint16_t* const Cz = pr.C + zo * p.c_outer + zi * p.c_inner;
     int klen0 = pr.K[0];
     if (p.k_len) klen0 = min(klen0, p.k_len[zo]);
@@ -330,7 +324,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
             }
         }
     };
-    if (p.norm_w && t2 / p.nbatch == 0) {
+    if (p.norm_w && prob == 0) {
         // RMS norm over each 128-column group (N and the tile are multiples of 128): the
         // group's columns sit in HW = 4 / WN waves with consecutive wn; row sums of squares
         // are exchanged through LDS, which no wave reads any more.
@@ -451,12 +445,13 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[NSA * RA::BYTES + NSB * RB::BYTES];
     static_assert(sizeof(lds) >= TM * TN * 2, "the C tile takes the stages' place");
 
+    fetch_kernargs<sizeof(GemmParams)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
     if (wid >= p.total_wg) return;
-    const int tn = wid % p.tiles_n, t1 = wid / p.tiles_n;
+    uint32_t tn, prob;
     // the problems of an M tile side by side: they share an operand (K and V the visual states), which then
     // is read from HBM once
-    const int prob = t1 % p.nprob, tm = t1 / p.nprob;
+    const int tm = p.by_nprob.split(p.by_tiles_n.split(wid, tn), prob);
     const GemmProblem& pr = p.prob[prob];
     const int m0 = tm * TM, n0 = tn * TN;
     const int tid = threadIdx.x;
@@ -634,15 +629,15 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
         if (((row >> 3) ^ (row >> 4)) & 1) val = u32x4{val[2], val[3], val[0], val[1]};
         const bool ok = m < p.M && n < p.N;
         if (norm) {
-            // RMS norm over the head's 128 columns, 16 lanes: y = rn(w * rn(x * r)), x the product as 16 bits
+            // RMS norm over the head's 128 columns, 16 lanes (summed by shuffles, K and V of 12808 rows with it took 224
+            // us; 221 so): y = rn(w * rn(x * r)), x the product as 16 bits
             float ss = 0.f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 ss = fmaf(E::lo(val[j]), E::lo(val[j]), ss);
                 ss = fmaf(E::hi(val[j]), E::hi(val[j]), ss);
             }
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o);
+            ss = sum16(ss);
             const float r = rsqrtf(ss * (1.f / 128.f) + p.norm_eps);
             if (ok && p.rstd && (cc & 15) == 0) p.rstd[(int64_t)m * (p.N >> 7) + (n >> 7)] = r;
             if (ok && p.c_raw) __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(p.c_raw + (int64_t)m * pr.ldc + n));
@@ -655,6 +650,23 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
         // (a streaming store: nobody on this CU reads the tile again)
         if (ok) __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(C + (int64_t)m * pr.ldc + n));
     }
+}
+
+// The tiles of a launch and the divisors by what its work-group numbers are made of.  (With the arguments fetched line by
+// line and eight integer divisions a work-group of a small dQ launch lost 0.6 us of 26 before its first load.)
+void fill_tiles(GemmParams& p, int TM, int TN) {
+    const int splits = p.k_splits > 1 ? p.k_splits : 1;
+    p.tiles_m = (p.M + TM - 1) / TM;
+    p.tiles_n = (p.N + TN - 1) / TN;
+    p.total_wg = p.nprob * p.nbatch * p.tiles_m * p.tiles_n * splits;
+    p.by_splits = divisor(splits);
+    p.by_tiles_n = divisor(p.tiles_n);
+    p.by_tiles_m = divisor(p.tiles_m);
+    p.by_nprob = divisor(p.nprob);
+    p.by_nbatch = divisor(p.nbatch);
+    p.by_inner = divisor(p.batch_inner);
+    p.by_outer = divisor(p.nbatch / p.batch_inner);
+    p.by_group = divisor(p.b_group);
 }
 
 template <int GM, int GN, int WM, int WN, int NS, bool F16>
@@ -673,10 +685,7 @@ hipError_t launch_cfg_t(const GemmParams& p, int grid, bool a_mcontig, bool b_nc
 
 template <int GM, int GN, int WM, int WN, int NS>
 hipError_t launch_cfg(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t st) {
-    constexpr int TM = 32 * WM * GM, TN = 32 * WN * GN;
-    p.tiles_m = (p.M + TM - 1) / TM;
-    p.tiles_n = (p.N + TN - 1) / TN;
-    p.total_wg = p.nprob * p.nbatch * p.tiles_m * p.tiles_n * (p.k_splits > 1 ? p.k_splits : 1);
+    fill_tiles(p, 32 * WM * GM, 32 * WN * GN);
     const int grid = ((p.total_wg + 7) / 8) * 8;
     if (p.f16) return launch_cfg_t<GM, GN, WM, WN, NS, true>(p, grid, a_mcontig, b_ncontig, st);
     return launch_cfg_t<GM, GN, WM, WN, NS, false>(p, grid, a_mcontig, b_ncontig, st);
@@ -685,9 +694,7 @@ hipError_t launch_cfg(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t 
 
 template <int TN, bool F16, int TM = 256>
 hipError_t launch_tile(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t st) {
-    p.tiles_m = (p.M + TM - 1) / TM;
-    p.tiles_n = (p.N + TN - 1) / TN;
-    p.total_wg = p.nprob * p.tiles_m * p.tiles_n;
+    fill_tiles(p, TM, TN);
     const dim3 grid((p.total_wg + 7) / 8 * 8);
     if (!a_mcontig && !b_ncontig) return launch1((gemm_tile_kernel<false, false, TN, F16, TM>), grid, dim3(256), st, p);
     if (!a_mcontig) return launch1((gemm_tile_kernel<false, true, TN, F16, TM>), grid, dim3(256), st, p);

@@ -290,6 +290,8 @@ struct GemmParams {
     // a_tiled_m of them per block of 128 k; lda is ignored
     int a_tiled_m;
     int a_stream;              // 1: A is loaded with the streaming hint (A and B stored [K][..] only)
+    // filled in by launch_gemm: divisors by k_splits, tiles_n, tiles_m, nprob, nbatch, batch_inner, their quotient, b_group
+    Divisor by_splits, by_tiles_n, by_tiles_m, by_nprob, by_nbatch, by_inner, by_outer, by_group;
 };
 
 hipError_t launch_fwd(const FwdParams& p, bool masked, hipStream_t st);   // p.bias selects the bias variant

@@ -622,9 +622,7 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_bwd_kernel(const NormBwdPar
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) c = fmaf(gg[j], xh[j], c);
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) c += __shfl_xor(c, o);
-            c *= 1.f / 128.f;
+            c = sum16(c) * (1.f / 128.f);
             u32x4 u;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
