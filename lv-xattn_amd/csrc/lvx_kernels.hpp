@@ -91,7 +91,8 @@ struct MergeParams {
     int f16;
     int D;                     // head dimension: 16, 32, 64 or 128 (0 reads as 128)
     int part_f32;              // 1: the parts are fp32 (not for one part folded into an accumulator)
-    Divisor by_rows, by_Hq;    // filled in by launch_merge: rows of the window, q heads
+    Divisor by_rows, by_Hq, by_B;   // filled in by launch_merge: rows of the window, q heads, samples
+    uint32_t blocks_per_xcd;        // and a share of the grid
 };
 
 // Per text row the hull of the keys a dense bias leaves visible (entries other than -inf).
@@ -230,7 +231,8 @@ struct CastParams {
     int64_t sum_stride;   // sum_stride floats apart
     int f16;          // destination type: 0 bf16, 1 fp16
     int D;            // head dimension: 16, 32, 64 or 128 (0 reads as 128)
-    Divisor by_L, by_H;    // filled in by launch_cast
+    Divisor by_L, by_H, by_B;       // filled in by launch_cast
+    uint32_t blocks_per_xcd;        // and a share of the grid
 };
 
 // One GEMM problem C[M,N] = sum over segments A_s[M,K_s] * B_s[K_s,N].
