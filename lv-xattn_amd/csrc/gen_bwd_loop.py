@@ -174,17 +174,17 @@ def p_read_op(st, u, n):
 
 
 def p_fetch(u, ahead):
-    """Request of tile i + ahead by a P-wave in step u, and the walk to the tile after it."""
+    """Request of tile i + ahead by a P-wave in step u, and the walk to the tile after it.  A load to LDS needs a
+    wait state behind the write of M0: a part of the walk, which for Q and the metadata is over by then."""
     sl_f = (u + 3 + ahead) % 6
     ws_new = 66 + 2 * sl_f
-    f = [["s_cmp_eq_u32 s65, 0", f"s_cbranch_scc1 LVX_BWD_NOMETA{u}{ahead}_%=", f"s_add_i32 m0, s63, {sl_f * META_SZ}",
+    f = [[f"s_add_i32 m0, s63, {sl_f * META_SZ}", "s_cmp_eq_u32 s65, 0", f"s_cbranch_scc1 LVX_BWD_NOMETA{u}{ahead}_%=",
           f"global_load_lds_dword v{G_META}, s[48:49]", f"LVX_BWD_NOMETA{u}{ahead}_%=:"]]
+    walk = [[f"s_mov_b64 {sr(ws_new, 2)}, s[50:51]"], ["s_add_u32 s50, s50, 8192", "s_addc_u32 s51, s51, 0"],
+            ["s_add_u32 s48, s48, s85", "s_addc_u32 s49, s49, 0"], ["s_add_u32 s44, s44, s41", "s_addc_u32 s45, s45, 0"]]
     for n, (base, src) in enumerate(((0, "s[44:45]"), (1024, "s[44:45]"), (DO_RING, "s[46:47]"), (DO_RING + 1024, "s[46:47]"))):
-        f.append(f"s_add_i32 m0, s62, {sl_f * TILE_B + base}")
-        f.append(f"global_load_lds_dwordx4 v{G_DMA + n}, {src}")
-    f.append(f"s_mov_b64 {sr(ws_new, 2)}, s[50:51]")
-    f += ["s_add_u32 s44, s44, s41", "s_addc_u32 s45, s45, 0", "s_add_u32 s46, s46, s42", "s_addc_u32 s47, s47, 0",
-          "s_add_u32 s48, s48, s85", "s_addc_u32 s49, s49, 0", "s_add_u32 s50, s50, 8192", "s_addc_u32 s51, s51, 0",
+        f += [f"s_add_i32 m0, s62, {sl_f * TILE_B + base}", *walk[n], f"global_load_lds_dwordx4 v{G_DMA + n}, {src}"]
+    f += ["s_add_u32 s46, s46, s42", "s_addc_u32 s47, s47, 0",
           ["s_sub_i32 s52, s52, 1", "s_cmp_lg_u32 s52, 0", f"s_cbranch_scc1 LVX_BWD_SAMEHEAD{u}{ahead}_%=",
            "s_add_u32 s44, s44, s54", "s_addc_u32 s45, s45, s55", "s_add_u32 s46, s46, s56", "s_addc_u32 s47, s47, s57",
            "s_add_u32 s48, s48, s80", "s_addc_u32 s49, s49, s81",
@@ -445,6 +445,10 @@ def check(ins):
             kind, rd = "vmem", regs(toks[0]) | regs(toks[1])
         elif op.startswith("global_load_lds"):
             kind, rd = "vmem", regs(toks[0])
+            if hist and hist[-1][0] == "m0":
+                raise SystemExit(f"hazard: {line} right behind the write of M0")
+        elif toks and toks[0] == "m0":
+            kind = "m0"
         dist = 0
         for pk, pw, pwt in reversed(hist):
             if pk == "mfma" and kind != "mfma" and (pw & (rd | wr)) and dist < 14:
@@ -472,7 +476,9 @@ def main():
         body += [x for x in ins if x is not None]
     check(body + body)
     cnt = "s64"
-    lines = (p_prologue() if ROLE == "p" else d_prologue()) + ["LVX_BWD_LOOP_%=:"] + body + [f"s_sub_i32 {cnt}, {cnt}, 1", f"s_cmp_lg_u32 {cnt}, 0", "s_cbranch_scc1 LVX_BWD_LOOP_%=",
+    prologue = p_prologue() if ROLE == "p" else d_prologue()
+    check(prologue)
+    lines = prologue + ["LVX_BWD_LOOP_%=:"] + body + [f"s_sub_i32 {cnt}, {cnt}, 1", f"s_cmp_lg_u32 {cnt}, 0", "s_cbranch_scc1 LVX_BWD_LOOP_%=",
                                            "s_waitcnt lgkmcnt(0)", "s_nop 15", "s_nop 3"]
     if ROLE == "p":
         lines += ["s_branch LVX_BWD_END_%="] + p_ragged(0, 2)

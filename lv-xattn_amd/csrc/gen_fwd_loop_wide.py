@@ -241,11 +241,12 @@ def advance(left, lo, hi, stride, offs, limit):
             f"LVX_FWDW_STAY{n}_%=:"]
 
 
-def request(offs, base, lds):
-    """This wave's pieces of a tile, into the buffer at byte `lds` of the tile buffers."""
+def request(offs, base, lds, between):
+    """This wave's pieces of a tile, into the buffer at byte `lds` of the tile buffers.  A load to LDS needs a wait
+    state behind the write of M0: an instruction taken from `between`."""
     out = []
     for j in range(NLD):
-        out += [f"s_add_i32 m0, s50, {lds + j * 4096}", f"global_load_lds_dwordx4 v{offs + j}, {base}"]
+        out += [f"s_add_i32 m0, s50, {lds + j * 4096}", between.pop(0), f"global_load_lds_dwordx4 v{offs + j}, {base}"]
     return out
 
 
@@ -335,11 +336,12 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
                 e(f"{MFMA} {ar(a, 16)}, {vr(slot, 4)}, {vr(PB[b] + 4 * j, 4)}, {ar(a, 16)}")
             n_mfma += 1
             if b == NB - 1:
-                if i + AHEAD < len(ops):
-                    read_op(ops[i + AHEAD])
-                if dma and k < NS and k % 2 == 1:
-                    x, y = dma[k // 2]
+                x, y = dma[k // 2] if dma and k < NS and k % 2 == 1 else (None, None)
+                if x:
                     e(x)
+                if i + AHEAD < len(ops):        # between the write of M0 and the load: its wait state
+                    read_op(ops[i + AHEAD])
+                if y:
                     e(y)
                 if do_dma and k == NS - 1:
                     e(advance("s57", "s44", "s45", "s48", DOK, "s64"))
@@ -407,6 +409,10 @@ def check(ins):
         elif op.startswith("global_load_lds"):
             kind = "vmem"
             rd = regs(toks[0])
+            if hist and hist[-1][0] == "m0":
+                raise SystemExit(f"hazard: {line} right behind the write of M0")
+        elif toks and toks[0] == "m0":
+            kind = "m0"
         dist = 0
         for pk, pw, pwt in reversed(hist):
             if pk == "mfma" and kind != "mfma" and (pw & (rd | wr)) and dist < 14:
@@ -426,15 +432,15 @@ def check(ins):
 def main():
     # Entry.  What the first scores need is requested first, K(0) and Q^T - Q^T straight into the accumulation
     # registers it lives in - then V(0) and K(1), which the wait leaves in flight.  O^T starts at 0 meanwhile.
-    pro = request(DOK, "s[44:45]", 0) + advance("s57", "s44", "s45", "s48", DOK, "s64")
+    zero = [f"v_accvgpr_write_b32 a{AACC[b] + r}, 0" for b in range(NB) for r in range(16 * NDT)]
+    pro = request(DOK, "s[44:45]", 0, zero) + advance("s57", "s44", "s45", "s48", DOK, "s64")
     for b in range(NB):
         for kk in range(NKK):
             pro.append(f"global_load_dwordx4 {ar(AQ[b] + 4 * kk, 4)}, {vr(128 + 2 * b, 2)}, off offset:{32 * kk}")
-    pro += request(DOV, "s[46:47]", TILE) + advance("s62", "s46", "s47", "s49", DOV, "s65")
-    pro += request(DOK, "s[44:45]", 2 * TILE) + advance("s57", "s44", "s45", "s48", DOK, "s64")
+    pro += request(DOV, "s[46:47]", TILE, zero) + advance("s62", "s46", "s47", "s49", DOV, "s65")
+    pro += request(DOK, "s[44:45]", 2 * TILE, zero) + advance("s57", "s44", "s45", "s48", DOK, "s64")
+    pro += zero
     for b in range(NB):
-        for r in range(16 * NDT):
-            pro.append(f"v_accvgpr_write_b32 a{AACC[b] + r}, 0")
         pro += [f"v_mov_b32 v{MI[b]}, s41", f"v_mov_b32 v{LI[b]}, 0", f"v_mov_b32 v{NMC[b]}, 0"]
     pro += [f"s_waitcnt vmcnt({2 * NLD})", "s_barrier"]
     # scores of the first tile (from K buffer 0 into score set A: the S phase of an odd tile)

@@ -88,7 +88,8 @@ def reads(u, kk, s):
 
 
 def request(which, u):
-    """This wave's pieces of A or B of stage u, the next one to be requested."""
+    """This wave's pieces of A or B of stage u, the next one to be requested: the write of M0 and the load, which
+    needs a wait state behind it."""
     out = []
     for j in range(NLA if which == "a" else NLB):
         if which == "a":
@@ -120,7 +121,8 @@ def advance(which):
 
 
 def kstep(s, rd, rq, tail):
-    """The MFMAs of operand set s with the reads `rd` and requests `rq` between them."""
+    """The MFMAs of operand set s with the reads `rd` and requests `rq` between them; M0 is written before an MFMA
+    and the load follows behind it."""
     out = []
     n = WM * WN
     rd, rq = list(rd), list(rq)
@@ -130,11 +132,15 @@ def kstep(s, rd, rq, tail):
     for nt in range(WN):
         for mt in range(WM):
             a = 16 * (WM * nt + mt)
+            loads = []
+            for _ in range(nq * (k + 1) // n - nq * k // n):
+                m0, load = rq.pop(0)
+                loads += [load] if not loads else [m0, "s_nop 0", load]
+                out += [m0] if len(loads) == 1 else []
             out.append(f"{MFMA} {ar(a, 16)}, {vr(bn(s, nt), 4)}, {vr(am(s, mt), 4)}, {ar(a, 16)}")
             for _ in range(nr * min(k + 1, span) // span - nr * min(k, span) // span):
                 out.append(rd.pop(0))
-            for _ in range(nq * (k + 1) // n - nq * k // n):
-                out += rq.pop(0)
+            out += loads
             k += 1
     assert not rd and not rq
     return out + tail
@@ -154,10 +160,13 @@ def stage(u):
 
 def main():
     lines = []
+    zero = [f"v_accvgpr_write_b32 a{r}, 0" for r in range(16 * WM * WN)]
     for u in range(NSB):            # B of stages 0 .. NSB - 1, A of stages 0 and 1
         for which in ("a", "b") if u < 2 else ("b",):
-            lines += sum(request(which, u), []) + advance(which)
-    lines += [f"v_accvgpr_write_b32 a{r}, 0" for r in range(16 * WM * WN)]
+            for m0, load in request(which, u):
+                lines += [m0, zero.pop(0), load]
+            lines += advance(which)
+    lines += zero
     lines += [f"s_waitcnt vmcnt({NL + (NLB if NSB == 3 else 0)})", "s_barrier"] + reads(0, 0, 0)
     lines += ["LVX_GEMM_LOOP_%=:"]
     for u in range(UNROLL):
@@ -182,6 +191,9 @@ def main():
                     lines += [f"{CVT} v{t}, v{t}, v{t + 1}", f"{CVT} v{t + 1}, v{t + 2}, v{t + 3}",
                               f"ds_write_b64 v{EPA + 4 * nt + vg}, {vr(t, 2)} offset:{(mt - m0) * 32 * TN * 2}"]
     lines += ["s_waitcnt lgkmcnt(0)"]
+    for x, y in zip(lines, lines[1:]):
+        if x.startswith("s_add_i32 m0") and y.startswith("buffer_load"):
+            raise SystemExit(f"hazard: {y} right behind the write of M0")
     if "nodma" in OPTS:
         lines = [l for l in lines if not l.startswith("buffer_load") and not l.startswith("s_add_i32 m0")]
     if "nolds" in OPTS:

@@ -111,6 +111,18 @@ def mfma_results_touched_early(body):
     return found
 
 
+def to_lds(ins):
+    """Is this a load straight to LDS?"""
+    return ins.op.startswith(("global_load", "buffer_load", "scratch_load")) and ("_lds_" in ins.op or "lds" in ins.args[-1].split(" "))
+
+
+def m0_used_early(body):
+    """[(write, load)]: loads to LDS with no wait state between them and a scalar write of M0, on some path."""
+    successors = after(body, {ins.addr: i for i, ins in enumerate(body)})
+    return [(ins, body[j]) for i, ins in enumerate(body) if ins.op.startswith("s_") and ins.args[0] == "m0"
+            for j in successors(i) if to_lds(body[j])]
+
+
 def loads_touched_early(body):
     """[(load, instruction)]: instructions that touch the destination of a load to registers on a path that has
     not come by any wait for loads yet: what a compiler would do with registers that inline assembly
@@ -119,8 +131,7 @@ def loads_touched_early(body):
     successors = after(body, index)
     found = []
     for i, ins in enumerate(body):
-        to_lds = "_lds_" in ins.op or ins.args[-1].split(" ")[-1] == "lds"
-        if not ins.op.startswith(("global_load", "buffer_load", "scratch_load", "flat_load")) or to_lds:
+        if not ins.op.startswith(("global_load", "buffer_load", "scratch_load", "flat_load")) or to_lds(ins):
             continue
         result = regs(ins.args[0])
         seen = set()

@@ -24,6 +24,13 @@ def test_mfma_results_have_their_wait_states(kernels):
 
 
 @needs_objdump
+def test_loads_to_lds_wait_for_m0(kernels):
+    assert sum(any(isa.to_lds(i) for i in body) for body in kernels.values()) > 50
+    early = {name: found for name, found in ((n, isa.m0_used_early(b)) for n, b in kernels.items()) if found}
+    assert not early, (len(early), {name: found[:2] for name, found in list(early.items())[:4]})
+
+
+@needs_objdump
 def test_registers_that_assembly_loads_are_left_alone_until_the_wait(kernels):
     """fwd_few_kernel requests Q by inline assembly long before it waits for it: no path of the built code may copy,
     spill or use those registers in between."""
@@ -68,3 +75,12 @@ def test_a_copy_of_a_register_in_flight_is_found():
     assert sorted(x[1].op for x in isa.loads_touched_early(body)) == ["v_max3_f32", "v_mov_b32"]
     (body,) = isa.parse(text.replace("s_nop 11 ", "s_waitcnt vmcnt(0) ").replace("v5, v6", "v8, v9")).values()
     assert not isa.loads_touched_early(body)
+
+
+def test_a_load_to_lds_right_behind_m0_is_found():
+    text = PLANTED.replace("v_mov_b32_e32 v4, 0  ", "s_add_i32 m0, s50, 0x400  ")
+    for load in ("global_load_lds_dwordx4 v8, s[4:5] offset:16  ", "buffer_load_dwordx4 v8, s[4:7], s9 offen lds  "):
+        (body,) = isa.parse(text.replace("v_max3_f32 v2, v30, v5, v6  ", load)).values()
+        assert [x[1].addr for x in isa.m0_used_early(body)] == [0x1014]
+        (body,) = isa.parse(text.replace("s_nop 11  ", load)).values()       # before the write, a branch over it
+        assert not isa.m0_used_early(body)
