@@ -264,6 +264,8 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     // carry reaches a result).  Wave 0 also fetches the tile's metadata record
     // (32 x LSE*log2e, 32 x delta*scale; 256 bytes) and, with an interval mask, waves
     // 1 and 2 the rows' first and last keys, ahead of their tile loads so that "tile landed" implies both.
+    // more scalars than registers (see dma16); the second load of an address finds it settled
+    constexpr bool RESTORED = MASKED && BIAS;
     auto prefetch = [&](int buf) {
         const int r0 = p.row_begin + cur_qt * BM;
         if (wave < META_WAVES) {
@@ -273,14 +275,14 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                 src = reinterpret_cast<const char*>((wave == 1 ? p.kv_start : p.kv_end) + (int64_t)b * p.Lq + r0);
                 off = (uint32_t)min(l32, p.row_end - 1 - r0) * 4u;
             }
-            dma4(src, off, meta0 + (uint32_t)buf * META_B + (uint32_t)wave * 256u);
+            dma4<RESTORED>(src, off, meta0 + (uint32_t)buf * META_B + (uint32_t)wave * 256u);
         }
         const uint32_t row0 = (uint32_t)min(r0 + ld_r, p.row_end - 1);
         const uint32_t row1 = (uint32_t)min(r0 + ld_r + 4, p.row_end - 1);
         const uint32_t slot = lds0 + (uint32_t)buf * (TILE_ELEMS * 2) + (uint32_t)slice * 2048u;
-        dma16(q_head, row0 * qrow_b + ld_c0, slot);
+        dma16<RESTORED>(q_head, row0 * qrow_b + ld_c0, slot);
         dma16(q_head, row1 * qrow_b + ld_c1, slot + 1024);
-        dma16(do_head, row0 * dorow_b + ld_c0, slot + OFF_DO * 2);
+        dma16<RESTORED>(do_head, row0 * dorow_b + ld_c0, slot + OFF_DO * 2);
         dma16(do_head, row1 * dorow_b + ld_c1, slot + OFF_DO * 2 + 1024);
     };
     auto advance = [&]() {   // next (head, row tile) of the walk, wrapping

@@ -131,9 +131,12 @@ __device__ __forceinline__ bf16x8 lds_operand_tr(const uint16_t* p, int half_off
 
 // 64 lanes x 16 bytes from global memory to the 1 KiB of LDS at byte address
 // lds_byte (wave-uniform); lane i lands at lds_byte + 16 i.  Counted by vmcnt.  A load to LDS may not follow the scalar
-// write of M0 it depends on without a wait state between them, which the compiler does not add inside assembly.
+// write of M0 it depends on without a wait state between them, which the compiler does not add inside assembly.  Nor does
+// it add those that a memory instruction needs behind the VALU instruction that wrote its scalar address, five:
+// RESTORED is for kernels that keep scalars in lanes of a vector register, from where v_readlane brings them back.
+template <bool RESTORED = false>
 __device__ __forceinline__ void dma16(const char* sbase, uint32_t voff, uint32_t lds_byte) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte), "v"(voff), "s"(sbase)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop %3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte), "v"(voff), "s"(sbase), "n"(RESTORED ? 3 : 0)
                  : "memory", "m0");
 }
 // the same, not kept in the caches: for what nobody reads again
@@ -145,8 +148,9 @@ __device__ __forceinline__ void dma16_addr(const char* addr, uint32_t lds_byte) 
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_byte), "v"(addr) : "memory", "m0");
 }
 // the same with 4 bytes per lane: lane i lands at lds_byte + 4 i
+template <bool RESTORED = false>
 __device__ __forceinline__ void dma4(const char* sbase, uint32_t voff, uint32_t lds_byte) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_byte), "v"(voff), "s"(sbase)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop %3\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_byte), "v"(voff), "s"(sbase), "n"(RESTORED ? 3 : 0)
                  : "memory", "m0");
 }
 template <int N>

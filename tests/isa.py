@@ -8,6 +8,9 @@ import subprocess
 
 OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
 
+# Wait states between a VALU instruction that writes a scalar register and a memory instruction that reads it
+SCALAR_WAIT = 5
+
 # Wait states between a 32x32x16 MFMA (8 passes) and whatever else touches its result: passes + 4 on gfx950
 MFMA_WAIT = 12
 
@@ -121,6 +124,41 @@ def m0_used_early(body):
     successors = after(body, {ins.addr: i for i, ins in enumerate(body)})
     return [(ins, body[j]) for i, ins in enumerate(body) if ins.op.startswith("s_") and ins.args[0] == "m0"
             for j in successors(i) if to_lds(body[j])]
+
+
+def scalars(arg):
+    """Numbers of the scalar registers an operand names ("vcc": that pair)."""
+    arg = arg.split(" ")[0]
+    m = re.match(r"s\[(\d+):(\d+)\]$", arg) or re.match(r"s(\d+)()$", arg)
+    return set(range(int(m.group(1)), int(m.group(2) or m.group(1)) + 1)) if m else {arg} & {"vcc"}
+
+
+def scalars_used_early(body):
+    """[(write, instruction, wait states)]: memory instructions that read a scalar register fewer than SCALAR_WAIT wait
+    states behind the VALU instruction that wrote it - a spilled scalar coming back from a lane, mostly -
+    on some path."""
+    successors = after(body, {ins.addr: i for i, ins in enumerate(body)})
+    found = []
+    for i, ins in enumerate(body):
+        if not ins.op.startswith(("v_readlane", "v_readfirstlane", "v_cmp_")):
+            continue
+        written = scalars(ins.args[0])
+        best = {}
+        todo = [(n, 0, written) for n in successors(i)]
+        while todo:
+            j, waited, left = todo.pop()
+            if waited >= SCALAR_WAIT or best.get(j, SCALAR_WAIT) <= waited:
+                continue
+            best[j] = waited
+            x = body[j]
+            if x.op.startswith(("global_", "buffer_", "scratch_", "flat_")):
+                if set().union(*(scalars(a) for a in x.args)) & left:
+                    found.append((ins, x, waited))
+            elif x.op.startswith("s_"):
+                left = left - scalars(x.args[0])        # a scalar write needs no wait
+            step = int(x.args[0], 0) + 1 if x.op == "s_nop" else 1
+            todo += [(n, waited + step, left) for n in successors(j)]
+    return found
 
 
 def loads_touched_early(body):

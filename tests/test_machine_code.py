@@ -31,6 +31,12 @@ def test_loads_to_lds_wait_for_m0(kernels):
 
 
 @needs_objdump
+def test_addresses_that_come_out_of_lanes_have_their_wait_states(kernels):
+    early = {name: found for name, found in ((n, isa.scalars_used_early(b)) for n, b in kernels.items()) if found}
+    assert not early, {name: found[:2] for name, found in early.items()}
+
+
+@needs_objdump
 def test_registers_that_assembly_loads_are_left_alone_until_the_wait(kernels):
     """fwd_few_kernel requests Q by inline assembly long before it waits for it: no path of the built code may copy,
     spill or use those registers in between."""
@@ -84,3 +90,13 @@ def test_a_load_to_lds_right_behind_m0_is_found():
         assert [x[1].addr for x in isa.m0_used_early(body)] == [0x1014]
         (body,) = isa.parse(text.replace("s_nop 11  ", load)).values()       # before the write, a branch over it
         assert not isa.m0_used_early(body)
+
+
+def test_an_address_right_out_of_a_lane_is_found():
+    text = PLANTED.replace("v_mfma_f32_32x32x16_bf16 v[4:19], v[20:23], v[82:85], 0  ", "v_readlane_b32 s5, v30, 7  ")
+    text = text.replace("v_max3_f32 v2, v30, v5, v6  ", "global_load_lds_dwordx4 v8, s[4:5]  ")
+    (body,) = isa.parse(text).values()
+    (found,) = isa.scalars_used_early(body)
+    assert found[1].addr == 0x1014 and found[2] == 1
+    (body,) = isa.parse(text.replace("s_cbranch_vccnz 2  ", "s_nop 4  ")).values()
+    assert not isa.scalars_used_early(body)
