@@ -614,7 +614,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     if (p.o_f32) {
         constexpr int CPF = DH / 4, RPS = 64 / CPF;              // chunks of a row of floats, rows per store
         float* const ob = reinterpret_cast<float*>(p.o) + o_head;
-        const uint32_t oo = (uint32_t)(lane / CPF) * (uint32_t)p.os.s + (uint32_t)(lane % CPF) * 4u;
+        const uint32_t oo = (uint32_t)(lane / CPF) * (uint32_t)p.os.s + (uint32_t)(lane % CPF) * 4u;    // a workspace's stride: DH
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
 #pragma unroll
@@ -658,13 +658,12 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
         u32x4 x[CPR];
 #pragma unroll
         for (int i = 0; i < CPR; ++i) x[i] = *reinterpret_cast<const u32x4*>(ep + (lane / CPR) * EP16 + (lane % CPR) * 16 + i * (RPL * EP16));
-        uint16_t* const ob = p.o + o_head;
-        const uint32_t oo = (uint32_t)(lane / CPR) * (uint32_t)p.os.s + (uint32_t)(lane % CPR) * 8u;
+        uint16_t* const ob = p.o + o_head + (lane / CPR) * p.os.s + (lane % CPR) * 8;       // a caller's stride: 64 bits
         auto store = [&](bool all) {
 #pragma unroll
             for (int i = 0; i < CPR; ++i) {
                 const u32x4 y = (i * RPL >> 4) & 1 ? u32x4{x[i][2], x[i][3], x[i][0], x[i][1]} : x[i];
-                if (all || i * RPL + lane / CPR < rows) *reinterpret_cast<u32x4*>(ob + i * RPL * p.os.s + oo) = y;
+                if (all || i * RPL + lane / CPR < rows) *reinterpret_cast<u32x4*>(ob + i * RPL * p.os.s) = y;
             }
         };
         if (rows >= 64) store(true);

@@ -187,3 +187,21 @@ def test_a_nan_is_not_lost_between_key_splits(form, D, kind, splits, key, monkey
                                kv_splits=splits, **bias_args)[3].cpu()
     assert torch.equal(o.isnan().all(-1), nan) and torch.equal(o.isnan().any(-1), nan)
     check_o(o[~nan], o_ref[~nan])
+
+
+# rows of O further apart than 32 bits of elements reach over the rows that one store instruction covers (eight with
+# heads of 64, four with heads of 128): 8.6 GB, of which only the rows are touched
+@pytest.mark.parametrize("D,Lq", [(64, 8), (128, 4)])
+def test_wide_form_with_rows_far_apart(D, Lq, monkeypatch):
+    from lv_xattn import ops
+    monkeypatch.setenv("LVX_FWD_WIDE", "1")
+    g = torch.Generator(device=DEV).manual_seed(D)
+    q, k, v = (torch.empty(1, 4, n, D, device=DEV, dtype=torch.bfloat16).normal_(generator=g) for n in (Lq, 100, 100))
+    stride = (2 ** 32 // (Lq - 1) + 4 * D + 8) // 8 * 8
+    assert (Lq - 1) * stride > 2 ** 32
+    far = torch.empty((Lq - 1) * stride + 4 * D, device=DEV, dtype=torch.bfloat16).as_strided((1, 4, Lq, D), (0, D, stride, 1))
+    near, lse = torch.empty_like(q), torch.empty(4, Lq, device=DEV)
+    for o in (near, far):
+        ops.fwd(q, k[:, :1], v[:, :1], o, lse, D ** -0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(near, far)
