@@ -14,6 +14,9 @@ SCALAR_WAIT = 5
 # Wait states between a 32x32x16 MFMA (8 passes) and whatever else touches its result: passes + 4 on gfx950
 MFMA_WAIT = 12
 
+MEMORY = ("global_", "buffer_", "scratch_", "flat_")
+LOADS = tuple(m + "load" for m in MEMORY)
+
 
 class Ins:
     __slots__ = ("addr", "op", "args", "target")
@@ -151,7 +154,7 @@ def scalars_used_early(body):
                 continue
             best[j] = waited
             x = body[j]
-            if x.op.startswith(("global_", "buffer_", "scratch_", "flat_")):
+            if x.op.startswith(MEMORY):
                 if set().union(*(scalars(a) for a in x.args)) & left:
                     found.append((ins, x, waited))
             elif x.op.startswith("s_"):
@@ -161,29 +164,37 @@ def scalars_used_early(body):
     return found
 
 
-def loads_touched_early(body):
+def waits_for(ins):
+    """How many of the youngest memory operations an instruction leaves in flight; None when it waits for none."""
+    m = re.search(r"vmcnt\((\d+)\)", " ".join(ins.args)) if ins.op == "s_waitcnt" else None
+    return int(m.group(1)) if m else None
+
+
+def loads_touched_early(body, stated=()):
     """[(load, instruction)]: instructions that touch the destination of a load to registers on a path that has
-    not come by any wait for loads yet: what a compiler would do with registers that inline assembly
-    requested, if it copied or spilled them."""
+    not come by a wait for it yet: what a compiler would do with registers that inline assembly requested, if
+    it copied or spilled them.  Operations complete in order, so a wait that leaves n in flight is one for this load
+    when at least n were issued behind it.  `stated`: waits that are taken for one whatever the path."""
     index = {ins.addr: i for i, ins in enumerate(body)}
     successors = after(body, index)
     found = []
     for i, ins in enumerate(body):
-        if not ins.op.startswith(("global_load", "buffer_load", "scratch_load", "flat_load")) or to_lds(ins):
+        if not ins.op.startswith(LOADS) or to_lds(ins):
             continue
         result = regs(ins.args[0])
-        seen = set()
-        todo = list(successors(i))
+        fewest = {}                 # operations issued behind the load, on the path that has the fewest
+        todo = [(n, 0) for n in successors(i)]
         while todo:
-            j = todo.pop()
-            if j in seen:
+            j, younger = todo.pop()
+            if fewest.get(j, younger + 1) <= younger:
                 continue
-            seen.add(j)
+            fewest[j] = younger
             x = body[j]
-            if x.op == "s_waitcnt" and "vmcnt" in " ".join(x.args):
+            left = waits_for(x)
+            if left is not None and (left <= younger or x in stated):
                 continue
             if touched(x) & result:
                 found.append((ins, x))
                 continue
-            todo += successors(j)
+            todo += [(n, younger + x.op.startswith(MEMORY)) for n in successors(j)]
     return found
