@@ -307,50 +307,53 @@ __global__ __launch_bounds__(256) void bwd_meta_kernel(const MetaParams p) {
     o[32] = d * p.scale;
 }
 
-// First and one-past-last key of a set that the threads of a work-group of 256 have each seen a part of.
-__device__ __forceinline__ void block_hull(int& lo, int& hi) {
-    __shared__ int red[4][2];
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        lo = min(lo, __shfl_xor(lo, o));
-        hi = max(hi, __shfl_xor(hi, o));
-    }
-    if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6][0] = lo; red[threadIdx.x >> 6][1] = hi; }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < 4; ++w) { lo = min(lo, red[w][0]); hi = max(hi, red[w][1]); }
-}
-
-// One work-group per (b, text row): first and one-past-last key whose bias is not -inf, over all heads the bias
-// distinguishes.  An empty row gets (0, 0).  Bound by reading the bias once: four loads of 16 bytes per thread in flight
-// (1024 rows x 4096 keys, 16.8 MB: 5.0 us; one wave per row, a load at a time, 8.7).
+// Per (b, text row) the first and one-past-last key whose bias is not -inf, over all heads the bias distinguishes.  An
+// empty row gets (0, 0).  WAVES: waves that share a row, 1 or 4; BATCH: loads of 16 bytes a thread has in flight (see
+// launch_bias_hull).  Bound by reading the bias once.
+template <int WAVES, int BATCH>
 __global__ __launch_bounds__(256) void bias_hull_kernel(const BiasHullParams p) {
+    constexpr int STEP = 4 * 64 * WAVES;                    // keys one load of the waves covers
     fetch_kernargs<sizeof(BiasHullParams)>();
-    for (uint32_t rw = blockIdx.x; rw < (uint32_t)(p.B * p.Lq); rw += gridDim.x) {
+    const uint32_t rows = (uint32_t)p.B * (uint32_t)p.Lq, wave = uniform32(threadIdx.x >> 6);
+    const int lane = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
+    for (uint32_t rw = WAVES == 1 ? blockIdx.x * 4 + wave : blockIdx.x; rw < rows; rw += gridDim.x * (4 / WAVES)) {
         uint32_t row;
         const uint32_t b = p.by_Lq.split(rw, row);
         int lo = INT_MAX, hi = 0;
         for (int h = 0; h < p.heads; ++h) {
             const float* br = p.bias + b * p.bias_b + h * p.bias_h + (int64_t)row * p.bias_r;
-            for (int k0 = 4 * (int)threadIdx.x; k0 < p.Lkv; k0 += 4 * 1024) {
-                f32x4 v[4];
+            for (int k0 = 4 * lane; k0 < p.Lkv; k0 += BATCH * STEP) {
+                f32x4 v[BATCH];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const f32x4*>(br + min(k0 + i * 1024, (p.Lkv - 1) & ~3));
+                for (int i = 0; i < BATCH; ++i)
+                    v[i] = *reinterpret_cast<const f32x4*>(br + min(k0 + i * STEP, (p.Lkv - 1) & ~3));
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < BATCH; ++i) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const int key = k0 + i * 1024 + j;
+                        const int key = k0 + i * STEP + j;
                         if (key < p.Lkv && !(v[i][j] == -INFINITY)) { lo = min(lo, key); hi = max(hi, key + 1); }
                     }
+                }
             }
         }
-        block_hull(lo, hi);
-        if (threadIdx.x == 0) {
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            lo = min(lo, __shfl_xor(lo, o));
+            hi = max(hi, __shfl_xor(hi, o));
+        }
+        if constexpr (WAVES > 1) {
+            __shared__ int red[WAVES][2];
+            __syncthreads();        // the row before has been read
+            if ((threadIdx.x & 63) == 0) { red[wave][0] = lo; red[wave][1] = hi; }
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) { lo = min(lo, red[w][0]); hi = max(hi, red[w][1]); }
+        }
+        if (lane == 0) {
             p.kv_start[rw] = hi > 0 ? lo : 0;
             p.kv_end[rw] = hi;
         }
-        __syncthreads();        // the work-group's numbers have been read
     }
 }
 
@@ -713,12 +716,21 @@ hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st) {
     return launch1(bwd_live_kernel, dim3((p.n_kv_blocks + 63) / 64 + rank_blocks, p.B), dim3(64), st, p);
 }
 
+// A wave to a row, with as many loads in flight as a row of so many keys has, up to four; a work-group to a row where rows
+// are long and there are too few of them to keep the chip reading.  us, a wave to a row / a work-group to a row, four loads:
+// 1024 rows x 1000 keys 2.5 / 3.5, x 2500 3.3 / 3.6, x 4096 3.9 / 3.7, x 6404 5.3 / 4.9; 2048 x 4096 4.8 / 5.2; 1 x 1300 2.26
+// / 2.13, 1 x 13000 5.7 / 3.1.  16384 x 400 with one, two and four loads 6.2, 5.9, 7.3 / 17.4; a wave to a row with one load
+// took 5.0 at 1024 x 4096 and 20.8 (10.7 with four) at 1024 x 13000.
 hipError_t launch_bias_hull(const BiasHullParams& params, hipStream_t st) {
     BiasHullParams p = params;
     const int64_t rows = (int64_t)p.B * p.Lq;
     if (rows == 0) return hipSuccess;
     p.by_Lq = divisor(p.Lq);
-    return launch1(bias_hull_kernel, dim3((unsigned)std::min<int64_t>(rows, 1 << 20)), dim3(256), st, p);
+    const dim3 by_wave((unsigned)std::min<int64_t>((rows + 3) / 4, 1 << 20));
+    if (p.Lkv <= 256) return launch1((bias_hull_kernel<1, 1>), by_wave, dim3(256), st, p);
+    if (p.Lkv <= 512) return launch1((bias_hull_kernel<1, 2>), by_wave, dim3(256), st, p);
+    if (p.Lkv <= 1024 || rows > std::min(1024, p.Lkv / 4)) return launch1((bias_hull_kernel<1, 4>), by_wave, dim3(256), st, p);
+    return launch1((bias_hull_kernel<4, 4>), dim3((unsigned)rows), dim3(256), st, p);
 }
 
 hipError_t launch_mask_intervals(const MaskIntervalParams& params, hipStream_t st) {

@@ -1,4 +1,4 @@
-"""lvx_mask_intervals: an additive mask as transformers builds it against the intervals it was made from, at
+"""lvx_bias_hull, and lvx_mask_intervals: an additive mask as transformers builds it against the intervals it was made from, at
 row lengths and alignments where the 8-byte words of a row begin before it or end behind it, and on
 masks that are more than intervals."""
 import pytest
@@ -35,6 +35,31 @@ def test_mask_intervals(dtype, B, Lq, Lkv, offset):
         gap = torch.zeros_like(mask)
         gap[0, 0, 0, Lkv // 2] = float("-inf")
         assert ops.mask_intervals(gap) is None
+
+
+# a wave to a row with one, two and four loads in flight and a work-group to a row, at the edges of their ranges
+# of keys and rows; samples and heads that share the bias or do not
+@pytest.mark.parametrize("B,nb,H,nh,Lq,Lkv", [
+    (1, 1, 2, 1, 1, 1), (2, 2, 2, 2, 5, 255), (3, 1, 2, 1, 2, 256), (1, 1, 2, 2, 9, 257), (2, 2, 2, 1, 3, 512), (1, 1, 3, 3, 6, 513),
+    (1, 1, 2, 1, 7, 1024), (1, 1, 2, 2, 257, 1025), (2, 2, 1, 1, 128, 1025), (2, 1, 1, 1, 129, 1031), (1, 1, 2, 2, 3, 4099), (3, 3, 1, 1, 342, 4100)])
+def test_hull_of_a_dense_bias(B, nb, H, nh, Lq, Lkv):
+    from lv_xattn import ops
+    g = torch.Generator().manual_seed(Lkv)
+    bias = torch.full((nb, nh, Lq, Lkv + -Lkv % 4), -torch.inf)
+    bias[..., Lkv:] = 1.0                                               # is no part of it
+    for _ in range(3):                                                  # up to three finite entries per row and head
+        at = torch.randint(0, Lkv, (nb, nh, Lq, 1), generator=g)
+        bias.scatter_(-1, at, torch.randn(nb, nh, Lq, 1, generator=g))
+    bias[0, :, 0, :Lkv] = -torch.inf                                    # an empty row
+    if Lq > 1:
+        bias[-1, -1, -1, 0] = bias[-1, -1, -1, Lkv - 1] = 0.0           # a whole one
+    seen = (bias[..., :Lkv] > -torch.inf).any(1).expand(B, Lq, Lkv)
+    start, end = seen.int().argmax(-1), Lkv - seen.int().flip(-1).argmax(-1)
+    none = ~seen.any(-1)
+    start[none], end[none] = 0, 0
+    q, k = torch.zeros(B, H, Lq, 16, device=DEV, dtype=torch.float16), torch.zeros(B, H, Lkv, 16, device=DEV, dtype=torch.float16)
+    got = ops.bias_hull(q, k, bias.to(DEV)[..., :Lkv])
+    assert torch.equal(got.kv_start.cpu(), start.int()) and torch.equal(got.kv_end.cpu(), end.int())
 
 
 class _Layer(torch.nn.Module):
