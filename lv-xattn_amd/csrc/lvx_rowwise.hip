@@ -382,8 +382,10 @@ __global__ __launch_bounds__(256) void bias_interval_kernel(const BiasHullParams
 // masked (an entry above -30000), and whether the row is that interval and nothing else - every
 // entry inside it exactly 0, at least one.  Reads the mask once, 2 bytes per (row, key), where turning
 // it into an fp32 bias and looking for the hull of that took ten launches and 16 bytes (2 x 300 rows x
-// 6404 keys: 75 us, this: 8; 4 x 1 rows 5.4, 7.0 with one 8-byte word of a thread in flight instead of four).  Rows start on any element, so an 8-byte load may begin before the row or end
-// behind it; it stays inside the 8-byte word that holds an element of the row.
+// 6404 keys: 75 us, this: 8).  Up to four 8-byte words of a thread are in flight, and a wave asks for none behind the row's
+// last (us back to back in bf16, so / one in flight / four whatever the row's length: 4 x 1 rows x 6404 keys 3.8 / 4.3 /
+// 3.9, x 400 2.3 / 2.3 / 2.9, 4 x 1024 x 801 6.6 / 6.6 / 9.2, x 6404 14.4 / 14.9 / 15.4).  Rows start on any element, so an 8-byte load
+// may begin before the row or end behind it; it stays inside the 8-byte word that holds an element of the row.
 template <typename T>
 __global__ __launch_bounds__(256) void mask_interval_kernel(const MaskIntervalParams p) {
     constexpr int EPW = 8 / sizeof(T);                  // elements per 8-byte word
@@ -395,15 +397,18 @@ __global__ __launch_bounds__(256) void mask_interval_kernel(const MaskIntervalPa
     const int skew = (int)((reinterpret_cast<uintptr_t>(r) & 7) / sizeof(T));       // elements of the first word before the row
     const uint2* words = reinterpret_cast<const uint2*>(r - skew);
     int lo = INT_MAX, hi = 0, n = 0, other = 0;
+    const int lane = threadIdx.x & 63;
     const int n_words = (p.Lkv + skew + EPW - 1) / EPW;
     constexpr int BATCH = 4;                            // words of a thread in flight
-    for (int w0 = threadIdx.x; w0 < n_words; w0 += BATCH * 256) {
+    for (int w0 = uniform32((int)threadIdx.x & ~63); w0 < n_words; w0 += BATCH * 256) {    // this wave's first word
       uint2 us[BATCH];
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i) us[i] = words[min(w0 + i * 256, n_words - 1)];
+      for (int i = 0; i < BATCH; ++i)
+        if (w0 + i * 256 < n_words) us[i] = words[min(w0 + i * 256 + lane, n_words - 1)];
 #pragma unroll
       for (int i = 0; i < BATCH; ++i) {
-        const int w = w0 + i * 256;
+        if (w0 + i * 256 >= n_words) break;
+        const int w = w0 + i * 256 + lane;
         const uint2 u = us[i];
 #pragma unroll
         for (int e = 0; e < EPW; ++e) {

@@ -9,7 +9,8 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("B,Lq,Lkv,offset", [(1, 1, 1, 0), (2, 3, 7, 0), (3, 4, 1601, 1), (2, 30, 333, 3), (1, 2, 4096, 2)])
+@pytest.mark.parametrize("B,Lq,Lkv,offset", [(1, 1, 1, 0), (2, 3, 7, 0), (3, 4, 1601, 1), (2, 30, 333, 3), (1, 2, 4096, 2),
+                                              (1, 3, 256, 3), (2, 2, 1025, 1), (1, 2, 4099, 0)])
 def test_mask_intervals(dtype, B, Lq, Lkv, offset):
     from lv_xattn import ops
     g = torch.Generator().manual_seed(Lkv)
