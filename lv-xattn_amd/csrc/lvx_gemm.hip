@@ -22,11 +22,10 @@
 //    is kept as it lies, [k][rows], and read with the transposing LDS read.
 //  * The MFMA computes C^T (A operand = rows of the B tile), so a lane ends up
 //    with 4 consecutive columns of one C row and stores 8 bytes.
-#include <algorithm>
-#include <cstdint>
 #include <type_traits>
 
 #include "lvx_common.hpp"
+#include "lvx_gemm_tiles.hpp"
 #include "lvx_kernels.hpp"
 
 namespace lvx {
@@ -717,13 +716,8 @@ bool gemm_tile_ok(const GemmParams& p, bool a_mcontig, bool b_ncontig) {
 
 }  // namespace
 
-// Work-group tile by shape.  C wider than 128 columns (projections, their gradients): the hand-scheduled tile
-// of 256 x 256, or 256 x 128 or 224 x 256 where that fills the chip's rounds better: a 128-wide tile takes about 0.6 of
-// the time of a 256-wide one (2046 x 4096 x 4096: 128 tiles of 256 on 256 CUs 81 us, 256 of 128 60; 12808 x 4096 x
-// 1024 twice: 2 rounds 176 us, 4 rounds 208), one of 224 rows about 0.9 (an eighth less work, a quarter more LDS reads per
-// MFMA, and more CUs at work under the same power: 6404 x 4096 x 1024 twice 208 tiles 97 us, 232 lower ones 90; dX
-// 6404 x 4096 of 2 x 1024 416 tiles 108, 464 lower 100; a layer's K and V, 12808 x 4096 x 1024 twice with the norm, 408 tiles
-// 234, 464 lower 224).
+// Work-group tile by shape.  C wider than 128 columns (projections, their gradients): a hand-scheduled tile of 256 x 256,
+// 256 x 128 or 224 x 256 (gemm_tile).
 // A narrow C (the dQ GEMM): 256 x 128, four stages, at which one load of a wave covers whole cache lines of
 // dS^T's 64-byte rows (two tokens x 256 rows; of a 512-row tile it takes one token, half of each line, and the
 // streaming hint then costs a second fetch: 6404 tokens x 4096 rows x 32 heads 1868 us a step against 1821),
@@ -737,13 +731,11 @@ hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipS
         if (pr.nseg > 1 && (pr.lda[1] != pr.lda[0] || pr.ldb[1] != pr.ldb[0])) return hipErrorInvalidValue;
     }
     if (p.N > 128 && gemm_tile_ok(p, a_mcontig, b_ncontig)) {
-        const int n_cu = cu_count();
-        auto rounds = [&](int tm, int tn) { return ((p.M + tm - 1) / tm * (int64_t)p.nprob * ((p.N + tn - 1) / tn) + n_cu - 1) / n_cu; };
-        const int64_t wide = 10 * rounds(256, 256), narrow = 6 * rounds(256, 128), lower = a_mcontig ? INT64_MAX : 9 * rounds(224, 256);
-        if (lower < std::min(wide, narrow))
-            return p.f16 ? launch_tile<256, true, 224>(p, a_mcontig, b_ncontig, st) : launch_tile<256, false, 224>(p, a_mcontig, b_ncontig, st);
-        if (narrow < wide) return p.f16 ? launch_tile<128, true>(p, a_mcontig, b_ncontig, st) : launch_tile<128, false>(p, a_mcontig, b_ncontig, st);
-        return p.f16 ? launch_tile<256, true>(p, a_mcontig, b_ncontig, st) : launch_tile<256, false>(p, a_mcontig, b_ncontig, st);
+        switch (gemm_tile(p.M, p.N, p.nprob, cu_count(), !a_mcontig)) {
+            case TILE_224_256: return p.f16 ? launch_tile<256, true, 224>(p, a_mcontig, b_ncontig, st) : launch_tile<256, false, 224>(p, a_mcontig, b_ncontig, st);
+            case TILE_256_128: return p.f16 ? launch_tile<128, true>(p, a_mcontig, b_ncontig, st) : launch_tile<128, false>(p, a_mcontig, b_ncontig, st);
+            default: return p.f16 ? launch_tile<256, true>(p, a_mcontig, b_ncontig, st) : launch_tile<256, false>(p, a_mcontig, b_ncontig, st);
+        }
     }
     if (p.N > 128) return launch_cfg<2, 4, 4, 2, 4>(p, a_mcontig, b_ncontig, st);
     if (p.m_order && (!p.k_range || p.nprob != 1 || p.k_splits > 1 || p.N > 128)) return hipErrorInvalidValue;
