@@ -149,7 +149,8 @@ static int fwd_split_len(const lvx_attn_shape* s, FwdForm form, int splits) {
 //   few  : 5 us, and per key of a work-group's range 8 ns (4.2 with heads of 64, 3 below) together with
 //          the time HBM takes for K and V (the root of the sum of squares: the two overlap in part).  One row x 32 heads x 6404 keys: 46 us whole, 12.5 in 16 - 32 parts;
 //          4 rows x 76848 keys in 32 parts: 61 us, 5.2 TB/s
-//   wide : 11 us per round of work-groups, and per 64-key tile 1.1 us on an idle chip, 1.5 on a full one
+//   wide : 11 us per round of work-groups (fitted before their way in and out got 2 us shorter; with 9 the ranges of 12 in
+//          504 launches of 1 to 4096 rows would differ), and per 64-key tile 1.1 us on an idle chip, 1.5 on a full one
 //          (0.9 and 1.05 with heads of 64).  256 rows x 6404 keys: 138 us whole, 39 in 8 parts
 //   plain: the same with 1.8 us per tile and two work-groups per CU
 // plus, with splits, 4 us for the launch that folds the parts and their bytes at 4 TB/s, what fp32 adds to them at 9.

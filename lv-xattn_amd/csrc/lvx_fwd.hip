@@ -191,6 +191,12 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
     // used, behind the loads of the next tile, they were waited for together with those: 1024 rows x 16 heads x 4096
     // keys forward and backward 268 us, so 255.)  The request is assembly,
     // so the compiler does not know of the wait: nothing may touch the registers before it.
+    // What is in flight is not waited for by these waits alone.  The compiler, which sees none of them, waits for Q in front
+    // of every tile's first MFMA, and with it for the tile requested just before.  Made to wait for Q once in front of
+    // the loop, the kernel takes 120 us instead of 151 where work-groups are few (1024 rows x 16 heads x 4096 keys in one
+    // range; in the ranges that are chosen nothing), but more where they fill the chip, out of step and with the bias no longer
+    // shared in the L2 (4096 x 32 heads x 6404 509 -> 520; heads of 64 396 -> 423, of 32 404 -> 435), and the
+    // forward and backward above 247 -> 251.
     u32x4 bq[8];
     const int last_k = (p.Lkv - 1) & ~3;
     auto request_bias = [&](int kv0) {
@@ -248,7 +254,7 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
         }
         __builtin_amdgcn_sched_barrier(0);
         if (BIAS) {
-            if (t + 1 < t_end) wait_vmcnt<8>();         // all but the loads of the next tile
+            if (t + 1 < t_end) wait_vmcnt<8>();         // all but the loads of the next tile (none by now, see above)
             else wait_vmcnt<0>();
 #pragma unroll
             for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(bq[i]));
@@ -438,9 +444,10 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     const int kv_hi = min(kv_len, kv_lo + p.split_len);
 
     // visible key interval of this lane's two rows.  Rows past the window and rows that see nothing
-    // are let see everything, with a Q of zeros - the former are never stored, the latter stored as zeros, which
-    // 0 times what a Q of infinities or NaN gives would not be - so that they do not make whole tiles take the
-    // element mask.
+    // are let see everything, so that they do not make whole tiles take the element mask.  The former have the
+    // window's last Q and are never stored: their scores are a lane's own, and if one moves its reference the wave rescales once
+    // more.  The latter have a Q of zeros and are stored as zeros, which 0 times what a Q of infinities or NaN gives would
+    // not be.
     int my_s[2] = {kv_lo, kv_lo}, my_e[2] = {kv_hi, kv_hi};
     bool empty[2] = {kv_hi <= kv_lo, kv_hi <= kv_lo};
     int lo = kv_lo, hi = kv_hi, in_lo = kv_lo, in_hi = kv_hi;

@@ -102,7 +102,7 @@ struct BiasHullParams {
     int32_t* kv_start;         // [B, Lq]: written by the hull kernel, read by the interval test
     int32_t* kv_end;           // [B, Lq]
     int B, heads, Lq, Lkv;     // heads: 1 (bias broadcast over heads) or Hq
-    Divisor by_Lq;             // filled in by the launchers
+    Divisor by_Lq;             // filled in by launch_bias_hull, for its kernel
     int32_t* flag;             // interval test only: set to 1 when the bias is not 0 everywhere inside the hull
 };
 // Per text row of an additive mask [B][Lq][Lkv] (type: LVX_BF16, LVX_F16 or 0 for fp32; element strides
