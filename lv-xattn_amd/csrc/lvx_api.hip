@@ -71,7 +71,6 @@ static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
 namespace {
 constexpr int MAX_DEVICES = 64;
-constexpr int MAX_RANKED_GROUPS = 1024;    // 256-row groups of a masked backward that are still ranked by length
 std::mutex scratch_mutex;
 void* scratch_ptr[MAX_DEVICES];      // per device: where that device keeps `scratch`
 
@@ -597,11 +596,11 @@ static size_t dq_partial_bytes(const lvx_attn_shape* s, int32_t row_count) {
 
 // Regions of the backward workspace, in order: dS^T tiles; fp32 dK/dV scratch (split-steps mode
 // with bf16 outputs); row metadata records (2 floats per row and head); fp32 dQ partial tiles,
-// one slice per split (split dQ contraction only); with an interval mask the live-tile tables (group hulls, runs
+// one slice per split (split dQ contraction only); with an interval mask the live-tile tables (hulls of row tiles, runs
 // of live tiles per token block, the groups ranked by hull length).  Every region is a multiple of 16 bytes.
 struct BwdWorkspace {
     size_t ds, dkv, meta, dq32, hull, runs, order, total;
-    int n_tiles, group, n_groups;
+    int n_tiles, n_groups;
 };
 
 static BwdWorkspace bwd_workspace(const lvx_attn_shape* s, int32_t row_count) {
@@ -610,8 +609,7 @@ static BwdWorkspace bwd_workspace(const lvx_attn_shape* s, int32_t row_count) {
     const size_t rows = ((size_t)row_count + 31) / 32 * 32;
     auto up16 = [](size_t n) { return (n + 15) / 16 * 16; };
     w.n_tiles = (int)(rows / 32);
-    w.group = 8;                            // row tiles per M tile of the masked dQ GEMM (256 rows)
-    w.n_groups = (w.n_tiles + w.group - 1) / w.group;
+    w.n_groups = (w.n_tiles + LIVE_GROUP - 1) / LIVE_GROUP;
     size_t off = 0;
     w.ds = off; off += (size_t)s->B * s->Hq * tokens * rows * sizeof(uint16_t);
     w.dkv = off; off += dkv_scratch_bytes(s);
@@ -619,7 +617,7 @@ static BwdWorkspace bwd_workspace(const lvx_attn_shape* s, int32_t row_count) {
     w.dq32 = off; off += dq_partial_bytes(s, row_count);
     if (s->kv_start) {
         const size_t nkb = tokens / 128;
-        w.hull = off; off += up16((size_t)s->B * w.n_groups * 2 * sizeof(int32_t));
+        w.hull = off; off += up16((size_t)s->B * w.n_tiles * 2 * sizeof(int32_t));
         w.runs = off; off += (size_t)s->B * nkb * 8 * sizeof(int32_t);
         w.order = off; off += up16((size_t)s->B * w.n_groups * sizeof(int32_t));
     }
@@ -722,7 +720,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
         if (ks <= 1 && s->B * wsl.n_groups <= MAX_RANKED_GROUPS) order = reinterpret_cast<int32_t*>(wsb + wsl.order);
         LiveParams lp{s->kv_len, s->kv_start, s->kv_end, hull, reinterpret_cast<int32_t*>(wsb + wsl.runs), order,
                       s->B, s->Lq, s->Lkv, row_begin,
-                      row_begin + row_count, wsl.n_tiles, wsl.group, wsl.n_groups, p.n_kv_blocks};
+                      row_begin + row_count, wsl.n_tiles, wsl.n_groups, p.n_kv_blocks};
         hipError_t el = launch_bwd_live(lp, st);
         if (el != hipSuccess) return static_cast<int>(el);
         p.live_runs = lp.live_runs;
@@ -766,7 +764,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     g.k_len = s->kv_len;
     g.a_tiled_m = (int)(rows / 32);
     g.a_stream = p.ds_stream;
-    g.k_range = hull;            // [B][M tiles][2]: the group hulls are per M tile of this GEMM
+    g.a_tile_range = hull;       // [B][row tiles][2]
     g.m_order = order;
     fill_grid(g, row_count, s->D, 1, s->B * s->Hq);
     if (ks <= 1) return static_cast<int>(launch_gemm(g, true, true, st));

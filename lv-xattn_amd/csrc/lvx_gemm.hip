@@ -100,7 +100,10 @@ struct Region {
 
 // GM x GN waves, each WM x WN MFMA tiles: work-group tile (32 WM GM) x (32 WN GN).
 // STREAM_A: A is loaded with the streaming hint (as a test at run time it costs a one-round dQ launch 10 %).
-template <bool A_MCONTIG, bool B_NCONTIG, int GM, int GN, int WM, int WN, int NS, bool F16, bool STREAM_A = false>
+// RANGED_A: a_tile_range is given.  A load of a wave takes two k of all eight row tiles, so a lane's row tile is
+// the same in every load; where that tile holds nothing its loads are sent out of a descriptor's range.  (With a zero
+// of one address, or of 2 KB of them, in its place the two forms of the load made the loop 6 % longer.)
+template <bool A_MCONTIG, bool B_NCONTIG, int GM, int GN, int WM, int WN, int NS, bool F16, bool STREAM_A = false, bool RANGED_A = false>
 __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     using E = Elt<F16>;
     static_assert(GM * GN == 8, "8 waves");
@@ -142,10 +145,22 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     if (p.k_len) klen0 = min(klen0, p.k_len[zo]);
     int k_lo = 0;                                   // start of this work-group's k range
     if (nks > 1) { k_lo = ksp * p.k_split_len; klen0 = min(klen0, k_lo + p.k_split_len); }
-    if (p.k_range) {
-        const int32_t* kr = p.k_range + ((int64_t)zo * p.tiles_m + tm) * 2;
-        k_lo = max(k_lo, kr[0]);
-        klen0 = min(klen0, kr[1]);
+    uint32_t a_lo = 0, a_len = 0;                   // k of this lane's row tile of A
+    if constexpr (RANGED_A) {
+        static_assert(A_MCONTIG && TM == 256, "eight row tiles, four lanes each");
+        const int ln = threadIdx.x & 63, k4 = 2 * ((threadIdx.x >> 6) & 1) + (ln >> 5);      // k mod 4 of its loads
+        const int t = min((m0 >> 5) + (((ln & 31) >> 2) ^ k4), p.a_tiled_m - 1);
+        const int32_t* r = p.a_tile_range + ((int64_t)zo * p.a_tiled_m + t) * 2;
+        a_lo = (uint32_t)r[0];
+        a_len = (uint32_t)(r[1] - r[0]);
+        int lo = r[1] ? r[0] : 0x7fffffff, hi = r[1];
+#pragma unroll
+        for (int off = 4; off < 32; off <<= 1) {
+            lo = min(lo, __shfl_xor(lo, off));
+            hi = max(hi, __shfl_xor(hi, off));
+        }
+        k_lo = max(k_lo, uniform32(min(lo, hi)));
+        klen0 = min(klen0, uniform32(hi));
     }
     klen0 = max(0, klen0 - k_lo);
     const int s_lo = k_lo / BK;                    // first stage of this work-group's k range
@@ -164,7 +179,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
 #pragma unroll
     for (int j = 0; j < LPG; ++j) {
         const int ch = wave + 8 * j;
-        if (j < LPG_A) voff[j] = RA::src(ch, lane, m0, p.M_ld, lda, p.a_tiled_m, kpos[j]);
+        if (j < LPG_A) voff[j] = RA::src(ch, lane, m0, p.M_ld, lda, p.a_tiled_m, kpos[j]) - (RANGED_A ? (uint32_t)(m0 >> 5) * 8192u : 0u);
         else voff[j] = RB::src(ch - RA::CHUNKS, lane, n0, p.N, ldb, 0, kpos[j]);
     }
     const char* abase[2];
@@ -173,7 +188,8 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     for (int sg = 0; sg < 2; ++sg) {
         const int ss = sg < pr.nseg ? sg : 0;
         abase[sg] = reinterpret_cast<const char*>(pr.A[ss] + a_off);
-        if (!p.a_tiled_m) abase[sg] += (A_MCONTIG ? (int64_t)m0 : (int64_t)m0 * lda) * 2;
+        if (RANGED_A) abase[sg] += (int64_t)(m0 >> 5) * 8192;
+        else if (!p.a_tiled_m) abase[sg] += (A_MCONTIG ? (int64_t)m0 : (int64_t)m0 * lda) * 2;
         bbase[sg] = reinterpret_cast<const char*>(pr.Bm[ss] + b_off) + (B_NCONTIG ? (int64_t)n0 : (int64_t)n0 * ldb) * 2;
     }
     const int64_t a_kstride = A_MCONTIG ? lda * BK * 2 : BK * 2;   // bytes per stage (untiled)
@@ -191,17 +207,19 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
             ab = abase[sg] + ((int64_t)(ks >> 2) * p.a_tiled_m * 4096 + (ks & 3) * (BK * 32)) * 2;
         const char* bb = bbase[sg] + ks * b_kstride;
         const uint32_t slot = lds0 + (uint32_t)(s % NS) * STAGE + (uint32_t)wave * 1024u;
+        const bool a_mine = !RANGED_A || (uint32_t)(ks * BK) - a_lo < a_len;
         if (krem >= BK) {
 #pragma unroll
             for (int j = 0; j < LPG; ++j)
-                if (STREAM_A && j < LPG_A) dma16_stream(ab, voff[j], slot + j * 8192);
+                if (RANGED_A && j < LPG_A) dma16_range<STREAM_A>(ab, TM / 32 * 8192, a_mine ? voff[j] : 0x80000000u, slot + j * 8192);
+                else if (STREAM_A && j < LPG_A) dma16_stream(ab, voff[j], slot + j * 8192);
                 else dma16(j < LPG_A ? ab : bb, voff[j], slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
         } else {
             const char* zc = reinterpret_cast<const char*>(zero_chunk);
 #pragma unroll
             for (int j = 0; j < LPG; ++j) {
                 const char* src = (j < LPG_A ? ab : bb) + voff[j];
-                dma16_addr(kpos[j] < krem ? src : zc, slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
+                dma16_addr(kpos[j] < krem && (j >= LPG_A || a_mine) ? src : zc, slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
             }
         }
     };
@@ -676,10 +694,15 @@ hipError_t launch_cfg_t(const GemmParams& p, int grid, bool a_mcontig, bool b_nc
         return launch1((gemm_kernel<false, true, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
     else if (a_mcontig && !b_ncontig)
         return launch1((gemm_kernel<true, false, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
-    else if (!p.a_stream)
-        return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
-    else
-        return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16, true>), dim3(grid), dim3(512), st, p);
+    if constexpr (32 * WN * GN == 128) {       // the dQ GEMM
+        if (p.a_tile_range && p.a_stream)
+            return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16, true, true>), dim3(grid), dim3(512), st, p);
+        if (p.a_tile_range)
+            return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16, false, true>), dim3(grid), dim3(512), st, p);
+        if (p.a_stream)
+            return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16, true>), dim3(grid), dim3(512), st, p);
+    }
+    return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
 }
 
 template <int GM, int GN, int WM, int WN, int NS>
@@ -705,7 +728,7 @@ hipError_t launch_tile(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t
 // there are two), offsets inside an operand below 2^32, and not the layout nothing uses.
 bool gemm_tile_ok(const GemmParams& p, bool a_mcontig, bool b_ncontig) {
     const GemmProblem& pr = p.prob[0];
-    if (p.nbatch != 1 || p.k_len || p.k_range || p.k_splits > 1 || p.a_tiled_m || (a_mcontig && !b_ncontig)) return false;
+    if (p.nbatch != 1 || p.k_len || p.a_tile_range || p.k_splits > 1 || p.a_tiled_m || (a_mcontig && !b_ncontig)) return false;
     if (pr.nseg > 1 && (pr.K[1] != pr.K[0] || pr.K[0] % TK)) return false;
     // (the descriptor of a row-major operand covers 2 GiB, the other kind ends with the contraction)
     const int64_t limit = (int64_t)1 << 32;
@@ -738,7 +761,8 @@ hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipS
         }
     }
     if (p.N > 128) return launch_cfg<2, 4, 4, 2, 4>(p, a_mcontig, b_ncontig, st);
-    if (p.m_order && (!p.k_range || p.nprob != 1 || p.k_splits > 1 || p.N > 128)) return hipErrorInvalidValue;
+    if (p.a_tile_range && (!a_mcontig || !b_ncontig || p.a_tiled_m <= 0 || p.N > 128)) return hipErrorInvalidValue;
+    if (p.m_order && (!p.a_tile_range || p.nprob != 1 || p.k_splits > 1 || p.N > 128)) return hipErrorInvalidValue;
     return launch_cfg<4, 2, 2, 2, 4>(p, a_mcontig, b_ncontig, st);
 }
 

@@ -173,20 +173,24 @@ struct BwdParams {
     Divisor by_splits, by_splits2, by_kv_blocks, by_B;     // filled in by launch_bwd
 };
 
-// Which (token block, 32-row tile) pairs an interval mask leaves alive, at the granularity the
-// dQ GEMM needs: rows are taken in groups of `group` tiles (one M tile of that GEMM); a group's
-// hull is the smallest range of whole token blocks that holds every key some row of the group
-// sees, and all tiles of a group are alive for exactly the blocks of its hull.
+// Which (token block, 32-row tile) pairs an interval mask leaves alive: a tile is alive for the blocks of its hull, the
+// smallest range of whole token blocks that holds every key some row of the tile sees.  The dQ GEMM takes its M tiles,
+// groups of LIVE_GROUP row tiles, over the hull of the group, and reads a tile's dS^T inside the tile's own hull only.
+// (With whole groups alive or not, 2 x 3000 rows that see the image before them visited 13 % more pairs, since images
+// begin inside groups: bwd_kernel 689 us, 599 now, forward and backward 1144 -> 1067; the two table kernels 2.5 us each, or
+// 5 where another kernel left its lines in no cache, as before.)
+constexpr int LIVE_GROUP = 8;
+constexpr int MAX_RANKED_GROUPS = 1024;    // groups of a launch that are still ranked by length
 struct LiveParams {
     const int32_t* kv_len;     // may be null
     const int32_t* kv_start;
     const int32_t* kv_end;
-    int32_t* hull;             // out: [B][n_groups][2] token range (multiples of 128), (0, 0) if empty
-    int32_t* live_runs;        // out, see BwdParams; a fifth run and later ones are merged into the
-                               // fourth together with the gaps between them (visiting more is harmless)
+    int32_t* tile_hull;        // out: [B][n_tiles][2] token range of a row tile (multiples of 128), (0, 0) if empty
+    int32_t* live_runs;        // out, see BwdParams; of more than four runs those the smallest gaps apart
+                               // become one (visiting more is harmless)
     int32_t* order;            // out (may be null): the B * n_groups group indices b * n_groups + grp,
                                // longest hull first (ties in index order)
-    int B, Lq, Lkv, row_begin, row_end, n_tiles, group, n_groups, n_kv_blocks;
+    int B, Lq, Lkv, row_begin, row_end, n_tiles, n_groups, n_kv_blocks;
 };
 hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st);
 
@@ -269,10 +273,11 @@ struct GemmParams {
     float norm_eps;
     uint16_t* c_raw;
     float* rstd;
-    // Per (outer batch index, M tile) contraction range of segment 0: k_range[(zo * tiles_m +
-    // tm) * 2 + {0, 1}] = first and one-past-last k (multiples of 128); null: all of K[0].
-    const int32_t* k_range;
-    // With k_range (one problem, no split contraction): the (outer batch index, M tile) pairs
+    // With a_tiled_m (null: off): per (outer batch index, 32-row tile of A) the k at which the tile holds anything,
+    // a_tile_range[(zo * a_tiled_m + tile) * 2 + {0, 1}] = first and one-past-last (multiples of 128; 0, 0: nowhere).
+    // An M tile contracts over the hull of its tiles' ranges; outside its own a tile counts as zeros and is not read.
+    const int32_t* a_tile_range;
+    // With a_tile_range (one problem, no split contraction): the (outer batch index, M tile) pairs
     // zo * tiles_m + tm in the order the work-groups are to take them, longest range first
     // (null: in index order).
     const int32_t* m_order;

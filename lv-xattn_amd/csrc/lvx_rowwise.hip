@@ -451,65 +451,96 @@ __global__ __launch_bounds__(256) void mask_interval_kernel(const MaskIntervalPa
     p.kv_end[blockIdx.x] = interval ? hi : 0;
 }
 
-// One wave per (group of row tiles, b): the hull of the rows' key intervals in whole token blocks.
-__global__ __launch_bounds__(64) void bwd_hull_kernel(const LiveParams p) {
-    const int grp = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
-    const int r0 = p.row_begin + grp * p.group * 32;
-    const int r1 = min(r0 + p.group * 32, p.row_end);
+// One thread per row: the hulls of the row tiles' key intervals in whole token blocks.
+__global__ __launch_bounds__(256) void bwd_hull_kernel(const LiveParams p) {
+    const int b = blockIdx.y, tile = blockIdx.x * 8 + (threadIdx.x >> 5);
+    const int r = p.row_begin + tile * 32 + (threadIdx.x & 31);
     const int kv_len = p.kv_len ? min(p.kv_len[b], p.Lkv) : p.Lkv;
     int lo = INT_MAX, hi = 0;
-    for (int r = r0 + lane; r < r1; r += 64) {
+    if (r < p.row_end) {
         const int s = max(p.kv_start[(int64_t)b * p.Lq + r], 0);
         const int e = min(p.kv_end[(int64_t)b * p.Lq + r], kv_len);
-        if (e > s) { lo = min(lo, s); hi = max(hi, e); }
+        if (e > s) { lo = s; hi = e; }
     }
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
+    for (int o = 1; o < 32; o <<= 1) {
         lo = min(lo, __shfl_xor(lo, o));
         hi = max(hi, __shfl_xor(hi, o));
     }
-    if (lane == 0) {
-        int32_t* h = p.hull + ((int64_t)b * p.n_groups + grp) * 2;
+    if ((threadIdx.x & 31) == 0 && tile < p.n_tiles) {
+        int32_t* h = p.tile_hull + ((int64_t)b * p.n_tiles + tile) * 2;
         h[0] = hi > 0 ? (lo / 128) * 128 : 0;
         h[1] = (hi + 127) / 128 * 128;
     }
 }
 
-// One thread per (token block, b): the runs of consecutive row tiles whose group's hull holds the block.
-// Blocks past those (b == 0 only) rank the groups by hull length, one thread per group.
+// One wave per (token block, b): the runs of consecutive row tiles whose hull holds the block.  Where there are more than
+// four, the two the narrowest gap apart become one, so that the three widest gaps are left out.
+// Blocks past those (b == 0 only) rank the groups of row tiles by the length of their hull, one thread per group.
 __global__ __launch_bounds__(64) void bwd_live_kernel(const LiveParams p) {
-    const int live_blocks = (p.n_kv_blocks + 63) / 64;
-    if ((int)blockIdx.x >= live_blocks) {
-        const int n = p.B * p.n_groups;
-        const int i = ((int)blockIdx.x - live_blocks) * 64 + threadIdx.x;
-        if (blockIdx.y != 0 || i >= n) return;
-        const int len = p.hull[2 * i + 1] - p.hull[2 * i];
-        int rank = 0;
-        for (int j = 0; j < n; ++j) {
-            const int lj = p.hull[2 * j + 1] - p.hull[2 * j];
-            rank += (lj > len || (lj == len && j < i)) ? 1 : 0;
+    const int lane = threadIdx.x;
+    if ((int)blockIdx.x >= p.n_kv_blocks) {
+        __shared__ int len[MAX_RANKED_GROUPS];
+        const int n = p.B * p.n_groups, i = ((int)blockIdx.x - p.n_kv_blocks) * 64 + lane;
+        if (blockIdx.y != 0) return;
+        for (int j = lane; j < n; j += 64) {
+            const int b = j / p.n_groups, t0 = (j - b * p.n_groups) * LIVE_GROUP;
+            const int32_t* h = p.tile_hull + (int64_t)b * p.n_tiles * 2;
+            int lo = INT_MAX, hi = 0;
+#pragma unroll
+            for (int k = 0; k < LIVE_GROUP; ++k) {
+                const int t = min(t0 + k, p.n_tiles - 1);
+                if (h[2 * t + 1] > 0) { lo = min(lo, h[2 * t]); hi = max(hi, h[2 * t + 1]); }
+            }
+            len[j] = max(0, hi - lo);
         }
+        __syncthreads();
+        if (i >= n) return;
+        const int mine = len[i];
+        int rank = 0;
+        for (int j = 0; j < n; ++j) rank += (len[j] > mine || (len[j] == mine && j < i)) ? 1 : 0;
         p.order[rank] = i;
         return;
     }
-    const int kblk = blockIdx.x * 64 + threadIdx.x, b = blockIdx.y;
-    if (kblk >= p.n_kv_blocks) return;
-    const int kvb = kblk * 128;
-    int32_t* out = p.live_runs + ((int64_t)b * p.n_kv_blocks + kblk) * 8;
-    int nr = 0, start = 0;
-    bool open = false;
-    for (int grp = 0; grp < p.n_groups; ++grp) {
-        const int32_t* h = p.hull + ((int64_t)b * p.n_groups + grp) * 2;
-        const bool live = h[0] <= kvb && kvb < h[1];
-        const int t0 = grp * p.group, t1 = min(t0 + p.group, p.n_tiles);
-        if (live) {
-            if (!open && nr < 4) { start = t0; ++nr; }
-            out[2 * (nr - 1)] = start;
-            out[2 * (nr - 1) + 1] = t1 - start;
+    const int kblk = blockIdx.x, b = blockIdx.y, kvb = kblk * 128;
+    int first[4] = {0, 0, 0, 0}, end[4] = {0, 0, 0, 0}, nr = 0, last_end = -1;
+    for (int t0 = 0; t0 < p.n_tiles; t0 += 64) {
+        const int32_t* h = p.tile_hull + ((int64_t)b * p.n_tiles + min(t0 + lane, p.n_tiles - 1)) * 2;
+        uint64_t live = __builtin_amdgcn_ballot_w64(t0 + lane < p.n_tiles && h[0] <= kvb && kvb < h[1]);
+        while (live) {
+            const int bit = __builtin_ctzll(live), s = t0 + bit;
+            const uint64_t gaps = ~(live >> bit);
+            const int n = min(gaps ? __builtin_ctzll(gaps) : 64, 64 - bit), e = s + n;
+            live &= n == 64 ? 0 : ~(((uint64_t{1} << n) - 1) << bit);
+            const bool apart = s != last_end, append = apart && nr < 4;
+            if (apart && !append) {
+                int width = s - end[3], at = 3;
+#pragma unroll
+                for (int i = 2; i >= 0; --i)
+                    if (first[i + 1] - end[i] < width) { width = first[i + 1] - end[i]; at = i; }
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {   // close gap `at`: the runs on its sides become one, the later ones move up
+                    if (i >= at) end[i] = end[i + 1];
+                    if (i > at) first[i] = first[i + 1];
+                }
+                if (at < 3) first[3] = s;
+            }
+            if (append) ++nr;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (i == nr - 1) { if (append) first[i] = s; end[i] = e; }
+            last_end = e;
         }
-        open = live;
     }
-    for (int i = nr; i < 4; ++i) { out[2 * i] = 0; out[2 * i + 1] = 0; }
+    if (lane < 8) {
+        int x = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (lane == 2 * i && i < nr) x = first[i];
+            if (lane == 2 * i + 1 && i < nr) x = end[i] - first[i];
+        }
+        p.live_runs[((int64_t)b * p.n_kv_blocks + kblk) * 8 + lane] = x;
+    }
 }
 
 template <bool F16>
@@ -715,10 +746,10 @@ hipError_t launch_bwd_meta(const MetaParams& p0, hipStream_t st) {
 
 hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st) {
     if (p.B <= 0 || p.n_groups <= 0 || p.n_kv_blocks <= 0) return hipSuccess;
-    const hipError_t e = launch1(bwd_hull_kernel, dim3(p.n_groups, p.B), dim3(64), st, p);
+    const hipError_t e = launch1(bwd_hull_kernel, dim3((p.n_tiles + 7) / 8, p.B), dim3(256), st, p);
     if (e != hipSuccess) return e;
     const int rank_blocks = p.order ? (p.B * p.n_groups + 63) / 64 : 0;
-    return launch1(bwd_live_kernel, dim3((p.n_kv_blocks + 63) / 64 + rank_blocks, p.B), dim3(64), st, p);
+    return launch1(bwd_live_kernel, dim3(p.n_kv_blocks + rank_blocks, p.B), dim3(64), st, p);
 }
 
 // A wave to a row, with as many loads in flight as a row of so many keys has, up to four; a work-group to a row where rows
