@@ -24,7 +24,7 @@ LIB = os.path.join(OUT_DIR, "liblvx.so")
 HOST_SRC = os.path.join(CSRC, "lvx_host.cpp")
 HOST_LIB = os.path.join(OUT_DIR, "_lvx_host.so")
 
-SOURCES = ["lvx_api.hip", "lvx_fwd.hip", "lvx_bwd.hip", "lvx_rowwise.hip", "lvx_gemm.hip"]
+SOURCES = ["lvx_api.hip", "lvx_fwd.hip", "lvx_bwd.hip", "lvx_dq.hip", "lvx_rowwise.hip", "lvx_gemm.hip"]
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",

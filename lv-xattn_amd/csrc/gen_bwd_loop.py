@@ -11,8 +11,8 @@ spread over its other instructions (LDS operand reads eight operands ahead, the 
 the dS arithmetic of an earlier tile, the global -> LDS loads and the dS^T copy-out), so that a
 wave keeps the matrix pipe fed by itself.
 
-LDS map in bytes (lvx_bwd.hip): Q ring 6 x 8192 at 0, dO ring at 49152, dS^T tiles 2 x 10240 at
-98304, P hand-over 2 x 8192 at 118784; the metadata of a tile, 6 x 768 bytes, is a separate array: 256 bytes
+LDS map in bytes (lvx_bwd.hip): Q ring 6 x 8192 at 0, dO ring at 49152, dS^T tiles 2 x 8192 at
+98304, P hand-over 2 x 8192 at 114688; the metadata of a tile, 6 x 768 bytes, is a separate array: 256 bytes
 of LSE and delta, with intervals per row 256 each of starts and ends (32 rows, twice).
 
 The last tile of a head may have fewer than 32 rows: when the walk comes to it, the lanes' load offsets are
@@ -26,8 +26,8 @@ Registers, both roles: v[0:63] resident accumulators (dV^T / dK^T)   v[64:95] re
 v[128:159] eight operand slots  v[200:207] row-read addresses into "its" ring (P: Q, D: dO)
 v[208:215] transposing-read addresses into the other ring.   s40 scale*log2(e) (P) / scale (D)
 P-waves: v[168:175] P packed   v[176:191] LSE*log2(e) of 16 rows   v[192:199] dS^T copy-out data
-  v216 P hand-over write address   v217 metadata read address   v218 dS^T copy-out read address
-  v219, v220 copy-out global offsets   v221..v224 global offsets of the four tile loads   v225 of
+  v216 P hand-over write address   v217 metadata read address   v218, v219 dS^T copy-out read addresses (transposing
+  reads: four tokens of a row each)   v220 copy-out global offset   v221..v224 global offsets of the four tile loads   v225 of
   the metadata load   v226, v227 rows by which the lane's two rows of a head's last tile are past the window
   v229 scratch   masked: v228 read address of the interval of row lane % 32   v229, v230 that interval
   v231 the lane's token, out of every interval if it is past the sample   v232 bytes by which the lane's row of
@@ -42,7 +42,8 @@ P-waves: v[168:175] P packed   v[176:191] LSE*log2(e) of 16 rows   v[192:199] dS
   rows, else -1   s83 / s84 bytes per Q / dO row   masked: s85 bytes of metadata per tile   s86 first token of the wave, s87 one
   past its last   s[90:91] all ones if not all of them exist   s92 1 if dS^T leaves as streaming stores
 D-waves: v[168:175] P handed over   v[176:183] dS packed   v[184:199] delta*scale of 16 rows
-  v216 P hand-over read address   v217 metadata read address   v218 dS^T staging write address
+  v216 P hand-over read address   v217 metadata read address   v218, v223..v225 dS^T staging write addresses, one per
+  group of four rows
 """
 import os
 import re
@@ -64,14 +65,14 @@ NOP = NKK + 2 * NDT                     # MFMAs of a step, one LDS operand each
 
 ACC, BREG, SET, STG, RA, TA = 0, 64, (96, 112), 128, 200, 208
 NSLOT, AHEAD = 8, 7
-TILE_B, DO_RING, DST_B, DST_SZ, PB_SZ, META_SZ = 8192, 49152, 98304, 10240, 8192, 768
+TILE_B, DO_RING, DST_B, DST_SZ, PB_SZ, META_SZ = 8192, 49152, 98304, 8192, 8192, 768
 # P role
 PU, LSE, CPD = 168, 176, 192
-A_PB, A_META, A_CP, G_CP0, G_CP1, G_DMA, G_META = 216, 217, 218, 219, 220, 221, 225
+A_PB, A_META, A_CP, G_CP, G_DMA, G_META = 216, 217, (218, 219), 220, 221, 225
 EXCESS, A_IV, IV, TOKEN = 226, 228, 229, 231
 IV_EXCESS = 232
 # D role
-DSU, DELTA, TMP = 176, 184, 219
+DSU, DELTA, TMP, A_DS = 176, 184, 219, (218, 223, 224, 225)
 
 
 def vr(base, n=1):
@@ -206,7 +207,7 @@ def p_ragged(u, ahead):
 
 
 def p_store(hint):
-    return [f"global_store_dwordx4 v{G_CP0}, {vr(CPD, 4)}, s[78:79]{hint}", f"global_store_dwordx4 v{G_CP1}, {vr(CPD + 4, 4)}, s[78:79]{hint}"]
+    return [f"global_store_dwordx4 v{G_CP}, {vr(CPD, 4)}, s[78:79]{hint}", f"global_store_dwordx4 v{G_CP}, {vr(CPD + 4, 4)}, s[78:79] offset:1024{hint}"]
 
 
 def p_keep(u):
@@ -282,14 +283,14 @@ def p_step(u, seed):
     # second half: request of tile i+3 and the walk, dS^T(i-3) copy-out.  The loads go first: the wait
     # at the top of a step then leaves the two stores of the step before last in flight as well
     tail = []
-    tail.append(lambda: st.lds(f"ds_read_b128 {vr(CPD, 4)}, v{A_CP} offset:{par * DST_SZ}", "cp0"))
-    tail.append(lambda: st.lds(f"ds_read_b128 {vr(CPD + 4, 4)}, v{A_CP} offset:{par * DST_SZ + 5120}", "cp1"))
+    for n in range(4):
+        tail.append(lambda n=n: st.lds(f"ds_read_b64_tr_b16 {vr(CPD + 2 * n, 2)}, v{A_CP[n % 2]} offset:{par * DST_SZ + 1024 * (n // 2)}", f"cp{n}"))
     ws_old = 66 + 2 * (u % 6)          # workspace address of tile i-3 (tile i+3 takes its place below)
     fetch = p_fetch(u, 3)
     if u == 5:      # the last step of the last trip requests nothing: the steps after the loop do
         fetch = [["s_cmp_eq_u32 s64, 1", "s_cbranch_scc1 LVX_BWD_NOFETCH_%="] + flat(fetch) + ["LVX_BWD_NOFETCH_%=:"]]
     # the stores read the workspace address of tile i-3 before the walk overwrites it: keep a copy
-    tail += [f"s_mov_b64 s[78:79], {sr(ws_old, 2)}"] + fetch + [lambda: st.wait("cp1")]
+    tail += [f"s_mov_b64 s[78:79], {sr(ws_old, 2)}"] + fetch + [lambda: st.wait("cp3")]
     tail.append(["s_cmp_eq_u32 s92, 0", f"s_cbranch_scc1 LVX_BWD_KEEP{u}_%=", *p_store(" nt"), f"LVX_BWD_STORED{u}_%=:"])
 
     mf = []
@@ -380,7 +381,7 @@ def d_step(u, seed):
         valu.append(f"{CVT} v{DSU + 2 * q}, v{carry + 4 * q}, v{carry + 4 * q + 1}")
         valu.append(f"{CVT} v{DSU + 2 * q + 1}, v{carry + 4 * q + 2}, v{carry + 4 * q + 3}")
     for vg in range(4):
-        valu.append(lambda vg=vg: st.lds(f"ds_write_b64 v{218}, {vr(DSU + 2 * vg, 2)} offset:{par * DST_SZ + 16 * vg}"))
+        valu.append(lambda vg=vg: st.lds(f"ds_write_b64 v{A_DS[vg]}, {vr(DSU + 2 * vg, 2)} offset:{par * DST_SZ}"))
 
     mf = []
     for k in range(NOP):

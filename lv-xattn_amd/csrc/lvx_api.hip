@@ -61,7 +61,7 @@ constexpr int MAX_SPLITS = 64;
 
 }  // namespace
 
-static void fill_grid(GemmParams& g, int M, int N, int nprob, int nbatch);
+static void fill_grid(GemmParams& g, int M, int N, int nprob);
 
 // Device memory of lvx_fwd_noalloc: the key-split partials live in this file-scope array
 // instead of a caller's workspace.  Every GPU the library runs on holds its own copy at its
@@ -568,7 +568,7 @@ static size_t dkv_scratch_bytes(const lvx_attn_shape* s) {
 // rounded to bf16 afterwards (fp32 atomics into one slice were measured slower).  Returns
 // the number of splits (1: none) and the tokens per split.
 static int dq_k_splits(const lvx_attn_shape* s, int32_t row_count, int* split_len) {
-    const int tiles = (row_count + 255) / 256;          // of launch_gemm's 256-row tile
+    const int tiles = (row_count + 255) / 256;          // of dq_kernel's 256 rows
     const int wgs = s->B * s->Hq * tiles;
     const int blocks = (s->Lkv + 127) / 128;
     int ks = 1;
@@ -747,34 +747,23 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     }
 
     // dQ[b, h, rows, :] = dS^T[b, h]^T (rows x tokens) * K[b, h / G] (tokens x D), scale already in dS
-    GemmParams g{};
-    g.f16 = p.f16;
-    GemmProblem& pr = g.prob[0];
-    pr.A[0] = p.ds_ws; pr.lda[0] = rows;
-    pr.Bm[0] = p.k; pr.ldb[0] = k->stride_s;
-    pr.K[0] = s->Lkv; pr.nseg = 1;
-    pr.C = static_cast<uint16_t*>(dq->ptr) + (int64_t)row_begin * dq->stride_s;
-    pr.ldc = dq->stride_s;
-    g.M_ld = (int)rows;
-    g.batch_inner = s->Hq;
-    g.b_group = p.G;
-    g.a_batch = p.ws_bh;
-    g.b_outer = k->stride_b; g.b_inner = k->stride_h;
-    g.c_outer = dq->stride_b; g.c_inner = dq->stride_h;
-    g.k_len = s->kv_len;
-    g.a_tiled_m = (int)(rows / 32);
-    g.a_stream = p.ds_stream;
-    g.a_tile_range = hull;       // [B][row tiles][2]
-    g.m_order = order;
-    fill_grid(g, row_count, s->D, 1, s->B * s->Hq);
-    if (ks <= 1) return static_cast<int>(launch_gemm(g, true, true, st));
+    DqParams g{};
+    g.ds = p.ds_ws; g.ds_bh = p.ws_bh;
+    g.k = p.k; g.ks = p.ks;
+    g.dq = static_cast<uint16_t*>(dq->ptr) + (int64_t)row_begin * dq->stride_s;
+    g.dqs = st3(dq);
+    g.B = s->B; g.Hq = s->Hq; g.G = p.G; g.D = s->D; g.f16 = p.f16;
+    g.rows = row_count; g.row_tiles = (int)(rows / 32); g.Lkv = s->Lkv;
+    g.stream = p.ds_stream;
+    g.kv_len = s->kv_len;
+    g.tile_range = hull;         // [B][row tiles][2]
+    g.order = order;
     // split contraction: every split stores its partial tiles in its own fp32 slice; the
     // cast sums the slices and rounds into dq
-    g.k_splits = ks; g.k_split_len = split_len;
-    g.c32 = dq32; g.c32_batch = (int64_t)row_count * s->D; g.c32_ld = row_count;   // [split][B * Hq][D][row_count]
-    g.c32_split = (int64_t)s->B * s->Hq * g.c32_batch;
-    e = launch_gemm(g, true, true, st);
-    if (e != hipSuccess) return static_cast<int>(e);
+    g.k_splits = ks; g.split_len = split_len;
+    g.part = dq32; g.part_split = (int64_t)s->B * s->Hq * row_count * s->D;      // [split][B * Hq][D][row_count]
+    e = launch_dq(g, st);
+    if (e != hipSuccess || ks <= 1) return static_cast<int>(e);
     CastParams cq{};
     cq.f16 = p.f16;
     cq.D = s->D;
@@ -783,7 +772,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     cq.ds = st3(dq);
     cq.B = s->B; cq.H = s->Hq; cq.L = row_count;
     cq.transposed = 1;
-    cq.nsum = ks; cq.sum_stride = g.c32_split;
+    cq.nsum = ks; cq.sum_stride = g.part_split;
     return static_cast<int>(launch_cast(cq, st));
 }
 
@@ -816,13 +805,7 @@ static int check_gemm_ptr(const void* p, int64_t ld) {
 
 }  // extern "C"
 
-static void fill_grid(GemmParams& g, int M, int N, int nprob, int nbatch = 1) {
-    g.M = M; g.N = N; g.nprob = nprob;
-    if (g.M_ld < M) g.M_ld = M;
-    g.nbatch = nbatch;
-    if (g.batch_inner < 1) g.batch_inner = 1;
-    if (g.b_group < 1) g.b_group = 1;
-}
+static void fill_grid(GemmParams& g, int M, int N, int nprob) { g.M = M; g.N = N; g.nprob = nprob; }
 
 extern "C" {
 

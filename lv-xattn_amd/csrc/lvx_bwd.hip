@@ -21,8 +21,10 @@
 // whole rest of the kernel on this machine (atomic adds sustain about 1.3 TB/s),
 // so dQ is not formed here: the D-waves gather scale*dS (bf16) in LDS and the
 // group streams it to a workspace in HBM, one contiguous 8 KB tile
-// [128 tokens][32 rows] per step, indexed [b, h, token block, row tile]; a
-// batched GEMM (launched by the caller right after) contracts it with K.  The workspace costs 2 bytes per
+// of 128 tokens x 32 rows per step, indexed [b, h, token block, row tile]; dq_kernel
+// (launched by the caller right after) contracts it with K.  The tile is turned on its way out of the LDS: it lies as
+// [token / 8][row][8 tokens], so that a lane's operand of that contraction is 16 bytes that it loads from memory into its
+// registers.  The workspace costs 2 bytes per
 // (row, token, head), written once and read once; the caller says when it is large enough for
 // streaming stores (ds_stream).
 //
@@ -50,14 +52,13 @@ constexpr int D = 128;
 constexpr int BN = 128;       // visual tokens per work-group
 constexpr int BM = 32;        // text rows per step
 constexpr int NT = 512;       // threads per work-group
-constexpr int DSS = BM + 8;   // row stride of the dS^T tile [token][row]
 
 // LDS map (uint16 units): a ring of six Q tiles, a ring of six dO tiles (each ring within the 64 KiB an LDS
 // instruction's immediate offset reaches from one address register), unpadded; two dS^T tiles; two P
 // hand-over buffers
 constexpr int TILE_ELEMS = BM * D;             // one Q or dO tile (8 KiB)
 constexpr int NQD = 6;
-constexpr int DST_ELEMS = BN * DSS;
+constexpr int DST_ELEMS = BN * BM;             // [token][row], the 16-byte chunk c of a token at c ^ ((token >> 2) & 3)
 constexpr int PB_ELEMS = 4 * 2 * 64 * 8;       // P hand-over: [slice][half][lane][16 bytes] as uint16
 constexpr int OFF_Q = 0;                       // x NQD
 constexpr int OFF_DO = OFF_Q + NQD * TILE_ELEMS; // x NQD
@@ -86,7 +87,7 @@ constexpr float LOG2E = 1.4426950408889634f;
     : LVX_BWD_COMMON_OUT, "+{s[44:45]}"(qp), "+{s[46:47]}"(dop), "+{s[48:49]}"(mp), "+{s[50:51]}"(wn), "+{s52}"(left), \
       "+{s[66:67]}"(w0), "+{s[68:69]}"(w1), "+{s[70:71]}"(w2), "+{s[72:73]}"(w3), "+{s[74:75]}"(w4), "+{s[76:77]}"(w5), \
       "+{v221}"(g_t[0]), "+{v222}"(g_t[1]), "+{v223}"(g_t[2]), "+{v224}"(g_t[3]), "+{v225}"(g_meta)                   \
-    : LVX_BWD_COMMON_IN, "{v218}"(a_cp), "{v219}"(g_cp0), "{v220}"(g_cp1), "{v232}"(past_iv),                        \
+    : LVX_BWD_COMMON_IN, "{v218}"(a_cp0), "{v219}"(a_cp1), "{v220}"(g_cp), "{v232}"(past_iv),                        \
       "{v226}"(past0), "{v227}"(past1), "{v228}"(a_iv), "{v231}"(token), "{s83}"(uniform32(qrow_b)), "{s84}"(uniform32(dorow_b)), \
       "{s40}"(uniform32(c)), "{s41}"(uniform32((uint32_t)BM * qrow_b)), "{s42}"(uniform32((uint32_t)BM * dorow_b)),  \
       "{s53}"(uniform32(n_live)), "{s[54:55]}"(hdq), "{s[56:57]}"(hddo), "{s[60:61]}"(hdws), "{s[80:81]}"(hdm),      \
@@ -97,7 +98,7 @@ constexpr float LOG2E = 1.4426950408889634f;
       "{s[90:91]}"(uniform64(slice_valid ? (int64_t)0 : (int64_t)-1))                                                \
     : "memory", "vcc", "scc", "m0", "s78", "s79", "s88", "s89", "v229", "v230", LVX_BWD_LOOP_CLOBBERS
 #define LVX_BWD_D_OPERANDS                                                                                           \
-    : LVX_BWD_COMMON_OUT : LVX_BWD_COMMON_IN, "{v218}"(a_ds), "{s40}"(uniform32(p.scale))                            \
+    : LVX_BWD_COMMON_OUT : LVX_BWD_COMMON_IN, "{v218}"(a_ds[0]), "{v223}"(a_ds[1]), "{v224}"(a_ds[2]), "{v225}"(a_ds[3]), "{s40}"(uniform32(p.scale))                            \
     : "memory", "vcc", "scc", LVX_BWD_LOOP_CLOBBERS, "v219", "v220", "v221", "v222"
 
 // BIAS: a dense fp32 bias joins the exponent, P = exp2(S*c + bias*log2e - LSE*log2e).
@@ -228,10 +229,19 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         }
     }
     const int pb_off = slice * (2 * 64 * 8) + lane * 8;
-    // dS^T copy-out, also by the P-waves: 512 chunks of 16 bytes, two per thread (tokens t >> 2 and 64 + (t >> 2))
-    const int cp_token = (tid & 255) >> 2, cp_part = tid & 3;
-    // workspace tile (b, h, token block, row tile): [128 tokens][32 rows], 8 KB, contiguous
-    uint16_t* ws_lane = p.ds_ws + (int64_t)kblk * p.ws_ld + cp_token * BM + cp_part * 8;
+    // dS^T copy-out, also by the P-waves, each its own 32 tokens: two chunks of 8 tokens of row l32 per lane, tokens
+    // 8 g .. and 16 + 8 g .. of the slice, four tokens from each of two transposing reads.  Writes of 8 bytes (4 rows of
+    // a token) and these reads are both conflict-free.  (In rows of 80 bytes, copied out as they lay, 13 % of the kernel's LDS
+    // cycles were conflicts.)
+    uint32_t cp_rd[2];                 // of the first chunk; the second is 1024 bytes on
+    {
+        const int r = (lane & 15) >> 2, t = lane & 3, u = (lane >> 4) & 1;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+            cp_rd[half] = (uint32_t)((32 * slice + 8 * g + 4 * half + r) * 64 + ((2 * u + (t >> 1)) ^ (2 * g + half)) * 16 + (t & 1) * 8);
+    }
+    // workspace tile (b, h, token block, row tile): [16 groups of 8 tokens][32 rows][8 tokens], 8 KB, contiguous
+    uint16_t* ws_lane = p.ds_ws + (int64_t)kblk * p.ws_ld + (128 * slice + lane) * 8;
 
     // The walk over (head of the group, 32-row tile): per-head base addresses are
     // re-derived only when the head changes, everything else advances by constants.
@@ -299,15 +309,16 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
 
     // the finished dS^T tile goes to HBM as one contiguous 8 KB block
     auto copy_out = [&](const uint16_t* dst, int64_t ws_off) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(dst + cp_token * DSS + cp_part * 8);
-        const u32x4 c2 = *reinterpret_cast<const u32x4*>(dst + (cp_token + 64) * DSS + cp_part * 8);
+        const uint16_t *const r0 = dst + cp_rd[0] / 2, *const r1 = dst + cp_rd[1] / 2;
+        const u32x2 a0 = lds_read_tr16(r0), a1 = lds_read_tr16(r1), c0 = lds_read_tr16(r0 + 512), c1 = lds_read_tr16(r1 + 512);
+        const u32x4 a = {a0[0], a0[1], a1[0], a1[1]}, c2 = {c0[0], c0[1], c1[0], c1[1]};
         u32x4* const o = reinterpret_cast<u32x4*>(ws_lane + ws_off);
         if (p.ds_stream) {
             __builtin_nontemporal_store(a, o);
-            __builtin_nontemporal_store(c2, o + 64 * BM / 8);
+            __builtin_nontemporal_store(c2, o + 64);
         } else {
             o[0] = a;
-            o[64 * BM / 8] = c2;
+            o[64] = c2;
         }
     };
 
@@ -463,11 +474,11 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                                           E::hi(pu[j][e]) * fmaf(dp_carry[8 * j + 2 * e + 1], p.scale, -d1));
                 }
             }
-            uint16_t* dsp = dst + (32 * slice + l32) * DSS + 4 * g;
+            uint16_t* const dsp = dst + (32 * slice + l32) * BM + 4 * g;
 #pragma unroll
             for (int vg = 0; vg < 4; ++vg) {
                 const u32x2 w = {dsu[vg >> 1][2 * (vg & 1)], dsu[vg >> 1][2 * (vg & 1) + 1]};
-                *reinterpret_cast<u32x2*>(dsp + 8 * vg) = w;
+                *reinterpret_cast<u32x2*>(dsp + 8 * (vg ^ ((l32 >> 2) & 3))) = w;
             }
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
@@ -594,8 +605,8 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                     const int64_t hddo = uniform64((int64_t)p.dos.h * 2 - (int64_t)n_live * BM * dorow_b);
                     const int64_t hdws = uniform64((int64_t)p.ws_bh * 2 - (int64_t)n_live * (BN * BM * 2));
                     const int64_t hdm = uniform64(meta_w ? -(int64_t)n_live * (BM * 4) : (int64_t)(n_qtiles - n_live) * 256);
-                    const uint32_t a_cp = lds0 + OFF_DST * 2 + (uint32_t)(cp_token * DSS + cp_part * 8) * 2;
-                    const uint32_t g_cp0 = (uint32_t)(cp_token * BM + cp_part * 8) * 2, g_cp1 = g_cp0 + 64 * BM * 2;
+                    const uint32_t a_cp0 = lds0 + OFF_DST * 2 + cp_rd[0], a_cp1 = lds0 + OFF_DST * 2 + cp_rd[1];
+                    const uint32_t g_cp = (uint32_t)(128 * slice + lane) * 16;
                     // the four loads of a tile; in a window's last one the rows end at `last`
                     const int last = (p.row_end - p.row_begin - 1) % BM;
                     const bool ragged = last != BM - 1 && run_s[0] + n_live == n_qtiles;
@@ -649,7 +660,10 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                     w_q[3] = reinterpret_cast<const uint16_t*>(w3) - ws_k;
                     w_q[4] = reinterpret_cast<const uint16_t*>(w4) - ws_k;
                 } else {
-                    const uint32_t a_ds = lds0 + OFF_DST * 2 + (uint32_t)((32 * slice + l32) * DSS + 4 * g) * 2;
+                    uint32_t a_ds[4];
+#pragma unroll
+                    for (int vg = 0; vg < 4; ++vg)
+                        a_ds[vg] = lds0 + OFF_DST * 2 + (uint32_t)((32 * slice + l32) * BM + 8 * (vg ^ ((l32 >> 2) & 3)) + 4 * g) * 2;
                     if constexpr (!F16 && DH == 128) {
                         asm volatile(
 #include "lvx_bwd_loop_d_bf16_128.inc"

@@ -1,7 +1,6 @@
 // bf16 GEMM for the K/V recompute (K = X W_k, V = X W_v), its input gradient
 // (dX = dK W_k^T + dV W_v^T, one GEMM whose contraction runs over two operand
-// pairs), the weight gradients (dW = X^T dK) and the batched dQ = dS K of the
-// attention backward.  fp32 accumulate on v_mfma_f32_32x32x16_bf16, bf16 output.
+// pairs) and the weight gradients (dW = X^T dK).  fp32 accumulate on v_mfma_f32_32x32x16_bf16, bf16 output.
 //
 // Structure (8 waves, two per SIMD, in lock-step "ping-pong"):
 //  * Operand tiles go from global memory straight into LDS with
@@ -55,8 +54,7 @@ struct Region {
 
     // what lane `lane` of the wave loading chunk `ch` fetches: byte offset from the
     // stage base of the operand, and the k position inside the stage
-    __device__ __forceinline__ static uint32_t src(int ch, int lane, int r0, int R, int64_t ld, int tiled_m,
-                                                   int& kpos) {
+    __device__ __forceinline__ static uint32_t src(int ch, int lane, int r0, int R, int64_t ld, int& kpos) {
         if (!ROW_CONTIG) {
             const int row = 16 * ch + (lane >> 2);
             const int c = (lane & 3) ^ ((lane >> 4) & 3);
@@ -67,7 +65,6 @@ struct Region {
         const int q = (lane % LPR) ^ ((k & 3) << 2);
         kpos = k;
         const int r = min(r0 + q * 8, R - 8);
-        if (tiled_m) return (uint32_t)(k * 32 + (r >> 5) * 4096 + (r & 31)) * 2u;
         return (uint32_t)k * (uint32_t)ld * 2u + (uint32_t)(r - r0) * 2u;
     }
 
@@ -99,11 +96,7 @@ struct Region {
 };
 
 // GM x GN waves, each WM x WN MFMA tiles: work-group tile (32 WM GM) x (32 WN GN).
-// STREAM_A: A is loaded with the streaming hint (as a test at run time it costs a one-round dQ launch 10 %).
-// RANGED_A: a_tile_range is given.  A load of a wave takes two k of all eight row tiles, so a lane's row tile is
-// the same in every load; where that tile holds nothing its loads are sent out of a descriptor's range.  (With a zero
-// of one address, or of 2 KB of them, in its place the two forms of the load made the loop 6 % longer.)
-template <bool A_MCONTIG, bool B_NCONTIG, int GM, int GN, int WM, int WN, int NS, bool F16, bool STREAM_A = false, bool RANGED_A = false>
+template <bool A_MCONTIG, bool B_NCONTIG, int GM, int GN, int WM, int WN, int NS, bool F16>
 __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     using E = Elt<F16>;
     static_assert(GM * GN == 8, "8 waves");
@@ -118,52 +111,13 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE];
 
     fetch_kernargs<sizeof(GemmParams)>();
-    const int wid0 = p.m_order ? (int)blockIdx.x : xcd_remap(blockIdx.x, p.total_wg);
-    if (wid0 >= p.total_wg) return;
-    const int nks = p.k_splits > 1 ? p.k_splits : 1;
-    uint32_t ksp, tn, tm, zo, zi, prob = 0;
-    const uint32_t t1 = p.by_tiles_n.split(p.by_splits.split(wid0, ksp), tn);
-    if (p.m_order) {
-        // M tiles with their own contraction ranges, ranked by length: the ids walk the ranking
-        // (the inner batch index fastest), so the hardware's in-order hand-out of work-groups
-        // starts the longest first, on every XCD alike
-        zo = p.by_tiles_m.split((uint32_t)p.m_order[p.by_inner.split(t1, zi)], tm);
-    } else {
-        // the outer batch index (the sample, where there is one) varies fastest over the ids, so that
-        // every XCD's contiguous id range holds work of all samples (ragged ones differ in length)
-        uint32_t zr;
-        prob = p.by_nbatch.split(p.by_tiles_m.split(t1, tm), zr);
-        zi = p.by_outer.split(zr, zo);
-    }
+    const int wid = xcd_remap(blockIdx.x, p.total_wg);
+    if (wid >= p.total_wg) return;
+    uint32_t tn, tm;
+    const uint32_t prob = p.by_tiles_m.split(p.by_tiles_n.split(wid, tn), tm);
     const GemmProblem& pr = p.prob[prob];
-    const int z = zo * p.batch_inner + zi;
     const int m0 = tm * TM, n0 = tn * TN;
-    const int64_t a_off = (int64_t)z * p.a_batch;
-    const int64_t b_off = zo * p.b_outer + p.by_group.quotient(zi) * p.b_inner;
-    uint16_t* const Cz = pr.C + zo * p.c_outer + zi * p.c_inner;
-    int klen0 = pr.K[0];
-    if (p.k_len) klen0 = min(klen0, p.k_len[zo]);
-    int k_lo = 0;                                   // start of this work-group's k range
-    if (nks > 1) { k_lo = ksp * p.k_split_len; klen0 = min(klen0, k_lo + p.k_split_len); }
-    uint32_t a_lo = 0, a_len = 0;                   // k of this lane's row tile of A
-    if constexpr (RANGED_A) {
-        static_assert(A_MCONTIG && TM == 256, "eight row tiles, four lanes each");
-        const int ln = threadIdx.x & 63, k4 = 2 * ((threadIdx.x >> 6) & 1) + (ln >> 5);      // k mod 4 of its loads
-        const int t = min((m0 >> 5) + (((ln & 31) >> 2) ^ k4), p.a_tiled_m - 1);
-        const int32_t* r = p.a_tile_range + ((int64_t)zo * p.a_tiled_m + t) * 2;
-        a_lo = (uint32_t)r[0];
-        a_len = (uint32_t)(r[1] - r[0]);
-        int lo = r[1] ? r[0] : 0x7fffffff, hi = r[1];
-#pragma unroll
-        for (int off = 4; off < 32; off <<= 1) {
-            lo = min(lo, __shfl_xor(lo, off));
-            hi = max(hi, __shfl_xor(hi, off));
-        }
-        k_lo = max(k_lo, uniform32(min(lo, hi)));
-        klen0 = min(klen0, uniform32(hi));
-    }
-    klen0 = max(0, klen0 - k_lo);
-    const int s_lo = k_lo / BK;                    // first stage of this work-group's k range
+    const int klen0 = pr.K[0];
     const int klen1 = pr.nseg > 1 ? pr.K[1] : 0;
 
     const int tid = threadIdx.x;
@@ -179,47 +133,39 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
 #pragma unroll
     for (int j = 0; j < LPG; ++j) {
         const int ch = wave + 8 * j;
-        if (j < LPG_A) voff[j] = RA::src(ch, lane, m0, p.M_ld, lda, p.a_tiled_m, kpos[j]) - (RANGED_A ? (uint32_t)(m0 >> 5) * 8192u : 0u);
-        else voff[j] = RB::src(ch - RA::CHUNKS, lane, n0, p.N, ldb, 0, kpos[j]);
+        if (j < LPG_A) voff[j] = RA::src(ch, lane, m0, p.M, lda, kpos[j]);
+        else voff[j] = RB::src(ch - RA::CHUNKS, lane, n0, p.N, ldb, kpos[j]);
     }
     const char* abase[2];
     const char* bbase[2];
 #pragma unroll
     for (int sg = 0; sg < 2; ++sg) {
         const int ss = sg < pr.nseg ? sg : 0;
-        abase[sg] = reinterpret_cast<const char*>(pr.A[ss] + a_off);
-        if (RANGED_A) abase[sg] += (int64_t)(m0 >> 5) * 8192;
-        else if (!p.a_tiled_m) abase[sg] += (A_MCONTIG ? (int64_t)m0 : (int64_t)m0 * lda) * 2;
-        bbase[sg] = reinterpret_cast<const char*>(pr.Bm[ss] + b_off) + (B_NCONTIG ? (int64_t)n0 : (int64_t)n0 * ldb) * 2;
+        abase[sg] = reinterpret_cast<const char*>(pr.A[ss]) + (A_MCONTIG ? (int64_t)m0 : (int64_t)m0 * lda) * 2;
+        bbase[sg] = reinterpret_cast<const char*>(pr.Bm[ss]) + (B_NCONTIG ? (int64_t)n0 : (int64_t)n0 * ldb) * 2;
     }
-    const int64_t a_kstride = A_MCONTIG ? lda * BK * 2 : BK * 2;   // bytes per stage (untiled)
+    const int64_t a_kstride = A_MCONTIG ? lda * BK * 2 : BK * 2;   // bytes per stage
     const int64_t b_kstride = B_NCONTIG ? ldb * BK * 2 : BK * 2;
     const int steps0 = (klen0 + BK - 1) / BK;
     const int steps = steps0 + (klen1 + BK - 1) / BK;
 
     auto issue = [&](int s) {     // loads of stage s into ring slot s % NS
         const int sg = s >= steps0 ? 1 : 0;
-        const int kr = sg ? s - steps0 : s;            // stage inside this work-group's range
-        const int krem = (sg ? klen1 : klen0) - kr * BK;
-        const int ks = sg ? kr : kr + s_lo;            // stage inside the operand
-        const char* ab = abase[sg] + ks * a_kstride;
-        if (A_MCONTIG && p.a_tiled_m)   // tiled A: [k / 128][m / 32][128 k][32 m]
-            ab = abase[sg] + ((int64_t)(ks >> 2) * p.a_tiled_m * 4096 + (ks & 3) * (BK * 32)) * 2;
-        const char* bb = bbase[sg] + ks * b_kstride;
+        const int ks = sg ? s - steps0 : s;            // stage inside the operand
+        const int krem = (sg ? klen1 : klen0) - ks * BK;
+        const char* const ab = abase[sg] + ks * a_kstride;
+        const char* const bb = bbase[sg] + ks * b_kstride;
         const uint32_t slot = lds0 + (uint32_t)(s % NS) * STAGE + (uint32_t)wave * 1024u;
-        const bool a_mine = !RANGED_A || (uint32_t)(ks * BK) - a_lo < a_len;
         if (krem >= BK) {
 #pragma unroll
             for (int j = 0; j < LPG; ++j)
-                if (RANGED_A && j < LPG_A) dma16_range<STREAM_A>(ab, TM / 32 * 8192, a_mine ? voff[j] : 0x80000000u, slot + j * 8192);
-                else if (STREAM_A && j < LPG_A) dma16_stream(ab, voff[j], slot + j * 8192);
-                else dma16(j < LPG_A ? ab : bb, voff[j], slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
+                dma16(j < LPG_A ? ab : bb, voff[j], slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
         } else {
             const char* zc = reinterpret_cast<const char*>(zero_chunk);
 #pragma unroll
             for (int j = 0; j < LPG; ++j) {
                 const char* src = (j < LPG_A ? ab : bb) + voff[j];
-                dma16_addr(kpos[j] < krem && (j >= LPG_A || a_mine) ? src : zc, slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
+                dma16_addr(kpos[j] < krem ? src : zc, slot + (j < LPG_A ? j * 8192 : RA::BYTES + (j - LPG_A) * 8192));
             }
         }
     };
@@ -282,25 +228,6 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
     if (set == 0) phase_barrier();
 
     // C^T tile: accumulator rows = n, cols = m
-    if (nks > 1) {   // partial tile of a split contraction: fp32, into this split's slice
-        float* const C32 = p.c32 + ksp * p.c32_split + (int64_t)z * p.c32_batch;
-#pragma unroll
-        for (int mt = 0; mt < WM; ++mt) {
-            const int m = m0 + 32 * (WM * wm + mt) + l32;
-            if (m >= p.M) continue;
-#pragma unroll
-            for (int nt = 0; nt < WN; ++nt)
-#pragma unroll
-                for (int vg = 0; vg < 4; ++vg) {
-                    const int n = n0 + 32 * (WN * wn + nt) + 8 * vg + 4 * g;
-                    if (n < p.N) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) C32[(int64_t)(n + r) * p.c32_ld + m] = acc[nt][mt][4 * vg + r];
-                    }
-                }
-        }
-        return;
-    }
     // A lane holds 4 consecutive columns of one C row, so storing from the registers writes 8
     // bytes per lane into 32 different rows per instruction.  The rows go through the stage buffers
     // (free by now) instead, 256 at a time, and leave as whole row segments (TN * 2 bytes; N is a
@@ -386,7 +313,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
                 w[0] = E::pack(acc[nt][mt][4 * vg], acc[nt][mt][4 * vg + 1]);
                 w[1] = E::pack(acc[nt][mt][4 * vg + 2], acc[nt][mt][4 * vg + 3]);
                 return w;
-            }, p.c_raw + (Cz - pr.C));
+            }, p.c_raw);
         store_via_lds([&](int mt, int nt, int vg) {
             const int n = 32 * (WN * wn + nt) + 8 * vg + 4 * g;       // n0 is a multiple of 128
             const u32x2 wt = *reinterpret_cast<const u32x2*>(p.norm_w + (n & 127));
@@ -397,7 +324,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
             y[0] = E::pack(E::lo(wt[0]) * E::lo(h[0]), E::hi(wt[0]) * E::hi(h[0]));
             y[1] = E::pack(E::lo(wt[1]) * E::lo(h[1]), E::hi(wt[1]) * E::hi(h[1]));
             return y;
-        }, Cz);
+        }, pr.C);
         return;
     }
     store_via_lds([&](int mt, int nt, int vg) {
@@ -405,7 +332,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmParams p) {
         w[0] = E::pack(acc[nt][mt][4 * vg], acc[nt][mt][4 * vg + 1]);
         w[1] = E::pack(acc[nt][mt][4 * vg + 2], acc[nt][mt][4 * vg + 3]);
         return w;
-    }, Cz);
+    }, pr.C);
 }
 
 // registers the hand-scheduled tile uses besides its operands (see gen_gemm_loop.py)
@@ -488,7 +415,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
         if (j >= NL) { voff[j] = vtail[j] = 0; continue; }
         int kpos;
         const int ch = wave + 4 * (j < NLA ? j : j - NLA);
-        voff[j] = j < NLA ? RA::src(ch, lane, m0, p.M_ld, lda, kpos) : RB::src(ch, lane, n0, p.N, ldb, kpos);
+        voff[j] = j < NLA ? RA::src(ch, lane, m0, p.M, lda, kpos) : RB::src(ch, lane, n0, p.N, ldb, kpos);
         vtail[j] = tail && kpos >= tail && !(j < NLA ? A_T : B_T) ? 0x80000000u : voff[j];
         if (nst == 1) voff[j] = vtail[j];
     }
@@ -669,21 +596,14 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_kernel(const GemmParams p) {
     }
 }
 
-// The tiles of a launch and the divisors by what its work-group numbers are made of.  (With the arguments fetched line by
-// line and eight integer divisions a work-group of a small dQ launch lost 0.6 us of 26 before its first load.)
+// The tiles of a launch and the divisors by what its work-group numbers are made of.
 void fill_tiles(GemmParams& p, int TM, int TN) {
-    const int splits = p.k_splits > 1 ? p.k_splits : 1;
     p.tiles_m = (p.M + TM - 1) / TM;
     p.tiles_n = (p.N + TN - 1) / TN;
-    p.total_wg = p.nprob * p.nbatch * p.tiles_m * p.tiles_n * splits;
-    p.by_splits = divisor(splits);
+    p.total_wg = p.nprob * p.tiles_m * p.tiles_n;
     p.by_tiles_n = divisor(p.tiles_n);
     p.by_tiles_m = divisor(p.tiles_m);
     p.by_nprob = divisor(p.nprob);
-    p.by_nbatch = divisor(p.nbatch);
-    p.by_inner = divisor(p.batch_inner);
-    p.by_outer = divisor(p.nbatch / p.batch_inner);
-    p.by_group = divisor(p.b_group);
 }
 
 template <int GM, int GN, int WM, int WN, int NS, bool F16>
@@ -694,14 +614,6 @@ hipError_t launch_cfg_t(const GemmParams& p, int grid, bool a_mcontig, bool b_nc
         return launch1((gemm_kernel<false, true, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
     else if (a_mcontig && !b_ncontig)
         return launch1((gemm_kernel<true, false, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
-    if constexpr (32 * WN * GN == 128) {       // the dQ GEMM
-        if (p.a_tile_range && p.a_stream)
-            return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16, true, true>), dim3(grid), dim3(512), st, p);
-        if (p.a_tile_range)
-            return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16, false, true>), dim3(grid), dim3(512), st, p);
-        if (p.a_stream)
-            return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16, true>), dim3(grid), dim3(512), st, p);
-    }
     return launch1((gemm_kernel<true, true, GM, GN, WM, WN, NS, F16>), dim3(grid), dim3(512), st, p);
 }
 
@@ -724,11 +636,11 @@ hipError_t launch_tile(GemmParams p, bool a_mcontig, bool b_ncontig, hipStream_t
     return hipErrorInvalidValue;
 }
 
-// What gemm_tile_kernel takes: no batch, one contraction length for both segments (whole stages of it where
+// What gemm_tile_kernel takes: one contraction length for both segments (whole stages of it where
 // there are two), offsets inside an operand below 2^32, and not the layout nothing uses.
 bool gemm_tile_ok(const GemmParams& p, bool a_mcontig, bool b_ncontig) {
     const GemmProblem& pr = p.prob[0];
-    if (p.nbatch != 1 || p.k_len || p.a_tile_range || p.k_splits > 1 || p.a_tiled_m || (a_mcontig && !b_ncontig)) return false;
+    if (a_mcontig && !b_ncontig) return false;
     if (pr.nseg > 1 && (pr.K[1] != pr.K[0] || pr.K[0] % TK)) return false;
     // (the descriptor of a row-major operand covers 2 GiB, the other kind ends with the contraction)
     const int64_t limit = (int64_t)1 << 32;
@@ -741,10 +653,7 @@ bool gemm_tile_ok(const GemmParams& p, bool a_mcontig, bool b_ncontig) {
 
 // Work-group tile by shape.  C wider than 128 columns (projections, their gradients): a hand-scheduled tile of 256 x 256,
 // 256 x 128 or 224 x 256 (gemm_tile).
-// A narrow C (the dQ GEMM): 256 x 128, four stages, at which one load of a wave covers whole cache lines of
-// dS^T's 64-byte rows (two tokens x 256 rows; of a 512-row tile it takes one token, half of each line, and the
-// streaming hint then costs a second fetch: 6404 tokens x 4096 rows x 32 heads 1868 us a step against 1821),
-// and the M tiles of a masked launch have finer contraction ranges.
+// A narrow C: 256 x 128, four stages.
 hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipStream_t st) {
     if (p.N % 8) return hipErrorInvalidValue;
     for (int i = 0; i < p.nprob; ++i) {
@@ -761,8 +670,6 @@ hipError_t launch_gemm(const GemmParams& p, bool a_mcontig, bool b_ncontig, hipS
         }
     }
     if (p.N > 128) return launch_cfg<2, 4, 4, 2, 4>(p, a_mcontig, b_ncontig, st);
-    if (p.a_tile_range && (!a_mcontig || !b_ncontig || p.a_tiled_m <= 0 || p.N > 128)) return hipErrorInvalidValue;
-    if (p.m_order && (!p.a_tile_range || p.nprob != 1 || p.k_splits > 1 || p.N > 128)) return hipErrorInvalidValue;
     return launch_cfg<4, 2, 2, 2, 4>(p, a_mcontig, b_ncontig, st);
 }
 

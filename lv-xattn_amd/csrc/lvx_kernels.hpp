@@ -137,7 +137,7 @@ struct BwdParams {
     const uint16_t* v;
     const uint16_t* dout;
     const float* meta;         // per (b, h, 32-row tile): 32 x LSE*log2(e) (+inf for dead rows), 32 x delta*scale
-    uint16_t* ds_ws;           // dS^T workspace [B*Hq][token blocks][row tiles][128 tokens][32 rows]
+    uint16_t* ds_ws;           // dS^T workspace [B*Hq][token blocks][row tiles][16 groups of tokens][32 rows][8 tokens]
     int64_t ws_ld;             // elements per token block (row tiles * 4096)
     int64_t ws_bh;             // elements per (b, h) slab
     int ds_stream;             // 1: dS^T is stored with streaming stores (see lvx_bwd)
@@ -239,6 +239,36 @@ struct CastParams {
     uint32_t blocks_per_xcd;        // and a share of the grid
 };
 
+// dQ = (scale dS) K of a window of `rows` rows, from the dS^T workspace.
+struct DqParams {
+    const uint16_t* ds;        // dS^T tiles [B * Hq][token blocks][row tiles][16 groups of tokens][32 rows][8 tokens]
+    int64_t ds_bh;             // elements per (b, h)
+    const uint16_t* k;
+    uint16_t* dq;              // of the window's first row
+    Strides3 ks, dqs;
+    int B, Hq, G, rows, row_tiles, Lkv;
+    int D;                     // head dimension: 16, 32, 64 or 128
+    int f16;                   // element type of dS^T, k and dq
+    int stream;                // 1: dS^T is loaded with the streaming hint
+    const int32_t* kv_len;     // null or [B]: tokens past it are not contracted
+    // Null, or [B][row_tiles][2]: the tokens at which a row tile holds anything, first and one-past-last (multiples of
+    // 128; 0, 0: nowhere).  Elsewhere it counts as zeros and is not read.
+    const int32_t* tile_range;
+    // With tile_range and one split: the (sample, group of 8 row tiles) pairs b * groups + group in the order the work-groups
+    // are to take them, longest first (null: in index order).
+    const int32_t* order;
+    // k_splits > 1: as many work-groups per tile of dQ, each contracting split_len tokens (a multiple of 128) into
+    // an fp32 slice of its own, part[split * part_split + (b * Hq + h) * D * rows + d * rows + row] (zeros where its range
+    // is empty); the caller sums the slices.
+    int k_splits, split_len;
+    float* part;
+    int64_t part_split;
+    // filled in by launch_dq
+    int total_wg;
+    Divisor by_splits, by_tiles_m, by_B, by_Hq, by_G;
+};
+hipError_t launch_dq(const DqParams& p, hipStream_t st);
+
 // One GEMM problem C[M,N] = sum over segments A_s[M,K_s] * B_s[K_s,N].
 struct GemmProblem {
     const uint16_t* A[2];
@@ -250,20 +280,12 @@ struct GemmProblem {
     int64_t ldc;
 };
 
-// `nprob` problems of one shape, each repeated over `nbatch` batch entries.
-// Batch entry z = zo * batch_inner + zi addresses
-//   A + z * a_batch,  B + zo * b_outer + (zi / b_group) * b_inner,
-//   C + zo * c_outer + zi * c_inner
-// and, when k_len is given, contracts over only the first k_len[zo] values of k.
+// `nprob` problems of one shape.
 struct GemmParams {
     GemmProblem prob[2];
     int nprob;
     int M, N;
-    int M_ld;                  // rows of A that may be loaded (>= M; rows in [M, M_ld) are padding)
     int tiles_m, tiles_n, total_wg;   // filled in by launch_gemm for the tile it picks
-    int nbatch, batch_inner, b_group;
-    int64_t a_batch, b_outer, b_inner, c_outer, c_inner;
-    const int32_t* k_len;
     // RMS norm over each aligned group of 128 columns of problem 0's C (the k_norm of the K
     // projection), applied to the accumulator before the store: y = bf16(w * bf16(x * r)),
     // r = rsqrt(mean(x^2) + eps), x = the bf16-rounded product.  norm_w: 128 bf16 weights
@@ -273,32 +295,8 @@ struct GemmParams {
     float norm_eps;
     uint16_t* c_raw;
     float* rstd;
-    // With a_tiled_m (null: off): per (outer batch index, 32-row tile of A) the k at which the tile holds anything,
-    // a_tile_range[(zo * a_tiled_m + tile) * 2 + {0, 1}] = first and one-past-last (multiples of 128; 0, 0: nowhere).
-    // An M tile contracts over the hull of its tiles' ranges; outside its own a tile counts as zeros and is not read.
-    const int32_t* a_tile_range;
-    // With a_tile_range (one problem, no split contraction): the (outer batch index, M tile) pairs
-    // zo * tiles_m + tm in the order the work-groups are to take them, longest range first
-    // (null: in index order).
-    const int32_t* m_order;
     int f16;                   // element type of A, B, C (and the norm weight): 0 bf16, 1 fp16
-    // Split contraction (single-segment problems): k_splits work-groups per C tile, each
-    // contracting k_split_len values of k (a multiple of 128) and storing its partial tile
-    // in fp32 to its own slice of the TRANSPOSED scratch
-    // c32[split * c32_split + z * c32_batch + n * c32_ld + m] (the accumulator holds C^T, so
-    // a wave's lanes then write consecutive addresses; every split writes its whole tile,
-    // zeros if its range is empty) instead of storing bf16 to C; the caller sums the slices.
-    // k_splits <= 1: off.
-    int k_splits, k_split_len;
-    float* c32;
-    int64_t c32_split, c32_batch;
-    int c32_ld;
-    // a_tiled_m > 0: A (stored [K][M]) is cut into contiguous [128 k][32 m] tiles,
-    // a_tiled_m of them per block of 128 k; lda is ignored
-    int a_tiled_m;
-    int a_stream;              // 1: A is loaded with the streaming hint (A and B stored [K][..] only)
-    // filled in by launch_gemm: divisors by k_splits, tiles_n, tiles_m, nprob, nbatch, batch_inner, their quotient, b_group
-    Divisor by_splits, by_tiles_n, by_tiles_m, by_nprob, by_nbatch, by_inner, by_outer, by_group;
+    Divisor by_tiles_n, by_tiles_m, by_nprob;      // filled in by launch_gemm: divisors by tiles_n, tiles_m, nprob
 };
 
 hipError_t launch_fwd(const FwdParams& p, bool masked, hipStream_t st);   // p.bias selects the bias variant
