@@ -561,22 +561,40 @@ static size_t dkv_scratch_bytes(const lvx_attn_shape* s) {
     return (size_t)2 * s->B * s->Lkv * s->Hkv * s->D * sizeof(float);
 }
 
-// The dQ GEMM of a small row window (a one-round launch, or few rows against many tokens) has
-// fewer C tiles than the chip has compute units; its
-// contraction over the tokens is then split over several work-groups that store fp32
-// partial tiles, each split into its own slice of a scratch; the slices are summed and
-// rounded to bf16 afterwards (fp32 atomics into one slice were measured slower).  Returns
-// the number of splits (1: none) and the tokens per split.
-static int dq_k_splits(const lvx_attn_shape* s, int32_t row_count, int* split_len) {
-    const int tiles = (row_count + 255) / 256;          // of dq_kernel's 256 rows
-    const int wgs = s->B * s->Hq * tiles;
-    const int blocks = (s->Lkv + 127) / 128;
-    int ks = 1;
+// How the dQ product of a window is cut.  A window of few rows has fewer tiles of 256 rows than half the compute units: it takes
+// work-groups of 64 rows (dq_few_kernel) then or, where those come out worse in rounds, stays with 256.  Where either leaves
+// CUs idle the contraction over the tokens is split over several work-groups that store fp32 partial tiles, each split
+// into its own slice of a scratch; the slices are summed and rounded to bf16 afterwards (fp32 atomics into one slice were
+// measured slower).
+struct DqCut {
+    bool few;
+    int splits, split_len;      // 1: none; tokens per split
+};
+
+// Splits of the contraction for this many work-groups without.
+static int dq_splits(int64_t wgs, int blocks) {
     const int n_cu = cu_count();
-    if (wgs <= n_cu / 2) ks = std::min(std::min(8, n_cu / wgs), blocks);
-    const int per = (blocks + ks - 1) / ks;
-    *split_len = per * 128;
-    return (blocks + per - 1) / per;
+    return wgs <= n_cu / 2 ? std::min(std::min(8, n_cu / (int)wgs), blocks) : 1;
+}
+
+static DqCut dq_cut(const lvx_attn_shape* s, int32_t row_count) {
+    constexpr int FEW = 32 * DQ_FEW_TILES;
+    const int blocks = (s->Lkv + 127) / 128, n_cu = cu_count();
+    const int64_t heads = (int64_t)s->B * s->Hq, wgs = heads * ((row_count + 255) / 256), wgs_few = heads * ((row_count + FEW - 1) / FEW);
+    DqCut cut{false, dq_splits(wgs, blocks), 0};
+    if (wgs <= n_cu / 2) {
+        // us: a CU reads 256 rows of dS^T at 22 ns a token; slices cost a launch and their bytes twice
+        auto us = [&](int64_t n, int ks, double rows) {
+            const double slices = ks > 1 ? 4.0 + (double)ks * heads * row_count * s->D * 8 / 5e6 : 0.0;
+            return (double)((n * ks + n_cu - 1) / n_cu) / ks * s->Lkv * 0.022 * rows / 256 + slices;
+        };
+        const int ks = dq_splits(wgs_few, blocks);
+        if (us(wgs_few, ks, FEW) <= us(wgs, cut.splits, 256)) { cut.few = true; cut.splits = ks; }
+    }
+    const int per = (blocks + cut.splits - 1) / cut.splits;
+    cut.split_len = per * 128;
+    cut.splits = (blocks + per - 1) / per;
+    return cut;
 }
 
 // Bytes of the split contraction's partial tiles that a window of up to row_count rows can need.  Fewer rows may
@@ -584,13 +602,13 @@ static int dq_k_splits(const lvx_attn_shape* s, int32_t row_count, int* split_le
 // 256 rows 33.6 MB, 4 of 257 18.9 MB), and a call sizes its workspace for the longest of its windows.
 static size_t dq_partial_bytes(const lvx_attn_shape* s, int32_t row_count) {
     size_t most = 0;
-    for (int32_t r = 0; r < row_count;) {
-        r = row_count - r > 256 ? r + 256 : row_count;
-        int split_len;
-        const int ks = dq_k_splits(s, r, &split_len);
-        if (ks <= 1) break;             // nor do longer windows split
-        most = std::max(most, (size_t)ks * s->B * s->Hq * (((size_t)r + 31) / 32 * 32) * s->D * sizeof(float));
-    }
+    for (const int step : {256, 32 * DQ_FEW_TILES})
+        for (int32_t r = 0; r < row_count;) {
+            r = row_count - r > step ? r + step : row_count;
+            const int ks = dq_splits((int64_t)s->B * s->Hq * ((r + step - 1) / step), (s->Lkv + 127) / 128);
+            if (ks <= 1) break;             // nor do longer windows split
+            most = std::max(most, (size_t)ks * s->B * s->Hq * (((size_t)r + 31) / 32 * 32) * s->D * sizeof(float));
+        }
     return most;
 }
 
@@ -696,9 +714,8 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     p.q_splits2 = cut.splits2;
     p.dkv_mode = cut.any_split() ? 2 : (dkv_accumulate ? 1 : 0);
     float* const scratch = (cut.any_split() && !dkv_accumulate) ? reinterpret_cast<float*>(wsb + wsl.dkv) : nullptr;
-    int split_len = 0;
-    const int ks = dq_k_splits(s, row_count, &split_len);
-    float* const dq32 = ks > 1 ? reinterpret_cast<float*>(wsb + wsl.dq32) : nullptr;
+    const DqCut dq_by = dq_cut(s, row_count);
+    float* const dq32 = dq_by.splits > 1 ? reinterpret_cast<float*>(wsb + wsl.dq32) : nullptr;
     // the token blocks several work-groups share, and the fp32 scratch of the call that sums them
     SharedBlocks sb{s->B, s->Hkv, s->Lkv, s->D, p.n_kv_blocks, p.n_blocks, p.blocks_per_xcd, p.whole_blocks};
     {
@@ -717,7 +734,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
         hull = reinterpret_cast<int32_t*>(wsb + wsl.hull);
         // the ranking is quadratic in the number of groups; where there are that many, the dQ
         // GEMM's work-groups even out in index order
-        if (ks <= 1 && s->B * wsl.n_groups <= MAX_RANKED_GROUPS) order = reinterpret_cast<int32_t*>(wsb + wsl.order);
+        if (!dq_by.few && dq_by.splits <= 1 && s->B * wsl.n_groups <= MAX_RANKED_GROUPS) order = reinterpret_cast<int32_t*>(wsb + wsl.order);
         LiveParams lp{s->kv_len, s->kv_start, s->kv_end, hull, reinterpret_cast<int32_t*>(wsb + wsl.runs), order,
                       s->B, s->Lq, s->Lkv, row_begin,
                       row_begin + row_count, wsl.n_tiles, wsl.n_groups, p.n_kv_blocks};
@@ -758,12 +775,13 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     g.kv_len = s->kv_len;
     g.tile_range = hull;         // [B][row tiles][2]
     g.order = order;
+    g.few = dq_by.few;
     // split contraction: every split stores its partial tiles in its own fp32 slice; the
     // cast sums the slices and rounds into dq
-    g.k_splits = ks; g.split_len = split_len;
+    g.k_splits = dq_by.splits; g.split_len = dq_by.split_len;
     g.part = dq32; g.part_split = (int64_t)s->B * s->Hq * row_count * s->D;      // [split][B * Hq][D][row_count]
     e = launch_dq(g, st);
-    if (e != hipSuccess || ks <= 1) return static_cast<int>(e);
+    if (e != hipSuccess || dq_by.splits <= 1) return static_cast<int>(e);
     CastParams cq{};
     cq.f16 = p.f16;
     cq.D = s->D;
@@ -772,7 +790,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     cq.ds = st3(dq);
     cq.B = s->B; cq.H = s->Hq; cq.L = row_count;
     cq.transposed = 1;
-    cq.nsum = ks; cq.sum_stride = g.part_split;
+    cq.nsum = dq_by.splits; cq.sum_stride = g.part_split;
     return static_cast<int>(launch_cast(cq, st));
 }
 

@@ -239,6 +239,8 @@ struct CastParams {
     uint32_t blocks_per_xcd;        // and a share of the grid
 };
 
+constexpr int DQ_FEW_TILES = 2;    // row tiles a work-group of dq_few_kernel takes
+
 // dQ = (scale dS) K of a window of `rows` rows, from the dS^T workspace.
 struct DqParams {
     const uint16_t* ds;        // dS^T tiles [B * Hq][token blocks][row tiles][16 groups of tokens][32 rows][8 tokens]
@@ -254,7 +256,8 @@ struct DqParams {
     // Null, or [B][row_tiles][2]: the tokens at which a row tile holds anything, first and one-past-last (multiples of
     // 128; 0, 0: nowhere).  Elsewhere it counts as zeros and is not read.
     const int32_t* tile_range;
-    // With tile_range and one split: the (sample, group of 8 row tiles) pairs b * groups + group in the order the work-groups
+    int few;                   // 1: dq_few_kernel, work-groups of DQ_FEW_TILES row tiles (0: of eight)
+    // With tile_range and one split, not few: the (sample, group of 8 row tiles) pairs b * groups + group in the order the work-groups
     // are to take them, longest first (null: in index order).
     const int32_t* order;
     // k_splits > 1: as many work-groups per tile of dQ, each contracting split_len tokens (a multiple of 128) into

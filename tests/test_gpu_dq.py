@@ -11,10 +11,12 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# 40 heads x 2 samples x 2 groups: more work-groups than half the CUs, one range; the others are cut into several
+# 40 heads x 2 samples x 2 groups: more work-groups than half the CUs; 10 x 2 x 9: work-groups of 64 rows, one range; the others
+# are cut into several
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("Hq,Hkv,D,Lq,Lkv,short", [
     (40, 2, 64, 300, 200, 163), (40, 4, 16, 257, 129, 1), (20, 20, 32, 513, 300, 257), (34, 1, 128, 290, 161, 159),
+    (10, 2, 128, 513, 300, 257), (8, 8, 64, 1000, 260, 129), (9, 3, 16, 577, 1000, 930),
     (2, 1, 128, 1, 33, 31), (2, 2, 128, 31, 500, 255), (1, 1, 64, 257, 1000, 641), (2, 1, 16, 33, 700, 384), (1, 1, 128, 64, 64, 64)])
 def test_dq(Hq, Hkv, D, Lq, Lkv, short, dtype):
     import lv_xattn
