@@ -583,13 +583,14 @@ static DqCut dq_cut(const lvx_attn_shape* s, int32_t row_count) {
     const int64_t heads = (int64_t)s->B * s->Hq, wgs = heads * ((row_count + 255) / 256), wgs_few = heads * ((row_count + FEW - 1) / FEW);
     DqCut cut{false, dq_splits(wgs, blocks), 0};
     if (wgs <= n_cu / 2) {
-        // us: a CU reads 256 rows of dS^T at 22 ns a token; slices cost a launch and their bytes twice
-        auto us = [&](int64_t n, int ks, double rows) {
+        // us: a CU takes 20.5 ns a token for 256 rows (dS^T) and 6.7 for 64 (as much of K); slices cost a launch and their
+        // bytes twice.  16 heads of 64, 464 rows x 22786 tokens: 58 + 6 with 256 rows, 73 + 5 with 64
+        auto us = [&](int64_t n, int ks, double per_token) {
             const double slices = ks > 1 ? 4.0 + (double)ks * heads * row_count * s->D * 8 / 5e6 : 0.0;
-            return (double)((n * ks + n_cu - 1) / n_cu) / ks * s->Lkv * 0.022 * rows / 256 + slices;
+            return (double)((n * ks + n_cu - 1) / n_cu) / ks * s->Lkv * per_token + slices;
         };
         const int ks = dq_splits(wgs_few, blocks);
-        if (us(wgs_few, ks, FEW) <= us(wgs, cut.splits, 256)) { cut.few = true; cut.splits = ks; }
+        if (us(wgs_few, ks, 0.0067) <= us(wgs, cut.splits, 0.0205)) { cut.few = true; cut.splits = ks; }
     }
     const int per = (blocks + cut.splits - 1) / cut.splits;
     cut.split_len = per * 128;
