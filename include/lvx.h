@@ -97,6 +97,9 @@ const char* lvx_strerror(int code);
  * (at most 64 ranges; lvx_fwd_auto_splits says how many suit a launch).  The O of a range waits for the
  * fold in 16 bits, a rounding that a launch of one range does not have (its error against exact arithmetic
  * grows by about a fifth), or with kv_splits = n | LVX_SPLITS_FP32 in fp32, in twice the workspace.
+ * With LVX_SPLITS_ROUNDS(n) added to kv_splits the rows are computed as n query blocks that visit one after the other: a launch
+ * for each, of ceil(row_count / n) rows.  The results are those of n calls; where the parts of a block's key ranges are 16-bit
+ * its fold rides in the launch of the next block, and the workspace holds the parts of two blocks.
  * The kernel has three forms: a wavefront owns 32 text rows of a head (with a dense bias, and at head_dim
  * 16 and 32); 64 rows and its SIMD to itself (head_dim 128 and 64 without a bias); or, where that is
  * estimated to take less, a share of the keys for up to 32 (row, head) pairs of a kv head at once (few rows
@@ -124,6 +127,7 @@ int lvx_fwd_acc(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tens
                 void* workspace, size_t workspace_bytes, void* stream);
 
 #define LVX_SPLITS_FP32 256
+#define LVX_SPLITS_ROUNDS(n) ((int32_t)(n) << 12)    /* n up to 2^18 */
 size_t lvx_fwd_workspace_bytes(const lvx_attn_shape* shape, int32_t row_count, int32_t kv_splits);
 
 /*

@@ -1,6 +1,7 @@
 // C-ABI layer: argument validation on the host (nothing is launched when a
 // check fails), translation to the internal launch parameters, error strings.
 #include "../../include/lvx.h"
+#include "lvx_fold.hpp"
 #include "lvx_kernels.hpp"
 
 #include <algorithm>
@@ -129,7 +130,16 @@ const char* lvx_strerror(int code) {
     return "unknown lvx error";
 }
 
+// The rounds that kv_splits asks for (1: none), taken out of it.
+static int fwd_rounds(int32_t& kv_splits) {
+    const int rounds = kv_splits > 0 ? kv_splits >> 12 : 0;
+    if (rounds > 0) kv_splits &= (1 << 12) - 1;
+    return std::max(rounds, 1);
+}
+
 size_t lvx_fwd_workspace_bytes(const lvx_attn_shape* s, int32_t row_count, int32_t kv_splits) {
+    if (const int rounds = fwd_rounds(kv_splits); rounds > 1 && row_count > 0)
+        return 2 * ((lvx_fwd_workspace_bytes(s, (row_count + rounds - 1) / rounds, kv_splits) + 15) / 16 * 16);
     const bool f32 = kv_splits > 0 && (kv_splits & LVX_SPLITS_FP32);
     if (f32) kv_splits &= ~LVX_SPLITS_FP32;
     if (!s || kv_splits <= 1 || row_count <= 0) return 0;
@@ -226,11 +236,40 @@ int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
     return best;
 }
 
+// The fold of one block's 16-bit parts as a launch of its own.
+static int fold_parts(const lvx_attn_shape* s, const FwdFold& f, hipStream_t st) {
+    MergeParams m{};
+    m.f16 = s->dtype == LVX_F16;
+    m.D = s->D;
+    m.o_acc = f.o - (int64_t)f.row_begin * f.os.s;
+    m.l_acc = f.l;
+    m.oa = f.os;
+    m.o_part = f.part - (int64_t)f.row_begin * s->D;
+    m.l_part = f.l_part - f.row_begin;
+    m.op = Strides3{(int64_t)s->Hq * f.rows * s->D, (int64_t)f.rows * s->D, s->D};
+    m.l_part_stride = (int64_t)s->B * s->Hq * f.rows;
+    m.o_part_stride = m.l_part_stride * s->D;
+    m.l_acc_bh = s->Lq;
+    m.l_part_bh = f.rows;
+    m.nparts = f.nparts;
+    if (f.acc) {
+        m.use_acc = 1;
+        m.o_in = f.acc - (int64_t)f.row_begin * f.as.s;
+        m.l_in = f.l_acc;
+        m.oi = f.as;
+        m.l_in_bh = s->Lq;
+    }
+    m.B = s->B; m.Hq = s->Hq; m.Lq = s->Lq;
+    m.row_begin = f.row_begin; m.row_end = f.row_begin + f.rows;
+    return static_cast<int>(launch_merge(m, st));
+}
+
 // lvx_fwd, and lvx_fwd_acc when (o_in, l_in) is given: the result is then merged with that
 // incoming accumulator before it is written to (o, lse).
 static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
                     const lvx_tensor* o, float* lse, int32_t row_begin, int32_t row_count, int32_t kv_splits,
-                    void* workspace, size_t workspace_bytes, void* stream, const lvx_tensor* o_in, const float* l_in) {
+                    void* workspace, size_t workspace_bytes, void* stream, const lvx_tensor* o_in, const float* l_in,
+                    FwdFold* before = nullptr) {
     LVX_TRY(check_shape(s));
     LVX_TRY(check_tensor(q));
     LVX_TRY(check_tensor(k));
@@ -238,6 +277,18 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     LVX_TRY(check_tensor(o));
     if (!lse) return LVX_ERR_NULL;
     LVX_TRY(check_rows(s, row_begin, row_count));
+    if (const int rounds = fwd_rounds(kv_splits); rounds > 1) {
+        // one launch per block; `before` carries the parts of a block to the launch that folds them
+        const int rows = (row_count + rounds - 1) / rounds;
+        const size_t half = lvx_fwd_workspace_bytes(s, row_count, kv_splits | LVX_SPLITS_ROUNDS(rounds)) / 2;
+        if (half && (!workspace || workspace_bytes < 2 * half)) return LVX_ERR_WORKSPACE;
+        if (half && !aligned16(workspace)) return LVX_ERR_ALIGN;
+        FwdFold parts{};
+        for (int r = 0; r * rows < row_count; ++r)
+            LVX_TRY(fwd_impl(s, q, k, v, o, lse, row_begin + r * rows, std::min(rows, row_count - r * rows), kv_splits,
+                             half ? static_cast<char*>(workspace) + (r & 1) * half : nullptr, half, stream, o_in, l_in, &parts));
+        return parts.part ? fold_parts(s, parts, static_cast<hipStream_t>(stream)) : LVX_OK;
+    }
     const int f32 = kv_splits > 0 ? kv_splits & LVX_SPLITS_FP32 : 0;
     kv_splits -= f32;
     if (kv_splits < 1 || kv_splits > MAX_SPLITS) return LVX_ERR_SHAPE;
@@ -277,6 +328,12 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     p.split_len = split_len;
     p.total_wg = s->B * p.n_head_groups * nsplit * p.n_row_tiles;
 
+    const bool rides = before && form == FWD_WIDE && nsplit > 1 && !f32 && fold_chains(nsplit, (int64_t)s->B * s->Hq * row_count) <= 2;
+    if (before && before->part) {
+        if (form == FWD_WIDE) p.fold = *before;
+        else LVX_TRY(fold_parts(s, *before, st));       // this block's launch does not take them along
+        before->part = nullptr;
+    }
     if (nsplit == 1) {
         p.o = static_cast<uint16_t*>(o->ptr);
         p.os = st3(o);
@@ -322,6 +379,12 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     p.lse_split_stride = rows;
     hipError_t e = launch_fwd(p, s->kv_start != nullptr, st);
     if (e != hipSuccess) return static_cast<int>(e);
+    if (rides) {
+        *before = FwdFold{o_ws, l_ws, static_cast<uint16_t*>(o->ptr) + (int64_t)row_begin * o->stride_s, lse,
+                          o_in ? static_cast<const uint16_t*>(o_in->ptr) + (int64_t)row_begin * o_in->stride_s : nullptr, l_in,
+                          st3(o), o_in ? st3(o_in) : Strides3{}, nsplit, row_count, row_begin};
+        return LVX_OK;
+    }
 
     MergeParams m{};
     m.f16 = s->dtype == LVX_F16;

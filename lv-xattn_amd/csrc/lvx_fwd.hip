@@ -31,6 +31,7 @@
 // groups - both conflict-free.  Loads past the end of the key range are
 // clamped to its last row (those keys are masked out of S).
 #include "lvx_common.hpp"
+#include "lvx_fold.hpp"
 #include "lvx_kernels.hpp"
 
 namespace lvx {
@@ -389,6 +390,72 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
 #define LVX_FWD_WIDE_CLOBBERS_64 "v32", "v33", "v34", "v35", "v36", "v37", "v38", "v39", "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127", "v132", "v133", "v134", "v135", "v136", "v137", "v138", "v139", "v140", "v141", "v142", "v143", "v144", "v145", "v146", "v147", "v148", "v149", "v150", "v151", "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v160", "v161", "v162", "v163", "v164", "v165", "v166", "v167", "v168", "v169", "v170", "v171", "v172", "v173", "v174", "v175", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", "v187", "v188", "v189", "v190", "v191", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v204", "v205", "v206", "v207", "v212", "v213", "v214", "v215", "v218", "v219", "v222", "v223", "v233", "v234", "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175"
 #define LVX_FWD_WIDE_CLOBBERS_S "memory", "vcc", "scc", "m0", "s52", "s53", "s54", "s55", "s56", "s58", "s59", "s60", "s61", "s70", "s71"
 
+// Folds a share of what the launch before left in parts: the rows of a query block that has been computed, while this launch
+// computes the next.  A launch of its own for it takes 6 us of the 35 that a round of 256 rows x 6404 keys does; here, all
+// parts of two chunks of a row in flight per thread, 5: what is left is 21 MB on their way back from the memory side, where the end
+// of a launch leaves them.  Sixteen such rounds 585 -> 560 us.
+// Heads go slowest over the work-groups, as in the launch that wrote the parts, which are then in the L2 of this XCD.
+template <int DH, bool F16, int CHAINS>
+__device__ __forceinline__ void fold_before(const FwdParams& p, uint32_t wid) {
+    using E = Elt<F16>;
+    constexpr int SH = DH == 128 ? 4 : 3;
+    const FwdFold& f = p.fold;
+    const uint32_t n = (uint32_t)(p.B * p.Hq * f.rows) << SH, end = min((wid + 1) * f.per_wg, n);
+    const int64_t l_stride = (int64_t)p.B * p.Hq * f.rows, stride = l_stride * DH;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    for (uint32_t at = wid * f.per_wg + threadIdx.x; at < end; at += 512) {
+        uint32_t row[2], b[2], h[2];
+        const int chunk = (int)(at & ((1 << SH) - 1));
+        float l[2][CHAINS][FOLD_BATCH], la[2];
+        u32x4 u[2][CHAINS][FOLD_BATCH], ua[2];
+        RowFold sum[2][CHAINS];
+        for (int k0 = 0; k0 < f.nparts; k0 += CHAINS * FOLD_BATCH) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const uint32_t r = min(at + 256 * c, n - 1) >> SH;      // a second chunk past the share is read and dropped
+                h[c] = p.by_B.split(f.by_rows.split(r, row[c]), b[c]);
+                const int64_t bh = (int64_t)b[c] * p.Hq + h[c];
+                const uint16_t* const op = f.part + (bh * f.rows + row[c]) * DH + chunk * 8;
+                const float* const lp = f.l_part + bh * f.rows + row[c];
+#pragma unroll
+                for (int x = 0; x < CHAINS; ++x)
+#pragma unroll
+                    for (int k = 0; k < FOLD_BATCH; ++k) {
+                        const int part = k0 + x + k * CHAINS, some = min(part, f.nparts - 1);
+                        l[c][x][k] = lp[some * l_stride];
+                        u[c][x][k] = *reinterpret_cast<const u32x4*>(op + some * stride);
+                    }
+                la[c] = -INFINITY;
+                ua[c] = zero;
+                if (f.acc) {
+                    la[c] = f.l_acc[bh * p.Lq + f.row_begin + row[c]];
+                    ua[c] = *reinterpret_cast<const u32x4*>(f.acc + b[c] * f.as.b + h[c] * f.as.h + row[c] * f.as.s + chunk * 8);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int x = 0; x < CHAINS; ++x) {
+#pragma unroll
+                    for (int k = 0; k < FOLD_BATCH; ++k)
+                        if (k0 + x + k * CHAINS >= f.nparts) l[c][x][k] = -INFINITY;
+                    sum[c][x].add(l[c][x], [&](int k, float (&v)[8]) { unpack8<E>(u[c][x][k], v); });
+                }
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            if (at + 256 * c >= end) break;
+            if (f.acc) {
+                const float only[FOLD_BATCH] = {la[c], -INFINITY, -INFINITY, -INFINITY};
+                sum[c][0].add(only, [&](int k, float (&v)[8]) { unpack8<E>(k ? zero : ua[c], v); });
+            }
+            if constexpr (CHAINS == 2) sum[c][0].join(sum[c][1]);
+            *reinterpret_cast<u32x4*>(f.o + b[c] * f.os.b + h[c] * f.os.h + row[c] * f.os.s + chunk * 8) = sum[c][0].template result<E>();
+            if (chunk == 0) f.l[((int64_t)b[c] * p.Hq + h[c]) * p.Lq + f.row_begin + row[c]] = sum[c][0].lse();
+        }
+    }
+}
+
 // The wide form (head dimensions 128 and 64, both element types, any mask but a dense bias): a wave
 // owns two blocks of 32 rows of its head and has its SIMD to itself (one work-group per CU, 512
 // registers per lane), so that every K / V operand read from LDS feeds two MFMAs: half the LDS reads
@@ -410,7 +477,8 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
 //             ((r >> 2) & 3): the eight even and the eight odd rows of sixteen consecutive ones land
 //             in eight different positions each, and of the four rows of a transposing read those of
 //             like parity in different 64-byte halves
-template <int DH, bool MASKED, bool F16>
+// FOLD: the launch also folds the parts of the one before it (a test at run time costs every launch 0.2 %).
+template <int DH, bool MASKED, bool F16, bool FOLD>
 __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     using E = Elt<F16>;
     static_assert(DH == 128 || DH == 64, "head dimension");
@@ -426,6 +494,10 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     fetch_kernargs<sizeof(FwdParams)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
     if (wid >= p.total_wg) return;
+    if constexpr (FOLD) {
+        if (p.fold.chains == 2) fold_before<DH, F16, 2>(p, wid);
+        else fold_before<DH, F16, 1>(p, wid);
+    }
     uint32_t tile, split, b;
     const uint32_t t1 = p.by_row_tiles.split(wid, tile), t2 = p.by_splits.split(t1, split);
     // samples vary faster than head groups: every XCD (a contiguous range of ids) then gets
@@ -968,8 +1040,12 @@ hipError_t launch_fwd_t(const FwdParams& p, bool masked, hipStream_t st) {
     }
     if constexpr (DH >= 64) {
         if (p.form == FWD_WIDE) {
-            if (masked) return launch1((fwd_wide_kernel<DH, true, F16>), dim3(grid), dim3(256), st, p);
-            return launch1((fwd_wide_kernel<DH, false, F16>), dim3(grid), dim3(256), st, p);
+            if (p.fold.part) {
+                if (masked) return launch1((fwd_wide_kernel<DH, true, F16, true>), dim3(grid), dim3(256), st, p);
+                return launch1((fwd_wide_kernel<DH, false, F16, true>), dim3(grid), dim3(256), st, p);
+            }
+            if (masked) return launch1((fwd_wide_kernel<DH, true, F16, false>), dim3(grid), dim3(256), st, p);
+            return launch1((fwd_wide_kernel<DH, false, F16, false>), dim3(grid), dim3(256), st, p);
         }
         if (!p.bias) return hipErrorInvalidValue;      // fwd_form never asks for it
     }
@@ -992,6 +1068,13 @@ hipError_t launch_fwd(const FwdParams& params, bool masked, hipStream_t st) {
     p.by_B = divisor(p.B);
     p.by_G = divisor(p.G);
     p.by_head_groups = divisor(p.G / p.HG);
+    if (p.fold.part) {
+        const int64_t chunks = (int64_t)p.B * p.Hq * p.fold.rows * (p.D / 8);
+        p.fold.chains = fold_chains(p.fold.nparts, (int64_t)p.B * p.Hq * p.fold.rows);
+        if (p.form != FWD_WIDE || chunks > UINT32_MAX / 2 || p.fold.chains > 2) return hipErrorInvalidValue;
+        p.fold.per_wg = (uint32_t)((chunks + p.total_wg - 1) / p.total_wg + 255) / 256 * 256;
+        p.fold.by_rows = divisor(p.fold.rows);
+    }
     switch (p.D) {
         case 16: return p.f16 ? launch_fwd_t<16, true>(p, masked, st) : launch_fwd_t<16, false>(p, masked, st);
         case 32: return p.f16 ? launch_fwd_t<32, true>(p, masked, st) : launch_fwd_t<32, false>(p, masked, st);

@@ -40,6 +40,22 @@ struct Divisor {
 };
 inline Divisor divisor(int d) { return Divisor{(uint32_t)d, 0xffffffffu / (uint32_t)d}; }
 
+// The parts of one launch that the next one folds on its way (16-bit parts; wide form).  Null part: none.
+struct FwdFold {
+    const uint16_t* part;      // [nparts][B * Hq][rows][D]
+    const float* l_part;       // [nparts][B * Hq][rows]
+    uint16_t* o;               // the result, of the folded window's first row (l: absolute rows, Lq to a (b, h))
+    float* l;
+    const uint16_t* acc;       // incoming accumulator, indexed like o and l, or null
+    const float* l_acc;
+    Strides3 os, as;
+    int nparts, rows, row_begin;
+    // filled in by launch_fwd
+    int chains;                // see fold_chains; more than two do not ride along
+    uint32_t per_wg;           // 16-byte chunks that a work-group folds, a multiple of its threads
+    Divisor by_rows;
+};
+
 struct FwdParams {
     const uint16_t* q;
     const uint16_t* k;
@@ -66,6 +82,7 @@ struct FwdParams {
     float scale, scale_log2e;
     int f16;                   // element type of q, k, v, o: 0 bf16, 1 fp16
     int o_f32;                 // 1: o (the parts of a launch with key splits) is fp32
+    FwdFold fold;
     // filled in by launch_fwd: divisors by n_row_tiles, nsplit, B, G and G / HG
     Divisor by_row_tiles, by_splits, by_B, by_G, by_head_groups;
 };

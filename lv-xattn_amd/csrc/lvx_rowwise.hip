@@ -4,6 +4,7 @@
 // so a 256-thread group streams 16 rows per pass with fully coalesced 256-byte
 // row segments; with head_dim 64 / 32 / 16 it is 8 / 4 / 2 lanes and 32 / 64 / 128 rows per pass.
 #include "lvx_common.hpp"
+#include "lvx_fold.hpp"
 #include "lvx_kernels.hpp"
 
 #include <algorithm>
@@ -41,15 +42,6 @@ __device__ __forceinline__ uint32_t producer_block(uint32_t blocks_per_xcd) {
     return (blockIdx.x & 7) * blocks_per_xcd + (blockIdx.x >> 3);
 }
 
-template <class E>
-__device__ __forceinline__ void unpack8(u32x4 u, float f[8]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        f[2 * j] = E::lo(u[j]);
-        f[2 * j + 1] = E::hi(u[j]);
-    }
-}
-
 // (o_acc, l_acc) <- merge(acc?, part_0 .. part_{n-1}) for every (b, h, row).  PL lanes share the parts
 // of a 16-byte column of a row: with few rows (a token being generated, cut into dozens of key
 // ranges) the launch is as long as a thread's chain of loads, so the parts of a row go side by side
@@ -58,7 +50,7 @@ __device__ __forceinline__ void unpack8(u32x4 u, float f[8]) {
 template <bool F16, int PL, bool PART32>
 __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     using E = Elt<F16>;
-    constexpr int PSH = PL == 4 ? 2 : PL == 2 ? 1 : 0, BATCH = 4;
+    constexpr int PSH = PL == 4 ? 2 : PL == 2 ? 1 : 0, BATCH = FOLD_BATCH;
     fetch_kernargs<sizeof(MergeParams)>();
     const int nrows = p.row_end - p.row_begin;
     const int64_t idx = (int64_t)producer_block(p.blocks_per_xcd) * 256 + threadIdx.x;
@@ -71,31 +63,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     const int h = (int)p.by_B.split(p.by_rows.split((uint32_t)r, r_in), b);
     const int row = p.row_begin + (int)r_in, bh = (int)b * p.Hq + h;
 
-    float m = -INFINITY, den = 0.f, out[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) out[j] = 0.f;
-    // folds the parts (l[k], u[k]) in; a part with weight 0 may hold anything (it saw no key, or nothing
-    // had been folded into the accumulator yet), one with weight NaN makes the row NaN
-    auto fold = [&](const float (&l)[BATCH], auto&& part) {
-        float mn = m;
-#pragma unroll
-        for (int k = 0; k < BATCH; ++k) mn = fmaxf(mn, l[k]);
-        const float ms = (mn == -INFINITY) ? 0.f : mn;
-        const float keep = __expf(m - ms);
-        den *= keep;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) out[j] *= keep;
-#pragma unroll
-        for (int k = 0; k < BATCH; ++k) {
-            const float w = __expf(l[k] - ms);
-            den += w;
-            float f[8];
-            part(k, f);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) out[j] = w != 0.f ? fmaf(f[j], w, out[j]) : out[j];
-        }
-        m = mn;
-    };
+    RowFold sum;
     uint16_t* oa = p.o_acc + b * p.oa.b + h * p.oa.h + (int64_t)row * p.oa.s + chunk * 8;
     const u32x4 zero = {0u, 0u, 0u, 0u};
     float la = -INFINITY;
@@ -123,7 +91,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
                 u[k] = ldg16(op + part * p.o_part_stride, ok);
             }
         }
-        fold(l, [&](int k, float (&f)[8]) {
+        sum.add(l, [&](int k, float (&f)[8]) {
             if constexpr (PART32) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) { f[j] = __uint_as_float(u[k][j]); f[4 + j] = __uint_as_float(u2[k][j]); }
@@ -134,26 +102,21 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     }
     if (p.use_acc) {
         const float l[BATCH] = {la, -INFINITY, -INFINITY, -INFINITY};
-        fold(l, [&](int k, float (&f)[8]) { unpack8<E>(k ? zero : ua, f); });
+        sum.add(l, [&](int k, float (&f)[8]) { unpack8<E>(k ? zero : ua, f); });
     }
 #pragma unroll
     for (int o = 1; o < PL; o <<= 1) {                  // the lanes that share a row's parts
         const int d = o << sh;
-        const float m2 = __shfl_xor(m, d), den2 = __shfl_xor(den, d);
-        const float mn = fmaxf(m, m2), ms = (mn == -INFINITY) ? 0.f : mn;
-        const float w1 = __expf(m - ms), w2 = __expf(m2 - ms);
-        den = den * w1 + den2 * w2;
+        RowFold other;
+        other.m = __shfl_xor(sum.m, d);
+        other.den = __shfl_xor(sum.den, d);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) out[j] = out[j] * w1 + __shfl_xor(out[j], d) * w2;
-        m = mn;
+        for (int j = 0; j < 8; ++j) other.out[j] = __shfl_xor(sum.out[j], d);
+        sum.join(other);
     }
     if (pl != 0) return;
-    const float inv = den > 0.f ? 1.f / den : 0.f;
-    u32x4 u;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) u[j] = E::pack(out[2 * j] * inv, out[2 * j + 1] * inv);
-    *reinterpret_cast<u32x4*>(oa) = u;
-    if (chunk == 0) p.l_acc[(int64_t)bh * p.l_acc_bh + row] = den > 0.f ? m + __logf(den) : -INFINITY;
+    *reinterpret_cast<u32x4*>(oa) = sum.result<E>();
+    if (chunk == 0) p.l_acc[(int64_t)bh * p.l_acc_bh + row] = sum.lse();
 }
 
 // The same for one part folded into the accumulator (what lvx_merge does every round), two rows
@@ -708,8 +671,7 @@ hipError_t launch_merge(const MergeParams& params, hipStream_t st) {
         if (p.f16) return launch1(merge_pair_kernel<true>, grid, dim3(256), st, p);
         return launch1(merge_pair_kernel<false>, grid, dim3(256), st, p);
     }
-    // as many lanes per row as the parts need (four parts each) and the chip has room for
-    const int pl = p.nparts > 8 && rows < 16384 ? 4 : p.nparts > 4 && rows < 32768 ? 2 : 1;
+    const int pl = fold_chains(p.nparts, rows);
     p.by_B = divisor(p.B);
     p.blocks_per_xcd = per_xcd((rows * pl << chunk_shift(p.D)));
     const dim3 grid(8 * p.blocks_per_xcd);

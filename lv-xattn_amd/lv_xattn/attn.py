@@ -22,7 +22,7 @@ import torch
 
 from . import ops
 from .async_communication import backward_workspace_cap, get_sequence_parallel_size, workspace
-from ._lib import LVX_BF16, AttnShape, host, load
+from ._lib import LVX_BF16, LVX_ERR_SHAPE, LVX_SPLITS_ROUNDS, AttnShape, check, host, load
 from .ops import Mask
 
 __all__ = ["_attn_forward", "_attn_backward", "q_block_bounds", "Mask"]
@@ -191,6 +191,10 @@ def _attn_forward(q, k, v, causal, sm_scale, comm_mode, bias_func=None,
     # the parts of the key splits live for this call only (from torch's caching allocator, as o and L); rounds
     # on several streams have a buffer per stream
     overlap = streams > 1 and len(windows) > 1
+    if kv_splits >> LVX_SPLITS_ROUNDS > 0:
+        check(LVX_ERR_SHAPE, "lvx_fwd")
+    if not overlap and 1 < len(windows) < 1 << 18:      # all rounds in one call, which folds a round's parts in the launch of the next
+        kv_splits, windows, max_rows = kv_splits | len(windows) << LVX_SPLITS_ROUNDS, [(0, Lq)], Lq
     o, L, ws = host().forward_buffers(q_, max_rows, 1 if overlap else kv_splits, _token_major)
 
     # the partial goes straight into (o, L), merged on its way with the incoming accumulator
