@@ -223,10 +223,13 @@ int lvx_bwd_preprocess(const lvx_attn_shape* shape, const lvx_tensor* o, const l
  *   dk, dv : at Hkv heads (the group sum is taken in registers);
  *            dkv_accumulate == 0: 16-bit tensors, overwritten;
  *            dkv_accumulate == 1: fp32 tensors of the same indexing, added to;
+ *            dkv_accumulate == 1 | LVX_BWD_ROUNDS(n): the same for n windows of ceil(row_count / n) rows, one after the other, with
+ *            the results of n calls and the workspace of the first;
  *   workspace : lvx_bwd_workspace_bytes(shape, row_count) bytes, 16-byte
  *            aligned; holds scale*dS (16-bit) between the kernels of the call, the row
  *            metadata and, for small windows, fp32 partial sums of dK/dV and partial tiles of dQ.
  */
+#define LVX_BWD_ROUNDS(n) ((int32_t)(n) << 12)       /* n up to 2^18 */
 int lvx_bwd(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tensor* k,
             const lvx_tensor* v, const lvx_tensor* dout, const float* lse, const float* delta,
             const lvx_tensor* dq, const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate,

@@ -176,7 +176,7 @@ bool bwd_preprocess(const Tensor& o, const Tensor& dout, const Tensor& delta, in
 
 bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
          const Tensor& dk, const Tensor& dv, double scale, int64_t row_begin, int64_t row_count, const OptTensor& kv_len,
-         const OptTensor& kv_start, const OptTensor& kv_end, bool accumulate_dkv, const Tensor& ws, const OptTensor& bias) {
+         const OptTensor& kv_start, const OptTensor& kv_end, int64_t accumulate_dkv, const Tensor& ws, const OptTensor& bias) {
     lvx_attn_shape s;
     if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end) || !fill_bias(s, bias, q)) return false;
     const at::ScalarType kv_type = accumulate_dkv ? at::kFloat : q.scalar_type();
@@ -189,7 +189,7 @@ bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, 
     void *const wp = ws.data_ptr(), *const st = current_stream();
     const size_t wb = ws.nbytes();
     call("lvx_bwd", [&] {
-        return lib.bwd(&s, &tq, &tk, &tv, &td, lp, dp, &tdq, &tdk, &tdv, accumulate_dkv ? 1 : 0, (int32_t)row_begin, (int32_t)row_count,
+        return lib.bwd(&s, &tq, &tk, &tv, &td, lp, dp, &tdq, &tdk, &tdv, (int32_t)accumulate_dkv, (int32_t)row_begin, (int32_t)row_count,
                        wp, wb, st);
     });
     return true;

@@ -225,6 +225,10 @@ struct MetaParams {
     const float* delta;
     float* out;
     int B, Hq, Lq, row_begin, row_end, n_tiles;
+    // one launch for `rounds` windows of round_rows rows each (n_tiles: of one of them; the last may have fewer), whose
+    // records are round_out floats apart
+    int rounds, round_rows;
+    int64_t round_out;
     float scale;
     float* scratch;            // null, or the fp32 dK / dV scratch whose shared token blocks the same launch zeroes
     SharedBlocks sb;

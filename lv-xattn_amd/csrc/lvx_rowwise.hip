@@ -261,11 +261,13 @@ __global__ __launch_bounds__(256) void bwd_meta_kernel(const MetaParams p) {
     if (idx >= (int64_t)p.B * p.Hq * rows_pad) return;
     uint32_t r;
     const int64_t bh = p.by_rows.split((uint32_t)idx, r);
-    const int row = p.row_begin + r;
-    const bool ok = row < p.row_end;
+    const int begin = p.row_begin + (int)blockIdx.y * p.round_rows, end = min(begin + p.round_rows, p.row_end);
+    const int row = begin + r, n_tiles = (end - begin + 31) / 32;
+    if ((int)(r >> 5) >= n_tiles) return;               // a shorter last window
+    const bool ok = row < end;
     const float l = ok ? p.lse[bh * p.Lq + row] : -INFINITY;
     const float d = ok ? p.delta[bh * p.Lq + row] : 0.f;
-    float* o = p.out + (bh * p.n_tiles + (r >> 5)) * 64 + (r & 31);
+    float* o = p.out + blockIdx.y * p.round_out + (bh * n_tiles + (r >> 5)) * 64 + (r & 31);
     o[0] = (l == -INFINITY) ? INFINITY : l * 1.4426950408889634f;
     o[32] = d * p.scale;
 }
@@ -703,7 +705,7 @@ hipError_t launch_bwd_meta(const MetaParams& p0, hipStream_t st) {
     if (n == 0 && zero_blocks == 0) return hipSuccess;
     p.meta_blocks = (int)((n + 255) / 256);
     p.by_rows = divisor(std::max(1, p.n_tiles * 32));
-    return launch1(bwd_meta_kernel, dim3((unsigned)(p.meta_blocks + zero_blocks)), dim3(256), st, p);
+    return launch1(bwd_meta_kernel, dim3((unsigned)(p.meta_blocks + zero_blocks), p.rounds), dim3(256), st, p);
 }
 
 hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st) {

@@ -17,6 +17,7 @@ LIB_PATH = os.environ.get("LVX_LIB") or os.path.join(_HERE, "liblvx.so")
 VERSION = 104           # of the library (include/lvx.h) this package is written against
 LVX_BF16 = 1
 LVX_SPLITS_ROUNDS = 12      # in kv_splits, the bit where the number of rounds begins (include/lvx.h)
+LVX_BWD_ROUNDS = 12         # likewise in dkv_accumulate
 LVX_F16 = 2
 LVX_ERR_SHAPE = -3
 

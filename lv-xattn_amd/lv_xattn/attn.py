@@ -300,8 +300,9 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
     delta = workspace("bwd_delta", (B * Hq, Lq), torch.float32, dev)
     dq, dk, dv = host().backward_outputs(q_, k_, _dq_like_q)
 
-    windows = [(0, Lq)] if batched else [w for w in q_block_bounds(Lq, P) if w[1] > w[0]]
-    windows = _cap_windows(windows, lambda rows: ops.bwd_workspace_bytes(q_, k_, rows, mask), backward_workspace_cap())
+    blocks = [(0, Lq)] if batched else [w for w in q_block_bounds(Lq, P) if w[1] > w[0]]
+    windows = _cap_windows(blocks, lambda rows: ops.bwd_workspace_bytes(q_, k_, rows, mask), backward_workspace_cap())
+    one_call = len(windows) == len(blocks) < 1 << 18            # the windows are the query blocks
     ws = workspace("bwd_ds", (ops.bwd_workspace_bytes(q_, k_, max(r1 - r0 for r0, r1 in windows), mask),),
                    torch.uint8, dev)
     if len(windows) == 1:
@@ -319,9 +320,9 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
         # all rows ahead of the rounds (a visit of a real ring would bring its own block's)
         ops.bwd_preprocess(o_, do_, delta, 0, Lq)
 
-        def one_round(r0, r1, acc, ws_r):
+        def one_round(r0, r1, acc, ws_r, rounds=1):
             ops.bwd(q_, k_, v_, do_, L_, delta, dq, acc[0].transpose(1, 2), acc[1].transpose(1, 2), sm_scale,
-                    r0, r1 - r0, mask, accumulate_dkv=True, workspace=ws_r, bias=bias)
+                    r0, r1 - r0, mask, accumulate_dkv=True, workspace=ws_r, bias=bias, rounds=rounds)
 
         acc = accumulators()
         n_streams = min(streams, len(windows))
@@ -338,6 +339,8 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
                         one_round(r0, r1, accs[i % n_streams], ws_i)
             for other in accs[1:]:
                 acc += other
+        elif one_call:
+            one_round(0, Lq, acc, ws, len(blocks))
         else:
             for r0, r1 in windows:
                 one_round(r0, r1, acc, ws)

@@ -222,16 +222,18 @@ def bwd_workspace_bytes(q, k, row_count: int, mask: Optional[Mask] = None) -> in
 
 def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=None,
         mask: Optional[Mask] = None, accumulate_dkv: bool = False,
-        workspace: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None) -> None:
+        workspace: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None, rounds: int = 1) -> None:
     """Writes dq (bf16) for the selected rows and writes (bf16) or accumulates
     (fp32) dk, dv at Hkv heads.  `workspace`: uint8 tensor of at least
     bwd_workspace_bytes(q, k, row_count, mask) bytes.  `bias` as in fwd (no gradient
-    is formed for it)."""
+    is formed for it).  `rounds` > 1 (with accumulate_dkv): the rows are that many windows, one after the other, in the
+    workspace of one of ceil(row_count / rounds) rows."""
+    flags = (1 if accumulate_dkv else 0) | (rounds << _lib.LVX_BWD_ROUNDS if rounds > 1 else 0)
     if workspace is not None:
         m = mask or _NO_MASK
         if host().bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin,
                       q.shape[2] - row_begin if row_count is None else row_count, m.kv_len, m.kv_start, m.kv_end,
-                      accumulate_dkv, workspace, bias):
+                      flags, workspace, bias):
             return
     s = _shape(q, k, scale, mask, bias)
     if row_count is None:
@@ -244,10 +246,10 @@ def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=Non
     if dk.dtype != want or dv.dtype != want or dk.shape != k.shape or dv.shape != k.shape:
         raise LvxError(f"dk/dv must be {want} tensors shaped like k")
     if workspace is None:
-        workspace = torch.empty(bwd_workspace_bytes(q, k, row_count, mask), dtype=torch.uint8, device=q.device)
+        workspace = torch.empty(bwd_workspace_bytes(q, k, -(-row_count // rounds), mask), dtype=torch.uint8, device=q.device)
     rc = load().lvx_bwd(C.byref(s), C.byref(t4(q)), C.byref(t4(k)), C.byref(t4(v)), C.byref(t4(dout)),
                         lse.data_ptr(), delta.data_ptr(), C.byref(t4(dq)), C.byref(t4(dk)), C.byref(t4(dv)),
-                        1 if accumulate_dkv else 0, row_begin, row_count,
+                        flags, row_begin, row_count,
                         workspace.data_ptr(), workspace.numel() * workspace.element_size(), stream_ptr())
     check(rc, "lvx_bwd")
 
