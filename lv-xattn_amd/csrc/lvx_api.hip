@@ -712,12 +712,18 @@ size_t lvx_bwd_workspace_bytes(const lvx_attn_shape* s, int32_t row_count) {
     return bwd_workspace(s, row_count).total;
 }
 
+// The slices of a window's dQ that wait for the next launch to sum them.
+struct WaitingDq {
+    bool any;
+    CastParams slices;
+};
+
 // One window, its arguments checked, in the workspace of one of ws_rows rows, at least as many.  meta: null, or the records of
-// its rows.
+// its rows.  before: null, or what the window before has left and this one may leave.
 static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
                       const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
                       const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate, int32_t row_begin, int32_t row_count,
-                      void* workspace, int32_t ws_rows, hipStream_t st, const float* meta);
+                      void* workspace, int32_t ws_rows, hipStream_t st, const float* meta, WaitingDq* before);
 
 int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
             const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
@@ -745,7 +751,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     if (!workspace || workspace_bytes < lvx_bwd_workspace_bytes(s, round_rows)) return LVX_ERR_WORKSPACE;
     if (!aligned16(workspace)) return LVX_ERR_ALIGN;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (rounds <= 1) return bwd_window(s, q, k, v, dout, lse, delta, dq, dk, dv, dkv_accumulate, row_begin, row_count, workspace, row_count, st, nullptr);
+    if (rounds <= 1) return bwd_window(s, q, k, v, dout, lse, delta, dq, dk, dv, dkv_accumulate, row_begin, row_count, workspace, row_count, st, nullptr, nullptr);
 
     // Several windows: the records of all their rows by one launch instead of one of 3 - 5 us each (32 heads x 16 rounds of 256 rows,
     // forward and backward 2775 -> 2741 us), where the scratch that only sums of 16-bit dk, dv use holds them.
@@ -759,16 +765,17 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
         const hipError_t e = launch_bwd_meta(mp, st);
         if (e != hipSuccess) return static_cast<int>(e);
     }
+    WaitingDq waiting{};
     for (int r = 0; r < n; ++r)
         LVX_TRY(bwd_window(s, q, k, v, dout, lse, delta, dq, dk, dv, 1, row_begin + r * round_rows, std::min(round_rows, row_count - r * round_rows),
-                           workspace, round_rows, st, meta ? meta + r * each : nullptr));
-    return LVX_OK;
+                           workspace, round_rows, st, meta ? meta + r * each : nullptr, &waiting));
+    return waiting.any ? static_cast<int>(launch_cast(waiting.slices, st)) : LVX_OK;
 }
 
 static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
                       const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
                       const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate, int32_t row_begin, int32_t row_count,
-                      void* workspace, int32_t ws_rows, hipStream_t st, const float* meta) {
+                      void* workspace, int32_t ws_rows, hipStream_t st, const float* meta, WaitingDq* before) {
     BwdParams p{};
     p.f16 = s->dtype == LVX_F16;
     p.D = s->D;
@@ -855,8 +862,10 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
         p.dv = scratch + dkv_elems;
         p.dks = p.dvs = Strides3{(int64_t)s->Lkv * s->Hkv * s->D, (int64_t)s->D, (int64_t)s->Hkv * s->D};
     }
-    hipError_t e = launch_bwd(p, s->kv_start != nullptr, st);
+    // (the slices lie where this window's own come, which only the launch after this one writes)
+    hipError_t e = launch_bwd(p, s->kv_start != nullptr, st, before && before->any ? &before->slices : nullptr);
     if (e != hipSuccess) return static_cast<int>(e);
+    if (before) before->any = false;
     if (scratch) {
         CastSharedParams cp{sb, scratch, static_cast<uint16_t*>(dk->ptr), static_cast<uint16_t*>(dv->ptr), st3(dk), st3(dv), p.f16};
         e = launch_cast_shared(cp, st);
@@ -891,6 +900,10 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     cq.B = s->B; cq.H = s->Hq; cq.L = row_count;
     cq.transposed = 1;
     cq.nsum = dq_by.splits; cq.sum_stride = g.part_split;
+    if (before) {
+        *before = WaitingDq{true, cq};
+        return LVX_OK;
+    }
     return static_cast<int>(launch_cast(cq, st));
 }
 

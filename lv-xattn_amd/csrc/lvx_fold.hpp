@@ -3,6 +3,7 @@
 // order and the same groups, so that a row's bits do not depend on which of them folded it.
 #pragma once
 #include "lvx_common.hpp"
+#include "lvx_kernels.hpp"
 
 namespace lvx {
 
@@ -58,6 +59,38 @@ struct RowFold {
     }
     __device__ __forceinline__ float lse() const { return den > 0.f ? m + __logf(den) : -INFINITY; }
 };
+
+// log2 of the 16-byte chunks (lanes) per row
+__host__ __device__ __forceinline__ int chunk_shift(int head_dim) {
+    return head_dim == 64 ? 3 : head_dim == 32 ? 2 : head_dim == 16 ? 1 : 4;
+}
+
+// Rounds eight values of a row of the fp32 source [B*H][D][L], or of the sum of several such: thread `idx` of the launch.  Adjacent
+// threads take adjacent rows, so the eight strided reads of a thread are coalesced across the wave.
+template <bool F16>
+__device__ __forceinline__ void cast_t(const CastParams& p, int64_t idx) {
+    using E = Elt<F16>;
+    const int sh = chunk_shift(p.D);
+    const int Dh = 8 << sh;
+    if (idx >= ((int64_t)p.B * p.H * p.L << sh)) return;
+    uint32_t row, b;       // plan_cast_t checks that a thread's number fits 32 bits
+    const uint32_t col = p.by_L.split((uint32_t)idx, row);      // a chunk of an (h, b)
+    const int chunk = (int)(col & ((1u << sh) - 1));
+    const int h = (int)p.by_B.split(col >> sh, b), bh = (int)b * p.H + h;
+    const float* s = p.src + ((int64_t)bh * Dh + chunk * 8) * p.L + row;
+    float a[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a[j] = s[(int64_t)j * p.L];
+    for (int k = 1; k < p.nsum; ++k) {
+        s += p.sum_stride;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] += s[(int64_t)j * p.L];
+    }
+    u32x4 u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) u[j] = E::pack(a[2 * j], a[2 * j + 1]);
+    *reinterpret_cast<u32x4*>(p.dst + b * p.ds.b + h * p.ds.h + (int64_t)row * p.ds.s + chunk * 8) = u;
+}
 
 template <class E>
 __device__ __forceinline__ void unpack8(u32x4 u, float f[8]) {

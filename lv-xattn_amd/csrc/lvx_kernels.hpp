@@ -148,6 +148,20 @@ struct PreParams {
     Divisor by_rows, by_Hq;    // filled in by launch_preprocess
 };
 
+struct CastParams {
+    const float* src;
+    uint16_t* dst;
+    Strides3 ds;
+    int B, H, L;
+    int transposed;   // 0: src is [B*H][L][D]; 1: src is [B*H][D][L]
+    int nsum;         // transposed only: the result is the sum of nsum such sources (0 or 1: one),
+    int64_t sum_stride;   // sum_stride floats apart
+    int f16;          // destination type: 0 bf16, 1 fp16
+    int D;            // head dimension: 16, 32, 64 or 128 (0 reads as 128)
+    Divisor by_L, by_H, by_B;       // filled in by launch_cast
+    uint32_t blocks_per_xcd;        // and a share of the grid
+};
+
 struct BwdParams {
     const uint16_t* q;
     const uint16_t* k;
@@ -188,6 +202,9 @@ struct BwdParams {
     const int32_t* live_runs;
     int f16;                   // element type of q, k, v, dout, the dS^T workspace and (mode 0) dk, dv
     Divisor by_splits, by_splits2, by_kv_blocks, by_B;     // filled in by launch_bwd
+    // and the work-groups that are the token blocks' (a multiple of 8): any past them sum the slices of dQ of the window before
+    int own_wg;
+    CastParams dq_before;
 };
 
 // Which (token block, 32-row tile) pairs an interval mask leaves alive: a tile is alive for the blocks of its hull, the
@@ -244,20 +261,6 @@ struct CastSharedParams {
     uint16_t* dv;
     Strides3 dks, dvs;
     int f16;
-};
-
-struct CastParams {
-    const float* src;
-    uint16_t* dst;
-    Strides3 ds;
-    int B, H, L;
-    int transposed;   // 0: src is [B*H][L][D]; 1: src is [B*H][D][L]
-    int nsum;         // transposed only: the result is the sum of nsum such sources (0 or 1: one),
-    int64_t sum_stride;   // sum_stride floats apart
-    int f16;          // destination type: 0 bf16, 1 fp16
-    int D;            // head dimension: 16, 32, 64 or 128 (0 reads as 128)
-    Divisor by_L, by_H, by_B;       // filled in by launch_cast
-    uint32_t blocks_per_xcd;        // and a share of the grid
 };
 
 constexpr int DQ_FEW_TILES = 2;    // row tiles a work-group of dq_few_kernel takes
@@ -326,7 +329,8 @@ struct GemmParams {
 hipError_t launch_fwd(const FwdParams& p, bool masked, hipStream_t st);   // p.bias selects the bias variant
 hipError_t launch_merge(const MergeParams& p, hipStream_t st);
 hipError_t launch_preprocess(const PreParams& p, hipStream_t st);
-hipError_t launch_bwd(const BwdParams& p, bool masked, hipStream_t st);
+hipError_t launch_bwd(const BwdParams& p, bool masked, hipStream_t st, const CastParams* dq_before = nullptr);
+hipError_t plan_cast_t(CastParams& p, int threads);
 hipError_t launch_cast(const CastParams& p, hipStream_t st);
 hipError_t launch_cast_shared(const CastSharedParams& p, hipStream_t st);
 hipError_t launch_bwd_meta(const MetaParams& p, hipStream_t st);

@@ -15,11 +15,6 @@ namespace lvx {
 
 namespace {
 
-// log2 of the 16-byte chunks (lanes) per row
-__host__ __device__ __forceinline__ int chunk_shift(int head_dim) {
-    return head_dim == 64 ? 3 : head_dim == 32 ? 2 : head_dim == 16 ? 1 : 4;
-}
-
 // Where the r-th of the rows of all (b, h) is.  Rows are counted in 32 bits: 2^32 of them, 32 bytes each at the least, are
 // not in the card's memory twice.
 struct RowOf {
@@ -554,33 +549,11 @@ __global__ __launch_bounds__(256) void cast_shared_kernel(const CastSharedParams
     }
 }
 
-// Same from a transposed source [B*H][D][L], or the sum of several: adjacent threads take
-// adjacent rows, so the eight strided reads of a thread are coalesced across the wave.
+// Same from a transposed source (cast_t).
 template <bool F16>
 __global__ __launch_bounds__(256) void cast_t_kernel(const CastParams p) {
-    using E = Elt<F16>;
     fetch_kernargs<sizeof(CastParams)>();
-    const int64_t idx = (int64_t)producer_block(p.blocks_per_xcd) * 256 + threadIdx.x;
-    const int sh = chunk_shift(p.D);
-    const int Dh = 8 << sh;
-    if (idx >= ((int64_t)p.B * p.H * p.L << sh)) return;
-    uint32_t row, b;       // launch_cast checks that a thread's number fits 32 bits
-    const uint32_t col = p.by_L.split((uint32_t)idx, row);      // a chunk of an (h, b)
-    const int chunk = (int)(col & ((1u << sh) - 1));
-    const int h = (int)p.by_B.split(col >> sh, b), bh = (int)b * p.H + h;
-    const float* s = p.src + ((int64_t)bh * Dh + chunk * 8) * p.L + row;
-    float a[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) a[j] = s[(int64_t)j * p.L];
-    for (int k = 1; k < p.nsum; ++k) {
-        s += p.sum_stride;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) a[j] += s[(int64_t)j * p.L];
-    }
-    u32x4 u;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) u[j] = E::pack(a[2 * j], a[2 * j + 1]);
-    *reinterpret_cast<u32x4*>(p.dst + b * p.ds.b + h * p.ds.h + (int64_t)row * p.ds.s + chunk * 8) = u;
+    cast_t<F16>(p, (int64_t)producer_block(p.blocks_per_xcd) * 256 + threadIdx.x);
 }
 
 // Backward of y = w * bf16(x * r) over 128-wide rows: with xh = x * r and gg = dy * w,
@@ -763,17 +736,26 @@ hipError_t launch_cast_shared(const CastSharedParams& p, hipStream_t st) {
     return launch1(cast_shared_kernel<false>, grid, dim3(256), st, p);
 }
 
+// For cast_t by work-groups of so many threads.
+hipError_t plan_cast_t(CastParams& p, int threads) {
+    const int64_t rows = (int64_t)p.B * p.H * p.L;
+    if (rows * 16 > UINT32_MAX) return hipErrorInvalidValue;    // 256 rows of dQ at most per CU
+    p.by_L = divisor(p.L);
+    p.by_B = divisor(p.B);
+    p.blocks_per_xcd = (uint32_t)((((rows << chunk_shift(p.D)) + threads - 1) / threads + 7) / 8);
+    return hipSuccess;
+}
+
 hipError_t launch_cast(const CastParams& params, hipStream_t st) {
     CastParams p = params;
     const int64_t rows = (int64_t)p.B * p.H * p.L;
     if (rows == 0) return hipSuccess;
-    if (p.transposed && rows * 16 > UINT32_MAX) return hipErrorInvalidValue;    // 256 rows of dQ at most per CU
     p.by_L = divisor(p.L);
     p.by_H = divisor(p.H);
     const dim3 grid(blocks_for(rows));
     if (p.transposed) {
-        p.by_B = divisor(p.B);
-        p.blocks_per_xcd = per_xcd(rows << chunk_shift(p.D));
+        const hipError_t e = plan_cast_t(p, 256);
+        if (e != hipSuccess) return e;
         const dim3 grid(8 * p.blocks_per_xcd);
         if (p.f16) return launch1(cast_t_kernel<true>, grid, dim3(256), st, p);
         else return launch1(cast_t_kernel<false>, grid, dim3(256), st, p);

@@ -1,6 +1,7 @@
 """Rounds computed in one call.  Forward: a round's parts are folded by the launch of the next one, the last round's by a launch of
 their own - bit for bit what a call per round gives, which folds every round itself - at the edges of the rounds, with and without an
-accumulator, masks, both chains of the fold, and where nothing rides along.  Backward: the rows' records of all rounds at once."""
+accumulator, masks, both chains of the fold, and where nothing rides along.  Backward: the rows' records of all rounds are written at once, and the
+slices of a round's dQ are summed by the launch of the next."""
 import pytest
 import torch
 
