@@ -4,7 +4,7 @@
     python gen_bwd_loop.py d bf16 128 > lvx_bwd_loop_d_bf16_128.inc               (D-waves: dP, dS, dK^T)
 
 for bf16 and f16, head dimensions 128 and 64, and P-waves without ("plain") and with ("masked") key
-intervals per row.  Each is one inline-asm statement with every register named here.  One trip does six steps (the
+intervals per row, the latter also with a dense bias ("bias").  Each is one inline-asm statement with every register named here.  One trip does six steps (the
 six tile buffers of each ring and the two-deep P / dS^T buffers then sit at immediate offsets);
 the first step of a trip is a step i with i % 6 == 3.  Inside a step the 16 MFMAs of a wave (8 with heads of 64) are
 spread over its other instructions (LDS operand reads eight operands ahead, the exponentials or
@@ -20,6 +20,13 @@ replaced by ones whose rows are clamped to the window's last (RAGGED, out of lin
 next head.  Masked: a step asks with one compare per lane whether any
 row of the tile cuts the wave's 32 tokens and only then goes through the out-of-line block that zeroes
 the hidden elements of P.
+
+Bias: 32 rows x the wave's 32 tokens of fp32, 4 KiB in an LDS tile of its own that no other wave touches.  In the second
+half of step i the bias of tile i is read from there into the registers that the bias of tile i-1 had, and
+behind those reads the four loads of tile i+1's are requested, a whole step before they are waited for.  A lane's
+loads would be 16 of 4 bytes per tile (two rows of 32 tokens each), four times as many as the tile's own.  An LDS row of 128
+bytes is 32 tokens of row 8 n + 4 (s & 1) + (s >> 1) for slot s of the n-th load: the lane's 16 rows are 256 bytes
+apart, and the two halves of a wave in different banks.
 
 Registers, both roles: v[0:63] resident accumulators (dV^T / dK^T)   v[64:95] resident B operands
 (K rows / V rows)   v[96:111], v[112:127] the two score sets (raw S / dP), swapping every step
@@ -41,6 +48,10 @@ P-waves: v[168:175] P packed   v[176:191] LSE*log2(e) of 16 rows   v[192:199] dS
   s[80:81] what a head change adds to the metadata address   s82 1 if the last tile of a head has clamped
   rows, else -1   s83 / s84 bytes per Q / dO row   masked: s85 bytes of metadata per tile   s86 first token of the wave, s87 one
   past its last   s[90:91] all ones if not all of them exist   s92 1 if dS^T leaves as streaming stores
+  bias: v[234:249] the bias of 16 rows   v233 its read address   v250 the lane's row in the first of a tile's four loads
+  v251 bytes of its chunk in a row   s39 LDS address of the tile   s93 bytes per row   s94 per 32 rows   s95 log2(e)
+  s[96:97] address of the next tile to request (its first row, token 0)   s98 tiles left in its head   s99 last row of a
+  head's last tile   s[100:101] what a head change adds
 D-waves: v[168:175] P handed over   v[176:183] dS packed   v[184:199] delta*scale of 16 rows
   v216 P hand-over read address   v217 metadata read address   v218, v223..v225 dS^T staging write addresses, one per
   group of four rows
@@ -57,7 +68,8 @@ for _o in list(OPTS):      # a switch for one role only: p_novalu, d_nolds, ...
         OPTS[_o[2:]] = OPTS[_o]
 F16 = len(sys.argv) > 2 and sys.argv[2] == "f16"
 DH = int(sys.argv[3]) if len(sys.argv) > 3 else 128
-MASKED = len(sys.argv) > 4 and sys.argv[4] == "masked"
+BIAS = len(sys.argv) > 4 and sys.argv[4] == "bias"
+MASKED = BIAS or len(sys.argv) > 4 and sys.argv[4] == "masked"
 MFMA = "v_mfma_f32_32x32x16_f16" if F16 else "v_mfma_f32_32x32x16_bf16"
 CVT = "v_cvt_pk_f16_f32" if F16 else "v_cvt_pk_bf16_f32"
 NKK, NDT = DH // 16, DH // 32           # k-steps of S / dP, 32-wide blocks of dV^T / dK^T
@@ -71,6 +83,7 @@ PU, LSE, CPD = 168, 176, 192
 A_PB, A_META, A_CP, G_CP, G_DMA, G_META = 216, 217, (218, 219), 220, 221, 225
 EXCESS, A_IV, IV, TOKEN = 226, 228, 229, 231
 IV_EXCESS = 232
+BV, A_BV, BROW, BCHUNK = 234, 233, 250, 251
 # D role
 DSU, DELTA, TMP, A_DS = 176, 184, 219, (218, 223, 224, 225)
 
@@ -132,8 +145,11 @@ class Stream:
         next step waits at its top until only these are in flight: LDS operations complete in order, so
         the writes other waves are about to read have then landed) and, among them, the reads of the
         first operands of the next step."""
-        n = self.n_lds - self.last_write
-        tag = {t: pos - self.last_write for t, pos in self.tag.items()     # <= 0: read before the write
+        done = self.last_write
+        if BIAS:        # more reads than can be counted, but their last ones were waited for behind the writes
+            done = max(done, self.done)
+        n = self.n_lds - done
+        tag = {t: pos - done for t, pos in self.tag.items()     # <= 0: read before the write
                if isinstance(t, tuple) and t[0] == "op" and t[1] == u_next}
         assert len(tag) == AHEAD and n <= 15, (n, tag)
         return {"n": n, "tag": tag}
@@ -231,6 +247,19 @@ def p_mask(u):
     return out + [f"s_branch LVX_BWD_SEEN{u}_%="]
 
 
+def p_bias(u):
+    """Request of tile i+1's bias in step u, rows clamped to the window's last, and the walk to the tile after it."""
+    f = [["s_cmp_eq_u32 s98, 1", "s_cselect_b32 s88, s99, 31"]]
+    for n in range(4):
+        t = IV + n % 2
+        f += [f"v_add_u32 v{t}, {8 * n}, v{BROW}", f"v_min_u32 v{t}, s88, v{t}",
+              [f"s_add_i32 m0, s39, {1024 * n}", f"v_mad_u32_u24 v{t}, v{t}, s93, v{BCHUNK}", f"global_load_lds_dwordx4 v{t}, s[96:97]"]]
+    f += [["s_add_u32 s96, s96, s94", "s_addc_u32 s97, s97, 0", "s_sub_i32 s98, s98, 1", "s_cmp_lg_u32 s98, 0",
+           f"s_cbranch_scc1 LVX_BWD_SAMEBIAS{u}_%=", "s_add_u32 s96, s96, s100", "s_addc_u32 s97, s97, s101", "s_mov_b32 s98, s53",
+           f"LVX_BWD_SAMEBIAS{u}_%=:"]]
+    return f
+
+
 def flat(items):
     out = []
     for x in items:
@@ -246,7 +275,8 @@ def p_step(u, seed):
     par = u & 1                                                  # (i + 1) & 1: P(i-1) hand-over, dS^T(i-3)
     carry, new = SET[u & 1], SET[(u + 1) & 1]
     # tile i+1 has landed: after its loads this wave issued 2 stores, 4 (wave 0: 5) loads and 2 stores
-    e("s_waitcnt vmcnt(8)")
+    # (with a bias four loads of that more)
+    e(f"s_waitcnt vmcnt({12 if BIAS else 8})")
     e(f"s_waitcnt lgkmcnt({st.n_lds})")
     e("s_barrier")
     for vg in range(4):
@@ -259,9 +289,12 @@ def p_step(u, seed):
     valu = []
     for vg in range(4):
         valu.append(lambda vg=vg: st.wait(("lse", vg)))
+        for r in range(4 if BIAS else 0):
+            v = 4 * vg + r
+            valu.append(f"v_fma_f32 v{LSE + v}, v{BV + v}, s95, -v{LSE + v}")
         for r in range(4):
             v = 4 * vg + r
-            valu.append(f"v_fma_f32 v{carry + v}, v{carry + v}, s40, -v{LSE + v}")
+            valu.append(f"v_fma_f32 v{carry + v}, v{carry + v}, s40, {'' if BIAS else '-'}v{LSE + v}")
         for r in range(4):
             valu.append(f"v_exp_f32 v{carry + 4 * vg + r}, v{carry + 4 * vg + r}")
         if vg >= 1 and not MASKED:
@@ -283,6 +316,10 @@ def p_step(u, seed):
     # second half: request of tile i+3 and the walk, dS^T(i-3) copy-out.  The loads go first: the wait
     # at the top of a step then leaves the two stores of the step before last in flight as well
     tail = []
+    if BIAS:    # behind the loads of tile i's bias the wave issued 4 (wave 0: 5) tile loads and 2 stores
+        tail.append("s_waitcnt vmcnt(6)")
+        for n in range(0, 16, 2):
+            tail.append(lambda n=n: st.lds(f"ds_read2st64_b32 {vr(BV + n, 2)}, v{A_BV} offset0:{n} offset1:{n + 1}", "bias"))
     for n in range(4):
         tail.append(lambda n=n: st.lds(f"ds_read_b64_tr_b16 {vr(CPD + 2 * n, 2)}, v{A_CP[n % 2]} offset:{par * DST_SZ + 1024 * (n // 2)}", f"cp{n}"))
     ws_old = 66 + 2 * (u % 6)          # workspace address of tile i-3 (tile i+3 takes its place below)
@@ -290,6 +327,8 @@ def p_step(u, seed):
     if u == 5:      # the last step of the last trip requests nothing: the steps after the loop do
         fetch = [["s_cmp_eq_u32 s64, 1", "s_cbranch_scc1 LVX_BWD_NOFETCH_%="] + flat(fetch) + ["LVX_BWD_NOFETCH_%=:"]]
     # the stores read the workspace address of tile i-3 before the walk overwrites it: keep a copy
+    if BIAS:
+        tail += [lambda: st.wait("bias")] + p_bias(u)
     tail += [f"s_mov_b64 s[78:79], {sr(ws_old, 2)}"] + fetch + [lambda: st.wait("cp3")]
     tail.append(["s_cmp_eq_u32 s92, 0", f"s_cbranch_scc1 LVX_BWD_KEEP{u}_%=", *p_store(" nt"), f"LVX_BWD_STORED{u}_%=:"])
 

@@ -66,9 +66,13 @@ constexpr int OFF_Q = 0;                       // x NQD
 constexpr int OFF_DO = OFF_Q + NQD * TILE_ELEMS; // x NQD
 constexpr int OFF_DST = OFF_DO + NQD * TILE_ELEMS; // x2
 constexpr int OFF_PB = OFF_DST + 2 * DST_ELEMS;  // x2
-constexpr int LOOP_ELEMS = OFF_PB + 2 * PB_ELEMS;
+constexpr int OFF_BIAS = OFF_PB + 2 * PB_ELEMS;  // masked with a dense bias: four tiles of 32 rows x 32 tokens fp32, one per P-wave
+constexpr int BIAS_ELEMS = 4 * 32 * 32 * 2;
 constexpr int EPI_ELEMS = 8 * 32 * (D + 4) * 2;     // 8 waves x [32 tokens][128 + 4] floats of the epilogue, in uint16 units
-constexpr int SMEM_ELEMS = LOOP_ELEMS > EPI_ELEMS ? LOOP_ELEMS : EPI_ELEMS;
+constexpr int smem_elems(bool bias) {
+    const int loop = OFF_BIAS + (bias ? BIAS_ELEMS : 0);
+    return loop > EPI_ELEMS ? loop : EPI_ELEMS;
+}
 
 constexpr uint32_t META_B = 768;   // bytes of a tile's metadata
 constexpr float LOG2E = 1.4426950408889634f;
@@ -85,11 +89,12 @@ constexpr float LOG2E = 1.4426950408889634f;
     "{v204}"(ra[4]), "{v205}"(ra[5]), "{v206}"(ra[6]), "{v207}"(ra[7]),                                              \
     "{v208}"(ta[0]), "{v209}"(ta[1]), "{v210}"(ta[2]), "{v211}"(ta[3]),                                              \
     "{v212}"(ta[4]), "{v213}"(ta[5]), "{v214}"(ta[6]), "{v215}"(ta[7]), "{v216}"(a_pb), "{v217}"(a_meta)
-#define LVX_BWD_P_OPERANDS                                                                                           \
-    : LVX_BWD_COMMON_OUT, "+{s[44:45]}"(qp), "+{s[46:47]}"(dop), "+{s[48:49]}"(mp), "+{s[50:51]}"(wn), "+{s52}"(left), \
+#define LVX_BWD_P_OUT                                                                                                \
+    LVX_BWD_COMMON_OUT, "+{s[44:45]}"(qp), "+{s[46:47]}"(dop), "+{s[48:49]}"(mp), "+{s[50:51]}"(wn), "+{s52}"(left), \
       "+{s[66:67]}"(w0), "+{s[68:69]}"(w1), "+{s[70:71]}"(w2), "+{s[72:73]}"(w3), "+{s[74:75]}"(w4), "+{s[76:77]}"(w5), \
-      "+{v221}"(g_t[0]), "+{v222}"(g_t[1]), "+{v223}"(g_t[2]), "+{v224}"(g_t[3]), "+{v225}"(g_meta)                   \
-    : LVX_BWD_COMMON_IN, "{v218}"(a_cp0), "{v219}"(a_cp1), "{v220}"(g_cp), "{v232}"(past_iv),                        \
+      "+{v221}"(g_t[0]), "+{v222}"(g_t[1]), "+{v223}"(g_t[2]), "+{v224}"(g_t[3]), "+{v225}"(g_meta)
+#define LVX_BWD_P_IN                                                                                                 \
+    LVX_BWD_COMMON_IN, "{v218}"(a_cp0), "{v219}"(a_cp1), "{v220}"(g_cp), "{v232}"(past_iv),                        \
       "{v226}"(past0), "{v227}"(past1), "{v228}"(a_iv), "{v231}"(token), "{s83}"(uniform32(qrow_b)), "{s84}"(uniform32(dorow_b)), \
       "{s40}"(uniform32(c)), "{s41}"(uniform32((uint32_t)BM * qrow_b)), "{s42}"(uniform32((uint32_t)BM * dorow_b)),  \
       "{s53}"(uniform32(n_live)), "{s[54:55]}"(hdq), "{s[56:57]}"(hddo), "{s[60:61]}"(hdws), "{s[80:81]}"(hdm),      \
@@ -97,8 +102,15 @@ constexpr float LOG2E = 1.4426950408889634f;
       "{s65}"(uniform32(wave < META_WAVES ? 1 : 0)), "{s82}"(uniform32(ragged ? 1 : -1)),                            \
       "{s85}"(uniform32(meta_w ? BM * 4 : 256)), "{s86}"(uniform32(slice_lo)), "{s87}"(uniform32(slice_lo + 32)),     \
       "{s92}"(uniform32(p.ds_stream)),                                                                               \
-      "{s[90:91]}"(uniform64(slice_valid ? (int64_t)0 : (int64_t)-1))                                                \
-    : "memory", "vcc", "scc", "m0", "s78", "s79", "s88", "s89", "v229", "v230", LVX_BWD_LOOP_CLOBBERS
+      "{s[90:91]}"(uniform64(slice_valid ? (int64_t)0 : (int64_t)-1))
+#define LVX_BWD_P_CLOBBERS "memory", "vcc", "scc", "m0", "s78", "s79", "s88", "s89", "v229", "v230", LVX_BWD_LOOP_CLOBBERS
+#define LVX_BWD_P_OPERANDS : LVX_BWD_P_OUT : LVX_BWD_P_IN : LVX_BWD_P_CLOBBERS
+#define LVX_BWD_P_BIAS_OPERANDS                                                                                      \
+    : LVX_BWD_P_OUT, "+{v[234:249]}"(bv), "+{s[96:97]}"(bp), "+{s98}"(b_left)                                     \
+    : LVX_BWD_P_IN, "{v233}"(a_bias), "{v250}"(b_row), "{v251}"(b_chunk), "{s39}"(uniform32(lds_bias)),               \
+      "{s93}"(uniform32(brow_b)), "{s94}"(uniform32((uint32_t)BM * brow_b)), "{s95}"(uniform32(LOG2E)),               \
+      "{s99}"(uniform32(ragged ? last : BM - 1)), "{s[100:101]}"(hdb)                                                \
+    : LVX_BWD_P_CLOBBERS
 #define LVX_BWD_D_OPERANDS                                                                                           \
     : LVX_BWD_COMMON_OUT : LVX_BWD_COMMON_IN, "{v218}"(a_ds[0]), "{v223}"(a_ds[1]), "{v224}"(a_ds[2]), "{v225}"(a_ds[3]), "{s40}"(uniform32(p.scale))                            \
     : "memory", "vcc", "scc", LVX_BWD_LOOP_CLOBBERS, "v219", "v220", "v221", "v222"
@@ -115,6 +127,7 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     static_assert(DH == 16 || DH == 32 || DH == 64 || DH == 128, "head dimension");
     constexpr int NKK = DH / 16, NDT = DH >= 32 ? DH / 32 : 1;
     constexpr int META_WAVES = MASKED ? 3 : 1;      // waves that fetch a part of a tile's metadata
+    constexpr int SMEM_ELEMS = smem_elems(MASKED && BIAS && DH >= 64);
     __shared__ __attribute__((aligned(1024))) uint16_t smem[SMEM_ELEMS];
     // per-row metadata of a staged tile, one per tile buffer: 8 x 16 bytes each of LSE*log2e and
     // delta*scale; with an interval mask kv_start and kv_end follow, each twice (a load moves 64 lanes)
@@ -342,16 +355,9 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     // Flags say which halves exist at the edges of the walk; they are compile-time
     // constants in the steady-state loop.
     auto p_step = [&](auto tail_c, bool s_live, bool pv_live, const uint16_t* tile_cur, const uint16_t* tile_prev,
-                      const u32x4* meta, uint16_t* pbuf, f32x16& s_carry, int64_t bias_off, int bias_r0)
+                      const u32x4* meta, uint16_t* pbuf, f32x16& s_carry, f32x16& bv, int64_t bias_off, int bias_r0)
                       __attribute__((always_inline)) {
         constexpr bool TAIL = decltype(tail_c)::value;
-        float bv[16];
-        if (BIAS && pv_live) {   // bias of (row 8 vg + 4 g + r of the previous tile, this lane's token)
-            const float* bp = p.bias + bias_off + min(my_kv, p.Lkv - 1);
-            const int last = p.row_end - 1 - bias_r0;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) bv[v] = bp[(int64_t)min(8 * (v >> 2) + 4 * g + (v & 3), last) * p.bias_r];
-        }
         const char* qt = reinterpret_cast<const char*>(tile_cur);     // Q of tile i
         const char* dot = reinterpret_cast<const char*>(tile_prev);   // dO of tile i-1
         bf16x8 qa[8];
@@ -397,6 +403,7 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                     s[4 * vg + r] = __builtin_amdgcn_exp2f(fmaf(s[4 * vg + r], c, off));
                 }
             }
+            if (BIAS) __builtin_amdgcn_sched_barrier(0);
             if (MASKED) {
                 // most (tile, token slice) pairs a mask leaves alive are alive as a whole; only a
                 // slice that some row of the tile cuts is masked element by element
@@ -431,6 +438,12 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                     const u32x4 a = {da[dt][j][0][0], da[dt][j][0][1], da[dt][j][1][0], da[dt][j][1][1]};
                     acc[dt] = E::mfma(as_bf16x8(a), as_bf16x8(pu[j]), acc[dt]);
                 }
+        }
+        if (BIAS && s_live) {   // for the next step: bias of (row 8 vg + 4 g + r of this tile, the lane's token)
+            const float* bp = p.bias + bias_off + min(my_kv, p.Lkv - 1);
+            const int last = p.row_end - 1 - bias_r0;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) bv[v] = bp[(int64_t)min(8 * (v >> 2) + 4 * g + (v & 3), last) * p.bias_r];
         }
         if (s_live) s_carry = s_new;
     };
@@ -534,6 +547,7 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         f32x16 carry;     // P-wave: raw S of the previous tile; D-wave: dP of the previous tile
 #pragma unroll
         for (int v = 0; v < 16; ++v) carry[v] = 0.f;
+        f32x16 bv = carry;      // BIAS, P-wave: of the previous tile, on its way since the step before
         int rc = 0;       // i % 6
 
         auto step = [&](int i, bool s_live, bool pv_live, bool ds_live, bool copy) __attribute__((always_inline)) {
@@ -550,11 +564,13 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                 else wait_vmcnt<4>();
             }
             lds_barrier();
+            // the bias has come before the next tile is requested, or its wait would be for that as well
+            if (BIAS && !DROLE) asm volatile("" : "+v"(bv));
             // tile i+2 replaces tile i-4, whose last readers finished long before this barrier
             if (i + 2 < n_iter) fetch(m6(rc + 2));
             const int r1 = m6(rc + 5), r2 = m6(rc + 4);     // (i - 1) % 6, (i - 2) % 6
             if (!DROLE)
-                p_step(tail_c, s_live, pv_live, qt(rc), dot(r1), meta_s4[r1], pbf((i + 1) & 1), carry, b_q[2], r_q[2]);
+                p_step(tail_c, s_live, pv_live, qt(rc), dot(r1), meta_s4[r1], pbf((i + 1) & 1), carry, bv, b_q[3], r_q[3]);
             else
                 d_step(pv_live, ds_live, dot(r1), qt(r2), meta_s4[r2], pbf(i & 1), dst(i & 1), carry);
             // dS^T(i-3) to HBM last: its LDS read queues behind this step's operand reads
@@ -573,14 +589,17 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         // Steady state: steps 3 .. 3 + 6 trips - 1 (every one of them with all its parts alive and a tile to
         // request) run in the hand-scheduled loops of gen_bwd_loop.py, six steps a trip; the steps after
         // them continue below as if they had run here.  Left to the code above: heads of 32 and 16, a dense
-        // bias, the last token block where there is no mask, and token blocks whose live tiles are not one run.
+        // bias without intervals per row (the host always has some: what the bias leaves visible), the last token block
+        // where there is no mask, and token blocks whose live tiles are not one run.
         // The code above leaves the matrix pipe to the compiler's order and, masked, keeps its walk in spilled
         // scalar registers.  Forward and backward of an attention, us, that code against the loops: 2 x 3000 rows,
         // images of 3202 tokens 1423 -> 1199; 2 x 1023 rows x 6404 tokens 2039 -> 1999 (whole layer);
-        // heads of 64, 2048 x 6404 708 -> 697.
-        if constexpr ((DH == 128 || DH == 64) && !BIAS && !decltype(tail_c)::value) {
+        // heads of 64, 2048 x 6404 708 -> 697.  With a dense bias (fp16, 16 heads, 1024 x 4096; bwd_kernel) 120 -> 109, and 106
+        // since the steps left above have their bias on its way a step ahead of its use, too.
+        if constexpr ((DH == 128 || DH == 64) && (MASKED || !BIAS) && !decltype(tail_c)::value) {
             int trips = uniform32((n_iter - 5) / 6);
-            if (i == 3 && trips >= 1 && run_n[1] == 0) {
+            // a row of the bias in bytes is a factor of 24 bits there
+            if (i == 3 && trips >= 1 && run_n[1] == 0 && (!BIAS || p.bias_r < (1 << 22))) {
                 const int steps = 6 * trips;
                 uint32_t ra[8], ta[8];      // with heads of 64 half of each stays unused
 #pragma unroll
@@ -628,8 +647,44 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                     uint32_t g_meta = (meta_w ? (uint32_t)l32 : (uint32_t)lane) * 4u - (now ? past_iv : 0u);
                     const uint32_t a_iv = meta0 + 256u + (uint32_t)l32 * 4u;
                     const int token = kv_valid ? my_kv : 0x7fffffff;
+                    // bias: of tile i - 1 in registers, of tile i on its way to LDS, of tile i + 1 the first the loop requests
+                    const uint32_t brow_b = (uint32_t)p.bias_r * 4u;
+                    const uint32_t lds_bias = lds0 + OFF_BIAS * 2 + (uint32_t)slice * 4096u;
+                    const uint32_t b_row = 4u * ((lane >> 3) & 1) + (lane >> 4);
+                    // 16 bytes of a row, the last of the row for lanes past it
+                    const uint32_t b_chunk = (uint32_t)min(slice_lo + 4 * (lane & 7), (p.Lkv - 1) & ~3) * 4u;
+                    const uint32_t a_bias = lds_bias + (uint32_t)g * 128u + (uint32_t)l32 * 4u;
+                    const char* bp = nullptr;
+                    int b_left = 0;
+                    int64_t hdb = 0;
+                    if constexpr (BIAS) {
+                        const char* b0 = uniform_ptr(reinterpret_cast<const char*>(p.bias + b_q[3]));
+#pragma unroll
+                        for (int n = 0; n < 4; ++n)
+                            dma16<RESTORED>(b0, (uint32_t)min((int)b_row + 8 * n, p.row_end - 1 - r_q[3]) * brow_b + b_chunk,
+                                            lds_bias + 1024u * n);
+                        bp = uniform_ptr(reinterpret_cast<const char*>(p.bias + b_q[4]));
+                        b_left = uniform32(n_live - (it_lo + i + 1) % n_live);
+                        hdb = uniform64((int64_t)p.bias_h * 4 - (int64_t)n_live * BM * brow_b);
+                    }
                     wait_vmcnt<4>();    // tile 3 (the loads of tile 4 may be in flight); the loop counts from there
-                    if constexpr (!F16 && DH == 128 && !MASKED) {
+                    if constexpr (BIAS && !F16 && DH == 128) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_bf16_128_bias.inc"
+                            LVX_BWD_P_BIAS_OPERANDS);
+                    } else if constexpr (BIAS && !F16) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_bf16_64_bias.inc"
+                            LVX_BWD_P_BIAS_OPERANDS);
+                    } else if constexpr (BIAS && DH == 128) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_f16_128_bias.inc"
+                            LVX_BWD_P_BIAS_OPERANDS);
+                    } else if constexpr (BIAS) {
+                        asm volatile(
+#include "lvx_bwd_loop_p_f16_64_bias.inc"
+                            LVX_BWD_P_BIAS_OPERANDS);
+                    } else if constexpr (!F16 && DH == 128 && !MASKED) {
                         asm volatile(
 #include "lvx_bwd_loop_p_bf16_128_plain.inc"
                             LVX_BWD_P_OPERANDS);
@@ -692,6 +747,14 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
                     }
                 }
                 i += steps;
+                if (BIAS) {     // tiles i-1 .. i+1
+#pragma unroll
+                    for (int k = 2; k < 5; ++k) {
+                        const int pos = it_lo + i - 3 + k;
+                        r_q[k] = p.row_begin + (run_s[0] + pos % n_live) * BM;
+                        b_q[k] = b * p.bias_b + (hk * p.G + pos / n_live) * p.bias_h + (int64_t)r_q[k] * p.bias_r;
+                    }
+                }
                 // the walk stands at the tile after the last one requested
                 const int pos = it_lo + i + 2;
                 cur_gi = pos / n_live;

@@ -56,3 +56,37 @@ def test_backward_loops(D, dtype, Hq, Hkv, Lq, Lkv, mask_kind):
     torch.cuda.synchronize()
     for name, a, b in zip(("dQ", "dK", "dV"), got, ref):
         check_grad(a, b, name)
+
+
+# a dense bias joins the loop with intervals per row; the bias of a row is read in chunks of four tokens
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lkv,nb,nh,hidden", [
+    (1, 1, 352, 128, 1, 1, "none"), (11, 1, 1, 131, 2, 11, "none"), (4, 2, 257, 202, 1, 4, "none"),
+    (4, 1, 97, 300, 2, 1, "none"), (2, 2, 1000, 517, 1, 2, "cuts"), (8, 1, 300, 385, 2, 8, "cuts"),
+    (4, 1, 353, 260, 1, 1, "late"), (3, 1, 545, 33, 2, 1, "holes")])
+def test_backward_loops_with_a_dense_bias(D, dtype, Hq, Hkv, Lq, Lkv, nb, nh, hidden):
+    import lv_xattn
+    from lv_xattn import _lib
+    _lib.load()
+    B, scale = 2, D ** -0.5
+    g = torch.Generator().manual_seed(Lq * 1000 + Lkv)
+    q, do = (torch.randn(B, Lq, Hq, D, generator=g).to(dtype).transpose(1, 2) for _ in range(2))
+    k, v = (torch.randn(B, Lkv, Hkv, D, generator=g).to(dtype).transpose(1, 2) for _ in range(2))
+    bias = torch.randn(nb, nh, Lq, Lkv, generator=g)
+    row, key = torch.arange(Lq)[:, None], torch.arange(Lkv)
+    if hidden == "cuts":                # another interval in every row
+        bias.masked_fill_((key < row * 7 % (Lkv // 2)) | (key >= Lkv // 2 + row * 5 % (Lkv // 2)), float("-inf"))
+    elif hidden == "late":              # only rows from the middle on see anything
+        bias.masked_fill_((row < Lq // 2) | (key >= Lkv - 3), float("-inf"))
+    elif hidden == "holes":             # hidden keys between visible ones, which an interval does not tell
+        bias.masked_fill_((row + key) % 3 == 1, float("-inf"))
+    o, lse = orc.attention_dense(q, k, v, scale, bias=bias)
+    ref = orc.attention_backward(do, q, k, v, o.to(dtype), lse, scale, bias=bias)
+    qd, kd, vd, dod = (t.transpose(1, 2).contiguous().to(DEV).transpose(1, 2) for t in (q, k, v, do))
+    args = (lambda t: t, [bias.to(DEV)], [])
+    _, _, _, od, ld = lv_xattn._attn_forward(qd, kd, vd, False, scale, None, *args, rounds=1, batched=True)
+    got = lv_xattn._attn_backward(dod, qd, kd, vd, od, ld, False, scale, None, "flash", *args, rounds=1, batched=True)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dQ", "dK", "dV"), got, ref):
+        check_grad(a, b, name)
