@@ -824,30 +824,34 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     float* const dq32 = dq_by.splits > 1 ? reinterpret_cast<float*>(wsb + wsl.dq32) : nullptr;
     // the token blocks several work-groups share, and the fp32 scratch of the call that sums them
     SharedBlocks sb{s->B, s->Hkv, s->Lkv, s->D, p.n_kv_blocks, p.n_blocks, p.blocks_per_xcd, p.whole_blocks};
-    if (!meta) {
-        float* const out = reinterpret_cast<float*>(wsb + wsl.meta);
-        MetaParams mp{lse, delta, out, s->B, s->Hq, s->Lq, row_begin, row_begin + row_count, n_tiles, 1, row_count, 0, s->scale};
-        mp.scratch = scratch;
-        mp.sb = sb;
-        hipError_t em = launch_bwd_meta(mp, st);
-        if (em != hipSuccess) return static_cast<int>(em);
-        meta = out;
-    }
-    p.meta = meta;
     int32_t* hull = nullptr;
     int32_t* order = nullptr;
+    LiveParams lp{};
     if (s->kv_start) {
         // interval mask: token blocks skip the row tiles that see none of their tokens
         hull = reinterpret_cast<int32_t*>(wsb + wsl.hull);
         // the ranking is quadratic in the number of groups; where there are that many, the dQ
         // GEMM's work-groups even out in index order
         if (!dq_by.few && dq_by.splits <= 1 && s->B * n_groups <= MAX_RANKED_GROUPS) order = reinterpret_cast<int32_t*>(wsb + wsl.order);
-        LiveParams lp{s->kv_len, s->kv_start, s->kv_end, hull, reinterpret_cast<int32_t*>(wsb + wsl.runs), order,
-                      s->B, s->Lq, s->Lkv, row_begin,
-                      row_begin + row_count, n_tiles, n_groups, p.n_kv_blocks};
-        hipError_t el = launch_bwd_live(lp, st);
-        if (el != hipSuccess) return static_cast<int>(el);
+        lp = LiveParams{s->kv_len, s->kv_start, s->kv_end, hull, reinterpret_cast<int32_t*>(wsb + wsl.runs), order,
+                        s->B, s->Lq, s->Lkv, row_begin,
+                        row_begin + row_count, n_tiles, n_groups, p.n_kv_blocks};
         p.live_runs = lp.live_runs;
+    }
+    const bool has_hulls = !meta;       // its records come by a launch of its own, which forms the hulls as well
+    if (!meta) {
+        float* const out = reinterpret_cast<float*>(wsb + wsl.meta);
+        MetaParams mp{lse, delta, out, s->B, s->Hq, s->Lq, row_begin, row_begin + row_count, n_tiles, 1, row_count, 0, s->scale};
+        mp.scratch = scratch;
+        mp.sb = sb;
+        hipError_t em = launch_bwd_meta(mp, st, hull ? &lp : nullptr);
+        if (em != hipSuccess) return static_cast<int>(em);
+        meta = out;
+    }
+    p.meta = meta;
+    if (hull) {
+        hipError_t el = launch_bwd_live(lp, st, has_hulls);
+        if (el != hipSuccess) return static_cast<int>(el);
     }
 
     const int64_t dkv_elems = (int64_t)s->B * s->Lkv * s->Hkv * s->D;

@@ -226,7 +226,8 @@ struct LiveParams {
                                // longest hull first (ties in index order)
     int B, Lq, Lkv, row_begin, row_end, n_tiles, n_groups, n_kv_blocks;
 };
-hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st);
+// has_hulls: tile_hull is written already
+hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st, bool has_hulls);
 
 // The token blocks of a backward launch that several work-groups share, hence whose dK / dV are summed in the
 // fp32 scratch [2][B, Lkv, Hkv, D].  They are listed (b, kv head, block) with the block fastest, the
@@ -250,7 +251,9 @@ struct MetaParams {
     float* scratch;            // null, or the fp32 dK / dV scratch whose shared token blocks the same launch zeroes
     SharedBlocks sb;
     int meta_blocks;           // filled by the launcher: blocks [0, meta_blocks) write records
+    int zero_end;              // blocks [meta_blocks, zero_end) zero the scratch, those past them form the hulls of `live`
     Divisor by_rows;           // and the divisor by the rows of the window's whole tiles
+    LiveParams live;
 };
 
 // The shared token blocks of the scratch, rounded into dK and dV.
@@ -333,7 +336,8 @@ hipError_t launch_bwd(const BwdParams& p, bool masked, hipStream_t st, const Cas
 hipError_t plan_cast_t(CastParams& p, int threads);
 hipError_t launch_cast(const CastParams& p, hipStream_t st);
 hipError_t launch_cast_shared(const CastSharedParams& p, hipStream_t st);
-hipError_t launch_bwd_meta(const MetaParams& p, hipStream_t st);
+// live: null, or what has its tile hulls formed by the same launch (of one window)
+hipError_t launch_bwd_meta(const MetaParams& p, hipStream_t st, const LiveParams* live = nullptr);
 
 // Backward of the 128-wide RMS norm: rows of dy, x [M][heads][128] (row strides ldy, ldx), r [M][heads].
 struct NormBwdParams {
