@@ -147,14 +147,6 @@ __device__ __forceinline__ void dma16_stream(const char* sbase, uint32_t voff, u
 __device__ __forceinline__ void dma16_addr(const char* addr, uint32_t lds_byte) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_byte), "v"(addr) : "memory", "m0");
 }
-// the same from `bytes` bytes at sbase: a lane whose offset is past them gets zeros and reads nothing
-template <bool STREAM>
-__device__ __forceinline__ void dma16_range(const char* sbase, uint32_t bytes, uint32_t voff, uint32_t lds_byte) {
-    const uint64_t a = (uint64_t)(uintptr_t)sbase;
-    const u32x4 d = {(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, 0x00020000u};
-    if (STREAM) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(lds_byte), "v"(voff), "s"(d) : "memory", "m0");
-    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_byte), "v"(voff), "s"(d) : "memory", "m0");
-}
 // the same with 4 bytes per lane: lane i lands at lds_byte + 4 i
 template <bool RESTORED = false>
 __device__ __forceinline__ void dma4(const char* sbase, uint32_t voff, uint32_t lds_byte) {

@@ -30,6 +30,8 @@
 // the 4 rows a transposing read of V touches land in 4 different 64-byte
 // groups - both conflict-free.  Loads past the end of the key range are
 // clamped to its last row (those keys are masked out of S).
+#include <cstddef>
+
 #include "lvx_common.hpp"
 #include "lvx_fold.hpp"
 #include "lvx_kernels.hpp"
@@ -68,7 +70,7 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
     __shared__ __attribute__((aligned(1024))) char kv_lds[2][2][TILE_BYTES];   // [buffer][K, V]
     __shared__ int red[4][4];
 
-    fetch_kernargs<sizeof(FwdParams)>();
+    fetch_kernargs<offsetof(FwdParams, fold)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
     if (wid >= p.total_wg) return;
     uint32_t tile, split, b;
@@ -491,7 +493,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
     __shared__ __attribute__((aligned(1024))) char kv_lds[4 * EPB]; // 4 TB: [buffer][K, V]; then O
     __shared__ int red[4][4];
 
-    fetch_kernargs<sizeof(FwdParams)>();
+    fetch_kernargs<FOLD ? sizeof(FwdParams) : offsetof(FwdParams, fold)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
     if (wid >= p.total_wg) return;
     if constexpr (FOLD) {
@@ -786,7 +788,7 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[RING > FOLD ? RING : FOLD];
     __shared__ float ml[4][2][32];                                  // per wave and column: reference maximum, row sum
 
-    fetch_kernargs<sizeof(FwdParams)>();
+    fetch_kernargs<offsetof(FwdParams, fold)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
     if (wid >= p.total_wg) return;
     uint32_t ct, split, b;                         // column tile, key range, sample

@@ -82,9 +82,9 @@ struct FwdParams {
     float scale, scale_log2e;
     int f16;                   // element type of q, k, v, o: 0 bf16, 1 fp16
     int o_f32;                 // 1: o (the parts of a launch with key splits) is fp32
-    FwdFold fold;
     // filled in by launch_fwd: divisors by n_row_tiles, nsplit, B, G and G / HG
     Divisor by_row_tiles, by_splits, by_B, by_G, by_head_groups;
+    FwdFold fold;              // last: only launches that fold the parts of the one before fetch it
 };
 
 struct MergeParams {
