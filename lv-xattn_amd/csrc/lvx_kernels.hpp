@@ -208,7 +208,7 @@ struct BwdParams {
 };
 
 // Which (token block, 32-row tile) pairs an interval mask leaves alive: a tile is alive for the blocks of its hull, the
-// smallest range of whole token blocks that holds every key some row of the tile sees.  The dQ GEMM takes its M tiles,
+// smallest range of whole token blocks that holds every key some row of the tile sees.  The dQ kernel takes its row tiles,
 // groups of LIVE_GROUP row tiles, over the hull of the group, and reads a tile's dS^T inside the tile's own hull only.
 // (With whole groups alive or not, 2 x 3000 rows that see the image before them visited 13 % more pairs, since images
 // begin inside groups: bwd_kernel 689 us, 599 now, forward and backward 1144 -> 1067; the two table kernels 2.5 us each, or
