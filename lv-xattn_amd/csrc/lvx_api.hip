@@ -284,9 +284,13 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
         if (half && (!workspace || workspace_bytes < 2 * half)) return LVX_ERR_WORKSPACE;
         if (half && !aligned16(workspace)) return LVX_ERR_ALIGN;
         FwdFold parts{};
-        for (int r = 0; r * rows < row_count; ++r)
-            LVX_TRY(fwd_impl(s, q, k, v, o, lse, row_begin + r * rows, std::min(rows, row_count - r * rows), kv_splits,
-                             half ? static_cast<char*>(workspace) + (r & 1) * half : nullptr, half, stream, o_in, l_in, &parts));
+        char* ws = half ? static_cast<char*>(workspace) : nullptr;
+        for (int r = 0; r * rows < row_count; ++r) {
+            // the other half only while parts wait in the one before: blocks that fold at once keep theirs in the caches
+            if (parts.part) ws = ws == workspace ? ws + half : static_cast<char*>(workspace);
+            LVX_TRY(fwd_impl(s, q, k, v, o, lse, row_begin + r * rows, std::min(rows, row_count - r * rows), kv_splits, ws, half,
+                             stream, o_in, l_in, &parts));
+        }
         return parts.part ? fold_parts(s, parts, static_cast<hipStream_t>(stream)) : LVX_OK;
     }
     const int f32 = kv_splits > 0 ? kv_splits & LVX_SPLITS_FP32 : 0;
