@@ -101,6 +101,8 @@ int lvx_max_rounds(void);
  * (at most 64 ranges; lvx_fwd_auto_splits says how many suit a launch).  The O of a range waits for the
  * fold in 16 bits, a rounding that a launch of one range does not have (its error against exact arithmetic
  * grows by about a fifth), or with kv_splits = n | LVX_SPLITS_FP32 in fp32, in twice the workspace.
+ * The window's rows of o are written to while the call runs, before their result is: a launch for very few rows counts in them which
+ * of its work-groups is the last, and folds the parts itself.
  * With LVX_SPLITS_ROUNDS(n) added to kv_splits the rows are computed as n query blocks that visit one after the other: a launch
  * for each, of ceil(row_count / n) rows.  The results are those of n calls, bit for bit; where that is estimated to be faster
  * a block's 16-bit parts are folded by the launch of the next block, and the workspace holds the parts of two blocks (else of

@@ -307,6 +307,21 @@ static int fold_parts(const lvx_attn_shape* s, const FwdFold& f, hipStream_t st)
     return static_cast<int>(launch_merge(m, st));
 }
 
+// Whether the memory that o spans has any of q, k and v in it, which a launch that folds its own parts may not yet have read when o is first
+// written to.
+static bool overlap(const lvx_attn_shape* s, const lvx_tensor* o, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v) {
+    const auto end = [&](const lvx_tensor* t, int heads, int rows, int sign) {      // the last element, or before the first (strides may be negative)
+        int64_t at = 0;
+        const int64_t steps[3] = {(s->B - 1) * t->stride_b, (heads - 1) * t->stride_h, (rows - 1) * t->stride_s};
+        for (const int64_t x : steps) at += sign * x > 0 ? x : 0;
+        return static_cast<const uint16_t*>(t->ptr) + at + (sign > 0 ? s->D : 0);
+    };
+    const auto meets = [&](const lvx_tensor* t, int heads, int rows) {
+        return end(o, s->Hq, s->Lq, -1) < end(t, heads, rows, 1) && end(t, heads, rows, -1) < end(o, s->Hq, s->Lq, 1);
+    };
+    return meets(q, s->Hq, s->Lq) || meets(k, s->Hkv, s->Lkv) || meets(v, s->Hkv, s->Lkv);
+}
+
 // lvx_fwd, and lvx_fwd_acc when (o_in, l_in) is given: the result is then merged with that
 // incoming accumulator before it is written to (o, lse).
 static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
@@ -416,6 +431,15 @@ static int fwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     uint16_t* o_ws = static_cast<uint16_t*>(workspace);
     const int words = f32 ? 2 : 1;       // of 16 bits per element of a part
     float* l_ws = reinterpret_cast<float*>(o_ws + (int64_t)nsplit * rows * s->D * words);
+    if (form == FWD_FEW && f32 && !o_in && fold_inside(nsplit, (int64_t)row_count * p.G) && !overlap(s, o, q, k, v)) {
+        p.o = static_cast<uint16_t*>(o->ptr);
+        p.os = st3(o);
+        p.lse = lse;
+        p.lse_bh_stride = s->Lq;
+        p.part = reinterpret_cast<float*>(o_ws);
+        p.l_part = l_ws;
+        return static_cast<int>(launch_fwd(p, s->kv_start != nullptr, st));
+    }
     // the kernel indexes partials by absolute row: bias the bases by -row_begin
     p.o = o_ws - (int64_t)row_begin * s->D * words;
     p.o_f32 = f32 != 0;

@@ -200,6 +200,21 @@ __device__ __forceinline__ float sum16(float x) {
     return x;
 }
 
+// Over the whole wave, in every lane: halves of a quad, quads, eights as above, then rows of 16 and halves of the wave exchanged.
+template <typename Op>
+__device__ __forceinline__ float wave_reduce(float x, Op op) {
+    x = op(x, lanes_moved<0xb1>(x));
+    x = op(x, lanes_moved<0x4e>(x));
+    x = op(x, lanes_moved<0x141>(x));
+    x = op(x, lanes_moved<0x140>(x));
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float wave_max(float x) { return wave_reduce(x, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ float wave_sum(float x) { return wave_reduce(x, [](float a, float b) { return a + b; }); }
+
 // Brings every 64-byte line of the kernel's arguments (BYTES of them, at most 512) into the scalar cache with one wait.  The
 // compiler loads an argument where it is needed, and a kernel that comes by five lines one after the other stands
 // still five times for the way to memory, 0.3 us each, before its first load of data leaves.

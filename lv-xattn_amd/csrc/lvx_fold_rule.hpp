@@ -31,4 +31,12 @@ inline bool fold_rides(int nparts, int64_t rows, int row_chunks, int64_t wgs, in
     return nparts > 1 && fold_chains(nparts, rows) <= 2 && wgs <= n_cu && (passes <= 1 || (passes == 2 && 4 * wgs > 3 * n_cu));
 }
 
+// Whether the launch of the form for few rows folds its own parts, of `cols` (row, head) columns per kv head.  The last work-group then has
+// the fold to itself: a column a wave, and 1.0 us more for every further column of a wave, where a launch of its own spreads them
+// over the chip.  us a pass, its own launch -> inside:
+//   4 columns  8 kv heads x 6404 keys in 29 parts 12.2 -> 11.4, 4 x 8 x 1601 in 8 11.2 -> 10.6, heads of 64 6404 in 51 11.0 -> 9.3
+//   8          8 x 6404 in 29 12.3 -> 13.4, 4 x 8 x 1601 in 8 11.2 -> 11.6, heads of 64 1601 in 26 9.0 -> 8.1, 6404 in 34 10.8 -> 11.8
+//   16         8 x 6404 in 29 12.7 -> 17.3
+inline bool fold_inside(int nparts, int64_t cols) { return nparts > 1 && cols <= 4; }
+
 }  // namespace lvx

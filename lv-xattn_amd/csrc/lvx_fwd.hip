@@ -761,6 +761,112 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const std::conditional
     }
 }
 
+// A launch of the form below whose parts are folded by the work-group that finishes last among those of the same columns (up to four, a
+// wave to each; see fold_inside).
+//
+// They count themselves in at the place of the columns' first four values of O, which nothing else uses before the result
+// is written over it: FEW_COUNT above a count of eight bits.  Whatever that memory held, a work-group that does not find FEW_COUNT
+// there at its start replaces what it found (and fails to where another has done so), long before anyone counts, so that
+// nothing has to be cleared before a launch or kept between two, and a replayed graph counts as the first launch did.
+// FEW_COUNT reads as three NaN of bits that no result has.
+// Parts and counts go past the L2, of which every XCD has one: stores and loads of agent scope, each step's done (vmcnt) before
+// the next begins.
+// A launch of its own for the fold takes 4.5 us on the GPU and 3 of the host's time.  In here it is three ways to the memory side one
+// behind the other (part, count, parts), 3.4 us: one row x 32 heads x 6404 keys, keys from HBM 11.9 -> 10.55 us a pass, from the cache
+// 12.4 -> 9.2; 4 x 1 rows, eight layers with a mask 206 -> 202.5.  (Counting before the sums are formed and waiting for parts that are
+// emptied at the start to be filled: 11.8 and 203.5, as the keys then queue behind that.  Loads of one part each and
+// reductions through LDS in the fold: 4.2 us.)
+constexpr uint64_t FEW_COUNT = 0xffa5ffc37fb95aull;
+
+template <int DH>
+struct FewColumns {
+    const FwdParams& p;
+    const uint32_t ct, b, hk;
+    const int rows = p.row_end - p.row_begin, cols = p.G * rows - (int)ct * 32;
+    __device__ __forceinline__ uint32_t head(uint32_t col, uint32_t& row) const {
+        uint32_t h;
+        row = p.by_G.split(ct * 32 + col, h);
+        return hk * p.G + h;
+    }
+    __device__ __forceinline__ uint16_t* o(uint32_t col) const {
+        uint32_t row;
+        const uint32_t h = head(col, row);
+        return p.o + b * p.os.b + (int64_t)h * p.os.h + (int64_t)(p.row_begin + row) * p.os.s;
+    }
+    __device__ __forceinline__ uint64_t* count() const { return reinterpret_cast<uint64_t*>(o(0)); }
+    __device__ __forceinline__ void open(uint64_t found) const {
+        if (found >> 8 != FEW_COUNT)
+            __hip_atomic_compare_exchange_strong(count(), &found, FEW_COUNT << 8, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ bool last() const {
+        return __hip_atomic_fetch_add(count(), 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (FEW_COUNT << 8) + (uint32_t)(p.nsplit - 1);
+    }
+    // where a column is in a part, and how far apart parts are, in rows
+    __device__ __forceinline__ int64_t at(uint32_t col) const {
+        uint32_t row;
+        const uint32_t h = head(col, row);
+        return ((int64_t)b * p.Hq + h) * rows + row;
+    }
+    __device__ __forceinline__ int64_t all_rows() const { return (int64_t)p.B * p.Hq * rows; }
+
+    // One wave: its column of a part, two values of d to a lane
+    __device__ __forceinline__ void store(uint32_t col, uint32_t split, float x0, float x1, float lse) const {
+        const int lane = threadIdx.x & 63;
+        const int64_t r = split * all_rows() + at(col);
+        const uint64_t u = (uint64_t)__float_as_uint(x1) << 32 | __float_as_uint(x0);
+        if (lane < DH / 2) __hip_atomic_store(reinterpret_cast<uint64_t*>(p.part + r * DH) + lane, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) __hip_atomic_store(p.l_part + r, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // One wave: a column's parts.  DH / 4 lanes share a part, so that eight loads of the wave have 16 parts of 128 values in
+    // flight, and lane k has the weight of part k.
+    template <class E>
+    __device__ __forceinline__ void fold(uint32_t col) const {
+        constexpr int LPP = DH / 4, PPL = 64 / LPP, LOADS = 8;
+        const int lane = threadIdx.x & 63, grp = lane / LPP, d = lane % LPP * 4, n = p.nsplit;
+        const int64_t all = all_rows(), r = at(col);
+        const float* const lp = p.l_part + r + min(lane, n - 1) * all;
+        const float* const src = p.part + r * DH + d;
+        float l, w = 0.f, m = 0.f, den = 0.f, x[4] = {0.f, 0.f, 0.f, 0.f};
+        asm volatile("global_load_dword %0, %1, off sc1" : "=v"(l) : "v"(lp) : "memory");
+        int k0 = 0;
+        do {
+            u32x4 u[LOADS];
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j)
+                asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(u[j]) : "v"(src + min(k0 + j * PPL + grp, n - 1) * (all * DH)) : "memory");
+            if (k0 == 0) {
+                wait_vmcnt<LOADS>();
+                asm volatile("" : "+v"(l));
+                if (lane >= n) l = -INFINITY;
+                m = wave_max(l);
+                w = __expf(l - (m == -INFINITY ? 0.f : m));
+                den = wave_sum(w);
+            }
+            wait_vmcnt<0>();
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j) asm volatile("" : "+v"(u[j]));
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j) {
+                const int k = k0 + j * PPL + grp;
+                float wk = __shfl(w, k & 63);                   // (past the last part: lanes of weight 0)
+                if (k >= 64) wk = 0.f;
+                // a part of weight 0 may hold anything, one of weight NaN makes the row NaN
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = wk != 0.f ? fmaf(__uint_as_float(u[j][e]), wk, x[e]) : x[e];
+            }
+        } while ((k0 += LOADS * PPL) < n);
+#pragma unroll
+        for (int off = LPP; off < 64; off <<= 1)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] += __shfl_xor(x[e], off);
+        const float inv = den > 0.f ? 1.f / den : 0.f;
+        if (grp == 0) *reinterpret_cast<u32x2*>(o(col) + d) = u32x2{E::pack(x[0] * inv, x[1] * inv), E::pack(x[2] * inv, x[3] * inv)};
+        uint32_t row;
+        const uint32_t h = head(col, row);
+        if (lane == 0) p.lse[((int64_t)b * p.Hq + h) * p.lse_bh_stride + p.row_begin + row] = den > 0.f ? m + __logf(den) : -INFINITY;
+    }
+};
+
 // Few rows (text being generated, short questions): the work is reading K and V once, 512 bytes per key
 // and kv head for a handful of multiplications, so the kernel is built around the loads.
 //
@@ -788,6 +894,7 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     constexpr int RING = 4 * 2 * 2 * PB, FOLD = 4 * 32 * EPS * 4;
     __shared__ __attribute__((aligned(1024))) char lds[RING > FOLD ? RING : FOLD];
     __shared__ float ml[4][2][32];                                  // per wave and column: reference maximum, row sum
+    __shared__ int last;
 
     fetch_kernargs<sizeof(FwdParams)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
@@ -801,6 +908,11 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     const int col = min((int)ct * 32 + l32, n_cols - 1);            // columns past the last repeat it and are not stored
     uint32_t head;
     const int row = p.row_begin + p.by_G.split(col, head), h = hk * p.G + head;
+
+    const FewColumns<DH> columns{p, ct, b, hk};     // (where p.part says so)
+    uint64_t word = 0;
+    asm volatile("s_cmp_eq_u64 %2, 0\n\ts_cbranch_scc1 LVX_FEW_WORD_%=\n\tglobal_load_dwordx2 %0, %1, off sc1\nLVX_FEW_WORD_%=:"
+                 : "+v"(word) : "v"(columns.count()), "s"(p.part) : "memory", "scc");
 
     u32x4 q[NKK];
     {
@@ -890,6 +1002,8 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
         asm volatile("" : "+v"(q[kk]));
         if (MASKED && empty) q[kk] = u32x4{0u, 0u, 0u, 0u};
     }
+    asm volatile("" : "+v"(word));          // requested before Q
+    if (p.part && tid == 0) columns.open(word);
 
     for (int i = 0; i < n; ++i) {
         const int kv0 = base + 32 * (wave + 4 * i);
@@ -984,6 +1098,29 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
         ml[wave][1][l32] = empty ? 0.f : l_tot;
     }
     __syncthreads();
+    if (p.part) {                   // the columns are four at most
+        if (wave < columns.cols) {
+            float M = -INFINITY, den = 0.f, x0 = 0.f, x1 = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) M = fmaxf(M, ml[k][0][wave]);
+            const float* const src = reinterpret_cast<const float*>(lds) + wave * EPS + 2 * min(lane, DH / 2 - 1);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float w = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((ml[k][0][wave] - M) * cc);
+                den = fmaf(w, ml[k][1][wave], den);
+                x0 = fmaf(w, src[k * (32 * EPS)], x0);
+                x1 = fmaf(w, src[k * (32 * EPS) + 1], x1);
+            }
+            const float inv = den > 0.f ? 1.f / den : 0.f;
+            columns.store(wave, split, x0 * inv, x1 * inv, den > 0.f ? M * p.scale + __logf(den) : no_lse(p, den));
+            wait_vmcnt<0>();        // it is where the last work-group will read it
+        }
+        __syncthreads();
+        if (tid == 0) last = columns.last();
+        __syncthreads();
+        if (last && wave < columns.cols) columns.template fold<E>(wave);
+        return;
+    }
     constexpr int TPC = 8, DPT = DH / TPC;          // threads per column, values of d per thread
     const int oc = tid / TPC, part = tid % TPC;
     if ((int)ct * 32 + oc >= n_cols) return;

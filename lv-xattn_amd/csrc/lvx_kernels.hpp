@@ -82,6 +82,10 @@ struct FwdParams {
     float scale, scale_log2e;
     int f16;                   // element type of q, k, v, o: 0 bf16, 1 fp16
     int o_f32;                 // 1: o (the parts of a launch with key splits) is fp32
+    // Form for few rows: not null, and the key ranges' work-groups leave their fp32 parts, [nsplit][B * Hq][rows][D] and
+    // [nsplit][B * Hq][rows], here; the last of a kv head folds them into o and lse, which are then the result's
+    float* part;
+    float* l_part;
     // filled in by launch_fwd: divisors by n_row_tiles, nsplit, B, G and G / HG
     Divisor by_row_tiles, by_splits, by_B, by_G, by_head_groups;
 };
