@@ -242,6 +242,15 @@ int lvx_bwd(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tensor* 
             const lvx_tensor* dq, const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate,
             int32_t row_begin, int32_t row_count, void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * lvx_bwd_preprocess and lvx_bwd in one: delta is formed from o (as the forward left it) by a launch that lvx_bwd has anyway.
+ * The results are those of the two, bit for bit.
+ */
+int lvx_bwd_from_o(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
+                   const lvx_tensor* o, const lvx_tensor* dout, const float* lse,
+                   const lvx_tensor* dq, const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate,
+                   int32_t row_begin, int32_t row_count, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Never less for more rows: a workspace of the longest window of a call serves all its windows. */
 size_t lvx_bwd_workspace_bytes(const lvx_attn_shape* shape, int32_t row_count);
 

@@ -759,16 +759,28 @@ struct WaitingDq {
 
 // One window, its arguments checked, in the workspace of one of ws_rows rows, at least as many.  meta: null, or the records of
 // its rows.  before: null, or what the window before has left and this one may leave.
-static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
+static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v, const lvx_tensor* o,
                       const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
                       const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate, int32_t row_begin, int32_t row_count,
                       void* workspace, int32_t ws_rows, hipStream_t st, const float* meta, WaitingDq* before);
 
-int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
-            const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
-            const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate,
-            int32_t row_begin, int32_t row_count, void* workspace, size_t workspace_bytes, void* stream) {
-    LVX_TRY(check_shape(s));
+// The row records' arguments.  Delta is read, or with o (and no delta) formed on the way.
+static MetaParams meta_params(const lvx_attn_shape* s, const lvx_tensor* o, const lvx_tensor* dout, const float* lse, const float* delta,
+                              float* out, int32_t row_begin, int32_t row_end, int n_tiles) {
+    MetaParams p{lse, delta, out, s->B, s->Hq, s->Lq, row_begin, row_end, n_tiles, 1, row_end - row_begin, 0, s->scale};
+    if (o) {
+        p.o = static_cast<const uint16_t*>(o->ptr); p.os = st3(o);
+        p.dout = static_cast<const uint16_t*>(dout->ptr); p.ds = st3(dout);
+        p.D = s->D;
+        p.f16 = s->dtype == LVX_F16;
+    }
+    return p;
+}
+
+static int bwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v, const lvx_tensor* o,
+                    const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
+                    const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate,
+                    int32_t row_begin, int32_t row_count, void* workspace, size_t workspace_bytes, void* stream) {
     LVX_TRY(check_tensor(q));
     LVX_TRY(check_tensor(k));
     LVX_TRY(check_tensor(v));
@@ -776,7 +788,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     LVX_TRY(check_tensor(dq));
     LVX_TRY(check_tensor(dk));
     LVX_TRY(check_tensor(dv));
-    if (!lse || !delta) return LVX_ERR_NULL;
+    if (!lse) return LVX_ERR_NULL;
     const int rounds = dkv_accumulate > 0 ? dkv_accumulate >> 12 : 0;
     if (rounds > 0) dkv_accumulate &= (1 << 12) - 1;
     if (dkv_accumulate != 0 && dkv_accumulate != 1) return LVX_ERR_SHAPE;
@@ -790,7 +802,7 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     if (!workspace || workspace_bytes < lvx_bwd_workspace_bytes(s, round_rows)) return LVX_ERR_WORKSPACE;
     if (!aligned16(workspace)) return LVX_ERR_ALIGN;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (rounds <= 1) return bwd_window(s, q, k, v, dout, lse, delta, dq, dk, dv, dkv_accumulate, row_begin, row_count, workspace, row_count, st, nullptr, nullptr);
+    if (rounds <= 1) return bwd_window(s, q, k, v, o, dout, lse, delta, dq, dk, dv, dkv_accumulate, row_begin, row_count, workspace, row_count, st, nullptr, nullptr);
 
     // Several windows: the records of all their rows by one launch instead of one of 3 - 5 us each (32 heads x 16 rounds of 256 rows,
     // forward and backward 2775 -> 2741 us), where the scratch that only sums of 16-bit dk, dv use holds them.
@@ -800,18 +812,36 @@ int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, c
     float* meta = nullptr;
     if (n <= 65535 && (size_t)each * n * sizeof(float) <= w.meta - w.dkv) {
         meta = reinterpret_cast<float*>(static_cast<char*>(workspace) + w.dkv);
-        MetaParams mp{lse, delta, meta, s->B, s->Hq, s->Lq, row_begin, row_begin + row_count, w.n_tiles, n, round_rows, each, s->scale};
+        MetaParams mp = meta_params(s, o, dout, lse, delta, meta, row_begin, row_begin + row_count, w.n_tiles);
+        mp.rounds = n; mp.round_rows = round_rows; mp.round_out = each;
         const hipError_t e = launch_bwd_meta(mp, st);
         if (e != hipSuccess) return static_cast<int>(e);
     }
     WaitingDq waiting{};
     for (int r = 0; r < n; ++r)
-        LVX_TRY(bwd_window(s, q, k, v, dout, lse, delta, dq, dk, dv, 1, row_begin + r * round_rows, std::min(round_rows, row_count - r * round_rows),
+        LVX_TRY(bwd_window(s, q, k, v, o, dout, lse, delta, dq, dk, dv, 1, row_begin + r * round_rows, std::min(round_rows, row_count - r * round_rows),
                            workspace, round_rows, st, meta ? meta + r * each : nullptr, &waiting));
     return waiting.any ? static_cast<int>(launch_cast(waiting.slices, st)) : LVX_OK;
 }
 
-static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
+int lvx_bwd(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v,
+            const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
+            const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate,
+            int32_t row_begin, int32_t row_count, void* workspace, size_t workspace_bytes, void* stream) {
+    LVX_TRY(check_shape(s));
+    if (!delta) return LVX_ERR_NULL;
+    return bwd_impl(s, q, k, v, nullptr, dout, lse, delta, dq, dk, dv, dkv_accumulate, row_begin, row_count, workspace, workspace_bytes, stream);
+}
+
+int lvx_bwd_from_o(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v, const lvx_tensor* o,
+                   const lvx_tensor* dout, const float* lse, const lvx_tensor* dq, const lvx_tensor* dk, const lvx_tensor* dv,
+                   int32_t dkv_accumulate, int32_t row_begin, int32_t row_count, void* workspace, size_t workspace_bytes, void* stream) {
+    LVX_TRY(check_shape(s));
+    LVX_TRY(check_tensor(o));
+    return bwd_impl(s, q, k, v, o, dout, lse, nullptr, dq, dk, dv, dkv_accumulate, row_begin, row_count, workspace, workspace_bytes, stream);
+}
+
+static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v, const lvx_tensor* o,
                       const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
                       const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate, int32_t row_begin, int32_t row_count,
                       void* workspace, int32_t ws_rows, hipStream_t st, const float* meta, WaitingDq* before) {
@@ -877,10 +907,10 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
                         row_begin + row_count, n_tiles, n_groups, p.n_kv_blocks};
         p.live_runs = lp.live_runs;
     }
-    const bool has_hulls = !meta;       // its records come by a launch of its own, which forms the hulls as well
+    const bool has_hulls = !meta;       // its records come by a launch of its own, which writes the tables as well, or their hulls
     if (!meta) {
         float* const out = reinterpret_cast<float*>(wsb + wsl.meta);
-        MetaParams mp{lse, delta, out, s->B, s->Hq, s->Lq, row_begin, row_begin + row_count, n_tiles, 1, row_count, 0, s->scale};
+        MetaParams mp = meta_params(s, o, dout, lse, delta, out, row_begin, row_begin + row_count, n_tiles);
         mp.scratch = scratch;
         mp.sb = sb;
         hipError_t em = launch_bwd_meta(mp, st, hull ? &lp : nullptr);

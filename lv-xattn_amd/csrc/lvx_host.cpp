@@ -31,6 +31,7 @@ struct Library {
     decltype(&lvx_fwd_acc) fwd_acc;
     decltype(&lvx_bwd_preprocess) bwd_preprocess;
     decltype(&lvx_bwd) bwd;
+    decltype(&lvx_bwd_from_o) bwd_from_o;
     decltype(&lvx_bwd_workspace_bytes) bwd_workspace_bytes;
     decltype(&lvx_bias_hull) bias_hull;
 } lib;
@@ -42,6 +43,7 @@ void bind(const std::map<std::string, uintptr_t>& addresses) {
     set(lib.fwd_acc, "lvx_fwd_acc");
     set(lib.bwd_preprocess, "lvx_bwd_preprocess");
     set(lib.bwd, "lvx_bwd");
+    set(lib.bwd_from_o, "lvx_bwd_from_o");
     set(lib.bwd_workspace_bytes, "lvx_bwd_workspace_bytes");
     set(lib.bias_hull, "lvx_bias_hull");
 }
@@ -182,21 +184,27 @@ bool bwd_preprocess(const Tensor& o, const Tensor& dout, const Tensor& delta, in
     return true;
 }
 
-bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
+// delta, or the o to form it from
+bool bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const OptTensor& delta, const Tensor& dq,
          const Tensor& dk, const Tensor& dv, double scale, int64_t row_begin, int64_t row_count, const OptTensor& kv_len,
-         const OptTensor& kv_start, const OptTensor& kv_end, int64_t accumulate_dkv, const Tensor& ws, const OptTensor& bias) {
+         const OptTensor& kv_start, const OptTensor& kv_end, int64_t accumulate_dkv, const Tensor& ws, const OptTensor& bias,
+         const OptTensor& o) {
     lvx_attn_shape s;
     if (!fill_shape(s, q, k, v, scale, kv_len, kv_start, kv_end) || !fill_bias(s, bias, q)) return false;
     const at::ScalarType kv_type = accumulate_dkv ? at::kFloat : q.scalar_type();
-    if (!plain4(dout, q, q.scalar_type()) || dout.sizes() != q.sizes() || !rows_ok(lse, q) || !rows_ok(delta, q) ||
-        !plain4(dq, q, q.scalar_type()) || dq.sizes() != q.sizes() || !plain4(dk, q, kv_type) || dk.sizes() != k.sizes() ||
+    if (!plain4(dout, q, q.scalar_type()) || dout.sizes() != q.sizes() || !rows_ok(lse, q) || !delta == !o ||
+        (delta && !rows_ok(*delta, q)) || (o && (!plain4(*o, q, q.scalar_type()) || o->sizes() != q.sizes())) || !plain4(dq, q, q.scalar_type()) || dq.sizes() != q.sizes() || !plain4(dk, q, kv_type) || dk.sizes() != k.sizes() ||
         !plain4(dv, q, kv_type) || dv.sizes() != k.sizes())
         return false;
     const lvx_tensor tq = t4(q), tk = t4(k), tv = t4(v), td = t4(dout), tdq = t4(dq), tdk = t4(dk), tdv = t4(dv);
-    const float *const lp = lse.data_ptr<float>(), *const dp = delta.data_ptr<float>();
+    const float *const lp = lse.data_ptr<float>(), *const dp = delta ? delta->data_ptr<float>() : nullptr;
+    const lvx_tensor to = o ? t4(*o) : lvx_tensor{};
     void *const wp = ws.data_ptr(), *const st = current_stream();
     const size_t wb = ws.nbytes();
     call("lvx_bwd", [&] {
+        if (o)
+            return lib.bwd_from_o(&s, &tq, &tk, &tv, &to, &td, lp, &tdq, &tdk, &tdv, (int32_t)accumulate_dkv, (int32_t)row_begin,
+                                  (int32_t)row_count, wp, wb, st);
         return lib.bwd(&s, &tq, &tk, &tv, &td, lp, dp, &tdq, &tdk, &tdv, (int32_t)accumulate_dkv, (int32_t)row_begin, (int32_t)row_count,
                        wp, wb, st);
     });

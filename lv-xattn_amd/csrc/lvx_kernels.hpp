@@ -219,8 +219,7 @@ struct BwdParams {
 // smallest range of whole token blocks that holds every key some row of the tile sees.  The dQ kernel takes its row tiles,
 // groups of LIVE_GROUP row tiles, over the hull of the group, and reads a tile's dS^T inside the tile's own hull only.
 // (With whole groups alive or not, 2 x 3000 rows that see the image before them visited 13 % more pairs, since images
-// begin inside groups: bwd_kernel 689 us, 599 now, forward and backward 1144 -> 1067; the two table kernels 2.5 us each, or
-// 5 where another kernel left its lines in no cache, as before.)
+// begin inside groups: bwd_kernel 689 us, 599 now, forward and backward 1144 -> 1067)
 constexpr int LIVE_GROUP = 8;
 constexpr int MAX_RANKED_GROUPS = 1024;    // groups of a launch that are still ranked by length
 struct LiveParams {
@@ -234,7 +233,11 @@ struct LiveParams {
                                // longest hull first (ties in index order)
     int B, Lq, Lkv, row_begin, row_end, n_tiles, n_groups, n_kv_blocks;
 };
-// has_hulls: tile_hull is written already
+// Whether one launch writes all three, its work-groups taking the hulls they need themselves instead of waiting for a launch of them:
+// each reads all intervals of a sample, and one those of all samples, 256 rows in a wave's 0.5 us.
+constexpr int MAX_LIVE_TILES = 512;
+inline bool live_in_one(const LiveParams& p) { return (int64_t)p.B * p.n_groups * LIVE_GROUP <= MAX_LIVE_TILES; }
+// has_hulls: launch_bwd_meta has been given the same (and written tile_hull, or all three)
 hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st, bool has_hulls);
 
 // The token blocks of a backward launch that several work-groups share, hence whose dK / dV are summed in the
@@ -256,11 +259,17 @@ struct MetaParams {
     int rounds, round_rows;
     int64_t round_out;
     float scale;
+    // not null: delta is formed from these and not read
+    const uint16_t* o;
+    const uint16_t* dout;
+    Strides3 os, ds;
+    int D, f16;
     float* scratch;            // null, or the fp32 dK / dV scratch whose shared token blocks the same launch zeroes
     SharedBlocks sb;
-    int meta_blocks;           // filled by the launcher: blocks [0, meta_blocks) write records
-    int zero_end;              // blocks [meta_blocks, zero_end) zero the scratch, those past them form the hulls of `live`
-    Divisor by_rows;           // and the divisor by the rows of the window's whole tiles
+    // filled in by the launcher: blocks [0, table_blocks) write the tables of `live` (or, not with `tables`, its tile_hull only),
+    // those up to meta_end the records (in every window, blockIdx.y), the others zero the scratch
+    int table_blocks, tables, meta_end;
+    Divisor by_rows, by_Hq;    // by the rows of the window's whole tiles, by q heads
     LiveParams live;
 };
 
@@ -343,7 +352,7 @@ hipError_t launch_bwd(const BwdParams& p, bool masked, hipStream_t st, const Cas
 hipError_t plan_cast_t(CastParams& p, int threads);
 hipError_t launch_cast(const CastParams& p, hipStream_t st);
 hipError_t launch_cast_shared(const CastSharedParams& p, hipStream_t st);
-// live: null, or what has its tile hulls formed by the same launch (of one window)
+// live: null, or what has its tables, or with many row tiles its hulls, written by the same launch (of one window)
 hipError_t launch_bwd_meta(const MetaParams& p, hipStream_t st, const LiveParams* live = nullptr);
 
 // Backward of the 128-wide RMS norm: rows of dy, x [M][heads][128] (row strides ldy, ldx), r [M][heads].

@@ -174,6 +174,20 @@ __global__ __launch_bounds__(256) void merge_pair_kernel(const MergeParams p) {
     }
 }
 
+// A row's sum of products, of the eight of each of its 1 << sh lanes.
+template <class E>
+__device__ __forceinline__ float row_dot(u32x4 a, u32x4 b, int sh) {
+    float x[8], y[8], s = 0.f;
+    unpack8<E>(a, x);
+    unpack8<E>(b, y);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s = fmaf(x[j], y[j], s);
+    if (sh >= 4) s += __shfl_xor(s, 8);
+    if (sh >= 3) s += __shfl_xor(s, 4);
+    if (sh >= 2) s += __shfl_xor(s, 2);
+    return s + __shfl_xor(s, 1);
+}
+
 // delta = rowsum(O * dO): head_dim / 8 lanes x 16 bytes per row and tensor, two rows per thread with all
 // four loads issued before the first use.  516 bytes per (row, head).
 template <bool F16>
@@ -203,16 +217,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(const PreParams p) {
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        float fo[8], fd[8];
-        unpack8<E>(uo[k], fo);
-        unpack8<E>(ud[k], fd);
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s = fmaf(fo[j], fd[j], s);
-        if (sh >= 4) s += __shfl_xor(s, 8);
-        if (sh >= 3) s += __shfl_xor(s, 4);
-        if (sh >= 2) s += __shfl_xor(s, 2);
-        s += __shfl_xor(s, 1);
+        const float s = row_dot<E>(uo[k], ud[k], sh);
         if ((k ? ok1 : ok0) && chunk == 0) *out[k] = s;
     }
 }
@@ -227,46 +232,174 @@ __device__ __forceinline__ int shared_block(const SharedBlocks& s, int i) {
     return blk0 + at;
 }
 
-// One thread per row: the hulls of the row tiles' key intervals in whole token blocks.  i: work-group, of hull_blocks.
-__host__ __device__ __forceinline__ int hull_blocks(const LiveParams& p) { return (p.n_tiles + 7) / 8 * p.B; }
-__device__ __forceinline__ void tile_hulls(const LiveParams& p, int i) {
-    const int per = (p.n_tiles + 7) / 8, b = i / per, tile = (i - b * per) * 8 + (threadIdx.x >> 5);
-    const int r = p.row_begin + tile * 32 + (threadIdx.x & 31);
-    const int kv_len = p.kv_len ? min(p.kv_len[b], p.Lkv) : p.Lkv;
-    int lo = INT_MAX, hi = 0;
-    if (r < p.row_end) {
-        const int s = max(p.kv_start[(int64_t)b * p.Lq + r], 0);
-        const int e = min(p.kv_end[(int64_t)b * p.Lq + r], kv_len);
-        if (e > s) { lo = s; hi = e; }
-    }
+// A row's key interval, (INT_MAX, 0) where it sees nothing or lies past the window.
+__device__ __forceinline__ void row_interval(const LiveParams& p, int b, int kv_len, int r, int& lo, int& hi) {
+    const int64_t at = (int64_t)b * p.Lq + min(r, p.row_end - 1);
+    lo = max(p.kv_start[at], 0);
+    hi = min(p.kv_end[at], kv_len);
+    if (r >= p.row_end || hi <= lo) { lo = INT_MAX; hi = 0; }
+}
+__device__ __forceinline__ int len_of(const LiveParams& p, int b) { return p.kv_len ? min(p.kv_len[b], p.Lkv) : p.Lkv; }
+// The hull of the intervals of a lane's 32, in whole token blocks.
+__device__ __forceinline__ void hull_of_32(int& lo, int& hi) {
 #pragma unroll
     for (int o = 1; o < 32; o <<= 1) {
         lo = min(lo, __shfl_xor(lo, o));
         hi = max(hi, __shfl_xor(hi, o));
     }
+    lo = hi > 0 ? (lo / 128) * 128 : 0;
+    hi = (hi + 127) / 128 * 128;
+}
+
+// One thread per row: the hulls of the row tiles' key intervals in whole token blocks.  i: work-group, of hull_blocks.
+__host__ __device__ __forceinline__ int hull_blocks(const LiveParams& p) { return (p.n_tiles + 7) / 8 * p.B; }
+__device__ __forceinline__ void tile_hulls(const LiveParams& p, int i) {
+    const int per = (p.n_tiles + 7) / 8, b = i / per, tile = (i - b * per) * 8 + (threadIdx.x >> 5);
+    int lo, hi;
+    row_interval(p, b, len_of(p, b), p.row_begin + tile * 32 + (threadIdx.x & 31), lo, hi);
+    hull_of_32(lo, hi);
     if ((threadIdx.x & 31) == 0 && tile < p.n_tiles) {
         int32_t* h = p.tile_hull + ((int64_t)b * p.n_tiles + tile) * 2;
-        h[0] = hi > 0 ? (lo / 128) * 128 : 0;
-        h[1] = (hi + 127) / 128 * 128;
+        h[0] = lo;
+        h[1] = hi;
     }
+}
+
+// One wave: the runs of consecutive row tiles whose hull (h, [n_tiles][2]) holds token block kblk.  Where there are more than
+// four, the two the narrowest gap apart become one, so that the three widest gaps are left out.
+__device__ __forceinline__ void live_runs(const LiveParams& p, const int32_t* h, int b, int kblk) {
+    const int lane = threadIdx.x & 63, kvb = kblk * 128;
+    int first[4] = {0, 0, 0, 0}, end[4] = {0, 0, 0, 0}, nr = 0, last_end = -1;
+    for (int t0 = 0; t0 < p.n_tiles; t0 += 64) {
+        const int32_t* const ht = h + min(t0 + lane, p.n_tiles - 1) * 2;
+        uint64_t live = __builtin_amdgcn_ballot_w64(t0 + lane < p.n_tiles && ht[0] <= kvb && kvb < ht[1]);
+        while (live) {
+            const int bit = __builtin_ctzll(live), s = t0 + bit;
+            const uint64_t gaps = ~(live >> bit);
+            const int n = min(gaps ? __builtin_ctzll(gaps) : 64, 64 - bit), e = s + n;
+            live &= n == 64 ? 0 : ~(((uint64_t{1} << n) - 1) << bit);
+            const bool apart = s != last_end, append = apart && nr < 4;
+            if (apart && !append) {
+                int width = s - end[3], at = 3;
+#pragma unroll
+                for (int i = 2; i >= 0; --i)
+                    if (first[i + 1] - end[i] < width) { width = first[i + 1] - end[i]; at = i; }
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {   // close gap `at`: the runs on its sides become one, the later ones move up
+                    if (i >= at) end[i] = end[i + 1];
+                    if (i > at) first[i] = first[i + 1];
+                }
+                if (at < 3) first[3] = s;
+            }
+            if (append) ++nr;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (i == nr - 1) { if (append) first[i] = s; end[i] = e; }
+            last_end = e;
+        }
+    }
+    if (lane < 8) {
+        int x = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (lane == 2 * i && i < nr) x = first[i];
+            if (lane == 2 * i + 1 && i < nr) x = end[i] - first[i];
+        }
+        p.live_runs[((int64_t)b * p.n_kv_blocks + kblk) * 8 + lane] = x;
+    }
+}
+
+// Group i of n is as many places behind the first as there are longer ones and, before it, equally long ones.
+__device__ __forceinline__ void rank_group(const LiveParams& p, const int* len, int i, int n) {
+    const int mine = len[i];
+    int rank = 0;
+    for (int j = 0; j < n; ++j) rank += (len[j] > mine || (len[j] == mine && j < i)) ? 1 : 0;
+    p.order[rank] = i;
+}
+
+// The same tables without one launch waiting for another, where there are few row tiles: four token blocks of a sample to a
+// work-group, which takes the hulls of the sample's tiles itself (a few loads per thread, all in flight, at most MAX_LIVE_TILES
+// tiles in all samples); the sample's first writes them down as well, and one more work-group takes the hulls of the groups
+// and ranks them.
+__host__ __device__ __forceinline__ int live_blocks(const LiveParams& p) { return (p.n_kv_blocks + 3) / 4 * p.B + (p.order ? 1 : 0); }
+__device__ __forceinline__ void live_tables(const LiveParams& p, int i) {
+    __shared__ int32_t hull[MAX_LIVE_TILES * 2];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, per = (p.n_kv_blocks + 3) / 4, b = i / per;
+    constexpr int AHEAD = 4;
+    if (b >= p.B) {
+        const int n = p.B * p.n_groups;
+        int* const len = hull;
+        for (int j = wave; j < n; j += 4) {
+            const int gb = j / p.n_groups, r0 = p.row_begin + (j - gb * p.n_groups) * (LIVE_GROUP * 32) + lane, kv_len = len_of(p, gb);
+            int lo[4], hi[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) row_interval(p, gb, kv_len, r0 + 64 * k, lo[k], hi[k]);
+            int l = min(min(lo[0], lo[1]), min(lo[2], lo[3])), h = max(max(hi[0], hi[1]), max(hi[2], hi[3]));
+            l = min(l, __shfl_xor(l, 32));
+            h = max(h, __shfl_xor(h, 32));
+            hull_of_32(l, h);
+            if (lane == 0) len[j] = h - l;
+        }
+        __syncthreads();
+        if ((int)threadIdx.x < n) rank_group(p, len, threadIdx.x, n);
+        return;
+    }
+    const int kv_len = len_of(p, b);
+    for (int t0 = 0; t0 < p.n_tiles; t0 += 8 * AHEAD) {
+        int lo[AHEAD], hi[AHEAD];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) row_interval(p, b, kv_len, p.row_begin + (t0 + 8 * k) * 32 + (int)threadIdx.x, lo[k], hi[k]);
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) {
+            const int tile = t0 + 8 * k + (threadIdx.x >> 5);
+            hull_of_32(lo[k], hi[k]);
+            if ((threadIdx.x & 31) == 0 && tile < p.n_tiles) { hull[2 * tile] = lo[k]; hull[2 * tile + 1] = hi[k]; }
+        }
+    }
+    __syncthreads();
+    const int kblk = (i - b * per) * 4 + wave;
+    if (kblk < p.n_kv_blocks) live_runs(p, hull, b, kblk);
+    if (i != b * per) return;
+    for (int k = threadIdx.x; k < 2 * p.n_tiles; k += 256) p.tile_hull[(int64_t)b * p.n_tiles * 2 + k] = hull[k];
 }
 
 // LSE and delta of the window, re-expressed once for the backward kernel: the
 // exponent offset LSE * log2(e), +inf for rows that saw no key or lie past the
 // window (so that P = exp2(x - inf) = 0 there), and delta * scale (0 past the
 // window), grouped per 32-row tile so that one 256-byte load fetches a tile's lot.
+struct MetaRow {
+    const MetaParams& p;
+    int begin, end, n_tiles;                // of this window
+    __device__ __forceinline__ explicit MetaRow(const MetaParams& params) : p(params) {
+        begin = p.row_begin + (int)blockIdx.y * p.round_rows;
+        end = min(begin + p.round_rows, p.row_end);
+        n_tiles = (end - begin + 31) / 32;  // a last window may be shorter
+    }
+    __device__ __forceinline__ void write(int64_t bh, uint32_t r, float l, float d) const {
+        float* o = p.out + blockIdx.y * p.round_out + (bh * n_tiles + (r >> 5)) * 64 + (r & 31);
+        o[0] = (l == -INFINITY) ? INFINITY : l * 1.4426950408889634f;
+        o[32] = d * p.scale;
+    }
+};
+
+// FROM_O: delta = rowsum(O * dO) is formed here, the loads and sums of preprocess_kernel, whose launch and whose 4 bytes a row there
+// and back it saves.  Bound by reading O and dO.  us alone, preprocess_kernel, records and tables of a mask in launches of their own ->
+// in one: 4096 rows x 32 heads 12.0 + 5.4 -> 16.0, 2048 x 32 of 64 5.6 + 6.9 -> 7.1, 2 x 3000 x 32 with a mask 16.1 + 5.1 + 5.6 -> 18.2,
+// 1024 x 16 with one 5.0 + 5.0 + 5.6 -> 5.3 (forward and backward 231 -> 225).
+template <bool FROM_O, bool F16>
 __global__ __launch_bounds__(256) void bwd_meta_kernel(const MetaParams p) {
-    fetch_kernargs<offsetof(MetaParams, live)>();
-    // With an interval mask the last blocks form the hulls of the row tiles: a launch less, 3 us (fp16, 16 heads, 1024 x 4096
-    // with a dense bias, forward and backward 232 -> 230)
-    if ((int)blockIdx.x >= p.zero_end) {
-        tile_hulls(p.live, (int)blockIdx.x - p.zero_end);
+    fetch_kernargs<sizeof(MetaParams)>();
+    // With an interval mask the first blocks write its tables, or where there are many row tiles their hulls
+    if ((int)blockIdx.x < p.table_blocks) {
+        if (blockIdx.y) return;
+        if (p.tables) live_tables(p.live, (int)blockIdx.x);
+        else tile_hulls(p.live, (int)blockIdx.x);
         return;
     }
-    // the other blocks of the launch zero the scratches (stores rather than hipMemsetAsync, so
+    // the last blocks of the launch zero the scratches (stores rather than hipMemsetAsync, so
     // that callers may capture the stream)
-    if ((int)blockIdx.x >= p.meta_blocks) {
-        const int z = (int)blockIdx.x - p.meta_blocks;
+    if ((int)blockIdx.x >= p.meta_end) {
+        const int z = (int)blockIdx.x - p.meta_end;
         const int blk = shared_block(p.sb, z / SHARE_PARTS);
         if (blk < 0) return;
         const int kblk = blk % p.sb.n_kv_blocks, bh = blk / p.sb.n_kv_blocks, zb = bh % p.sb.B, hk = bh / p.sb.B;
@@ -281,20 +414,43 @@ __global__ __launch_bounds__(256) void bwd_meta_kernel(const MetaParams p) {
         }
         return;
     }
-    const int rows_pad = p.n_tiles * 32;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (int64_t)p.B * p.Hq * rows_pad) return;
-    uint32_t r;
-    const int64_t bh = p.by_rows.split((uint32_t)idx, r);
-    const int begin = p.row_begin + (int)blockIdx.y * p.round_rows, end = min(begin + p.round_rows, p.row_end);
-    const int row = begin + r, n_tiles = (end - begin + 31) / 32;
-    if ((int)(r >> 5) >= n_tiles) return;               // a shorter last window
-    const bool ok = row < end;
-    const float l = ok ? p.lse[bh * p.Lq + row] : -INFINITY;
-    const float d = ok ? p.delta[bh * p.Lq + row] : 0.f;
-    float* o = p.out + blockIdx.y * p.round_out + (bh * n_tiles + (r >> 5)) * 64 + (r & 31);
-    o[0] = (l == -INFINITY) ? INFINITY : l * 1.4426950408889634f;
-    o[32] = d * p.scale;
+    const MetaRow rec(p);
+    const int64_t total = (int64_t)p.B * p.Hq * p.n_tiles * 32;
+    const int64_t idx = (int64_t)((int)blockIdx.x - p.table_blocks) * 256 + threadIdx.x;
+    if constexpr (!FROM_O) {
+        if (idx >= total) return;
+        uint32_t r;
+        const int64_t bh = p.by_rows.split((uint32_t)idx, r);
+        if ((int)(r >> 5) >= rec.n_tiles) return;
+        const int row = rec.begin + (int)r;
+        const bool ok = row < rec.end;
+        rec.write(bh, r, ok ? p.lse[bh * p.Lq + row] : -INFINITY, ok ? p.delta[bh * p.Lq + row] : 0.f);
+    } else {
+        using E = Elt<F16>;
+        const int sh = chunk_shift(p.D), chunk = (int)(idx & ((1 << sh) - 1));
+        const int64_t half = total / 2, r0 = idx >> sh;             // total: whole tiles
+        if (r0 >= half) return;                                     // (the lanes of a row leave together)
+        u32x4 uo[2], ud[2];
+        float l[2];
+        uint32_t r[2];
+        int64_t bh[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const RowOf at((uint32_t)(r0 + k * half), p.by_rows, p.by_Hq);
+            r[k] = (uint32_t)at.row;
+            bh[k] = at.bh;
+            const int row = rec.begin + at.row;
+            const bool ok = row < rec.end;
+            uo[k] = ldg16(p.o + at.b * p.os.b + at.h * p.os.h + (int64_t)row * p.os.s + chunk * 8, ok);
+            ud[k] = ldg16(p.dout + at.b * p.ds.b + at.h * p.ds.h + (int64_t)row * p.ds.s + chunk * 8, ok);
+            l[k] = ok ? p.lse[bh[k] * p.Lq + row] : -INFINITY;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float s = row_dot<E>(uo[k], ud[k], sh);
+            if (chunk == 0 && (int)(r[k] >> 5) < rec.n_tiles) rec.write(bh[k], r[k], l[k], s);
+        }
+    }
 }
 
 // Per (b, text row) the first and one-past-last key whose bias is not -inf, over all heads the bias distinguishes.  An
@@ -443,8 +599,7 @@ __global__ __launch_bounds__(256) void mask_interval_kernel(const MaskIntervalPa
 
 __global__ __launch_bounds__(256) void bwd_hull_kernel(const LiveParams p) { tile_hulls(p, blockIdx.x); }
 
-// One wave per (token block, b): the runs of consecutive row tiles whose hull holds the block.  Where there are more than
-// four, the two the narrowest gap apart become one, so that the three widest gaps are left out.
+// One wave per (token block, b): its runs.
 // Blocks past those (b == 0 only) rank the groups of row tiles by the length of their hull, one thread per group.
 __global__ __launch_bounds__(64) void bwd_live_kernel(const LiveParams p) {
     const int lane = threadIdx.x;
@@ -464,52 +619,10 @@ __global__ __launch_bounds__(64) void bwd_live_kernel(const LiveParams p) {
             len[j] = max(0, hi - lo);
         }
         __syncthreads();
-        if (i >= n) return;
-        const int mine = len[i];
-        int rank = 0;
-        for (int j = 0; j < n; ++j) rank += (len[j] > mine || (len[j] == mine && j < i)) ? 1 : 0;
-        p.order[rank] = i;
+        if (i < n) rank_group(p, len, i, n);
         return;
     }
-    const int kblk = blockIdx.x, b = blockIdx.y, kvb = kblk * 128;
-    int first[4] = {0, 0, 0, 0}, end[4] = {0, 0, 0, 0}, nr = 0, last_end = -1;
-    for (int t0 = 0; t0 < p.n_tiles; t0 += 64) {
-        const int32_t* h = p.tile_hull + ((int64_t)b * p.n_tiles + min(t0 + lane, p.n_tiles - 1)) * 2;
-        uint64_t live = __builtin_amdgcn_ballot_w64(t0 + lane < p.n_tiles && h[0] <= kvb && kvb < h[1]);
-        while (live) {
-            const int bit = __builtin_ctzll(live), s = t0 + bit;
-            const uint64_t gaps = ~(live >> bit);
-            const int n = min(gaps ? __builtin_ctzll(gaps) : 64, 64 - bit), e = s + n;
-            live &= n == 64 ? 0 : ~(((uint64_t{1} << n) - 1) << bit);
-            const bool apart = s != last_end, append = apart && nr < 4;
-            if (apart && !append) {
-                int width = s - end[3], at = 3;
-#pragma unroll
-                for (int i = 2; i >= 0; --i)
-                    if (first[i + 1] - end[i] < width) { width = first[i + 1] - end[i]; at = i; }
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {   // close gap `at`: the runs on its sides become one, the later ones move up
-                    if (i >= at) end[i] = end[i + 1];
-                    if (i > at) first[i] = first[i + 1];
-                }
-                if (at < 3) first[3] = s;
-            }
-            if (append) ++nr;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (i == nr - 1) { if (append) first[i] = s; end[i] = e; }
-            last_end = e;
-        }
-    }
-    if (lane < 8) {
-        int x = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (lane == 2 * i && i < nr) x = first[i];
-            if (lane == 2 * i + 1 && i < nr) x = end[i] - first[i];
-        }
-        p.live_runs[((int64_t)b * p.n_kv_blocks + kblk) * 8 + lane] = x;
-    }
+    live_runs(p, p.tile_hull + (int64_t)blockIdx.y * p.n_tiles * 2, blockIdx.y, blockIdx.x);
 }
 
 template <bool F16>
@@ -682,19 +795,26 @@ hipError_t launch_preprocess(const PreParams& params, hipStream_t st) {
 
 hipError_t launch_bwd_meta(const MetaParams& p0, hipStream_t st, const LiveParams* live) {
     MetaParams p = p0;
-    if (live) p.live = *live;
-    const int hulls = live && live->n_tiles > 0 ? hull_blocks(*live) : 0;
-    const int64_t n = (int64_t)p.B * p.Hq * p.n_tiles * 32;
+    if (live && live->n_tiles > 0 && live->B > 0) {
+        p.live = *live;
+        p.tables = live_in_one(*live);
+        p.table_blocks = p.tables ? live_blocks(*live) : hull_blocks(*live);
+    }
+    const int64_t rows = p.out ? (int64_t)p.B * p.Hq * p.n_tiles * 32 : 0, n = p.o ? rows / 2 << chunk_shift(p.D) : rows;
     const int zero_blocks = p.scratch ? 8 * (p.sb.blocks_per_xcd - p.sb.whole) * SHARE_PARTS : 0;
-    if (n == 0 && zero_blocks == 0 && hulls == 0) return hipSuccess;
-    p.zero_end = (int)((n + 255) / 256) + zero_blocks;
-    p.meta_blocks = (int)((n + 255) / 256);
+    if (n == 0 && zero_blocks == 0 && p.table_blocks == 0) return hipSuccess;
+    p.meta_end = p.table_blocks + (int)((n + 255) / 256);
     p.by_rows = divisor(std::max(1, p.n_tiles * 32));
-    return launch1(bwd_meta_kernel, dim3((unsigned)(p.zero_end + hulls), p.rounds), dim3(256), st, p);
+    p.by_Hq = divisor(std::max(1, p.Hq));
+    const dim3 grid((unsigned)(p.meta_end + zero_blocks), std::max(1, p.rounds));
+    if (!p.o) return launch1(bwd_meta_kernel<false, false>, grid, dim3(256), st, p);
+    if (p.f16) return launch1(bwd_meta_kernel<true, true>, grid, dim3(256), st, p);
+    return launch1(bwd_meta_kernel<true, false>, grid, dim3(256), st, p);
 }
 
 hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st, bool has_hulls) {
     if (p.B <= 0 || p.n_groups <= 0 || p.n_kv_blocks <= 0) return hipSuccess;
+    if (live_in_one(p)) return has_hulls ? hipSuccess : launch_bwd_meta(MetaParams{}, st, &p);
     if (!has_hulls) {
         const hipError_t e = launch1(bwd_hull_kernel, dim3(hull_blocks(p)), dim3(256), st, p);
         if (e != hipSuccess) return e;

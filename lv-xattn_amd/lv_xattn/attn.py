@@ -301,7 +301,6 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
         bias, mask = _bias_and_hull(bias, q_, k_)    # as in the forward: the same hull, hence the same pairs
     L_ = L.to(torch.float32).reshape(B * Hq, Lq).contiguous()
 
-    delta = workspace("bwd_delta", (B * Hq, Lq), torch.float32, dev)
     dq, dk, dv = host().backward_outputs(q_, k_, _dq_like_q)
 
     blocks = [(0, Lq)] if batched else [w for w in q_block_bounds(Lq, P) if w[1] > w[0]]
@@ -311,22 +310,17 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
                    torch.uint8, dev)
     if len(windows) == 1:
         r0, r1 = windows[0]
-        ops.bwd_preprocess(o_, do_, delta, r0, r1 - r0)
-        ops.bwd(q_, k_, v_, do_, L_, delta, dq, dk, dv, sm_scale, r0, r1 - r0, mask, accumulate_dkv=False,
-                workspace=ws, bias=bias)
+        ops.bwd(q_, k_, v_, do_, L_, None, dq, dk, dv, sm_scale, r0, r1 - r0, mask, accumulate_dkv=False,
+                workspace=ws, bias=bias, o=o_)
     else:
         def accumulators():
             a = workspace("bwd_dkv_acc", (2, B, Lkv, Hkv, D), torch.float32, dev)
             a.zero_()
             return a
 
-        # delta depends on O and dO alone, and all P blocks of both are here: one launch for
-        # all rows ahead of the rounds (a visit of a real ring would bring its own block's)
-        ops.bwd_preprocess(o_, do_, delta, 0, Lq)
-
         def one_round(r0, r1, acc, ws_r, rounds=1):
-            ops.bwd(q_, k_, v_, do_, L_, delta, dq, acc[0].transpose(1, 2), acc[1].transpose(1, 2), sm_scale,
-                    r0, r1 - r0, mask, accumulate_dkv=True, workspace=ws_r, bias=bias, rounds=rounds)
+            ops.bwd(q_, k_, v_, do_, L_, None, dq, acc[0].transpose(1, 2), acc[1].transpose(1, 2), sm_scale,
+                    r0, r1 - r0, mask, accumulate_dkv=True, workspace=ws_r, bias=bias, rounds=rounds, o=o_)
 
         acc = accumulators()
         n_streams = min(streams, len(windows))

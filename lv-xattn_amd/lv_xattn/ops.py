@@ -222,24 +222,29 @@ def bwd_workspace_bytes(q, k, row_count: int, mask: Optional[Mask] = None) -> in
 
 def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=None,
         mask: Optional[Mask] = None, accumulate_dkv: bool = False,
-        workspace: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None, rounds: int = 1) -> None:
+        workspace: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None, rounds: int = 1,
+        o: Optional[torch.Tensor] = None) -> None:
     """Writes dq (bf16) for the selected rows and writes (bf16) or accumulates
     (fp32) dk, dv at Hkv heads.  `workspace`: uint8 tensor of at least
     bwd_workspace_bytes(q, k, row_count, mask) bytes.  `bias` as in fwd (no gradient
     is formed for it).  `rounds` > 1 (with accumulate_dkv): the rows are that many windows, one after the other, in the
-    workspace of one of ceil(row_count / rounds) rows."""
+    workspace of one of ceil(row_count / rounds) rows.  `o`, with delta None: delta is formed from it on the way (see
+    bwd_preprocess)."""
     flags = (1 if accumulate_dkv else 0) | (rounds << _lib.LVX_BWD_ROUNDS if rounds > 1 else 0)
     if workspace is not None:
         m = mask or _NO_MASK
         if host().bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin,
                       q.shape[2] - row_begin if row_count is None else row_count, m.kv_len, m.kv_start, m.kv_end,
-                      flags, workspace, bias):
+                      flags, workspace, bias, o):
             return
     s = _shape(q, k, scale, mask, bias)
     if row_count is None:
         row_count = q.shape[2] - row_begin
     _check_lse(lse, q)
-    _check_lse(delta, q)
+    if o is None:
+        _check_lse(delta, q)
+    elif delta is not None or o.dtype != q.dtype or o.shape != q.shape:
+        raise LvxError("o must be a tensor of q's type and shape, and delta None")
     if dq.dtype != q.dtype or dq.shape != q.shape:
         raise LvxError("dq must be a tensor of q's type and shape")
     want = torch.float32 if accumulate_dkv else q.dtype
@@ -247,10 +252,13 @@ def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=Non
         raise LvxError(f"dk/dv must be {want} tensors shaped like k")
     if workspace is None:
         workspace = torch.empty(bwd_workspace_bytes(q, k, -(-row_count // rounds), mask), dtype=torch.uint8, device=q.device)
-    rc = load().lvx_bwd(C.byref(s), C.byref(t4(q)), C.byref(t4(k)), C.byref(t4(v)), C.byref(t4(dout)),
-                        lse.data_ptr(), delta.data_ptr(), C.byref(t4(dq)), C.byref(t4(dk)), C.byref(t4(dv)),
-                        flags, row_begin, row_count,
-                        workspace.data_ptr(), workspace.numel() * workspace.element_size(), stream_ptr())
+    end = (C.byref(t4(dq)), C.byref(t4(dk)), C.byref(t4(dv)), flags, row_begin, row_count, workspace.data_ptr(),
+           workspace.numel() * workspace.element_size(), stream_ptr())
+    qkv = (C.byref(s), C.byref(t4(q)), C.byref(t4(k)), C.byref(t4(v)))
+    if o is None:
+        rc = load().lvx_bwd(*qkv, C.byref(t4(dout)), lse.data_ptr(), delta.data_ptr(), *end)
+    else:
+        rc = load().lvx_bwd_from_o(*qkv, C.byref(t4(o)), C.byref(t4(dout)), lse.data_ptr(), *end)
     check(rc, "lvx_bwd")
 
 

@@ -144,6 +144,9 @@ def test_other_entry_points_reject_bad_arguments(lib):
                        C.byref(t), C.byref(t), 0, 0, 64, 0x4000, 1 << 30, None) == -1
     assert lib.lvx_bwd(C.byref(s), C.byref(t), C.byref(t), C.byref(t), C.byref(t), 0x2000, 0x2000, C.byref(t),
                        C.byref(t), C.byref(t), 2, 0, 64, 0x4000, 1 << 30, None) == -3
+    for o, lse, code in ((None, 0x2000, -1), (C.byref(_t(ptr=8)), 0x2000, -2), (C.byref(t), None, -1)):
+        assert lib.lvx_bwd_from_o(C.byref(s), C.byref(t), C.byref(t), C.byref(t), o, C.byref(t), lse, C.byref(t),
+                                  C.byref(t), C.byref(t), 0, 0, 64, 0x4000, 1 << 30, None) == code
     need = lib.lvx_bwd_workspace_bytes(C.byref(s), 64)
     # dS^T tiles + fp32 dK/dV scratch + row metadata records (2 floats per row and head)
     # + fp32 dQ partial tiles (a window this small splits the dQ contraction over the tokens:
