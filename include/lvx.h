@@ -107,12 +107,11 @@ int lvx_max_rounds(void);
  * for each, of ceil(row_count / n) rows.  The results are those of n calls, bit for bit; where that is estimated to be faster
  * a block's 16-bit parts are folded by the launch of the next block, and the workspace holds the parts of two blocks (else of
  * one; lvx_fwd_workspace_bytes says two as well for a shape whose Hkv and Lkv are 0).
- * The kernel has three forms: a wavefront owns 32 text rows of a head (with a dense bias, and at head_dim
- * 16 and 32); 64 rows and its SIMD to itself (head_dim 128 and 64 without a bias); or, where that is
- * estimated to take less, a share of the keys for up to 32 (row, head) pairs of a kv head at once (few rows
- * without a bias, any head_dim: the launch reads K and V once at the speed of HBM).  The environment
- * variable LVX_FWD_WIDE, read at every call, overrides that last choice: 2 the third form where it can run,
- * any other value (0 and 1 alike) never.
+ * The kernel has three forms: a wavefront owns 32 text rows of a head (at head_dim 16 and 32, and with a dense bias);
+ * 64 rows and its SIMD to itself (head_dim 128 and 64); or a share of the keys for up to 32 (row, head) pairs of a kv head at
+ * once (few rows without a bias, any head_dim: the launch reads K and V once at the speed of HBM).  Of those that can run
+ * the one that is estimated to take least does.  The environment variable LVX_FWD_WIDE, read at every call, overrides that
+ * choice: 2 the third form where it can run, any other value (0 and 1 alike) the second.
  * The forms give results within the same tolerance of each other, not the same bits.
  */
 int lvx_fwd(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_tensor* k,

@@ -57,7 +57,8 @@ def _run(cmd, verbose):
 
 
 # hand-scheduled inner loops: (generator, arguments, include file it writes)
-GENERATED = [*[("gen_fwd_loop_wide.py", [t, d], f"lvx_fwd_loop_wide_{t}_{d}.inc") for t in ("bf16", "f16") for d in ("128", "64")],
+GENERATED = [*[("gen_fwd_loop_wide.py", [t, d, *m], f"lvx_fwd_loop_wide_{'_'.join([t, d, *m])}.inc")
+               for t in ("bf16", "f16") for d in ("128", "64") for m in ([], ["bias"])],
              *[("gen_bwd_loop.py", ["p", t, d, m], f"lvx_bwd_loop_p_{t}_{d}_{m}.inc")
                for t in ("bf16", "f16") for d in ("128", "64") for m in ("plain", "masked", "bias")],
              *[("gen_bwd_loop.py", ["d", t, d], f"lvx_bwd_loop_d_{t}_{d}.inc") for t in ("bf16", "f16") for d in ("128", "64")],

@@ -1,7 +1,7 @@
 """Writes the key-tile loop of the forward kernel whose waves own TWO blocks of 32 text rows
 (lvx_fwd.hip, fwd_wide_kernel), for one element type and head dimension:
 
-    python gen_fwd_loop_wide.py bf16|f16 128|64 > lvx_fwd_loop_wide_<type>_<dim>.inc
+    python gen_fwd_loop_wide.py bf16|f16 128|64 [bias] > lvx_fwd_loop_wide_<type>_<dim>[_bias].inc
 
 The statement runs ALL key tiles of a work-group, one or more.  Per key tile t it issues in program
 order the MFMAs of S(t+1) = K(t+1) Q^T and of O += V(t)^T P(t), and between any two of them a few
@@ -15,6 +15,13 @@ What only some tiles need sits behind the loop as out-of-line blocks the stream 
 scalar compare: the move of a row's reference maximum and the rescale of O, the element mask of a
 tile that some row of the work-group does not see in full, and the clamp of the load addresses to
 the last row of the key range when the next tile to be requested is the last.
+
+With a dense bias the scores of tile t+1 become S * c + bias * log2(e) before their row maximum is taken, and c is 1 elsewhere.
+(S * scale + bias would be an instruction less, but where a row sees nothing above -1e9 its exponents, log2(e) * (x - max) by
+one multiply-add, would be as far off as that product's rounding.)  The wave's 64 rows x 64 keys of fp32 come through an LDS tile of its own, 4 rows (1 KiB and 16 bytes of
+padding) to a load: a lane's 16 bytes of a key group are then a read without bank conflicts, and loads cover whole cache lines.
+There is one such tile: it is read while O += V(t)^T P(t), and refilled from there (BIAS_LATE loads) on into the S phase of the
+next tile, in front of that tile's K and V, so that counts of loads in flight tell all of them apart.
 
 Register map (must match the constraints of the asm statement in lvx_fwd.hip), b = row block:
   at entry: v[128 + 2 b : 129 + 2 b] this lane's address in the Q row of block b
@@ -33,6 +40,10 @@ Register map (must match the constraints of the asm statement in lvx_fwd.hip), b
   s66 first key of the tile whose scores are formed   s67, s68 no row masks anything in the tiles
   with (s66 - s67) <= s68, unsigned   s[52:53], s[60:61], s[70:71], s56 scratch
   s[54:55], s[58:59] rows whose reference moved in the tile before
+  bias: v245 scratch   v246 byte offset of this lane's piece of the next load from the tile's first element
+        v[248:251] at entry: read addresses of key groups 0, 16, 32, 48 (a[192:195] inside)
+        v[248:255], v[238:241] three read slots   s[72:75] buffer of the next tile, from its first element to the tensor's last
+        s76 bytes of 4 rows   s77 LDS address of the wave's tile   s78 scale*log2(e)   s80 log2(e)   s79 tiles after the next bias tile
 """
 import os
 import re
@@ -42,6 +53,7 @@ import sys
 OPTS = dict((o.split("=") + ["1"])[:2] for o in os.environ.get("LVX_GEN_OPTS", "").split(",") if o)
 F16 = len(sys.argv) > 1 and sys.argv[1] == "f16"
 DH = int(sys.argv[2]) if len(sys.argv) > 2 else 128
+BIAS = len(sys.argv) > 3 and sys.argv[3] == "bias"
 MFMA = "v_mfma_f32_32x32x16_f16" if F16 else "v_mfma_f32_32x32x16_bf16"
 CVT = "v_cvt_pk_f16_f32" if F16 else "v_cvt_pk_bf16_f32"
 
@@ -59,11 +71,15 @@ MI, LI, AL = [229, 230], [231, 232], [233, 234]
 NMC = [235, 236]
 MX, T0, T1, RS1 = [237, 238], [239, 240], [241, 242], [243, 244]
 AACC, AQ = [0, 64], [128, 160]
+BADDR, BOFF, BREAD, BSLOT = 245, 246, 192, [248, 252, 238]
+BLOCKB = 1040                       # bytes of four rows of bias in LDS
+BIAS_LOADS, BIAS_LATE = 16, int(OPTS.get("blate", 8))       # of a tile; of them, in the tile that reads the one before
 RMASK = ["s[54:55]", "s[58:59]"]
 CMASK = ["s[52:53]", "s[60:61]"]
 NSLOT, AHEAD, WBATCH = 10, int(OPTS.get("ahead", 8)), int(OPTS.get("wbatch", 2))
 # VALU instructions behind an MFMA of the S / V phase: with heads of 64 the same softmax has half as many
-TAKE_S, TAKE_V = (int(OPTS.get("s1", 4)), int(OPTS.get("s2", 5))) if DH == 128 else (int(OPTS.get("s1", 8)), int(OPTS.get("s2", 10)))
+TAKE_S, TAKE_V = (int(OPTS.get("s1", 5 if BIAS else 4)), int(OPTS.get("s2", 7 if BIAS else 5))) if DH == 128 else \
+    (int(OPTS.get("s1", 9 if BIAS else 8)), int(OPTS.get("s2", 14 if BIAS else 10)))
 
 
 def vr(base, n=1):
@@ -83,6 +99,9 @@ class Stream:
         self.ready_after = {}   # operand id -> number of LDS reads issued when its last read was issued
 
     def emit(self, s):
+        if callable(s):
+            s()
+            return
         if isinstance(s, list):     # instructions that must stay together
             for x in s:
                 self.emit(x)
@@ -241,6 +260,44 @@ def advance(left, lo, hi, stride, offs, limit):
             f"LVX_FWDW_STAY{n}_%=:"]
 
 
+def bias_advance():
+    """The source of the next bias tile moves on unless it stands at the last tile."""
+    n = new_label()
+    return [["s_cmp_eq_u32 s79, 0", f"s_cbranch_scc1 LVX_FWDW_BSTAY{n}_%=", "s_add_u32 s72, s72, 256", "s_addc_u32 s73, s73, 0",
+             "s_sub_u32 s74, s74, 256", "s_sub_u32 s79, s79, 1", f"LVX_FWDW_BSTAY{n}_%=:"]]
+
+
+def bias_request(j):
+    """The j-th load of the bias tile that the source stands at: rows 4 j .. 4 j + 3."""
+    out = [f"s_add_i32 m0, s77, {j * BLOCKB}", "s_nop 0", f"buffer_load_dwordx4 v{BOFF}, s[72:75], 0 offen lds"]
+    if j < BIAS_LOADS - 1:
+        return [out + [f"v_add_u32 v{BOFF}, s76, v{BOFF}"]]
+    return [out + [f"s_mul_i32 s56, s76, {BIAS_LOADS - 1}", f"v_subrev_u32 v{BOFF}, s56, v{BOFF}"]]
+
+
+def bias_scores(nxt, st, behind):
+    """The next tile's scores times scale, plus its bias.  behind: loads in flight behind the bias's last."""
+    groups = [(m, b, x) for m in range(4) for b in range(NB) for x in range(2)]      # keys 16 m + 8 x + 4 (lane / 32) ..
+
+    def read(i):
+        m, b, x = groups[i]
+        if b == 0 and x == 0:
+            st.emit(f"v_accvgpr_read_b32 v{BADDR}, a{BREAD + m}")
+        st.lds_read(f"ds_read_b128 {vr(BSLOT[i % 3], 4)}, v{BADDR} offset:{8 * BLOCKB * b + 32 * x}", ("bias", i))
+
+    out = [f"s_waitcnt vmcnt({behind})"] + [lambda i=i: read(i) for i in range(3)]
+    for i, (m, b, x) in enumerate(groups):
+        out.append(lambda i=i: st.wait_op(("bias", i)))
+        for r in range(4):
+            out.append(f"v_mul_f32 v{BSLOT[i % 3] + r}, s80, v{BSLOT[i % 3] + r}")
+        for r in range(4):
+            v = SC[b][nxt] + 16 * (m // 2) + 8 * (m % 2) + 4 * x + r
+            out.append(f"v_fma_f32 v{v}, v{v}, s78, v{BSLOT[i % 3] + r}")
+        if i + 3 < len(groups):
+            out.append(lambda i=i: read(i + 3))
+    return out
+
+
 def request(offs, base, lds, between):
     """This wave's pieces of a tile, into the buffer at byte `lds` of the tile buffers.  A load to LDS needs a wait
     state behind the write of M0: an instruction taken from `between`."""
@@ -261,7 +318,7 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
     tag = f"{par}{int(do_cur)}{int(do_next)}"
     if top:
         # K(t+1) and V(t) have landed; nobody reads K(t) / V(t-1) any more
-        e("s_waitcnt vmcnt(0)")
+        e(f"s_waitcnt vmcnt({BIAS_LATE if BIAS and do_next else 0})")
         e("s_barrier")
         if do_next:
             e("s_add_u32 s66, s66, 64")
@@ -303,9 +360,16 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
             valu.append(f"v_add_f32 v{LI[b]}, v{LI[b]}, v{RS1[b]}")
     if do_next:
         first_max = len(valu)
+        if BIAS:
+            valu += bias_scores(nxt, st, 2 * NLD)
+            valu += bias_advance()
         valu += mask_test(nxt)
-        for b in range(NB):
-            valu += next_max(b, nxt)
+        rest = [x for b in range(NB) for x in next_max(b, nxt)]
+        if BIAS:        # its refill begins among them
+            gap = len(rest) // BIAS_LATE
+            for j in reversed(range(BIAS_LATE)):
+                rest.insert(j * gap, bias_request(j)[0])
+        valu += rest
     for s in valu[:n_pre]:
         e(s)
     pos = n_pre
@@ -316,6 +380,10 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
             dma.append((f"s_add_i32 m0, s50, {par * 2 * TILE + j * 4096}", f"global_load_lds_dwordx4 v{DOK + j}, s[44:45]"))
         for j in range(NLD):
             dma.append((f"s_add_i32 m0, s50, {(par ^ 1) * 2 * TILE + TILE + j * 4096}", f"global_load_lds_dwordx4 v{DOV + j}, s[46:47]"))
+    early = [bias_request(j)[0] for j in range(BIAS_LATE, BIAS_LOADS)] if BIAS and do_dma else []
+    # operands of the S phase behind which a load of K or V goes: every other one, or those the bias has left
+    n_early = NS // 4 if BIAS else 0
+    at_dma = [k for k in range(NS) if k % 2 == 1] if not BIAS else [n_early + i * (NS - n_early) // (2 * NLD) for i in range(2 * NLD)]
     n_mfma = 0
     last_s = -100       # index of the last S MFMA
     for i, k in enumerate(ops):
@@ -336,7 +404,10 @@ def tile(par, do_cur=True, do_next=True, do_dma=True, top=True):
                 e(f"{MFMA} {ar(a, 16)}, {vr(slot, 4)}, {vr(PB[b] + 4 * j, 4)}, {ar(a, 16)}")
             n_mfma += 1
             if b == NB - 1:
-                x, y = dma[k // 2] if dma and k < NS and k % 2 == 1 else (None, None)
+                x, y = dma[at_dma.index(k)] if dma and k in at_dma else (None, None)
+                if k < n_early:
+                    for z in early[k * len(early) // n_early:(k + 1) * len(early) // n_early]:
+                        e(z)
                 if x:
                     e(x)
                 if i + AHEAD < len(ops):        # between the write of M0 and the load: its wait state
@@ -406,7 +477,7 @@ def check(ins):
             kind = "lds"
             wr = regs(toks[0])
             rd = regs(toks[1])
-        elif op.startswith("global_load_lds"):
+        elif op.startswith("global_load_lds") or op.startswith("buffer_load"):
             kind = "vmem"
             rd = regs(toks[0])
             if hist and hist[-1][0] == "m0":
@@ -437,12 +508,16 @@ def main():
     for b in range(NB):
         for kk in range(NKK):
             pro.append(f"global_load_dwordx4 {ar(AQ[b] + 4 * kk, 4)}, {vr(128 + 2 * b, 2)}, off offset:{32 * kk}")
+    if BIAS:
+        pro += [f"v_accvgpr_write_b32 a{BREAD + m}, v{248 + m}" for m in range(4)]
+        for j in range(BIAS_LOADS):
+            pro += bias_request(j)[0]
     pro += request(DOV, "s[46:47]", TILE, zero) + advance("s62", "s46", "s47", "s49", DOV, "s65")
     pro += request(DOK, "s[44:45]", 2 * TILE, zero) + advance("s57", "s44", "s45", "s48", DOK, "s64")
     pro += zero
     for b in range(NB):
         pro += [f"v_mov_b32 v{MI[b]}, s41", f"v_mov_b32 v{LI[b]}, 0", f"v_mov_b32 v{NMC[b]}, 0"]
-    pro += [f"s_waitcnt vmcnt({2 * NLD})", "s_barrier"]
+    pro += [f"s_waitcnt vmcnt({2 * NLD + (BIAS_LOADS if BIAS else 0)})", "s_barrier"]
     # scores of the first tile (from K buffer 0 into score set A: the S phase of an odd tile)
     pro += tile(1, do_cur=False, do_next=True, do_dma=False, top=False)
     # there is nothing to rescale yet

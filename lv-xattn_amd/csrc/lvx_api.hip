@@ -174,8 +174,24 @@ static int fwd_split_len(const lvx_attn_shape* s, FwdForm form, int splits) {
 //          504 launches of 1 to 4096 rows would differ), and per 64-key tile 1.1 us on an idle chip, 1.5 on a full one
 //          (0.9 and 1.05 with heads of 64).  256 rows x 6404 keys: 138 us whole, 39 in 8 parts
 //   plain: the same with 1.8 us per tile and two work-groups per CU
+// with a dense bias and heads of 128 / 64 (launches of 1 .. 2000 rows against 400 .. 13000 keys, ranges of 1 to 64):
+//   wide : 7 us per round and per tile 1.65 us on an idle chip, 2.1 on a full one (6 us, 1.45, 1.55)
+//   plain: 4 us and 2.15, or 2.8 once CUs have two work-groups (3.5 us, 1.95 and 2.35)
 // plus, with splits, 4 us for the launch that folds the parts and their bytes at 4 TB/s, what fp32 adds to them at 9.
-static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32) {
+struct FwdPrice {
+    double tile_us, load_us, round_us;      // per key tile on an idle chip, what a full one adds, per round of work-groups
+    bool shared;                            // it is two work-groups on a CU that add it, however many there are
+};
+constexpr FwdPrice PLAIN_PRICE{0.8, 1.0, 11.0, false};
+static FwdPrice fwd_price(const lvx_attn_shape* s, FwdForm form) {
+    const bool wide = form == FWD_WIDE;
+    if (s->bias && s->D == 128) return wide ? FwdPrice{1.65, 0.45, 7.0, false} : FwdPrice{2.15, 0.65, 4.0, true};
+    if (s->bias && s->D == 64) return wide ? FwdPrice{1.45, 0.1, 6.0, false} : FwdPrice{1.95, 0.4, 3.5, true};
+    if (!wide) return PLAIN_PRICE;
+    return s->D == 128 ? FwdPrice{1.1, 0.4, 11.0, false} : FwdPrice{0.9, 0.15, 11.0, false};
+}
+
+static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32, const FwdPrice& price) {
     const int G = s->Hq / s->Hkv, hg = gcd(G, 4), rs = 4 / hg, n_cu = cu_count();
     const int64_t split_len = fwd_split_len(s, form, splits);
     const int64_t n = (s->Lkv + split_len - 1) / split_len;
@@ -191,9 +207,11 @@ static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int spli
     const int wg_rows = (form == FWD_WIDE ? 64 : 32) * rs;
     const int64_t wgs = (int64_t)s->B * (s->Hq / hg) * ((rows + wg_rows - 1) / wg_rows) * n;
     const int64_t slots = form == FWD_WIDE ? n_cu : 2 * n_cu;
-    const double load = std::min(1.0, (double)wgs / slots);
-    const double tile_us = form == FWD_PLAIN ? 0.8 + load : s->D == 128 ? 1.1 + 0.4 * load : 0.9 + 0.15 * load;
-    return t + (double)((wgs + slots - 1) / slots) * (split_len / FWD_BN * tile_us + 11.0);
+    const double tile_us = price.tile_us + price.load_us * (price.shared ? (wgs > n_cu ? 1.0 : 0.0) : std::min(1.0, (double)wgs / slots));
+    return t + (double)((wgs + slots - 1) / slots) * (split_len / FWD_BN * tile_us + price.round_us);
+}
+static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32) {
+    return fwd_cost(s, rows, form, splits, parts_f32, fwd_price(s, form));
 }
 
 // The form for few rows is for up to 256 (row, head) columns per kv head: it reads K and V from L2 once
@@ -203,17 +221,35 @@ static bool fwd_few_ok(const lvx_attn_shape* s, int rows) {
     return !s->bias && (int64_t)rows * (s->Hq / s->Hkv) <= FEW_MAX_COLS;
 }
 
-// The form of the forward kernel for a window of `rows` rows whose keys are cut into `splits` ranges.
-// Head dimensions 128 and 64 without a dense bias take the wide form or, where reading K and V is the
+// The forms that a shape's launches may have: heads of 128 and 64 take the wide form or, where reading K and V is the
 // larger part of the work, the form for few rows; the plain one was slower at every size measured
-// (4096 rows x 6404 keys: 429 us against 354; 300 rows x 2 samples: 92 against 88) and is not built for them.
+// (4096 rows x 6404 keys: 429 us against 354; 300 rows x 2 samples: 92 against 88) and is not built for them without a dense
+// bias.  With one the wide form wins where there are enough rows for its work-groups of 64 per wave, the plain one where
+// there are few, its work-groups being two to a CU and its way in and out shorter.  us with the best number of ranges, plain / wide:
+// 1024 rows x 16 heads x 4096 keys 61.6 / 53.7 (heads of 64 50.1 / 40.1), 1024 x 32 x 6404 152 / 130, 3 x 2000 x 16 x 2500 213 / 175,
+// 2 x 700 x 32 x 800 of 64 43.9 / 27.2, 256 x 16 x 4096 30.0 / 27.2; 1 x 16 x 4096 14.0 / 18.2, 33 x 16 x 13000 31.9 / 36.6, 300 x 8 x
+// 3000 20.2 / 22.0.  (A row of a bias in bytes is a factor of 24 bits in the wide form.)
+static bool fwd_form_ok(const lvx_attn_shape* s, int rows, FwdForm form) {
+    const bool heads = s->D == 128 || s->D == 64;
+    if (form == FWD_FEW) return fwd_few_ok(s, rows);
+    if (form == FWD_PLAIN) return !heads || s->bias;
+    return heads && (!s->bias || s->bias_stride_r < (1 << 22));
+}
+constexpr FwdForm FWD_FORMS[] = {FWD_PLAIN, FWD_WIDE, FWD_FEW};
+
+// The form of the forward kernel for a window of `rows` rows whose keys are cut into `splits` ranges.
 static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits, bool parts_f32) {
-    if (s->bias) return FWD_PLAIN;
-    const FwdForm many = s->D == 128 || s->D == 64 ? FWD_WIDE : FWD_PLAIN;
-    if (const char* e = getenv("LVX_FWD_WIDE")) {
-        return atoi(e) == 2 && fwd_few_ok(s, rows) ? FWD_FEW : many;
+    const char* const e = getenv("LVX_FWD_WIDE");
+    FwdForm best = FWD_PLAIN;
+    double best_cost = 0.0;
+    for (const FwdForm form : FWD_FORMS) {
+        if (!fwd_form_ok(s, rows, form)) continue;
+        if (e && form == (atoi(e) == 2 ? FWD_FEW : FWD_WIDE)) return form;
+        if (e && form == FWD_FEW) continue;
+        const double c = fwd_cost(s, rows, form, splits, parts_f32);
+        if (best_cost == 0.0 || c < best_cost || (form == FWD_FEW && c == best_cost)) { best = form; best_cost = c; }
     }
-    return fwd_few_ok(s, rows) && fwd_cost(s, rows, FWD_FEW, splits, parts_f32) <= fwd_cost(s, rows, many, splits, parts_f32) ? FWD_FEW : many;
+    return best;
 }
 
 // Whether the parts of a launch whose splits are chosen here wait for the fold in fp32.  In 16 bits they are a
@@ -234,16 +270,25 @@ static bool fwd_parts_f32(const lvx_attn_shape* s, int rows, FwdForm form) {
 
 int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
     if (check_shape(s) != LVX_OK || row_count <= 0) return 1;
-    const FwdForm many = !s->bias && (s->D == 128 || s->D == 64) ? FWD_WIDE : FWD_PLAIN;
+    // The number of ranges for less than best_cost (0: for any), or 0.
+    const auto cheapest = [&](FwdForm form, bool f32, const FwdPrice& price, double& best_cost) {
+        int best = 0;
+        for (int n = 1; n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
+            const double c = fwd_cost(s, row_count, form, n, f32, price);
+            if (best_cost == 0.0 || c < best_cost) { best = n; best_cost = c; }
+        }
+        return best;
+    };
     int best = 1;
     double best_cost = 0.0;
-    for (const FwdForm form : {many, FWD_FEW}) {
-        if (form == FWD_FEW && !fwd_few_ok(s, row_count)) continue;
-        const bool f32 = fwd_parts_f32(s, row_count, form);
-        for (int n = 1; n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
-            const double c = fwd_cost(s, row_count, form, n, f32);
-            if (best_cost == 0.0 || c < best_cost) { best = n > 1 && f32 ? n | LVX_SPLITS_FP32 : n; best_cost = c; }
+    for (const FwdForm form : FWD_FORMS) {
+        if (!fwd_form_ok(s, row_count, form)) continue;
+        bool f32 = fwd_parts_f32(s, row_count, form);
+        if (form == FWD_WIDE && s->bias && !f32) {      // a launch that only this form cuts keeps its precision
+            double plain_cost = 0.0;
+            f32 = cheapest(FWD_PLAIN, false, PLAIN_PRICE, plain_cost) == 1;
         }
+        if (const int n = cheapest(form, f32, fwd_price(s, form), best_cost)) best = n > 1 && f32 ? n | LVX_SPLITS_FP32 : n;
     }
     return best;
 }

@@ -6,8 +6,8 @@
 // ONE q head; the 4 waves of a group cover the q heads that share a kv head
 // (G = 4: four heads x 32 rows; G = 1: one head x 128 rows), so the K/V tile
 // staged in LDS is read by the whole GQA group and nothing is expanded in HBM.
-// (That is fwd_kernel.  Head dimensions 128 and 64 without a dense bias run fwd_wide_kernel, in which a
-// wavefront owns 64 rows, and few rows fwd_few_kernel; see there.)
+// (That is fwd_kernel, which heads of 16 and 32 run and few rows with a dense bias.  Head dimensions 128 and 64 run
+// fwd_wide_kernel, in which a wavefront owns 64 rows, and few rows fwd_few_kernel; see there.)
 //
 // Per 64-key tile and wave (all MFMA are v_mfma_f32_32x32x16_bf16):
 //   S^T[key, row]  = K_tile (A, from LDS)  x  Q^T (B, 32 VGPRs held for the whole kernel)
@@ -459,7 +459,7 @@ __device__ __forceinline__ void fold_before(const FwdFoldParams& p, uint32_t wid
     }
 }
 
-// The wide form (head dimensions 128 and 64, both element types, any mask but a dense bias): a wave
+// The wide form (head dimensions 128 and 64, both element types, any mask): a wave
 // owns two blocks of 32 rows of its head and has its SIMD to itself (one work-group per CU, 512
 // registers per lane), so that every K / V operand read from LDS feeds two MFMAs: half the LDS reads
 // and half the global -> LDS bytes per MFMA of fwd_kernel.  All key tiles of the work-group - whole,
@@ -481,7 +481,11 @@ __device__ __forceinline__ void fold_before(const FwdFoldParams& p, uint32_t wid
 //             in eight different positions each, and of the four rows of a transposing read those of
 //             like parity in different 64-byte halves
 // FOLD: the launch also folds the parts of the one before it (a test at run time costs every launch 0.2 %).
-template <int DH, bool MASKED, bool F16, bool FOLD>
+// BIAS: the bias is added in the loop (see gen_fwd_loop_wide.py); intervals per row are optional then.  1024 rows x 16 heads x 4096
+// keys, with the fold of four ranges 61.6 us in fwd_kernel -> 53.7, heads of 64 50.1 -> 40.1, 1024 x 32 x 6404 152 -> 130.  Without the
+// bias's loads it would be 5 - 6 us less, without K's and V's as well 10; heads dealt to the XCDs side by side, so that they share
+// a bias in L2, and more or fewer of its loads in the S phase change nothing (within 1 %).
+template <int DH, bool MASKED, bool F16, bool FOLD, bool BIAS = false>
 __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const std::conditional_t<FOLD, FwdFoldParams, FwdParams> p) {
     using E = Elt<F16>;
     static_assert(DH == 128 || DH == 64, "head dimension");
@@ -491,7 +495,8 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const std::conditional
     constexpr int EP16 = ROWB + 16, EP32 = 4 * DH + 16;             // row strides of the tile that O leaves through
     constexpr int EPB = 64 * EP16;                                  // its bytes per wave (32 rows of floats fit too)
     static_assert(32 * EP32 <= EPB);
-    __shared__ __attribute__((aligned(1024))) char kv_lds[4 * EPB]; // 4 TB: [buffer][K, V]; then O
+    constexpr int BIAS_BLOCK = 4 * 256 + 16, BIAS_TILE = 16 * BIAS_BLOCK;   // four rows of 64 floats, padded; 64 rows: a wave's tile
+    __shared__ __attribute__((aligned(1024))) char kv_lds[4 * EPB + (BIAS ? 4 * BIAS_TILE : 0)];    // 4 TB: [buffer][K, V]; then O
     __shared__ int red[4][4];
 
     fetch_kernargs<sizeof(p)>();
@@ -526,7 +531,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const std::conditional
     int my_s[2] = {kv_lo, kv_lo}, my_e[2] = {kv_hi, kv_hi};
     bool empty[2] = {kv_hi <= kv_lo, kv_hi <= kv_lo};
     int lo = kv_lo, hi = kv_hi, in_lo = kv_lo, in_hi = kv_hi;
-    if (MASKED) {
+    if (MASKED && (!BIAS || p.kv_start)) {
         lo = BIG; hi = 0; in_lo = 0; in_hi = BIG;
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
@@ -627,7 +632,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const std::conditional
         const uint32_t inner_n = inner_any ? (uint32_t)(in_hi - BN - in_lo) : 0u;
         uint32_t left = uniform32((uint32_t)(n - 1)), left_k = left, left_v = left, kv = uniform32((uint32_t)kv0);
 #define LVX_FWD_WIDE_SCALARS                                                                                       \
-    "{s40}"(uniform32(p.scale_log2e)), "{s41}"(-INFINITY), "{s42}"(RESCALE_LOG2), "{s48}"(uniform32((uint32_t)BN * krow_b)), \
+    "{s40}"(uniform32(BIAS ? 1.f : p.scale_log2e)), "{s41}"(-INFINITY), "{s42}"(RESCALE_LOG2), "{s48}"(uniform32((uint32_t)BN * krow_b)), \
         "{s49}"(uniform32((uint32_t)BN * vrow_b)), "{s50}"(uniform32(lds_w)), "{s64}"(uniform32((uint32_t)last * krow_b)),   \
         "{s65}"(uniform32((uint32_t)last * vrow_b)), "{s67}"(uniform32(inner)), "{s68}"(uniform32(inner_n)),               \
         "{v224}"(ld_c), "{v225}"(me0), "{v226}"(me1), "{v227}"(ml0), "{v228}"(ml1)
@@ -649,7 +654,54 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const std::conditional
 #define LVX_FWD_WIDE_IN_64                                                                                         \
           "{v200}"(ka[0]), "{v201}"(ka[1]), "{v202}"(ka[2]), "{v203}"(ka[3]),                                      \
           "{v208}"(va[0]), "{v209}"(va[1]), "{v210}"(va[2]), "{v211}"(va[3]), LVX_FWD_WIDE_SCALARS
-        if constexpr (DH == 128 && !F16) {
+        if constexpr (BIAS) {
+            // this wave's rows of the bias, from the first tile on.  Loads past the tensor's end give zeros; what they read of rows
+            // past the window or of keys past the range is never used.
+            const int row = min(row0, p.Lq - 1);
+            const float* const base = p.bias + b * p.bias_b + h * p.bias_h + (int64_t)row * p.bias_r + kv0;
+            const int64_t bytes = 4 * ((p.Lq - 1 - row) * p.bias_r + (p.Lkv + 3) / 4 * 4 - kv0);
+            const uint32_t brow_b = (uint32_t)p.bias_r * 4u;
+            const uint64_t at = (uint64_t)(uintptr_t)uniform_ptr(reinterpret_cast<const char*>(base));
+            u32x4 srd = {(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, uniform32((uint32_t)min(bytes, (int64_t)0x7fffffff)), 0x00020000u};
+            uint32_t off = (uint32_t)(lane >> 4) * brow_b + (uint32_t)((lane & 15) ^ ((lane >> 4) << 2)) * 16u, left_b = left;
+            const uint32_t lds_b = lds0 + 4 * EPB + (uint32_t)wave * BIAS_TILE;
+            // chunk 4 m + g (+ 2: the read's offset) of row l32: of block l32 / 4, where its bits 2 and 3 have l32 % 4 XORed in
+            u32x4 rd;
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                rd[m] = lds_b + (uint32_t)(l32 >> 2) * BIAS_BLOCK + (uint32_t)(l32 & 3) * 256u + (uint32_t)(((4 * m) ^ ((l32 & 3) << 2)) + g) * 16u;
+#define LVX_FWD_WIDE_OUT_BIAS "+{v246}"(off), "+{v[248:251]}"(rd), "+{s[72:75]}"(srd), "+{s79}"(left_b)
+#define LVX_FWD_WIDE_IN_BIAS "{s76}"(uniform32(4u * brow_b)), "{s77}"(uniform32(lds_b)), "{s78}"(uniform32(p.scale_log2e)), "{s80}"(LOG2E_F)
+#define LVX_FWD_WIDE_CLOBBERS_BIAS LVX_FWD_WIDE_CLOBBERS_S, "v245", "v252", "v253", "v254", "v255", "a192", "a193", "a194", "a195"
+            if constexpr (DH == 128 && !F16) {
+                asm volatile(
+#include "lvx_fwd_loop_wide_bf16_128_bias.inc"
+                    : LVX_FWD_WIDE_OUT_128, LVX_FWD_WIDE_OUT_BIAS : LVX_FWD_WIDE_IN_128, LVX_FWD_WIDE_IN_BIAS
+                    : LVX_FWD_WIDE_CLOBBERS_BIAS, LVX_FWD_WIDE_CLOBBERS_128);
+            } else if constexpr (DH == 128) {
+                asm volatile(
+#include "lvx_fwd_loop_wide_f16_128_bias.inc"
+                    : LVX_FWD_WIDE_OUT_128, LVX_FWD_WIDE_OUT_BIAS : LVX_FWD_WIDE_IN_128, LVX_FWD_WIDE_IN_BIAS
+                    : LVX_FWD_WIDE_CLOBBERS_BIAS, LVX_FWD_WIDE_CLOBBERS_128);
+            } else if constexpr (!F16) {
+                asm volatile(
+#include "lvx_fwd_loop_wide_bf16_64_bias.inc"
+                    : LVX_FWD_WIDE_OUT_64, LVX_FWD_WIDE_OUT_BIAS : LVX_FWD_WIDE_IN_64, LVX_FWD_WIDE_IN_BIAS
+                    : LVX_FWD_WIDE_CLOBBERS_BIAS, LVX_FWD_WIDE_CLOBBERS_64);
+            } else {
+                asm volatile(
+#include "lvx_fwd_loop_wide_f16_64_bias.inc"
+                    : LVX_FWD_WIDE_OUT_64, LVX_FWD_WIDE_OUT_BIAS : LVX_FWD_WIDE_IN_64, LVX_FWD_WIDE_IN_BIAS
+                    : LVX_FWD_WIDE_CLOBBERS_BIAS, LVX_FWD_WIDE_CLOBBERS_64);
+            }
+            // what a row that sees nothing adds its bias to is not zero times a finite value
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[blk][dt][v] = empty[blk] ? 0.f : acc[blk][dt][v];
+        } else if constexpr (DH == 128 && !F16) {
             asm volatile(
 #include "lvx_fwd_loop_wide_bf16_128.inc"
                 : LVX_FWD_WIDE_OUT_128 : LVX_FWD_WIDE_IN_128 : LVX_FWD_WIDE_CLOBBERS_S, LVX_FWD_WIDE_CLOBBERS_128);
@@ -755,7 +807,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const std::conditional
     for (int blk = 0; blk < 2; ++blk) {
         const int r = 32 * blk + l32;
         if (g == 0 && r < rows) {
-            const float lse = l_tot[blk] > 0.f ? m_i[blk] * p.scale + __logf(l_tot[blk]) : no_lse(p, l_tot[blk]);
+            const float lse = l_tot[blk] > 0.f ? m_i[blk] * (BIAS ? LN2_F : p.scale) + __logf(l_tot[blk]) : no_lse(p, l_tot[blk]);
             p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + h) * p.lse_bh_stride + row0 + r] = lse;
         }
     }
@@ -1180,6 +1232,7 @@ hipError_t launch_fwd_t(const FwdParams& p, bool masked, hipStream_t st, const F
     }
     if constexpr (DH >= 64) {
         if (p.form == FWD_WIDE) {
+            if (p.bias) return launch1((fwd_wide_kernel<DH, true, F16, false, true>), dim3(grid), dim3(256), st, p);
             if (fold) {
                 const FwdFoldParams both{p, *fold};
                 if (masked) return launch1((fwd_wide_kernel<DH, true, F16, true>), dim3(grid), dim3(256), st, both);

@@ -22,7 +22,7 @@ struct Strides3 {
     int64_t b, h, s;
 };
 
-// Which forward kernel: a wave owns 32 rows of a head (any head dimension, dense bias), 64 rows and its
+// Which forward kernel: a wave owns 32 rows of a head (heads of 16 and 32, dense bias), 64 rows and its
 // SIMD (head dimensions 128 and 64), or a share of the keys for up to 32 (row, head) pairs at once.
 enum FwdForm { FWD_PLAIN = 0, FWD_WIDE = 1, FWD_FEW = 2 };
 

@@ -127,3 +127,45 @@ def test_backward_loop_with_a_bias_reads_it_behind_the_wait_of_its_loads(out):
         assert old in lines
         with pytest.raises(AssertionError):
             walk([new if l == old else l for l in lines])
+
+
+@pytest.mark.parametrize("out", [g[2] for g in _generated() if g[0] == "gen_fwd_loop_wide.py" and "bias" in g[1]])
+def test_forward_loop_with_a_bias_reads_it_behind_the_wait_of_its_loads(out):
+    """As above: all 16 loads of a tile are waited for by count before the first read of it, a refill follows a wait for the last read,
+    and in front of a tile's barrier the count covers every load of K and V."""
+    text = [l[1:-3] for l in open(os.path.join(CSRC, out)).read().splitlines()[1:]]
+    top, end = text.index("LVX_FWDW_LOOP_%=:"), text.index("s_branch LVX_FWDW_LOOP_%=")
+    lines = text[:top] + 3 * text[top + 1:end]
+
+    def walk(lines):
+        issued = lds = waited = read_until = last_read = 0
+        bias, tiles, seen = [], [], []
+        for line in lines:
+            op, _, rest = line.partition(" ")
+            if op.startswith("global_load") or op.startswith("buffer_load"):
+                issued += 1
+                if op.startswith("buffer"):
+                    assert last_read <= read_until, line
+                    bias.append(issued)
+                elif "lds" in op:
+                    tiles.append(issued)
+            elif op == "s_waitcnt" and "vmcnt" in rest:
+                waited = max(waited, issued - int(re.search(r"vmcnt\((\d+)\)", rest).group(1)))
+            elif op == "s_waitcnt":
+                read_until = max(read_until, lds - int(re.search(r"lgkmcnt\((\d+)\)", rest).group(1)))
+            elif op == "s_barrier" and seen:
+                assert tiles[-1] <= waited
+            elif op.startswith("ds_"):
+                lds += 1
+                if re.search(r", v245\b", rest):
+                    assert all(n <= waited for n in bias), (line, bias[-4:], waited)
+                    seen.append(len(bias))
+                    last_read = lds
+        return seen
+    seen = walk(lines)
+    assert seen == [16 * (1 + k // 16) for k in range(7 * 16)]       # the prologue's tile and two a trip
+    kv = 8 if "_128" in out else 4
+    for old, new in ((f"s_waitcnt vmcnt({kv})", f"s_waitcnt vmcnt({kv + 1})"), ("s_waitcnt lgkmcnt(0)", "s_waitcnt lgkmcnt(1)")):
+        assert old in lines
+        with pytest.raises(AssertionError):
+            walk([new if l == old else l for l in lines])
