@@ -926,6 +926,26 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     const int blocks = s->B * s->Hkv * p.n_kv_blocks;
     const int steps = p.G * (int)(rows / 32);
     const BwdCut cut = choose_bwd_cut(blocks, steps, s->kv_start != nullptr);
+    // With intervals per row how long a block is shows on the device, which then plans the launch, in the fp32 scratch.  (A bias
+    // seldom hides anything, and the plan would be 3 us for nothing.)
+    PlanParams plan{};
+    const int cus = cu_count() / 8;
+    if (s->kv_start && !s->bias && !meta && !dkv_accumulate && cus > 0 && cus <= 64 && cut.blocks_per_xcd >= 2 * cus &&
+        cut.blocks_per_xcd <= MAX_PLANNED_BLOCKS && !cut.any_split() && steps >= 2 * MIN_PLANNED_RANGE &&
+        (int64_t)s->B * n_groups * LIVE_GROUP <= MAX_LIVE_TILES) {
+        plan.cus = plan.shared_max = cus;
+        plan.slots = cut.blocks_per_xcd + cus;
+        plan.n_blocks = blocks; plan.blocks_per_xcd = cut.blocks_per_xcd; plan.G = p.G;
+        plan.entries = reinterpret_cast<uint32_t*>(wsb + wsl.dkv);
+        plan.shared = plan.entries + 8 * plan.slots * PLAN_ENTRY;
+        const size_t tables = ((size_t)(8 * plan.slots * PLAN_ENTRY + 8 * plan.shared_max * SHARED_ENTRY) * sizeof(uint32_t) + 255) / 256 * 256;
+        const size_t room = wsl.meta - wsl.dkv, slice = (size_t)2 * 128 * s->D * sizeof(float);
+        p.slices = reinterpret_cast<float*>(wsb + wsl.dkv + tables);
+        plan.slices = room > tables ? (int)std::min<size_t>((room - tables) / slice / 8, 2 * cus) : 0;
+        if (plan.slices < 2) plan.entries = nullptr;
+        p.plan = plan.entries;
+        p.plan_slots = plan.slots;
+    }
     p.n_blocks = blocks;
     p.blocks_per_xcd = cut.blocks_per_xcd;
     p.whole_blocks = cut.whole;
@@ -949,7 +969,7 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
         if (!dq_by.few && dq_by.splits <= 1 && s->B * n_groups <= MAX_RANKED_GROUPS) order = reinterpret_cast<int32_t*>(wsb + wsl.order);
         lp = LiveParams{s->kv_len, s->kv_start, s->kv_end, hull, reinterpret_cast<int32_t*>(wsb + wsl.runs), order,
                         s->B, s->Lq, s->Lkv, row_begin,
-                        row_begin + row_count, n_tiles, n_groups, p.n_kv_blocks};
+                        row_begin + row_count, n_tiles, n_groups, p.n_kv_blocks, plan};
         p.live_runs = lp.live_runs;
     }
     const bool has_hulls = !meta;       // its records come by a launch of its own, which writes the tables as well, or their hulls
@@ -987,6 +1007,13 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     if (scratch) {
         CastSharedParams cp{sb, scratch, static_cast<uint16_t*>(dk->ptr), static_cast<uint16_t*>(dv->ptr), st3(dk), st3(dv), p.f16};
         e = launch_cast_shared(cp, st);
+        if (e != hipSuccess) return static_cast<int>(e);
+    }
+
+    if (plan.entries) {
+        const CastSlicesParams cp{plan.shared, p.slices, plan.shared_max, s->B, s->Lkv, s->D, p.n_kv_blocks, p.f16, static_cast<uint16_t*>(dk->ptr),
+                                  static_cast<uint16_t*>(dv->ptr), st3(dk), st3(dv)};
+        e = launch_cast_slices(cp, st);
         if (e != hipSuccess) return static_cast<int>(e);
     }
 

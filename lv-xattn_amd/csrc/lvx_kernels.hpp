@@ -208,11 +208,35 @@ struct BwdParams {
     // its tokens) as up to 4 runs of consecutive tiles, live_runs[(b * n_kv_blocks + block) * 8
     // + 2 i + {0, 1}] = first tile and number of tiles of run i (0 tiles: unused).  Null: every tile.
     const int32_t* live_runs;
+    // Not null: which block and range a work-group takes, in place of whole_blocks and the rest (see PlanParams)
+    const uint32_t* plan;
+    int plan_slots;
+    float* slices;
     int f16;                   // element type of q, k, v, dout, the dS^T workspace and (mode 0) dk, dv
     Divisor by_splits, by_splits2, by_kv_blocks, by_B;     // filled in by launch_bwd
     // and the work-groups that are the token blocks' (a multiple of 8): any past them sum the slices of dQ of the window before
     int own_wg;
     CastParams dq_before;
+};
+
+// How the token blocks of a launch with an interval mask are handed to work-groups, where there are at least two of them to a CU.  Their
+// lengths are known on the device only, where one work-group per XCD sorts the XCD's blocks: the longest, as many
+// as fill whole rounds of its CUs, get a work-group each, the others are cut into ranges of steps, and those nobody sees come last.  A range
+// leaves fp32 sums in a slice of its own, [dK, dV][128 tokens][D], and cast_slices_kernel adds and rounds them.
+// 2 x 3000 rows that see the image before them (77 blocks of 180 to 368 steps on 32 CUs: 602 steps until the last CU ends, 512 with 13
+// cut in two, by a count of steps): bwd_kernel 657 -> 615 us, what the launches before and after it take 18 -> 35, forward and
+// backward 1054 -> 1021.  (More CUs at work run at a lower clock.  Whole blocks chosen by simulating which CU is free when, to 512
+// steps instead of 552, gave the same kernel and took 20 us longer to plan.)  Others of 500 blocks and more 0 to -6 %.
+// Entry l of XCD x: the block's number in the XCD's list | ranges << 16 | range << 24, and the slice of the block's first range; ~0: none.
+constexpr int MAX_PLANNED_BLOCKS = 256;         // of an XCD; with more rounds than eight there is little left to even out
+constexpr int MIN_PLANNED_RANGE = 24;           // steps: shorter ranges are all ramp
+constexpr int PLAN_ENTRY = 2, SHARED_ENTRY = 4;     // words; of a shared block: its number, ranges (0: no such block), slice, unused
+struct PlanParams {
+    uint32_t* entries;         // out: [8][slots][PLAN_ENTRY]; null: no plan
+    uint32_t* shared;          // out: [8][shared_max][SHARED_ENTRY]
+    int slots, cus;            // entries and CUs of an XCD
+    int shared_max, slices;    // most blocks of an XCD that are cut, most slices (slices x * slices + ..)
+    int n_blocks, blocks_per_xcd, G;
 };
 
 // Which (token block, 32-row tile) pairs an interval mask leaves alive: a tile is alive for the blocks of its hull, the
@@ -232,6 +256,8 @@ struct LiveParams {
     int32_t* order;            // out (may be null): the B * n_groups group indices b * n_groups + grp,
                                // longest hull first (ties in index order)
     int B, Lq, Lkv, row_begin, row_end, n_tiles, n_groups, n_kv_blocks;
+    PlanParams plan;           // only where live_in_one
+    Divisor by_tiles;          // filled in by launch_bwd_meta, by n_tiles
 };
 // Whether one launch writes all three, its work-groups taking the hulls they need themselves instead of waiting for a launch of them:
 // each reads all intervals of a sample, and one those of all samples, 256 rows in a wave's 0.5 us.
@@ -282,6 +308,17 @@ struct CastSharedParams {
     Strides3 dks, dvs;
     int f16;
 };
+
+// The sums of the blocks that a plan has cut, rounded into dK and dV.
+struct CastSlicesParams {
+    const uint32_t* shared;
+    const float* slices;
+    int shared_max, B, Lkv, D, n_kv_blocks, f16;
+    uint16_t* dk;
+    uint16_t* dv;
+    Strides3 dks, dvs;
+};
+hipError_t launch_cast_slices(const CastSlicesParams& p, hipStream_t st);
 
 // dQ = (scale dS) K of a window of `rows` rows, from the dS^T workspace.
 struct DqParams {

@@ -321,11 +321,101 @@ __device__ __forceinline__ void rank_group(const LiveParams& p, const int* len, 
 // work-group, which takes the hulls of the sample's tiles itself (a few loads per thread, all in flight, at most MAX_LIVE_TILES
 // tiles in all samples); the sample's first writes them down as well, and one more work-group takes the hulls of the groups
 // and ranks them.
-__host__ __device__ __forceinline__ int live_blocks(const LiveParams& p) { return (p.n_kv_blocks + 3) / 4 * p.B + (p.order ? 1 : 0); }
+__host__ __device__ __forceinline__ int live_blocks(const LiveParams& p) {
+    return (p.plan.entries ? 8 : 0) + (p.n_kv_blocks + 3) / 4 * p.B + (p.order ? 1 : 0);
+}
+
+// The hulls of the tiles of samples [b0, b0 + nb) into LDS, by the whole work-group, 2 AHEAD loads per thread in flight.
+template <int AHEAD>
+__device__ __forceinline__ void hulls_to_lds(const LiveParams& p, int b0, int nb, int32_t* hull) {
+    const int n = nb * p.n_tiles;
+    for (int t0 = 0; t0 < n; t0 += 8 * AHEAD) {
+        int lo[AHEAD], hi[AHEAD];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) {
+            uint32_t tile;
+            const int b = b0 + (int)p.by_tiles.split((uint32_t)min(t0 + 8 * k + (int)(threadIdx.x >> 5), n - 1), tile);
+            row_interval(p, b, len_of(p, b), p.row_begin + (int)tile * 32 + (int)(threadIdx.x & 31), lo[k], hi[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) {
+            const int t = t0 + 8 * k + (int)(threadIdx.x >> 5);
+            hull_of_32(lo[k], hi[k]);
+            if ((threadIdx.x & 31) == 0 && t < n) { hull[2 * t] = lo[k]; hull[2 * t + 1] = hi[k]; }
+        }
+    }
+}
+
+// See PlanParams; one work-group, for XCD x.  hull: of the tiles of all samples.  The longest blocks, as many as make whole rounds of the XCD's CUs, stay whole.  The ranges of
+// the others are priced as choose_bwd_cut does, in steps (about a microsecond): six for what a work-group spends outside them, and for
+// writing the slices and adding them up 8 and 0.3 per slice.
+__device__ __forceinline__ void plan_xcd(const LiveParams& p, int x, const int32_t* hull) {
+    __shared__ __attribute__((aligned(16))) int key[MAX_PLANNED_BLOCKS];
+    __shared__ int sorted[MAX_PLANNED_BLOCKS];          // steps << 8 | block
+    const PlanParams& q = p.plan;
+    const int tid = threadIdx.x;
+    const int blk0 = x * q.blocks_per_xcd, n = max(0, min(q.blocks_per_xcd, q.n_blocks - blk0));
+    static_assert(MAX_PLANNED_BLOCKS == 256, "a thread to a block, eight bits of a key");
+    key[tid] = -1;
+    __syncthreads();
+    const int sh = n <= 64 ? 2 : n <= 128 ? 1 : 0, j = tid >> sh;       // threads to a block
+    int tiles = 0;
+    if (j < n) {
+        const int id = blk0 + j, kvb = id % p.n_kv_blocks * 128, b = id / p.n_kv_blocks % p.B;
+        const int32_t* const h = hull + 2 * b * p.n_tiles;
+#pragma unroll 4
+        for (int t = tid & ((1 << sh) - 1); t < p.n_tiles; t += 1 << sh) tiles += h[2 * t] <= kvb && kvb < h[2 * t + 1] ? 1 : 0;
+    }
+    for (int o = 1; o < 1 << sh; o <<= 1) tiles += __shfl_xor(tiles, o);
+    if (j < n) key[j] = tiles * q.G << 8 | j;
+    __syncthreads();
+    const int mine = key[tid];
+    int rank = 0;
+#pragma unroll 2
+    for (int k = 0; k < (n + 3) / 4; ++k) {
+        const u32x4 other = reinterpret_cast<const u32x4*>(key)[k];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rank += (int)other[e] > mine ? 1 : 0;
+    }
+    if (tid < n) sorted[rank] = mine;
+    const int n_live = __syncthreads_count(mine > 255);     // of one step and more
+    const int whole = n_live / q.cus * q.cus, rest = n_live - whole;
+    const float longest = rest ? (float)(sorted[whole] >> 8) : 0.f;
+    int S = 1;
+    float best = longest + 6.f;
+    for (int s = 2; s <= 8 && longest >= (float)(MIN_PLANNED_RANGE * s) && rest * (s - 1) <= q.slots - q.blocks_per_xcd && rest * s <= q.slices; ++s) {
+        const float cost = (float)((rest * s + q.cus - 1) / q.cus) * (longest / (float)s + 6.f) + 8.f + 0.3f * (float)(rest * s);
+        if (cost < best) { best = cost; S = s; }
+    }
+    const int ranges = S > 1 ? rest * S : 0, first_dead = n_live + (ranges ? ranges - rest : 0);
+    uint32_t* const out = q.entries + (int64_t)x * q.slots * PLAN_ENTRY;
+    for (int l = tid; l < q.slots; l += 256) {
+        uint32_t e = ~0u, slice = 0;
+        const int r = l - whole;
+        if (r >= 0 && r < ranges) {
+            e = (uint32_t)(sorted[whole + r / S] & 255) | (uint32_t)S << 16 | (uint32_t)(r % S) << 24;
+            slice = (uint32_t)(x * q.slices + r - r % S);
+        } else {
+            const int at = l < first_dead ? l : l - first_dead + n_live;
+            if (at < n) e = (uint32_t)(sorted[at] & 255) | 1u << 16;
+        }
+        out[l * PLAN_ENTRY] = e;
+        out[l * PLAN_ENTRY + 1] = slice;
+    }
+    for (int j = tid; j < q.shared_max; j += 256) {
+        uint32_t* const e = q.shared + (int64_t)(x * q.shared_max + j) * SHARED_ENTRY;
+        const bool cut = ranges && j < rest;
+        e[0] = cut ? (uint32_t)(blk0 + (sorted[whole + j] & 255)) : 0u;
+        e[1] = cut ? (uint32_t)S : 0u;
+        e[2] = (uint32_t)(x * q.slices + j * S);
+    }
+}
+
 __device__ __forceinline__ void live_tables(const LiveParams& p, int i) {
     __shared__ int32_t hull[MAX_LIVE_TILES * 2];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, per = (p.n_kv_blocks + 3) / 4, b = i / per;
-    constexpr int AHEAD = 4;
+    // the plans first, they take longest
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, per = (p.n_kv_blocks + 3) / 4, plans = p.plan.entries ? 8 : 0;
+    const int b = i < plans ? 0 : (i - plans) / per;
     if (b >= p.B) {
         const int n = p.B * p.n_groups;
         int* const len = hull;
@@ -344,19 +434,14 @@ __device__ __forceinline__ void live_tables(const LiveParams& p, int i) {
         if ((int)threadIdx.x < n) rank_group(p, len, threadIdx.x, n);
         return;
     }
-    const int kv_len = len_of(p, b);
-    for (int t0 = 0; t0 < p.n_tiles; t0 += 8 * AHEAD) {
-        int lo[AHEAD], hi[AHEAD];
-#pragma unroll
-        for (int k = 0; k < AHEAD; ++k) row_interval(p, b, kv_len, p.row_begin + (t0 + 8 * k) * 32 + (int)threadIdx.x, lo[k], hi[k]);
-#pragma unroll
-        for (int k = 0; k < AHEAD; ++k) {
-            const int tile = t0 + 8 * k + (threadIdx.x >> 5);
-            hull_of_32(lo[k], hi[k]);
-            if ((threadIdx.x & 31) == 0 && tile < p.n_tiles) { hull[2 * tile] = lo[k]; hull[2 * tile + 1] = hi[k]; }
-        }
-    }
+    // (one copy of it: what a launch as short as this waits for is its instructions on their way from memory)
+    hulls_to_lds<8>(p, b, i < plans ? p.B : 1, hull);
     __syncthreads();
+    if (i < plans) {
+        plan_xcd(p, i, hull);
+        return;
+    }
+    i -= plans;
     const int kblk = (i - b * per) * 4 + wave;
     if (kblk < p.n_kv_blocks) live_runs(p, hull, b, kblk);
     if (i != b * per) return;
@@ -671,7 +756,36 @@ __global__ __launch_bounds__(256) void cast_shared_kernel(const CastSharedParams
     }
 }
 
-// Same from a transposed source (cast_t).
+// The blocks that a plan has cut, SHARE_PARTS work-groups each: their slices added in the order of their ranges and rounded.
+template <bool F16>
+__global__ __launch_bounds__(256) void cast_slices_kernel(const CastSlicesParams p) {
+    using E = Elt<F16>;
+    const uint32_t* const e = p.shared + (int64_t)(blockIdx.x / SHARE_PARTS) * SHARED_ENTRY;
+    const int blk = (int)e[0], S = (int)e[1];
+    if (S == 0) return;
+    const int kblk = blk % p.n_kv_blocks, bh = blk / p.n_kv_blocks, b = bh % p.B, hk = bh / p.B;
+    const int sh = chunk_shift(p.D);
+    const int64_t half = (int64_t)128 * p.D;
+    const float* const src = p.slices + (int64_t)e[2] * 2 * half;
+    for (int i = threadIdx.x; i < (SHARE_ROWS << sh); i += 256) {
+        const int r = (int)(blockIdx.x % SHARE_PARTS) * SHARE_ROWS + (i >> sh), token = kblk * 128 + r, chunk = i & ((1 << sh) - 1);
+        if (token >= p.Lkv) return;
+        const float* s = src + (int64_t)r * p.D + chunk * 8;
+        f32x4 x[4] = {};
+        for (int k = 0; k < S; ++k, s += 2 * half) {
+            x[0] += *reinterpret_cast<const f32x4*>(s);
+            x[1] += *reinterpret_cast<const f32x4*>(s + 4);
+            x[2] += *reinterpret_cast<const f32x4*>(s + half);
+            x[3] += *reinterpret_cast<const f32x4*>(s + half + 4);
+        }
+        const u32x4 ku = {E::pack(x[0][0], x[0][1]), E::pack(x[0][2], x[0][3]), E::pack(x[1][0], x[1][1]), E::pack(x[1][2], x[1][3])};
+        const u32x4 vu = {E::pack(x[2][0], x[2][1]), E::pack(x[2][2], x[2][3]), E::pack(x[3][0], x[3][1]), E::pack(x[3][2], x[3][3])};
+        *reinterpret_cast<u32x4*>(p.dk + b * p.dks.b + hk * p.dks.h + (int64_t)token * p.dks.s + chunk * 8) = ku;
+        *reinterpret_cast<u32x4*>(p.dv + b * p.dvs.b + hk * p.dvs.h + (int64_t)token * p.dvs.s + chunk * 8) = vu;
+    }
+}
+
+// cast_kernel from a transposed source (cast_t).
 template <bool F16>
 __global__ __launch_bounds__(256) void cast_t_kernel(const CastParams p) {
     fetch_kernargs<sizeof(CastParams)>();
@@ -797,6 +911,7 @@ hipError_t launch_bwd_meta(const MetaParams& p0, hipStream_t st, const LiveParam
     MetaParams p = p0;
     if (live && live->n_tiles > 0 && live->B > 0) {
         p.live = *live;
+        p.live.by_tiles = divisor(live->n_tiles);
         p.tables = live_in_one(*live);
         p.table_blocks = p.tables ? live_blocks(*live) : hull_blocks(*live);
     }
@@ -868,6 +983,12 @@ hipError_t launch_cast_shared(const CastSharedParams& p, hipStream_t st) {
     if (grid.x == 0) return hipSuccess;
     if (p.f16) return launch1(cast_shared_kernel<true>, grid, dim3(256), st, p);
     return launch1(cast_shared_kernel<false>, grid, dim3(256), st, p);
+}
+
+hipError_t launch_cast_slices(const CastSlicesParams& p, hipStream_t st) {
+    const dim3 grid(8 * p.shared_max * SHARE_PARTS);
+    if (p.f16) return launch1(cast_slices_kernel<true>, grid, dim3(256), st, p);
+    return launch1(cast_slices_kernel<false>, grid, dim3(256), st, p);
 }
 
 // For cast_t by work-groups of so many threads.
