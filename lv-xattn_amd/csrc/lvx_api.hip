@@ -661,30 +661,35 @@ int lvx_bwd_preprocess(const lvx_attn_shape* s, const lvx_tensor* o, const lvx_t
 
 // Work-groups of the backward are long (every step of a token block) and one
 // fits a CU, so a grid that is not a multiple of the CU count wastes up to one
-// whole round.  Splitting the steps of every token block over `S` work-groups
-// (which then add their dK/dV with atomics into an fp32 scratch that is zeroed before
-// and rounded after) evens that out.  S minimises
-//     rounds(S) * (steps / S + WG_COST) + (S > 1 ? SPLIT_COST : 0)        [in steps]
+// whole round.  Splitting the steps of every token block over `S` work-groups evens that out.  Each leaves its fp32 sums in a slice of
+// the workspace, and a launch adds a block's slices in order and rounds them; where the slices have no room, or the call accumulates,
+// they are added with atomics into an fp32 scratch that is zeroed before and rounded after (or the caller's accumulator).  S minimises
+//     rounds(S) * (steps / S + WG_COST) + (S > 1 ? split_cost : 0)        [in steps]
 // with ranges of at least 32 steps; WG_COST is what a work-group spends outside its
-// steps (operand load, ring fill, epilogue: about 8 us = 6 steps), SPLIT_COST what sharing blocks
-// adds to the launch.  55 steps, about 70 us, were measured where every block is shared and the
-// whole scratch zeroed and rounded; only the shared blocks are by now, and nothing is in a call that
-// accumulates, so for a few shared blocks it is an upper bound, which errs on the side of not
-// cutting.  rounds(S) = ceil(blocks * S / CUs)
+// steps (operand load, ring fill, epilogue: about 8 us = 6 steps), split_cost what sharing blocks
+// adds to the launch: with slices 8 and 0.3 for each of an XCD's, with atomics 55, about 70 us, measured where every block is
+// shared and the whole scratch zeroed and rounded (an upper bound for a few blocks, which errs on the side of not cutting).
+// lvx_bwd with atomics -> slices, us: 540 rows x 16 heads x 1346 tokens 80 -> 57.5, 3 x 500 x 12 heads of 32 x 5000 130 -> 112, 1000 x 32
+// x 2000 140 -> 124, 4000 x 8 x 3000 190 -> 180, 2048 x 32 of 64 x 6404 456 -> 444, 4096 x 32 x 6404 the same.
+//     rounds(S) = ceil(blocks * S / CUs)
 // for equal work-groups.  With an interval mask they differ in length (a token block
 // visits only the row tiles that see it; half of them is assumed); given at least two per CU the
 // dispatcher fills the tail by itself and rounds(S) is the plain quotient: splitting then
 // rarely pays (cfg4: 0.98 ms with 5 splits, 0.86 ms with none).
+constexpr int MAX_SLICES = 96;          // of an XCD
+
 // How the token blocks of a launch are handed to work-groups (see bwd_kernel): per XCD, the first
 // `whole` blocks get one work-group each, the next `mid` blocks `splits` work-groups each and the
 // others `splits2` each.
 struct BwdCut {
     int blocks_per_xcd, whole, mid, splits, splits2;
+    int ranges() const { return mid * splits + (blocks_per_xcd - whole - mid) * splits2; }      // of the blocks that are cut, per XCD
     bool any_split() const { return (mid > 0 && splits > 1) || (whole + mid < blocks_per_xcd && splits2 > 1); }
 };
 
-static BwdCut choose_bwd_cut(int blocks, int steps, bool masked) {
-    constexpr double WG_COST = 6.0, SPLIT_COST = 55.0;
+static BwdCut choose_bwd_cut(int blocks, int steps, bool masked, bool sliced) {
+    constexpr double WG_COST = 6.0;
+    const auto split_cost = [&](int ranges_per_xcd) { return sliced && ranges_per_xcd <= MAX_SLICES ? 8.0 + 0.3 * ranges_per_xcd : 55.0; };
     constexpr int XCDS = 8, MAX_SPLITS_PER_BLOCK = 16, MIN_RANGE = 32;
     const int n_cu = cu_count();
     BwdCut cut;
@@ -697,7 +702,7 @@ static BwdCut choose_bwd_cut(int blocks, int steps, bool masked) {
     auto cost = [&](int S) {
         const double rounds = ragged ? (double)blocks * S / n_cu
                                      : (double)(((int64_t)blocks * S + n_cu - 1) / n_cu);
-        return rounds * (work / S + WG_COST) + (S > 1 ? SPLIT_COST : 0.0);
+        return rounds * (work / S + WG_COST) + (S > 1 ? split_cost(cut.blocks_per_xcd * S) : 0.0);
     };
     int best = 1;
     double best_cost = cost(1);
@@ -718,10 +723,10 @@ static BwdCut choose_bwd_cut(int blocks, int steps, bool masked) {
     if (!ragged && cu_x > 0 && cut.blocks_per_xcd > cu_x && blocks % XCDS == 0) {
         const int full = cut.blocks_per_xcd / cu_x * cu_x, rest = cut.blocks_per_xcd - full;
         if (rest == 0) return cut;       // (best is 1 then)
-        const double whole_cost = (full / cu_x) * (steps + WG_COST) + SPLIT_COST;
+        const double whole_cost = (full / cu_x) * (steps + WG_COST);
         for (int S = 2; S <= 8; ++S) {
             if (steps / S < MIN_RANGE) break;
-            const double c = whole_cost + ((rest * S + cu_x - 1) / cu_x) * ((double)steps / S + WG_COST);
+            const double c = whole_cost + ((rest * S + cu_x - 1) / cu_x) * ((double)steps / S + WG_COST) + split_cost(rest * S);
             if (c < best_cost) { best_cost = c; cut.whole = full; cut.mid = rest; cut.splits = S; cut.splits2 = 1; }
         }
         const int S1 = (cu_x + rest - 1) / rest;
@@ -729,7 +734,7 @@ static BwdCut choose_bwd_cut(int blocks, int steps, bool masked) {
         if (S1 >= 2 && steps / S1 >= MIN_RANGE && left > 0) {
             int S2 = std::min(std::min(cu_x / left, MAX_SPLITS_PER_BLOCK), steps / MIN_RANGE);
             if (S2 >= 2) {
-                const double c = whole_cost + ((double)steps / S1 + WG_COST) + ((double)steps / S2 + WG_COST);
+                const double c = whole_cost + ((double)steps / S1 + WG_COST) + ((double)steps / S2 + WG_COST) + split_cost(n1 * S1 + left * S2);
                 if (c < best_cost) { best_cost = c; cut.whole = full; cut.mid = n1; cut.splits = S1; cut.splits2 = S2; }
             }
         }
@@ -737,8 +742,15 @@ static BwdCut choose_bwd_cut(int blocks, int steps, bool masked) {
     return cut;
 }
 
+static size_t slice_bytes(const lvx_attn_shape* s) { return (size_t)2 * 128 * s->D * sizeof(float); }
+static int token_blocks(const lvx_attn_shape* s) { return s->B * s->Hkv * ((s->Lkv + 127) / 128); }
+
+// Room for fp32 sums of dK and dV: of all tokens, or of MAX_SLICES ranges an XCD where it has any blocks to cut.  (Whatever the rows, so that a
+// workspace of the longest window serves all.)
 static size_t dkv_scratch_bytes(const lvx_attn_shape* s) {
-    return (size_t)2 * s->B * s->Lkv * s->Hkv * s->D * sizeof(float);
+    const size_t all = (size_t)2 * s->B * s->Lkv * s->Hkv * s->D * sizeof(float);
+    const int blocks = token_blocks(s);
+    return blocks < 8 ? all : std::max(all, (size_t)8 * std::min(MAX_SLICES, 8 * ((blocks + 7) / 8)) * slice_bytes(s));
 }
 
 static DqCut dq_cut(const lvx_attn_shape* s, int32_t row_count) {
@@ -760,8 +772,8 @@ static size_t dq_partial_bytes(const lvx_attn_shape* s, int32_t row_count) {
     return most;
 }
 
-// Regions of the backward workspace, in order: dS^T tiles; fp32 dK/dV scratch (split-steps mode
-// with bf16 outputs); row metadata records (2 floats per row and head); fp32 dQ partial tiles,
+// Regions of the backward workspace, in order: dS^T tiles; fp32 sums of dK/dV (slices, behind the plan where there is one, or
+// a scratch for atomics; with 16-bit outputs); row metadata records (2 floats per row and head); fp32 dQ partial tiles,
 // one slice per split (split dQ contraction only); with an interval mask the live-tile tables (hulls of row tiles, runs
 // of live tiles per token block, the groups ranked by hull length).  Every region is a multiple of 16 bytes.
 struct BwdWorkspace {
@@ -925,7 +937,11 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     // metadata kernel zeroes them on its way
     const int blocks = s->B * s->Hkv * p.n_kv_blocks;
     const int steps = p.G * (int)(rows / 32);
-    const BwdCut cut = choose_bwd_cut(blocks, steps, s->kv_start != nullptr);
+    const BwdCut cut = choose_bwd_cut(blocks, steps, s->kv_start != nullptr, blocks >= 8 && !dkv_accumulate);
+    if (cut.any_split() && !dkv_accumulate && (size_t)8 * cut.ranges() * slice_bytes(s) <= wsl.meta - wsl.dkv) {
+        p.slices = reinterpret_cast<float*>(wsb + wsl.dkv);
+        p.per_xcd = cut.ranges();
+    }
     // With intervals per row how long a block is shows on the device, which then plans the launch, in the fp32 scratch.  (A bias
     // seldom hides anything, and the plan would be 3 us for nothing.)
     PlanParams plan{};
@@ -939,12 +955,12 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
         plan.entries = reinterpret_cast<uint32_t*>(wsb + wsl.dkv);
         plan.shared = plan.entries + 8 * plan.slots * PLAN_ENTRY;
         const size_t tables = ((size_t)(8 * plan.slots * PLAN_ENTRY + 8 * plan.shared_max * SHARED_ENTRY) * sizeof(uint32_t) + 255) / 256 * 256;
-        const size_t room = wsl.meta - wsl.dkv, slice = (size_t)2 * 128 * s->D * sizeof(float);
-        p.slices = reinterpret_cast<float*>(wsb + wsl.dkv + tables);
-        plan.slices = room > tables ? (int)std::min<size_t>((room - tables) / slice / 8, 2 * cus) : 0;
+        const size_t room = wsl.meta - wsl.dkv;
+        plan.slices = room > tables ? (int)std::min<size_t>((room - tables) / slice_bytes(s) / 8, 2 * cus) : 0;
         if (plan.slices < 2) plan.entries = nullptr;
+        else p.slices = reinterpret_cast<float*>(wsb + wsl.dkv + tables);
         p.plan = plan.entries;
-        p.plan_slots = plan.slots;
+        if (plan.entries) p.per_xcd = plan.slots;
     }
     p.n_blocks = blocks;
     p.blocks_per_xcd = cut.blocks_per_xcd;
@@ -952,8 +968,8 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     p.mid_blocks = cut.mid;
     p.q_splits = cut.splits;
     p.q_splits2 = cut.splits2;
-    p.dkv_mode = cut.any_split() ? 2 : (dkv_accumulate ? 1 : 0);
-    float* const scratch = (cut.any_split() && !dkv_accumulate) ? reinterpret_cast<float*>(wsb + wsl.dkv) : nullptr;
+    p.dkv_mode = cut.any_split() && !p.slices ? 2 : (dkv_accumulate ? 1 : 0);
+    float* const scratch = p.dkv_mode == 2 && !dkv_accumulate ? reinterpret_cast<float*>(wsb + wsl.dkv) : nullptr;
     const DqCut dq_by = dq_cut(s, row_count);
     float* const dq32 = dq_by.splits > 1 ? reinterpret_cast<float*>(wsb + wsl.dq32) : nullptr;
     // the token blocks several work-groups share, and the fp32 scratch of the call that sums them
@@ -1010,8 +1026,10 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
         if (e != hipSuccess) return static_cast<int>(e);
     }
 
-    if (plan.entries) {
-        const CastSlicesParams cp{plan.shared, p.slices, plan.shared_max, s->B, s->Lkv, s->D, p.n_kv_blocks, p.f16, static_cast<uint16_t*>(dk->ptr),
+    if (p.slices) {
+        const CastSlicesParams cp{plan.entries ? plan.shared : nullptr, plan.entries ? plan.shared_max : cut.blocks_per_xcd - cut.whole,
+                                  cut.whole, cut.mid, cut.splits, cut.splits2, p.per_xcd, blocks, cut.blocks_per_xcd,
+                                  p.slices, s->B, s->Lkv, s->D, p.n_kv_blocks, p.f16, static_cast<uint16_t*>(dk->ptr),
                                   static_cast<uint16_t*>(dv->ptr), st3(dk), st3(dv)};
         e = launch_cast_slices(cp, st);
         if (e != hipSuccess) return static_cast<int>(e);

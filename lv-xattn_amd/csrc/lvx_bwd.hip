@@ -153,16 +153,14 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     const int whole = max(0, min(p.whole_blocks, nblk));
     const int mid = max(0, min(p.mid_blocks, nblk - whole));
     int blk, S = 1;
-    uint32_t sp = 0, kblk, b, range_slice = 0;
-    const bool planned = MASKED && p.plan;
-    if (planned) {
-        const uint32_t* const e = p.plan + (int64_t)(xcd * p.plan_slots + local) * PLAN_ENTRY;
+    uint32_t sp = 0, kblk, b;
+    if (MASKED && p.plan) {
+        const uint32_t* const e = p.plan + (int64_t)(xcd * p.per_xcd + local) * PLAN_ENTRY;
         const uint32_t what = __builtin_amdgcn_readfirstlane(e[0]);
         if (what == ~0u) return;
         blk = blk0 + (int)(what & 0xffffu);
         S = (int)(what >> 16 & 0xffu);
         sp = what >> 24;
-        range_slice = __builtin_amdgcn_readfirstlane(e[1]) + sp;
     } else if (local < whole) {
         blk = blk0 + local;
     } else if (local < whole + mid * p.q_splits) {
@@ -213,7 +211,7 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
     // nothing to visit and nothing to overwrite: done (bf16 outputs, mode 0, still get their zeros)
     // a block that its work-group owns alone is written by it directly, also when others are shared
     const bool alone = p.dkv_mode == 2 && S == 1;
-    const int dkv_mode = planned && S > 1 ? 3 : alone ? p.whole_mode : p.dkv_mode;
+    const int dkv_mode = S > 1 && p.slices ? 3 : alone ? p.whole_mode : p.dkv_mode;
     if (n_iter == 0 && dkv_mode != 0 && dkv_mode != 3) return;
 
     // ---- resident B operand: this wave's K rows (P-wave) or V rows (D-wave)
@@ -830,10 +828,16 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
             if (DH == 128) unsafeAtomicAdd(op + t * os.s + 64, src[t * (EP32 / 4) + 64]);
         }
     } else if (dkv_mode == 3) {
-        // A range of a plan: its slice, whole lines per instruction
+        // A range of a block that has several: its slice, whole lines per instruction
         constexpr int CPF = DH / 4, RPS = 64 / CPF;
         turn_f32();
-        float* const op = p.slices + (int64_t)range_slice * (2 * BN * DH) + (d_role ? 0 : BN * DH) + (32 * slice + lane / CPF) * DH + (lane % CPF) * 4;
+        const int at = xcd * p.per_xcd + local;         // (asked for once more: no scalar is to live through the steps for it)
+        int64_t range_slice = at - whole;
+        if (MASKED && p.plan) {
+            const uint32_t* const e = p.plan + (int64_t)at * PLAN_ENTRY;
+            range_slice = e[1] + (e[0] >> 24);
+        }
+        float* const op = p.slices + range_slice * (2 * BN * DH) + (d_role ? 0 : BN * DH) + (32 * slice + lane / CPF) * DH + (lane % CPF) * 4;
 #pragma unroll
         for (int i = 0; i < 32 / RPS; ++i)
             *reinterpret_cast<f32x4*>(op + i * RPS * DH) = *reinterpret_cast<const f32x4*>(ep + (lane / CPF) * EP32 + (lane % CPF) * 16 + i * (RPS * EP32));
@@ -893,7 +897,7 @@ hipError_t launch_bwd_t(const BwdParams& p, bool masked, hipStream_t st) {
 
 hipError_t launch_bwd(const BwdParams& params, bool masked, hipStream_t st, const CastParams* dq_before) {
     BwdParams p = params;
-    p.own_wg = p.plan ? 8 * p.plan_slots : 8 * (p.whole_blocks + p.mid_blocks * p.q_splits + (p.blocks_per_xcd - p.whole_blocks - p.mid_blocks) * p.q_splits2);
+    p.own_wg = p.plan ? 8 * p.per_xcd : 8 * (p.whole_blocks + p.mid_blocks * p.q_splits + (p.blocks_per_xcd - p.whole_blocks - p.mid_blocks) * p.q_splits2);
     p.dq_before = CastParams{};
     if (dq_before) {
         p.dq_before = *dq_before;

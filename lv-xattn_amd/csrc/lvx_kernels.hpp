@@ -197,7 +197,7 @@ struct BwdParams {
     int whole_blocks;          // of an XCD's blocks, the first so many get one work-group each (0 .. blocks_per_xcd),
     int mid_blocks, q_splits;  // the next mid_blocks are shared by q_splits work-groups each, every one taking a range of steps,
     int q_splits2;             // and the others by q_splits2 (>= 1) work-groups each
-    int dkv_mode;              // 0: store 16-bit, 1: fp32 +=, 2: fp32 atomic += (q_splits > 1: the shared blocks)
+    int dkv_mode;              // 0: store 16-bit, 1: fp32 +=, 2: fp32 atomic += (the shared blocks, not with slices)
     // mode 2: where and how the work-group of a block it owns alone writes (whole_mode 0 or 1)
     void* dk_whole;
     void* dv_whole;
@@ -210,8 +210,10 @@ struct BwdParams {
     const int32_t* live_runs;
     // Not null: which block and range a work-group takes, in place of whole_blocks and the rest (see PlanParams)
     const uint32_t* plan;
-    int plan_slots;
+    // Not null: a range of a block that has several leaves fp32 sums in a slice of its own, [dK, dV][128 tokens][D]: those of an XCD
+    // in the order of its work-groups (with a plan: where it says)
     float* slices;
+    int per_xcd;               // entries of the plan, or slices, of an XCD
     int f16;                   // element type of q, k, v, dout, the dS^T workspace and (mode 0) dk, dv
     Divisor by_splits, by_splits2, by_kv_blocks, by_B;     // filled in by launch_bwd
     // and the work-groups that are the token blocks' (a multiple of 8): any past them sum the slices of dQ of the window before
@@ -309,11 +311,13 @@ struct CastSharedParams {
     int f16;
 };
 
-// The sums of the blocks that a plan has cut, rounded into dK and dV.
+// The blocks that have been cut: their slices added and rounded into dK and dV.
 struct CastSlicesParams {
-    const uint32_t* shared;
+    const uint32_t* shared;    // of a plan, [8][shared_max][SHARED_ENTRY]; null: an XCD shares all but its first `whole` blocks, `mid` of
+    int shared_max;            // them among `splits` and the others among `splits2` work-groups
+    int whole, mid, splits, splits2, slices_per_xcd, n_blocks, blocks_per_xcd;
     const float* slices;
-    int shared_max, B, Lkv, D, n_kv_blocks, f16;
+    int B, Lkv, D, n_kv_blocks, f16;
     uint16_t* dk;
     uint16_t* dv;
     Strides3 dks, dvs;

@@ -756,22 +756,36 @@ __global__ __launch_bounds__(256) void cast_shared_kernel(const CastSharedParams
     }
 }
 
-// The blocks that a plan has cut, SHARE_PARTS work-groups each: their slices added in the order of their ranges and rounded.
+// The blocks that have been cut, SHARE_PARTS work-groups each: their slices added in the order of their ranges and rounded.  All blocks of
+// an XCD's list are its own again, whose L2 may still hold the slices.
 template <bool F16>
 __global__ __launch_bounds__(256) void cast_slices_kernel(const CastSlicesParams p) {
     using E = Elt<F16>;
-    const uint32_t* const e = p.shared + (int64_t)(blockIdx.x / SHARE_PARTS) * SHARED_ENTRY;
-    const int blk = (int)e[0], S = (int)e[1];
-    if (S == 0) return;
+    const int xcd = blockIdx.x % 8, part = (int)(blockIdx.x / 8 % SHARE_PARTS), j = (int)(blockIdx.x / (8 * SHARE_PARTS));
+    int blk, S, slice;
+    if (p.shared) {
+        const uint32_t* const e = p.shared + (int64_t)(xcd * p.shared_max + j) * SHARED_ENTRY;
+        blk = (int)e[0];
+        S = (int)e[1];
+        slice = (int)e[2];
+        if (S == 0) return;
+    } else {
+        const bool second = j >= p.mid;
+        S = second ? p.splits2 : p.splits;
+        slice = xcd * p.slices_per_xcd + (second ? p.mid * p.splits + (j - p.mid) * S : j * S);
+        blk = xcd * p.blocks_per_xcd + p.whole + j;
+        if (blk >= min((xcd + 1) * p.blocks_per_xcd, p.n_blocks)) return;
+    }
     const int kblk = blk % p.n_kv_blocks, bh = blk / p.n_kv_blocks, b = bh % p.B, hk = bh / p.B;
     const int sh = chunk_shift(p.D);
     const int64_t half = (int64_t)128 * p.D;
-    const float* const src = p.slices + (int64_t)e[2] * 2 * half;
+    const float* const src = p.slices + (int64_t)slice * 2 * half;
     for (int i = threadIdx.x; i < (SHARE_ROWS << sh); i += 256) {
-        const int r = (int)(blockIdx.x % SHARE_PARTS) * SHARE_ROWS + (i >> sh), token = kblk * 128 + r, chunk = i & ((1 << sh) - 1);
+        const int r = part * SHARE_ROWS + (i >> sh), token = kblk * 128 + r, chunk = i & ((1 << sh) - 1);
         if (token >= p.Lkv) return;
         const float* s = src + (int64_t)r * p.D + chunk * 8;
         f32x4 x[4] = {};
+#pragma unroll 4
         for (int k = 0; k < S; ++k, s += 2 * half) {
             x[0] += *reinterpret_cast<const f32x4*>(s);
             x[1] += *reinterpret_cast<const f32x4*>(s + 4);
@@ -987,6 +1001,7 @@ hipError_t launch_cast_shared(const CastSharedParams& p, hipStream_t st) {
 
 hipError_t launch_cast_slices(const CastSlicesParams& p, hipStream_t st) {
     const dim3 grid(8 * p.shared_max * SHARE_PARTS);
+    if (grid.x == 0) return hipSuccess;
     if (p.f16) return launch1(cast_slices_kernel<true>, grid, dim3(256), st, p);
     return launch1(cast_slices_kernel<false>, grid, dim3(256), st, p);
 }

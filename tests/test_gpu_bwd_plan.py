@@ -55,3 +55,25 @@ def test_every_block_is_summed_once(D, dtype, B, Hq, Hkv, Lq, Lkv, images, lens)
         _close(got[2], want[2], dtype)
         for x, y in zip(got[1:], want[1:]):
             assert (x[y == 0] == 0).all()           # what nobody sees
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16), (32, torch.bfloat16), (16, torch.float16)])
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lkv", [
+    (1, 16, 4, 540, 1346),          # every block cut alike, 6 or 5 an XCD
+    (1, 64, 8, 700, 700), (1, 8, 1, 2100, 1000),        # one block an XCD and more
+    (3, 12, 3, 500, 5000),          # 45 an XCD: whole rounds, the others cut
+    (1, 32, 8, 1000, 6404),         # two groups of others
+    (1, 8, 2, 600, 300)])           # six blocks: sums by atomics
+def test_blocks_of_several_work_groups(D, dtype, B, Hq, Hkv, Lq, Lkv):
+    from lv_xattn import _attn_forward
+    g = torch.Generator(device=DEV).manual_seed(Lq + D)
+    q, do = (torch.empty(B, Hq, Lq, D, dtype=dtype, device=DEV).normal_(generator=g) for _ in range(2))
+    k, v = (torch.empty(B, Hkv, Lkv, D, dtype=dtype, device=DEV).normal_(generator=g) for _ in range(2))
+    o, lse = _attn_forward(q, k, v, False, D ** -0.5, None, rounds=1, batched=True)[3:]
+    want = _run(q, k, v, o, do, lse, None, True)
+    got, again = (_run(q, k, v, o, do, lse, None, False) for _ in range(2))
+    assert torch.equal(got[0], want[0])
+    for x, y, z in zip(got[1:], want[1:], again[1:]):
+        _close(x, y, dtype)
+        assert B * Hkv * -(-Lkv // 128) < 8 or torch.equal(x, z)        # slices are added in one order
