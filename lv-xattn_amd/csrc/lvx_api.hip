@@ -1026,13 +1026,22 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
         if (e != hipSuccess) return static_cast<int>(e);
     }
 
+    CastSlicesParams cp{};
+    bool rides = false;
     if (p.slices) {
-        const CastSlicesParams cp{plan.entries ? plan.shared : nullptr, plan.entries ? plan.shared_max : cut.blocks_per_xcd - cut.whole,
-                                  cut.whole, cut.mid, cut.splits, cut.splits2, p.per_xcd, blocks, cut.blocks_per_xcd,
-                                  p.slices, s->B, s->Lkv, s->D, p.n_kv_blocks, p.f16, static_cast<uint16_t*>(dk->ptr),
-                                  static_cast<uint16_t*>(dv->ptr), st3(dk), st3(dv)};
-        e = launch_cast_slices(cp, st);
-        if (e != hipSuccess) return static_cast<int>(e);
+        cp = CastSlicesParams{plan.entries ? plan.shared : nullptr, plan.entries ? plan.shared_max : cut.blocks_per_xcd - cut.whole,
+                              cut.whole, cut.mid, cut.splits, cut.splits2, p.per_xcd, blocks, cut.blocks_per_xcd,
+                              p.slices, s->B, s->Lkv, s->D, p.n_kv_blocks, p.f16, static_cast<uint16_t*>(dk->ptr),
+                              static_cast<uint16_t*>(dv->ptr), st3(dk), st3(dv)};
+        // In the launch of dQ where there are few of them: its work-groups have a CU's registers to themselves or share them with one
+        // other, and more than a round of the slices' would keep it waiting.  lvx_bwd, a launch of its own -> in dQ's, us: 540 rows x 16
+        // heads x 1346 tokens (192 work-groups) 58.7 -> 54.0, 2378 x 64 of 64 x 700 159.8 -> 154.3; 3 x 500 x 12 of 32 x 5000 (416) would go
+        // 112 -> 120, 2048 x 32 of 64 x 6404 (608) 439 -> 469.
+        rides = cast_slices_blocks(cp) <= cu_count();
+        if (!rides) {
+            e = launch_cast_slices(cp, st);
+            if (e != hipSuccess) return static_cast<int>(e);
+        }
     }
 
     // dQ[b, h, rows, :] = dS^T[b, h]^T (rows x tokens) * K[b, h / G] (tokens x D), scale already in dS
@@ -1052,7 +1061,7 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     // cast sums the slices and rounds into dq
     g.k_splits = dq_by.splits; g.split_len = dq_by.split_len;
     g.part = dq32; g.part_split = (int64_t)s->B * s->Hq * row_count * s->D;      // [split][B * Hq][D][row_count]
-    e = launch_dq(g, st);
+    e = launch_dq(g, st, rides ? &cp : nullptr);
     if (e != hipSuccess || dq_by.splits <= 1) return static_cast<int>(e);
     CastParams cq{};
     cq.f16 = p.f16;

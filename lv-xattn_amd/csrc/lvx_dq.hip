@@ -1,6 +1,9 @@
 // dQ = (scale dS) K of the attention backward, from the dS^T workspace that bwd_kernel leaves: per (sample, q head) a
 // product [rows x tokens] [tokens x head dimension] whose left operand is read from memory exactly once.
+#include <cstddef>
+
 #include "lvx_common.hpp"
+#include "lvx_fold.hpp"
 #include "lvx_dq_rule.hpp"
 #include "lvx_kernels.hpp"
 
@@ -38,8 +41,9 @@ __global__ __launch_bounds__(256, 1) void dq_kernel(const DqParams p) {
     constexpr int RING = NS * STAGE, OUT = 4 * 32 * EP;
     __shared__ __attribute__((aligned(1024))) char lds[RING > OUT ? RING : OUT];
 
-    fetch_kernargs<sizeof(DqParams)>();
-    const int wid = p.order ? (int)blockIdx.x : xcd_remap(blockIdx.x, p.total_wg);
+    fetch_kernargs<offsetof(DqParams, cast)>();
+    if ((int)blockIdx.x < p.cast_wg) { cast_slices<F16>(p.cast, blockIdx.x); return; }
+    const int wid = p.order ? (int)blockIdx.x - p.cast_wg : xcd_remap(blockIdx.x - p.cast_wg, p.total_wg);
     if (wid >= p.total_wg) return;
     uint32_t split, tm, b, h;
     const uint32_t t1 = p.by_splits.split(wid, split);
@@ -242,8 +246,9 @@ __global__ __launch_bounds__(256, 1) void dq_few_kernel(const DqParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[RING > SUMS ? RING : SUMS];
     static_assert(4 * 32 * EP <= RING);
 
-    fetch_kernargs<sizeof(DqParams)>();
-    const int wid = xcd_remap(blockIdx.x, p.total_wg);
+    fetch_kernargs<offsetof(DqParams, cast)>();
+    if ((int)blockIdx.x < p.cast_wg) { cast_slices<F16>(p.cast, blockIdx.x); return; }
+    const int wid = xcd_remap(blockIdx.x - p.cast_wg, p.total_wg);
     if (wid >= p.total_wg) return;
     uint32_t split, tm, b;
     const uint32_t t1 = p.by_splits.split(wid, split);
@@ -410,7 +415,7 @@ __global__ __launch_bounds__(256, 1) void dq_few_kernel(const DqParams p) {
 
 template <int DH, bool F16>
 hipError_t launch_dq_t(const DqParams& p, hipStream_t st) {
-    const dim3 grid((p.total_wg + 7) / 8 * 8);
+    const dim3 grid(p.cast_wg + (p.total_wg + 7) / 8 * 8);
     auto go = [&](auto stream, auto ranged) {
         constexpr bool S = decltype(stream)::value, R = decltype(ranged)::value;
         if (p.few) return launch1((dq_few_kernel<DH, F16, S, R>), grid, dim3(256), st, p);
@@ -422,8 +427,12 @@ hipError_t launch_dq_t(const DqParams& p, hipStream_t st) {
 
 }  // namespace
 
-hipError_t launch_dq(const DqParams& params, hipStream_t st) {
+hipError_t launch_dq(const DqParams& params, hipStream_t st, const CastSlicesParams* cast) {
     DqParams p = params;
+    if (cast) {
+        p.cast = *cast;
+        p.cast_wg = cast_slices_blocks(*cast);
+    }
     if (p.order && (!p.tile_range || p.k_splits > 1 || p.few)) return hipErrorInvalidValue;
     const int group = p.few ? DQ_FEW_TILES : 8;
     const int tiles_m = (p.row_tiles + group - 1) / group, splits = p.k_splits > 1 ? p.k_splits : 1;

@@ -87,6 +87,52 @@ __device__ __forceinline__ void cast_t(const CastParams& p, int64_t idx) {
     *reinterpret_cast<u32x4*>(p.dst + b * p.ds.b + h * p.ds.h + (int64_t)row * p.ds.s + chunk * 8) = u;
 }
 
+// A token block of the scratch is zeroed and rounded by SHARE_PARTS work-groups of SHARE_ROWS tokens each.
+constexpr int SHARE_ROWS = 128 / SHARE_PARTS;
+
+// Work-group i of 256 threads.  The blocks that have been cut, SHARE_PARTS work-groups each: their slices added in the order of their ranges and rounded.  All blocks of
+// an XCD's list are its own again, whose L2 may still hold the slices.
+template <bool F16>
+__device__ __forceinline__ void cast_slices(const CastSlicesParams& p, uint32_t i) {
+    using E = Elt<F16>;
+    const int xcd = i % 8, part = (int)(i / 8 % SHARE_PARTS), j = (int)(i / (8 * SHARE_PARTS));
+    int blk, S, slice;
+    if (p.shared) {
+        const uint32_t* const e = p.shared + (int64_t)(xcd * p.shared_max + j) * SHARED_ENTRY;
+        blk = (int)e[0];
+        S = (int)e[1];
+        slice = (int)e[2];
+        if (S == 0) return;
+    } else {
+        const bool second = j >= p.mid;
+        S = second ? p.splits2 : p.splits;
+        slice = xcd * p.slices_per_xcd + (second ? p.mid * p.splits + (j - p.mid) * S : j * S);
+        blk = xcd * p.blocks_per_xcd + p.whole + j;
+        if (blk >= min((xcd + 1) * p.blocks_per_xcd, p.n_blocks)) return;
+    }
+    const int kblk = blk % p.n_kv_blocks, bh = blk / p.n_kv_blocks, b = bh % p.B, hk = bh / p.B;
+    const int sh = chunk_shift(p.D);
+    const int64_t half = (int64_t)128 * p.D;
+    const float* const src = p.slices + (int64_t)slice * 2 * half;
+    for (int k = threadIdx.x; k < (SHARE_ROWS << sh); k += 256) {
+        const int r = part * SHARE_ROWS + (k >> sh), token = kblk * 128 + r, chunk = k & ((1 << sh) - 1);
+        if (token >= p.Lkv) return;
+        const float* s = src + (int64_t)r * p.D + chunk * 8;
+        f32x4 x[4] = {};
+#pragma unroll 4
+        for (int n = 0; n < S; ++n, s += 2 * half) {
+            x[0] += *reinterpret_cast<const f32x4*>(s);
+            x[1] += *reinterpret_cast<const f32x4*>(s + 4);
+            x[2] += *reinterpret_cast<const f32x4*>(s + half);
+            x[3] += *reinterpret_cast<const f32x4*>(s + half + 4);
+        }
+        const u32x4 ku = {E::pack(x[0][0], x[0][1]), E::pack(x[0][2], x[0][3]), E::pack(x[1][0], x[1][1]), E::pack(x[1][2], x[1][3])};
+        const u32x4 vu = {E::pack(x[2][0], x[2][1]), E::pack(x[2][2], x[2][3]), E::pack(x[3][0], x[3][1]), E::pack(x[3][2], x[3][3])};
+        *reinterpret_cast<u32x4*>(p.dk + b * p.dks.b + hk * p.dks.h + (int64_t)token * p.dks.s + chunk * 8) = ku;
+        *reinterpret_cast<u32x4*>(p.dv + b * p.dvs.b + hk * p.dvs.h + (int64_t)token * p.dvs.s + chunk * 8) = vu;
+    }
+}
+
 template <class E>
 __device__ __forceinline__ void unpack8(u32x4 u, float f[8]) {
 #pragma unroll

@@ -324,6 +324,9 @@ struct CastSlicesParams {
 };
 hipError_t launch_cast_slices(const CastSlicesParams& p, hipStream_t st);
 
+constexpr int SHARE_PARTS = 4;          // work-groups to a block
+inline int cast_slices_blocks(const CastSlicesParams& p) { return 8 * p.shared_max * SHARE_PARTS; }
+
 // dQ = (scale dS) K of a window of `rows` rows, from the dS^T workspace.
 struct DqParams {
     const uint16_t* ds;        // dS^T tiles [B * Hq][token blocks][row tiles][16 groups of tokens][32 rows][8 tokens]
@@ -352,8 +355,10 @@ struct DqParams {
     // filled in by launch_dq
     int total_wg;
     Divisor by_splits, by_tiles_m, by_B, by_Hq, by_G;
+    int cast_wg;               // the first so many work-groups (a multiple of 8) do this, which is dK's and dV's
+    CastSlicesParams cast;
 };
-hipError_t launch_dq(const DqParams& p, hipStream_t st);
+hipError_t launch_dq(const DqParams& p, hipStream_t st, const CastSlicesParams* cast = nullptr);
 
 // One GEMM problem C[M,N] = sum over segments A_s[M,K_s] * B_s[K_s,N].
 struct GemmProblem {
