@@ -538,7 +538,8 @@ __global__ __launch_bounds__(256) void bwd_meta_kernel(const MetaParams p) {
 
 // Per (b, text row) the first and one-past-last key whose bias is not -inf, over all heads the bias distinguishes.  An
 // empty row gets (0, 0).  WAVES: waves that share a row, 1 or 4; BATCH: loads of 16 bytes a thread has in flight (see
-// launch_bias_hull).  Bound by reading the bias once.
+// launch_bias_hull).  Bound by reading the bias, once; a wave reads long rows from both ends inwards, as far as these hide
+// something (most biases hide neither, and nothing between them matters then).
 template <int WAVES, int BATCH>
 __global__ __launch_bounds__(256) void bias_hull_kernel(const BiasHullParams p) {
     constexpr int STEP = 4 * 64 * WAVES;                    // keys one load of the waves covers
@@ -549,21 +550,41 @@ __global__ __launch_bounds__(256) void bias_hull_kernel(const BiasHullParams p) 
         uint32_t row;
         const uint32_t b = p.by_Lq.split(rw, row);
         int lo = INT_MAX, hi = 0;
+        const auto see = [&](const f32x4& v, int k) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (k + j < p.Lkv && !(v[j] == -INFINITY)) { lo = min(lo, k + j); hi = max(hi, k + j + 1); }
+        };
         for (int h = 0; h < p.heads; ++h) {
             const float* br = p.bias + b * p.bias_b + h * p.bias_h + (int64_t)row * p.bias_r;
+            if (WAVES == 1 && BATCH == 4 && p.Lkv > BATCH * STEP) {
+                int first = 0, end = (p.Lkv + 3) & ~3;          // the keys that are left
+                bool low = true, high = true;                   // nothing seen below them, above them
+                while (first < end && (low || high)) {
+                    const int n = low ? high ? (BATCH + 1) / 2 : BATCH : 0;
+                    f32x4 v[BATCH];
+                    int k[BATCH];
+#pragma unroll
+                    for (int i = 0; i < BATCH; ++i) {
+                        k[i] = max(4 * lane + (i < n ? first + STEP * i : end - STEP * (i - n + 1)), 0);
+                        v[i] = *reinterpret_cast<const f32x4*>(br + min(k[i], (p.Lkv - 1) & ~3));
+                    }
+#pragma unroll
+                    for (int i = 0; i < BATCH; ++i) see(v[i], k[i]);
+                    first += STEP * n;
+                    end -= STEP * (BATCH - n);
+                    low = low && __builtin_amdgcn_ballot_w64(lo < first) == 0;
+                    high = high && __builtin_amdgcn_ballot_w64(hi > end) == 0;
+                }
+                continue;
+            }
             for (int k0 = 4 * lane; k0 < p.Lkv; k0 += BATCH * STEP) {
                 f32x4 v[BATCH];
 #pragma unroll
                 for (int i = 0; i < BATCH; ++i)
                     v[i] = *reinterpret_cast<const f32x4*>(br + min(k0 + i * STEP, (p.Lkv - 1) & ~3));
 #pragma unroll
-                for (int i = 0; i < BATCH; ++i) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int key = k0 + i * STEP + j;
-                        if (key < p.Lkv && !(v[i][j] == -INFINITY)) { lo = min(lo, key); hi = max(hi, key + 1); }
-                    }
-                }
+                for (int i = 0; i < BATCH; ++i) see(v[i], k0 + i * STEP);
             }
         }
 #pragma unroll
@@ -915,6 +936,9 @@ hipError_t launch_bwd_live(const LiveParams& p, hipStream_t st, bool has_hulls) 
 // 1024 rows x 1000 keys 2.5 / 3.5, x 2500 3.3 / 3.6, x 4096 3.9 / 3.7, x 6404 5.3 / 4.9; 2048 x 4096 4.8 / 5.2; 1 x 1300 2.26
 // / 2.13, 1 x 13000 5.7 / 3.1.  16384 x 400 with one, two and four loads 6.2, 5.9, 7.3 / 17.4; a wave to a row with one load
 // took 5.0 at 1024 x 4096 and 20.8 (10.7 with four) at 1024 x 13000.
+// From both ends inwards, nothing hidden / half of the row at one end, before -> now: 1024 x 4096 3.5 (a work-group to a row) -> 2.5 / 3.4,
+// 2048 x 4096 4.8 -> 2.8 / 4.1, 1024 x 6404 4.6 -> 2.5 / 3.9, 1024 x 13000 9.6 -> 2.5 / 6.5; 256 x 4096 would go 2.6 -> 2.45 / 3.3 and 64 x 13000
+// 3.5 -> 2.4 / 5.
 hipError_t launch_bias_hull(const BiasHullParams& params, hipStream_t st) {
     BiasHullParams p = params;
     const int64_t rows = (int64_t)p.B * p.Lq;
@@ -923,7 +947,7 @@ hipError_t launch_bias_hull(const BiasHullParams& params, hipStream_t st) {
     const dim3 by_wave((unsigned)std::min<int64_t>((rows + 3) / 4, 1 << 20));
     if (p.Lkv <= 256) return launch1((bias_hull_kernel<1, 1>), by_wave, dim3(256), st, p);
     if (p.Lkv <= 512) return launch1((bias_hull_kernel<1, 2>), by_wave, dim3(256), st, p);
-    if (p.Lkv <= 1024 || rows > std::min(1024, p.Lkv / 4)) return launch1((bias_hull_kernel<1, 4>), by_wave, dim3(256), st, p);
+    if (p.Lkv <= 1024 || rows > std::min(512, p.Lkv / 4)) return launch1((bias_hull_kernel<1, 4>), by_wave, dim3(256), st, p);
     return launch1((bias_hull_kernel<4, 4>), dim3((unsigned)rows), dim3(256), st, p);
 }
 
