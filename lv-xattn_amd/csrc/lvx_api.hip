@@ -214,6 +214,29 @@ static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int spli
     return fwd_cost(s, rows, form, splits, parts_f32, fwd_price(s, form));
 }
 
+// A second, closer fit, for launches without a dense bias: what the forms take by now, among them the fold inside a launch for few rows, K
+// and V from memory in every form.  520 random launches (1 .. 4096 rows against 300 .. 77000 keys, all head dimensions, K and V not in the
+// caches): the ranges and the form it finds cheapest are 1.4 % from the best on average, those of the one above 3.4.
+static double fwd_cost2(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32) {
+    struct Fit { double key_us, tile_us, load_us, round_us; };
+    const Fit f = s->D == 128 ? Fit{7.7e-3, 1.2, 0.26, 4.5} : s->D == 64 ? Fit{6.8e-3, 1.1, 0.0, 3.4} : s->D == 32 ? Fit{2.8e-3, 1.2, 0.2, 1.6} : Fit{3.6e-3, 1.1, 0.0, 1.7};
+    const int G = s->Hq / s->Hkv, hg = gcd(G, 4), n_cu = cu_count();
+    const int64_t split_len = fwd_split_len(s, form, splits), n = (s->Lkv + split_len - 1) / split_len;
+    const double kv_mb = (double)s->B * s->Hkv * s->Lkv * s->D * 4e-6;
+    double t = 0.0;
+    if (n > 1 && form == FWD_FEW && fold_inside((int)n, (int64_t)rows * G)) t = 2.4 + 0.054 * n;
+    else if (n > 1) t = 3.4 + 0.054 * n + (double)n * s->B * s->Hq * rows * ((4 * s->D + 8) / 6.9e6 + (parts_f32 ? 4 * s->D / 7.1e6 : 0.0));
+    const int64_t slots = form == FWD_WIDE || (form == FWD_FEW && s->D == 128) ? n_cu : 2 * n_cu;
+    if (form == FWD_FEW) {
+        const int64_t wgs = (int64_t)s->B * s->Hkv * (((int64_t)rows * G + 31) / 32) * n;
+        return t + 2.9 + std::hypot((double)((wgs + slots - 1) / slots) * (split_len * f.key_us + 3.2) - 3.2, kv_mb / 6.8);
+    }
+    const int wg_rows = (form == FWD_WIDE ? 64 : 32) * (4 / hg);
+    const int64_t wgs = (int64_t)s->B * (s->Hq / hg) * (((int64_t)rows + wg_rows - 1) / wg_rows) * n;
+    const double tile_us = f.tile_us + f.load_us * std::min(1.0, (double)wgs / slots);
+    return t + std::hypot((double)((wgs + slots - 1) / slots) * (split_len / FWD_BN * tile_us + f.round_us), kv_mb / 8.2);
+}
+
 // The form for few rows is for up to 256 (row, head) columns per kv head: it reads K and V from L2 once
 // per 32 of them, and with more the other forms only lose where they are cut into too few splits.
 constexpr int64_t FEW_MAX_COLS = 256;
@@ -237,19 +260,24 @@ static bool fwd_form_ok(const lvx_attn_shape* s, int rows, FwdForm form) {
 }
 constexpr FwdForm FWD_FORMS[] = {FWD_PLAIN, FWD_WIDE, FWD_FEW};
 
+// What the closer fit has to promise before a launch takes another form or other ranges than the first one says.  Of 520 random launches 29
+// are then faster by over 3 % (few rows of many keys by up to 30), 3 slower by up to 5; without it, 99 and 23 by up to 13.
+constexpr double CLOSER_FIT = 1.12;
+
 // The form of the forward kernel for a window of `rows` rows whose keys are cut into `splits` ranges.
 static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits, bool parts_f32) {
     const char* const e = getenv("LVX_FWD_WIDE");
-    FwdForm best = FWD_PLAIN;
-    double best_cost = 0.0;
+    FwdForm best[2] = {FWD_PLAIN, FWD_PLAIN};
+    double cost[2] = {0.0, 0.0};        // by either fit
     for (const FwdForm form : FWD_FORMS) {
         if (!fwd_form_ok(s, rows, form)) continue;
         if (e && form == (atoi(e) == 2 ? FWD_FEW : FWD_WIDE)) return form;
         if (e && form == FWD_FEW) continue;
-        const double c = fwd_cost(s, rows, form, splits, parts_f32);
-        if (best_cost == 0.0 || c < best_cost || (form == FWD_FEW && c == best_cost)) { best = form; best_cost = c; }
+        const double c[2] = {fwd_cost(s, rows, form, splits, parts_f32), s->bias ? 0.0 : fwd_cost2(s, rows, form, splits, parts_f32)};
+        for (int i = 0; i < 2; ++i)
+            if (cost[i] == 0.0 || c[i] < cost[i] || (form == FWD_FEW && c[i] == cost[i])) { best[i] = form; cost[i] = c[i]; }
     }
-    return best;
+    return s->bias || fwd_cost2(s, rows, best[0], splits, parts_f32) <= CLOSER_FIT * cost[1] ? best[0] : best[1];
 }
 
 // Whether the parts of a launch whose splits are chosen here wait for the fold in fp32.  In 16 bits they are a
@@ -290,7 +318,21 @@ int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
         }
         if (const int n = cheapest(form, f32, fwd_price(s, form), best_cost)) best = n > 1 && f32 ? n | LVX_SPLITS_FP32 : n;
     }
-    return best;
+    if (s->bias) return best;
+    // Parts are in 16 bits only where they were in a launch of as many rows before.
+    const bool whole = best == 1;
+    const auto parts = [&](int n, FwdForm form) { return n > 1 && (whole || fwd_parts_f32(s, row_count, form)) ? n | LVX_SPLITS_FP32 : n; };
+    int best2 = 1;
+    double best2_cost = 0.0;
+    for (const FwdForm form : FWD_FORMS)
+        for (int n = 1; fwd_form_ok(s, row_count, form) && n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
+            const double c = fwd_cost2(s, row_count, form, n, parts(n, form) != n);
+            if (best2_cost == 0.0 || c < best2_cost) { best2 = parts(n, form); best2_cost = c; }
+        }
+    const int n = best & ~LVX_SPLITS_FP32;
+    const FwdForm form = fwd_form(s, row_count, n, best != n);
+    if (fwd_cost2(s, row_count, form, n, best != n) > CLOSER_FIT * best2_cost) return best2;
+    return form == FWD_FEW ? parts(n, form) : best;
 }
 
 struct FwdGrid {
