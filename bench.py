@@ -508,7 +508,7 @@ def main():
         kb = kernel_breakdown(layer, npairs, torch)
         out["kernels"] = kb
         dom = kb["bwd_all_rounds_one_launch"]
-        out["roofline"] = {"bound": "mfma", "kernel": "lvx_bwd = bwd_meta_kernel (incl. zero-fill of the shared token blocks) + bwd_kernel + cast_shared_kernel + dq_kernel",
+        out["roofline"] = {"bound": "mfma", "kernel": "lvx_bwd = bwd_meta_kernel + bwd_kernel + cast_slices_kernel + dq_kernel",
                            "achieved": dom["tflops"], "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                            "frac": round(dom["tflops"] / PEAK_BF16_TFLOPS, 4),
                            "traffic": bwd_traffic_bytes(w.name) if a.mode == "batched" else None,

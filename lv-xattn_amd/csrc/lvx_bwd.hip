@@ -831,8 +831,10 @@ __global__ __launch_bounds__(NT, 1) void bwd_kernel(const BwdParams p) {
         // A range of a block that has several: its slice, whole lines per instruction
         constexpr int CPF = DH / 4, RPS = 64 / CPF;
         turn_f32();
-        const int at = xcd * p.per_xcd + local;         // (asked for once more: no scalar is to live through the steps for it)
-        int64_t range_slice = at - whole;
+        uint32_t id = blockIdx.x;           // taken apart once more: no scalar is to live through the steps for it
+        asm volatile("" : "+s"(id));
+        const int x = (int)(id % 8), at = x * p.per_xcd + (int)(id / 8);
+        int64_t range_slice = at - min(p.whole_blocks, p.n_blocks - x * p.blocks_per_xcd);
         if (MASKED && p.plan) {
             const uint32_t* const e = p.plan + (int64_t)at * PLAN_ENTRY;
             range_slice = e[1] + (e[0] >> 24);
