@@ -222,6 +222,7 @@ static double fwd_cost2(const lvx_attn_shape* s, int rows, FwdForm form, int spl
     const Fit f = s->D == 128 ? Fit{7.7e-3, 1.2, 0.26, 4.5} : s->D == 64 ? Fit{6.8e-3, 1.1, 0.0, 3.4} : s->D == 32 ? Fit{2.8e-3, 1.2, 0.2, 1.6} : Fit{3.6e-3, 1.1, 0.0, 1.7};
     const int G = s->Hq / s->Hkv, hg = gcd(G, 4), n_cu = cu_count();
     const int64_t split_len = fwd_split_len(s, form, splits), n = (s->Lkv + split_len - 1) / split_len;
+    const auto both = [](double x, double y) { return std::sqrt(x * x + y * y); };      // (hypot takes three times as long, for ranges that are not ours)
     const double kv_mb = (double)s->B * s->Hkv * s->Lkv * s->D * 4e-6;
     double t = 0.0;
     if (n > 1 && form == FWD_FEW && fold_inside((int)n, (int64_t)rows * G)) t = 2.4 + 0.054 * n;
@@ -229,12 +230,12 @@ static double fwd_cost2(const lvx_attn_shape* s, int rows, FwdForm form, int spl
     const int64_t slots = form == FWD_WIDE || (form == FWD_FEW && s->D == 128) ? n_cu : 2 * n_cu;
     if (form == FWD_FEW) {
         const int64_t wgs = (int64_t)s->B * s->Hkv * (((int64_t)rows * G + 31) / 32) * n;
-        return t + 2.9 + std::hypot((double)((wgs + slots - 1) / slots) * (split_len * f.key_us + 3.2) - 3.2, kv_mb / 6.8);
+        return t + 2.9 + both((double)((wgs + slots - 1) / slots) * (split_len * f.key_us + 3.2) - 3.2, kv_mb / 6.8);
     }
     const int wg_rows = (form == FWD_WIDE ? 64 : 32) * (4 / hg);
     const int64_t wgs = (int64_t)s->B * (s->Hq / hg) * (((int64_t)rows + wg_rows - 1) / wg_rows) * n;
     const double tile_us = f.tile_us + f.load_us * std::min(1.0, (double)wgs / slots);
-    return t + std::hypot((double)((wgs + slots - 1) / slots) * (split_len / FWD_BN * tile_us + f.round_us), kv_mb / 8.2);
+    return t + both((double)((wgs + slots - 1) / slots) * (split_len / FWD_BN * tile_us + f.round_us), kv_mb / 8.2);
 }
 
 // The form for few rows is for up to 256 (row, head) columns per kv head: it reads K and V from L2 once
@@ -267,17 +268,24 @@ constexpr double CLOSER_FIT = 1.12;
 // The form of the forward kernel for a window of `rows` rows whose keys are cut into `splits` ranges.
 static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits, bool parts_f32) {
     const char* const e = getenv("LVX_FWD_WIDE");
-    FwdForm best[2] = {FWD_PLAIN, FWD_PLAIN};
-    double cost[2] = {0.0, 0.0};        // by either fit
+    FwdForm ok[3];
+    int n = 0;
     for (const FwdForm form : FWD_FORMS) {
         if (!fwd_form_ok(s, rows, form)) continue;
         if (e && form == (atoi(e) == 2 ? FWD_FEW : FWD_WIDE)) return form;
         if (e && form == FWD_FEW) continue;
-        const double c[2] = {fwd_cost(s, rows, form, splits, parts_f32), s->bias ? 0.0 : fwd_cost2(s, rows, form, splits, parts_f32)};
-        for (int i = 0; i < 2; ++i)
-            if (cost[i] == 0.0 || c[i] < cost[i] || (form == FWD_FEW && c[i] == cost[i])) { best[i] = form; cost[i] = c[i]; }
+        ok[n++] = form;
     }
-    return s->bias || fwd_cost2(s, rows, best[0], splits, parts_f32) <= CLOSER_FIT * cost[1] ? best[0] : best[1];
+    if (n == 1) return ok[0];
+    double first[3], closer[3];
+    int a = 0, b = 0;                   // cheapest by either fit
+    for (int i = 0; i < n; ++i) {
+        first[i] = fwd_cost(s, rows, ok[i], splits, parts_f32);
+        closer[i] = s->bias ? 0.0 : fwd_cost2(s, rows, ok[i], splits, parts_f32);
+        if (first[i] < first[a] || (ok[i] == FWD_FEW && first[i] == first[a])) a = i;
+        if (closer[i] < closer[b]) b = i;
+    }
+    return ok[closer[a] <= CLOSER_FIT * closer[b] ? a : b];
 }
 
 // Whether the parts of a launch whose splits are chosen here wait for the fold in fp32.  In 16 bits they are a

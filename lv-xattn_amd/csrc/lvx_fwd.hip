@@ -935,8 +935,10 @@ struct FewColumns {
 //   O^T[d, 32 cols]      += V^T (A, transposing LDS reads) x P^T (B, straight from S^T)
 // LDS rows are 2 DH bytes (128 below head dimension 64, the lanes past the head dimension repeat a
 // chunk of the row), chunks permuted as in fwd_wide_kernel.
-template <int DH, bool MASKED, bool F16>
-__global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
+// INSIDE (fwd_fewest_kernel): the launch folds its own parts (a test at run time costs every other launch 0.2 us: four rounds of 140 rows x 3 heads of 32 35.6
+// us a pass without it, 36.3 with).
+template <int DH, bool MASKED, bool F16, bool INSIDE>
+__device__ __forceinline__ void fwd_few(const FwdParams& p) {
     using E = Elt<F16>;
     constexpr int LW = DH >= 64 ? DH : 64;                          // elements per LDS row
     constexpr int NKK = DH / 16, NDT = DH >= 32 ? DH / 32 : 1;
@@ -946,7 +948,6 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     constexpr int RING = 4 * 2 * 2 * PB, FOLD = 4 * 32 * EPS * 4;
     __shared__ __attribute__((aligned(1024))) char lds[RING > FOLD ? RING : FOLD];
     __shared__ float ml[4][2][32];                                  // per wave and column: reference maximum, row sum
-    __shared__ int last;
 
     fetch_kernargs<sizeof(FwdParams)>();
     const int wid = xcd_remap(blockIdx.x, p.total_wg);
@@ -961,10 +962,9 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
     uint32_t head;
     const int row = p.row_begin + p.by_G.split(col, head), h = hk * p.G + head;
 
-    const FewColumns<DH> columns{p, ct, b, hk};     // (where p.part says so)
+    const FewColumns<DH> columns{p, ct, b, hk};     // (INSIDE)
     uint64_t word = 0;
-    asm volatile("s_cmp_eq_u64 %2, 0\n\ts_cbranch_scc1 LVX_FEW_WORD_%=\n\tglobal_load_dwordx2 %0, %1, off sc1\nLVX_FEW_WORD_%=:"
-                 : "+v"(word) : "v"(columns.count()), "s"(p.part) : "memory", "scc");
+    if constexpr (INSIDE) asm volatile("global_load_dwordx2 %0, %1, off sc1" : "=v"(word) : "v"(columns.count()) : "memory");
 
     u32x4 q[NKK];
     {
@@ -1054,8 +1054,10 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
         asm volatile("" : "+v"(q[kk]));
         if (MASKED && empty) q[kk] = u32x4{0u, 0u, 0u, 0u};
     }
-    asm volatile("" : "+v"(word));          // requested before Q
-    if (p.part && tid == 0) columns.open(word);
+    if constexpr (INSIDE) {
+        asm volatile("" : "+v"(word));      // requested before Q
+        if (tid == 0) columns.open(word);
+    }
 
     for (int i = 0; i < n; ++i) {
         const int kv0 = base + 32 * (wave + 4 * i);
@@ -1150,7 +1152,7 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
         ml[wave][1][l32] = empty ? 0.f : l_tot;
     }
     __syncthreads();
-    if (p.part) {                   // the columns are four at most
+    if constexpr (INSIDE) {         // the columns are four at most
         if (wave < columns.cols) {
             float M = -INFINITY, den = 0.f, x0 = 0.f, x1 = 0.f;
 #pragma unroll
@@ -1168,6 +1170,7 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
             wait_vmcnt<0>();        // it is where the last work-group will read it
         }
         __syncthreads();
+        __shared__ int last;
         if (tid == 0) last = columns.last();
         __syncthreads();
         if (last && wave < columns.cols) columns.template fold<E>(wave);
@@ -1219,6 +1222,10 @@ __global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) {
         p.lse[split * p.lse_split_stride + ((int64_t)b * p.Hq + oh) * p.lse_bh_stride + orow] =
             den > 0.f ? M * p.scale + __logf(den) : no_lse(p, den);
 }
+template <int DH, bool MASKED, bool F16>
+__global__ __launch_bounds__(256, 1) void fwd_few_kernel(const FwdParams p) { fwd_few<DH, MASKED, F16, false>(p); }
+template <int DH, bool MASKED, bool F16>
+__global__ __launch_bounds__(256, 1) void fwd_fewest_kernel(const FwdParams p) { fwd_few<DH, MASKED, F16, true>(p); }
 
 }  // namespace
 
@@ -1227,6 +1234,10 @@ template <int DH, bool F16>
 hipError_t launch_fwd_t(const FwdParams& p, bool masked, hipStream_t st, const FwdFold* fold = nullptr) {
     const int grid = ((p.total_wg + 7) / 8) * 8;
     if (p.form == FWD_FEW) {
+        if (p.part) {
+            if (masked) return launch1((fwd_fewest_kernel<DH, true, F16>), dim3(grid), dim3(256), st, p);
+            return launch1((fwd_fewest_kernel<DH, false, F16>), dim3(grid), dim3(256), st, p);
+        }
         if (masked) return launch1((fwd_few_kernel<DH, true, F16>), dim3(grid), dim3(256), st, p);
         return launch1((fwd_few_kernel<DH, false, F16>), dim3(grid), dim3(256), st, p);
     }

@@ -55,6 +55,18 @@ def test_registers_that_assembly_loads_are_left_alone_until_the_wait(kernels):
 
 
 @needs_objdump
+def test_the_form_that_folds_its_own_parts_leaves_them_alone_too(kernels):
+    """fwd_fewest_kernel: the same, its count requested in front of Q, and the parts that are read back."""
+    fewest = {n: b for n, b in kernels.items() if "fwd_fewest_kernel" in n}
+    assert len(fewest) == 16
+    for name, body in fewest.items():
+        jump = next(i for i, ins in enumerate(body) if ins.target and "LVX_FEW_TWO" in ins.args[0])
+        assert next(i for i, ins in enumerate(body) if ins.op == "global_load_dwordx2") < \
+            next(i for i, ins in enumerate(body) if ins.op == "global_load_dwordx4"), name
+        assert isa.waits_for(body[jump + 1]) == 0 and not isa.loads_touched_early(body, stated=[body[jump + 2]]), name
+
+
+@needs_objdump
 def test_a_bias_on_its_way_is_left_alone_until_the_wait(kernels):
     """The forward with a dense bias requests it by inline assembly a tile ahead: the same."""
     biased = {n: b for n, b in kernels.items() if re.search(r"fwd_kernelILi\d+ELb[01]ELb1E", n)}
