@@ -327,9 +327,10 @@ int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
         if (const int n = cheapest(form, f32, fwd_price(s, form), best_cost)) best = n > 1 && f32 ? n | LVX_SPLITS_FP32 : n;
     }
     if (s->bias) return best;
-    // Parts are in 16 bits only where they were in a launch of as many rows before.
-    const bool whole = best == 1;
-    const auto parts = [&](int n, FwdForm form) { return n > 1 && (whole || fwd_parts_f32(s, row_count, form)) ? n | LVX_SPLITS_FP32 : n; };
+    // Parts are in 16 bits only where those of the first fit are: not where it leaves the launch whole, nor where it takes the form for few
+    // rows, in whichever form they then come about.
+    const bool f32 = best == 1 || (best & LVX_SPLITS_FP32);
+    const auto parts = [&](int n, FwdForm form) { return n > 1 && (f32 || form == FWD_FEW) ? n | LVX_SPLITS_FP32 : n; };
     int best2 = 1;
     double best2_cost = 0.0;
     for (const FwdForm form : FWD_FORMS)

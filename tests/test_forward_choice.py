@@ -1,4 +1,7 @@
 """The ranges a forward launch is cut into: where the closer fit takes over from the first (us, first -> closer), and where it does not."""
+import math
+import random
+
 import pytest
 
 
@@ -18,3 +21,52 @@ def test_parts_that_were_not_there_before_wait_in_fp32():
     for shape in [(4, 8, 2, 24, 749, 64), (4, 16, 4, 706, 9539, 128), (2, 64, 8, 303, 4410, 16), (1, 32, 16, 1129, 3353, 32)]:
         n = auto_kv_splits(*shape)
         assert n == 1 or n & 256
+
+
+def _first_fit(B, Hq, Hkv, rows, Lkv, D, cus=256):
+    """The number of ranges that the first fit finds cheapest for a launch without a dense bias, and whether their parts wait in fp32."""
+    G = Hq // Hkv
+    hg = math.gcd(G, 4)
+    wide = D in (64, 128)
+
+    def cost(few, splits, f32):
+        step = 32 if few else 64
+        length = -(-(-(-Lkv // splits)) // step) * step
+        n = -(-Lkv // length)
+        us = 4.0 + n * B * Hq * rows * ((4 * D + 8) / 4e6 + (4 * D / 9e6 if f32 else 0.0)) if n > 1 else 0.0
+        if few:
+            wgs, slots = B * Hkv * -(-rows * G // 32) * n, cus if D == 128 else 2 * cus
+            key_us = {128: 8e-3, 64: 4.2e-3}.get(D, 3e-3)
+            return us + 5.0 + math.hypot(-(-wgs // slots) * (length * key_us + 3.0) - 3.0, B * Hkv * Lkv * D * 4 / 5.2e6)
+        wgs, slots = B * (Hq // hg) * -(-rows // ((64 if wide else 32) * (4 // hg))) * n, cus if wide else 2 * cus
+        tile_us, load_us = (1.1, 0.4) if D == 128 else (0.9, 0.15) if D == 64 else (0.8, 1.0)
+        return us + -(-wgs // slots) * (length // 64 * (tile_us + load_us * min(1.0, wgs / slots)) + 11.0)
+
+    few_f32, many_f32 = True, B * (Hq // hg) * -(-rows // (32 * (4 // hg))) >= 2 * cus or Lkv < 1024
+    return min((cost(few, n, f32), few, n, n > 1 and f32) for few, f32 in ((False, many_f32), (True, few_f32)) if not few or rows * G <= 256
+               for n in range(1, 65) if n == 1 or Lkv // n >= 32)[2:]
+
+
+def _launches(seed, count, most_keys):
+    rng = random.Random(seed)
+
+    def log_int(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+    for _ in range(count):
+        hkv = rng.choice([1, 2, 4, 8, 8, 16])
+        yield (rng.choice([1, 1, 2, 3, 4]), hkv * rng.choice([1, 2, 4, 4, 8]), hkv, log_int(1, 4096), log_int(300, most_keys),
+               rng.choice([128, 128, 128, 64, 64, 32, 16]))
+
+
+def _held_in_16_bits(n):
+    return n > 1 and not n & 256
+
+
+def test_no_part_waits_in_fewer_bits_than_the_first_fit_says():
+    from lv_xattn.attn import auto_kv_splits
+    few_to_wide = [(2, 32, 8, 45, 3450, 128), (1, 8, 8, 206, 7423, 128), (1, 32, 8, 49, 62466, 64), (4, 4, 4, 250, 20294, 64),
+                   (3, 8, 2, 62, 25098, 64), (1, 16, 16, 188, 46687, 64), (3, 4, 4, 220, 5649, 128)]
+    assert [_first_fit(*s) for s in few_to_wide[:2]] == [(2, True), (4, True)]
+    for shape in few_to_wide + list(_launches(11, 6000, 77000)):
+        n, f32 = _first_fit(*shape)
+        assert not _held_in_16_bits(auto_kv_splits(*shape)) or (n > 1 and not f32), shape
