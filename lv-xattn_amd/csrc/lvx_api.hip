@@ -315,15 +315,15 @@ int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
         }
         return best;
     };
+    // With a dense bias, parts are in 16 bits only where the plain form at the price it has without one would be cut: a launch that only the
+    // prices with a bias cut keeps the precision of the whole one, in either form.
+    double plain_cost = 0.0;
+    const bool only_here = s->bias && cheapest(FWD_PLAIN, fwd_parts_f32(s, row_count, FWD_PLAIN), PLAIN_PRICE, plain_cost) == 1;
     int best = 1;
     double best_cost = 0.0;
     for (const FwdForm form : FWD_FORMS) {
         if (!fwd_form_ok(s, row_count, form)) continue;
-        bool f32 = fwd_parts_f32(s, row_count, form);
-        if (form == FWD_WIDE && s->bias && !f32) {      // a launch that only this form cuts keeps its precision
-            double plain_cost = 0.0;
-            f32 = cheapest(FWD_PLAIN, false, PLAIN_PRICE, plain_cost) == 1;
-        }
+        const bool f32 = only_here || fwd_parts_f32(s, row_count, form);
         if (const int n = cheapest(form, f32, fwd_price(s, form), best_cost)) best = n > 1 && f32 ? n | LVX_SPLITS_FP32 : n;
     }
     if (s->bias) return best;

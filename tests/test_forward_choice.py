@@ -23,11 +23,12 @@ def test_parts_that_were_not_there_before_wait_in_fp32():
         assert n == 1 or n & 256
 
 
-def _first_fit(B, Hq, Hkv, rows, Lkv, D, cus=256):
-    """The number of ranges that the first fit finds cheapest for a launch without a dense bias, and whether their parts wait in fp32."""
+def _first_fit(B, Hq, Hkv, rows, Lkv, D, bias=False, cus=256):
+    """The number of ranges that the first fit finds cheapest, and whether their parts wait in fp32.  With a dense bias: of the plain form, at
+    the price it has without one."""
     G = Hq // Hkv
     hg = math.gcd(G, 4)
-    wide = D in (64, 128)
+    wide = D in (64, 128) and not bias
 
     def cost(few, splits, f32):
         step = 32 if few else 64
@@ -39,11 +40,11 @@ def _first_fit(B, Hq, Hkv, rows, Lkv, D, cus=256):
             key_us = {128: 8e-3, 64: 4.2e-3}.get(D, 3e-3)
             return us + 5.0 + math.hypot(-(-wgs // slots) * (length * key_us + 3.0) - 3.0, B * Hkv * Lkv * D * 4 / 5.2e6)
         wgs, slots = B * (Hq // hg) * -(-rows // ((64 if wide else 32) * (4 // hg))) * n, cus if wide else 2 * cus
-        tile_us, load_us = (1.1, 0.4) if D == 128 else (0.9, 0.15) if D == 64 else (0.8, 1.0)
+        tile_us, load_us = (0.8, 1.0) if not wide else (1.1, 0.4) if D == 128 else (0.9, 0.15)
         return us + -(-wgs // slots) * (length // 64 * (tile_us + load_us * min(1.0, wgs / slots)) + 11.0)
 
     few_f32, many_f32 = True, B * (Hq // hg) * -(-rows // (32 * (4 // hg))) >= 2 * cus or Lkv < 1024
-    return min((cost(few, n, f32), few, n, n > 1 and f32) for few, f32 in ((False, many_f32), (True, few_f32)) if not few or rows * G <= 256
+    return min((cost(few, n, f32), few, n, n > 1 and f32) for few, f32 in ((False, many_f32), (True, few_f32)) if not few or (rows * G <= 256 and not bias)
                for n in range(1, 65) if n == 1 or Lkv // n >= 32)[2:]
 
 
@@ -70,3 +71,13 @@ def test_no_part_waits_in_fewer_bits_than_the_first_fit_says():
     for shape in few_to_wide + list(_launches(11, 6000, 77000)):
         n, f32 = _first_fit(*shape)
         assert not _held_in_16_bits(auto_kv_splits(*shape)) or (n > 1 and not f32), shape
+
+
+def test_no_part_of_a_launch_with_a_bias_waits_in_fewer_bits_than_the_plain_form_says():
+    from lv_xattn.attn import auto_kv_splits
+    left_whole = [(1, 32, 4, 638, 1059, 128), (1, 8, 1, 1903, 1090, 128), (1, 64, 8, 293, 1095, 128), (1, 64, 8, 254, 1251, 128),
+                  (3, 16, 8, 441, 1563, 128), (3, 64, 16, 96, 1024, 64)]
+    for shape in left_whole + list(_launches(12, 6000, 13000)):
+        n, f32 = _first_fit(*shape, bias=True)
+        assert shape not in left_whole or n == 1
+        assert not _held_in_16_bits(auto_kv_splits(*shape, True)) or (n > 1 and not f32), shape
