@@ -177,18 +177,22 @@ static int fwd_split_len(const lvx_attn_shape* s, FwdForm form, int splits) {
 // with a dense bias and heads of 128 / 64 (launches of 1 .. 2000 rows against 400 .. 13000 keys, ranges of 1 to 64):
 //   wide : 7 us per round and per tile 1.65 us on an idle chip, 2.1 on a full one (6 us, 1.45, 1.55)
 //   plain: 4 us and 2.15, or 2.8 once CUs have two work-groups (3.5 us, 1.95 and 2.35)
-// plus, with splits, 4 us for the launch that folds the parts and their bytes at 4 TB/s, what fp32 adds to them at 9.
+// plus, with splits, 4 us for the launch that folds the parts and their bytes at 4 TB/s, what fp32 adds to them at 9.  With a dense bias and
+// heads of 128 and 64 each part takes the fold 0.054 us besides (in the other prices the 11 us of a round stand for it): of 647 such
+// launches, ranges that are dearer by over 3 % than those of the plain form at its earlier price are chosen for 6, without it for 19,
+// by up to 18 % (142 rows x 3 heads x 3391 keys: 27 ranges 14.5 us, 53 18.3).
 struct FwdPrice {
     double tile_us, load_us, round_us;      // per key tile on an idle chip, what a full one adds, per round of work-groups
     bool shared;                            // it is two work-groups on a CU that add it, however many there are
+    double part_us;                         // per part, in the fold
 };
-constexpr FwdPrice PLAIN_PRICE{0.8, 1.0, 11.0, false};
+constexpr FwdPrice PLAIN_PRICE{0.8, 1.0, 11.0, false, 0.0};
 static FwdPrice fwd_price(const lvx_attn_shape* s, FwdForm form) {
     const bool wide = form == FWD_WIDE;
-    if (s->bias && s->D == 128) return wide ? FwdPrice{1.65, 0.45, 7.0, false} : FwdPrice{2.15, 0.65, 4.0, true};
-    if (s->bias && s->D == 64) return wide ? FwdPrice{1.45, 0.1, 6.0, false} : FwdPrice{1.95, 0.4, 3.5, true};
+    if (s->bias && s->D == 128) return wide ? FwdPrice{1.65, 0.45, 7.0, false, 0.054} : FwdPrice{2.15, 0.65, 4.0, true, 0.054};
+    if (s->bias && s->D == 64) return wide ? FwdPrice{1.45, 0.1, 6.0, false, 0.054} : FwdPrice{1.95, 0.4, 3.5, true, 0.054};
     if (!wide) return PLAIN_PRICE;
-    return s->D == 128 ? FwdPrice{1.1, 0.4, 11.0, false} : FwdPrice{0.9, 0.15, 11.0, false};
+    return s->D == 128 ? FwdPrice{1.1, 0.4, 11.0, false, 0.0} : FwdPrice{0.9, 0.15, 11.0, false, 0.0};
 }
 
 static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32, const FwdPrice& price) {
@@ -196,7 +200,7 @@ static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int spli
     const int64_t split_len = fwd_split_len(s, form, splits);
     const int64_t n = (s->Lkv + split_len - 1) / split_len;
     const double fold_us = (4 * s->D + 8) / 4e6 + (parts_f32 ? 4 * s->D / 9e6 : 0.0);       // per row, head and part
-    double t = n > 1 ? 4.0 + (double)n * s->B * s->Hq * rows * fold_us : 0.0;
+    double t = n > 1 ? 4.0 + n * price.part_us + (double)n * s->B * s->Hq * rows * fold_us : 0.0;
     if (form == FWD_FEW) {
         const int64_t wgs = (int64_t)s->B * s->Hkv * (((int64_t)rows * G + 31) / 32) * n;
         const int64_t slots = s->D == 128 ? n_cu : 2 * n_cu;

@@ -81,3 +81,13 @@ def test_no_part_of_a_launch_with_a_bias_waits_in_fewer_bits_than_the_plain_form
         n, f32 = _first_fit(*shape, bias=True)
         assert shape not in left_whole or n == 1
         assert not _held_in_16_bits(auto_kv_splits(*shape, True)) or (n > 1 and not f32), shape
+
+
+@pytest.mark.parametrize("shape,most", [         # us with so many ranges, with those of a price without what a part costs
+    ((3, 1, 1, 142, 3391, 128), 40),                # 27: 14.5, 53: 18.3
+    ((1, 4, 1, 198, 3374, 64), 40),                 # 27: 12.9, 53: 15.6
+    ((4, 8, 2, 40, 1151, 128), 14),                 # 9: 15.2, 18: 17.8
+    ((4, 4, 1, 39, 7360, 128), 40), ((2, 8, 2, 75, 4281, 128), 26), ((1, 8, 2, 160, 4018, 64), 26), ((1, 8, 8, 739, 860, 64), 6)])
+def test_a_launch_with_a_bias_is_not_cut_for_less_than_its_parts_cost(shape, most):
+    from lv_xattn.attn import auto_kv_splits
+    assert 1 < auto_kv_splits(*shape, True) & 255 <= most
