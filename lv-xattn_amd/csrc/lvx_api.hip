@@ -219,22 +219,26 @@ static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int spli
 }
 
 // A second, closer fit, for launches without a dense bias: what the forms take by now, among them the fold inside a launch for few rows, K
-// and V from memory in every form.  520 random launches (1 .. 4096 rows against 300 .. 77000 keys, all head dimensions, K and V not in the
-// caches): the ranges and the form it finds cheapest are 1.4 % from the best on average, those of the one above 3.4.
+// and V from memory in every form.  900 random launches (1 .. 2500 rows against 300 .. 40000 keys, all head dimensions, K and V not in the
+// caches): the ranges and the form it finds cheapest are 1.7 % from the best on average, those of the one above 3.4.  (A work-group for few rows that
+// shares its CU takes longer per key, with heads of 64 by half; and a load of the fold inside a launch holds 2048 / D parts.  With one price for both, and
+// for parts of any size, short launches and small heads were cut where that costs: 155 rows x 3 x 16 heads of 64 x 2652 keys 17.5 us whole,
+// 19.8 in two parts, 3 x 2 x 2 of 32 x 12498 7.5 in 56, 8.6 in 23.)
 static double fwd_cost2(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32) {
-    struct Fit { double key_us, tile_us, load_us, round_us; };
-    const Fit f = s->D == 128 ? Fit{7.7e-3, 1.2, 0.26, 4.5} : s->D == 64 ? Fit{6.8e-3, 1.1, 0.0, 3.4} : s->D == 32 ? Fit{2.8e-3, 1.2, 0.2, 1.6} : Fit{3.6e-3, 1.1, 0.0, 1.7};
+    struct Fit { double key_us, key2_us, tile_us, load_us, round_us; };     // per key of a work-group that has its CU to itself, that shares it
+    const Fit f = s->D == 128 ? Fit{7.7e-3, 7.7e-3, 1.2, 0.26, 4.5} : s->D == 64 ? Fit{4.4e-3, 6.9e-3, 1.1, 0.0, 3.4}
+                : s->D == 32 ? Fit{3.8e-3, 5.3e-3, 1.2, 0.2, 1.6} : Fit{3.7e-3, 4.9e-3, 1.1, 0.0, 1.7};
     const int G = s->Hq / s->Hkv, hg = gcd(G, 4), n_cu = cu_count();
     const int64_t split_len = fwd_split_len(s, form, splits), n = (s->Lkv + split_len - 1) / split_len;
     const auto both = [](double x, double y) { return std::sqrt(x * x + y * y); };      // (hypot takes three times as long, for ranges that are not ours)
     const double kv_mb = (double)s->B * s->Hkv * s->Lkv * s->D * 4e-6;
     double t = 0.0;
-    if (n > 1 && form == FWD_FEW && fold_inside((int)n, (int64_t)rows * G)) t = 2.4 + 0.054 * n;
+    if (n > 1 && form == FWD_FEW && fold_inside((int)n, (int64_t)rows * G)) t = (s->D == 128 ? 2.4 : 1.5) + 0.054 * n * s->D / 128;
     else if (n > 1) t = 3.4 + 0.054 * n + (double)n * s->B * s->Hq * rows * ((4 * s->D + 8) / 6.9e6 + (parts_f32 ? 4 * s->D / 7.1e6 : 0.0));
     const int64_t slots = form == FWD_WIDE || (form == FWD_FEW && s->D == 128) ? n_cu : 2 * n_cu;
     if (form == FWD_FEW) {
         const int64_t wgs = (int64_t)s->B * s->Hkv * (((int64_t)rows * G + 31) / 32) * n;
-        return t + 2.9 + both((double)((wgs + slots - 1) / slots) * (split_len * f.key_us + 3.2) - 3.2, kv_mb / 6.8);
+        return t + 2.9 + both((double)((wgs + slots - 1) / slots) * (split_len * (wgs <= n_cu ? f.key_us : f.key2_us) + 3.2) - 3.2, kv_mb / 6.8);
     }
     const int wg_rows = (form == FWD_WIDE ? 64 : 32) * (4 / hg);
     const int64_t wgs = (int64_t)s->B * (s->Hq / hg) * (((int64_t)rows + wg_rows - 1) / wg_rows) * n;
@@ -265,8 +269,9 @@ static bool fwd_form_ok(const lvx_attn_shape* s, int rows, FwdForm form) {
 }
 constexpr FwdForm FWD_FORMS[] = {FWD_PLAIN, FWD_WIDE, FWD_FEW};
 
-// What the closer fit has to promise before a launch takes another form or other ranges than the first one says.  Of 520 random launches 29
-// are then faster by over 3 % (few rows of many keys by up to 30), 3 slower by up to 5; without it, 99 and 23 by up to 13.
+// What the closer fit has to promise before a launch takes another form or other ranges than the first one says.  Of 12000 random launches 592
+// then do, 450 of them faster by over 3 % (few rows of many keys by up to 32), 12 slower by up to 9.  (Of 900 others 30 and 2;
+// at 1.05 107 and 12, without it 184 and 30 by up to 22.)
 constexpr double CLOSER_FIT = 1.12;
 
 // The form of the forward kernel for a window of `rows` rows whose keys are cut into `splits` ranges.

@@ -91,3 +91,15 @@ def test_no_part_of_a_launch_with_a_bias_waits_in_fewer_bits_than_the_plain_form
 def test_a_launch_with_a_bias_is_not_cut_for_less_than_its_parts_cost(shape, most):
     from lv_xattn.attn import auto_kv_splits
     assert 1 < auto_kv_splits(*shape, True) & 255 <= most
+
+
+@pytest.mark.parametrize("shape", [             # us with the first fit's ranges, with those of one price per key and part
+    (3, 16, 16, 155, 2652, 64),                     # 17.5, 19.8
+    (1, 8, 8, 167, 1018, 64),                       # 8.6, 9.5
+    (4, 16, 4, 58, 1347, 64), (3, 8, 1, 5, 955, 64), (2, 16, 8, 35, 1141, 64),
+    (2, 2, 2, 3, 12498, 32),                        # 7.5, 8.6
+    (1, 8, 4, 1, 11309, 32), (1, 2, 2, 2, 10552, 32), (4, 1, 1, 2, 7849, 32)])
+def test_short_launches_and_small_heads_keep_the_ranges_of_the_first_fit(shape):
+    from lv_xattn.attn import auto_kv_splits
+    n, f32 = _first_fit(*shape)
+    assert auto_kv_splits(*shape) == n | 256 * f32
