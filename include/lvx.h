@@ -254,6 +254,12 @@ int lvx_bwd_from_o(const lvx_attn_shape* shape, const lvx_tensor* q, const lvx_t
 size_t lvx_bwd_workspace_bytes(const lvx_attn_shape* shape, int32_t row_count);
 
 /*
+ * The same for calls that accumulate, and the least that lvx_bwd takes: without the room in which work-groups that share tokens leave their sums
+ * of 16-bit dk and dv (up to 100 MB with heads of 128).  A call that does not accumulate has them added up by atomics in less.
+ */
+size_t lvx_bwd_acc_workspace_bytes(const lvx_attn_shape* shape, int32_t row_count);
+
+/*
  * dst(dtype, strided) = src(fp32, [B, H, L, D] contiguous): the final rounding of
  * an fp32 accumulator (the `dq.copy_(dq_accum)` of flash_attn_kernels.py:1020).
  */

@@ -747,70 +747,97 @@ struct BwdCut {
     bool any_split() const { return (mid > 0 && splits > 1) || (whole + mid < blocks_per_xcd && splits2 > 1); }
 };
 
-static BwdCut choose_bwd_cut(int blocks, int steps, bool masked, bool sliced) {
+// Every cut that is priced, the one that leaves all blocks whole first.
+struct BwdCuts {
+    BwdCut cut[16];
+    double cost[16];
+    int n;
+};
+static BwdCuts bwd_cuts(int blocks, int steps, bool masked, bool sliced) {
+    BwdCuts all;
+    all.n = 0;
+    const auto add = [&](const BwdCut& cut, double cost) { all.cut[all.n] = cut; all.cost[all.n++] = cost; };
     constexpr double WG_COST = 6.0;
     const auto split_cost = [&](int ranges_per_xcd) { return sliced && ranges_per_xcd <= MAX_SLICES ? 8.0 + 0.3 * ranges_per_xcd : 55.0; };
     constexpr int XCDS = 8, MAX_SPLITS_PER_BLOCK = 16, MIN_RANGE = 32;
     const int n_cu = cu_count();
-    BwdCut cut;
-    cut.blocks_per_xcd = (blocks + XCDS - 1) / XCDS;
-    cut.splits2 = 1;
+    const int per_xcd = (blocks + XCDS - 1) / XCDS;
     // unequal work-groups only even out when there are enough of them; a small masked launch
     // is priced like a dense one (which is also right when its mask hides nothing)
     const bool ragged = masked && blocks >= 2 * n_cu;
     const double work = ragged ? 0.5 * steps : (double)steps;
-    auto cost = [&](int S) {
+    for (int S = 1; S <= 8; ++S) {
+        if (S > 1 && steps / S < MIN_RANGE) break;
         const double rounds = ragged ? (double)blocks * S / n_cu
                                      : (double)(((int64_t)blocks * S + n_cu - 1) / n_cu);
-        return rounds * (work / S + WG_COST) + (S > 1 ? split_cost(cut.blocks_per_xcd * S) : 0.0);
-    };
-    int best = 1;
-    double best_cost = cost(1);
-    for (int S = 2; S <= 8; ++S) {
-        if (steps / S < MIN_RANGE) break;
-        const double c = cost(S);
-        if (c < best_cost) { best_cost = c; best = S; }
+        const int whole = S > 1 ? 0 : per_xcd;
+        add(BwdCut{per_xcd, whole, per_xcd - whole, S, 1}, rounds * (work / S + WG_COST) + (S > 1 ? split_cost(per_xcd * S) : 0.0));
     }
-    cut.splits = best;
-    cut.whole = best == 1 ? cut.blocks_per_xcd : 0;
-    cut.mid = cut.blocks_per_xcd - cut.whole;
     // Equal blocks, more of them than CUs: whole rounds of unsplit blocks first (no partial sums,
     // one ramp per block), and only the blocks past the last whole round are cut - all alike into
     // as many ranges as fill their rounds best, or in two groups that make one round each: as
     // many blocks as give every CU one work-group when cut in S1 = ceil(CUs / blocks), and what
     // is left then in as many ranges as the CUs can take.
     const int cu_x = n_cu / XCDS;
-    if (!ragged && cu_x > 0 && cut.blocks_per_xcd > cu_x && blocks % XCDS == 0) {
-        const int full = cut.blocks_per_xcd / cu_x * cu_x, rest = cut.blocks_per_xcd - full;
-        if (rest == 0) return cut;       // (best is 1 then)
+    if (!ragged && cu_x > 0 && per_xcd > cu_x && blocks % XCDS == 0) {
+        const int full = per_xcd / cu_x * cu_x, rest = per_xcd - full;
+        if (rest == 0) return all;       // (whole is best then)
         const double whole_cost = (full / cu_x) * (steps + WG_COST);
         for (int S = 2; S <= 8; ++S) {
             if (steps / S < MIN_RANGE) break;
-            const double c = whole_cost + ((rest * S + cu_x - 1) / cu_x) * ((double)steps / S + WG_COST) + split_cost(rest * S);
-            if (c < best_cost) { best_cost = c; cut.whole = full; cut.mid = rest; cut.splits = S; cut.splits2 = 1; }
+            add(BwdCut{per_xcd, full, rest, S, 1}, whole_cost + ((rest * S + cu_x - 1) / cu_x) * ((double)steps / S + WG_COST) + split_cost(rest * S));
         }
         const int S1 = (cu_x + rest - 1) / rest;
         const int n1 = std::min(rest, cu_x / S1), left = rest - n1;
         if (S1 >= 2 && steps / S1 >= MIN_RANGE && left > 0) {
             int S2 = std::min(std::min(cu_x / left, MAX_SPLITS_PER_BLOCK), steps / MIN_RANGE);
-            if (S2 >= 2) {
-                const double c = whole_cost + ((double)steps / S1 + WG_COST) + ((double)steps / S2 + WG_COST) + split_cost(n1 * S1 + left * S2);
-                if (c < best_cost) { best_cost = c; cut.whole = full; cut.mid = n1; cut.splits = S1; cut.splits2 = S2; }
-            }
+            if (S2 >= 2)
+                add(BwdCut{per_xcd, full, n1, S1, S2},
+                    whole_cost + ((double)steps / S1 + WG_COST) + ((double)steps / S2 + WG_COST) + split_cost(n1 * S1 + left * S2));
         }
     }
-    return cut;
+    return all;
+}
+
+static BwdCut choose_bwd_cut(int blocks, int steps, bool masked, bool sliced) {
+    const BwdCuts all = bwd_cuts(blocks, steps, masked, sliced);
+    int best = 0;
+    for (int i = 1; i < all.n; ++i)
+        if (all.cost[i] < all.cost[best]) best = i;
+    return all.cut[best];
+}
+
+// The most slices an XCD can have in a window of up to so many steps: of any cut that is cheaper than none, which it is for more steps too if it
+// is for these.
+static int most_slices(int blocks, int steps, bool masked) {
+    const BwdCuts all = bwd_cuts(blocks, steps, masked, true);
+    int most = 0;
+    for (int i = 1; i < all.n; ++i)
+        if (all.cost[i] < all.cost[0] && all.cut[i].ranges() <= MAX_SLICES) most = std::max(most, all.cut[i].ranges());
+    return most;
 }
 
 static size_t slice_bytes(const lvx_attn_shape* s) { return (size_t)2 * 128 * s->D * sizeof(float); }
 static int token_blocks(const lvx_attn_shape* s) { return s->B * s->Hkv * ((s->Lkv + 127) / 128); }
 
-// Room for fp32 sums of dK and dV: of all tokens, or of MAX_SLICES ranges an XCD where it has any blocks to cut.  (Whatever the rows, so that a
-// workspace of the longest window serves all.)
-static size_t dkv_scratch_bytes(const lvx_attn_shape* s) {
+// The device plans a masked launch (see PlanParams) of blocks_per_xcd token blocks that is cut nowhere.
+static bool plans(const lvx_attn_shape* s, int blocks_per_xcd, int steps) {
+    const int cus = cu_count() / 8;
+    return s->kv_start && !s->bias && cus > 0 && cus <= 64 && blocks_per_xcd >= 2 * cus && blocks_per_xcd <= MAX_PLANNED_BLOCKS && steps >= 2 * MIN_PLANNED_RANGE;
+}
+static size_t plan_bytes(int slots, int shared_max) {
+    return ((size_t)(8 * slots * PLAN_ENTRY + 8 * shared_max * SHARED_ENTRY) * sizeof(uint32_t) + 255) / 256 * 256;
+}
+
+// Room for fp32 sums of dK and dV: of all tokens; or, `sliced`, also of the slices that a window of up to row_count rows can have, and the plan before them.
+static size_t dkv_scratch_bytes(const lvx_attn_shape* s, int32_t row_count, bool sliced) {
     const size_t all = (size_t)2 * s->B * s->Lkv * s->Hkv * s->D * sizeof(float);
-    const int blocks = token_blocks(s);
-    return blocks < 8 ? all : std::max(all, (size_t)8 * std::min(MAX_SLICES, 8 * ((blocks + 7) / 8)) * slice_bytes(s));
+    const int blocks = token_blocks(s), per_xcd = (blocks + 7) / 8, cus = cu_count() / 8;
+    if (!sliced || blocks < 8 || s->Hkv <= 0 || s->Hq <= 0) return all;     // (nothing has been checked yet where only the room is asked for)
+    const int steps = (int)(s->Hq / s->Hkv * (((int64_t)row_count + 31) / 32));
+    size_t room = 8 * most_slices(blocks, steps, s->kv_start != nullptr) * slice_bytes(s);
+    if (plans(s, per_xcd, steps)) room = std::max(room, plan_bytes(per_xcd + cus, cus) + 8 * 2 * cus * slice_bytes(s));
+    return std::max(all, room);
 }
 
 static DqCut dq_cut(const lvx_attn_shape* s, int32_t row_count) {
@@ -841,7 +868,7 @@ struct BwdWorkspace {
     int n_tiles, n_groups;
 };
 
-static BwdWorkspace bwd_workspace(const lvx_attn_shape* s, int32_t row_count) {
+static BwdWorkspace bwd_workspace(const lvx_attn_shape* s, int32_t row_count, bool sliced) {
     BwdWorkspace w{};
     const size_t tokens = ((size_t)s->Lkv + 127) / 128 * 128;
     const size_t rows = ((size_t)row_count + 31) / 32 * 32;
@@ -850,7 +877,7 @@ static BwdWorkspace bwd_workspace(const lvx_attn_shape* s, int32_t row_count) {
     w.n_groups = (w.n_tiles + LIVE_GROUP - 1) / LIVE_GROUP;
     size_t off = 0;
     w.ds = off; off += (size_t)s->B * s->Hq * tokens * rows * sizeof(uint16_t);
-    w.dkv = off; off += dkv_scratch_bytes(s);
+    w.dkv = off; off += dkv_scratch_bytes(s, row_count, sliced);
     w.meta = off; off += (size_t)s->B * s->Hq * rows * 2 * sizeof(float);
     w.dq32 = off; off += dq_partial_bytes(s, row_count);
     if (s->kv_start) {
@@ -865,7 +892,12 @@ static BwdWorkspace bwd_workspace(const lvx_attn_shape* s, int32_t row_count) {
 
 size_t lvx_bwd_workspace_bytes(const lvx_attn_shape* s, int32_t row_count) {
     if (!s || row_count <= 0) return 0;
-    return bwd_workspace(s, row_count).total;
+    return bwd_workspace(s, row_count, true).total;
+}
+
+size_t lvx_bwd_acc_workspace_bytes(const lvx_attn_shape* s, int32_t row_count) {
+    if (!s || row_count <= 0) return 0;
+    return bwd_workspace(s, row_count, false).total;
 }
 
 // The slices of a window's dQ that wait for the next launch to sum them.
@@ -874,12 +906,12 @@ struct WaitingDq {
     CastParams slices;
 };
 
-// One window, its arguments checked, in the workspace of one of ws_rows rows, at least as many.  meta: null, or the records of
+// One window, its arguments checked, in the workspace of one of ws_rows rows, at least as many, with room for slices or without.  meta: null, or the records of
 // its rows.  before: null, or what the window before has left and this one may leave.
 static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v, const lvx_tensor* o,
                       const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
                       const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate, int32_t row_begin, int32_t row_count,
-                      void* workspace, int32_t ws_rows, hipStream_t st, const float* meta, WaitingDq* before);
+                      void* workspace, int32_t ws_rows, bool sliced, hipStream_t st, const float* meta, WaitingDq* before);
 
 // The row records' arguments.  Delta is read, or with o (and no delta) formed on the way.
 static MetaParams meta_params(const lvx_attn_shape* s, const lvx_tensor* o, const lvx_tensor* dout, const float* lse, const float* delta,
@@ -916,15 +948,18 @@ static int bwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     if ((int64_t)s->Lq * q->stride_s >= (int64_t)1 << 31 || (int64_t)s->Lq * dout->stride_s >= (int64_t)1 << 31)
         return LVX_ERR_UNSUPPORTED;
     const int round_rows = rounds > 1 ? (row_count + rounds - 1) / rounds : row_count;
-    if (!workspace || workspace_bytes < lvx_bwd_workspace_bytes(s, round_rows)) return LVX_ERR_WORKSPACE;
+    if (!workspace || workspace_bytes < lvx_bwd_acc_workspace_bytes(s, round_rows)) return LVX_ERR_WORKSPACE;
     if (!aligned16(workspace)) return LVX_ERR_ALIGN;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (rounds <= 1) return bwd_window(s, q, k, v, o, dout, lse, delta, dq, dk, dv, dkv_accumulate, row_begin, row_count, workspace, row_count, st, nullptr, nullptr);
+    if (rounds <= 1) {
+        const bool sliced = !dkv_accumulate && workspace_bytes >= lvx_bwd_workspace_bytes(s, row_count);
+        return bwd_window(s, q, k, v, o, dout, lse, delta, dq, dk, dv, dkv_accumulate, row_begin, row_count, workspace, row_count, sliced, st, nullptr, nullptr);
+    }
 
     // Several windows: the records of all their rows by one launch instead of one of 3 - 5 us each (32 heads x 16 rounds of 256 rows,
     // forward and backward 2775 -> 2741 us), where the scratch that only sums of 16-bit dk, dv use holds them.
     const int n = (row_count + round_rows - 1) / round_rows;
-    const BwdWorkspace w = bwd_workspace(s, round_rows);
+    const BwdWorkspace w = bwd_workspace(s, round_rows, false);
     const int64_t each = (int64_t)s->B * s->Hq * w.n_tiles * 64;
     float* meta = nullptr;
     if (n <= 65535 && (size_t)each * n * sizeof(float) <= w.meta - w.dkv) {
@@ -937,7 +972,7 @@ static int bwd_impl(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tens
     WaitingDq waiting{};
     for (int r = 0; r < n; ++r)
         LVX_TRY(bwd_window(s, q, k, v, o, dout, lse, delta, dq, dk, dv, 1, row_begin + r * round_rows, std::min(round_rows, row_count - r * round_rows),
-                           workspace, round_rows, st, meta ? meta + r * each : nullptr, &waiting));
+                           workspace, round_rows, false, st, meta ? meta + r * each : nullptr, &waiting));
     return waiting.any ? static_cast<int>(launch_cast(waiting.slices, st)) : LVX_OK;
 }
 
@@ -961,7 +996,7 @@ int lvx_bwd_from_o(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tenso
 static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_tensor* k, const lvx_tensor* v, const lvx_tensor* o,
                       const lvx_tensor* dout, const float* lse, const float* delta, const lvx_tensor* dq,
                       const lvx_tensor* dk, const lvx_tensor* dv, int32_t dkv_accumulate, int32_t row_begin, int32_t row_count,
-                      void* workspace, int32_t ws_rows, hipStream_t st, const float* meta, WaitingDq* before) {
+                      void* workspace, int32_t ws_rows, bool sliced, hipStream_t st, const float* meta, WaitingDq* before) {
     BwdParams p{};
     p.f16 = s->dtype == LVX_F16;
     p.D = s->D;
@@ -990,15 +1025,15 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     // heads of 64 (0.2 GB) 208 -> 213, rounds of 256 rows (0.1 GB) 2940 -> 2966 for sixteen.
     p.ds_stream = (int64_t)s->B * s->Hq * p.ws_bh * 2 > ((int64_t)240 << 20);
 
-    const BwdWorkspace wsl = bwd_workspace(s, ws_rows);
+    const BwdWorkspace wsl = bwd_workspace(s, ws_rows, sliced);
     const int n_tiles = (int)(rows / 32), n_groups = (n_tiles + LIVE_GROUP - 1) / LIVE_GROUP;
     char* const wsb = static_cast<char*>(workspace);
     // how the launch is shaped decides which fp32 scratches it accumulates into; the
     // metadata kernel zeroes them on its way
     const int blocks = s->B * s->Hkv * p.n_kv_blocks;
     const int steps = p.G * (int)(rows / 32);
-    const BwdCut cut = choose_bwd_cut(blocks, steps, s->kv_start != nullptr, blocks >= 8 && !dkv_accumulate);
-    if (cut.any_split() && !dkv_accumulate && (size_t)8 * cut.ranges() * slice_bytes(s) <= wsl.meta - wsl.dkv) {
+    const BwdCut cut = choose_bwd_cut(blocks, steps, s->kv_start != nullptr, blocks >= 8 && sliced);
+    if (cut.any_split() && sliced && (size_t)8 * cut.ranges() * slice_bytes(s) <= wsl.meta - wsl.dkv) {
         p.slices = reinterpret_cast<float*>(wsb + wsl.dkv);
         p.per_xcd = cut.ranges();
     }
@@ -1006,15 +1041,13 @@ static int bwd_window(const lvx_attn_shape* s, const lvx_tensor* q, const lvx_te
     // seldom hides anything, and the plan would be 3 us for nothing.)
     PlanParams plan{};
     const int cus = cu_count() / 8;
-    if (s->kv_start && !s->bias && !meta && !dkv_accumulate && cus > 0 && cus <= 64 && cut.blocks_per_xcd >= 2 * cus &&
-        cut.blocks_per_xcd <= MAX_PLANNED_BLOCKS && !cut.any_split() && steps >= 2 * MIN_PLANNED_RANGE &&
-        (int64_t)s->B * n_groups * LIVE_GROUP <= MAX_LIVE_TILES) {
+    if (plans(s, cut.blocks_per_xcd, steps) && !meta && !dkv_accumulate && !cut.any_split() && (int64_t)s->B * n_groups * LIVE_GROUP <= MAX_LIVE_TILES) {
         plan.cus = plan.shared_max = cus;
         plan.slots = cut.blocks_per_xcd + cus;
         plan.n_blocks = blocks; plan.blocks_per_xcd = cut.blocks_per_xcd; plan.G = p.G;
         plan.entries = reinterpret_cast<uint32_t*>(wsb + wsl.dkv);
         plan.shared = plan.entries + 8 * plan.slots * PLAN_ENTRY;
-        const size_t tables = ((size_t)(8 * plan.slots * PLAN_ENTRY + 8 * plan.shared_max * SHARED_ENTRY) * sizeof(uint32_t) + 255) / 256 * 256;
+        const size_t tables = plan_bytes(plan.slots, plan.shared_max);
         const size_t room = wsl.meta - wsl.dkv;
         plan.slices = room > tables ? (int)std::min<size_t>((room - tables) / slice_bytes(s) / 8, 2 * cus) : 0;
         if (plan.slices < 2) plan.entries = nullptr;

@@ -32,7 +32,7 @@ struct Library {
     decltype(&lvx_bwd_preprocess) bwd_preprocess;
     decltype(&lvx_bwd) bwd;
     decltype(&lvx_bwd_from_o) bwd_from_o;
-    decltype(&lvx_bwd_workspace_bytes) bwd_workspace_bytes;
+    decltype(&lvx_bwd_workspace_bytes) bwd_workspace_bytes, bwd_acc_workspace_bytes;
     decltype(&lvx_bias_hull) bias_hull;
 } lib;
 
@@ -45,6 +45,7 @@ void bind(const std::map<std::string, uintptr_t>& addresses) {
     set(lib.bwd, "lvx_bwd");
     set(lib.bwd_from_o, "lvx_bwd_from_o");
     set(lib.bwd_workspace_bytes, "lvx_bwd_workspace_bytes");
+    set(lib.bwd_acc_workspace_bytes, "lvx_bwd_acc_workspace_bytes");
     set(lib.bias_hull, "lvx_bias_hull");
 }
 
@@ -224,10 +225,10 @@ py::object bias_hull(const Tensor& q, const Tensor& k, const Tensor& bias) {
 
 // Bytes of the backward's workspace for a window of `rows` rows, or -1.
 int64_t bwd_workspace_bytes(const Tensor& q, const Tensor& k, int64_t rows, const OptTensor& kv_len, const OptTensor& kv_start,
-                            const OptTensor& kv_end) {
+                            const OptTensor& kv_end, bool accumulate_dkv) {
     lvx_attn_shape s;
     if (!fill_shape(s, q, k, k, 1.0, kv_len, kv_start, kv_end)) return -1;
-    return (int64_t)lib.bwd_workspace_bytes(&s, (int32_t)rows);
+    return (int64_t)(accumulate_dkv ? lib.bwd_acc_workspace_bytes : lib.bwd_workspace_bytes)(&s, (int32_t)rows);
 }
 
 // (dq, dk, dv) of a backward: dq contiguous, or in q's memory order with `like_q`; dk and dv views of

@@ -303,11 +303,18 @@ def _attn_backward(do, q, k, v, o, L, causal, sm_scale, comm_mode, backward_engi
 
     dq, dk, dv = host().backward_outputs(q_, k_, _dq_like_q)
 
+    def least_bytes(rows):
+        return ops.bwd_workspace_bytes(q_, k_, rows, mask, accumulate_dkv=True)
+
     blocks = [(0, Lq)] if batched else [w for w in q_block_bounds(Lq, P) if w[1] > w[0]]
-    windows = _cap_windows(blocks, lambda rows: ops.bwd_workspace_bytes(q_, k_, rows, mask), backward_workspace_cap())
+    cap = backward_workspace_cap()
+    windows = _cap_windows(blocks, least_bytes, cap)
     one_call = len(windows) == len(blocks) < 1 << 18            # the windows are the query blocks
-    ws = workspace("bwd_ds", (ops.bwd_workspace_bytes(q_, k_, max(r1 - r0 for r0, r1 in windows), mask),),
-                   torch.uint8, dev)
+    rows = max(r1 - r0 for r0, r1 in windows)
+    nbytes = ops.bwd_workspace_bytes(q_, k_, rows, mask, accumulate_dkv=len(windows) > 1)
+    if nbytes > cap:            # sums of dK and dV by atomics rather than in more windows
+        nbytes = least_bytes(rows)
+    ws = workspace("bwd_ds", (nbytes,), torch.uint8, dev)
     if len(windows) == 1:
         r0, r1 = windows[0]
         ops.bwd(q_, k_, v_, do_, L_, None, dq, dk, dv, sm_scale, r0, r1 - r0, mask, accumulate_dkv=False,

@@ -209,15 +209,16 @@ def bwd_preprocess(o, dout, delta, row_begin=0, row_count=None) -> None:
     check(rc, "lvx_bwd_preprocess")
 
 
-def bwd_workspace_bytes(q, k, row_count: int, mask: Optional[Mask] = None) -> int:
+def bwd_workspace_bytes(q, k, row_count: int, mask: Optional[Mask] = None, accumulate_dkv: bool = False) -> int:
     """Bytes lvx_bwd needs for `row_count` rows; pass the mask the call will use
-    (an interval mask adds its live-tile tables)."""
+    (an interval mask adds its live-tile tables).  With `accumulate_dkv`: those of a call that accumulates, which any call can do with."""
     m = mask or _NO_MASK
-    n = host().bwd_workspace_bytes(q, k, row_count, m.kv_len, m.kv_start, m.kv_end)
+    n = host().bwd_workspace_bytes(q, k, row_count, m.kv_len, m.kv_start, m.kv_end, accumulate_dkv)
     if n >= 0:
         return n
     s = _shape(q, k, 1.0, mask)
-    return int(load().lvx_bwd_workspace_bytes(C.byref(s), row_count))
+    ask = load().lvx_bwd_acc_workspace_bytes if accumulate_dkv else load().lvx_bwd_workspace_bytes
+    return int(ask(C.byref(s), row_count))
 
 
 def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=None,
@@ -226,7 +227,7 @@ def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=Non
         o: Optional[torch.Tensor] = None) -> None:
     """Writes dq (bf16) for the selected rows and writes (bf16) or accumulates
     (fp32) dk, dv at Hkv heads.  `workspace`: uint8 tensor of at least
-    bwd_workspace_bytes(q, k, row_count, mask) bytes.  `bias` as in fwd (no gradient
+    bwd_workspace_bytes(q, k, row_count, mask, accumulate_dkv) bytes.  `bias` as in fwd (no gradient
     is formed for it).  `rounds` > 1 (with accumulate_dkv): the rows are that many windows, one after the other, in the
     workspace of one of ceil(row_count / rounds) rows.  `o`, with delta None: delta is formed from it on the way (see
     bwd_preprocess)."""
@@ -251,7 +252,7 @@ def bwd(q, k, v, dout, lse, delta, dq, dk, dv, scale, row_begin=0, row_count=Non
     if dk.dtype != want or dv.dtype != want or dk.shape != k.shape or dv.shape != k.shape:
         raise LvxError(f"dk/dv must be {want} tensors shaped like k")
     if workspace is None:
-        workspace = torch.empty(bwd_workspace_bytes(q, k, -(-row_count // rounds), mask), dtype=torch.uint8, device=q.device)
+        workspace = torch.empty(bwd_workspace_bytes(q, k, -(-row_count // rounds), mask, accumulate_dkv), dtype=torch.uint8, device=q.device)
     end = (C.byref(t4(dq)), C.byref(t4(dk)), C.byref(t4(dv)), flags, row_begin, row_count, workspace.data_ptr(),
            workspace.numel() * workspace.element_size(), stream_ptr())
     qkv = (C.byref(s), C.byref(t4(q)), C.byref(t4(k)), C.byref(t4(v)))
