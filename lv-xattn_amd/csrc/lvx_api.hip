@@ -195,8 +195,8 @@ static FwdPrice fwd_price(const lvx_attn_shape* s, FwdForm form) {
     return s->D == 128 ? FwdPrice{1.1, 0.4, 11.0, false, 0.0} : FwdPrice{0.9, 0.15, 11.0, false, 0.0};
 }
 
-static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32, const FwdPrice& price) {
-    const int G = s->Hq / s->Hkv, hg = gcd(G, 4), rs = 4 / hg, n_cu = cu_count();
+static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32, int n_cu, const FwdPrice& price) {
+    const int G = s->Hq / s->Hkv, hg = gcd(G, 4), rs = 4 / hg;
     const int64_t split_len = fwd_split_len(s, form, splits);
     const int64_t n = (s->Lkv + split_len - 1) / split_len;
     const double fold_us = (4 * s->D + 8) / 4e6 + (parts_f32 ? 4 * s->D / 9e6 : 0.0);       // per row, head and part
@@ -214,8 +214,8 @@ static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int spli
     const double tile_us = price.tile_us + price.load_us * (price.shared ? (wgs > n_cu ? 1.0 : 0.0) : std::min(1.0, (double)wgs / slots));
     return t + (double)((wgs + slots - 1) / slots) * (split_len / FWD_BN * tile_us + price.round_us);
 }
-static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32) {
-    return fwd_cost(s, rows, form, splits, parts_f32, fwd_price(s, form));
+static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32, int n_cu) {
+    return fwd_cost(s, rows, form, splits, parts_f32, n_cu, fwd_price(s, form));
 }
 
 // A second, closer fit, for launches without a dense bias: what the forms take by now, among them the fold inside a launch for few rows, K
@@ -224,11 +224,11 @@ static double fwd_cost(const lvx_attn_shape* s, int rows, FwdForm form, int spli
 // shares its CU takes longer per key, with heads of 64 by half; and a load of the fold inside a launch holds 2048 / D parts.  With one price for both, and
 // for parts of any size, short launches and small heads were cut where that costs: 155 rows x 3 x 16 heads of 64 x 2652 keys 17.5 us whole,
 // 19.8 in two parts, 3 x 2 x 2 of 32 x 12498 7.5 in 56, 8.6 in 23.)
-static double fwd_cost2(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32) {
+static double fwd_cost2(const lvx_attn_shape* s, int rows, FwdForm form, int splits, bool parts_f32, int n_cu) {
     struct Fit { double key_us, key2_us, tile_us, load_us, round_us; };     // per key of a work-group that has its CU to itself, that shares it
     const Fit f = s->D == 128 ? Fit{7.7e-3, 7.7e-3, 1.2, 0.26, 4.5} : s->D == 64 ? Fit{4.4e-3, 6.9e-3, 1.1, 0.0, 3.4}
                 : s->D == 32 ? Fit{3.8e-3, 5.3e-3, 1.2, 0.2, 1.6} : Fit{3.7e-3, 4.9e-3, 1.1, 0.0, 1.7};
-    const int G = s->Hq / s->Hkv, hg = gcd(G, 4), n_cu = cu_count();
+    const int G = s->Hq / s->Hkv, hg = gcd(G, 4);
     const int64_t split_len = fwd_split_len(s, form, splits), n = (s->Lkv + split_len - 1) / split_len;
     const auto both = [](double x, double y) { return std::sqrt(x * x + y * y); };      // (hypot takes three times as long, for ranges that are not ours)
     const double kv_mb = (double)s->B * s->Hkv * s->Lkv * s->D * 4e-6;
@@ -288,9 +288,10 @@ static FwdForm fwd_form(const lvx_attn_shape* s, int rows, int splits, bool part
     if (n == 1) return ok[0];
     double first[3], closer[3];
     int a = 0, b = 0;                   // cheapest by either fit
+    const int n_cu = cu_count();
     for (int i = 0; i < n; ++i) {
-        first[i] = fwd_cost(s, rows, ok[i], splits, parts_f32);
-        closer[i] = s->bias ? 0.0 : fwd_cost2(s, rows, ok[i], splits, parts_f32);
+        first[i] = fwd_cost(s, rows, ok[i], splits, parts_f32, n_cu);
+        closer[i] = s->bias ? 0.0 : fwd_cost2(s, rows, ok[i], splits, parts_f32, n_cu);
         if (first[i] < first[a] || (ok[i] == FWD_FEW && first[i] == first[a])) a = i;
         if (closer[i] < closer[b]) b = i;
     }
@@ -315,11 +316,12 @@ static bool fwd_parts_f32(const lvx_attn_shape* s, int rows, FwdForm form) {
 
 int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
     if (check_shape(s) != LVX_OK || row_count <= 0) return 1;
+    const int n_cu = cu_count();
     // The number of ranges for less than best_cost (0: for any), or 0.
     const auto cheapest = [&](FwdForm form, bool f32, const FwdPrice& price, double& best_cost) {
         int best = 0;
         for (int n = 1; n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
-            const double c = fwd_cost(s, row_count, form, n, f32, price);
+            const double c = fwd_cost(s, row_count, form, n, f32, n_cu, price);
             if (best_cost == 0.0 || c < best_cost) { best = n; best_cost = c; }
         }
         return best;
@@ -344,12 +346,12 @@ int lvx_fwd_auto_splits(const lvx_attn_shape* s, int32_t row_count) {
     double best2_cost = 0.0;
     for (const FwdForm form : FWD_FORMS)
         for (int n = 1; fwd_form_ok(s, row_count, form) && n <= MAX_SPLITS && (n == 1 || s->Lkv / n >= 32); ++n) {
-            const double c = fwd_cost2(s, row_count, form, n, parts(n, form) != n);
+            const double c = fwd_cost2(s, row_count, form, n, parts(n, form) != n, n_cu);
             if (best2_cost == 0.0 || c < best2_cost) { best2 = parts(n, form); best2_cost = c; }
         }
     const int n = best & ~LVX_SPLITS_FP32;
     const FwdForm form = fwd_form(s, row_count, n, best != n);
-    if (fwd_cost2(s, row_count, form, n, best != n) > CLOSER_FIT * best2_cost) return best2;
+    if (fwd_cost2(s, row_count, form, n, best != n, n_cu) > CLOSER_FIT * best2_cost) return best2;
     return form == FWD_FEW ? parts(n, form) : best;
 }
 

@@ -139,7 +139,7 @@ def auto_kv_splits(B: int, Hq: int, Hkv: int, rows: int, Lkv: int, D: int = HEAD
     enough work-groups, as few as keep storing and folding the parts cheap.  The library prices
     the launch (lvx_fwd_auto_splits) and says by LVX_SPLITS_FP32 in the number whether their O waits for the
     fold in fp32; its answer depends on the sizes alone and is kept for the last 1024 of them (asking costs
-    5 us of host time, a decoded token's launches take 12 on the GPU)."""
+    4 to 7 us of host time, a decoded token's launch takes 10 on the GPU)."""
     s = AttnShape(B, Hq, Hkv, D, rows, Lkv, LVX_BF16, 1.0, None, None, None)
     if bias:        # only whether there is one matters; any aligned address and strides do
         s.bias, s.bias_stride_r = 16, (Lkv + 3) // 4 * 4
