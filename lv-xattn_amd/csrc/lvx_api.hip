@@ -736,8 +736,9 @@ int lvx_bwd_preprocess(const lvx_attn_shape* s, const lvx_tensor* o, const lvx_t
 //     rounds(S) = ceil(blocks * S / CUs)
 // for equal work-groups.  With an interval mask they differ in length (a token block
 // visits only the row tiles that see it; half of them is assumed); given at least two per CU the
-// dispatcher fills the tail by itself and rounds(S) is the plain quotient: splitting then
-// rarely pays (cfg4: 0.98 ms with 5 splits, 0.86 ms with none).
+// dispatcher fills the tail by itself and rounds(S) is the plain quotient: cutting every block then
+// rarely pays (2 x 3000 rows that see the image before them: 0.98 ms in 5 ranges, added with atomics, 0.86 in none).  What fills no round is cut
+// on the device there (see PlanParams).
 constexpr int MAX_SLICES = 96;          // of an XCD
 
 // How the token blocks of a launch are handed to work-groups (see bwd_kernel): per XCD, the first

@@ -929,8 +929,8 @@ struct FewColumns {
 // are requested before anything else happens: 128 KiB in flight per CU, and with ranges of 256 keys
 // or less every byte the work-group will read.  Bound by HBM where there is enough to read: 4 rows x 32
 // heads x 76848 keys (315 MB) take 61 us, 5.2 TB/s, the rate of a large copy, against 75 us in the
-// wide form; one row x 6404 keys (26 MB) 12.0 us with the fold of the parts against 17.4, most of
-// it latency (the kernel alone 6.1 us; 6.7 with the arguments fetched line by line and integer divisions for where it is).
+// wide form; one row x 6404 keys (26 MB) 10.1 us with the fold of the parts inside against 17.4 in two launches, most of
+// it latency (9.1 us in the kernel, 6.1 without the fold; 6.7 with the arguments fetched line by line and integer divisions for where it is).
 //   S^T[32 keys, 32 cols] = K (A, 16-byte LDS reads) x Q^T (B, registers)
 //   O^T[d, 32 cols]      += V^T (A, transposing LDS reads) x P^T (B, straight from S^T)
 // LDS rows are 2 DH bytes (128 below head dimension 64, the lanes past the head dimension repeat a

@@ -226,8 +226,8 @@ struct BwdParams {
 // as fill whole rounds of its CUs, get a work-group each, the others are cut into ranges of steps, and those nobody sees come last.  A range
 // leaves fp32 sums in a slice of its own, [dK, dV][128 tokens][D], and cast_slices_kernel adds and rounds them.
 // 2 x 3000 rows that see the image before them (77 blocks of 180 to 368 steps on 32 CUs: 602 steps until the last CU ends, 512 with 13
-// cut in two, by a count of steps): bwd_kernel 657 -> 615 us, what the launches before and after it take 18 -> 35, forward and
-// backward 1054 -> 1021.  (More CUs at work run at a lower clock.  Whole blocks chosen by simulating which CU is free when, to 512
+// cut in two, by a count of steps): bwd_kernel 620 -> 579 us, what the launches before and after it take 19 -> 33, forward and
+// backward 1057 -> 1037.  (More CUs at work run at a lower clock.  Whole blocks chosen by simulating which CU is free when, to 512
 // steps instead of 552, gave the same kernel and took 20 us longer to plan.)  Others of 500 blocks and more 0 to -6 %.
 // Entry l of XCD x: the block's number in the XCD's list | ranges << 16 | range << 24, and the slice of the block's first range; ~0: none.
 constexpr int MAX_PLANNED_BLOCKS = 256;         // of an XCD; with more rounds than eight there is little left to even out
