@@ -824,7 +824,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const std::conditional
 // Parts and counts go past the L2, of which every XCD has one: stores and loads of agent scope, each step's done (vmcnt) before
 // the next begins.
 // A launch of its own for the fold takes 4.5 us on the GPU and 3 of the host's time.  In here it is three ways to the memory side one
-// behind the other (part, count, parts), 3.4 us: one row x 32 heads x 6404 keys, keys from HBM 11.9 -> 10.55 us a pass, from the cache
+// behind the other (part, count, parts), 3.4 us: one row x 32 heads x 6404 keys, keys from HBM 11.6 -> 10.1 us a pass, from the cache
 // 12.4 -> 9.2; 4 x 1 rows, eight layers with a mask 206 -> 202.5.  (Counting before the sums are formed and waiting for parts that are
 // emptied at the start to be filled: 11.8 and 203.5, as the keys then queue behind that.  Loads of one part each and
 // reductions through LDS in the fold: 4.2 us.)
